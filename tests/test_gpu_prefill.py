@@ -215,6 +215,29 @@ def test_prefill_paired_blocks_with_offset_and_window_sampled_rows(nq, nkv, hd, 
     kv.close()
 
 
+@pytest.mark.parametrize("nq,nkv,hd,p0,T,win", [
+    (32, 8, 128, 8192, 177, 0),     # five parts
+    (32, 8, 128, 5000, 1, 0),       # one row, as many parts as there may be
+    (16, 8, 128, 4100, 45, 0),      # a block of 64 positions that is not full, tiles that do not divide evenly
+    (16, 8, 128, 2047, 700, 1500),  # a window: blocks whose ranges start inside a tile
+    (4, 4, 64, 3001, 140, 0),       # MHA: a block's last rows end before its last part
+    (8, 1, 64, 2500, 97, 0),        # two head chunks per KV head
+    (8, 4, 256, 3000, 100, 0),
+    (4, 4, 256, 1999, 130, 900),
+])
+def test_few_rows_over_many_keys_sampled_rows(nq, nkv, hd, p0, T, win):
+    # blocks whose keys are cut into parts for workgroups of their own, put together by a second launch: the
+    # rows put together agree with the oracle and are the same every time
+    print("prefill parts", nq, nkv, hd, p0, T, win, flush=True)
+    kv, q, k16, v16 = _setup(nq, nkv, hd, p0, T, seed=6000 + hd + T)
+    got = kv.prefill(0, p0, q, 0.0, win)
+    rows = sorted({0, T // 3, T // 2, min(31, T - 1), min(32, T - 1), max(T - 33, 0), max(T - 2, 0), T - 1})
+    want = oracle.causal_prefill(q, k16, v16, p0=p0, window=win, rows=rows, threads=8)
+    print("  errors", util.assert_close(got[rows], want[rows]), flush=True)
+    assert np.isfinite(got).all() and np.array_equal(got, kv.prefill(0, p0, q, 0.0, win))
+    kv.close()
+
+
 @pytest.mark.parametrize("every", [1, 3])
 @pytest.mark.parametrize("nq,nkv,hd,p0", [(16, 8, 256, 0), (8, 4, 256, 70), (32, 8, 128, 0), (4, 2, 64, 0)])
 def test_prefill_with_a_softmax_reference_that_moves_from_tile_to_tile(nq, nkv, hd, p0, every):

@@ -20,6 +20,14 @@ struct PrefillArgs {
     uint32_t p0, T, nq, nkv, group, hd, ctx_pad, window;
     float qscale;            // softmax scale * log2(e)
     uint32_t single;         // MFMA kernels: one position block per workgroup (grid = blocks) instead of a pair
+    // n_parts > 1 (with single; prefill_il / prefill_ild kernels): a block's tiles are cut into that many
+    // parts, a workgroup each (grid.z), and prefill_combine_kernel puts the parts' rows together
+    // (Measured, 32/8/128, appends included: 177 rows behind 8192 keys, 48 blocks in 5 parts: 102 -> 51 us, 16 rows
+    // behind 16 384, 8 in 32: 174 -> 48; 16/8/128, 1000 behind 16 384, 128 in 2: 230 -> 177; 8/4/256, 100 behind
+    // 8192: 208 -> 52.)
+    uint32_t n_parts;
+    float* part_o;           // [part][T][nq][hd], relative to the part's own softmax reference, not normalised
+    float* part_ml;          // [part][T][nq][2]: reference (log2 units, -inf: the row sees no key of the part), sum
 };
 
 // Any head_dim / group: one workgroup per (row, head), vector ALU only.
@@ -318,6 +326,52 @@ __device__ __forceinline__ void prefill_block_tiles(const PrefillArgs& a, uint32
         (a.window > 0 && wg_first_pos + 1 > a.window) ? wg_first_pos + 1 - a.window : 0;
     t_first = wg_lo / kTileKeys;
     t_last = (a.p0 + wg_last_row) / kTileKeys;            // inclusive
+}
+
+// Part `part` of such a range: equal runs of tiles, the last ones possibly short.  False: nothing is left for it.
+__device__ __forceinline__ bool prefill_part_tiles(const PrefillArgs& a, uint32_t part, uint32_t& t_first, uint32_t& t_last)
+{
+    const uint32_t per = (t_last - t_first + a.n_parts) / a.n_parts;      // tiles / parts, rounded up
+    t_first += part * per;
+    t_last = min(t_last, t_first + per - 1);
+    return t_first <= t_last;
+}
+
+// A part without tiles: its rows are marked as seeing no key.
+__device__ __forceinline__ void prefill_part_empty(const PrefillArgs& a, uint32_t part, uint32_t row0, uint32_t head, int lane)
+{
+    const uint32_t row = row0 + lane;
+    if (lane < 32 && row < a.T)
+        *reinterpret_cast<float2*>(a.part_ml + (((size_t)part * a.T + row) * a.nq + head) * 2) = make_float2(-INFINITY, 0.f);
+}
+
+// out = sum over the parts of O 2^(m - M), divided by the sum of l 2^(m - M), M the largest reference; parts in
+// order, so the result does not depend on which workgroup finished first.  A thread makes four values of a row;
+// a part in which the row sees no key is not read.  Bound by the parts' bytes (177 rows of 32 x 128 in five parts:
+// 14.5 MB, 5 us).
+__global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs a)
+{
+    const uint32_t per_row = a.hd / 4;
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, rows = (size_t)a.T * a.nq;
+    const size_t row = i / per_row;                       // (row, head)
+    if (row >= rows) return;
+    float M = -INFINITY;
+    for (uint32_t p = 0; p < a.n_parts; p++) M = fmaxf(M, a.part_ml[(p * rows + row) * 2]);
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    float l = 0.f;
+    for (uint32_t p = 0; p < a.n_parts; p++) {
+        const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + (p * rows + row) * 2);
+        if (ml.y == 0.f) continue;                        // (the sum, so that a NaN among the scores stays one)
+        const float w = fast_exp2(ml.x - M);
+        const float4 v = *reinterpret_cast<const float4*>(a.part_o + p * rows * a.hd + i * 4);
+        l += ml.y * w;
+        o.x += v.x * w;
+        o.y += v.y * w;
+        o.z += v.z * w;
+        o.w += v.w * w;
+    }
+    const float inv = (l > 0.f) ? 1.0f / l : 0.f;
+    *reinterpret_cast<float4*>(a.out + i * 4) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
 }
 
 // One position block of one workgroup: loads Q, streams the visible K / Vt

@@ -426,14 +426,18 @@ __device__ __forceinline__ void il_load_q(IlQRows<HD>& q, const PrefillArgs& a, 
 }
 
 // The tile range of position block pb for key set kg, into the context.
-template <int HD>
-__device__ __forceinline__ void il_ctx_tiles(IlCtx<HD>& cx, const PrefillArgs& a, uint32_t pb, uint32_t BP,
-                                             int kg, uint32_t& t_first, uint32_t& t_last)
+template <int HD, bool PART>
+__device__ __forceinline__ bool il_ctx_tiles(IlCtx<HD>& cx, const PrefillArgs& a, uint32_t pb, uint32_t BP,
+                                             int kg, uint32_t& t_first, uint32_t& t_last, uint32_t part)
 {
     prefill_block_tiles(a, pb, BP, t_first, t_last);
+    if constexpr (PART) {
+        if (!prefill_part_tiles(a, part, t_first, t_last)) return false;
+    }
     cx.t0 = t_first + kg;                                 // this set's tiles: t0, t0 + 2, ...
     cx.nt = (cx.t0 <= t_last) ? (t_last - cx.t0) / 2 + 1 : 0;
     cx.t_last = t_last;
+    return true;
 }
 
 // The copies and loads a block starts with: the first three K tiles and two Vt
@@ -453,11 +457,12 @@ __device__ __forceinline__ void il_first_loads(const IlCtx<HD>& cx, IlQRows<HD>&
 // One position block.  started: the block's first loads are already on their way
 // (q holds its Q rows).  next_pb >= 0: once this block's loop is over, the first
 // loads of block next_pb are issued, before the merge and the stores, and q
-// returns its Q rows.
-template <int HD>
+// returns its Q rows.  PART: part `part` of the block's tiles only; the rows leave
+// unnormalised, beside their reference and sum.
+template <int HD, bool PART>
 __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* smem, uint32_t pb,
                                          uint32_t kvh, uint32_t hc, const unsigned char* kbase, const unsigned char* vtbase,
-                                         bool started, IlQRows<HD>& q, int next_pb)
+                                         bool started, IlQRows<HD>& q, int next_pb, uint32_t part)
 {
     using L = SplitLds<HD>;
     static_assert(L::NL == 1 || L::NL == 2, "one or two copies per wave, tile and operand");
@@ -482,7 +487,10 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
     prefill_rows_init<HD, false>(R, a, row0, head, n, g);
 
     IlCtx<HD> cx;
-    il_ctx_tiles<HD>(cx, a, pb, BP, kg, t_first, t_last);
+    if (!il_ctx_tiles<HD, PART>(cx, a, pb, BP, kg, t_first, t_last, part)) {    // (uniform over the workgroup)
+        if (kg == 0) prefill_part_empty(a, part, row0, head, lane);
+        return;
+    }
     cx.tail_tile = kv_valid / kTileKeys;
     cx.kbase = kbase;
     cx.vtbase = vtbase;
@@ -621,13 +629,13 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
     __syncthreads();
     const int lane_e = il_fresh_lane();                   // lane, n, g again, for the code after the loop
     const int n_e = lane_e & 31, g_e = lane_e >> 5;
-    if (next_pb >= 0) {
+    if (!PART && next_pb >= 0) {
         // the rings are quiet and the merge below does not touch the slots these
         // go to: the next block's first tiles and Q rows travel while this block
         // is merged and stored
         IlCtx<HD> cn = cx;
         uint32_t nf, nl;
-        il_ctx_tiles<HD>(cn, a, (uint32_t)next_pb, BP, kg, nf, nl);
+        (void)il_ctx_tiles<HD, false>(cn, a, (uint32_t)next_pb, BP, kg, nf, nl, 0);
         il_first_loads<HD>(cn, q, a, (uint32_t)next_pb * BP + sub_rows, head, kg, lane_e);
     }
     if (kg == 1) {
@@ -649,8 +657,14 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
         const float f0m = (R.m_run == -INFINITY) ? 0.f : fast_exp2(R.m_run - m);
         const float f1m = (m1 == -INFINITY) ? 0.f : fast_exp2(m1 - m);
         const float l_tot = wave_pair32_sum(R.l_run * f0m + l1 * f1m);
-        const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
+        const float inv = PART ? 1.0f : (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
         const float w0 = f0m * inv, w1 = f1m * inv;
+        if constexpr (PART) {
+            const uint32_t my_row = row0 + n_e;
+            if (g_e == 0 && my_row < a.T)
+                *reinterpret_cast<float2*>(a.part_ml + (((size_t)part * a.T + my_row) * a.nq + head) * 2) =
+                    make_float2(m, l_tot);
+        }
 #pragma unroll
         for (int dt = 0; dt < HD / 32; dt++)
 #pragma unroll
@@ -677,9 +691,9 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
         for (int j = 0; j < 16 / RPI; j++) {
             const int r = kg * 16 + j * RPI + lane_e / LPR;
             const float4 v = *reinterpret_cast<const float4*>(&os[r][(lane_e % LPR) * 4]);
+            float* to = PART ? a.part_o + (size_t)part * a.T * a.nq * HD : a.out;
             if (row0 + r < a.T)
-                *reinterpret_cast<float4*>(a.out + ((size_t)(row0 + r) * a.nq + head) * HD +
-                                           (lane_e % LPR) * 4) = v;
+                *reinterpret_cast<float4*>(to + ((size_t)(row0 + r) * a.nq + head) * HD + (lane_e % LPR) * 4) = v;
         }
     }
 }
@@ -690,7 +704,9 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
 // (blocks-1-y) and then block y: a long block and a short one, so every
 // workgroup streams the same number of tiles despite the causal triangle.
 // a.single: grid.y = blocks, one block per workgroup, long blocks first.
-template <int HD>
+// PART (with a.single): grid.z = parts of a block's tiles, for few rows over many
+// keys, whose blocks alone would leave most CUs idle (the host's rule says when).
+template <int HD, bool PART>
 __global__ __launch_bounds__(kSplitThreads, 1) void prefill_il_kernel(const PrefillArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char prefill_smem_raw[];
@@ -708,12 +724,12 @@ __global__ __launch_bounds__(kSplitThreads, 1) void prefill_il_kernel(const Pref
     const unsigned char* vtbase = uniform_ptr(reinterpret_cast<const unsigned char*>(
         a.vt + (size_t)kvh * (a.ctx_pad / kVBlock) * HD * kVBlock));
     IlQRows<HD> q;
-    if (a.single || hi == lo) {
-        il_block<HD>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, false, q, -1);
-    } else {
-        il_block<HD>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, false, q, (int)lo);
+    if (PART || a.single || hi == lo) {
+        il_block<HD, PART>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, false, q, -1, blockIdx.z);
+    } else if constexpr (!PART) {
+        il_block<HD, false>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, false, q, (int)lo, 0);
         lds_barrier();                                    // LDS changes hands
-        il_block<HD>(a, prefill_smem_raw, lo, kvh, hc, kbase, vtbase, true, q, -1);
+        il_block<HD, false>(a, prefill_smem_raw, lo, kvh, hc, kbase, vtbase, true, q, -1, 0);
     }
 }
 

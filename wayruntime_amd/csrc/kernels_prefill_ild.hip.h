@@ -298,9 +298,11 @@ __device__ __forceinline__ void ild_step(PrefillRows<kIldHalf>& R, IlCtx<kIldHal
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// One position block.
+// One position block (PART: part `part` of its tiles, as il_block).
+template <bool PART>
 __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* smem, uint32_t pb, uint32_t kvh,
-                                          uint32_t hc, const unsigned char* kbase, const unsigned char* vtbase)
+                                          uint32_t hc, const unsigned char* kbase, const unsigned char* vtbase,
+                                          uint32_t part)
 {
     using L = SplitLds<kIldHalf>;
     constexpr int HD = 2 * kIldHalf, H = kIldHalf;
@@ -325,6 +327,12 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
 
     IlCtx<H> cx;
     prefill_block_tiles(a, pb, BP, t_first, t_last);
+    if constexpr (PART) {
+        if (!prefill_part_tiles(a, part, t_first, t_last)) {    // (uniform over the workgroup)
+            if (kg == 0) prefill_part_empty(a, part, row0, head, lane);
+            return;
+        }
+    }
     cx.t0 = t_first;
     cx.nt = t_last - t_first + 1;
     cx.t_last = t_last;
@@ -465,7 +473,13 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
     const int lane_e = il_fresh_lane();
     const int n_e = lane_e & 31, g_e = lane_e >> 5;
     const float l_tot = wave_pair32_sum(R.l_run);
-    const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
+    const float inv = PART ? 1.0f : (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
+    if constexpr (PART) {
+        const uint32_t my_row = row0 + n_e;
+        if (kg == 0 && g_e == 0 && my_row < a.T)          // (both halves hold the same reference and sum)
+            *reinterpret_cast<float2*>(a.part_ml + (((size_t)part * a.T + my_row) * a.nq + head) * 2) =
+                make_float2(R.m_run, l_tot);
+    }
     // rows leave through LDS: the wave's tile row-major in its own scratch, then
     // whole half rows (512 contiguous bytes) per 32 lanes
     float (*os)[H + 4] = reinterpret_cast<float (*)[H + 4]>(smem + (size_t)wave * IldLds::O_WAVE);
@@ -488,14 +502,16 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
         for (int jj = 0; jj < 32 / RPI; jj++) {
             const int r = jj * RPI + lane_e / LPR;
             const float4 v = *reinterpret_cast<const float4*>(&os[r][(lane_e % LPR) * 4]);
+            float* to = PART ? a.part_o + (size_t)part * a.T * a.nq * HD : a.out;
             if (row0 + r < a.T)
-                *reinterpret_cast<float4*>(a.out + ((size_t)(row0 + r) * a.nq + head) * HD + kg * H +
+                *reinterpret_cast<float4*>(to + ((size_t)(row0 + r) * a.nq + head) * HD + kg * H +
                                            (lane_e % LPR) * 4) = v;
         }
     }
 }
 
-// grid = (KV heads x head chunks, ceil(blocks / 2)), as prefill_il_kernel.
+// grid = (KV heads x head chunks, ceil(blocks / 2)), as prefill_il_kernel; PART: grid.z = parts.
+template <bool PART>
 __global__ __launch_bounds__(kSplitThreads, 1) void prefill_ild_kernel(const PrefillArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char prefill_smem_raw[];
@@ -512,10 +528,12 @@ __global__ __launch_bounds__(kSplitThreads, 1) void prefill_ild_kernel(const Pre
         uniform_ptr(reinterpret_cast<const unsigned char*>(a.k + (size_t)kvh * a.ctx_pad * HD));
     const unsigned char* vtbase = uniform_ptr(reinterpret_cast<const unsigned char*>(
         a.vt + (size_t)kvh * (a.ctx_pad / kVBlock) * HD * kVBlock));
-    ild_block(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase);
-    if (!a.single && hi != lo) {
-        __syncthreads();                                  // LDS changes hands
-        ild_block(a, prefill_smem_raw, lo, kvh, hc, kbase, vtbase);
+    ild_block<PART>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, blockIdx.z);
+    if constexpr (!PART) {
+        if (!a.single && hi != lo) {
+            __syncthreads();                              // LDS changes hands
+            ild_block<false>(a, prefill_smem_raw, lo, kvh, hc, kbase, vtbase, 0);
+        }
     }
 }
 

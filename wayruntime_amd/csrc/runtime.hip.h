@@ -78,6 +78,8 @@ extern thread_local Ctx* cx;
 constexpr uint32_t kDevErrLayerMask = 0x0000FFFFu;     // error word: bit 31 set (kDevErrWaitExpired), the layer in the low bits
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr uint32_t kDefaultTilesPerWg = 32;  // split-K decode: 1024 keys per workgroup
+constexpr uint32_t kMaxPrefillParts = 32;    // prefill: parts a block's keys are cut into at most,
+constexpr float kMaxPrefillPartMb = 128.f;   // and the bytes of the parts' rows
 constexpr uint32_t kMaxHeads = 4096;        // query heads per session the ticket array is sized for
 constexpr size_t kPinSmall = 1u << 20;      // host copies up to this size go through pinned staging
 

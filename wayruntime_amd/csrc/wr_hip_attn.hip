@@ -500,6 +500,48 @@ int check_decode(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32_
     return WR_HIP_OK;
 }
 
+// Into how many parts a launch's blocks are cut (one: not at all).  A launch of few rows lasts as long as its
+// longest block, whose keys one workgroup walks while most CUs stand idle; cut, every part pays a block's ends
+// (Q in, the sets' merge, rows out) and the rows go through memory once more.  In microseconds: the ends of a block,
+// a step (64 keys of a 32-row unit at head dims up to 128, 32 keys at 256; fewer workgroups than CUs), the combine
+// launch, and the bytes it and the parts move.
+uint32_t prefill_parts(const PrefillArgs& a, uint32_t BP, uint32_t nblk, uint32_t ny)
+{
+    const float ends = 8.f, step = a.hd == 256 ? 0.95f : 0.8f, combine = 5.f;
+    const float row_mb = (float)a.T * a.nq * a.hd * 4e-6f;
+    const uint32_t last_lo = a.p0 + (nblk - 1) * BP, hi = a.p0 + a.T;          // the last block's first position, keys
+    const uint32_t lo = (a.window > 0 && last_lo + 1 > a.window) ? last_lo + 1 - a.window : 0;
+    const uint32_t tiles = (hi + kTileKeys - 1) / kTileKeys - lo / kTileKeys, per_step = a.hd == 256 ? 1 : 2;
+    uint32_t best = 1;
+    float least = 0.f;
+    for (uint32_t p = 1; p <= kMaxPrefillParts; p++) {
+        if (p > 1 && p * row_mb > kMaxPrefillPartMb) break;
+        const uint32_t rounds = (nblk * ny * p + g.n_cus - 1) / g.n_cus;
+        const uint32_t steps = ((tiles + p - 1) / p + per_step - 1) / per_step;
+        float t = rounds * (ends + step * steps);
+        if (p > 1) t += combine + 2.f * p * row_mb / 4.f;                       // written and read at about 4 TB/s
+        if (p == 1 || t < least) {
+            least = t;
+            best = p;
+        }
+    }
+    return best;
+}
+
+// Room for the parts' rows in the thread's partial buffer.  False: there is none, and the launch goes uncut.
+bool prefill_parts_ready(PrefillArgs& a, uint32_t parts)
+{
+    const size_t rows = (size_t)parts * a.T * a.nq, o = rows * a.hd * sizeof(float);
+    if (ensure_device(cx->d_part, o + rows * 2 * sizeof(float)) != WR_HIP_OK) {
+        (void)hipGetLastError();
+        return false;
+    }
+    a.n_parts = parts;
+    a.part_o = reinterpret_cast<float*>(cx->d_part.p);
+    a.part_ml = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(cx->d_part.p) + o);
+    return true;
+}
+
 int prefill_locked(wr_hip_kv* kv, uint32_t layer, uint32_t p0, uint32_t T, const float* q_dev,
                    float* out_dev, uint32_t nq, float scale_override, uint32_t window,
                    const uint16_t* q16_dev = nullptr)
@@ -538,8 +580,21 @@ int prefill_locked(wr_hip_kv* kv, uint32_t layer, uint32_t p0, uint32_t T, const
         // prologue and epilogue.
         a.single = ((nblk + 1) / 2) * ny < g.n_cus ? 1 : 0;
         const uint32_t nwg = a.single ? nblk : (nblk + 1) / 2;
-        if (hd == 64)
-            launch_main(prefill_il_kernel<64>, dim3(ny, nwg), dim3(kSplitThreads), a,
+        const bool parts_form = hd == 64 || (hd == 128 && g.prefill_two_waves) || (hd == 256 && !g.prefill_256_four_waves);
+        const uint32_t parts = parts_form && a.single ? prefill_parts(a, BP, nblk, ny) : 1;
+        if (parts > 1 && prefill_parts_ready(a, parts)) {
+            const dim3 grid(ny, nblk, parts);
+            if (hd == 64)
+                launch_main(prefill_il_kernel<64, true>, grid, dim3(kSplitThreads), a, split_smem_bytes<64>());
+            else if (hd == 128)
+                launch_main(prefill_il_kernel<128, true>, grid, dim3(kSplitThreads), a, split_smem_bytes<128>());
+            else
+                launch_main(prefill_ild_kernel<true>, grid, dim3(kSplitThreads), a, ild_smem_bytes());
+            HIP_TRY(hipGetLastError(), "prefill launch", layer);
+            const uint32_t units = T * nq * (hd / 4);     // (bounded: few workgroups made these rows)
+            hipLaunchKernelGGL(prefill_combine_kernel, dim3((units + 255) / 256), dim3(256), 0, cx->stream, a);
+        } else if (hd == 64)
+            launch_main(prefill_il_kernel<64, false>, dim3(ny, nwg), dim3(kSplitThreads), a,
                         split_smem_bytes<64>());
         else if (hd == 128 && !g.prefill_two_waves) {
             if (q16_dev)
@@ -549,10 +604,10 @@ int prefill_locked(wr_hip_kv* kv, uint32_t layer, uint32_t p0, uint32_t T, const
                 launch_main(prefill_pair_kernel<128, false>, dim3(ny, nwg), dim3(kPairThreads), a,
                             pair_smem_bytes<128>());
         } else if (hd == 128)
-            launch_main(prefill_il_kernel<128>, dim3(ny, nwg), dim3(kSplitThreads), a,
+            launch_main(prefill_il_kernel<128, false>, dim3(ny, nwg), dim3(kSplitThreads), a,
                         split_smem_bytes<128>());
         else if (!g.prefill_256_four_waves)   // 256: the wave sets divide the dimensions
-            launch_main(prefill_ild_kernel, dim3(ny, nwg), dim3(kSplitThreads), a, ild_smem_bytes());
+            launch_main(prefill_ild_kernel<false>, dim3(ny, nwg), dim3(kSplitThreads), a, ild_smem_bytes());
         else   // the earlier form: one wave per SIMD owns all 256 dimensions of its rows
             launch_main(prefill_mfma_kernel<256>, dim3(nwg, ny), dim3(kPrefillThreads), a);
     } else {
@@ -955,13 +1010,22 @@ int wr_hip_attn_init(int device)
     if (rc == WR_HIP_OK) {
         // the two-waves-per-SIMD prefill kernels stage more than the 64 KiB a
         // kernel may use without asking
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<64>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<64, false>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)split_smem_bytes<64>());
         if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<128>),
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<128, false>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)split_smem_bytes<128>());
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<64, true>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_smem_bytes<64>());
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<128, true>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_smem_bytes<128>());
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_ild_kernel<true>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)ild_smem_bytes());
         if (e == hipSuccess)
             e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_pair_kernel<128, false>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -971,7 +1035,7 @@ int wr_hip_attn_init(int device)
                                     hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)pair_smem_bytes<128>());
         if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_ild_kernel),
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_ild_kernel<false>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)ild_smem_bytes());
         if (e == hipSuccess)
             e = hipFuncSetAttribute(reinterpret_cast<const void*>(proj_gemm_lds_kernel<8, 2, 3>),
