@@ -55,6 +55,36 @@ def test_append_is_bit_exact_and_leaves_neighbours_alone(nkv, hd, max_ctx, chunk
     kv.close()
 
 
+@pytest.mark.parametrize("nkv,hd,pos,n", [
+    (3, 136, 5, 90),      # a second run of eight dimensions; blocks covered in part at both ends
+    (2, 8, 31, 2),        # the smallest head, a position either side of a block's edge
+    (8, 128, 32, 64),     # whole blocks
+    (1, 264, 0, 33),
+])
+def test_append_takes_sources_on_any_address_and_as_stored_bits(nkv, hd, pos, n):
+    # the vector form (sources on 16 bytes), the general one (four bytes further) and stored rows: the same cache,
+    # and positions outside the call keep what they held
+    rows = pos + n + 40
+    k, v = synth.normal(150, (n, nkv, hd)), synth.normal(151, (n, nkv, hd))
+    old = synth.f32_to_f16_trunc(synth.normal(152, (rows, nkv, hd)))
+    kd = [hipattn.DeviceBuffer.from_host(np.concatenate([np.zeros(s, np.float32), k.ravel()])) for s in (0, 1)]
+    vd = [hipattn.DeviceBuffer.from_host(np.concatenate([np.zeros(s, np.float32), v.ravel()])) for s in (0, 1)]
+    want_k, want_v = old.copy(), old.copy()
+    want_k[pos:pos + n], want_v[pos:pos + n] = synth.f32_to_f16_trunc(k), synth.f32_to_f16_trunc(v)
+    for form in range(3):
+        print("append source", nkv, hd, pos, n, form, flush=True)
+        kv = hipattn.KVCache(1, hd, nkv, rows)
+        kv.write_f16(0, 0, old, old)
+        if form < 2:
+            assert hipattn.lib().wr_hip_attn_append_dev(kv.h, 0, pos, n, kd[form].p + 4 * form, vd[form].p + 4 * form) == hipattn.OK
+            hipattn.sync()
+        else:
+            kv.write_f16(0, pos, want_k[pos:pos + n], want_v[pos:pos + n])
+        got_k, got_v = kv.read_f16(0, 0, rows)
+        assert np.array_equal(got_k, want_k) and np.array_equal(got_v, want_v)
+        kv.close()
+
+
 def test_append_matches_oracle_append_row():
     import ctypes as C
     nkv, hd, cap = 2, 64, 37

@@ -76,6 +76,89 @@ __global__ __launch_bounds__(256) void append_v_kernel(const Src* __restrict__ s
     }
 }
 
+// Both sides in one launch, for head dims that are multiples of 8 and sources on
+// 16-byte boundaries (the two kernels above take the rest).  grid = (blocks of 32
+// positions, KV heads x runs of 128 dimensions, K or V): a workgroup owns a block's
+// 32 x 128 tile.  K: a thread reads eight dimensions of a position as vectors and
+// writes them as the 16-byte unit they are in the cache.  V: a thread reads four
+// dimensions of two neighbouring positions, the tile turns through LDS (rows of 17
+// words: two-way bank conflicts at most), and leaves as 16-byte units, eight
+// positions of a dimension, whole KiBs a wave; a block that is not covered from end
+// to end is written element by element, so its other positions stay as they are.
+// Bound by bytes, and at small sizes by the launch, of which it saves one: 2048 rows
+// of 8 x 128, 25 MB, 8.4 + 5.8 -> 5.7 us (append and attention together 61.9 -> 52.8).
+constexpr uint32_t kAppendDims = 128;
+
+template <typename Src> struct AppendVec;
+template <> struct AppendVec<float> {
+    typedef float V4 __attribute__((ext_vector_type(4)));
+};
+template <> struct AppendVec<uint16_t> {
+    typedef uint16_t V4 __attribute__((ext_vector_type(4)));
+};
+
+template <typename Src>
+__global__ __launch_bounds__(256) void append_kv_kernel(const Src* __restrict__ k_src, const Src* __restrict__ v_src,
+                                                        uint16_t* __restrict__ k, uint16_t* __restrict__ vt,
+                                                        uint32_t pos, uint32_t n_rows, uint32_t nkv, uint32_t hd,
+                                                        uint32_t ctx_pad)
+{
+    using V4 = typename AppendVec<Src>::V4;
+    __shared__ uint32_t turn[kAppendDims][17];
+    const uint32_t t = threadIdx.x, runs = (hd + kAppendDims - 1) / kAppendDims;
+    const uint32_t kvh = blockIdx.y / runs, d0 = blockIdx.y % runs * kAppendDims, nd = min(hd - d0, kAppendDims);
+    const uint32_t blk = pos / kVBlock + blockIdx.x, p0 = blk * kVBlock, end = pos + n_rows;
+    if (blockIdx.z == 0) {
+        const uint32_t q = t & 15;                        // eight dimensions
+        if (q * 8 >= nd) return;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t p = p0 + i * 16 + (t >> 4);
+            if (p < pos || p >= end) continue;
+            const V4* s = reinterpret_cast<const V4*>(k_src + ((size_t)(p - pos) * nkv + kvh) * hd + d0 + q * 8);
+            const V4 a = s[0], b = s[1];
+            u32x4 o;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                o[j] = (uint32_t)to_cache_bits<Src>(a[2 * j]) | (uint32_t)to_cache_bits<Src>(a[2 * j + 1]) << 16;
+                o[2 + j] = (uint32_t)to_cache_bits<Src>(b[2 * j]) | (uint32_t)to_cache_bits<Src>(b[2 * j + 1]) << 16;
+            }
+            *reinterpret_cast<u32x4*>(k + k_offset(kvh, ctx_pad, p, d0 + q * 8, hd)) = o;
+        }
+        return;
+    }
+    const uint32_t q = t & 31;                            // four dimensions
+    if (q * 4 < nd) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t pair = i * 8 + (t >> 5), p = p0 + 2 * pair;
+            V4 x[2];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                x[e] = V4{0, 0, 0, 0};
+                if (p + e >= pos && p + e < end)
+                    x[e] = *reinterpret_cast<const V4*>(v_src + ((size_t)(p + e - pos) * nkv + kvh) * hd + d0 + q * 4);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                turn[q * 4 + j][pair] = (uint32_t)to_cache_bits<Src>(x[0][j]) | (uint32_t)to_cache_bits<Src>(x[1][j]) << 16;
+        }
+    }
+    __syncthreads();
+    uint16_t* to = vt + vt_offset(kvh, ctx_pad, p0, d0, hd);      // the tile's dimensions, 32 positions each
+    if (p0 >= pos && p0 + kVBlock <= end) {
+        for (uint32_t u = t; u < nd * 4; u += 256) {
+            const uint32_t* w = &turn[u >> 2][(u & 3) * 4];
+            *reinterpret_cast<u32x4*>(to + (size_t)u * 8) = u32x4{w[0], w[1], w[2], w[3]};
+        }
+    } else {
+        for (uint32_t e = t; e < nd * kVBlock; e += 256) {
+            const uint32_t p = p0 + e % kVBlock;
+            if (p >= pos && p < end) to[e] = (uint16_t)(turn[e / kVBlock][e % kVBlock / 2] >> 16 * (e & 1));
+        }
+    }
+}
+
 // Rotary position embedding in place on F32 rows [rows][heads][hd], split-half
 // pairing (element j with element j + hd/2, j < n_rot), as the reference
 // applies it before the append (reference: src/core/kernels.c:1356-1412):

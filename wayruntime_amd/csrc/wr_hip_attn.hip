@@ -217,11 +217,20 @@ int append_rows_locked(wr_hip_kv* kv, uint32_t layer, uint32_t pos, uint32_t n_r
     const uint32_t hd = kv->hd[layer], nkv = kv->nkv;
     uint16_t* kbase = reinterpret_cast<uint16_t*>(kv->slab + kv->k_off[layer]);
     uint16_t* vbase = reinterpret_cast<uint16_t*>(kv->slab + kv->vt_off[layer]);
+    const uint32_t nblk = (pos + n_rows - 1) / kVBlock - pos / kVBlock + 1;
+    const uint32_t runs = (hd + kAppendDims - 1) / kAppendDims;
+    // vectors of eight dimensions: where they are whole and the sources lie on 16 bytes (and the grid's second
+    // dimension has room for the heads)
+    if (hd % 8 == 0 && (((uintptr_t)k_dev | (uintptr_t)v_dev) & 15) == 0 && (uint64_t)nkv * runs < 65536) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(append_kv_kernel<Src>), dim3(nblk, nkv * runs, 2), dim3(256), 0, cx->stream,
+                           k_dev, v_dev, kbase, vbase, pos, n_rows, nkv, hd, kv->ctx_pad);
+        HIP_TRY(hipGetLastError(), "append launch", layer);
+        return WR_HIP_OK;
+    }
     const size_t total = (size_t)n_rows * nkv * hd;
     const uint32_t blocks = (uint32_t)((total + 255) / 256);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(append_k_kernel<Src>), dim3(blocks), dim3(256), 0, cx->stream,
                        k_dev, kbase, pos, n_rows, nkv, hd, kv->ctx_pad);
-    const uint32_t nblk = (pos + n_rows - 1) / kVBlock - pos / kVBlock + 1;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(append_v_kernel<Src>), dim3((hd + 63) / 64, nkv, nblk),
                        dim3(256), 0, cx->stream, v_dev, vbase, pos, n_rows, nkv, hd, kv->ctx_pad);
     HIP_TRY(hipGetLastError(), "append launch", layer);
