@@ -360,3 +360,42 @@ def test_projection_random_shapes():
         w.close()
         done += 1
     assert done == 28
+
+
+@pytest.mark.parametrize("rows,n_in,n_out", [
+    (17, 1024, 4096),             # register GEMM of 16 x 16 tiles: the fewest rows, a whole share in one turn of eight
+    (48, 2080, 16),               # ... the most, 65 input tiles (a wave with one more than the others), one output tile
+    (31, 32, 48),                 # ... a single input tile: three waves with none
+    (49, 1056, 4112),             # 32 x 16 tiles: a last row group of one row, partial output tiles
+    (256, 3072, 80),              # ... the last row count whose fragments are made row by row
+    (257, 288, 1040),             # ... by row groups
+    (250, 1056, 4112),            # 32 x 32 tiles, 33 input tiles
+])
+def test_products_of_a_short_prompt(rows, n_in, n_out):
+    print("proj short prompt", rows, n_in, n_out, flush=True)
+    x, w16 = synth.normal(rows * 7 + n_in, (rows, n_in)), _w16(n_out + 3, n_out, n_in, 0.05)
+    w = hipattn.Weight([w16])
+    got = w.rows(x)
+    _check(got, x, w16, f"{rows}x{n_in}x{n_out}")
+    assert w.rows(x).tobytes() == got.tobytes()
+    w.close()
+
+
+@pytest.mark.parametrize("rows", [20, 270])
+@pytest.mark.parametrize("n_in", [256, 1056, 2080, 4128])
+def test_normed_and_gated_rows_by_rows_and_by_groups(rows, n_in):
+    # the two fragment kernels a product of many rows may take, all forms of each
+    lib, D, n_out, eps = hipattn.lib(), hipattn.DeviceBuffer, 48, 1e-6
+    x, gu = synth.normal(161 + n_in, (rows, n_in), std=2.0), synth.normal(163 + n_in, (rows, 2 * n_in), std=2.0)
+    nw, w16 = synth.normal(162, (n_in,)) * np.float32(0.2) + np.float32(1.0), _w16(165, n_out, n_in, 0.1)
+    w, xd, nwd, gud, y = hipattn.Weight([w16]), D.from_host(x), D.from_host(nw), D.from_host(gu), D(rows * n_out * 4)
+    assert lib.wr_hip_proj_rows_norm_dev(w.h, rows, xd.p, n_in, nwd.p, eps, None, y.p, n_out) == hipattn.OK
+    normed = oracle.rmsnorm(x, nw, eps)
+    mag = np.abs(normed.astype(np.float64)) @ np.abs(_widen(w16)).T
+    assert np.all(np.abs(y.to_host((rows, n_out)) - oracle.matmul_w16(normed, w16)) <= 1e-6 * np.sqrt(n_in) * mag)
+    assert lib.wr_hip_proj_rows_swiglu_dev(w.h, rows, gud.p, 2 * n_in, None, y.p, n_out) == hipattn.OK
+    act = oracle.silu_mul(np.ascontiguousarray(gu[:, :n_in]), np.ascontiguousarray(gu[:, n_in:]))
+    _check(y.to_host((rows, n_out)), act, w16, f"swiglu {rows} {n_in}")
+    for d in (xd, nwd, gud, y):
+        d.free()
+    w.close()

@@ -26,11 +26,12 @@
 //
 // Kernels, by row count of a launch:
 //   1 row        proj_row1_kernel: the fragment step inside the product;
-//   2 .. 63      proj_prep_kernel, then proj_rows_kernel (a wave owns one to four
-//                16-output tiles for one to four row groups; HBM-bound);
-//   64 .. 4096   proj_prep_group_kernel, then an MFMA-bound GEMM:
-//                proj_gemm_lds_kernel (operands staged through LDS) where its
-//                tiles fill the chip, proj_gemm_split_kernel below that.
+//   2 .. 16      proj_prep_kernel, then proj_rows_kernel (a wave owns one or two
+//                16-output tiles for one or two row groups; HBM-bound);
+//   17 .. 4096   proj_prep_kernel (proj_prep_group_kernel from 257 rows), then a
+//                GEMM: proj_gemm_lds_kernel (operands staged through LDS,
+//                MFMA-bound) where its tiles fill the chip,
+//                proj_gemm_split_kernel below that.
 // N must be a multiple of 16 and K a multiple of 32.
 #pragma once
 
@@ -282,7 +283,7 @@ __global__ __launch_bounds__(256) void proj_prep_kernel(const ProjPrepArgs a)
 // Same sources, expressions and scaling as proj_prep_kernel; the row sums are
 // formed in a different order (each thread over its own chunks, then the 32
 // threads of the row), so a normalised row agrees with the one-row kernel's to
-// rounding, not bit for bit: only launches of 64 rows and more come here.
+// rounding, not bit for bit: only launches of many rows come here.
 //
 // CH > 0: K <= 256 * CH and the row group's values stay in registers between
 // the passes; CH = 0: any K, the passes re-read and re-compute.
@@ -476,9 +477,8 @@ __device__ __forceinline__ void proj_step(f32x4 (&acc)[NT][GROUPS], const half8 
     }
 }
 
-// GROUPS = row groups of eight per wave, NT = 16-output tiles per wave
-// (templates, so the accumulators stay in registers); grid.y walks further
-// runs of GROUPS row groups when a launch carries more rows than that.  A workgroup is four
+// GROUPS = row groups of eight (one or two), NT = 16-output tiles per wave
+// (templates, so the accumulators stay in registers).  A workgroup is four
 // waves.  With ksplit = 1 they own four consecutive runs of 16*NT outputs; with
 // ksplit = 2 or 4 that many waves share a run and take contiguous parts of the
 // input range (a narrow weight then still puts a thousand waves on the chip),
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
 {
     constexpr int KB = kProjKBatch / NT;                               // k-steps per register batch
     // partial sums of the waves with part > 0: (4 / S) runs x (S - 1) parts <= 3 entries
-    __shared__ f32x4 s_part[(GROUPS <= 2) ? 3 * NT * GROUPS * 64 : 1];
+    __shared__ f32x4 s_part[3 * NT * GROUPS * 64];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t S = a.ksplit;
@@ -503,9 +503,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
     const uint32_t ktiles = a.K / 32;
     const uint32_t kper = ktiles / S;                            // host guarantees divisibility
     const uint32_t k_begin = part * kper, k_end = k_begin + kper;
-    // blockIdx.y: which run of GROUPS row groups (prefill-sized row counts only)
-    const uint32_t group0 = blockIdx.y * GROUPS;
-    const half8* xp = a.xfrag + (size_t)group0 * ktiles * 64 + lane;
+    const half8* xp = a.xfrag + lane;
 
     f32x4 acc[NT][GROUPS];
 #pragma unroll
@@ -582,27 +580,25 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
         }
     }
 
-    if constexpr (GROUPS <= 2) {
-        if (S > 1) {                                             // uniform over the workgroup
-            if (part > 0) {
+    if (S > 1) {                                                 // uniform over the workgroup
+        if (part > 0) {
 #pragma unroll
-                for (int t = 0; t < NT; t++)
+            for (int t = 0; t < NT; t++)
 #pragma unroll
-                    for (int gi = 0; gi < GROUPS; gi++)
-                        s_part[(((slot * (S - 1) + (part - 1)) * NT + t) * GROUPS + gi) * 64 + lane] = acc[t][gi];
-            }
-            __syncthreads();
-            if (part > 0) return;
-            for (uint32_t p = 1; p < S; p++) {
+                for (int gi = 0; gi < GROUPS; gi++)
+                    s_part[(((slot * (S - 1) + (part - 1)) * NT + t) * GROUPS + gi) * 64 + lane] = acc[t][gi];
+        }
+        __syncthreads();
+        if (part > 0) return;
+        for (uint32_t p = 1; p < S; p++) {
 #pragma unroll
-                for (int t = 0; t < NT; t++)
+            for (int t = 0; t < NT; t++)
 #pragma unroll
-                    for (int gi = 0; gi < GROUPS; gi++) {
-                        const f32x4 o = s_part[(((slot * (S - 1) + (p - 1)) * NT + t) * GROUPS + gi) * 64 + lane];
+                for (int gi = 0; gi < GROUPS; gi++) {
+                    const f32x4 o = s_part[(((slot * (S - 1) + (p - 1)) * NT + t) * GROUPS + gi) * 64 + lane];
 #pragma unroll
-                        for (int i = 0; i < 4; i++) acc[t][gi][i] += o[i];
-                    }
-            }
+                    for (int i = 0; i < 4; i++) acc[t][gi][i] += o[i];
+                }
         }
     }
     if (!live) return;
@@ -610,7 +606,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int gi = 0; gi < GROUPS; gi++) proj_store_tile(a, acc[t][gi], nt0 + t, group0 + gi, lane);
+        for (int gi = 0; gi < GROUPS; gi++) proj_store_tile(a, acc[t][gi], nt0 + t, gi, lane);
 }
 
 // One row (a decode step): proj_rows_kernel<1, 1> with the fragment kernel
@@ -858,39 +854,50 @@ __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs 
         proj_row1_body<SRC, 0>(a, p, sfrag, s_part, s4, &s_scale);
 }
 
-// Many rows (prefill chunks), products too small to fill the chip with the
-// LDS-staged tiles below: a register-tiled GEMM on the same two layouts.  The
-// four waves of a workgroup share one tile of NT x GROUPS accumulator tiles
-// (16 NT outputs x 8 GROUPS rows) and take a quarter of the input range each;
-// their sums are added through LDS in wave order.  Every k-step loads NT weight
-// tiles and GROUPS operand fragments, one KiB each and both already in operand
-// order, and feeds NT x GROUPS MFMAs; the next k-step's operands are requested
-// while this one's MFMAs run (two register sets, the loop unrolled by two so no
-// set is copied).  Small tiles and the split range put several waves on every
-// SIMD and keep the chains of dependent k-steps short: these products are
-// bound by load latency, not by bytes.  grid.x walks the outputs, so the
-// workgroups the dispatcher deals round-robin to the eight XCDs differ in
-// output tile.  At least three workgroups per CU (<= 168 registers), which
-// also keeps the accumulators in ordinary vector registers.
-template <int GROUPS, int NT>
-__global__ __launch_bounds__(kProjThreads, 3) void proj_gemm_split_kernel(const ProjArgs a)
+// 17 rows and more, products too small to fill the chip with the LDS-staged
+// tiles below: a register-tiled GEMM on the same two layouts.  The four waves of a
+// workgroup share one tile of NT x GROUPS accumulator tiles (16 NT outputs x
+// 8 GROUPS rows) and take a quarter of the input range each; their sums meet in
+// LDS and are added in wave order, each wave adding and storing every fourth tile.
+// Every k-step loads NT weight tiles and GROUPS operand fragments, one KiB each and
+// both already in operand order, and feeds NT x GROUPS MFMAs.  These products are
+// bound by load latency (the weights come from HBM, a few MB, one to three
+// microseconds of it) and, as the rows grow, by the bytes that pass the vector
+// cache, so a wave keeps D k-steps on their way: eight of a small tile are the
+// whole share of a wave at 1024 inputs.  Loads stand behind the MFMAs that free
+// their registers and are issued whether needed or not only in whole turns of D,
+// so the compiler's count of loads in flight is exact.  grid.x walks the outputs,
+// so the workgroups the dispatcher deals round-robin to the eight XCDs differ in
+// output tile.
+//
+// Measured (us, weights from HBM; one k-step ahead, tiles <4, 2>, as this kernel
+// was, against <2, 1, 8> at 20 and 45 rows, <2, 2, 8> at 100 and 200, <4, 2, 4> at 511):
+//   rows            20           45           100          200          511
+//   1024 -> 4096    8.4 / 4.8    8.7 / 5.9    9.8 / 8.4    13.2 / 11.9  (LDS tiles)
+//   2048 -> 1024    8.5 / 4.0    9.0 / 4.2    8.9 / 5.2     9.0 / 7.2   14.6 / 13.8
+//   3072 -> 1024   15.1 / 6.2   15.4 / 7.2   15.3 / 7.9    15.7 / 11.5  20.4 / 19.3
+// (Below 64 rows a kernel of one wave per 64 outputs x 32 rows ran before: 20 us
+// for the first, 51 for the third.)  Eight waves to the input range, or deeper
+// turns on larger tiles, gave nothing.
+template <int GROUPS, int NT, int D>
+__global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_gemm_split_kernel(const ProjArgs a)
 {
-    __shared__ f32x4 s_red[3 * NT * GROUPS * 64];
+    __shared__ f32x4 s_red[4 * NT * GROUPS * 64];
     const int lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t ktiles = a.K / 32, ntiles = a.N / 16, ngroups = (a.R + 7) / 8;
     const uint32_t nt0 = blockIdx.x * NT, group0 = blockIdx.y * GROUPS;
-    const uint32_t k_begin = ktiles * wave / 4, k_end = ktiles * (wave + 1) / 4;
+    const uint32_t k_begin = ktiles * wave / 4, n = ktiles * (wave + 1) / 4 - k_begin;   // (none: a wave adds zeros)
 
     // a tile or group past the end re-reads the last one; its result is dropped
     const half8* wp[NT];
     const half8* xp[GROUPS];
 #pragma unroll
     for (int t = 0; t < NT; t++)
-        wp[t] = a.w + (size_t)min(nt0 + t, ntiles - 1) * ktiles * 64;
+        wp[t] = a.w + ((size_t)min(nt0 + t, ntiles - 1) * ktiles + k_begin) * 64;
 #pragma unroll
     for (int gi = 0; gi < GROUPS; gi++)
-        xp[gi] = a.xfrag + (size_t)min(group0 + gi, ngroups - 1) * ktiles * 64;
+        xp[gi] = a.xfrag + ((size_t)min(group0 + gi, ngroups - 1) * ktiles + k_begin) * 64;
 
     f32x4 acc[NT][GROUPS];
 #pragma unroll
@@ -898,63 +905,57 @@ __global__ __launch_bounds__(kProjThreads, 3) void proj_gemm_split_kernel(const 
 #pragma unroll
         for (int gi = 0; gi < GROUPS; gi++) acc[t][gi] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    half8 w0[NT], x0[GROUPS], w1[NT], x1[GROUPS];
-    auto load_set = [&](half8 (&wv)[NT], half8 (&xv)[GROUPS], uint32_t kt) {
-        const size_t o = (size_t)kt * 64 + lane;
+    half8 w[D][NT], x[D][GROUPS];
+    auto load_set = [&](int d, uint32_t k) {
+        const uint32_t o = k * 64 + lane;
 #pragma unroll
-        for (int t = 0; t < NT; t++) wv[t] = wp[t][o];
+        for (int t = 0; t < NT; t++) w[d][t] = wp[t][o];
 #pragma unroll
-        for (int gi = 0; gi < GROUPS; gi++) xv[gi] = xp[gi][o];
+        for (int gi = 0; gi < GROUPS; gi++) x[d][gi] = xp[gi][o];
     };
-    auto mfma_set = [&](const half8 (&wv)[NT], const half8 (&xv)[GROUPS]) {
+    auto mfma_set = [&](int d) {
 #pragma unroll
         for (int gi = 0; gi < GROUPS; gi++)
 #pragma unroll
             for (int t = 0; t < NT; t++)
-                acc[t][gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[t], xv[gi], acc[t][gi], 0, 0, 0);
+                acc[t][gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[d][t], x[d][gi], acc[t][gi], 0, 0, 0);
     };
-
-    // loads inside the loop are unconditional (a k-step past the end re-reads the
-    // last one, unused), so the load counter the compiler waits on stays exact;
-    // a wave whose part of the range is empty (fewer than four k-steps) adds zeros
-    const uint32_t klast = ktiles - 1;
-    load_set(w0, x0, min(k_begin, klast));
-    uint32_t kt = k_begin;
-    for (; kt + 2 <= k_end; kt += 2) {
-        load_set(w1, x1, kt + 1);
-        mfma_set(w0, x0);
-        load_set(w0, x0, min(kt + 2, klast));
-        mfma_set(w1, x1);
-    }
-    if (kt < k_end) mfma_set(w0, x0);                     // odd number of k-steps
-
-    if (wave > 0) {
+    const uint32_t turns = n / D;
+    if (turns) {
 #pragma unroll
-        for (int t = 0; t < NT; t++)
+        for (int d = 0; d < D; d++) load_set(d, d);
+        for (uint32_t turn = 1; turn < turns; turn++) {
 #pragma unroll
-            for (int gi = 0; gi < GROUPS; gi++)
-                s_red[(((wave - 1) * NT + t) * GROUPS + gi) * 64 + lane] = acc[t][gi];
-    }
-    __syncthreads();
-    if (wave > 0) return;
-    // wave order: 0 + 1 + 2 + 3; a real loop over the waves, so that at most
-    // one wave's partial tiles are in registers beside the accumulators
-#pragma unroll 1
-    for (int p = 0; p < 3; p++) {
-        const f32x4* from = s_red + (size_t)p * NT * GROUPS * 64 + lane;
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int gi = 0; gi < GROUPS; gi++) {
-                const f32x4 o = from[(t * GROUPS + gi) * 64];
-#pragma unroll
-                for (int i = 0; i < 4; i++) acc[t][gi][i] += o[i];
+            for (int d = 0; d < D; d++) {
+                mfma_set(d);
+                load_set(d, turn * D + d);
+                __builtin_amdgcn_sched_barrier(0);
             }
+        }
+#pragma unroll
+        for (int d = 0; d < D; d++) mfma_set(d);
     }
+    for (uint32_t k = turns * D; k < n; k++) {
+        load_set(0, k);
+        mfma_set(0);
+    }
+
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int gi = 0; gi < GROUPS; gi++) proj_store_tile(a, acc[t][gi], nt0 + t, group0 + gi, lane);
+        for (int gi = 0; gi < GROUPS; gi++) s_red[((wave * NT + t) * GROUPS + gi) * 64 + lane] = acc[t][gi];
+    lds_barrier();
+#pragma unroll 1
+    for (uint32_t i = wave; i < NT * GROUPS; i += 4) {
+        f32x4 v = s_red[i * 64 + lane];
+#pragma unroll
+        for (int p = 1; p < 4; p++) {
+            const f32x4 o = s_red[(p * NT * GROUPS + i) * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] += o[j];
+        }
+        proj_store_tile(a, v, nt0 + i / GROUPS, group0 + i % GROUPS, lane);
+    }
 }
 
 // Many rows, products that fill the chip with 128-output x 128-row workgroup

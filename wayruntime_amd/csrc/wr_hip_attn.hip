@@ -750,28 +750,28 @@ Entered::Entered()
 namespace {
 
 template <int GROUPS, int NT>
-void launch_proj(const ProjArgs& a, uint32_t groups)
+void launch_proj(const ProjArgs& a)
 {
     const uint32_t runs = (a.N / 16 + NT - 1) / NT;              // runs of 16*NT outputs
     const uint32_t per_block = 4 / a.ksplit;
-    launch_main(proj_rows_kernel<GROUPS, NT>,
-                dim3((runs + per_block - 1) / per_block, (groups + GROUPS - 1) / GROUPS),
-                dim3(kProjThreads), a);
+    launch_main(proj_rows_kernel<GROUPS, NT>, dim3((runs + per_block - 1) / per_block), dim3(kProjThreads), a);
 }
 
 // Prefill-sized row counts: the largest tile that still fills the chip.
 //   LDS-staged, eight waves, 256 outputs x 128 rows per workgroup, from one workgroup per CU;
 //   LDS-staged, 128 x 128, from two workgroups per CU;
 //   LDS-staged, 128 x 64, from one per CU (software-pipelined: a SIMD may hold a single wave);
-//   registers, 64 x 32, the four waves split the input range;
-//   registers, 32 x 32, likewise.
-constexpr int kProjGemmMinRows = 64;
+//   registers, the four waves split the input range: 16 x 16 (up to 48 rows, weights up to 4096 outputs),
+//   32 x 16 (up to 1024 workgroups of it), 32 x 32.
+constexpr int kProjGemmMinRows = 17;
+constexpr uint32_t kProjGroupRows = 257;           // from here on the fragments are made by row groups: at 200 rows a
+                                                   // workgroup per row is 0.6 to 2.2 us faster, at 300 as fast, at 511 1 us slower
 constexpr size_t kProjRow1MaxLds = 60 * 1024;      // inputs up to 15 360 take the one-row kernel
 
-template <int GROUPS, int NT>
+template <int GROUPS, int NT, int D>
 void launch_proj_gemm_split(const ProjArgs& a, uint32_t groups)
 {
-    launch_main(proj_gemm_split_kernel<GROUPS, NT>,
+    launch_main(proj_gemm_split_kernel<GROUPS, NT, D>,
                 dim3((a.N / 16 + NT - 1) / NT, (groups + GROUPS - 1) / GROUPS), dim3(kProjThreads), a);
 }
 
@@ -820,10 +820,12 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
     else if (panels * ((groups + 7) / 8) >= 256)          // one per CU, one wave per SIMD: pipelined reads
         launch_main(proj_gemm_lds_kernel<4, 2, 4, true>, dim3(share * ((groups + 7) / 8)), dim3(kProjThreads), a,
                     gemm_lds_bytes<4, 2, 4>());
-    else if (((nt + 3) / 4) * ((groups + 3) / 4) >= 384)
-        launch_proj_gemm_split<4, 4>(a, groups);
+    else if (groups <= 6 && nt <= 256)                    // (45 rows, 1024 -> 6144: 7.6 us against 7.4 with the next)
+        launch_proj_gemm_split<2, 1, 8>(a, groups);
+    else if (((nt + 1) / 2) * ((groups + 1) / 2) <= 1024) // (200 rows, 1024 -> 6144: 16.8 against 16.4 with the next)
+        launch_proj_gemm_split<2, 2, 8>(a, groups);
     else
-        launch_proj_gemm_split<4, 2>(a, groups);
+        launch_proj_gemm_split<4, 2, 4>(a, groups);
 }
 
 // What feeds a projection: the rows as they are, their RMS normalisation, or
@@ -839,10 +841,8 @@ struct ProjSource {
 int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev, uint32_t ldx,
                       const ProjSource& src, const float* add_dev, float* y_dev, uint32_t ldy)
 {
-    // row groups of eight, padded to what one wave takes (1, 2, or runs of 4)
-    uint32_t groups = (rows + 7) / 8;
-    const bool gemm = rows >= (uint32_t)kProjGemmMinRows;  // the GEMM kernel clamps instead of padding
-    if (groups > 2 && !gemm) groups = (groups + 3) / 4 * 4;
+    const uint32_t groups = (rows + 7) / 8;                // row groups of eight
+    const bool gemm = rows >= (uint32_t)kProjGemmMinRows;
     const uint32_t ktiles = w->n_in / 32;
     // one row: the fragment step runs inside the product's kernel (4 bytes of LDS per input)
     const bool row1 = rows == 1 && (size_t)w->n_in * 4 <= kProjRow1MaxLds;
@@ -864,7 +864,7 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     const bool in_regs = w->n_in <= 4096;           // two chunks of eight values per thread
     // many rows: a workgroup per row group (whole-line writes); it reads rows
     // with 16-byte loads
-    const bool by_group = gemm && ldx % 4 == 0 && ((uintptr_t)x_dev & 15) == 0 &&
+    const bool by_group = rows >= kProjGroupRows && ldx % 4 == 0 && ((uintptr_t)x_dev & 15) == 0 &&
                           ((uintptr_t)src.norm_w & 15) == 0;
     const uint32_t kin = w->n_in;
 #define WR_LAUNCH_PREP_GROUP(SRC, CH) \
@@ -935,13 +935,11 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     } else if (gemm)
         launch_proj_gemm(a, groups);
     else if (groups == 1)
-        launch_proj<1, 1>(a, groups);
-    else if (groups == 2 && tiles * ksplit >= 2048)
-        launch_proj<2, 2>(a, groups);       // wide weight: two output tiles per operand load
-    else if (groups == 2)
-        launch_proj<2, 1>(a, groups);       // narrow weight: every wave counts
+        launch_proj<1, 1>(a);
+    else if (tiles * ksplit >= 2048)
+        launch_proj<2, 2>(a);               // wide weight: two output tiles per operand load
     else
-        launch_proj<4, 4>(a, groups);       // grid.y = groups / 4
+        launch_proj<2, 1>(a);               // narrow weight: every wave counts
     HIP_TRY(hipGetLastError(), "projection launch", 0);
     return WR_HIP_OK;
 }
