@@ -332,7 +332,7 @@ int wr_hip_mix_latent_attend(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t
  * outputs form that many equal groups of neighbours, and only those of the `keep` groups
  * with the largest choice value in them can be chosen.
  * slot[r][t]: the pair's slot, ~0 for an identity output; perm: row of each slot, or ~0;
- * group_expert: expert of each group of 16 slots, or -1; side[r] (may be NULL): the sum of
+ * group_expert: expert of each group of 16 slots, or -1 where a group holds no pair; side[r] (may be NULL): the sum of
  * the identity outputs' weights, and, with shared_gate, the logistic of the logit behind
  * the outputs' (else 0).
  * slot_weight (may be NULL): the weight of each slot's pair, 0 for an empty slot.
@@ -350,7 +350,7 @@ uint32_t wr_hip_mix_route_groups(uint32_t rows, uint32_t experts, uint32_t top, 
 int wr_hip_mix_route(wr_hip_mix_step *s, const float *z_dev, uint32_t ldz, const wr_hip_mix_router *g,
                      uint32_t tile_groups, float *gate_dev, float *side_dev, float *slot_weight_dev, uint32_t *slot_dev,
                      uint32_t *perm_dev, int32_t *group_expert_dev);
-/* The rows of h in slot order: xs (frag). */
+/* The rows of h in slot order: xs (frag); groups without a pair are left as they are. */
 int wr_hip_mix_route_gather(wr_hip_mix_step *s, int f32, const void *h_dev, uint32_t kt, uint32_t n_groups,
                             const uint32_t *perm_dev, const int32_t *group_expert_dev, void *xs_dev);
 

@@ -705,8 +705,8 @@ int wr_hip_mix_route(wr_hip_mix_step *s, const float *z, uint32_t ldz, const wr_
                 if (slot_weight) slot_weight[at] = gate[i];
                 out[i] = at++;
             }
+        for (uint32_t i = begin / 16; i < (at + 15) / 16; i++) group_expert[i] = (int32_t)e;
         at = (at + run - 1) / run * run;
-        for (uint32_t i = begin / 16; i < at / 16; i++) group_expert[i] = (int32_t)e;
     }
     memcpy(slot, out, (size_t)s->rows * top * 4);
     free(out);

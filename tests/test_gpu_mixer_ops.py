@@ -195,6 +195,51 @@ def test_batch_of_matrices(lib, f32, batch, N, K, rows):
         b.free()
 
 
+# every tile the rule picks among: register tiles of 1 x 1, 1 x 2, 2 x 2, 2 x 3, 2 x 4, 4 x 3, 4 x 4 (outputs x rows,
+# sixteens; gated outputs take even ones), LDS tiles of 64, 128 and 256 rows.  Input ranges that leave waves without
+# k-steps (96) and that split unevenly with a rest behind whole turns (1056).
+@pytest.mark.parametrize("K", [96, 1056])
+@pytest.mark.parametrize("N,rows", [(48, 17), (1088, 50), (1088, 130), (2112, 100), (2816, 100), (2112, 300), (6208, 100),
+                                    (6208, 511), (12352, 511), (12352, 700)])
+def test_every_tile_of_many_rows(lib, N, K, rows):
+    r = Run(lib, False, 1, N, K, rows)
+    x = r.act(rows, K)
+    xd, y = r.up(x), hipattn.DeviceBuffer(rows * N * 4)
+    want = x.astype(np.float64) @ r.w[0].T.astype(np.float64)
+    r.go(xd, out=ROWS_F32, y_f32=y.p, ldy=N)
+    r.close(y.to_host((rows, N)), want)
+    if N % 64 == 0:
+        h = hipattn.DeviceBuffer(-(-rows // 16) * 16 * N)
+        r.go(xd, out=GATED, h=h.p, h_kt=N // 64)
+        t = want.reshape(rows, N // 32, 2, 16)
+        r.close(r.frag_down(h, rows, N // 2), (O.silu(t[:, :, 0]) * t[:, :, 1]).reshape(rows, -1), eight_bits=True)
+        h.free()
+    r.end()
+    for b in (xd, y):
+        b.free()
+
+
+@pytest.mark.parametrize("N,K,runs_each", [(64, 352, 1), (2080, 96, 1), (64, 352, 3), (2080, 96, 3), (1056, 32, 2)])
+def test_runs_whose_last_groups_hold_no_pair(lib, N, K, runs_each):
+    # runs of eight groups per expert, the last one's rest empty, as routing leaves it: few rows an expert and many
+    experts = 3
+    r = Run(lib, False, experts, N, K, 0)
+    which = np.full(8 * experts * runs_each, -1, dtype=np.int32)
+    for e in range(experts):
+        n = 8 * (runs_each - 1) + (1, 4, 7)[e]             # groups that hold pairs
+        which[8 * runs_each * e:8 * runs_each * e + n] = e
+    rows, live = 16 * len(which), np.repeat(which, 16) >= 0
+    x = r.act(rows, K)
+    xd, gd = r.up(x), hipattn.DeviceBuffer.from_host(which.view(np.float32))
+    y = hipattn.DeviceBuffer(rows * N * 4)
+    r.go(xd, rows=rows, group_expert=gd.p, tile_groups=8, out=ROWS_F32, y_f32=y.p, ldy=N)
+    want = np.concatenate([x[16 * g:16 * g + 16].astype(np.float64) @ r.w[e].T.astype(np.float64) for g, e in enumerate(which) if e >= 0])
+    r.close(y.to_host((rows, N))[live], want)
+    r.end()
+    for b in (xd, gd, y):
+        b.free()
+
+
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("N,K,tile", [(64, 96, 1), (48, 64, 8), (4096, 64, 8), (1024, 32, 1)])
 def test_matrix_per_row_group(lib, f32, N, K, tile):

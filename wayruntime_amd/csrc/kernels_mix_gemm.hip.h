@@ -3,12 +3,11 @@
 // the next step wants it: 32-bit or activation-type rows, or directly the
 // fragment of the next product.
 //
-//   mix_gemm_stream_kernel  any row count, both activation types: a workgroup's
-//                           four waves share one run of NT x 16 outputs and GR x 16
-//                           rows and split the input range; weights stream from HBM
-//                           once (decode: HBM-bound on the weight bytes)
-//   mix_gemm_lds_kernel     prompt-sized row counts, bfloat16: 128-output tiles
-//                           staged through LDS (MFMA-bound)
+//   mix_gemm_split_kernel  any row count, both activation types: a workgroup's waves
+//                          share a tile and split the input range (decode: HBM-bound
+//                          on the weight bytes)
+//   mix_gemm_lds_kernel    prompt-sized row counts, bfloat16: 128-output tiles
+//                          staged through LDS (MFMA-bound)
 #pragma once
 
 #include "mix_common.hip.h"
@@ -142,36 +141,46 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
     }
 }
 
-template <bool F32, int NT, int GR>
-__global__ __launch_bounds__(256) void mix_gemm_stream_kernel(const MixGemmArgs a)
+// A workgroup's WAVES waves share NT x 16 outputs and GR x 16 rows and take an equal
+// part of the input range each; their sums meet in LDS and are added in wave order,
+// every wave adding and storing its share of the tiles.  A wave keeps D k-steps on
+// their way (operands from HBM are one to three microseconds away under load):
+// loads stand behind the products that free their registers, and only whole turns
+// of D are loaded ahead, so the compiler's count of loads in flight is exact.
+// Few rows: bound by the weights' bytes.  More rows: by the bytes that pass a
+// compute unit's vector cache, NT + GR KiB a k-step for NT x GR products.
+// STREAM: every weight tile is read by one workgroup only (no use in keeping it).
+// With group_expert the GR groups share an expert (GR divides tile_groups).
+template <bool F32, int NT, int GR, int WAVES, int D, bool STREAM>
+__global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_kernel(const MixGemmArgs a)
 {
     using V8 = typename MixAct<F32>::V8;
-    // k-steps in flight per buffer: about eight KiB of operands
-    constexpr int KB = (F32 ? 4 : 8) / (NT > GR ? NT : GR) > 0 ? (F32 ? 4 : 8) / (NT > GR ? NT : GR) : 1;
-    __shared__ f32x4 s_part[3 * NT * GR * 64];
+    __shared__ f32x4 s_part[WAVES * NT * GR * 64];
     const int lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t nt0 = blockIdx.x * NT, group0 = blockIdx.y * GR, z = blockIdx.z;
     uint32_t mat = z;
-    if (a.group_expert) {                                  // GR == 1
+    if (a.group_expert) {
         const int e = a.group_expert[group0];
         if (e < 0) return;                                 // uniform over the workgroup
         mat = (uint32_t)e;
     }
-    const uint32_t k_begin = a.ktiles * wave / 4, k_end = a.ktiles * (wave + 1) / 4, klast = a.ktiles - 1;
+    const uint32_t k_begin = a.ktiles * wave / WAVES, n = a.ktiles * (wave + 1) / WAVES - k_begin;
 
     const bf16x8* wp[NT];
     const V8* xp[GR];
 #pragma unroll
     for (int t = 0; t < NT; t++)
-        wp[t] = a.w + ((size_t)mat * a.ntiles + min(nt0 + t, a.ntiles - 1)) * a.ktiles * 64 + lane;
+        wp[t] = a.w + (((size_t)mat * a.ntiles + min(nt0 + t, a.ntiles - 1)) * a.ktiles + k_begin) * 64;
 #pragma unroll
     for (int i = 0; i < GR; i++)
-        xp[i] = reinterpret_cast<const V8*>(a.x) + ((size_t)min(group0 + i, a.groups - 1) * a.x_kt + (size_t)z * a.x_kt_z) * 64 + lane;
+        xp[i] = reinterpret_cast<const V8*>(a.x) + ((size_t)min(group0 + i, a.groups - 1) * a.x_kt + (size_t)z * a.x_kt_z + k_begin) * 64;
+    uint32_t x_lane = lane;
     if constexpr (GR == 1) {
         if (a.x_perm) {                                    // rows picked one by one: the operand's lanes fetch their own
             const uint32_t pick = a.x_perm[group0 * 16 + (lane & 15)], row = pick == 0xFFFFFFFFu ? 0 : pick;
-            xp[0] = reinterpret_cast<const V8*>(a.x) + (size_t)(row >> 4) * a.x_kt * 64 + (lane & 48) + (row & 15);
+            xp[0] = reinterpret_cast<const V8*>(a.x) + (size_t)k_begin * 64;
+            x_lane = (row >> 4) * a.x_kt * 64 + (lane & 48) + (row & 15);
         }
     }
 
@@ -181,73 +190,71 @@ __global__ __launch_bounds__(256) void mix_gemm_stream_kernel(const MixGemmArgs 
 #pragma unroll
         for (int i = 0; i < GR; i++) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // loads are unconditional (a k-step past the end re-reads the last one and is
-    // not multiplied), so the batch asked for ahead stays in flight
-    bf16x8 wa[KB][NT], wb[KB][NT];
-    V8 xa[KB][GR], xb[KB][GR];
-    auto load = [&](bf16x8 (&w)[KB][NT], V8 (&x)[KB][GR], uint32_t k0) {
-#pragma unroll
-        for (int u = 0; u < KB; u++) {
-            const size_t k = (size_t)min(k0 + u, klast) * 64;
-#pragma unroll
-            for (int t = 0; t < NT; t++) w[u][t] = __builtin_nontemporal_load(&wp[t][k]);
-#pragma unroll
-            for (int i = 0; i < GR; i++) x[u][i] = xp[i][k];
-        }
-    };
-    auto multiply = [&](const bf16x8 (&w)[KB][NT], const V8 (&x)[KB][GR], uint32_t k0) {
-#pragma unroll
-        for (int u = 0; u < KB; u++) {
-            if (k0 + u < k_end) {                          // uniform
-#pragma unroll
-                for (int i = 0; i < GR; i++)
-#pragma unroll
-                    for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(w[u][t], x[u][i], acc[t][i]);
-            }
-        }
-    };
-    if (k_begin < k_end) {
-        load(wa, xa, k_begin);
-        for (uint32_t kt = k_begin; kt < k_end; kt += 2 * KB) {
-            load(wb, xb, kt + KB);
-            multiply(wa, xa, kt);
-            load(wa, xa, kt + 2 * KB);
-            multiply(wb, xb, kt + KB);
-        }
-    }
-    if (wave > 0) {
+    bf16x8 w[D][NT];
+    V8 x[D][GR];
+    auto load = [&](int d, uint32_t k) {
 #pragma unroll
         for (int t = 0; t < NT; t++)
+            w[d][t] = STREAM ? __builtin_nontemporal_load(&wp[t][k * 64 + lane]) : wp[t][k * 64 + lane];
 #pragma unroll
-            for (int i = 0; i < GR; i++) s_part[(((wave - 1) * NT + t) * GR + i) * 64 + lane] = acc[t][i];
-    }
-    __syncthreads();
-    if (wave > 0) return;
-#pragma unroll 1
-    for (int p = 0; p < 3; p++) {
+        for (int i = 0; i < GR; i++) x[d][i] = xp[i][k * 64 + x_lane];
+    };
+    auto multiply = [&](int d) {
 #pragma unroll
-        for (int t = 0; t < NT; t++)
+        for (int i = 0; i < GR; i++)
 #pragma unroll
-            for (int i = 0; i < GR; i++) {
-                const f32x4 o = s_part[((p * NT + t) * GR + i) * 64 + lane];
+            for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(w[d][t], x[d][i], acc[t][i]);
+    };
+    const uint32_t turns = n / D;
+    if (turns) {
 #pragma unroll
-                for (int j = 0; j < 4; j++) acc[t][i][j] += o[j];
+        for (int d = 0; d < D; d++) load(d, d);
+        for (uint32_t turn = 1; turn < turns; turn++) {
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                multiply(d);
+                load(d, turn * D + d);
+                __builtin_amdgcn_sched_barrier(0);
             }
-    }
-    if (a.out >= kMixOutGated) {
-        if constexpr (NT % 2 == 0) {
-#pragma unroll
-            for (int t = 0; t < NT; t += 2)
-#pragma unroll
-                for (int i = 0; i < GR; i++)
-                    mix_store_tile<F32>(a, acc[t][i], acc[t + 1][i], nt0 + t, group0 + i, z, lane);
         }
-        return;
+#pragma unroll
+        for (int d = 0; d < D; d++) multiply(d);
     }
+    for (uint32_t k = turns * D; k < n; k++) {
+        load(0, k);
+        multiply(0);
+    }
+
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int i = 0; i < GR; i++) mix_store_tile<F32>(a, acc[t][i], acc[t][i], nt0 + t, group0 + i, z, lane);
+        for (int i = 0; i < GR; i++) s_part[((wave * NT + t) * GR + i) * 64 + lane] = acc[t][i];
+    lds_barrier();
+    auto sum = [&](uint32_t i) {
+        f32x4 v = s_part[i * 64 + lane];
+#pragma unroll
+        for (int p = 1; p < WAVES; p++) {
+            const f32x4 o = s_part[(p * NT * GR + i) * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] += o[j];
+        }
+        return v;
+    };
+    if (a.out >= kMixOutGated) {
+        if constexpr (NT % 2 == 0) {
+#pragma unroll 1
+            for (uint32_t u = wave; u < NT / 2 * GR; u += WAVES) {
+                const uint32_t t = u / GR * 2, i = u % GR;
+                mix_store_tile<F32>(a, sum(t * GR + i), sum((t + 1) * GR + i), nt0 + t, group0 + i, z, lane);
+            }
+        }
+        return;
+    }
+#pragma unroll 1
+    for (uint32_t u = wave; u < NT * GR; u += WAVES) {
+        const f32x4 v = sum(u);
+        mix_store_tile<F32>(a, v, v, nt0 + u / GR, group0 + u % GR, z, lane);
+    }
 }
 
 // 2 x 2 waves of 64 outputs x 16 GROUPS rows each: 128 outputs x 32 GROUPS rows a

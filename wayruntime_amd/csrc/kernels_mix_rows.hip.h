@@ -679,7 +679,7 @@ __global__ __launch_bounds__(1024) void mix_order_kernel(const MixRouteArgs a)
     if (lane == 63) wave_sum[wave] = upto;
     __syncthreads();
     for (uint32_t w = 0; w < wave; w++) upto += wave_sum[w];
-    for (uint32_t g = 0; g < mine / 16; g++) a.group_expert[(upto - mine) / 16 + g] = (int32_t)t;
+    for (uint32_t g = 0; g < (count[t] + 15) / 16; g++) a.group_expert[(upto - mine) / 16 + g] = (int32_t)t;   // (a run's empty groups stay -1)
     count[t] = upto - mine;                                // from here on: the expert's next slot
     __syncthreads();
     for (uint32_t i = t; i < pairs; i += 1024) {

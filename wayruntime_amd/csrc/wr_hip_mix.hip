@@ -427,11 +427,11 @@ int wr_hip_mix_shift(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, in
 
 // --------------------------------------------------------------- products --
 
-template <bool F32, int NT, int GR>
-static int launch_stream(const MixGemmArgs& a, uint32_t batch)
+template <bool F32, int NT, int GR, int WAVES, int D, bool STREAM>
+static int launch_split(const MixGemmArgs& a, uint32_t batch)
 {
-    launch_main(mix_gemm_stream_kernel<F32, NT, GR>, dim3((a.ntiles + NT - 1) / NT, (a.groups + GR - 1) / GR, batch),
-                dim3(256), a);
+    launch_main(mix_gemm_split_kernel<F32, NT, GR, WAVES, D, STREAM>,
+                dim3((a.ntiles + NT - 1) / NT, (a.groups + GR - 1) / GR, batch), dim3(WAVES * 64), a);
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
 }
@@ -446,6 +446,48 @@ static int launch_lds(const MixGemmArgs& a, uint32_t batch)
                 mix_gemm_lds_bytes<GROUPS>());
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
+}
+
+// Products of 17 rows and more, bfloat16: the form whose estimate is the least.  A register tile of NT x GR waits for
+// NT + GR KiB a k-step through a compute unit's vector cache, workgroup after workgroup; an LDS tile for its barrier
+// and its operands' latency per k-step, or, with several workgroups on a unit, for its share of the matrix pipes.
+// (Measured on one device, 20 to 1000 rows of 2048 and 4096 inputs and more; microseconds per k-step of 32 inputs:
+// 0.018 for a KiB of the one; 0.34, 0.39, 0.58 and 0.18, 0.27, 0.5 for the three of the other.)  What it changed, us
+// before / now: 2048 -> 2048 at 130 rows 9.2 / 7.2, at 300 13.9 / 9.3, at 1000 23.3 / 17.7; 8192 -> 2048 37.6 / 26.7
+// at 300, 80 / 54 at 1000; 12 288 -> 4096 at 300 111 / 68; 2048 -> 14 400 at 45 27 / 15.3.
+static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
+{
+    struct Form {
+        uint32_t nt, gr;
+        int (*launch)(const MixGemmArgs&, uint32_t);
+    };
+    static const Form split[] = {{1, 1, launch_split<false, 1, 1, 4, 8, false>}, {1, 2, launch_split<false, 1, 2, 4, 8, false>},
+                                 {2, 2, launch_split<false, 2, 2, 4, 8, false>}, {2, 3, launch_split<false, 2, 3, 4, 4, false>},
+                                 {2, 4, launch_split<false, 2, 4, 4, 4, false>}, {4, 3, launch_split<false, 4, 3, 4, 4, false>},
+                                 {4, 4, launch_split<false, 4, 4, 4, 2, false>}};
+    static const struct {
+        uint32_t groups;
+        float step, share;
+        int (*launch)(const MixGemmArgs&, uint32_t);
+    } lds[] = {{4, 0.34f, 0.177f, launch_lds<2>}, {8, 0.39f, 0.27f, launch_lds<4>}, {16, 0.58f, 0.5f, launch_lds<8>}};
+    int (*best)(const MixGemmArgs&, uint32_t) = nullptr;
+    float least = 0.f;
+    auto offer = [&](float cost, int (*launch)(const MixGemmArgs&, uint32_t)) {
+        if (best && cost >= least) return;
+        least = cost;
+        best = launch;
+    };
+    for (const Form& f : split) {
+        if (f.gr > a.groups || (gated && f.nt % 2)) continue;
+        const uint64_t wgs = (uint64_t)((a.ntiles + f.nt - 1) / f.nt) * ((a.groups + f.gr - 1) / f.gr) * batch;
+        offer(0.018f * (float)((wgs + g.n_cus - 1) / g.n_cus) * (f.nt + f.gr), f.launch);
+    }
+    if (a.groups >= 4)
+        for (const auto& f : lds) {
+            const uint64_t wgs = (uint64_t)((a.ntiles + 7) / 8) * ((a.groups + f.groups - 1) / f.groups) * batch;
+            offer(std::max(f.step, f.share * wgs / g.n_cus), f.launch);
+        }
+    return best(a, batch);
 }
 
 int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
@@ -507,30 +549,33 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     a.ya = q->y_act;
     a.h = frag ? static_cast<uint8_t*>(q->h) + (size_t)q->h_kt0 * 512 * (f32 ? 4 : 2) : q->h;
     if (q->group_expert) {
-        if (!f32 && q->tile_groups == 8) return launch_lds<4>(a, 1);
-        if (f32) return gated ? launch_stream<true, 2, 1>(a, 1) : launch_stream<true, 1, 1>(a, 1);
-        return gated ? launch_stream<false, 2, 1>(a, 1) : launch_stream<false, 1, 1>(a, 1);
+        if (!f32 && q->tile_groups == 8) {
+            // Rows an expert has on average, from how many groups a step of that many pairs can take at most.  Up to 64
+            // the product is a stream of the experts' weights (64 experts of 2048 x 1024, 268 MB, 48 rows each: 64 us
+            // against 82 to 89 with the tile of 128 rows, most of them empty).  Above, narrow weights take tiles of 64
+            // rows, which skip the empty halves of runs (64 x (2048 -> 1024), 192 rows each: 115 us against 131; 4096 ->
+            // 2048: 226 against 176).
+            const uint64_t runs = a.groups / 8, e = q->w->batch;
+            const bool few = runs <= e || (runs - e) * 128 <= e * 64;
+            return few ? launch_split<false, 2, 4, 4, 4, true>(a, 1) : a.ntiles <= 64 ? launch_lds<2>(a, 1) : launch_lds<4>(a, 1);
+        }
+        if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 4, true>(a, 1);
+        return launch_split<false, 2, 1, 4, 8, true>(a, 1);
     }
     if (f32) {
-        if (a.groups <= 1) return gated ? launch_stream<true, 2, 1>(a, batch) : launch_stream<true, 1, 1>(a, batch);
-        return launch_stream<true, 2, 2>(a, batch);
+        if (a.groups <= 1) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, batch) : launch_split<true, 1, 1, 4, 4, true>(a, batch);
+        return launch_split<true, 2, 2, 4, 2, false>(a, batch);
     }
-    if (a.groups >= 4) {
-        // the largest tile that still gives every compute unit a workgroup; over a short input range a smaller
-        // one, of which a unit holds three: most of such a launch is its ends
-        const uint64_t panels = (uint64_t)(a.ntiles + 7) / 8 * batch;
-        if (a.ktiles > 16 && panels * ((a.groups + 15) / 16) >= 256) return launch_lds<8>(a, batch);
-        if (panels * ((a.groups + 7) / 8) >= 256) return launch_lds<4>(a, batch);
-        if (panels * ((a.groups + 3) / 4) >= 256) return launch_lds<2>(a, batch);
-        const uint64_t tiles44 = (uint64_t)((a.ntiles + 3) / 4) * ((a.groups + 3) / 4) * batch;
-        if (tiles44 >= 256) return launch_stream<false, 4, 4>(a, batch);
-        if (tiles44 >= 64) return launch_stream<false, 2, 4>(a, batch);
-        return gated ? launch_stream<false, 2, 1>(a, batch) : launch_stream<false, 1, 1>(a, batch);
+    if (a.groups == 1) {
+        // a short input range: more outputs per workgroup, or the launch is all workgroups and no work
+        if (!gated && a.ktiles <= 8 && a.ntiles % 4 == 0 && a.ntiles * batch >= 1024) return launch_split<false, 4, 1, 4, 2, true>(a, batch);
+        // wide weights share the rows' operand between two tiles; over a short range eight waves, over a long one
+        // four with twice the k-steps each (16 rows; us, before / now: 2048 -> 14 400 16.8 / 11.4, -> 32 768
+        // 32.7 / 21.6, 4096 -> 24 576 40.4 / 36.0, -> 6144 13.7 / 11.1; narrow ones 4096 -> 4096 8.4 / 7.8)
+        if (!gated && a.ntiles * batch < 384) return launch_split<false, 1, 1, 4, 8, true>(a, batch);
+        return a.ktiles <= 64 ? launch_split<false, 2, 1, 8, 4, true>(a, batch) : launch_split<false, 2, 1, 4, 8, true>(a, batch);
     }
-    if (a.groups >= 2) return launch_stream<false, 2, 2>(a, batch);
-    // a short input range: more outputs per workgroup, or the launch is all workgroups and no work
-    if (!gated && a.ktiles <= 8 && a.ntiles % 4 == 0 && a.ntiles * batch >= 1024) return launch_stream<false, 4, 1>(a, batch);
-    return gated || a.ntiles * batch >= 4096 ? launch_stream<false, 2, 1>(a, batch) : launch_stream<false, 1, 1>(a, batch);
+    return launch_rows(a, batch, gated);
 }
 
 // -------------------------------------------------------------- lightning --
