@@ -198,9 +198,15 @@ wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *
 /* ---- mixer-stack models (wr_mix.c) ------------------------------------------ */
 wr_status wrh_mix_session_create(wr_model *m, wr_session *s);
 void      wrh_mix_session_destroy(wr_session *s);
+/* Where a step's logits go, host, in the order of the entries and of `want`: rows of a block
+ * [sum of n_want][vocab], or with `rows` a pointer for each. */
+typedef struct wrh_logit_rows {
+    float        *block;
+    float *const *rows;
+} wrh_logit_rows;
 /* The sessions are locked and checked; positions advance on success and nothing
- * changes otherwise.  logits [sum of n_want][vocab], host. */
-wr_status wrh_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, float *logits, int fail_run);
+ * changes otherwise. */
+wr_status wrh_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, const wrh_logit_rows *logits, int fail_run);
 /* Test hook: the residual rows [rows][width] after every layer run of the coming
  * steps are appended to `rows` until `floats` are used up; NULL ends it. */
 void      wrh_debug_capture_residual(wr_model *m, float *rows, size_t floats);

@@ -763,9 +763,11 @@ static wr_status walk_layers(wr_model *m, walk *w, bump b, uint32_t R, int fail_
     return WR_OK;
 }
 
-/* Logits of the step's wanted rows, packed in h's rows after the final norm;
- * row i goes to logits + dest[i] * vocab. */
-static wr_status walk_logits(wr_model *m, const walk *w, uint32_t n_want, const uint32_t *dest, float *logits)
+/* Logits of the step's wanted rows, packed in h's rows after the final norm; row i goes to where `dest[i]` is in
+ * `out`.  The rows come down in one copy per product and are handed out by as many threads as there are rows worth
+ * one (sixteen of 32 768, 2 MB: a step of sixteen sessions 487 -> 441 us, with the copy through a block of the
+ * caller's that it replaces). */
+static wr_status walk_logits(wr_model *m, const walk *w, uint32_t n_want, const uint32_t *dest, const wrh_logit_rows *out)
 {
     struct wrh_mix_model *mm = m->mix;
     const uint32_t r = mm->n_runs, wkt = mm->width_p / 32;
@@ -779,9 +781,13 @@ static wr_status walk_logits(wr_model *m, const walk *w, uint32_t n_want, const 
                                       .y_f32 = mm->logits_dev, .ldy = mm->vocab_p, .scale = mm->logit_scale};
         TRY(wr_hip_mix_gemm_run(mm->f32, &head), "head");
         TRY(wr_hip_attn_d2h(mm->logits_host, mm->logits_dev, (size_t)n * mm->vocab_p * sizeof(float)), "logits down");
-        for (uint32_t i = 0; i < n; i++)
-            memcpy(logits + (size_t)dest[at + i] * m->vocab, mm->logits_host + (size_t)i * mm->vocab_p,
+        const int threads = (m->engine && m->engine->n_threads > 0) ? m->engine->n_threads : 1;
+#pragma omp parallel for num_threads(threads) schedule(static) if (n >= 4 && m->vocab >= 8192)
+        for (uint32_t i = 0; i < n; i++) {
+            const uint32_t d = dest[at + i];
+            memcpy(out->rows ? out->rows[d] : out->block + (size_t)d * m->vocab, mm->logits_host + (size_t)i * mm->vocab_p,
                    (size_t)m->vocab * sizeof(float));
+        }
     }
     return WR_OK;
 }
@@ -817,7 +823,7 @@ static void shrink_pages(struct wrh_mix_model *mm, wrh_mix_session *ms, uint32_t
     while (ms->n_pages > n_pages) mm->free_pages[mm->n_free_pages++] = ms->pages[--ms->n_pages];
 }
 
-wr_status wrh_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, float *logits, int fail_run)
+wr_status wrh_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, const wrh_logit_rows *logits, int fail_run)
 {
     struct wrh_mix_model *mm = m->mix;
     uint32_t done[WR_BATCH_MAX] = {0}, pages_before[WR_BATCH_MAX], longest = 0;

@@ -443,7 +443,8 @@ const float *wr_step(wr_session *s, uint32_t token)
     } else if (m->mix) {
         const uint32_t first = 0;
         const wr_step_entry q = {s, &token, 1, 1, &first};
-        st = wrh_mix_step(m, &q, 1, s->logits, take_fail_layer(m));
+        const wrh_logit_rows to = {s->logits, NULL};
+        st = wrh_mix_step(m, &q, 1, &to, take_fail_layer(m));
     } else {
         wr_session *one[1] = {s};
         if (m->dev) {
@@ -541,7 +542,7 @@ static void sort_by_address(wr_session **a, uint32_t n)
 }
 
 /* Locks the entries' sessions, runs them as one step and publishes the status. */
-static wr_status locked_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, float *logits)
+static wr_status locked_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, const wrh_logit_rows *logits)
 {
     wr_session *locked[WR_BATCH_MAX];
     for (uint32_t i = 0; i < n; i++) locked[i] = entries[i].session;
@@ -559,14 +560,12 @@ static int batch_step_mix(wr_model *m, wr_session *const *sessions, const uint32
     static const uint32_t first = 0;
     wr_step_entry q[WR_BATCH_MAX];
     for (uint32_t i = 0; i < n; i++) q[i] = (wr_step_entry){sessions[i], tokens + i, 1, 1, &first};
-    float *rows = malloc((size_t)n * m->vocab * sizeof *rows);
-    if (!rows) return WR_ERR_NOMEM;
-    const wr_status st = locked_mix_step(m, q, n, rows);
-    for (uint32_t i = 0; i < n && st == WR_OK; i++) {
-        memcpy(sessions[i]->logits, rows + (size_t)i * m->vocab, (size_t)m->vocab * sizeof *rows);
-        if (logits_out) logits_out[i] = sessions[i]->logits;
-    }
-    free(rows);
+    float *rows[WR_BATCH_MAX];
+    for (uint32_t i = 0; i < n; i++) rows[i] = sessions[i]->logits;
+    const wrh_logit_rows to = {NULL, rows};
+    const wr_status st = locked_mix_step(m, q, n, &to);
+    for (uint32_t i = 0; i < n && st == WR_OK; i++)
+        if (logits_out) logits_out[i] = rows[i];
     return (st == WR_OK) ? (int)n : (int)st;
 }
 
@@ -651,7 +650,8 @@ int wr_mixed_step(const wr_step_entry *entries, uint32_t n, float *logits)
     }
     if (wanted && !logits) return WR_ERR_INVAL;
     if (wanted > 0x7FFFFFFFu) return WR_ERR_LIMIT;
-    const wr_status st = m->mix ? locked_mix_step(m, entries, n, logits) : mixed_step_owned(entries, n, logits);
+    const wrh_logit_rows to = {logits, NULL};
+    const wr_status st = m->mix ? locked_mix_step(m, entries, n, &to) : mixed_step_owned(entries, n, logits);
     return (st == WR_OK) ? (int)wanted : (int)st;
 }
 
