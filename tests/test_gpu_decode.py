@@ -607,6 +607,55 @@ def test_append_and_decode_in_one_launch_with_sixteen_short_sessions_paired_spli
             kv.close()
 
 
+@pytest.mark.parametrize("base", [1090, 1500])
+def test_sixteen_sessions_equal_each_alone_with_splits_alone_and_paired(base):
+    # At the Llama shape 16 sessions of 1090 keys are 640 workgroups of one split each
+    # (as many as run at once, 768, would do), of 1500 keys 896, which are paired: two
+    # splits to a workgroup, the last of them the tail that holds the new row.  A
+    # session alone always has a workgroup per split.  Same bits, and the same row in
+    # the cache.
+    import ctypes as C
+    nq, nkv, hd, n = 32, 8, 128, 16
+    lib = hipattn.lib()
+    pos = [base + 5 * i for i in range(n)]
+    width = (nq + 2 * nkv) * hd
+    x = synth.normal(9950, (n, width), std=1.5)
+    xd = hipattn.DeviceBuffer.from_host(x)
+    td = hipattn.DeviceBuffer.from_host(np.concatenate([oracle.rope_table(1, hd, p, 5e5, 0) for p in pos]))
+    sets = []
+    for twin in range(2):
+        kvs = []
+        for i in range(n):
+            _a, _b, k16, v16 = util.make_kv(9900 + 2 * i, pos[i], nkv, hd)
+            kv = hipattn.KVCache(1, hd, nkv, pos[i] + 1)
+            kv.write_f16(0, 0, k16, v16)
+            kvs.append(kv)
+        sets.append(kvs)
+    out = [hipattn.DeviceBuffer.from_host(np.full((n, nq, hd), np.nan, dtype=np.float32)) for _ in range(2)]
+
+    def step(kvs, at, count, to):
+        rc = lib.wr_hip_attn_append_decode_batched_dev(
+            count, (C.c_void_p * count)(*[kv.h for kv in kvs[at:at + count]]), 0,
+            (C.c_uint32 * count)(*pos[at:at + count]), C.c_void_p(xd.p + at * width * 4), width, nq, None, None, 1e-6,
+            C.c_void_p(td.p + at * hd * 4), hd // 2, C.c_void_p(to.p + at * nq * hd * 4), 0.0, 0)
+        assert rc == hipattn.OK
+
+    step(sets[0], 0, n, out[0])
+    for i in range(n):
+        step(sets[1], i, 1, out[1])
+    hipattn.sync()
+    together, alone = out[0].to_host((n, nq, hd)), out[1].to_host((n, nq, hd))
+    assert np.isfinite(together).all() and np.array_equal(together, alone)
+    for i in range(n):
+        ka, va = sets[0][i].read_f16(0, 0, pos[i] + 1)
+        kb, vb = sets[1][i].read_f16(0, 0, pos[i] + 1)
+        assert np.array_equal(ka, kb) and np.array_equal(va, vb), f"cache of session {i}"
+    for b in (xd, td, *out):
+        b.free()
+    for kv in sets[0] + sets[1]:
+        kv.close()
+
+
 def test_append_and_decode_in_one_launch_refuses_what_it_must():
     # argument contract of wr_hip_attn_append_decode_batched_dev: pointers, counts,
     # head shapes and strides are checked before anything is counted or written

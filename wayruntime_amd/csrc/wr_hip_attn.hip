@@ -317,12 +317,11 @@ int decode_locked(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32
     (void)tiles_total;
     uint32_t max_splits = 1;
     const uint32_t tune = g.tune_keys_per_wg.load(std::memory_order_relaxed);
-    bool pairs[kBatchMax];
-    uint32_t wgs_paired = 0;
+    bool pairs[kBatchMax], shorts[kBatchMax];
+    uint32_t wgs_paired = 0, wgs_shorts_alone = 0;
     for (uint32_t i = 0; i < n; i++) {
         uint32_t tpw, tail = 0;
-        pairs[i] = false;
-        bool short_pairs = false;
+        pairs[i] = shorts[i] = false;
         if (tune) {
             tpw = tune / kTileKeys;
             if (tpw == 0) tpw = 1;
@@ -344,11 +343,10 @@ int decode_locked(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32
                 // appended the row itself pays for the extra split instead: one
                 // session of 1024 keys 7.8 -> 8.2 us, of 2048 keys 8.1 -> 8.8 us.
                 if (tiles[i] >= 6) tail = 4;
-                // In a launch that fills the device two consecutive splits of a short
-                // session share a workgroup as well (the splits keep their size):
-                // the ragged batch of 16 has 816 workgroups for 768 places otherwise,
-                // 33.5 -> 32.8 us; sixteen sessions of ~500 keys unchanged.
-                short_pairs = use_mfma && hd <= 128;
+                // In a launch that would not find a place for every split at once two
+                // consecutive splits of a short session share a workgroup as well (the
+                // splits keep their size): see below.
+                shorts[i] = use_mfma && hd <= 128;
             } else if (tiles[i] < 4 * cap) {
                 cap = cap >= 2 ? cap / 2 : 1;                           // a medium one: see above
             } else if (cap <= tiles[i] / 8) {
@@ -359,7 +357,7 @@ int decode_locked(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32
             const uint32_t want = (body + cap - 1) / cap;              // workgroups
             tpw = (body + want - 1) / want;                            // even share
             if (pairs[i]) tpw = (tpw + 1) / 2;                         // two splits per workgroup
-            if (short_pairs) pairs[i] = true;
+            if (shorts[i]) pairs[i] = true;
         }
         const uint32_t body = tiles[i] - tail;
         const uint32_t room = kMaxSplits - (tail ? 1u : 0u);
@@ -370,13 +368,23 @@ int decode_locked(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32
         a.s[i].parts_per_wg = 1;
         a.s[i].n_splits = (body + tpw - 1) / tpw + (tail ? 1u : 0u);
         if (a.s[i].n_splits > max_splits) max_splits = a.s[i].n_splits;
-        wgs_paired += pairs[i] ? (a.s[i].n_splits + 1) / 2 : a.s[i].n_splits;
+        const uint32_t halves = (a.s[i].n_splits + 1) / 2;
+        wgs_paired += pairs[i] ? halves : a.s[i].n_splits;
+        wgs_shorts_alone += pairs[i] && !shorts[i] ? halves : a.s[i].n_splits;
     }
-    // (the launch as a whole decides this, not the session: it changes which
-    // workgroup does a split, never the split)
+    // The launch as a whole decides this, not the session: it changes which
+    // workgroup does a split, never the split.  Splits of short sessions keep a
+    // workgroup each as long as all of the launch's workgroups run at once (three per
+    // CU): a split alone has its tiles in flight from the start and one merge behind
+    // them, and half the places standing empty is the larger loss (sixteen sessions of
+    // 100 .. 1500 keys, 36 entries against 65 per KV head: 18.0 -> 16.8 us; the ragged
+    // batch of 16, 736 workgroups, 27.6 -> 26.8).  Beyond that a second round of
+    // workgroups costs more than the pairing (a batch of 816 entries: 33.5 us alone,
+    // 32.8 paired).
+    const bool shorts_pair = (uint64_t)wgs_shorts_alone * nkv > (uint64_t)g.n_cus * 3;
     if ((uint64_t)wgs_paired * nkv >= g.n_cus)
         for (uint32_t i = 0; i < n; i++)
-            if (pairs[i]) a.s[i].parts_per_wg = 2;
+            if (pairs[i] && (!shorts[i] || shorts_pair)) a.s[i].parts_per_wg = 2;
     // work list, longest entries first (ties keep session, split order)
     {
         uint32_t len[kBatchMax * kMaxSplits];
