@@ -364,7 +364,9 @@ def test_projection_random_shapes():
 
 @pytest.mark.parametrize("rows,n_in,n_out", [
     (17, 1024, 4096),             # register GEMM of 16 x 16 tiles: the fewest rows, a whole share in one turn of eight
-    (48, 2080, 16),               # ... the most, 65 input tiles (a wave with one more than the others), one output tile
+    (48, 2080, 1392),             # ... the most, 65 input tiles (a wave with one more than the others), 522 tiles of 16 x 8
+    (48, 2080, 16),               # 16 x 8 tiles: one output tile
+    (17, 1056, 2720),             # ... 510 of them, the last row group of one row
     (31, 32, 48),                 # ... a single input tile: three waves with none
     (49, 1056, 4112),             # 32 x 16 tiles: a last row group of one row, partial output tiles
     (256, 3072, 80),              # ... the last row count whose fragments are made row by row

@@ -26,8 +26,9 @@
 //
 // Kernels, by row count of a launch:
 //   1 row        proj_row1_kernel: the fragment step inside the product;
-//   2 .. 16      proj_prep_kernel, then proj_rows_kernel (a wave owns one or two
-//                16-output tiles for one or two row groups; HBM-bound);
+//   2 .. 16      proj_prep_kernel, then proj_gemm_split_kernel<1, 1, 8> where four
+//                waves share a tile's inputs, proj_rows_kernel (a wave owns one or two
+//                16-output tiles for one or two row groups; HBM-bound) elsewhere;
 //   17 .. 4096   proj_prep_kernel (proj_prep_group_kernel from 257 rows), then a
 //                GEMM: proj_gemm_lds_kernel (operands staged through LDS,
 //                MFMA-bound) where its tiles fill the chip,
@@ -854,8 +855,8 @@ __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs 
         proj_row1_body<SRC, 0>(a, p, sfrag, s_part, s4, &s_scale);
 }
 
-// 17 rows and more, products too small to fill the chip with the LDS-staged
-// tiles below: a register-tiled GEMM on the same two layouts.  The four waves of a
+// Products too small to fill the chip with the LDS-staged tiles below, from two
+// rows on: a register-tiled GEMM on the same two layouts.  The four waves of a
 // workgroup share one tile of NT x GROUPS accumulator tiles (16 NT outputs x
 // 8 GROUPS rows) and take a quarter of the input range each; their sums meet in
 // LDS and are added in wave order, each wave adding and storing every fourth tile.
@@ -871,13 +872,13 @@ __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs 
 // output tile.
 //
 // Measured (us, weights from HBM; one k-step ahead, tiles <4, 2>, as this kernel
-// was, against <2, 1, 8> at 20 and 45 rows, <2, 2, 8> at 100 and 200, <4, 2, 4> at 511):
+// was, against <2, 1, 8> (<1, 1, 8> for 1024 outputs) at 20 and 45 rows, <2, 2, 8> at
+// 100 and 200, <4, 2, 4> at 511):
 //   rows            20           45           100          200          511
-//   1024 -> 4096    8.4 / 4.8    8.7 / 5.9    9.8 / 8.4    13.2 / 11.9  (LDS tiles)
-//   2048 -> 1024    8.5 / 4.0    9.0 / 4.2    8.9 / 5.2     9.0 / 7.2   14.6 / 13.8
-//   3072 -> 1024   15.1 / 6.2   15.4 / 7.2   15.3 / 7.9    15.7 / 11.5  20.4 / 19.3
+//   1024 -> 4096    8.4 / 4.8    8.7 / 6.0    9.8 / 8.5    13.2 / 12.2  (LDS tiles)
+//   3072 -> 1024   15.1 / 5.5   15.4 / 6.7   15.3 / 8.0    15.7 / 11.5  20.4 / 19.3
 // (Below 64 rows a kernel of one wave per 64 outputs x 32 rows ran before: 20 us
-// for the first, 51 for the third.)  Eight waves to the input range, or deeper
+// for the first, 51 for the second.)  Eight waves to the input range, or deeper
 // turns on larger tiles, gave nothing.
 template <int GROUPS, int NT, int D>
 __global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_gemm_split_kernel(const ProjArgs a)

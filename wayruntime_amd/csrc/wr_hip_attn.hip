@@ -769,7 +769,8 @@ void launch_proj(const ProjArgs& a)
 //   LDS-staged, eight waves, 256 outputs x 128 rows per workgroup, from one workgroup per CU;
 //   LDS-staged, 128 x 128, from two workgroups per CU;
 //   LDS-staged, 128 x 64, from one per CU (software-pipelined: a SIMD may hold a single wave);
-//   registers, the four waves split the input range: 16 x 16 (up to 48 rows, weights up to 4096 outputs),
+//   registers, the four waves split the input range: 16 x 8 (up to two workgroups of it per CU),
+//   16 x 16 (up to 48 rows, weights up to 4096 outputs),
 //   32 x 16 (up to 1024 workgroups of it), 32 x 32.
 constexpr int kProjGemmMinRows = 17;
 constexpr uint32_t kProjGroupRows = 257;           // from here on the fragments are made by row groups: at 200 rows a
@@ -828,6 +829,8 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
     else if (panels * ((groups + 7) / 8) >= 256)          // one per CU, one wave per SIMD: pipelined reads
         launch_main(proj_gemm_lds_kernel<4, 2, 4, true>, dim3(share * ((groups + 7) / 8)), dim3(kProjThreads), a,
                     gemm_lds_bytes<4, 2, 4>());
+    else if (nt * groups <= 512)                          // (64 rows, 2048 -> 1024: 5.4 us against 5.6 with the next)
+        launch_proj_gemm_split<1, 1, 8>(a, groups);
     else if (groups <= 6 && nt <= 256)                    // (45 rows, 1024 -> 6144: 7.6 us against 7.4 with the next)
         launch_proj_gemm_split<2, 1, 8>(a, groups);
     else if (((nt + 1) / 2) * ((groups + 1) / 2) <= 1024) // (200 rows, 1024 -> 6144: 16.8 against 16.4 with the next)
@@ -942,6 +945,14 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
             launch_main(proj_row1_kernel<kProjSrcPlain>, grid, block, a, pa, lds);
     } else if (gemm)
         launch_proj_gemm(a, groups);
+    else if (ksplit == 4)
+        // A workgroup per tile and group of eight rows, four waves to the input range: the
+        // same parts in the same order as below, so the same bits.  For 9 .. 16 rows the
+        // weights pass L2 twice, but a workgroup reads half the operand fragments, which
+        // at 16 rows are twice the weights' bytes: 16 rows, weights from HBM, 1024 -> 4096
+        // 4.7 -> 4.2 us, 2048 -> 1024 5.3 -> 4.3, 1024 -> 6144 6.0 -> 5.4, 3072 -> 1024
+        // 7.0 -> 5.5 (4 rows: 4.2 -> 3.7, 4.4, 5.2 -> 4.9, 5.9 -> 5.6).
+        launch_proj_gemm_split<1, 1, 8>(a, groups);
     else if (groups == 1)
         launch_proj<1, 1>(a);
     else if (tiles * ksplit >= 2048)
