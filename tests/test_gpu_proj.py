@@ -369,7 +369,8 @@ def test_projection_random_shapes():
     (17, 1056, 2720),             # ... 510 of them, the last row group of one row
     (31, 32, 48),                 # ... a single input tile: three waves with none
     (49, 1056, 4112),             # 32 x 16 tiles: a last row group of one row, partial output tiles
-    (256, 3072, 80),              # ... the last row count whose fragments are made row by row
+    (256, 3104, 80),              # ... the last row count whose fragments are made row by row
+    (256, 3072, 80),              # (each workgroup makes its own)
     (257, 288, 1040),             # ... by row groups
     (250, 1056, 4112),            # 32 x 32 tiles, 33 input tiles
 ])
@@ -399,5 +400,58 @@ def test_normed_and_gated_rows_by_rows_and_by_groups(rows, n_in):
     act = oracle.silu_mul(np.ascontiguousarray(gu[:, :n_in]), np.ascontiguousarray(gu[:, n_in:]))
     _check(y.to_host((rows, n_out)), act, w16, f"swiglu {rows} {n_in}")
     for d in (xd, nwd, gud, y):
+        d.free()
+    w.close()
+
+
+@pytest.mark.parametrize("rows,n_in,n_out", [
+    (2, 512, 16), (16, 512, 8176),                   # one tile; three tiles a workgroup, 511 of them
+    (8, 1024, 16368), (16, 1024, 4112),              # four, 1023 of them; three, 257
+    (9, 1536, 4112), (5, 1536, 8192),                # two tiles a workgroup, the last with one; the most for it
+    (16, 2048, 2064), (11, 2560, 48), (16, 3072, 1024), (9, 1024, 1024),
+    (17, 1024, 4096), (41, 2048, 656),               # more than a decode step's rows: the last group of one row
+])
+def test_rows_whose_workgroups_make_their_own_terms(rows, n_in, n_out):
+    # Every row has the bits of the row alone (up to sixteen of them) and of the same
+    # rows on an address that only the separate fragment launch takes, plain and
+    # normalised, with a residual.  Row 1 is zero, a row holds magnitudes down to
+    # where either term rounds away, one an infinity and one a NaN.
+    print("own terms", rows, n_in, n_out, flush=True)
+    lib, D, eps = hipattn.lib(), hipattn.DeviceBuffer, 1e-6
+    x = synth.normal(211 + n_in, (rows, n_in), std=2.0)
+    x[1] = 0.0
+    x[0, 7::5] *= np.float32(2.0) ** -np.arange(len(x[0, 7::5]), dtype=np.float32).clip(0, 60)
+    if rows > 4:
+        x[3, 11], x[4, n_in - 1] = np.inf, np.nan
+    nw, w16 = synth.normal(212, (n_in,)) * np.float32(0.2) + np.float32(1.0), _w16(213, n_out, n_in, 0.1)
+    add = synth.normal(214, (rows, n_out))
+    w, xd, nwd, addd = hipattn.Weight([w16]), D.from_host(x), D.from_host(nw), D.from_host(add)
+    off = D.from_host(np.concatenate([np.zeros(1, np.float32), x.ravel()]))
+    y, ya, y1 = D(rows * n_out * 4), D(rows * n_out * 4), D(n_out * 4)
+
+    def run(norm, n, xp, addp, yp):
+        if norm:
+            return lib.wr_hip_proj_rows_norm_dev(w.h, n, xp, n_in, nwd.p, eps, addp, yp, n_out)
+        return lib.wr_hip_proj_rows_dev(w.h, n, xp, n_in, addp, yp, n_out)
+
+    finite = [i for i in range(rows) if np.isfinite(x[i]).all()]
+    for norm in (False, True):
+        assert run(norm, rows, xd.p, addd.p, y.p) == hipattn.OK
+        assert run(norm, rows, off.p + 4, addd.p, ya.p) == hipattn.OK
+        got, apart = y.to_host((rows, n_out)), ya.to_host((rows, n_out))
+        assert got.tobytes() == apart.tobytes(), f"norm {norm}: not the bits of the separate fragments"
+        src = oracle.rmsnorm(x, nw, eps) if norm else x
+        want = oracle.matmul_w16(src, w16) + add
+        mag = np.abs(src.astype(np.float64)) @ np.abs(_widen(w16)).T + np.abs(add)
+        assert np.all(np.abs(got - want)[finite] <= 1e-6 * np.sqrt(n_in) * mag[finite])
+        for i in range(min(rows, 16) if rows <= 16 else 0):
+            assert run(norm, 1, xd.p + i * n_in * 4, addd.p + i * n_out * 4, y1.p) == hipattn.OK
+            assert got[i].tobytes() == y1.to_host((n_out,)).tobytes(), f"norm {norm} row {i}"
+    if n_in == n_out:
+        assert run(False, rows, xd.p, None, ya.p) == hipattn.OK
+        apart = ya.to_host((rows, n_out))
+        assert run(False, rows, xd.p, None, xd.p) == hipattn.OK
+        assert xd.to_host((rows, n_out)).tobytes() == apart.tobytes()
+    for d in (xd, nwd, addd, off, y, ya, y1):
         d.free()
     w.close()

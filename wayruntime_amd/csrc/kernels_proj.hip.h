@@ -433,12 +433,8 @@ struct ProjArgs {
 // of column c; column c (< 8) is the hi term of row c of the group, column c + 8
 // its lo term.  The two are combined, the row's scale undone, the optional
 // residual added.  Tiles past N and rows past R are dropped.
-__device__ __forceinline__ void proj_store_tile(const ProjArgs& a, f32x4 v, uint32_t nt, uint32_t group,
-                                                int lane, const float* scales = nullptr,
-                                                const f32x4* residual = nullptr)
+__device__ __forceinline__ f32x4 proj_join_terms(f32x4 v)
 {
-    if (!scales) scales = a.scales;
-    const int c = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         // the lo column of row c is eight lanes on in the same row of sixteen: a
@@ -447,9 +443,18 @@ __device__ __forceinline__ void proj_store_tile(const ProjArgs& a, f32x4 v, uint
             __builtin_amdgcn_update_dpp(0, __float_as_int(v[i]), 0x128, 0xF, 0xF, false));
         v[i] += other * (1.0f / kProjLoScale);      // meaningful in the hi columns only
     }
+    return v;
+}
+
+__device__ __forceinline__ void proj_store_tile(const ProjArgs& a, f32x4 v, uint32_t nt, uint32_t group,
+                                                int lane, const float* scale = nullptr,
+                                                const f32x4* residual = nullptr)
+{
+    const int c = lane & 15, g = lane >> 4;
+    v = proj_join_terms(v);
     const uint32_t row = group * 8 + (c & 7);
     if (c < 8 && row < a.R && nt < a.N / 16) {
-        const float sc = scales[row];
+        const float sc = scale ? *scale : a.scales[row];
         const size_t o = (size_t)row * a.ldy + nt * 16 + g * 4;
         f32x4 r;
 #pragma unroll
@@ -853,6 +858,170 @@ __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs 
         proj_row1_body<SRC, 1>(a, p, sfrag, s_part, s4, &s_scale);
     else
         proj_row1_body<SRC, 0>(a, p, sfrag, s_part, s4, &s_scale);
+}
+
+// Two rows to a few dozen, inputs of 512 D / 4: the fragment step inside the product.
+// A batched decode step is a chain of short launches, and of its nine per layer four
+// only wrote fragments (4.6 us each, 16 workgroups).  Here a workgroup, NT tiles of 16
+// outputs by a row group, makes the fragments of its eight rows itself: every wave
+// those of its own quarter of the inputs, in LDS nobody else reads, while its whole
+// share of the weights is on the way (D x NT KiB in registers).  The rows are asked
+// for first (a wave's loads come back in order).  Bound by latency, and by the vector
+// ALU time of the terms, which is the same however many outputs a workgroup has: the
+// host gives a CU one workgroup.  Values, scale, the order of the norm's sum and the
+// order of the product's are those of proj_prep_kernel and of the kernels that share a
+// tile's inputs between four waves, so the result has the same bits.
+//
+// 16 rows, weights from HBM, against proj_prep_kernel + proj_gemm_split_kernel<1, 1, 8>
+// (us): norm + 1024 -> 4096 8.1 -> 5.2, norm + 1024 -> 6144 9.3 -> 6.2, 2048 -> 1024
+// 7.7 -> 5.5, 3072 -> 1024 9.5 -> 7.8; 32 rows of the third 7.8 -> 5.5.  (A lane making
+// the terms of four inputs of its own operand column and trading them with the lane
+// eight on, no LDS: 5.7, 6.7, 5.8, 8.1.)
+template <int SRC, int D, int NT>
+__global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const ProjArgs a, const ProjPrepArgs p)
+{
+    static_assert(D % 2 == 0 && (SRC == kProjSrcPlain || (SRC == kProjSrcRmsNorm && D <= 16)), "sources held in registers");
+    constexpr bool NORM = SRC == kProjSrcRmsNorm;
+    constexpr int KT = 4 * D;                                    // k-steps of a row
+    constexpr int CH = D / 2;                                    // chunks of eight inputs per lane
+    extern __shared__ __attribute__((aligned(16))) unsigned char fused_smem[];
+    // sums of squares of the chunks, by row, chunk of a k-step and k-step
+    __shared__ __attribute__((aligned(16))) float s_ss[NORM ? 8 : 1][NORM ? 4 : 1][NORM ? KT + 4 : 1];
+    __shared__ float s_mx[4][8];
+    __shared__ f32x4 s_red[3 * NT * 64];
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t ntiles = a.N / 16, nt0 = blockIdx.x * NT, group = blockIdx.y;
+    const uint32_t k0 = wave * D;                                // this wave's quarter of the k-steps
+    half8* frag = reinterpret_cast<half8*>(fused_smem) + k0 * 64;
+
+    // 1. the rows, what goes with them, then the weights, all at once.  A lane takes chunk lane / 8 of every two k-steps
+    // of row lane % 8: eight lanes read 256 bytes of a row.  (A row past the end re-reads the last; its columns are dropped.)
+    const uint32_t r = lane & 7, q = lane >> 3;
+    const uint32_t at = k0 * 32 + q * 8;
+    const float* xr = p.x + (size_t)min(group * 8 + r, a.R - 1) * p.ldx + at;
+    f32x4 x[CH][2], nw[NORM ? CH : 1][2];
+#pragma unroll
+    for (int i = 0; i < CH; i++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            x[i][h] = *reinterpret_cast<const f32x4*>(xr + i * 64 + h * 4);
+            if constexpr (NORM) nw[i][h] = *reinterpret_cast<const f32x4*>(p.norm_w + at + i * 64 + h * 4);
+        }
+    f32x4 resid[NT];
+    half8 w[D][NT];
+    const half8* wp[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const uint32_t tile = min(nt0 + t, ntiles - 1);          // (one past the end: dropped)
+        const uint32_t row = min(group * 8 + (lane & 7), a.R - 1);
+        resid[t] = *reinterpret_cast<const f32x4*>(
+            a.bias_rows ? a.bias_rows + (size_t)row * a.ldy + tile * 16 + (lane >> 4) * 4 : xr);
+        wp[t] = a.w + ((size_t)tile * KT + k0) * 64;
+    }
+#pragma unroll
+    for (int u = 0; u < D; u++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) w[u][t] = wp[t][u * 64 + lane];
+
+    // 2. the rows' norms: every chunk of eight summed in order, the chunks by the tree of block_sum_256
+    if constexpr (NORM) {
+#pragma unroll
+        for (int i = 0; i < CH; i++) {
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) ss = fmaf(x[i][j / 4][j % 4], x[i][j / 4][j % 4], ss);
+            s_ss[r][q & 3][k0 + 2 * i + (q >> 2)] = ss;
+        }
+        lds_barrier();
+        // of 64 chunks = 16 k-steps: bits 5 .. 2 of a chunk's number are the k-step's, added in registers; bits 1 and 0
+        // the chunk of the k-step, which lanes 8 r' + r hold (q & 3 here, so that the lanes 16 and 8 on have the others)
+        float part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < (KT + 15) / 16; j++) {
+            float v[16];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                f32x4 four = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (16 * j + 4 * i < KT) four = *reinterpret_cast<const f32x4*>(&s_ss[r][q & 3][16 * j + 4 * i]);
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[4 * i + e] = four[e];
+            }
+#pragma unroll
+            for (int half = 8; half >= 1; half /= 2)
+#pragma unroll
+                for (int i = 0; i < half; i++) v[i] += v[i + half];
+            v[0] += wave_xor_f32(v[0], 16);
+            part[j] = v[0] + wave_xor_f32(v[0], 8);
+        }
+        const float inv_rms = 1.0f / sqrtf(((part[0] + part[1]) + (part[2] + part[3])) / (float)a.K + p.eps);
+#pragma unroll
+        for (int i = 0; i < CH; i++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[i][j / 4][j % 4] = x[i][j / 4][j % 4] * inv_rms * nw[i][j / 4][j % 4];
+    }
+
+    // 3. the rows' scales
+    float mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < CH; i++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) mx = fmaxf(mx, fabsf(x[i][j / 4][j % 4]));
+    mx = fmaxf(mx, wave_xor_f32(mx, 8));
+    mx = fmaxf(mx, wave_xor_f32(mx, 16));
+    mx = fmaxf(mx, wave_xor_f32(mx, 32));
+    if (lane < 8) s_mx[wave][lane] = mx;
+    lds_barrier();
+    mx = fmaxf(fmaxf(s_mx[0][r], s_mx[1][r]), fmaxf(s_mx[2][r], s_mx[3][r]));
+    uint32_t ex = (__float_as_uint(mx) >> 23) & 0xFFu;
+    if (ex == 0 || ex == 0xFF) ex = 127;
+    if (ex > 253) ex = 253;
+    const float scale = __uint_as_float(ex << 23), inv = __uint_as_float((254u - ex) << 23);
+
+    // 4. the terms, into this wave's own fragments (no barrier: a wave's LDS accesses stay in order), and the product
+    f32x4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+        half8 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            // (proj_write_chunk's terms in fewer instructions: (s - h) 2^11 and s 2^11 - h 2^11 are both exact)
+            const float sv = x[i][j / 4][j % 4] * inv;
+            _Float16 h = (_Float16)sv;
+            if (__builtin_fabsf16(h) < (_Float16)6.103515625e-05f) h = (_Float16)0.0f;      // 2^-14
+            hi[j] = h;
+            lo[j] = (_Float16)fmaf((float)h, -kProjLoScale, sv * kProjLoScale);
+        }
+        half8* to = frag + (2 * i + (q >> 2)) * 64 + 16 * (q & 3) + r;
+        to[0] = hi;
+        to[8] = lo;
+    }
+#pragma unroll
+    for (int u = 0; u < D; u++) {
+        const half8 xb = frag[u * 64 + lane];
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[u][t], xb, acc[t], 0, 0, 0);
+    }
+
+    // 5. the waves' parts, in order
+    if (wave > 0) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) s_red[((wave - 1) * NT + t) * 64 + lane] = acc[t];
+    }
+    lds_barrier();
+    if (wave > 0) return;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+#pragma unroll
+        for (int part = 0; part < 3; part++) {
+            const f32x4 other = s_red[(part * NT + t) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[t][i] += other[i];
+        }
+        proj_store_tile(a, acc[t], nt0 + t, group, lane, &scale, &resid[t]);
+    }
 }
 
 // Products too small to fill the chip with the LDS-staged tiles below, from two

@@ -839,6 +839,49 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
         launch_proj_gemm_split<4, 2, 4>(a, groups);
 }
 
+// proj_rows_fused_kernel<SRC, n_in / 128, nt>, or nullptr where none is built.
+using FusedKernel = void (*)(const ProjArgs, const ProjPrepArgs);
+
+template <int SRC, int D>
+FusedKernel fused_of(uint32_t nt)
+{
+    if (nt == 1) return proj_rows_fused_kernel<SRC, D, 1>;
+    if constexpr (D <= 16)
+        if (nt == 2) return proj_rows_fused_kernel<SRC, D, 2>;
+    if constexpr (D <= 8) {
+        if (nt == 3) return proj_rows_fused_kernel<SRC, D, 3>;
+        if (nt == 4) return proj_rows_fused_kernel<SRC, D, 4>;
+    }
+    return nullptr;
+}
+
+FusedKernel fused_kernel(int src, uint32_t n_in, uint32_t nt)
+{
+    const bool norm = src == kProjSrcRmsNorm;
+    if (!norm && src != kProjSrcPlain) return nullptr;
+    switch (n_in) {
+    case 512: return norm ? fused_of<kProjSrcRmsNorm, 4>(nt) : fused_of<kProjSrcPlain, 4>(nt);
+    case 1024: return norm ? fused_of<kProjSrcRmsNorm, 8>(nt) : fused_of<kProjSrcPlain, 8>(nt);
+    case 1536: return norm ? fused_of<kProjSrcRmsNorm, 12>(nt) : fused_of<kProjSrcPlain, 12>(nt);
+    case 2048: return norm ? fused_of<kProjSrcRmsNorm, 16>(nt) : fused_of<kProjSrcPlain, 16>(nt);
+    case 2560: return norm ? nullptr : fused_of<kProjSrcPlain, 20>(nt);
+    case 3072: return norm ? nullptr : fused_of<kProjSrcPlain, 24>(nt);
+    default: return nullptr;
+    }
+}
+
+// The kernel that makes its own operand fragments, and its tiles per workgroup: the
+// fewest with which the launch is one workgroup per CU at most.  A second workgroup on
+// a CU would make the same rows' terms again, and that is vector-ALU time nothing
+// hides: 16 rows, norm + 1024 -> 4096, one / two / three / four tiles (512 / 256 / 172 /
+// 128 workgroups) 6.7 / 5.2 / 5.9 / 6.5 us; -> 6144 8.6 / 7.8 / 6.2 / 6.8.
+FusedKernel pick_fused(int src, uint32_t n_in, uint32_t tiles, uint32_t groups, uint32_t* nt)
+{
+    for (*nt = 1; *nt <= 4; ++*nt)
+        if ((tiles + *nt - 1) / *nt * groups <= (uint32_t)g.n_cus) return fused_kernel(src, n_in, *nt);
+    return nullptr;
+}
+
 // What feeds a projection: the rows as they are, their RMS normalisation, or
 // the gated activation of rows that hold gate and up values side by side.
 struct ProjSource {
@@ -857,6 +900,30 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     const uint32_t ktiles = w->n_in / 32;
     // one row: the fragment step runs inside the product's kernel (4 bytes of LDS per input)
     const bool row1 = rows == 1 && (size_t)w->n_in * 4 <= kProjRow1MaxLds;
+    // Waves that share a run of outputs (contiguous parts of the inputs, summed
+    // through LDS in a fixed order): enough that a narrow weight still gives
+    // one to two thousand waves.  A function of the weight's shape only: a row's
+    // sums are then split the same way whether it travels alone or with up to
+    // fifteen others, so a batched step's rows equal the serial steps' bit
+    // for bit (reference contract: src/core/batch.c:15-19).  Larger row counts
+    // (prefill chunks) use one wave per run.
+    const uint32_t tiles = w->n_out / 16;
+    uint32_t ksplit = 1;
+    if (groups <= 2) {
+        while (ksplit < 4 && tiles * ksplit < 2048 && ktiles % (ksplit * 2) == 0 &&
+               ktiles / (ksplit * 2) >= 4)
+            ksplit *= 2;
+    }
+    // up to a few dozen rows, where one workgroup per CU can take them all: so does each workgroup of the product.  It
+    // reads the rows with 16-byte loads, and while others already write results.
+    // (Four waves to the inputs, as the kernel of one row then has: a row's bits are its own in a step of up to sixteen.)
+    const uintptr_t x0 = (uintptr_t)x_dev, y0 = (uintptr_t)y_dev;
+    const bool apart = x0 + ((size_t)(rows - 1) * ldx + w->n_in) * 4 <= y0 || y0 + ((size_t)(rows - 1) * ldy + w->n_out) * 4 <= x0;
+    uint32_t fused_nt = 0;
+    const FusedKernel fused =
+        rows > 1 && rows < kProjGroupRows && (gemm || ksplit == 4) && ldx % 4 == 0 && ((x0 | (uintptr_t)src.norm_w) & 15) == 0 && apart
+            ? pick_fused(src.kind, w->n_in, w->n_out / 16, groups, &fused_nt)
+            : nullptr;
     const size_t frag_bytes = (size_t)groups * ktiles * 1024;
     int rc = ensure_device(cx->d_proj, frag_bytes + kProjMaxRows * sizeof(float));
     if (rc) return rc;
@@ -895,7 +962,7 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
         else                                                                                         \
             hipLaunchKernelGGL(HIP_KERNEL_NAME(proj_prep_kernel<SRC, 0>), pgrid, pblock, 0, cx->stream, pa); \
     } while (0)
-    if (row1)
+    if (row1 || fused)
         ;                                           // no fragment launch
     else if (src.kind == kProjSrcRmsNorm)
         WR_LAUNCH_PREP(kProjSrcRmsNorm);
@@ -917,20 +984,6 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     a.K = w->n_in;
     a.R = rows;
     a.ldy = ldy;
-    // Waves that share a run of outputs (contiguous parts of the inputs, summed
-    // through LDS in a fixed order): enough that a narrow weight still gives
-    // one to two thousand waves.  A function of the weight's shape only: a row's
-    // sums are then split the same way whether it travels alone or with up to
-    // fifteen others, so a batched step's rows equal the serial steps' bit
-    // for bit (reference contract: src/core/batch.c:15-19).  Larger row counts
-    // (prefill chunks) use one wave per run.
-    const uint32_t tiles = w->n_out / 16;
-    uint32_t ksplit = 1;
-    if (groups <= 2) {
-        while (ksplit < 4 && tiles * ksplit < 2048 && ktiles % (ksplit * 2) == 0 &&
-               ktiles / (ksplit * 2) >= 4)
-            ksplit *= 2;
-    }
     a.ksplit = ksplit;
     if (row1) {
         const dim3 grid((tiles + 4 / ksplit - 1) / (4 / ksplit)), block(kProjThreads);
@@ -943,7 +996,9 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
             launch_main(proj_row1_kernel<kProjSrcGeglu>, grid, block, a, pa, lds);
         else
             launch_main(proj_row1_kernel<kProjSrcPlain>, grid, block, a, pa, lds);
-    } else if (gemm)
+    } else if (fused)
+        launch_main(fused, dim3((tiles + fused_nt - 1) / fused_nt, groups), dim3(kProjThreads), a, pa, (size_t)w->n_in * 32);
+    else if (gemm)
         launch_proj_gemm(a, groups);
     else if (ksplit == 4)
         // A workgroup per tile and group of eight rows, four waves to the input range: the
@@ -1075,6 +1130,12 @@ int wr_hip_attn_init(int device)
         if (e == hipSuccess)
             e = hipFuncSetAttribute(reinterpret_cast<const void*>(proj_gemm_lds_kernel<8, 4, 4>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes<8, 4, 4>());
+        for (uint32_t n_in = 512; n_in <= 3072; n_in += 512)
+            for (uint32_t nt = 1; nt <= 4; nt++)
+                for (const int src : {kProjSrcPlain, kProjSrcRmsNorm})
+                    if (const FusedKernel k = fused_kernel(src, n_in, nt); k && e == hipSuccess)
+                        e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                (int)(n_in * 32));
         if (e != hipSuccess) rc = hip_fail(e, "kernel LDS size", 0);
     }
     if (rc != WR_HIP_OK) {
