@@ -381,6 +381,17 @@ int wr_hip_proj_rows_geglu_dev(const wr_hip_weight *w, uint32_t rows,
                                const float *gate_up_dev, uint32_t ld,
                                const float *add_dev, float *y_dev, uint32_t ldy);
 
+/* The step before it: act[r][j] = a(x[r] . W[j]) * (x[r] . W[n_out / 2 + j]), a = SiLU
+ * or (gelu) the tanh form of GELU, for a weight that stacks gates and the values they
+ * gate; x normalised first if norm_w_dev is not NULL.  n_out a multiple of 32, ldo >=
+ * n_out / 2 and a multiple of 4, act_dev 16-byte aligned.  Values are those of
+ * wr_hip_proj_rows_dev or _norm_dev followed by the activation (wr_hip_rows_swiglu_dev,
+ * or the one in _geglu_dev), bit for bit. */
+int wr_hip_proj_rows_gated_dev(const wr_hip_weight *w, uint32_t rows,
+                               const float *x_dev, uint32_t ldx,
+                               const float *norm_w_dev, float eps, int gelu,
+                               float *act_dev, uint32_t ldo);
+
 /* ---- row steps between the projections and the attention path --------------
  * For callers that keep a layer's activations on the device.  All arguments
  * are device pointers (wr_hip_attn_dev_alloc), all calls are asynchronous on

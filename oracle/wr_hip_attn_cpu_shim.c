@@ -405,6 +405,12 @@ int wr_hip_proj_rows_geglu_dev(const wr_hip_weight *w, uint32_t rows, const floa
     (void)w; (void)rows; (void)gu; (void)ld; (void)add; (void)y; (void)ldy;
     return WR_HIP_ERR_STATE;
 }
+int wr_hip_proj_rows_gated_dev(const wr_hip_weight *w, uint32_t rows, const float *x, uint32_t ldx,
+                               const float *nw, float eps, int gelu, float *act, uint32_t ldo)
+{
+    (void)w; (void)rows; (void)x; (void)ldx; (void)nw; (void)eps; (void)gelu; (void)act; (void)ldo;
+    return WR_HIP_ERR_STATE;
+}
 int wr_hip_rows_swiglu_dev(const float *gu, uint32_t ld, float *act, uint32_t ldo, uint32_t rows,
                            uint32_t ffn)
 {

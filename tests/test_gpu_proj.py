@@ -455,3 +455,60 @@ def test_rows_whose_workgroups_make_their_own_terms(rows, n_in, n_out):
     for d in (xd, nwd, addd, off, y, ya, y1):
         d.free()
     w.close()
+
+
+@pytest.mark.parametrize("rows,n_in,ffn", [
+    (1, 1024, 3072), (1, 96, 48), (1, 3104, 8208),                # one row: four waves a pair, none shared, two, an odd count
+    (2, 512, 16), (16, 1024, 3072), (8, 1536, 2064), (9, 512, 4080),   # workgroups that make their own terms: a pair, two
+    (5, 1056, 528), (16, 160, 48), (16, 1024, 16400),             # a wave per pair of tiles, inputs split and not
+    (17, 1056, 528), (100, 288, 2064), (200, 1056, 8208),         # register tiles of 32 x 8, 32 x 16, 32 x 32
+    (300, 1024, 4112), (700, 2048, 2064), (700, 1056, 2064),      # LDS tiles of 128 x 64 (two and more a CU; one, two sets of waves; one)
+    (1030, 288, 6160), (2050, 288, 4112),                         # of 128 x 128, of 256 x 128
+])
+def test_gates_and_values_in_one_product_equal_product_then_activation(rows, n_in, ffn):
+    # act(gate) * value from the product itself has the bits of the product followed
+    # by the activation's own step, SiLU directly and GELU through the next product,
+    # normalised or not; nothing is written beyond ffn.
+    print("gated", rows, n_in, ffn, flush=True)
+    lib, D, eps, n2 = hipattn.lib(), hipattn.DeviceBuffer, 1e-6, 32
+    x = synth.normal(221 + n_in, (rows, n_in), std=2.0)
+    nw = synth.normal(222, (n_in,)) * np.float32(0.2) + np.float32(1.0)
+    w, wd = hipattn.Weight([_w16(223, ffn, n_in, 0.1), _w16(224, ffn, n_in, 0.1)]), None
+    xd, nwd, gu = D.from_host(x), D.from_host(nw), D(rows * 2 * ffn * 4)
+    act, ld = D(rows * ffn * 4), ffn + 4
+    fill = np.full((rows, ld), 7.0, dtype=np.float32)
+    got = D.from_host(fill)
+    if ffn % 32 == 0:
+        wd = hipattn.Weight([_w16(225, n2, ffn, 0.1)])
+        ya, yb = D(rows * n2 * 4), D(rows * n2 * 4)
+    for norm in (True, False):
+        if norm:
+            assert lib.wr_hip_proj_rows_norm_dev(w.h, rows, xd.p, n_in, nwd.p, eps, None, gu.p, 2 * ffn) == hipattn.OK
+        else:
+            w.rows_dev(rows, xd, n_in, gu, 2 * ffn)
+        assert lib.wr_hip_rows_swiglu_dev(gu.p, 2 * ffn, act.p, ffn, rows, ffn) == hipattn.OK
+        assert lib.wr_hip_proj_rows_gated_dev(w.h, rows, xd.p, n_in, nwd.p if norm else None, eps, 0, got.p, ld) == hipattn.OK
+        g = got.to_host((rows, ld))
+        assert np.isfinite(g).all() and g[:, :ffn].tobytes() == act.to_host((rows, ffn)).tobytes(), f"norm {norm}"
+        assert np.all(g[:, ffn:] == 7.0)
+        if wd:
+            assert lib.wr_hip_proj_rows_geglu_dev(wd.h, rows, gu.p, 2 * ffn, None, ya.p, n2) == hipattn.OK
+            assert lib.wr_hip_proj_rows_gated_dev(w.h, rows, xd.p, n_in, nwd.p if norm else None, eps, 1, act.p, ffn) == hipattn.OK
+            wd.rows_dev(rows, act, ffn, yb, n2)
+            assert ya.to_host((rows, n2)).tobytes() == yb.to_host((rows, n2)).tobytes(), f"norm {norm} gelu"
+    assert lib.wr_hip_proj_rows_gated_dev(w.h, rows, xd.p, n_in, None, eps, 0, got.p, ffn - 4) == hipattn.ERR_INVAL
+    assert lib.wr_hip_proj_rows_gated_dev(w.h, rows, xd.p, n_in, None, eps, 0, got.p + 4, ld) == hipattn.ERR_INVAL
+    assert lib.wr_hip_proj_rows_gated_dev(w.h, 0, xd.p, n_in, None, eps, 0, got.p, ld) == hipattn.OK
+    for d in (xd, nwd, gu, act, got) + ((ya, yb) if wd else ()):
+        d.free()
+    for h in (w, wd):
+        if h:
+            h.close()
+
+
+def test_gated_product_refuses_an_odd_number_of_tiles():
+    w = hipattn.Weight([_w16(226, 48, 64, 0.1)])
+    b = hipattn.DeviceBuffer(4096)
+    assert hipattn.lib().wr_hip_proj_rows_gated_dev(w.h, 1, b.p, 64, None, 1e-6, 0, b.p, 24) == hipattn.ERR_INVAL
+    b.free()
+    w.close()

@@ -427,6 +427,7 @@ struct ProjArgs {
     float* y;                // [R][ldy]
     uint32_t N, K, R, ldy;
     uint32_t ksplit;         // waves of a workgroup that share one run of outputs: 1, 2 or 4
+    int gate;                // GATED kernels: kProjSrcSwiglu or kProjSrcGeglu
 };
 
 // Writes one accumulator tile.  Layout: lane 16g + c holds outputs 16nt + 4g .. +3
@@ -469,6 +470,40 @@ __device__ __forceinline__ void proj_store_tile(const ProjArgs& a, f32x4 v, uint
     }
 }
 
+// GATED kernels take a weight whose first half of outputs are gates, the second the
+// values they gate: tile p and tile p + N / 32 are worked on by the same wave, and
+// what is stored is act(gate) * value, [R][N / 2].  The next product then reads half
+// the bytes and has no activation to work out (once per workgroup, in the kernels that
+// make their own operand terms).  The gate and the value are rounded as they would be
+// stored, so the result has the bits of the product followed by the activation.
+// 1024 -> 2 x 3072 -> 1024, launches of both products (us): one row 6.1 + 6.2 -> 5.8 +
+// 5.4; 16 rows 6.4 + 5.4 (fragments) + 5.9 -> 7.2 + 8.0; 2047 rows 70 + 14.2 + 44 ->
+// 62 + 11.5 + 44.
+__device__ __forceinline__ uint32_t proj_paired_tile(uint32_t pair, uint32_t t, uint32_t ntiles)
+{
+    return min(pair, ntiles / 2 - 1) + t * (ntiles / 2);         // (a pair past the end re-reads the last; dropped)
+}
+
+__device__ __forceinline__ void proj_store_pair(const ProjArgs& a, f32x4 gate, f32x4 value, uint32_t pair, uint32_t group,
+                                                int lane, const float* scale = nullptr)
+{
+    const int c = lane & 15, g = lane >> 4;
+    gate = proj_join_terms(gate);
+    value = proj_join_terms(value);
+    const uint32_t row = group * 8 + (c & 7);
+    if (c < 8 && row < a.R && pair < a.N / 32) {
+        const float sc = scale ? *scale : a.scales[row];
+        f32x4 r;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float x = gate[i] * sc, y = value[i] * sc;
+            asm volatile("" : "+v"(x), "+v"(y));                 // the products end here: no contraction into the activation
+            r[i] = a.gate == kProjSrcGeglu ? proj_gated<kProjSrcGeglu>(x, y) : proj_gated<kProjSrcSwiglu>(x, y);
+        }
+        *reinterpret_cast<f32x4*>(a.y + (size_t)row * a.ldy + pair * 16 + g * 4) = r;
+    }
+}
+
 // One wave-step: NT weight tiles against GROUPS operand fragments.
 template <int GROUPS, int NT>
 __device__ __forceinline__ void proj_step(f32x4 (&acc)[NT][GROUPS], const half8 (&wv)[NT],
@@ -492,9 +527,10 @@ __device__ __forceinline__ void proj_step(f32x4 (&acc)[NT][GROUPS], const half8 
 // depend on timing.  Every X fragment a wave loads serves NT weight tiles:
 // with two row groups (9..16 rows) NT = 2 keeps the operand traffic through
 // the vector cache at the two bytes per weight byte of the one-group case.
-template <int GROUPS, int NT>
+template <int GROUPS, int NT, bool GATED = false>
 __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs a)
 {
+    static_assert(!GATED || NT == 2, "a gate's tile and a value's");
     constexpr int KB = kProjKBatch / NT;                               // k-steps per register batch
     // partial sums of the waves with part > 0: (4 / S) runs x (S - 1) parts <= 3 entries
     __shared__ f32x4 s_part[3 * NT * GROUPS * 64];
@@ -503,9 +539,9 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
     const uint32_t S = a.ksplit;
     const uint32_t slot = wave / S, part = wave % S;
     const uint32_t run = blockIdx.x * (4 / S) + slot;            // this wave's run of 16*NT outputs
-    const uint32_t nt0 = run * NT;
+    const uint32_t nt0 = GATED ? run : run * NT;                 // (GATED: a pair of tiles)
     const uint32_t ntiles = a.N / 16;
-    const bool live = nt0 < ntiles;                              // N/16 need not be a multiple of the runs per block
+    const bool live = nt0 < (GATED ? ntiles / 2 : ntiles);                              // N/16 need not be a multiple of the runs per block
     const uint32_t ktiles = a.K / 32;
     const uint32_t kper = ktiles / S;                            // host guarantees divisibility
     const uint32_t k_begin = part * kper, k_end = k_begin + kper;
@@ -522,7 +558,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
         const half8* wp[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-            const uint32_t nt = (nt0 + t < ntiles) ? nt0 + t : ntiles - 1;
+            const uint32_t nt = GATED ? proj_paired_tile(nt0, t, ntiles) : (nt0 + t < ntiles) ? nt0 + t : ntiles - 1;
             wp[t] = a.w + (size_t)nt * ktiles * 64 + lane;
         }
         // W is read exactly once per launch (non-temporal); X fragments are
@@ -609,6 +645,11 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
     }
     if (!live) return;
 
+    if constexpr (GATED) {
+#pragma unroll
+        for (int gi = 0; gi < GROUPS; gi++) proj_store_pair(a, acc[0][gi], acc[1][gi], nt0, gi, lane);
+        return;
+    }
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -634,11 +675,12 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
 // row run while the weights travel.  NB0 = batches asked for up front, a
 // template parameter so that every load before the first wait is unconditional
 // and the compiler's count of loads in flight is exact.
-template <int SRC, int NB0>
+template <int SRC, int NB0, bool GATED>
 __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrepArgs& p, half8* sfrag,
                                                f32x4* s_part, float* s4, float* s_scale)
 {
-    constexpr int KB = kProjKBatch;
+    constexpr int NT = GATED ? 2 : 1;                            // weight tiles of a wave
+    constexpr int KB = kProjKBatch / NT;
     constexpr int CH = 2;                                        // chunks of eight inputs a thread can hold
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t t = threadIdx.x;
@@ -646,11 +688,14 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
     const uint32_t slot = wave / S, part = wave % S;
     const uint32_t nt0 = blockIdx.x * (4 / S) + slot;
     const uint32_t ntiles = a.N / 16;
-    const bool live = nt0 < ntiles;
+    const bool live = nt0 < (GATED ? ntiles / 2 : ntiles);       // (GATED: nt0 is a pair of tiles)
     const uint32_t ktiles = a.K / 32, nchunks = a.K / 8;
     const uint32_t kper = ktiles / S;
     const uint32_t k_begin = part * kper, k_end = k_begin + kper;
-    const half8* wp = a.w + (size_t)(live ? nt0 : ntiles - 1) * ktiles * 64 + lane;
+    const half8* wp[NT];
+#pragma unroll
+    for (int tt = 0; tt < NT; tt++)
+        wp[tt] = a.w + (size_t)(GATED ? proj_paired_tile(nt0, tt, ntiles) : live ? nt0 : ntiles - 1) * ktiles * 64 + lane;
     const float* xr = p.x;
     const bool in_regs = a.K <= 2048u * CH;                      // uniform
 
@@ -686,11 +731,14 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
     }
 
     // 2. the weights: NB0 batches now, the rest as the buffers come free
-    half8 wa[KB], wb[KB], wc[KB];
+    half8 wa[KB][NT], wb[KB][NT], wc[KB][NT];
     const uint32_t nb = kper / KB;                               // whole batches of this wave (>= NB0)
-    auto load_batch = [&](half8 (&w)[KB], uint32_t b) {
+    auto load_batch = [&](half8 (&w)[KB][NT], uint32_t b) {
 #pragma unroll
-        for (int u = 0; u < KB; u++) w[u] = __builtin_nontemporal_load(&wp[(size_t)(k_begin + b * KB + u) * 64]);
+        for (int u = 0; u < KB; u++)
+#pragma unroll
+            for (int tt = 0; tt < NT; tt++)
+                w[u][tt] = __builtin_nontemporal_load(&wp[tt][(size_t)(k_begin + b * KB + u) * 64]);
     };
     if constexpr (NB0 > 0) load_batch(wa, 0);
     if constexpr (NB0 > 1) load_batch(wb, 1);
@@ -795,14 +843,17 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
     half8 zero;
 #pragma unroll
     for (int j = 0; j < 8; j++) zero[j] = (_Float16)0.0f;
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto step = [&](const half8& wv, uint32_t k) {
+    f32x4 acc[NT];
+#pragma unroll
+    for (int tt = 0; tt < NT; tt++) acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](const half8 (&wv)[NT], uint32_t k) {
         const half8 xb = has ? my[(size_t)k * 8] : zero;
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xb, acc, 0, 0, 0);
+#pragma unroll
+        for (int tt = 0; tt < NT; tt++) acc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[tt], xb, acc[tt], 0, 0, 0);
     };
     // k-steps in ascending order, whatever buffer holds them (the order of the sum
     // is that of proj_rows_kernel<1, 1>)
-    auto steps = [&](const half8 (&w)[KB], uint32_t b) {
+    auto steps = [&](const half8 (&w)[KB][NT], uint32_t b) {
 #pragma unroll
         for (int u = 0; u < KB; u++) step(w[u], k_begin + b * KB + u);
     };
@@ -825,39 +876,53 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
             }
         }
     }
-    for (uint32_t kt = k_begin + nb * KB; kt < k_end; kt++) step(__builtin_nontemporal_load(&wp[(size_t)kt * 64]), kt);
+    for (uint32_t kt = k_begin + nb * KB; kt < k_end; kt++) {
+        half8 wv[NT];
+#pragma unroll
+        for (int tt = 0; tt < NT; tt++) wv[tt] = __builtin_nontemporal_load(&wp[tt][(size_t)kt * 64]);
+        step(wv, kt);
+    }
 
     if (S > 1) {                                                 // uniform over the workgroup
-        if (part > 0) s_part[(slot * (S - 1) + (part - 1)) * 64 + lane] = acc;
+        if (part > 0) {
+#pragma unroll
+            for (int tt = 0; tt < NT; tt++) s_part[((slot * (S - 1) + (part - 1)) * NT + tt) * 64 + lane] = acc[tt];
+        }
         __syncthreads();
         if (part > 0) return;
         for (uint32_t pp = 1; pp < S; pp++) {
-            const f32x4 o = s_part[(slot * (S - 1) + (pp - 1)) * 64 + lane];
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[i] += o[i];
+            for (int tt = 0; tt < NT; tt++) {
+                const f32x4 o = s_part[((slot * (S - 1) + (pp - 1)) * NT + tt) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[tt][i] += o[i];
+            }
         }
     }
     if (!live) return;
-    proj_store_tile(a, acc, nt0, 0, lane, s_scale, &resid);
+    if constexpr (GATED)
+        proj_store_pair(a, acc[0], acc[1], nt0, 0, lane, s_scale);
+    else
+        proj_store_tile(a, acc[0], nt0, 0, lane, s_scale, &resid);
 }
 
-template <int SRC>
+template <int SRC, bool GATED = false>
 __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs a, const ProjPrepArgs p)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char row1_smem[];
     half8* sfrag = reinterpret_cast<half8*>(row1_smem);           // [K/8][2]: hi, lo of chunk q
-    __shared__ f32x4 s_part[3 * 64];
+    __shared__ f32x4 s_part[(GATED ? 6 : 3) * 64];
     __shared__ float s4[8];
     __shared__ float s_scale;
-    const uint32_t nb = a.K / 32 / a.ksplit / kProjKBatch;        // whole batches of weights per wave: uniform
+    const uint32_t nb = a.K / 32 / a.ksplit / (kProjKBatch / (GATED ? 2 : 1));        // whole batches of weights per wave: uniform
     if (nb >= 3)
-        proj_row1_body<SRC, 3>(a, p, sfrag, s_part, s4, &s_scale);
+        proj_row1_body<SRC, 3, GATED>(a, p, sfrag, s_part, s4, &s_scale);
     else if (nb == 2)
-        proj_row1_body<SRC, 2>(a, p, sfrag, s_part, s4, &s_scale);
+        proj_row1_body<SRC, 2, GATED>(a, p, sfrag, s_part, s4, &s_scale);
     else if (nb == 1)
-        proj_row1_body<SRC, 1>(a, p, sfrag, s_part, s4, &s_scale);
+        proj_row1_body<SRC, 1, GATED>(a, p, sfrag, s_part, s4, &s_scale);
     else
-        proj_row1_body<SRC, 0>(a, p, sfrag, s_part, s4, &s_scale);
+        proj_row1_body<SRC, 0, GATED>(a, p, sfrag, s_part, s4, &s_scale);
 }
 
 // Two rows to a few dozen, inputs of 512 D / 4: the fragment step inside the product.
@@ -877,10 +942,11 @@ __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs 
 // 7.7 -> 5.5, 3072 -> 1024 9.5 -> 7.8; 32 rows of the third 7.8 -> 5.5.  (A lane making
 // the terms of four inputs of its own operand column and trading them with the lane
 // eight on, no LDS: 5.7, 6.7, 5.8, 8.1.)
-template <int SRC, int D, int NT>
+template <int SRC, int D, int NT, bool GATED = false>
 __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const ProjArgs a, const ProjPrepArgs p)
 {
     static_assert(D % 2 == 0 && (SRC == kProjSrcPlain || (SRC == kProjSrcRmsNorm && D <= 16)), "sources held in registers");
+    static_assert(!GATED || NT % 2 == 0, "gates' tiles and values'");
     constexpr bool NORM = SRC == kProjSrcRmsNorm;
     constexpr int KT = 4 * D;                                    // k-steps of a row
     constexpr int CH = D / 2;                                    // chunks of eight inputs per lane
@@ -913,10 +979,10 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
     const half8* wp[NT];
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-        const uint32_t tile = min(nt0 + t, ntiles - 1);          // (one past the end: dropped)
+        const uint32_t tile = GATED ? proj_paired_tile((nt0 + t) / 2, t % 2, ntiles) : min(nt0 + t, ntiles - 1);   // (one past the end: dropped)
         const uint32_t row = min(group * 8 + (lane & 7), a.R - 1);
         resid[t] = *reinterpret_cast<const f32x4*>(
-            a.bias_rows ? a.bias_rows + (size_t)row * a.ldy + tile * 16 + (lane >> 4) * 4 : xr);
+            !GATED && a.bias_rows ? a.bias_rows + (size_t)row * a.ldy + tile * 16 + (lane >> 4) * 4 : xr);
         wp[t] = a.w + ((size_t)tile * KT + k0) * 64;
     }
 #pragma unroll
@@ -1020,7 +1086,10 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
 #pragma unroll
             for (int i = 0; i < 4; i++) acc[t][i] += other[i];
         }
-        proj_store_tile(a, acc[t], nt0 + t, group, lane, &scale, &resid[t]);
+        if constexpr (!GATED)
+            proj_store_tile(a, acc[t], nt0 + t, group, lane, &scale, &resid[t]);
+        else if (t % 2 == 1)
+            proj_store_pair(a, acc[t - 1], acc[t], (nt0 + t) / 2, group, lane, &scale);
     }
 }
 
@@ -1049,7 +1118,7 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
 // (Below 64 rows a kernel of one wave per 64 outputs x 32 rows ran before: 20 us
 // for the first, 51 for the second.)  Eight waves to the input range, or deeper
 // turns on larger tiles, gave nothing.
-template <int GROUPS, int NT, int D>
+template <int GROUPS, int NT, int D, bool GATED = false>
 __global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_gemm_split_kernel(const ProjArgs a)
 {
     __shared__ f32x4 s_red[4 * NT * GROUPS * 64];
@@ -1064,7 +1133,7 @@ __global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_g
     const half8* xp[GROUPS];
 #pragma unroll
     for (int t = 0; t < NT; t++)
-        wp[t] = a.w + ((size_t)min(nt0 + t, ntiles - 1) * ktiles + k_begin) * 64;
+        wp[t] = a.w + ((size_t)(GATED ? proj_paired_tile((nt0 + t) / 2, t % 2, ntiles) : min(nt0 + t, ntiles - 1)) * ktiles + k_begin) * 64;
 #pragma unroll
     for (int gi = 0; gi < GROUPS; gi++)
         xp[gi] = a.xfrag + ((size_t)min(group0 + gi, ngroups - 1) * ktiles + k_begin) * 64;
@@ -1115,8 +1184,7 @@ __global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_g
 #pragma unroll
         for (int gi = 0; gi < GROUPS; gi++) s_red[((wave * NT + t) * GROUPS + gi) * 64 + lane] = acc[t][gi];
     lds_barrier();
-#pragma unroll 1
-    for (uint32_t i = wave; i < NT * GROUPS; i += 4) {
+    auto sum = [&](uint32_t i) {
         f32x4 v = s_red[i * 64 + lane];
 #pragma unroll
         for (int p = 1; p < 4; p++) {
@@ -1124,7 +1192,16 @@ __global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_g
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] += o[j];
         }
-        proj_store_tile(a, v, nt0 + i / GROUPS, group0 + i % GROUPS, lane);
+        return v;
+    };
+    if constexpr (GATED) {
+        static_assert(NT == 2, "a gate's tile and a value's");
+#pragma unroll 1
+        for (uint32_t i = wave; i < GROUPS; i += 4) proj_store_pair(a, sum(i), sum(GROUPS + i), blockIdx.x, group0 + i, lane);
+    } else {
+#pragma unroll 1
+        for (uint32_t i = wave; i < NT * GROUPS; i += 4)
+            proj_store_tile(a, sum(i), nt0 + i / GROUPS, group0 + i % GROUPS, lane);
     }
 }
 
@@ -1170,7 +1247,7 @@ constexpr size_t gemm_lds_bytes()
 // lower half adds them to its own, always in that order.  For products whose
 // tiles give every CU one workgroup and no more (a SIMD would hold a single wave
 // for a long chain of k-steps): twice the waves per SIMD, half the chain.
-template <int GROUPS, int WN, int RING, bool PIPE = false, int KS = 1>
+template <int GROUPS, int WN, int RING, bool PIPE = false, int KS = 1, bool GATED = false>
 __global__ __launch_bounds__(128 * WN * KS, (WN == 2 && KS == 1) ? 2 : 1) void proj_gemm_lds_kernel(const ProjArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char gemm_smem[];
@@ -1199,12 +1276,16 @@ __global__ __launch_bounds__(128 * WN * KS, (WN == 2 && KS == 1) ? 2 : 1) void p
 
     // chunk c of a stage: weight tile nt_wg + c (c < WN * NT) or fragment group
     // g_wg + c - WN * NT; one past the end re-reads the last one, and its results are dropped
+    // (GATED: of a wave's four tiles the first two are gates', the others their values')
+    auto tile_of = [&](uint32_t v) {
+        return GATED ? proj_paired_tile(v / 4 * 2 + v % 2, v / 2 % 2, ntiles) : min(v, ntiles - 1);
+    };
     const unsigned char* src[CPW];
 #pragma unroll
     for (int i = 0; i < CPW; i++) {
         const uint32_t c = wave * CPW + i;
         const unsigned char* p =
-            c < WN * NT ? reinterpret_cast<const unsigned char*>(a.w) + (size_t)min(nt_wg + c, ntiles - 1) * ktiles_row * 1024
+            c < WN * NT ? reinterpret_cast<const unsigned char*>(a.w) + (size_t)tile_of(nt_wg + c) * ktiles_row * 1024
                         : reinterpret_cast<const unsigned char*>(a.xfrag) +
                               (size_t)min(g_wg + c - WN * NT, ngroups - 1) * ktiles_row * 1024;
         src[i] = uniform_ptr(p + (size_t)kfirst * 1024);
@@ -1317,6 +1398,14 @@ __global__ __launch_bounds__(128 * WN * KS, (WN == 2 && KS == 1) ? 2 : 1) void p
 
     const uint32_t nt0 = nt_wg + wn * NT, group0 = g_wg + wr * GROUPS;
     if (nt0 >= ntiles || group0 >= ngroups) return;
+    if constexpr (GATED) {
+#pragma unroll
+        for (int t = 0; t < NT / 2; t++)
+#pragma unroll
+            for (int gi = 0; gi < GROUPS; gi++)
+                proj_store_pair(a, acc[t][gi], acc[t + 2][gi], nt0 / 2 + t, group0 + gi, lane);
+        return;
+    }
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll

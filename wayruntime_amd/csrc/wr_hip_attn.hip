@@ -757,12 +757,12 @@ Entered::Entered()
 // projections: launch helpers (the caller has entered)
 namespace {
 
-template <int GROUPS, int NT>
+template <int GROUPS, int NT, bool GATED = false>
 void launch_proj(const ProjArgs& a)
 {
     const uint32_t runs = (a.N / 16 + NT - 1) / NT;              // runs of 16*NT outputs
     const uint32_t per_block = 4 / a.ksplit;
-    launch_main(proj_rows_kernel<GROUPS, NT>, dim3((runs + per_block - 1) / per_block), dim3(kProjThreads), a);
+    launch_main(proj_rows_kernel<GROUPS, NT, GATED>, dim3((runs + per_block - 1) / per_block), dim3(kProjThreads), a);
 }
 
 // Prefill-sized row counts: the largest tile that still fills the chip.
@@ -777,10 +777,10 @@ constexpr uint32_t kProjGroupRows = 257;           // from here on the fragments
                                                    // workgroup per row is 0.6 to 2.2 us faster, at 300 as fast, at 511 1 us slower
 constexpr size_t kProjRow1MaxLds = 60 * 1024;      // inputs up to 15 360 take the one-row kernel
 
-template <int GROUPS, int NT, int D>
+template <int GROUPS, int NT, int D, bool GATED = false>
 void launch_proj_gemm_split(const ProjArgs& a, uint32_t groups)
 {
-    launch_main(proj_gemm_split_kernel<GROUPS, NT, D>,
+    launch_main(proj_gemm_split_kernel<GROUPS, NT, D, GATED>,
                 dim3((a.N / 16 + NT - 1) / NT, (groups + GROUPS - 1) / GROUPS), dim3(kProjThreads), a);
 }
 
@@ -812,24 +812,31 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
     const bool small_fills_better = n_small >= 512 && n_big * 100 < rounds_b * 512 * 70 &&
                                     (uint64_t)n_small * rounds_b * 100 >= (uint64_t)n_big * rounds_s * 100 + (uint64_t)rounds_b * rounds_s * 512 * 10;
     if (wide_fills)
-        launch_main(proj_gemm_lds_kernel<8, 4, 4>, dim3(wshare * ((groups + 15) / 16)), dim3(512), a,
+        launch_main(a.gate ? proj_gemm_lds_kernel<8, 4, 4, false, 1, true> : proj_gemm_lds_kernel<8, 4, 4>, dim3(wshare * ((groups + 15) / 16)), dim3(512), a,
                     gemm_lds_bytes<8, 4, 4>());
     else if (n_big >= 512 && !small_fills_better)
-        launch_main(proj_gemm_lds_kernel<8, 2, 3>, dim3(share * ((groups + 15) / 16)), dim3(kProjThreads), a,
+        launch_main(a.gate ? proj_gemm_lds_kernel<8, 2, 3, false, 1, true> : proj_gemm_lds_kernel<8, 2, 3>, dim3(share * ((groups + 15) / 16)), dim3(kProjThreads), a,
                     gemm_lds_bytes<8, 2, 3>());
     else if (panels * ((groups + 7) / 8) >= 512)          // two and more per CU cover each other's latency
-        launch_main(proj_gemm_lds_kernel<4, 2, 3>, dim3(share * ((groups + 7) / 8)), dim3(kProjThreads), a,
+        launch_main(a.gate ? proj_gemm_lds_kernel<4, 2, 3, false, 1, true> : proj_gemm_lds_kernel<4, 2, 3>, dim3(share * ((groups + 7) / 8)), dim3(kProjThreads), a,
                     gemm_lds_bytes<4, 2, 3>());
     else if (panels * ((groups + 7) / 8) >= 256 && (a.K / 32) % 2 == 0 && a.K >= 2048)
         // one per CU and a long input range: two sets of waves halve it (two waves per SIMD, half the
         // chain of k-steps; 2047 rows x 2048 -> 1024: 40.3 -> 28.3 us, x 3072 -> 1024: 40 -> 36.6; at
         // 1024 inputs the sum through LDS costs more than the shorter chain gives)
-        launch_main(proj_gemm_lds_kernel<4, 2, 4, true, 2>, dim3(share * ((groups + 7) / 8)), dim3(2 * kProjThreads), a,
+        launch_main(a.gate ? proj_gemm_lds_kernel<4, 2, 4, true, 2, true> : proj_gemm_lds_kernel<4, 2, 4, true, 2>, dim3(share * ((groups + 7) / 8)), dim3(2 * kProjThreads), a,
                     gemm_lds_bytes<4, 2, 4, 2>());
     else if (panels * ((groups + 7) / 8) >= 256)          // one per CU, one wave per SIMD: pipelined reads
-        launch_main(proj_gemm_lds_kernel<4, 2, 4, true>, dim3(share * ((groups + 7) / 8)), dim3(kProjThreads), a,
+        launch_main(a.gate ? proj_gemm_lds_kernel<4, 2, 4, true, 1, true> : proj_gemm_lds_kernel<4, 2, 4, true>, dim3(share * ((groups + 7) / 8)), dim3(kProjThreads), a,
                     gemm_lds_bytes<4, 2, 4>());
-    else if (nt * groups <= 512)                          // (64 rows, 2048 -> 1024: 5.4 us against 5.6 with the next)
+    else if (a.gate) {                                    // tiles in pairs: 32 x 8, 32 x 16, 32 x 32
+        if (nt / 2 * groups <= 512)
+            launch_proj_gemm_split<1, 2, 8, true>(a, groups);
+        else if (nt / 2 * ((groups + 1) / 2) <= 1024)
+            launch_proj_gemm_split<2, 2, 8, true>(a, groups);
+        else
+            launch_proj_gemm_split<4, 2, 4, true>(a, groups);
+    } else if (nt * groups <= 512)                          // (64 rows, 2048 -> 1024: 5.4 us against 5.6 with the next)
         launch_proj_gemm_split<1, 1, 8>(a, groups);
     else if (groups <= 6 && nt <= 256)                    // (45 rows, 1024 -> 6144: 7.6 us against 7.4 with the next)
         launch_proj_gemm_split<2, 1, 8>(a, groups);
@@ -843,8 +850,15 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
 using FusedKernel = void (*)(const ProjArgs, const ProjPrepArgs);
 
 template <int SRC, int D>
-FusedKernel fused_of(uint32_t nt)
+FusedKernel fused_of(uint32_t nt, bool gated)
 {
+    if (gated) {
+        if constexpr (D <= 16)
+            if (nt == 2) return proj_rows_fused_kernel<SRC, D, 2, true>;
+        if constexpr (D <= 8)
+            if (nt == 4) return proj_rows_fused_kernel<SRC, D, 4, true>;
+        return nullptr;
+    }
     if (nt == 1) return proj_rows_fused_kernel<SRC, D, 1>;
     if constexpr (D <= 16)
         if (nt == 2) return proj_rows_fused_kernel<SRC, D, 2>;
@@ -855,17 +869,17 @@ FusedKernel fused_of(uint32_t nt)
     return nullptr;
 }
 
-FusedKernel fused_kernel(int src, uint32_t n_in, uint32_t nt)
+FusedKernel fused_kernel(int src, uint32_t n_in, uint32_t nt, bool gated)
 {
     const bool norm = src == kProjSrcRmsNorm;
     if (!norm && src != kProjSrcPlain) return nullptr;
     switch (n_in) {
-    case 512: return norm ? fused_of<kProjSrcRmsNorm, 4>(nt) : fused_of<kProjSrcPlain, 4>(nt);
-    case 1024: return norm ? fused_of<kProjSrcRmsNorm, 8>(nt) : fused_of<kProjSrcPlain, 8>(nt);
-    case 1536: return norm ? fused_of<kProjSrcRmsNorm, 12>(nt) : fused_of<kProjSrcPlain, 12>(nt);
-    case 2048: return norm ? fused_of<kProjSrcRmsNorm, 16>(nt) : fused_of<kProjSrcPlain, 16>(nt);
-    case 2560: return norm ? nullptr : fused_of<kProjSrcPlain, 20>(nt);
-    case 3072: return norm ? nullptr : fused_of<kProjSrcPlain, 24>(nt);
+    case 512: return norm ? fused_of<kProjSrcRmsNorm, 4>(nt, gated) : fused_of<kProjSrcPlain, 4>(nt, gated);
+    case 1024: return norm ? fused_of<kProjSrcRmsNorm, 8>(nt, gated) : fused_of<kProjSrcPlain, 8>(nt, gated);
+    case 1536: return norm ? fused_of<kProjSrcRmsNorm, 12>(nt, gated) : fused_of<kProjSrcPlain, 12>(nt, gated);
+    case 2048: return norm ? fused_of<kProjSrcRmsNorm, 16>(nt, gated) : fused_of<kProjSrcPlain, 16>(nt, gated);
+    case 2560: return norm ? nullptr : fused_of<kProjSrcPlain, 20>(nt, gated);
+    case 3072: return norm ? nullptr : fused_of<kProjSrcPlain, 24>(nt, gated);
     default: return nullptr;
     }
 }
@@ -875,10 +889,10 @@ FusedKernel fused_kernel(int src, uint32_t n_in, uint32_t nt)
 // a CU would make the same rows' terms again, and that is vector-ALU time nothing
 // hides: 16 rows, norm + 1024 -> 4096, one / two / three / four tiles (512 / 256 / 172 /
 // 128 workgroups) 6.7 / 5.2 / 5.9 / 6.5 us; -> 6144 8.6 / 7.8 / 6.2 / 6.8.
-FusedKernel pick_fused(int src, uint32_t n_in, uint32_t tiles, uint32_t groups, uint32_t* nt)
+FusedKernel pick_fused(int src, uint32_t n_in, uint32_t tiles, uint32_t groups, bool gated, uint32_t* nt)
 {
-    for (*nt = 1; *nt <= 4; ++*nt)
-        if ((tiles + *nt - 1) / *nt * groups <= (uint32_t)g.n_cus) return fused_kernel(src, n_in, *nt);
+    for (*nt = gated ? 2 : 1; *nt <= 4; *nt += gated ? 2 : 1)
+        if ((tiles + *nt - 1) / *nt * groups <= (uint32_t)g.n_cus) return fused_kernel(src, n_in, *nt, gated);
     return nullptr;
 }
 
@@ -888,6 +902,7 @@ struct ProjSource {
     int kind = kProjSrcPlain;
     const float* norm_w = nullptr;
     float eps = 0.f;
+    int gate = 0;            // kProjSrcSwiglu, kProjSrcGeglu: the weight's halves are gates and values (GATED kernels)
 };
 
 // y_dev[rows][ldy] = source(x_dev)[rows][n_in] . W^T (+ add_dev), rows <= kProjMaxRows.
@@ -917,12 +932,13 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     // up to a few dozen rows, where one workgroup per CU can take them all: so does each workgroup of the product.  It
     // reads the rows with 16-byte loads, and while others already write results.
     // (Four waves to the inputs, as the kernel of one row then has: a row's bits are its own in a step of up to sixteen.)
+    const uint32_t y_cols = src.gate ? w->n_out / 2 : w->n_out;
     const uintptr_t x0 = (uintptr_t)x_dev, y0 = (uintptr_t)y_dev;
-    const bool apart = x0 + ((size_t)(rows - 1) * ldx + w->n_in) * 4 <= y0 || y0 + ((size_t)(rows - 1) * ldy + w->n_out) * 4 <= x0;
+    const bool apart = x0 + ((size_t)(rows - 1) * ldx + w->n_in) * 4 <= y0 || y0 + ((size_t)(rows - 1) * ldy + y_cols) * 4 <= x0;
     uint32_t fused_nt = 0;
     const FusedKernel fused =
         rows > 1 && rows < kProjGroupRows && (gemm || ksplit == 4) && ldx % 4 == 0 && ((x0 | (uintptr_t)src.norm_w) & 15) == 0 && apart
-            ? pick_fused(src.kind, w->n_in, w->n_out / 16, groups, &fused_nt)
+            ? pick_fused(src.kind, w->n_in, tiles, groups, src.gate != 0, &fused_nt)
             : nullptr;
     const size_t frag_bytes = (size_t)groups * ktiles * 1024;
     int rc = ensure_device(cx->d_proj, frag_bytes + kProjMaxRows * sizeof(float));
@@ -984,11 +1000,17 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     a.K = w->n_in;
     a.R = rows;
     a.ldy = ldy;
+    a.gate = src.gate;
     a.ksplit = ksplit;
     if (row1) {
-        const dim3 grid((tiles + 4 / ksplit - 1) / (4 / ksplit)), block(kProjThreads);
+        const uint32_t runs = src.gate ? tiles / 2 : tiles;
+        const dim3 grid((runs + 4 / ksplit - 1) / (4 / ksplit)), block(kProjThreads);
         const size_t lds = (size_t)w->n_in * 4;
-        if (src.kind == kProjSrcRmsNorm)
+        if (src.gate && src.kind == kProjSrcRmsNorm)
+            launch_main(proj_row1_kernel<kProjSrcRmsNorm, true>, grid, block, a, pa, lds);
+        else if (src.gate)
+            launch_main(proj_row1_kernel<kProjSrcPlain, true>, grid, block, a, pa, lds);
+        else if (src.kind == kProjSrcRmsNorm)
             launch_main(proj_row1_kernel<kProjSrcRmsNorm>, grid, block, a, pa, lds);
         else if (src.kind == kProjSrcSwiglu)
             launch_main(proj_row1_kernel<kProjSrcSwiglu>, grid, block, a, pa, lds);
@@ -1000,6 +1022,10 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
         launch_main(fused, dim3((tiles + fused_nt - 1) / fused_nt, groups), dim3(kProjThreads), a, pa, (size_t)w->n_in * 32);
     else if (gemm)
         launch_proj_gemm(a, groups);
+    else if (src.gate && groups == 1)
+        launch_proj<1, 2, true>(a);
+    else if (src.gate)
+        launch_proj<2, 2, true>(a);
     else if (ksplit == 4)
         // A workgroup per tile and group of eight rows, four waves to the input range: the
         // same parts in the same order as below, so the same bits.  For 9 .. 16 rows the
@@ -1118,24 +1144,22 @@ int wr_hip_attn_init(int device)
         if (e == hipSuccess)
             e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_ild_kernel<false>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)ild_smem_bytes());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(proj_gemm_lds_kernel<8, 2, 3>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes<8, 2, 3>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(proj_gemm_lds_kernel<4, 2, 4, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes<4, 2, 4>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(proj_gemm_lds_kernel<4, 2, 4, true, 2>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes<4, 2, 4, 2>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(proj_gemm_lds_kernel<8, 4, 4>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes<8, 4, 4>());
+        const auto allow_lds = [&](auto kernel, size_t bytes) {
+            if (kernel && e == hipSuccess)
+                e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        };
+        allow_lds(proj_gemm_lds_kernel<8, 2, 3>, gemm_lds_bytes<8, 2, 3>());
+        allow_lds(proj_gemm_lds_kernel<8, 2, 3, false, 1, true>, gemm_lds_bytes<8, 2, 3>());
+        allow_lds(proj_gemm_lds_kernel<4, 2, 4, true>, gemm_lds_bytes<4, 2, 4>());
+        allow_lds(proj_gemm_lds_kernel<4, 2, 4, true, 1, true>, gemm_lds_bytes<4, 2, 4>());
+        allow_lds(proj_gemm_lds_kernel<4, 2, 4, true, 2>, gemm_lds_bytes<4, 2, 4, 2>());
+        allow_lds(proj_gemm_lds_kernel<4, 2, 4, true, 2, true>, gemm_lds_bytes<4, 2, 4, 2>());
+        allow_lds(proj_gemm_lds_kernel<8, 4, 4>, gemm_lds_bytes<8, 4, 4>());
+        allow_lds(proj_gemm_lds_kernel<8, 4, 4, false, 1, true>, gemm_lds_bytes<8, 4, 4>());
         for (uint32_t n_in = 512; n_in <= 3072; n_in += 512)
             for (uint32_t nt = 1; nt <= 4; nt++)
                 for (const int src : {kProjSrcPlain, kProjSrcRmsNorm})
-                    if (const FusedKernel k = fused_kernel(src, n_in, nt); k && e == hipSuccess)
-                        e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                (int)(n_in * 32));
+                    for (const bool gated : {false, true}) allow_lds(fused_kernel(src, n_in, nt, gated), (size_t)n_in * 32);
         if (e != hipSuccess) rc = hip_fail(e, "kernel LDS size", 0);
     }
     if (rc != WR_HIP_OK) {
@@ -1849,12 +1873,12 @@ void wr_hip_proj_weight_destroy(wr_hip_weight* w)
 }
 
 static int check_proj(const wr_hip_weight* w, uint32_t rows, const void* x, uint32_t ldx,
-                      uint32_t min_ldx, const void* y, uint32_t ldy)
+                      uint32_t min_ldx, const void* y, uint32_t ldy, uint32_t min_ldy)
 {
     if (!g.inited) return WR_HIP_ERR_STATE;
     if (!w || !x || !y) return WR_HIP_ERR_INVAL;
     if (rows == 0) return WR_HIP_OK;
-    if (ldx < min_ldx || ldy < w->n_out || ldy % 4 != 0) return WR_HIP_ERR_INVAL;
+    if (ldx < min_ldx || ldy < min_ldy || ldy % 4 != 0) return WR_HIP_ERR_INVAL;
     return WR_HIP_OK;
 }
 
@@ -1862,7 +1886,7 @@ static int proj_dev_common(const wr_hip_weight* w, uint32_t rows, const float* x
                            uint32_t min_ldx, const ProjSource& src, const float* add_dev,
                            float* y_dev, uint32_t ldy)
 {
-    int rc = check_proj(w, rows, x_dev, ldx, min_ldx, y_dev, ldy);
+    int rc = check_proj(w, rows, x_dev, ldx, min_ldx, y_dev, ldy, w ? w->n_out : 0);
     if (rc || rows == 0) return rc;
     if (((uintptr_t)y_dev & 15) || (add_dev && ((uintptr_t)add_dev & 15))) return WR_HIP_ERR_INVAL;
     ENTER();
@@ -1903,10 +1927,26 @@ int wr_hip_proj_rows_geglu_dev(const wr_hip_weight* w, uint32_t rows, const floa
     return proj_dev_common(w, rows, gate_up_dev, ld, w ? 2 * w->n_in : 0, src, add_dev, y_dev, ldy);
 }
 
+int wr_hip_proj_rows_gated_dev(const wr_hip_weight* w, uint32_t rows, const float* x_dev, uint32_t ldx,
+                               const float* norm_w_dev, float eps, int gelu, float* act_dev, uint32_t ldo)
+{
+    if (w && w->n_out % 32) return WR_HIP_ERR_INVAL;
+    int rc = check_proj(w, rows, x_dev, ldx, w ? w->n_in : 0, act_dev, ldo, w ? w->n_out / 2 : 0);
+    if (rc || rows == 0) return rc;
+    if ((uintptr_t)act_dev & 15) return WR_HIP_ERR_INVAL;
+    ProjSource src;
+    src.kind = norm_w_dev ? kProjSrcRmsNorm : kProjSrcPlain;
+    src.norm_w = norm_w_dev;
+    src.eps = eps;
+    src.gate = gelu ? kProjSrcGeglu : kProjSrcSwiglu;
+    ENTER();
+    return proj_locked(w, rows, x_dev, ldx, src, nullptr, act_dev, ldo);
+}
+
 int wr_hip_proj_rows(const wr_hip_weight* w, uint32_t rows, const float* x, float* y)
 {
     if (w && (w->n_out % 4 != 0)) return WR_HIP_ERR_INVAL;
-    int rc = check_proj(w, rows, x, w ? w->n_in : 0, w ? w->n_in : 0, y, w ? w->n_out : 0);
+    int rc = check_proj(w, rows, x, w ? w->n_in : 0, w ? w->n_in : 0, y, w ? w->n_out : 0, w ? w->n_out : 0);
     if (rc || rows == 0) return rc;
     const size_t xb = ((size_t)rows * w->n_in * sizeof(float) + 255) & ~(size_t)255;
     const size_t yb = (size_t)rows * w->n_out * sizeof(float);

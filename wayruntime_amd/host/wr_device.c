@@ -174,7 +174,7 @@ int wrh_devspace_init(wrh_devspace *ws, const wr_model *m, uint32_t rows, uint32
     const size_t hidden = m->hidden, qd = (size_t)m->n_q * hd, kd = (size_t)m->n_kv * hd;
     const size_t ffn = m->ffn, R = rows;
     const size_t total = 2 * r64(R * hidden) + r64(R * (qd + 2 * kd)) + 2 * r64(R * qd) + 2 * r64(R * kd) +
-                         r64(R * 2 * ffn) + 2 * r64(R * hd) + r64((size_t)logit_rows * m->vocab);
+                         r64(R * ffn) + 2 * r64(R * hd) + r64((size_t)logit_rows * m->vocab);
     float *b = wr_hip_attn_dev_alloc(total * sizeof(float));
     if (!b) return WR_ERR_NOMEM;
     ws->block = b;
@@ -187,7 +187,7 @@ int wrh_devspace_init(wrh_devspace *ws, const wr_model *m, uint32_t rows, uint32
     ws->attn = b;    b += r64(R * qd);
     ws->k = b;       b += r64(R * kd);
     ws->v = b;       b += r64(R * kd);
-    ws->gu = b;      b += r64(R * 2 * ffn);
+    ws->act = b;     b += r64(R * ffn);
     ws->rope = b;    b += r64(R * hd);
     ws->rope_swa = b; b += r64(R * hd);
     ws->logits = b;
@@ -469,19 +469,17 @@ wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *
             TRY(wr_hip_proj_rows_dev(dl->wo, R, ds->attn, qd, NULL, ds->proj, hidden), "output projection");
             TRY(wr_hip_rows_rmsnorm_add_dev(ds->proj, hidden, dl->post_attn_norm, hidden, ds->resid, hidden, R,
                                             hidden, m->rms_eps), "post-attention norm + residual");
-            TRY(wr_hip_proj_rows_norm_dev(dl->wgu, R, ds->resid, hidden, dl->ffn_norm, m->rms_eps, NULL,
-                                          ds->gu, 2 * ffn), "ffn norm + gate/up projection");
-            TRY(wr_hip_proj_rows_geglu_dev(dl->wdown, R, ds->gu, 2 * ffn, NULL, ds->proj, hidden),
-                "geglu + down projection");
+            TRY(wr_hip_proj_rows_gated_dev(dl->wgu, R, ds->resid, hidden, dl->ffn_norm, m->rms_eps, 1, ds->act, ffn),
+                "ffn norm + gate/up projection + geglu");
+            TRY(wr_hip_proj_rows_dev(dl->wdown, R, ds->act, ffn, NULL, ds->proj, hidden), "down projection");
             TRY(wr_hip_rows_rmsnorm_add_dev(ds->proj, hidden, dl->post_ffw_norm, hidden, ds->resid, hidden, R,
                                             hidden, m->rms_eps), "post-ffn norm + residual");
         } else {
             TRY(wr_hip_proj_rows_dev(dl->wo, R, ds->attn, qd, ds->resid, ds->resid, hidden),
                 "output projection");
-            TRY(wr_hip_proj_rows_norm_dev(dl->wgu, R, ds->resid, hidden, dl->ffn_norm, m->rms_eps, NULL,
-                                          ds->gu, 2 * ffn), "ffn norm + gate/up projection");
-            TRY(wr_hip_proj_rows_swiglu_dev(dl->wdown, R, ds->gu, 2 * ffn, ds->resid, ds->resid, hidden),
-                "swiglu + down projection");
+            TRY(wr_hip_proj_rows_gated_dev(dl->wgu, R, ds->resid, hidden, dl->ffn_norm, m->rms_eps, 0, ds->act, ffn),
+                "ffn norm + gate/up projection + swiglu");
+            TRY(wr_hip_proj_rows_dev(dl->wdown, R, ds->act, ffn, ds->resid, ds->resid, hidden), "down projection");
         }
     }
     L = m->n_layers;

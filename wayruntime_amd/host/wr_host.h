@@ -124,7 +124,7 @@ typedef struct wrh_devspace {
     float *qkv;                          /* [R][(n_q + 2 n_kv) * hd] */
     float *q, *attn;                     /* [R][n_q*hd] */
     float *k, *v;                        /* [R][n_kv*hd] */
-    float *gu;                           /* [R][2 ffn]: gate | up */
+    float *act;                          /* [R][ffn]: act(gate) up */
     float *rope;                         /* [R][hd/2][2] */
     float *rope_swa;                     /* the same for Gemma's sliding-window layers */
     float *proj;                         /* [R][hidden]: a sublayer output on its way through a post-norm */
