@@ -373,6 +373,9 @@ def test_projection_random_shapes():
     (256, 3072, 80),              # (each workgroup makes its own)
     (257, 288, 1040),             # ... by row groups
     (250, 1056, 4112),            # 32 x 32 tiles, 33 input tiles
+    (2047, 64, 1040),             # LDS tiles whose panels are shared out over few XCDs: 9 by 32 of them
+    (4095, 96, 528),              # ... 5 by 64
+    (1100, 64, 8208),             # ... the outputs over all eight: 33 by 18
 ])
 def test_products_of_a_short_prompt(rows, n_in, n_out):
     print("proj short prompt", rows, n_in, n_out, flush=True)

@@ -27,6 +27,7 @@ struct MixGemmArgs {
     uint32_t out, ldy, h_kt, col_z, n_split, silu_end, sigmoid_end, tanh_end, relu2, gelu;
     float scale, limit, slope, up_bias;
     const float* bias;
+    uint32_t cols;                   // mix_gemm_lds_kernel without experts: XCDs that share out the outputs (xcd_tile)
     const uint32_t* x_perm;
     const float* x_scale;            // a factor per row of the input (applied to its products), or nullptr
     float* y;
@@ -275,17 +276,21 @@ __global__ __launch_bounds__(256, 2) void mix_gemm_lds_kernel(const MixGemmArgs 
     const int lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t wn = wave & 1, wr = wave >> 1;
-    // XCD x takes the output panels x, x + 8, ...: one after the other through all row panels; with experts
-    // up to four side by side, so that the rows (few per expert, and each expert has weights of its own) are
-    // fetched into the XCD's L2 once for the four
-    const uint32_t nx = (a.ntiles + 7) / 8, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
-    const uint32_t xcd = blockIdx.x % 8, slot = blockIdx.x / 8, share = (nx + 7) / 8;
-    const uint32_t side = a.group_expert ? (share % 4 == 0 ? 4u : (share % 2 == 0 ? 2u : 1u)) : 1u;
-    // (fewer panels than XCDs: panels and rows dealt out as they come, or most XCDs would stand idle)
-    const bool few = nx < 8;
-    const uint32_t px = few ? blockIdx.x % nx : (slot / (ny * side) * side + slot % side) * 8 + xcd;
-    const uint32_t py = few ? blockIdx.x / nx : slot / side % ny, z = blockIdx.y;
-    if (px >= nx) return;
+    const uint32_t nx = (a.ntiles + 7) / 8, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS), z = blockIdx.y;
+    uint32_t px, py;
+    if (!a.group_expert) {
+        if (!xcd_tile(blockIdx.x, a.cols, nx, ny, px, py)) return;
+    } else {
+        // XCD x takes the output panels x, x + 8, ...: up to four side by side through all row panels, so that the rows
+        // (few per expert, and each expert has weights of its own) are fetched into the XCD's L2 once for the four
+        const uint32_t xcd = blockIdx.x % 8, slot = blockIdx.x / 8, share = (nx + 7) / 8;
+        const uint32_t side = share % 4 == 0 ? 4u : (share % 2 == 0 ? 2u : 1u);
+        // (fewer panels than XCDs: panels and rows dealt out as they come, or most XCDs would stand idle)
+        const bool few = nx < 8;
+        px = few ? blockIdx.x % nx : (slot / (ny * side) * side + slot % side) * 8 + xcd;
+        py = few ? blockIdx.x / nx : slot / side % ny;
+        if (px >= nx) return;
+    }
     const uint32_t nt_wg = px * 8, g_wg = py * 2 * GROUPS;
     uint32_t mat = z;
     if (a.group_expert) {

@@ -427,6 +427,7 @@ struct ProjArgs {
     float* y;                // [R][ldy]
     uint32_t N, K, R, ldy;
     uint32_t ksplit;         // waves of a workgroup that share one run of outputs: 1, 2 or 4
+    uint32_t cols;           // proj_gemm_lds_kernel: XCDs that share out the outputs (xcd_tile)
     int gate;                // GATED kernels: kProjSrcSwiglu or kProjSrcGeglu
 };
 
@@ -1262,15 +1263,9 @@ __global__ __launch_bounds__(128 * WN * KS, (WN == 2 && KS == 1) ? 2 : 1) void p
     const uint32_t ktiles_row = a.K / 32, ntiles = a.N / 16, ngroups = (a.R + 7) / 8;
     const uint32_t ktiles = ktiles_row / KS, kfirst = kh * ktiles;    // this set's k-steps
     const uint32_t klast = ktiles - 1;
-    // Workgroup -> tile.  The dispatcher deals consecutive workgroups round-robin
-    // to the eight XCDs; XCD x takes the output panels x, x + 8, ..., and runs
-    // through all row panels of one before the next, so the workgroups resident
-    // on an XCD at one time share a few weight panels (fetched once into its L2)
-    // and the fragments of all rows.
     const uint32_t nx = (ntiles + WN * NT - 1) / (WN * NT), ny = (ngroups + 2 * GROUPS - 1) / (2 * GROUPS);
-    const uint32_t xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const uint32_t px = (slot / ny) * 8 + xcd, py = slot % ny;
-    if (px >= nx) return;                                 // the grid is padded to eight equal shares
+    uint32_t px, py;
+    if (!xcd_tile(blockIdx.x, a.cols, nx, ny, px, py)) return;
     const uint32_t nt_wg = px * WN * NT, g_wg = py * 2 * GROUPS;
     const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)gemm_smem);
 

@@ -784,12 +784,21 @@ void launch_proj_gemm_split(const ProjArgs& a, uint32_t groups)
                 dim3((a.N / 16 + NT - 1) / NT, (groups + GROUPS - 1) / GROUPS), dim3(kProjThreads), a);
 }
 
+// `per_xcd`: workgroups an XCD holds at once
+template <int GROUPS, int WN, int RING, bool PIPE, int KS>
+void launch_proj_lds(ProjArgs a, uint32_t groups, uint32_t per_xcd)
+{
+    uint32_t blocks = 0;
+    a.cols = xcd_cols((a.N / 16 + WN * 4 - 1) / (WN * 4), (groups + 2 * GROUPS - 1) / (2 * GROUPS), (uint64_t)a.N * a.K * 2,
+                      (uint64_t)groups * 8 * a.K * 4, per_xcd, &blocks);
+    launch_main(a.gate ? proj_gemm_lds_kernel<GROUPS, WN, RING, PIPE, KS, true> : proj_gemm_lds_kernel<GROUPS, WN, RING, PIPE, KS>,
+                dim3(blocks), dim3(128 * WN * KS), a, gemm_lds_bytes<GROUPS, WN, RING, KS>());
+}
+
 void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
 {
     const uint32_t nt = a.N / 16, panels = (nt + 7) / 8;
-    // one-dimensional grids: eight equal shares of output panels, times the row panels
-    const uint32_t share = (panels + 7) / 8 * 8;
-    const uint32_t wide = (nt + 15) / 16, wshare = (wide + 7) / 8 * 8;
+    const uint32_t wide = (nt + 15) / 16;
     // The eight-wave tile runs one workgroup per CU, in rounds of 256: when its
     // last round would leave more than 10 % of the CUs idle, the four-wave tile
     // (two per CU, half the work each) loses less (2047 rows x 6144 outputs:
@@ -812,23 +821,18 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
     const bool small_fills_better = n_small >= 512 && n_big * 100 < rounds_b * 512 * 70 &&
                                     (uint64_t)n_small * rounds_b * 100 >= (uint64_t)n_big * rounds_s * 100 + (uint64_t)rounds_b * rounds_s * 512 * 10;
     if (wide_fills)
-        launch_main(a.gate ? proj_gemm_lds_kernel<8, 4, 4, false, 1, true> : proj_gemm_lds_kernel<8, 4, 4>, dim3(wshare * ((groups + 15) / 16)), dim3(512), a,
-                    gemm_lds_bytes<8, 4, 4>());
+        launch_proj_lds<8, 4, 4, false, 1>(a, groups, 32);
     else if (n_big >= 512 && !small_fills_better)
-        launch_main(a.gate ? proj_gemm_lds_kernel<8, 2, 3, false, 1, true> : proj_gemm_lds_kernel<8, 2, 3>, dim3(share * ((groups + 15) / 16)), dim3(kProjThreads), a,
-                    gemm_lds_bytes<8, 2, 3>());
+        launch_proj_lds<8, 2, 3, false, 1>(a, groups, 64);
     else if (panels * ((groups + 7) / 8) >= 512)          // two and more per CU cover each other's latency
-        launch_main(a.gate ? proj_gemm_lds_kernel<4, 2, 3, false, 1, true> : proj_gemm_lds_kernel<4, 2, 3>, dim3(share * ((groups + 7) / 8)), dim3(kProjThreads), a,
-                    gemm_lds_bytes<4, 2, 3>());
+        launch_proj_lds<4, 2, 3, false, 1>(a, groups, 64);
     else if (panels * ((groups + 7) / 8) >= 256 && (a.K / 32) % 2 == 0 && a.K >= 2048)
         // one per CU and a long input range: two sets of waves halve it (two waves per SIMD, half the
         // chain of k-steps; 2047 rows x 2048 -> 1024: 40.3 -> 28.3 us, x 3072 -> 1024: 40 -> 36.6; at
         // 1024 inputs the sum through LDS costs more than the shorter chain gives)
-        launch_main(a.gate ? proj_gemm_lds_kernel<4, 2, 4, true, 2, true> : proj_gemm_lds_kernel<4, 2, 4, true, 2>, dim3(share * ((groups + 7) / 8)), dim3(2 * kProjThreads), a,
-                    gemm_lds_bytes<4, 2, 4, 2>());
+        launch_proj_lds<4, 2, 4, true, 2>(a, groups, 32);
     else if (panels * ((groups + 7) / 8) >= 256)          // one per CU, one wave per SIMD: pipelined reads
-        launch_main(a.gate ? proj_gemm_lds_kernel<4, 2, 4, true, 1, true> : proj_gemm_lds_kernel<4, 2, 4, true>, dim3(share * ((groups + 7) / 8)), dim3(kProjThreads), a,
-                    gemm_lds_bytes<4, 2, 4>());
+        launch_proj_lds<4, 2, 4, true, 1>(a, groups, 32);
     else if (a.gate) {                                    // tiles in pairs: 32 x 8, 32 x 16, 32 x 32
         if (nt / 2 * groups <= 512)
             launch_proj_gemm_split<1, 2, 8, true>(a, groups);

@@ -437,13 +437,16 @@ static int launch_split(const MixGemmArgs& a, uint32_t batch)
 }
 
 template <int GROUPS>
-static int launch_lds(const MixGemmArgs& a, uint32_t batch)
+static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 {
     int rc = allow_lds<mix_gemm_lds_kernel<GROUPS>>(mix_gemm_lds_bytes<GROUPS>());
     if (rc) return rc;
-    const uint32_t nx = (a.ntiles + 7) / 8, share = nx < 8 ? nx : (nx + 7) / 8 * 8;
-    launch_main(mix_gemm_lds_kernel<GROUPS>, dim3(share * ((a.groups + 2 * GROUPS - 1) / (2 * GROUPS)), batch), dim3(256), a,
-                mix_gemm_lds_bytes<GROUPS>());
+    MixGemmArgs a = args;
+    const uint32_t nx = (a.ntiles + 7) / 8, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
+    uint32_t blocks = (nx < 8 ? nx : (nx + 7) / 8 * 8) * ny;
+    if (!a.group_expert)
+        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, 64, &blocks);
+    launch_main(mix_gemm_lds_kernel<GROUPS>, dim3(blocks, batch), dim3(256), a, mix_gemm_lds_bytes<GROUPS>());
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
 }
