@@ -436,17 +436,17 @@ static int launch_split(const MixGemmArgs& a, uint32_t batch)
     return WR_HIP_OK;
 }
 
-template <int GROUPS>
+template <int GROUPS, int KS = 1>
 static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 {
-    int rc = allow_lds<mix_gemm_lds_kernel<GROUPS>>(mix_gemm_lds_bytes<GROUPS>());
+    int rc = allow_lds<mix_gemm_lds_kernel<GROUPS, KS>>(mix_gemm_lds_bytes<GROUPS, KS>());
     if (rc) return rc;
     MixGemmArgs a = args;
     const uint32_t nx = (a.ntiles + 7) / 8, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
     uint32_t blocks = (nx < 8 ? nx : (nx + 7) / 8 * 8) * ny;
     if (!a.group_expert)
-        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, 64, &blocks);
-    launch_main(mix_gemm_lds_kernel<GROUPS>, dim3(blocks, batch), dim3(256), a, mix_gemm_lds_bytes<GROUPS>());
+        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, KS == 2 ? 32 : 64, &blocks);
+    launch_main(mix_gemm_lds_kernel<GROUPS, KS>, dim3(blocks, batch), dim3(256 * KS), a, mix_gemm_lds_bytes<GROUPS, KS>());
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
 }
@@ -455,9 +455,13 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 // NT + GR KiB a k-step through a compute unit's vector cache, workgroup after workgroup; an LDS tile for its barrier
 // and its operands' latency per k-step, or, with several workgroups on a unit, for its share of the matrix pipes.
 // (Measured on one device, 20 to 1000 rows of 2048 and 4096 inputs and more; microseconds per k-step of 32 inputs:
-// 0.018 for a KiB of the one; 0.34, 0.39, 0.58 and 0.18, 0.27, 0.5 for the three of the other.)  What it changed, us
-// before / now: 2048 -> 2048 at 130 rows 9.2 / 7.2, at 300 13.9 / 9.3, at 1000 23.3 / 17.7; 8192 -> 2048 37.6 / 26.7
-// at 300, 80 / 54 at 1000; 12 288 -> 4096 at 300 111 / 68; 2048 -> 14 400 at 45 27 / 15.3.
+// 0.018 for a KiB of the one; 0.34, 0.39, 0.58 and 0.18, 0.27, 0.5 for the three of the other; 0.26 and 0.28 a round
+// of one workgroup per unit where two sets of waves halve a long input range.)  What the register tiles changed, us
+// before / with them: 2048 -> 2048 at 130 rows 9.2 / 7.2, at 300 13.9 / 9.3; 8192 -> 2048 37.6 / 26.7 at 300; 12 288
+// -> 4096 at 300 111 / 68; 2048 -> 14 400 at 45 27 / 15.3.  The halves: 8192 -> 2048 at 1000 rows 80 / 55, at 2047 93
+// / 73; 4096 -> 2048 at 2047 50 / 41; 12 288 -> 4096 at 1000 153 / 108.
+// Over 12 row counts from 20 to 2047 and 8 weights the form picked is 0.5 % off the best one on average (3.5 % before
+// the halves), 21 % at worst.
 static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
 {
     struct Form {
@@ -472,7 +476,8 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
         uint32_t groups;
         float step, share;
         int (*launch)(const MixGemmArgs&, uint32_t);
-    } lds[] = {{4, 0.34f, 0.177f, launch_lds<2>}, {8, 0.39f, 0.27f, launch_lds<4>}, {16, 0.58f, 0.5f, launch_lds<8>}};
+    } lds[] = {{4, 0.34f, 0.177f, launch_lds<2>}, {8, 0.39f, 0.27f, launch_lds<4>}, {16, 0.58f, 0.5f, launch_lds<8>}},
+      halves[] = {{4, 0.26f, 0.f, launch_lds<2, 2>}, {8, 0.28f, 0.f, launch_lds<4, 2>}};
     int (*best)(const MixGemmArgs&, uint32_t) = nullptr;
     float least = 0.f;
     auto offer = [&](float cost, int (*launch)(const MixGemmArgs&, uint32_t)) {
@@ -489,6 +494,11 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
         for (const auto& f : lds) {
             const uint64_t wgs = (uint64_t)((a.ntiles + 7) / 8) * ((a.groups + f.groups - 1) / f.groups) * batch;
             offer(std::max(f.step, f.share * wgs / g.n_cus), f.launch);
+        }
+    if (a.groups >= 4 && a.ktiles % 2 == 0 && a.ktiles >= 64)
+        for (const auto& f : halves) {
+            const uint64_t wgs = (uint64_t)((a.ntiles + 7) / 8) * ((a.groups + f.groups - 1) / f.groups) * batch;
+            offer(f.step * (float)((wgs + g.n_cus - 1) / g.n_cus), f.launch);
         }
     return best(a, batch);
 }
