@@ -221,6 +221,33 @@ def test_every_tile_of_many_rows(lib, N, K, rows):
         b.free()
 
 
+@pytest.mark.parametrize("N,K", [(16, 4096), (2048, 4128), (80, 8192), (2064, 4096), (48, 4064)])
+def test_two_workgroups_to_a_tile(lib, N, K):
+    # narrow weights over long inputs, up to sixteen rows: one tile, as many as a launch holds, an odd number of k-steps;
+    # one tile more and one k-step less, which a single workgroup takes.  A row's bits are its own whatever rows go with
+    # it and whichever workgroup is last, sixteen launches over; every destination.
+    r = Run(lib, False, 1, N, K, 16)
+    x = r.act(16, K)
+    xd, y, y1 = r.up(x), hipattn.DeviceBuffer(16 * N * 4), hipattn.DeviceBuffer(N * 4)
+    want = x.astype(np.float64) @ r.w[0].T.astype(np.float64)
+    r.go(xd, out=ROWS_F32, y_f32=y.p, ldy=N)
+    got = y.to_host((16, N))
+    r.close(got, want)
+    for i in range(16):
+        one = r.up(x[i:i + 1])
+        r.go(one, rows=1, out=ROWS_F32, y_f32=y1.p, ldy=N)
+        assert y1.to_host((N,)).tobytes() == got[i].tobytes(), f"row {i}"
+        one.free()
+    if N % 32 == 0:
+        h = hipattn.DeviceBuffer(16 * N * 2)
+        r.go(xd, out=FRAG, h=h.p, h_kt=N // 32, relu2=1)
+        r.close(r.frag_down(h, 16, N), np.maximum(want, 0) ** 2, eight_bits=True)
+        h.free()
+    r.end()
+    for b in (xd, y, y1):
+        b.free()
+
+
 @pytest.mark.parametrize("N,K,runs_each", [(64, 352, 1), (2080, 96, 1), (64, 352, 3), (2080, 96, 3), (1056, 32, 2)])
 def test_runs_whose_last_groups_hold_no_pair(lib, N, K, runs_each):
     # runs of eight groups per expert, the last one's rest empty, as routing leaves it: few rows an expert and many

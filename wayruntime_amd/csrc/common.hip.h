@@ -226,6 +226,20 @@ __device__ __forceinline__ void lds_barrier()
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// Partial results that another workgroup adds: stored through to memory, read from there
+// (the order around them is set out at publish_and_merge, kernels_decode.hip.h).
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "the cross-workgroup exchange below relies on how gfx950 executes agent-scope relaxed atomics (sc1 write-through stores, L2-coherent loads); it has not been argued for any other target"
+#endif
+__device__ __forceinline__ float part_load(const float* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void part_store(float* p, float v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Which tile a workgroup of a matrix product takes.  The dispatcher deals consecutive
 // workgroups round-robin to the eight XCDs, each with an L2 of its own, so the output
 // panels (nx) are shared out over `cols` of the XCDs and the row panels (ny) over the

@@ -160,18 +160,7 @@ static_assert(sizeof(DecodeArgs::items) == kBatchMax * kMaxSplits * sizeof(uint1
 // compiles to no wait at all here, because the waves of a workgroup share one
 // CU) and a workgroup barrier before one thread takes the ticket.  A
 // device-wide release fence instead would write back the whole L2
-// (buffer_wbl2) from every workgroup: measured at 5-10x the kernel's run time.
-#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
-#error "the cross-workgroup exchange below relies on how gfx950 executes agent-scope relaxed atomics (sc1 write-through stores, L2-coherent loads); it has not been argued for any other target"
-#endif
-__device__ __forceinline__ float part_load(const float* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void part_store(float* p, float v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
+// (buffer_wbl2) from every workgroup: measured at 5-10x the kernel's run time. (part_store, part_load: common.hip.h.)
 
 // Merge of up to N partials per head, everything a thread needs asked for at
 // once: its output element's partial values and the head's (m, l) pairs; the

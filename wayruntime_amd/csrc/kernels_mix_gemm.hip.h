@@ -33,6 +33,8 @@ struct MixGemmArgs {
     float* y;
     void* ya;
     void* h;
+    float* part;                     // PARTS = 2: partial tiles [2][ntiles][64][4]
+    uint32_t* tickets;               // ... one per tile, zero between launches
 };
 
 __global__ __launch_bounds__(256) void mix_pack_kernel(const uint16_t* __restrict__ w, u32x4* __restrict__ tiles,
@@ -152,21 +154,31 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // compute unit's vector cache, NT + GR KiB a k-step for NT x GR products.
 // STREAM: every weight tile is read by one workgroup only (no use in keeping it).
 // With group_expert the GR groups share an expert (GR divides tile_groups).
-template <bool F32, int NT, int GR, int WAVES, int D, bool STREAM>
+//
+// PARTS = 2 (one group of rows, one matrix, no gate): two workgroups take half of the
+// input range each, and the one that draws the tile's second ticket adds the other's
+// partial tile (a sum of two: the same bits either way).  A narrow weight has 128 tiles
+// for 256 compute units, and a unit takes in 46 GB/s of weights and rows at best, so
+// half of them idle is half the rate.  16 rows, weights from HBM: 8192 -> 2048 11.5 -> 9.4
+// us, -> 512 10.6 -> 7.8; 6144 -> 2048 9.4 -> 7.8; 4096 -> 2048 7.0 -> 6.6, -> 1024 6.7 ->
+// 6.0; at 2048 inputs the exchange costs more (4.8 -> 5.2).
+template <bool F32, int NT, int GR, int WAVES, int D, bool STREAM, int PARTS = 1>
 __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_kernel(const MixGemmArgs a)
 {
     using V8 = typename MixAct<F32>::V8;
     __shared__ f32x4 s_part[WAVES * NT * GR * 64];
     const int lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t nt0 = blockIdx.x * NT, group0 = blockIdx.y * GR, z = blockIdx.z;
+    static_assert(PARTS == 1 || (PARTS == 2 && NT == 1 && GR == 1), "one tile, two halves");
+    const uint32_t nt0 = blockIdx.x * NT, group0 = PARTS > 1 ? 0 : blockIdx.y * GR, part = PARTS > 1 ? blockIdx.y : 0, z = blockIdx.z;
     uint32_t mat = z;
     if (a.group_expert) {
         const int e = a.group_expert[group0];
         if (e < 0) return;                                 // uniform over the workgroup
         mat = (uint32_t)e;
     }
-    const uint32_t k_begin = a.ktiles * wave / WAVES, n = a.ktiles * (wave + 1) / WAVES - k_begin;
+    const uint32_t k_begin = a.ktiles * (part * WAVES + wave) / (PARTS * WAVES),
+                   n = a.ktiles * (part * WAVES + wave + 1) / (PARTS * WAVES) - k_begin;
 
     const bf16x8* wp[NT];
     const V8* xp[GR];
@@ -241,6 +253,25 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
         }
         return v;
     };
+    if constexpr (PARTS > 1) {
+        if (wave > 0) return;
+        f32x4 v = sum(0);
+        float* mine = a.part + ((size_t)(part * a.ntiles + nt0) * 64 + lane) * 4;
+#pragma unroll
+        for (int j = 0; j < 4; j++) part_store(mine + j, v[j]);
+        // the stores are acknowledged before the ticket is drawn: who draws the second one reads them
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint32_t ticket = 0;
+        if (lane == 0) ticket = __hip_atomic_fetch_add(&a.tickets[nt0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane(ticket) == 0) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        const float* other = a.part + ((size_t)((1 - part) * a.ntiles + nt0) * 64 + lane) * 4;
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] += part_load(other + j);
+        if (lane == 0) a.tickets[nt0] = 0;
+        mix_store_tile<F32>(a, v, v, nt0, 0, z, lane);
+        return;
+    }
     if (a.out >= kMixOutGated) {
         if constexpr (NT % 2 == 0) {
 #pragma unroll 1

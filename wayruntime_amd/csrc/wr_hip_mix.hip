@@ -436,6 +436,21 @@ static int launch_split(const MixGemmArgs& a, uint32_t batch)
     return WR_HIP_OK;
 }
 
+// Two workgroups to a tile (PARTS), where both halves of all tiles run at once; from 4096 inputs on (figures at the
+// kernel).
+constexpr uint32_t kPartsMinKtiles = 128;
+
+static int launch_parts(MixGemmArgs a)
+{
+    int rc = ensure_device(cx->d_part, (size_t)2 * a.ntiles * 64 * sizeof(f32x4));
+    if (rc) return rc;
+    a.part = static_cast<float*>(cx->d_part.p);
+    a.tickets = cx->d_counters;
+    launch_main(mix_gemm_split_kernel<false, 1, 1, 4, 8, true, 2>, dim3(a.ntiles, 2), dim3(256), a);
+    HIP_TRY(hipGetLastError(), "product launch", 0);
+    return WR_HIP_OK;
+}
+
 template <int GROUPS, int KS = 1>
 static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 {
@@ -585,6 +600,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
         // wide weights share the rows' operand between two tiles; over a short range eight waves, over a long one
         // four with twice the k-steps each (16 rows; us, before / now: 2048 -> 14 400 16.8 / 11.4, -> 32 768
         // 32.7 / 21.6, 4096 -> 24 576 40.4 / 36.0, -> 6144 13.7 / 11.1; narrow ones 4096 -> 4096 8.4 / 7.8)
+        if (!gated && batch == 1 && a.ktiles >= kPartsMinKtiles && a.ntiles * 2 <= g.n_cus) return launch_parts(a);
         if (!gated && a.ntiles * batch < 384) return launch_split<false, 1, 1, 4, 8, true>(a, batch);
         return a.ktiles <= 64 ? launch_split<false, 2, 1, 8, 4, true>(a, batch) : launch_split<false, 2, 1, 4, 8, true>(a, batch);
     }
