@@ -789,7 +789,7 @@ template <int GROUPS, int WN, int RING, bool PIPE, int KS>
 void launch_proj_lds(ProjArgs a, uint32_t groups, uint32_t per_xcd)
 {
     uint32_t blocks = 0;
-    a.cols = xcd_cols((a.N / 16 + WN * 4 - 1) / (WN * 4), (groups + 2 * GROUPS - 1) / (2 * GROUPS), (uint64_t)a.N * a.K * 2,
+    a.cols = (uint8_t)xcd_cols((a.N / 16 + WN * 4 - 1) / (WN * 4), (groups + 2 * GROUPS - 1) / (2 * GROUPS), (uint64_t)a.N * a.K * 2,
                       (uint64_t)groups * 8 * a.K * 4, per_xcd, &blocks);
     launch_main(a.gate ? proj_gemm_lds_kernel<GROUPS, WN, RING, PIPE, KS, true> : proj_gemm_lds_kernel<GROUPS, WN, RING, PIPE, KS>,
                 dim3(blocks), dim3(128 * WN * KS), a, gemm_lds_bytes<GROUPS, WN, RING, KS>());
@@ -1004,8 +1004,8 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     a.K = w->n_in;
     a.R = rows;
     a.ldy = ldy;
-    a.gate = src.gate;
-    a.ksplit = ksplit;
+    a.gate = (uint8_t)src.gate;
+    a.ksplit = (uint8_t)ksplit;
     if (row1) {
         const uint32_t runs = src.gate ? tiles / 2 : tiles;
         const dim3 grid((runs + 4 / ksplit - 1) / (4 / ksplit)), block(kProjThreads);
