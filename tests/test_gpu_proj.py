@@ -463,6 +463,7 @@ def test_rows_whose_workgroups_make_their_own_terms(rows, n_in, n_out):
 
 @pytest.mark.parametrize("rows,n_in,ffn", [
     (1, 1024, 3072), (1, 96, 48), (1, 3104, 8208),                # one row: four waves a pair, none shared, two, an odd count
+    (1, 14816, 32), (1, 14848, 32), (1, 15360, 32), (1, 15392, 32),    # ... 64 KiB of LDS and one unit more, the most, fragments apart
     (2, 512, 16), (16, 1024, 3072), (8, 1536, 2064), (9, 512, 4080),   # workgroups that make their own terms: a pair, two
     (5, 1056, 528), (16, 160, 48), (16, 1024, 16400),             # a wave per pair of tiles, inputs split and not
     (17, 1056, 528), (100, 288, 2064), (200, 1056, 8208),         # register tiles of 32 x 8, 32 x 16, 32 x 32

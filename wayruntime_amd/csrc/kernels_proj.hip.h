@@ -957,6 +957,9 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
         proj_store_tile(a, acc[0], nt0, 0, lane, s_scale, &resid);
 }
 
+// LDS of proj_row1_kernel beside the row's terms: partial tiles, the row's sums, its scale.
+constexpr size_t row1_static_lds(bool gated) { return (gated ? 6 : 3) * 64 * sizeof(f32x4) + 8 * sizeof(float) + sizeof(float); }
+
 template <int SRC, bool GATED = false>
 __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs a, const ProjPrepArgs p)
 {

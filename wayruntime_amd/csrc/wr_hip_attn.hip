@@ -776,6 +776,8 @@ constexpr int kProjGemmMinRows = 17;
 constexpr uint32_t kProjGroupRows = 257;           // from here on the fragments are made by row groups: at 200 rows a
                                                    // workgroup per row is 0.6 to 2.2 us faster, at 300 as fast, at 511 1 us slower
 constexpr size_t kProjRow1MaxLds = 60 * 1024;      // inputs up to 15 360 take the one-row kernel
+static_assert(kProjRow1MaxLds + row1_static_lds(false) <= 64 * 1024, "what a kernel may use without asking");
+static_assert(kProjRow1MaxLds + row1_static_lds(true) <= 160 * 1024, "gated: asked for at init");
 
 template <int GROUPS, int NT, int D, bool GATED = false>
 void launch_proj_gemm_split(const ProjArgs& a, uint32_t groups)
@@ -1152,6 +1154,9 @@ int wr_hip_attn_init(int device)
             if (kernel && e == hipSuccess)
                 e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         };
+        // (a gated row: 6 KiB of partial tiles beside its terms, more than 64 KiB together from 14 848 inputs on)
+        allow_lds(proj_row1_kernel<kProjSrcRmsNorm, true>, kProjRow1MaxLds);
+        allow_lds(proj_row1_kernel<kProjSrcPlain, true>, kProjRow1MaxLds);
         allow_lds(proj_gemm_lds_kernel<8, 2, 3>, gemm_lds_bytes<8, 2, 3>());
         allow_lds(proj_gemm_lds_kernel<8, 2, 3, false, 1, true>, gemm_lds_bytes<8, 2, 3>());
         allow_lds(proj_gemm_lds_kernel<4, 2, 4, true>, gemm_lds_bytes<4, 2, 4>());
