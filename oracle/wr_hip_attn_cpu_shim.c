@@ -282,7 +282,11 @@ void *wr_hip_attn_dev_alloc(size_t bytes)
 void wr_hip_attn_dev_free(void *p) { free(p); }
 int wr_hip_attn_h2d(void *d, const void *s, size_t n) { memcpy(d, s, n); return WR_HIP_OK; }
 int wr_hip_attn_d2h(void *d, const void *s, size_t n) { memcpy(d, s, n); return WR_HIP_OK; }
-int wr_hip_attn_sync(void) { return WR_HIP_OK; }
+/* The k-th wait from now reports what a device error found there would. */
+static int g_fail_wait_in;
+void wr_hip_attn_debug_fail_wait_in(int k);
+void wr_hip_attn_debug_fail_wait_in(int k) { g_fail_wait_in = k; }
+int wr_hip_attn_sync(void) { return g_fail_wait_in > 0 && --g_fail_wait_in == 0 ? WR_HIP_ERR_INTERNAL : WR_HIP_OK; }
 int wr_hip_attn_append_dev(wr_hip_kv *kv, uint32_t layer, uint32_t pos, uint32_t n_rows,
                            const float *k, const float *v)
 {

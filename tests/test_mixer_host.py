@@ -2,6 +2,7 @@
 in place of the device steps, 32-bit): reading and rearranging weights, the cache
 pool, the mixed step, rollback and the error contract, against the plain
 implementation of tests/mixer_oracle.py."""
+import ctypes as C
 import json
 import os
 
@@ -140,6 +141,31 @@ def test_failure_anywhere_changes_nothing(model, made):
     near(lg[1], want[3:5])
     s.close()
     other.close()
+
+
+def test_wait_that_fails_leaves_positions_and_logits(model, made):
+    # the wait behind a step's logits reports an error: sessions keep the logits of the step before, whose rows the
+    # caller still holds, and their positions
+    t = toks(12)
+    ss, fn = [model.session() for _ in range(3)], model.eng.lib.wr_hip_attn_debug_fail_wait_in
+    assert all(s.prefill(t[:5]) == 5 for s in ss)
+    hs, at = (C.c_void_p * 3)(*[s.h for s in ss]), (C.c_uint32 * 3)(1, 2, 3)
+    rows = (C.POINTER(C.c_float) * 3)()
+    assert model.lib.wr_batch_step(hs, at, 3, rows) == 3
+    kept = [np.ctypeslib.as_array(r, shape=(model.vocab,)) for r in rows]
+    before = [k.copy() for k in kept]
+    for single in (False, True):
+        fn(1)
+        if single:
+            assert ss[0].step(9) is None
+        else:
+            assert model.lib.wr_batch_step(hs, (C.c_uint32 * 3)(7, 8, 9), 3, None) == E.WR_ERR_INTERNAL
+        fn(0)
+        assert [s.pos for s in ss] == [6, 6, 6] and ss[0].status == E.WR_ERR_INTERNAL
+        assert all(np.array_equal(a, b) for a, b in zip(kept, before))
+    near(ss[1].step(9)[None], O.forward(CFG, made[1], list(t[:5]) + [2, 9], np.float64)[-1:])
+    for s in ss:
+        s.close()
 
 
 def test_refusals(model):

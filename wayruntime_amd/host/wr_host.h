@@ -205,7 +205,8 @@ typedef struct wrh_logit_rows {
     float *const *rows;
 } wrh_logit_rows;
 /* The sessions are locked and checked; positions advance on success and nothing
- * changes otherwise. */
+ * changes otherwise, logits included where the step wants one row per entry
+ * (portions that want more may have left some of theirs). */
 wr_status wrh_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, const wrh_logit_rows *logits, int fail_run);
 /* Test hook: the residual rows [rows][width] after every layer run of the coming
  * steps are appended to `rows` until `floats` are used up; NULL ends it. */

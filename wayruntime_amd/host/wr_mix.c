@@ -763,31 +763,38 @@ static wr_status walk_layers(wr_model *m, walk *w, bump b, uint32_t R, int fail_
     return WR_OK;
 }
 
-/* Logits of the step's wanted rows, packed in h's rows after the final norm; row i goes to where `dest[i]` is in
- * `out`.  The rows come down in one copy per product and are handed out by as many threads as there are rows worth
- * one (sixteen of 32 768, 2 MB: a step of sixteen sessions 487 -> 441 us, with the copy through a block of the
- * caller's that it replaces). */
-static wr_status walk_logits(wr_model *m, const walk *w, uint32_t n_want, const uint32_t *dest, const wrh_logit_rows *out)
+/* Rows of the page-locked block go to where `dest` is in `out`, by as many threads as there are rows worth one
+ * (sixteen of 32 768, 2 MB: a step of sixteen sessions 487 -> 441 us, with the copy through a block of the caller's
+ * that it replaces). */
+static void hand_out(const wr_model *m, uint32_t n, const uint32_t *dest, const wrh_logit_rows *out)
+{
+    const struct wrh_mix_model *mm = m->mix;
+    const int threads = (m->engine && m->engine->n_threads > 0) ? m->engine->n_threads : 1;
+#pragma omp parallel for num_threads(threads) schedule(static) if (n >= 4 && m->vocab >= 8192)
+    for (uint32_t i = 0; i < n; i++)
+        memcpy(out->rows ? out->rows[dest[i]] : out->block + (size_t)dest[i] * m->vocab, mm->logits_host + (size_t)i * mm->vocab_p,
+               (size_t)m->vocab * sizeof(float));
+}
+
+/* Logits of the step's wanted rows, packed in h's rows after the final norm; row i belongs where `dest[i]` is in
+ * `out`.  The rows come down in one copy per product.  The last product's, all there are in a step of single tokens,
+ * stay in the block for the caller to hand out once the step is known to have worked; *rest is how many. */
+static wr_status walk_logits(wr_model *m, const walk *w, uint32_t n_want, const uint32_t *dest, const wrh_logit_rows *out,
+                             uint32_t *rest)
 {
     struct wrh_mix_model *mm = m->mix;
     const uint32_t r = mm->n_runs, wkt = mm->width_p / 32;
     const size_t e = mm->f32 ? 4 : 2;
     const wr_hip_mix_resid fin = {.width = mm->width, .eps = mm->eps, .x = w->x, .next = mm->final_norm, .wanted = 1, .h = w->h};
     TRY(wr_hip_mix_residual(mm->step, mm->f32, &fin), "final norm");
-    for (uint32_t at = 0; at < n_want; at += WRH_MIX_LOGIT_ROWS) {
-        const uint32_t n = n_want - at < WRH_MIX_LOGIT_ROWS ? n_want - at : WRH_MIX_LOGIT_ROWS;
+    for (uint32_t at = 0; at < n_want; at += *rest) {
+        if (at) hand_out(m, *rest, dest + at - *rest, out);
+        *rest = n_want - at < WRH_MIX_LOGIT_ROWS ? n_want - at : WRH_MIX_LOGIT_ROWS;
         const uint8_t *x = (const uint8_t *)w->h + (size_t)at * mm->width_p * e;      /* whole groups of 16 rows */
-        const wr_hip_mix_gemm head = {.w = mm->head, .x = x, .x_kt = wkt, .rows = n, .out = WR_HIP_MIX_OUT_ROWS_F32,
+        const wr_hip_mix_gemm head = {.w = mm->head, .x = x, .x_kt = wkt, .rows = *rest, .out = WR_HIP_MIX_OUT_ROWS_F32,
                                       .y_f32 = mm->logits_dev, .ldy = mm->vocab_p, .scale = mm->logit_scale};
         TRY(wr_hip_mix_gemm_run(mm->f32, &head), "head");
-        TRY(wr_hip_attn_d2h(mm->logits_host, mm->logits_dev, (size_t)n * mm->vocab_p * sizeof(float)), "logits down");
-        const int threads = (m->engine && m->engine->n_threads > 0) ? m->engine->n_threads : 1;
-#pragma omp parallel for num_threads(threads) schedule(static) if (n >= 4 && m->vocab >= 8192)
-        for (uint32_t i = 0; i < n; i++) {
-            const uint32_t d = dest[at + i];
-            memcpy(out->rows ? out->rows[d] : out->block + (size_t)d * m->vocab, mm->logits_host + (size_t)i * mm->vocab_p,
-                   (size_t)m->vocab * sizeof(float));
-        }
+        TRY(wr_hip_attn_d2h(mm->logits_host, mm->logits_dev, (size_t)*rest * mm->vocab_p * sizeof(float)), "logits down");
     }
     return WR_OK;
 }
@@ -852,7 +859,7 @@ wr_status wrh_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, co
     while (left && st == WR_OK) {
         /* the rows of this pass: as much of each entry as fits, in order */
         wr_hip_mix_seq seqs[WR_BATCH_MAX];
-        uint32_t at[WR_BATCH_MAX], n_seq = 0, R = 0, row0 = 0, n_want = 0;
+        uint32_t at[WR_BATCH_MAX], n_seq = 0, R = 0, row0 = 0, n_want = 0, rest = 0;
         for (uint32_t i = 0; i < n && R < longest; i++) {
             const wr_step_entry *q = &entries[i];
             wrh_mix_session *ms = q->session->mix;
@@ -897,10 +904,11 @@ wr_status wrh_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, co
         bump b = {mm->scratch, 0};
         walk w = take_walk(&b, mm, R);
         st = walk_layers(m, &w, b, R, fail_run);
-        if (st == WR_OK && n_want) st = walk_logits(m, &w, n_want, dest, logits);
+        if (st == WR_OK && n_want) st = walk_logits(m, &w, n_want, dest, logits, &rest);
         /* the step's descriptors are in page-locked memory: they are free again after the wait */
         const int sync = wr_hip_attn_sync();
         if (st == WR_OK && sync != WR_HIP_OK) st = op_fail(m, "sync", mm->n_runs, sync);
+        if (st == WR_OK) hand_out(m, rest, dest + n_want - rest, logits);
         for (s = 0; s < n_seq; s++) done[at[s]] += seqs[s].rows;
         left -= R;
     }
