@@ -353,7 +353,9 @@ int wr_hip_proj_rows(const wr_hip_weight *w, uint32_t rows, const float *x,
 /* Device-resident form, asynchronous on the stream: row strides ldx >=
  * n_in and ldy >= n_out (ldy a multiple of 4, y_dev 16-byte aligned);
  * add_dev, if not NULL, is [rows][ldy] and is added to the product (the
- * residual add that follows wo, src/core/session.c:505-506). */
+ * residual add that follows wo, src/core/session.c:505-506).  y_dev may be
+ * add_dev, and may overlap x_dev as long as rows <= 4096 (so may the outputs of
+ * the forms below). */
 int wr_hip_proj_rows_dev(const wr_hip_weight *w, uint32_t rows,
                          const float *x_dev, uint32_t ldx,
                          const float *add_dev, float *y_dev, uint32_t ldy);

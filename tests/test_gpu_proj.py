@@ -511,6 +511,41 @@ def test_gates_and_values_in_one_product_equal_product_then_activation(rows, n_i
             h.close()
 
 
+@pytest.mark.parametrize("rows", [1, 2, 16, 20])
+@pytest.mark.parametrize("n", [1024, 4096])
+def test_result_over_its_own_input(rows, n):
+    # every source, written over the rows it came from: the bits of the result beside them
+    lib, D, eps = hipattn.lib(), hipattn.DeviceBuffer, 1e-6
+    print("in place", rows, n, flush=True)
+    x, two = synth.normal(231, (rows, n), std=2.0), synth.normal(232, (rows, 2 * n), std=2.0)
+    nw = D.from_host(synth.normal(233, (n,)) * np.float32(0.2) + np.float32(1.0))
+    w, wg = hipattn.Weight([_w16(234, n, n, 0.1)]), hipattn.Weight([_w16(235, n, n, 0.1), _w16(236, n, n, 0.1)])
+    for form in ("plain", "norm", "gated", "gated norm", "swiglu"):
+        src = two if form == "swiglu" else x
+        xd, y = D.from_host(src), D(rows * 2 * n * 4)
+
+        def run(to, ld):
+            if form == "plain":
+                return lib.wr_hip_proj_rows_dev(w.h, rows, xd.p, n, None, to, ld)
+            if form == "norm":
+                return lib.wr_hip_proj_rows_norm_dev(w.h, rows, xd.p, n, nw.p, eps, None, to, ld)
+            if form == "swiglu":
+                return lib.wr_hip_proj_rows_swiglu_dev(w.h, rows, xd.p, 2 * n, None, to, ld)
+            return lib.wr_hip_proj_rows_gated_dev(wg.h, rows, xd.p, n, nw.p if "norm" in form else None, eps, 0, to, ld)
+
+        ld = src.shape[1]
+        assert run(y.p, ld) == hipattn.OK
+        want = y.to_host((rows, ld))[:, :n].copy()
+        at = n if form == "swiglu" else 0                  # (over the second half, the gated values)
+        assert run(xd.p + at * 4, ld) == hipattn.OK
+        assert xd.to_host((rows, ld))[:, at:at + n].tobytes() == want.tobytes(), form
+        for d in (xd, y):
+            d.free()
+    nw.free()
+    w.close()
+    wg.close()
+
+
 def test_gated_product_refuses_an_odd_number_of_tiles():
     w = hipattn.Weight([_w16(226, 48, 64, 0.1)])
     b = hipattn.DeviceBuffer(4096)

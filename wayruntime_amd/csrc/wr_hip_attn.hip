@@ -919,8 +919,13 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     const uint32_t groups = (rows + 7) / 8;                // row groups of eight
     const bool gemm = rows >= (uint32_t)kProjGemmMinRows;
     const uint32_t ktiles = w->n_in / 32;
+    // The kernels that make the operand terms themselves read the rows while others already write results.
+    const uint32_t x_cols = src.kind == kProjSrcSwiglu || src.kind == kProjSrcGeglu ? 2 * w->n_in : w->n_in;
+    const uint32_t y_cols = src.gate ? w->n_out / 2 : w->n_out;
+    const uintptr_t x0 = (uintptr_t)x_dev, y0 = (uintptr_t)y_dev;
+    const bool apart = x0 + ((size_t)(rows - 1) * ldx + x_cols) * 4 <= y0 || y0 + ((size_t)(rows - 1) * ldy + y_cols) * 4 <= x0;
     // one row: the fragment step runs inside the product's kernel (4 bytes of LDS per input)
-    const bool row1 = rows == 1 && (size_t)w->n_in * 4 <= kProjRow1MaxLds;
+    const bool row1 = rows == 1 && apart && (size_t)w->n_in * 4 <= kProjRow1MaxLds;
     // Waves that share a run of outputs (contiguous parts of the inputs, summed
     // through LDS in a fixed order): enough that a narrow weight still gives
     // one to two thousand waves.  A function of the weight's shape only: a row's
@@ -936,11 +941,8 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
             ksplit *= 2;
     }
     // up to a few dozen rows, where one workgroup per CU can take them all: so does each workgroup of the product.  It
-    // reads the rows with 16-byte loads, and while others already write results.
+    // reads the rows with 16-byte loads.
     // (Four waves to the inputs, as the kernel of one row then has: a row's bits are its own in a step of up to sixteen.)
-    const uint32_t y_cols = src.gate ? w->n_out / 2 : w->n_out;
-    const uintptr_t x0 = (uintptr_t)x_dev, y0 = (uintptr_t)y_dev;
-    const bool apart = x0 + ((size_t)(rows - 1) * ldx + w->n_in) * 4 <= y0 || y0 + ((size_t)(rows - 1) * ldy + y_cols) * 4 <= x0;
     uint32_t fused_nt = 0;
     const FusedKernel fused =
         rows > 1 && rows < kProjGroupRows && (gemm || ksplit == 4) && ldx % 4 == 0 && ((x0 | (uintptr_t)src.norm_w) & 15) == 0 && apart
