@@ -186,7 +186,11 @@ int wr_hip_attn_append_decode_batched(uint32_t n, wr_hip_kv *const *kv,
  * Replaces the loop of seq_q = 1 attention calls that prefill runs
  * (src/core/session.c:615-625): rows p0 .. p0+T-1 have already been appended;
  * row i of q [T, nq, hd_layer] attends keys 0 .. p0+i (with `window` > 0, the
- * last `window` of those).  out is host F32 [T, nq, hd_layer]. */
+ * last `window` of those).  out is host F32 [T, nq, hd_layer].  A row's sums
+ * are taken in an order that depends on the call's sizes: few rows over many
+ * keys are worked on in parts that are added at the end, in their order.  So
+ * equal calls give equal bits, and a prompt cut into other portions gives the
+ * same rows to rounding (see wr_hip_attn_set_prefill_part_mb). */
 int wr_hip_attn_prefill(wr_hip_kv *kv, uint32_t layer, uint32_t p0,
                         uint32_t T, const float *q, float *out, uint32_t nq,
                         float scale_override, uint32_t window);
@@ -480,6 +484,14 @@ void wr_hip_attn_set_tuning(uint32_t decode_keys_per_wg, int force_generic);
  * waves, one per SIMD, two units per wave.  Same results to rounding; the
  * second form is kept for comparison and is the slower one at present. */
 void wr_hip_attn_set_prefill_one_wave(int on);
+
+/* The memory that parts of long prefill blocks may take, per calling thread: at
+ * most `mb` MiB (128, the default, is also the most; WR_HIP_PREFILL_PART_MB at
+ * init sets it too).  A thread's buffer grows to the largest launch that was cut
+ * (a power of two of MiB) and is kept until shutdown; where the device has no
+ * room for it, launches go uncut.  0: no launch is cut, so the bits of a row do
+ * not depend on the portion it came in. */
+void wr_hip_attn_set_prefill_part_mb(uint32_t mb);
 
 /* Kernel timing for the roofline figure.  Between profile_begin and
  * profile_end every launch of the MAIN kernel of a call (the split-K decode

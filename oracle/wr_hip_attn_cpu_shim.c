@@ -272,6 +272,7 @@ int wr_hip_attn_prefill(wr_hip_kv *kv, uint32_t layer, uint32_t p0, uint32_t T, 
 uint32_t wr_hip_attn_caps(void) { return 0; }
 void wr_hip_attn_set_tuning(uint32_t keys_per_wg, int force_generic) { (void)keys_per_wg; (void)force_generic; }
 void wr_hip_attn_set_prefill_one_wave(int on) { (void)on; }
+void wr_hip_attn_set_prefill_part_mb(uint32_t mb) { (void)mb; }
 /* "device" memory is host memory here, filled with NaN bit patterns: what nobody wrote shows when it is used */
 void *wr_hip_attn_dev_alloc(size_t bytes)
 {

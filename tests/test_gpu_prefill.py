@@ -238,6 +238,48 @@ def test_few_rows_over_many_keys_sampled_rows(nq, nkv, hd, p0, T, win):
     kv.close()
 
 
+def test_parts_take_a_bounded_buffer_of_their_own():
+    # 177 rows of 32 x 128 in five parts are 14.7 MB: a calling thread that cuts them takes 16 MiB for it, no more, and
+    # nothing when it may take none.  Then no launch is cut, and a prompt's rows have the same bits in any portions.
+    import ctypes as C
+    import threading
+    nq, nkv, hd, p0, T = 32, 8, 128, 8192, 177
+    kv, q, _k16, _v16 = _setup(nq, nkv, hd, p0, T, seed=6100)
+    free, total, hip, lib = C.c_size_t(), C.c_size_t(), C.CDLL("libamdhip64.so"), hipattn.lib()
+    qd, out, taken, rows = hipattn.DeviceBuffer.from_host(q), hipattn.DeviceBuffer(q.nbytes), [], []
+
+    def left():
+        hipattn.sync()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    def run(mb, cuts):
+        hipattn.set_prefill_part_mb(mb)
+        at, before = 0, left()
+        for n in cuts:
+            o = at * nq * hd * 4
+            assert lib.wr_hip_attn_prefill_dev(kv.h, 0, p0 + at, n, qd.p + o, out.p + o, nq, 0.0, 0) == hipattn.OK
+            at += n
+        taken.append(before - left())
+        rows.append(out.to_host((T, nq, hd)))
+
+    def work():
+        for mb, cuts in ((0, [T]), (0, [64, 1, 112]), (128, [T]), (128, [T])):
+            run(mb, cuts)
+
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    hipattn.set_prefill_part_mb()
+    print("bytes taken", taken, flush=True)
+    assert len(taken) == 4 and taken[0] == taken[1] == taken[3] == 0 and taken[2] <= 17 << 20
+    assert np.array_equal(rows[0], rows[1]) and np.array_equal(rows[2], rows[3])
+    util.assert_close(rows[2], rows[0])
+    for b in (qd, out):
+        b.free()
+    kv.close()
+
+
 @pytest.mark.parametrize("every", [1, 3])
 @pytest.mark.parametrize("nq,nkv,hd,p0", [(16, 8, 256, 0), (8, 4, 256, 70), (32, 8, 128, 0), (4, 2, 64, 0)])
 def test_prefill_with_a_softmax_reference_that_moves_from_tile_to_tile(nq, nkv, hd, p0, every):

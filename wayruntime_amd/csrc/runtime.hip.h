@@ -16,6 +16,9 @@
 namespace wr {
 
 constexpr int kMaxDevices = 16;
+constexpr uint32_t kMaxPrefillParts = 32;    // prefill: parts a block's keys are cut into at most,
+constexpr uint32_t kMaxPrefillPartMb = 128;  // and the MiB that the parts' rows take
+constexpr uint32_t kPrefillRefusedLaunches = 1000;
 
 struct Buffer {
     void* p = nullptr;
@@ -30,6 +33,8 @@ struct Ctx {
     hipStream_t stream = nullptr;
     Buffer d_stage;              // device staging for host-pointer entry points
     Buffer d_part;               // split-K partials
+    Buffer d_prefill;            // rows of prefill blocks cut into parts: at most kMaxPrefillPartMb, none where it is refused
+    uint32_t prefill_refused = 0;     // launches that go uncut before memory for them is asked for again
     Buffer d_proj;               // projection operand fragments and row scales
     uint32_t* d_counters = nullptr;   // split-K tickets, zero whenever no launch is in flight
     // Error word: page-locked host memory that kernels can write.  A kernel that
@@ -67,6 +72,7 @@ struct Lib {
     void* log_user = nullptr;
     std::atomic<uint32_t> tune_keys_per_wg{0};
     std::atomic<int> force_generic{0};
+    std::atomic<uint32_t> prefill_part_mb{kMaxPrefillPartMb};    // WR_HIP_PREFILL_PART_MB: a thread's parts take no more; 0: no block is cut
     std::atomic<int> prefill_256_four_waves{0};   // WR_HIP_PREFILL_256_FOUR_WAVES=1: head dim 256 keeps the earlier four-wave prefill kernel
     std::atomic<int> prefill_two_waves{1};        // WR_HIP_PREFILL_TWO_WAVES=0: head dim 128 takes the one-wave-per-SIMD prefill kernel
 };
@@ -78,8 +84,6 @@ extern thread_local Ctx* cx;
 constexpr uint32_t kDevErrLayerMask = 0x0000FFFFu;     // error word: bit 31 set (kDevErrWaitExpired), the layer in the low bits
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr uint32_t kDefaultTilesPerWg = 32;  // split-K decode: 1024 keys per workgroup
-constexpr uint32_t kMaxPrefillParts = 32;    // prefill: parts a block's keys are cut into at most,
-constexpr float kMaxPrefillPartMb = 128.f;   // and the bytes of the parts' rows
 constexpr uint32_t kMaxHeads = 4096;        // query heads per session the ticket array is sized for
 constexpr size_t kPinSmall = 1u << 20;      // host copies up to this size go through pinned staging
 

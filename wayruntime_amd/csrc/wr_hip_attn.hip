@@ -526,13 +526,15 @@ uint32_t prefill_parts(const PrefillArgs& a, uint32_t BP, uint32_t nblk, uint32_
 {
     const float ends = 8.f, step = a.hd == 256 ? 0.95f : 0.8f, combine = 5.f;
     const float row_mb = (float)a.T * a.nq * a.hd * 4e-6f;
+    const uint64_t row_bytes = (uint64_t)a.T * a.nq * (a.hd + 2) * 4;
+    const uint64_t room = (uint64_t)g.prefill_part_mb.load(std::memory_order_relaxed) << 20;
     const uint32_t last_lo = a.p0 + (nblk - 1) * BP, hi = a.p0 + a.T;          // the last block's first position, keys
     const uint32_t lo = (a.window > 0 && last_lo + 1 > a.window) ? last_lo + 1 - a.window : 0;
     const uint32_t tiles = (hi + kTileKeys - 1) / kTileKeys - lo / kTileKeys, per_step = a.hd == 256 ? 1 : 2;
     uint32_t best = 1;
     float least = 0.f;
     for (uint32_t p = 1; p <= kMaxPrefillParts; p++) {
-        if (p > 1 && p * row_mb > kMaxPrefillPartMb) break;
+        if (p > 1 && p * row_bytes > room) break;
         const uint32_t rounds = (nblk * ny * p + g.n_cus - 1) / g.n_cus;
         const uint32_t steps = ((tiles + p - 1) / p + per_step - 1) / per_step;
         float t = rounds * (ends + step * steps);
@@ -545,17 +547,39 @@ uint32_t prefill_parts(const PrefillArgs& a, uint32_t BP, uint32_t nblk, uint32_
     return best;
 }
 
-// Room for the parts' rows in the thread's partial buffer.  False: there is none, and the launch goes uncut.
+// Room for the parts' rows, in a buffer of their own: a launch can do without them, so nothing another launch must have
+// is given up to make it, and a refusal is no error.  A power of two of MiB; the old one goes only when the new one is
+// there.  False: there is none, and the launch goes uncut (as do the next ones: asking costs a failed call each time).
 bool prefill_parts_ready(PrefillArgs& a, uint32_t parts)
 {
-    const size_t rows = (size_t)parts * a.T * a.nq, o = rows * a.hd * sizeof(float);
-    if (ensure_device(cx->d_part, o + rows * 2 * sizeof(float)) != WR_HIP_OK) {
-        (void)hipGetLastError();
-        return false;
+    const size_t rows = (size_t)parts * a.T * a.nq, o = rows * a.hd * sizeof(float), need = o + rows * 2 * sizeof(float);
+    if (need > cx->d_prefill.cap) {
+        if (cx->prefill_refused) {
+            cx->prefill_refused--;
+            return false;
+        }
+        size_t want = (size_t)1 << 20;
+        while (want < need) want *= 2;
+        void* bigger = nullptr;
+        if (hipMalloc(&bigger, want) != hipSuccess) {
+            (void)hipGetLastError();
+            logmsg(1, "prefill: no %zu MiB for parts of long blocks; they go uncut", want >> 20);
+            cx->prefill_refused = kPrefillRefusedLaunches;
+            return false;
+        }
+        if (cx->d_prefill.p) {                     // launches that use it may still be on their way
+            if (hipStreamSynchronize(cx->stream) != hipSuccess) {
+                (void)hipFree(bigger);
+                return false;
+            }
+            (void)hipFree(cx->d_prefill.p);
+        }
+        cx->d_prefill.p = bigger;
+        cx->d_prefill.cap = want;
     }
     a.n_parts = parts;
-    a.part_o = reinterpret_cast<float*>(cx->d_part.p);
-    a.part_ml = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(cx->d_part.p) + o);
+    a.part_o = reinterpret_cast<float*>(cx->d_prefill.p);
+    a.part_ml = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(cx->d_prefill.p) + o);
     return true;
 }
 
@@ -661,6 +685,7 @@ void ctx_destroy(Ctx* c)
     for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
     if (c->d_stage.p) (void)hipFree(c->d_stage.p);
     if (c->d_part.p) (void)hipFree(c->d_part.p);
+    if (c->d_prefill.p) (void)hipFree(c->d_prefill.p);
     if (c->d_proj.p) (void)hipFree(c->d_proj.p);
     if (c->d_counters) (void)hipFree(c->d_counters);
     if (c->h_pin.p) (void)hipHostFree(c->h_pin.p);
@@ -1098,6 +1123,8 @@ int wr_hip_attn_init(int device)
     {
         const char* e = getenv("WR_HIP_PREFILL_TWO_WAVES");
         g.prefill_two_waves = (e && e[0] == '0') ? 0 : 1;
+        e = getenv("WR_HIP_PREFILL_PART_MB");
+        g.prefill_part_mb = e && e[0] ? (uint32_t)std::min(strtoul(e, nullptr, 10), (unsigned long)kMaxPrefillPartMb) : kMaxPrefillPartMb;
         e = getenv("WR_HIP_PREFILL_256_FOUR_WAVES");
         g.prefill_256_four_waves = (e && e[0] == '1') ? 1 : 0;
     }
@@ -1209,6 +1236,8 @@ uint64_t wr_hip_attn_calls(void) { return g.calls.load(std::memory_order_relaxed
 const char* wr_hip_attn_device_name(void) { return g.name; }
 
 uint32_t wr_hip_attn_caps(void) { return WR_HIP_CAP_PROJ; }
+
+void wr_hip_attn_set_prefill_part_mb(uint32_t mb) { g.prefill_part_mb = std::min(mb, kMaxPrefillPartMb); }
 
 void wr_hip_attn_set_prefill_one_wave(int on)
 {
