@@ -88,7 +88,7 @@ class Run:
 
 
 # (outputs, inputs, rows): what each picks among the streaming kernels and the three LDS-staged tiles
-SHAPES = [(16, 32, 1), (48, 96, 7), (32, 416, 16), (4096, 64, 3), (80, 4096, 16), (64, 64, 17), (96, 160, 33), (160, 96, 70),
+SHAPES = [(16, 32, 1), (48, 800, 5), (64, 1504, 16), (6400, 736, 9), (48, 96, 7), (32, 416, 16), (4096, 64, 3), (80, 4096, 16), (64, 64, 17), (96, 160, 33), (160, 96, 70),
           (1024, 512, 200), (8192, 96, 256), (16384, 64, 250), (16384, 64, 600), (2064, 352, 1100)]
 
 
@@ -197,11 +197,12 @@ def test_batch_of_matrices(lib, f32, batch, N, K, rows):
 
 # every tile the rule picks among: register tiles of 1 x 1, 1 x 2, 2 x 2, 2 x 3, 2 x 4, 4 x 3, 4 x 4 (outputs x rows,
 # sixteens; gated outputs take even ones), LDS tiles of 64, 128 and 256 rows.  Input ranges that leave waves without
-# k-steps (96) and that split unevenly with a rest behind whole turns (1056), and two that two sets of waves halve, an
+# k-steps (96), that are less than a turn of eight and a turn and a rest of four (800), and that split unevenly with
+# a rest behind whole turns (1056), and two that two sets of waves halve, an
 # odd number of k-steps each and an even one (2112, 2176; tiles of 64 and 128 rows).
 @pytest.mark.parametrize("N,rows,K", [(n, r, k) for n, r in [(48, 17), (1088, 50), (1088, 130), (2112, 100), (2816, 100),
                                                              (2112, 300), (6208, 100), (6208, 511), (12352, 511),
-                                                             (12352, 700)] for k in (96, 1056)] +
+                                                             (12352, 700)] for k in (96, 800, 1056)] +
                          [(2112, 700, 2112), (2112, 1100, 2112), (2112, 1100, 2176), (2112, 700, 2176)])
 def test_every_tile_of_many_rows(lib, N, K, rows):
     r = Run(lib, False, 1, N, K, rows)

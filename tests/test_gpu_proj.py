@@ -368,6 +368,9 @@ def test_projection_random_shapes():
     (48, 2080, 16),               # 16 x 8 tiles: one output tile
     (17, 1056, 2720),             # ... 510 of them, the last row group of one row
     (31, 32, 48),                 # ... a single input tile: three waves with none
+    (31, 800, 48),                # ... 25: six and seven k-steps a wave, less than a turn
+    (49, 800, 4112),              # the same in 32 x 16 tiles,
+    (250, 800, 4112),             # and in 32 x 32 tiles
     (49, 1056, 4112),             # 32 x 16 tiles: a last row group of one row, partial output tiles
     (256, 3104, 80),              # ... the last row count whose fragments are made row by row
     (256, 3072, 80),              # (each workgroup makes its own)

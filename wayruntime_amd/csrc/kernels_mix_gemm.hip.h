@@ -148,8 +148,11 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // part of the input range each; their sums meet in LDS and are added in wave order,
 // every wave adding and storing its share of the tiles.  A wave keeps D k-steps on
 // their way (operands from HBM are one to three microseconds away under load):
-// loads stand behind the products that free their registers, and only whole turns
-// of D are loaded ahead, so the compiler's count of loads in flight is exact.
+// loads stand behind the products that free their registers; in whole turns of D
+// none is conditional, so the compiler's count of loads in flight is exact, and what
+// is left behind the last turn is asked for all at once (in registers of its own name:
+// kept in those of the turns, the compiler holds both).  One after the other they were a
+// trip to memory each: 16 rows, 768 -> 2048 5.5 us, 3.9 now; 1536 -> 512 5.5, 4.2.
 // Few rows: bound by the weights' bytes.  More rows: by the bytes that pass a
 // compute unit's vector cache, NT + GR KiB a k-step for NT x GR products.
 // STREAM: every weight tile is read by one workgroup only (no use in keeping it).
@@ -205,37 +208,43 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
 
     bf16x8 w[D][NT];
     V8 x[D][GR];
-    auto load = [&](int d, uint32_t k) {
+    auto load = [&](bf16x8 (&wv)[NT], V8 (&xv)[GR], uint32_t k) {
 #pragma unroll
         for (int t = 0; t < NT; t++)
-            w[d][t] = STREAM ? __builtin_nontemporal_load(&wp[t][k * 64 + lane]) : wp[t][k * 64 + lane];
+            wv[t] = STREAM ? __builtin_nontemporal_load(&wp[t][k * 64 + lane]) : wp[t][k * 64 + lane];
 #pragma unroll
-        for (int i = 0; i < GR; i++) x[d][i] = xp[i][k * 64 + x_lane];
+        for (int i = 0; i < GR; i++) xv[i] = xp[i][k * 64 + x_lane];
     };
-    auto multiply = [&](int d) {
+    auto multiply = [&](const bf16x8 (&wv)[NT], const V8 (&xv)[GR]) {
 #pragma unroll
         for (int i = 0; i < GR; i++)
 #pragma unroll
-            for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(w[d][t], x[d][i], acc[t][i]);
+            for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(wv[t], xv[i], acc[t][i]);
     };
-    const uint32_t turns = n / D;
+    const uint32_t turns = n / D, rest = n - turns * D;
     if (turns) {
 #pragma unroll
-        for (int d = 0; d < D; d++) load(d, d);
+        for (int d = 0; d < D; d++) load(w[d], x[d], d);
         for (uint32_t turn = 1; turn < turns; turn++) {
 #pragma unroll
             for (int d = 0; d < D; d++) {
-                multiply(d);
-                load(d, turn * D + d);
+                multiply(w[d], x[d]);
+                load(w[d], x[d], turn * D + d);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
 #pragma unroll
-        for (int d = 0; d < D; d++) multiply(d);
+        for (int d = 0; d < D; d++) multiply(w[d], x[d]);
     }
-    for (uint32_t k = turns * D; k < n; k++) {
-        load(0, k);
-        multiply(0);
+    if (rest) {
+        bf16x8 wr[D - 1][NT];
+        V8 xr[D - 1][GR];
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+            if ((uint32_t)d < rest) load(wr[d], xr[d], turns * D + d);
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+            if ((uint32_t)d < rest) multiply(wr[d], xr[d]);
     }
 
 #pragma unroll

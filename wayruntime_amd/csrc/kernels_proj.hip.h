@@ -1158,8 +1158,11 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
 // microseconds of it) and, as the rows grow, by the bytes that pass the vector
 // cache, so a wave keeps D k-steps on their way: eight of a small tile are the
 // whole share of a wave at 1024 inputs.  Loads stand behind the MFMAs that free
-// their registers and are issued whether needed or not only in whole turns of D,
-// so the compiler's count of loads in flight is exact.  grid.x walks the outputs,
+// their registers; in whole turns of D none is conditional, so the compiler's count
+// of loads in flight is exact, and what is left behind the last turn is asked for all
+// at once (in registers of its own name: kept in those of the turns, the compiler
+// holds both; one after the other, 8 rows of 896 -> 4096 took 8.0 us, 6.4 now).
+// grid.x walks the outputs,
 // so the workgroups the dispatcher deals round-robin to the eight XCDs differ in
 // output tile.
 //
@@ -1199,38 +1202,43 @@ __global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_g
         for (int gi = 0; gi < GROUPS; gi++) acc[t][gi] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     half8 w[D][NT], x[D][GROUPS];
-    auto load_set = [&](int d, uint32_t k) {
+    auto load_set = [&](half8 (&wv)[NT], half8 (&xv)[GROUPS], uint32_t k) {
         const uint32_t o = k * 64 + lane;
 #pragma unroll
-        for (int t = 0; t < NT; t++) w[d][t] = wp[t][o];
+        for (int t = 0; t < NT; t++) wv[t] = wp[t][o];
 #pragma unroll
-        for (int gi = 0; gi < GROUPS; gi++) x[d][gi] = xp[gi][o];
+        for (int gi = 0; gi < GROUPS; gi++) xv[gi] = xp[gi][o];
     };
-    auto mfma_set = [&](int d) {
+    auto mfma_set = [&](const half8 (&wv)[NT], const half8 (&xv)[GROUPS]) {
 #pragma unroll
         for (int gi = 0; gi < GROUPS; gi++)
 #pragma unroll
             for (int t = 0; t < NT; t++)
-                acc[t][gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[d][t], x[d][gi], acc[t][gi], 0, 0, 0);
+                acc[t][gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[t], xv[gi], acc[t][gi], 0, 0, 0);
     };
-    const uint32_t turns = n / D;
+    const uint32_t turns = n / D, rest = n - turns * D;
     if (turns) {
 #pragma unroll
-        for (int d = 0; d < D; d++) load_set(d, d);
+        for (int d = 0; d < D; d++) load_set(w[d], x[d], d);
         for (uint32_t turn = 1; turn < turns; turn++) {
 #pragma unroll
             for (int d = 0; d < D; d++) {
-                mfma_set(d);
-                load_set(d, turn * D + d);
+                mfma_set(w[d], x[d]);
+                load_set(w[d], x[d], turn * D + d);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
 #pragma unroll
-        for (int d = 0; d < D; d++) mfma_set(d);
+        for (int d = 0; d < D; d++) mfma_set(w[d], x[d]);
     }
-    for (uint32_t k = turns * D; k < n; k++) {
-        load_set(0, k);
-        mfma_set(0);
+    if (rest) {
+        half8 wr[D - 1][NT], xr[D - 1][GROUPS];
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+            if ((uint32_t)d < rest) load_set(wr[d], xr[d], turns * D + d);
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+            if ((uint32_t)d < rest) mfma_set(wr[d], xr[d]);
     }
 
 #pragma unroll
