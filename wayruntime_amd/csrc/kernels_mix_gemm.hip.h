@@ -152,7 +152,7 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // none is conditional, so the compiler's count of loads in flight is exact, and what
 // is left behind the last turn is asked for all at once (in registers of its own name:
 // kept in those of the turns, the compiler holds both).  One after the other they were a
-// trip to memory each: 16 rows, 768 -> 2048 5.5 us, 3.9 now; 1536 -> 512 5.5, 4.2.
+// trip to memory each: 16 rows, 768 -> 2048 5.5 us, 3.9 now; 1536 -> 512 5.5, 4.3.
 // Few rows: bound by the weights' bytes.  More rows: by the bytes that pass a
 // compute unit's vector cache, NT + GR KiB a k-step for NT x GR products.
 // STREAM: every weight tile is read by one workgroup only (no use in keeping it).
@@ -221,7 +221,30 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(wv[t], xv[i], acc[t][i]);
     };
-    const uint32_t turns = n / D, rest = n - turns * D;
+    constexpr bool HALVES = F32 && GR > 1;
+    if constexpr (HALVES) {
+        // Half a turn is asked for, then the other half multiplied: 32 of these products to a k-step are as long as a
+        // load, and asked for behind them it is late (4096 -> 4096 at 24 rows 26.2 us, 21.2 now).  Past the end the last
+        // step is read again and not used.
+        static_assert(D == 4, "two halves of two");
+        auto ask = [&](int d, uint32_t k) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) load(w[d + u], x[d + u], min(k + u, n - 1));
+        };
+        auto take = [&](int d, uint32_t k) {
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                if (k + u < n) multiply(w[d + u], x[d + u]);
+        };
+        if (n) ask(0, 0);
+        for (uint32_t k = 0; k < n; k += 4) {
+            ask(2, k + 2);
+            take(0, k);
+            ask(0, k + 4);
+            take(2, k + 2);
+        }
+    }
+    const uint32_t turns = HALVES ? 0 : n / D, rest = HALVES ? 0 : n - turns * D;
     if (turns) {
 #pragma unroll
         for (int d = 0; d < D; d++) load(w[d], x[d], d);

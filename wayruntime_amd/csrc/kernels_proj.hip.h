@@ -1161,7 +1161,7 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
 // their registers; in whole turns of D none is conditional, so the compiler's count
 // of loads in flight is exact, and what is left behind the last turn is asked for all
 // at once (in registers of its own name: kept in those of the turns, the compiler
-// holds both; one after the other, 8 rows of 896 -> 4096 took 8.0 us, 6.4 now).
+// holds both; one after the other, 8 rows of 896 -> 4096 took 8.0 us, 6.3 now).
 // grid.x walks the outputs,
 // so the workgroups the dispatcher deals round-robin to the eight XCDs differ in
 // output tile.

@@ -592,7 +592,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     }
     if (f32) {
         if (a.groups <= 1) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, batch) : launch_split<true, 1, 1, 4, 4, true>(a, batch);
-        return launch_split<true, 2, 2, 4, 2, false>(a, batch);
+        return launch_split<true, 2, 2, 4, 4, false>(a, batch);
     }
     if (a.groups == 1) {
         // a short input range: more outputs per workgroup, or the launch is all workgroups and no work
