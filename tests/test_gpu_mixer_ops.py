@@ -195,12 +195,12 @@ def test_batch_of_matrices(lib, f32, batch, N, K, rows):
         b.free()
 
 
-# every tile the rule picks among: register tiles of 1 x 1, 1 x 2, 2 x 2, 2 x 3, 2 x 4, 4 x 3, 4 x 4 (outputs x rows,
+# every tile the rule picks among: register tiles of 1 x 1, 1 x 2, 2 x 1 (gated outputs), 2 x 2, 2 x 3, 2 x 4, 4 x 3, 4 x 4 (outputs x rows,
 # sixteens; gated outputs take even ones), LDS tiles of 64, 128 and 256 rows.  Input ranges that leave waves without
 # k-steps (96), that are less than a turn of eight and a turn and a rest of four (800), and that split unevenly with
 # a rest behind whole turns (1056), and two that two sets of waves halve, an
 # odd number of k-steps each and an even one (2112, 2176; tiles of 64 and 128 rows).
-@pytest.mark.parametrize("N,rows,K", [(n, r, k) for n, r in [(48, 17), (1088, 50), (1088, 130), (2112, 100), (2816, 100),
+@pytest.mark.parametrize("N,rows,K", [(n, r, k) for n, r in [(48, 17), (512, 64), (1088, 50), (1088, 130), (2112, 100), (2816, 100),
                                                              (2112, 300), (6208, 100), (6208, 511), (12352, 511),
                                                              (12352, 700)] for k in (96, 800, 1056)] +
                          [(2112, 700, 2112), (2112, 1100, 2112), (2112, 1100, 2176), (2112, 700, 2176)])

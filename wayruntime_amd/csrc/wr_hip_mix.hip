@@ -475,8 +475,11 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 // before / with them: 2048 -> 2048 at 130 rows 9.2 / 7.2, at 300 13.9 / 9.3; 8192 -> 2048 37.6 / 26.7 at 300; 12 288
 // -> 4096 at 300 111 / 68; 2048 -> 14 400 at 45 27 / 15.3.  The halves: 8192 -> 2048 at 1000 rows 80 / 55, at 2047 93
 // / 73; 4096 -> 2048 at 2047 50 / 41; 12 288 -> 4096 at 1000 153 / 108.
-// Over 12 row counts from 20 to 2047 and 8 weights the form picked is 0.5 % off the best one on average (3.5 % before
-// the halves), 21 % at worst.
+// Gated outputs take an even number of tiles: of one group of rows each where that spreads few tiles over more units
+// (64 rows, 8192 -> 512: 17.4 us in tiles of two groups, 13.2; 2048 -> 2048 6.9, 5.7).  Tiles of 256 rows are counted in
+// whole workgroups per unit (1500 rows, 256 -> 8192: 17.8 us against 16.3 with tiles of 128).
+// Over 11 row counts from 17 to 2047, 8 input ranges and 4 widths (profiles/stack_product_forms.txt has every form's
+// time) the form picked is 2.3 % off the best one on average, 30 % (1 us of 4) at worst.
 static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
 {
     struct Form {
@@ -484,9 +487,9 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
         int (*launch)(const MixGemmArgs&, uint32_t);
     };
     static const Form split[] = {{1, 1, launch_split<false, 1, 1, 4, 8, false>}, {1, 2, launch_split<false, 1, 2, 4, 8, false>},
-                                 {2, 2, launch_split<false, 2, 2, 4, 8, false>}, {2, 3, launch_split<false, 2, 3, 4, 4, false>},
-                                 {2, 4, launch_split<false, 2, 4, 4, 4, false>}, {4, 3, launch_split<false, 4, 3, 4, 4, false>},
-                                 {4, 4, launch_split<false, 4, 4, 4, 2, false>}};
+                                 {2, 1, launch_split<false, 2, 1, 4, 8, false>}, {2, 2, launch_split<false, 2, 2, 4, 8, false>},
+                                 {2, 3, launch_split<false, 2, 3, 4, 4, false>}, {2, 4, launch_split<false, 2, 4, 4, 4, false>},
+                                 {4, 3, launch_split<false, 4, 3, 4, 4, false>}, {4, 4, launch_split<false, 4, 4, 4, 2, false>}};
     static const struct {
         uint32_t groups;
         float step, share;
@@ -508,7 +511,8 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
     if (a.groups >= 4)
         for (const auto& f : lds) {
             const uint64_t wgs = (uint64_t)((a.ntiles + 7) / 8) * ((a.groups + f.groups - 1) / f.groups) * batch;
-            offer(std::max(f.step, f.share * wgs / g.n_cus), f.launch);
+            const float each = f.groups == 16 ? (float)((wgs + g.n_cus - 1) / g.n_cus) : (float)wgs / g.n_cus;
+            offer(std::max(f.step, f.share * each), f.launch);
         }
     if (a.groups >= 4 && a.ktiles % 2 == 0 && a.ktiles >= 64)
         for (const auto& f : halves) {
