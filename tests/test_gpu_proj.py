@@ -363,19 +363,23 @@ def test_projection_random_shapes():
 
 
 @pytest.mark.parametrize("rows,n_in,n_out", [
-    (17, 1024, 4096),             # register GEMM of 16 x 16 tiles: the fewest rows, a whole share in one turn of eight
-    (48, 2080, 1392),             # ... the most, 65 input tiles (a wave with one more than the others), 522 tiles of 16 x 8
-    (48, 2080, 16),               # 16 x 8 tiles: one output tile
-    (17, 1056, 2720),             # ... 510 of them, the last row group of one row
+    (17, 1024, 4096),             # (each workgroup makes its own fragments; whole shares in one turn of eight)
+    (48, 2080, 16),               # register tiles of 16 x 8: one output tile, 65 input tiles (a wave with one more than the others)
+    (17, 1056, 1360),             # ... 255 of them, the last row group of one row
     (31, 32, 48),                 # ... a single input tile: three waves with none
     (31, 800, 48),                # ... 25: six and seven k-steps a wave, less than a turn
-    (49, 800, 4112),              # the same in 32 x 16 tiles,
-    (250, 800, 4112),             # and in 32 x 32 tiles
-    (49, 1056, 4112),             # 32 x 16 tiles: a last row group of one row, partial output tiles
     (256, 3104, 80),              # ... the last row count whose fragments are made row by row
     (256, 3072, 80),              # (each workgroup makes its own)
-    (257, 288, 1040),             # ... by row groups
-    (250, 1056, 4112),            # 32 x 32 tiles, 33 input tiles
+    (17, 800, 1392),              # 16 x 16: 87 by 2, the last row group of one row
+    (300, 256, 144),              # ... a row group past the end
+    (48, 2080, 1392),             # 32 x 16 tiles
+    (31, 1056, 3488),             # ... 109 by 2, 33 input tiles
+    (20, 800, 7296),              # 32 x 32: fewer row groups than a tile has
+    (17, 1056, 8208),             # 64 x 32: likewise, a last run of one output tile
+    (49, 800, 4112),              # ... and 25 input tiles,
+    (250, 1056, 4112),            # ... 33, row groups past the end
+    (257, 288, 1040),             # ... fragments by row groups
+    (130, 1088, 9872),            # LDS tiles with two sets of waves and too few workgroups for all CUs
     (2047, 64, 1040),             # LDS tiles whose panels are shared out over few XCDs: 9 by 32 of them
     (4095, 96, 528),              # ... 5 by 64
     (1100, 64, 8208),             # ... the outputs over all eight: 33 by 18
@@ -469,7 +473,8 @@ def test_rows_whose_workgroups_make_their_own_terms(rows, n_in, n_out):
     (1, 14816, 32), (1, 14848, 32), (1, 15360, 32), (1, 15392, 32),    # ... 64 KiB of LDS and one unit more, the most, fragments apart
     (2, 512, 16), (16, 1024, 3072), (8, 1536, 2064), (9, 512, 4080),   # workgroups that make their own terms: a pair, two
     (5, 1056, 528), (16, 160, 48), (16, 1024, 16400),             # a wave per pair of tiles, inputs split and not
-    (17, 1056, 528), (100, 288, 2064), (200, 1056, 8208),         # register tiles of 32 x 8, 32 x 16, 32 x 32
+    (17, 1056, 528), (17, 800, 1376), (100, 288, 2064), (17, 800, 2736), (17, 1056, 4128),    # register tiles of 32 x 8, 32 x 16 (two), 32 x 32, 64 x 32
+    (130, 1088, 4944), (200, 1056, 8208),                         # LDS tiles of 128 x 64 (few, two sets of waves; two a CU)
     (300, 1024, 4112), (700, 2048, 2064), (700, 1056, 2064),      # LDS tiles of 128 x 64 (two and more a CU; one, two sets of waves; one)
     (1030, 288, 6160), (2050, 288, 4112),                         # of 128 x 128, of 256 x 128
 ])

@@ -1176,7 +1176,7 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
 // for the first, 51 for the second.)  Eight waves to the input range, or deeper
 // turns on larger tiles, gave nothing.
 template <int GROUPS, int NT, int D, bool GATED = false>
-__global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_gemm_split_kernel(const ProjArgs a)
+__global__ __launch_bounds__(kProjThreads, GROUPS * NT == 8 ? 3 : 2) void proj_gemm_split_kernel(const ProjArgs a)
 {
     __shared__ f32x4 s_red[4 * NT * GROUPS * 64];
     const int lane = threadIdx.x & 63;
@@ -1257,9 +1257,12 @@ __global__ __launch_bounds__(kProjThreads, GROUPS * NT >= 8 ? 3 : 2) void proj_g
         return v;
     };
     if constexpr (GATED) {
-        static_assert(NT == 2, "a gate's tile and a value's");
+        static_assert(NT % 2 == 0, "gates' tiles and values'");
 #pragma unroll 1
-        for (uint32_t i = wave; i < GROUPS; i += 4) proj_store_pair(a, sum(i), sum(GROUPS + i), blockIdx.x, group0 + i, lane);
+        for (uint32_t i = wave; i < NT / 2 * GROUPS; i += 4) {
+            const uint32_t pair = i / GROUPS, gi = i % GROUPS;
+            proj_store_pair(a, sum(2 * pair * GROUPS + gi), sum((2 * pair + 1) * GROUPS + gi), nt0 / 2 + pair, group0 + gi, lane);
+        }
     } else {
 #pragma unroll 1
         for (uint32_t i = wave; i < NT * GROUPS; i += 4)

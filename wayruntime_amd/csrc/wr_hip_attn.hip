@@ -794,9 +794,7 @@ void launch_proj(const ProjArgs& a)
 //   LDS-staged, eight waves, 256 outputs x 128 rows per workgroup, from one workgroup per CU;
 //   LDS-staged, 128 x 128, from two workgroups per CU;
 //   LDS-staged, 128 x 64, from one per CU (software-pipelined: a SIMD may hold a single wave);
-//   registers, the four waves split the input range: 16 x 8 (up to two workgroups of it per CU),
-//   16 x 16 (up to 48 rows, weights up to 4096 outputs),
-//   32 x 16 (up to 1024 workgroups of it), 32 x 32.
+//   registers, the four waves split the input range: 16 x 8 to 64 x 32.
 constexpr int kProjGemmMinRows = 17;
 constexpr uint32_t kProjGroupRows = 257;           // from here on the fragments are made by row groups: at 200 rows a
                                                    // workgroup per row is 0.6 to 2.2 us faster, at 300 as fast, at 511 1 us slower
@@ -820,6 +818,50 @@ void launch_proj_lds(ProjArgs a, uint32_t groups, uint32_t per_xcd)
                       (uint64_t)groups * 8 * a.K * 4, per_xcd, &blocks);
     launch_main(a.gate ? proj_gemm_lds_kernel<GROUPS, WN, RING, PIPE, KS, true> : proj_gemm_lds_kernel<GROUPS, WN, RING, PIPE, KS>,
                 dim3(blocks), dim3(128 * WN * KS), a, gemm_lds_bytes<GROUPS, WN, RING, KS>());
+}
+
+// Register tiles: the one whose estimate is the least.  A tile of NT x GROUPS waits for NT + GROUPS KiB a k-step
+// through a compute unit's vector cache, workgroup after workgroup; an LDS tile of two sets of waves for as long as 17
+// of them (from 1024 inputs on).  Chosen by workgroups alone before, wide weights took tiles too small (64 rows, 4096 ->
+// 8192: 52 us in tiles of 32 x 16, 30 in 64 x 32; 160 rows 65, 41; 1500 rows, 5120 -> 1024 86, 75).  Over 15 row counts
+// from 17 to 1500, 10 input ranges and 7 widths (profiles/projection_product_forms.txt has every form's time) the form
+// picked is 1.4 % off the best one on average, 24 % (1.3 us of 5.4) at worst.
+// The gated tiles follow the plain ones in the choice between registers and LDS: only then do both take the same sums
+// (a register tile of any size has the same ones), and the gated product the bits of the plain one's activation.
+void launch_proj_tiles(const ProjArgs& a, uint32_t groups)
+{
+    struct Form {
+        uint32_t groups, nt;
+        void (*launch)(const ProjArgs&, uint32_t);
+    };
+    static const Form plain[] = {{1, 1, launch_proj_gemm_split<1, 1, 8>}, {2, 1, launch_proj_gemm_split<2, 1, 8>},
+                                 {2, 2, launch_proj_gemm_split<2, 2, 8>}, {4, 2, launch_proj_gemm_split<4, 2, 4>},
+                                 {4, 4, launch_proj_gemm_split<4, 4, 2>}},
+                      gated[] = {{1, 2, launch_proj_gemm_split<1, 2, 8, true>}, {2, 2, launch_proj_gemm_split<2, 2, 8, true>},
+                                 {4, 2, launch_proj_gemm_split<4, 2, 4, true>}, {4, 4, launch_proj_gemm_split<4, 4, 2, true>}};
+    const uint32_t nt = a.N / 16;
+    const auto rounds = [&](uint32_t w, uint32_t h) {
+        return (uint32_t)(((uint64_t)((nt + w - 1) / w) * ((groups + h - 1) / h) + g.n_cus - 1) / g.n_cus);
+    };
+    uint32_t least = ~0u;
+    const Form* best = nullptr;
+    const auto offer = [&](const Form& f) {
+        const uint32_t cost = rounds(f.nt, f.groups) * (f.nt + f.groups);
+        if (cost < least) {
+            least = cost;
+            best = &f;
+        }
+    };
+    for (const Form& f : plain) offer(f);
+    if (a.K >= 1024 && a.K % 64 == 0 && rounds(8, 8) * 17 < least) {
+        launch_proj_lds<4, 2, 4, true, 2>(a, groups, 32);
+        return;
+    }
+    if (a.gate) {
+        least = ~0u;
+        for (const Form& f : gated) offer(f);
+    }
+    best->launch(a, groups);
 }
 
 void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
@@ -860,21 +902,8 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
         launch_proj_lds<4, 2, 4, true, 2>(a, groups, 32);
     else if (panels * ((groups + 7) / 8) >= 256)          // one per CU, one wave per SIMD: pipelined reads
         launch_proj_lds<4, 2, 4, true, 1>(a, groups, 32);
-    else if (a.gate) {                                    // tiles in pairs: 32 x 8, 32 x 16, 32 x 32
-        if (nt / 2 * groups <= 512)
-            launch_proj_gemm_split<1, 2, 8, true>(a, groups);
-        else if (nt / 2 * ((groups + 1) / 2) <= 1024)
-            launch_proj_gemm_split<2, 2, 8, true>(a, groups);
-        else
-            launch_proj_gemm_split<4, 2, 4, true>(a, groups);
-    } else if (nt * groups <= 512)                          // (64 rows, 2048 -> 1024: 5.4 us against 5.6 with the next)
-        launch_proj_gemm_split<1, 1, 8>(a, groups);
-    else if (groups <= 6 && nt <= 256)                    // (45 rows, 1024 -> 6144: 7.6 us against 7.4 with the next)
-        launch_proj_gemm_split<2, 1, 8>(a, groups);
-    else if (((nt + 1) / 2) * ((groups + 1) / 2) <= 1024) // (200 rows, 1024 -> 6144: 16.8 against 16.4 with the next)
-        launch_proj_gemm_split<2, 2, 8>(a, groups);
     else
-        launch_proj_gemm_split<4, 2, 4>(a, groups);
+        launch_proj_tiles(a, groups);
 }
 
 // proj_rows_fused_kernel<SRC, n_in / 128, nt>, or nullptr where none is built.
