@@ -420,6 +420,7 @@ def test_normed_and_gated_rows_by_rows_and_by_groups(rows, n_in):
     (9, 1536, 4112), (5, 1536, 8192),                # two tiles a workgroup, the last with one; the most for it
     (16, 2048, 2064), (11, 2560, 48), (16, 3072, 1024), (9, 1024, 1024),
     (17, 1024, 4096), (41, 2048, 656),               # more than a decode step's rows: the last group of one row
+    (16, 640, 4112), (9, 640, 4096), (9, 4224, 4112), (3, 5120, 3280),   # inputs none takes: 32 x 16 tiles, 16 x 8, streams
 ])
 def test_rows_whose_workgroups_make_their_own_terms(rows, n_in, n_out):
     # Every row has the bits of the row alone (up to sixteen of them) and of the same

@@ -26,9 +26,10 @@
 //
 // Kernels, by row count of a launch:
 //   1 row        proj_row1_kernel: the fragment step inside the product;
-//   2 .. 16      proj_prep_kernel, then proj_gemm_split_kernel<1, 1, 8> where four
-//                waves share a tile's inputs, proj_rows_kernel (a wave owns one or two
-//                16-output tiles for one or two row groups; HBM-bound) elsewhere;
+//   2 .. 16      proj_prep_kernel, then proj_gemm_split_kernel where four waves share
+//                a tile's inputs and they are few or the weight small, proj_rows_kernel
+//                (a wave owns one or two 16-output tiles for one or two row groups;
+//                HBM-bound) elsewhere;
 //   17 .. 4096   proj_prep_kernel (proj_prep_group_kernel from 257 rows), then a
 //                GEMM: proj_gemm_lds_kernel (operands staged through LDS,
 //                MFMA-bound) where its tiles fill the chip,

@@ -1088,15 +1088,23 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
         launch_proj<1, 2, true>(a);
     else if (src.gate)
         launch_proj<2, 2, true>(a);
-    else if (ksplit == 4)
+    else if (ksplit == 4 && !(w->n_in > 4096 && (uint64_t)w->n_in * w->n_out >= 12u << 20)) {
         // A workgroup per tile and group of eight rows, four waves to the input range: the
         // same parts in the same order as below, so the same bits.  For 9 .. 16 rows the
         // weights pass L2 twice, but a workgroup reads half the operand fragments, which
         // at 16 rows are twice the weights' bytes: 16 rows, weights from HBM, 1024 -> 4096
         // 4.7 -> 4.2 us, 2048 -> 1024 5.3 -> 4.3, 1024 -> 6144 6.0 -> 5.4, 3072 -> 1024
-        // 7.0 -> 5.5 (4 rows: 4.2 -> 3.7, 4.4, 5.2 -> 4.9, 5.9 -> 5.6).
-        launch_proj_gemm_split<1, 1, 8>(a, groups);
-    else if (groups == 1)
+        // 7.0 -> 5.5 (4 rows: 4.2 -> 3.7, 4.4, 5.2 -> 4.9, 5.9 -> 5.6).  Where the tiles are
+        // more than the CUs the weights' second pass is the larger loss: 32 x 16 (16 rows,
+        // 4096 -> 8192 26.6 us in tiles of 16 x 8, 22.4 below, 22.1; 2048 -> 6144 12.4, 12.6,
+        // 11.3).  Long ranges of large weights stream faster below: 8192 -> 4096 34.4 us
+        // against 25.9, 14 336 -> 8192 101 against 55 (4 rows 27.0, 22.0; 61, 52); the line
+        // lies between 5120 -> 2048 (13.7 us, 14.3 below) and 6144 -> 2048 (18.4, 15.8).
+        if (groups == 2 && tiles > g.n_cus)
+            launch_proj_gemm_split<2, 2, 8>(a, groups);
+        else
+            launch_proj_gemm_split<1, 1, 8>(a, groups);
+    } else if (groups == 1)
         launch_proj<1, 1>(a);
     else if (tiles * ksplit >= 2048)
         launch_proj<2, 2>(a);               // wide weight: two output tiles per operand load
