@@ -471,7 +471,8 @@ def test_rows_whose_workgroups_make_their_own_terms(rows, n_in, n_out):
 
 @pytest.mark.parametrize("rows,n_in,ffn", [
     (1, 1024, 3072), (1, 96, 48), (1, 3104, 8208),                # one row: four waves a pair, none shared, two, an odd count
-    (1, 14816, 32), (1, 14848, 32), (1, 15360, 32), (1, 15392, 32),    # ... 64 KiB of LDS and one unit more, the most, fragments apart
+    (1, 1024, 1040), (1, 768, 16), (1, 1536, 2048), (1, 320, 528),    # ... eight gates with their values, batches of eight and four, rests
+    (1, 15360, 2064), (1, 15360, 32), (1, 15392, 32),             # ... more than 64 KiB of LDS, the most inputs, fragments apart
     (2, 512, 16), (16, 1024, 3072), (8, 1536, 2064), (9, 512, 4080),   # workgroups that make their own terms: a pair, two
     (5, 1056, 528), (16, 160, 48), (16, 1024, 16400),             # a wave per pair of tiles, inputs split and not
     (17, 1056, 528), (17, 800, 1376), (100, 288, 2064), (17, 800, 2736), (17, 1056, 4128),    # register tiles of 32 x 8, 32 x 16 (two), 32 x 32, 64 x 32

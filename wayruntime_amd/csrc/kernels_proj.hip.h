@@ -37,6 +37,8 @@
 // N must be a multiple of 16 and K a multiple of 32.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hip.h"
 
 namespace wr {
@@ -556,6 +558,22 @@ __device__ __forceinline__ void proj_store_pair(const ProjArgs& a, f32x4 gate, f
     }
 }
 
+// One row, a tile of eight gates (outputs 8 h .. 8 h + 7 of pair `pair`) and their values: lanes 32 and up hold the
+// values' half.
+__device__ __forceinline__ void proj_store_half_pair(const ProjArgs& a, f32x4 v, uint32_t pair, uint32_t h, int lane, float scale)
+{
+    v = proj_join_terms(v);
+    f32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float x = v[i] * scale;
+        asm volatile("" : "+v"(x));                              // (as above)
+        const float y = wave_xor_f32(x, 32);
+        r[i] = a.gate == kProjSrcGeglu ? proj_gated<kProjSrcGeglu>(x, y) : proj_gated<kProjSrcSwiglu>(x, y);
+    }
+    if ((lane & 47) == 0) *reinterpret_cast<f32x4*>(a.y + pair * 16 + h * 8 + (lane >> 4) * 4) = r;
+}
+
 // One wave-step: NT weight tiles against GROUPS operand fragments.
 template <int GROUPS, int NT>
 __device__ __forceinline__ void proj_step(f32x4 (&acc)[NT][GROUPS], const half8 (&wv)[NT],
@@ -727,12 +745,23 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
 // row run while the weights travel.  NB0 = batches asked for up front, a
 // template parameter so that every load before the first wait is unconditional
 // and the compiler's count of loads in flight is exact.
-template <int SRC, int NB0, bool GATED>
+//
+// FORM: kRow1Gated takes the gates' tile and the values' (KB = 4 k-steps of both to a
+// batch), and half as many workgroups as the plain form.  kRow1GatedHalf takes eight
+// gates and their eight values as one tile, so a workgroup reads what a plain one does,
+// in pieces of a line; for products whose pairs would leave half the CUs without a
+// workgroup (whole FFNs of one row, us: 4096 -> 2 x 1024 11.4, against 13.3 of pairs and
+// 11.3 of products that keep gates and values apart; 1024 -> 2 x 1024 8.2, 8.6, 7.6; 1056
+// -> 2 x 4096 14.0, 15.8, 14.0; from 2 x 2560 on pairs are the faster: 4096 -> 18.0, 19.0
+// apart).
+constexpr int kRow1Plain = 0, kRow1Gated = 1, kRow1GatedHalf = 2;
+
+template <int SRC, int NB0, int FORM, int KB>
 __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrepArgs& p, half8* sfrag,
                                                f32x4* s_part, float* s4, float* s_scale)
 {
+    constexpr bool GATED = FORM == kRow1Gated, HALF = FORM == kRow1GatedHalf;
     constexpr int NT = GATED ? 2 : 1;                            // weight tiles of a wave
-    constexpr int KB = kProjKBatch / NT;
     constexpr int CH = 2;                                        // chunks of eight inputs a thread can hold
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t t = threadIdx.x;
@@ -740,7 +769,7 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
     const uint32_t slot = wave / S, part = wave % S;
     const uint32_t nt0 = blockIdx.x * (4 / S) + slot;
     const uint32_t ntiles = a.N / 16;
-    const bool live = nt0 < (GATED ? ntiles / 2 : ntiles);       // (GATED: nt0 is a pair of tiles)
+    const bool live = nt0 < (GATED ? ntiles / 2 : ntiles);       // (GATED: nt0 is a pair of tiles, HALF: half a pair)
     const uint32_t ktiles = a.K / 32, nchunks = a.K / 8;
     const uint32_t kper = ktiles / S;
     const uint32_t k_begin = part * kper, k_end = k_begin + kper;
@@ -748,6 +777,8 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
 #pragma unroll
     for (int tt = 0; tt < NT; tt++)
         wp[tt] = a.w + (size_t)(GATED ? proj_paired_tile(nt0, tt, ntiles) : live ? nt0 : ntiles - 1) * ktiles * 64 + lane;
+    if constexpr (HALF)      // rows 8 h .. 8 h + 7 of the gates' tile, then of the values'
+        wp[0] = a.w + (size_t)proj_paired_tile(nt0 / 2, (lane >> 3) & 1, ntiles) * ktiles * 64 + (lane & 48) + nt0 % 2 * 8 + (lane & 7);
     const float* xr = p.x;
     const bool in_regs = a.K <= 2048u * CH;                      // uniform
 
@@ -954,6 +985,8 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
     if (!live) return;
     if constexpr (GATED)
         proj_store_pair(a, acc[0], acc[1], nt0, 0, lane, s_scale);
+    else if constexpr (HALF)
+        proj_store_half_pair(a, acc[0], nt0 / 2, nt0 % 2, lane, *s_scale);
     else
         proj_store_tile(a, acc[0], nt0, 0, lane, s_scale, &resid);
 }
@@ -961,23 +994,31 @@ __device__ __forceinline__ void proj_row1_body(const ProjArgs& a, const ProjPrep
 // LDS of proj_row1_kernel beside the row's terms: partial tiles, the row's sums, its scale.
 constexpr size_t row1_static_lds(bool gated) { return (gated ? 6 : 3) * 64 * sizeof(f32x4) + 8 * sizeof(float) + sizeof(float); }
 
-template <int SRC, bool GATED = false>
+template <int SRC, int FORM = kRow1Plain>
 __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs a, const ProjPrepArgs p)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char row1_smem[];
     half8* sfrag = reinterpret_cast<half8*>(row1_smem);           // [K/8][2]: hi, lo of chunk q
-    __shared__ f32x4 s_part[(GATED ? 6 : 3) * 64];
+    __shared__ f32x4 s_part[(FORM == kRow1Gated ? 6 : 3) * 64];
     __shared__ float s4[8];
     __shared__ float s_scale;
-    const uint32_t nb = a.K / 32 / a.ksplit / (kProjKBatch / (GATED ? 2 : 1));        // whole batches of weights per wave: uniform
-    if (nb >= 3)
-        proj_row1_body<SRC, 3, GATED>(a, p, sfrag, s_part, s4, &s_scale);
-    else if (nb == 2)
-        proj_row1_body<SRC, 2, GATED>(a, p, sfrag, s_part, s4, &s_scale);
-    else if (nb == 1)
-        proj_row1_body<SRC, 1, GATED>(a, p, sfrag, s_part, s4, &s_scale);
+    const uint32_t kper = a.K / 32 / a.ksplit;                    // a wave's k-steps; whole batches of KB: uniform
+    const auto body = [&](auto batch) {
+        constexpr int KB = decltype(batch)::value;
+        const uint32_t nb = kper / KB;
+        if (nb >= 3)
+            proj_row1_body<SRC, 3, FORM, KB>(a, p, sfrag, s_part, s4, &s_scale);
+        else if (nb == 2)
+            proj_row1_body<SRC, 2, FORM, KB>(a, p, sfrag, s_part, s4, &s_scale);
+        else if (nb == 1)
+            proj_row1_body<SRC, 1, FORM, KB>(a, p, sfrag, s_part, s4, &s_scale);
+        else
+            proj_row1_body<SRC, 0, FORM, KB>(a, p, sfrag, s_part, s4, &s_scale);
+    };
+    if (FORM == kRow1Gated || (FORM == kRow1GatedHalf && kper % kProjKBatch))
+        body(std::integral_constant<int, kProjKBatch / 2>());
     else
-        proj_row1_body<SRC, 0, GATED>(a, p, sfrag, s_part, s4, &s_scale);
+        body(std::integral_constant<int, kProjKBatch>());
 }
 
 // Two rows to a few dozen, inputs of 512 D / 4: the fragment step inside the product.

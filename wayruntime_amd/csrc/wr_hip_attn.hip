@@ -823,7 +823,7 @@ void launch_proj_lds(ProjArgs a, uint32_t groups, uint32_t per_xcd)
 // Register tiles: the one whose estimate is the least.  A tile of NT x GROUPS waits for NT + GROUPS KiB a k-step
 // through a compute unit's vector cache, workgroup after workgroup; an LDS tile of two sets of waves for as long as 17
 // of them (from 1024 inputs on).  Chosen by workgroups alone before, wide weights took tiles too small (64 rows, 4096 ->
-// 8192: 52 us in tiles of 32 x 16, 30 in 64 x 32; 160 rows 65, 41; 1500 rows, 5120 -> 1024 86, 75).  Over 15 row counts
+// 8192: 52 us in tiles of 32 x 16, 30 in 64 x 32; 160 rows 65, 41; 1500 rows, 5120 -> 1024 86, 66).  Over 15 row counts
 // from 17 to 1500, 10 input ranges and 7 widths (profiles/projection_product_forms.txt has every form's time) the form
 // picked is 1.4 % off the best one on average, 24 % (1.3 us of 5.4) at worst.
 // The gated tiles follow the plain ones in the choice between registers and LDS: only then do both take the same sums
@@ -1065,13 +1065,18 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     a.gate = (uint8_t)src.gate;
     a.ksplit = (uint8_t)ksplit;
     if (row1) {
-        const uint32_t runs = src.gate ? tiles / 2 : tiles;
-        const dim3 grid((runs + 4 / ksplit - 1) / (4 / ksplit)), block(kProjThreads);
+        const uint32_t per_block = 4 / ksplit, pair_blocks = (tiles / 2 + per_block - 1) / per_block;
+        const bool pairs = src.gate && pair_blocks * 2 > g.n_cus;
+        const dim3 grid(pairs ? pair_blocks : (tiles + per_block - 1) / per_block), block(kProjThreads);
         const size_t lds = (size_t)w->n_in * 4;
-        if (src.gate && src.kind == kProjSrcRmsNorm)
-            launch_main(proj_row1_kernel<kProjSrcRmsNorm, true>, grid, block, a, pa, lds);
+        if (pairs && src.kind == kProjSrcRmsNorm)
+            launch_main(proj_row1_kernel<kProjSrcRmsNorm, kRow1Gated>, grid, block, a, pa, lds);
+        else if (pairs)
+            launch_main(proj_row1_kernel<kProjSrcPlain, kRow1Gated>, grid, block, a, pa, lds);
+        else if (src.gate && src.kind == kProjSrcRmsNorm)
+            launch_main(proj_row1_kernel<kProjSrcRmsNorm, kRow1GatedHalf>, grid, block, a, pa, lds);
         else if (src.gate)
-            launch_main(proj_row1_kernel<kProjSrcPlain, true>, grid, block, a, pa, lds);
+            launch_main(proj_row1_kernel<kProjSrcPlain, kRow1GatedHalf>, grid, block, a, pa, lds);
         else if (src.kind == kProjSrcRmsNorm)
             launch_main(proj_row1_kernel<kProjSrcRmsNorm>, grid, block, a, pa, lds);
         else if (src.kind == kProjSrcSwiglu)
@@ -1221,8 +1226,8 @@ int wr_hip_attn_init(int device)
                 e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         };
         // (a gated row: 6 KiB of partial tiles beside its terms, more than 64 KiB together from 14 848 inputs on)
-        allow_lds(proj_row1_kernel<kProjSrcRmsNorm, true>, kProjRow1MaxLds);
-        allow_lds(proj_row1_kernel<kProjSrcPlain, true>, kProjRow1MaxLds);
+        allow_lds(proj_row1_kernel<kProjSrcRmsNorm, kRow1Gated>, kProjRow1MaxLds);
+        allow_lds(proj_row1_kernel<kProjSrcPlain, kRow1Gated>, kProjRow1MaxLds);
         allow_lds(proj_gemm_lds_kernel<8, 2, 3>, gemm_lds_bytes<8, 2, 3>());
         allow_lds(proj_gemm_lds_kernel<8, 2, 3, false, 1, true>, gemm_lds_bytes<8, 2, 3>());
         allow_lds(proj_gemm_lds_kernel<4, 2, 4, true>, gemm_lds_bytes<4, 2, 4>());
