@@ -521,10 +521,18 @@ int check_decode(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32_
 // longest block, whose keys one workgroup walks while most CUs stand idle; cut, every part pays a block's ends
 // (Q in, the sets' merge, rows out) and the rows go through memory once more.  In microseconds: the ends of a block,
 // a step (64 keys of a 32-row unit at head dims up to 128, 32 keys at 256; fewer workgroups than CUs), the combine
-// launch, and the bytes it and the parts move.
+// launch, what it takes a part, and the bytes it and the parts move.
+// Fitted to nine shapes by ten row counts by eight lengths before them, 1 to 32 parts each (profiles/prefill_parts.txt):
+// the parts picked are 0.6 to 1.1 % off the best on average, 19 % (2 us of 10) at worst, and never slower than none by
+// more than 4 %.  With one set of figures for all head dims, from 128, launches of 64 were cut too often and too fine
+// (500 rows behind 1024 keys, 32/8/64: 17.9 us whole, 20.6 cut).
 uint32_t prefill_parts(const PrefillArgs& a, uint32_t BP, uint32_t nblk, uint32_t ny)
 {
-    const float ends = 8.f, step = a.hd == 256 ? 0.95f : 0.8f, combine = 5.f;
+    struct Cost {
+        float step, mb_us, part;
+    };
+    const Cost c = a.hd == 64 ? Cost{0.7f, 2.f, 0.2f} : a.hd == 128 ? Cost{0.8f, 2.5f, 0.2f} : Cost{1.f, 4.f, 0.25f};
+    const float ends = 8.f, combine = 3.f;
     const float row_mb = (float)a.T * a.nq * a.hd * 4e-6f;
     const uint64_t row_bytes = (uint64_t)a.T * a.nq * (a.hd + 2) * 4;
     const uint64_t room = (uint64_t)g.prefill_part_mb.load(std::memory_order_relaxed) << 20;
@@ -537,8 +545,8 @@ uint32_t prefill_parts(const PrefillArgs& a, uint32_t BP, uint32_t nblk, uint32_
         if (p > 1 && p * row_bytes > room) break;
         const uint32_t rounds = (nblk * ny * p + g.n_cus - 1) / g.n_cus;
         const uint32_t steps = ((tiles + p - 1) / p + per_step - 1) / per_step;
-        float t = rounds * (ends + step * steps);
-        if (p > 1) t += combine + 2.f * p * row_mb / 4.f;                       // written and read at about 4 TB/s
+        float t = rounds * (ends + c.step * steps);
+        if (p > 1) t += combine + c.part * p + 2.f * p * row_mb / c.mb_us;
         if (p == 1 || t < least) {
             least = t;
             best = p;
