@@ -217,9 +217,11 @@ def test_prefill_paired_blocks_with_offset_and_window_sampled_rows(nq, nkv, hd, 
 
 @pytest.mark.parametrize("nq,nkv,hd,p0,T,win", [
     (32, 8, 128, 8192, 177, 0),     # five parts
-    (32, 8, 128, 5000, 1, 0),       # one row, as many parts as there may be
+    (32, 8, 128, 5000, 1, 0),       # one row, sixteen
+    (4, 1, 64, 30000, 1, 0),        # ..., as many parts as there may be
+    (16, 8, 128, 2047, 150, 1500),  # a window: parts of blocks whose ranges start inside a tile
     (16, 8, 128, 4100, 45, 0),      # a block of 64 positions that is not full, tiles that do not divide evenly
-    (16, 8, 128, 2047, 700, 1500),  # a window: blocks whose ranges start inside a tile
+    (16, 8, 128, 2047, 700, 1500),  # a window, too many rows to be cut
     (4, 4, 64, 3001, 140, 0),       # MHA: a block's last rows end before its last part
     (8, 1, 64, 2500, 97, 0),        # two head chunks per KV head
     (8, 4, 256, 3000, 100, 0),
@@ -235,6 +237,49 @@ def test_few_rows_over_many_keys_sampled_rows(nq, nkv, hd, p0, T, win):
     want = oracle.causal_prefill(q, k16, v16, p0=p0, window=win, rows=rows, threads=8)
     print("  errors", util.assert_close(got[rows], want[rows]), flush=True)
     assert np.isfinite(got).all() and np.array_equal(got, kv.prefill(0, p0, q, 0.0, win))
+    kv.close()
+
+
+@pytest.mark.parametrize("where", ["first", "middle", "last", "down", "up"])
+@pytest.mark.parametrize("nq,nkv,hd", [(32, 8, 128), (4, 4, 64), (8, 4, 256)])
+def test_parts_whose_references_lie_far_apart(nq, nkv, hd, where):
+    # all but one part's weights vanish beside it, or each part's beside the next: which part holds the largest scores
+    # must not matter.  Scores differ by 63 at most: between -88 and -87.6 the oracle's exponential, the reference's
+    # polynomial, is near one in place of 10^-38 (its exponent is not added there).
+    p0, T = 4001, 21
+    rows = p0 + T
+    print("prefill parts far apart", nq, nkv, hd, where, flush=True)
+    k32, v32 = synth.normal(6200 + hd, (rows, nkv, hd), std=0.05), synth.normal(6201 + hd, (rows, nkv, hd))
+    q = synth.normal(6202 + hd, (T, nq, hd), std=0.05)
+    at = np.arange(rows)
+    ramp = {"first": 60.0 * (at < 40), "middle": 60.0 * (abs(at - 2000) < 20), "last": 60.0 * (at >= rows - T),
+            "down": (rows - at) / 64.0, "up": at / 64.0}[where]
+    k32[:, :, 0] = ramp[:, None]
+    q[:, :, 0] = np.sqrt(hd)                             # score = ramp(key) + noise
+    kv = hipattn.KVCache(1, hd, nkv, rows)
+    assert kv.append(0, 0, k32, v32) == hipattn.OK
+    got = kv.prefill(0, p0, q)
+    want = oracle.causal_prefill(q, synth.f32_to_f16_trunc(k32), synth.f32_to_f16_trunc(v32), p0=p0, threads=8)
+    print("  errors", util.assert_close(got, want), flush=True)
+    kv.close()
+
+
+@pytest.mark.parametrize("nq,nkv,hd", [(32, 8, 128), (4, 4, 64), (8, 4, 256)])
+def test_what_is_not_finite_reaches_the_same_rows_in_parts(nq, nkv, hd):
+    # a NaN key that only the later rows see, an infinite value further back: the rows and dimensions they reach are
+    # those of the launch that is not cut
+    p0, T = 4001, 45
+    kv, q, k16, v16 = _setup(nq, nkv, hd, p0, T, seed=6300 + hd)
+    k16[p0 + 7, 0, 3], v16[1500, nkv - 1, 5] = 0x7E00, 0x7C00
+    kv.write_f16(0, 0, k16, v16)
+    got = kv.prefill(0, p0, q)
+    hipattn.set_prefill_part_mb(0)
+    whole = kv.prefill(0, p0, q)
+    hipattn.set_prefill_part_mb()
+    assert np.isnan(got[7:, 0]).all() and np.isfinite(got[:7, 0]).all() and np.isinf(got[:, nq - 1, 5]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(whole)) and np.array_equal(np.isinf(got), np.isinf(whole))
+    ok = np.isfinite(whole)
+    util.assert_close(got[ok], whole[ok])
     kv.close()
 
 
@@ -358,6 +403,7 @@ def test_prefill_error_contract():
     (32, 8, 2048, 0, False, 0.0, 0),     # Llama shape: paired blocks
     (16, 8, 300, 500, True, 0.25, 0),    # a later chunk of a prompt, scale override
     (32, 8, 700, 0, False, 0.0, 256),    # sliding window
+    (32, 8, 45, 4000, True, 0.0, 0),     # few rows behind many keys: blocks in parts
 ])
 def test_prefill_from_f16_query_rows_equals_the_f32_form(nq, nkv, T, p0, norm, scale, window):
     # wr_hip_rows_qkv_append_q16_dev + wr_hip_attn_prefill_q16_dev against
