@@ -249,14 +249,19 @@ def test_two_workgroups_to_a_tile(lib, N, K):
         b.free()
 
 
-@pytest.mark.parametrize("N,K,runs_each", [(64, 352, 1), (2080, 96, 1), (64, 352, 3), (2080, 96, 3), (1056, 32, 2)])
-def test_runs_whose_last_groups_hold_no_pair(lib, N, K, runs_each):
-    # runs of eight groups per expert, the last one's rest empty, as routing leaves it: few rows an expert and many
-    experts = 3
+@pytest.mark.parametrize("N,K,runs_each,spare,experts", [
+    (64, 352, 1, 1, 3), (2080, 96, 1, 1, 3),                   # few rows an expert: a stream of the weights
+    (64, 352, 1, 0, 3), (2080, 96, 1, 0, 3),                   # as many runs as experts, tiles of 128 rows
+    (64, 352, 3, 0, 3), (2080, 96, 3, 0, 3), (1056, 32, 2, 0, 3),
+    (1040, 64, 2, 0, 3), (64, 352, 2, 0, 3),                   # ... of 64 rows, and of 128 on wider weights
+    (144, 2080, 1, 1, 60), (144, 2016, 1, 1, 60),              # narrow weights, a tile to a CU; one input tile fewer
+])
+def test_runs_whose_last_groups_hold_no_pair(lib, N, K, runs_each, spare, experts):
+    # runs of eight groups per expert, the last one's rest and whole runs behind them empty, as routing leaves them
     r = Run(lib, False, experts, N, K, 0)
-    which = np.full(8 * experts * runs_each, -1, dtype=np.int32)
+    which = np.full(8 * (experts * runs_each + spare), -1, dtype=np.int32)
     for e in range(experts):
-        n = 8 * (runs_each - 1) + (1, 4, 7)[e]             # groups that hold pairs
+        n = 8 * (runs_each - 1) + (1, 4, 7)[e % 3]         # groups that hold pairs
         which[8 * runs_each * e:8 * runs_each * e + n] = e
     rows, live = 16 * len(which), np.repeat(which, 16) >= 0
     x = r.act(rows, K)
