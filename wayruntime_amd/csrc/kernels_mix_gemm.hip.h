@@ -259,7 +259,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
 #pragma unroll
         for (int d = 0; d < D; d++) multiply(w[d], x[d]);
     }
-    if (rest) {
+    if (__builtin_expect(rest != 0, 0)) {
         bf16x8 wr[D - 1][NT];
         V8 xr[D - 1][GR];
 #pragma unroll

@@ -1273,7 +1273,7 @@ __global__ __launch_bounds__(kProjThreads, GROUPS * NT == 8 ? 3 : 2) void proj_g
 #pragma unroll
         for (int d = 0; d < D; d++) mfma_set(w[d], x[d]);
     }
-    if (rest) {
+    if (__builtin_expect(rest != 0, 0)) {
         half8 wr[D - 1][NT], xr[D - 1][GROUPS];
 #pragma unroll
         for (int d = 0; d < D - 1; d++)

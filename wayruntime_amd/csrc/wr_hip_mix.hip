@@ -477,7 +477,8 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 // / 73; 4096 -> 2048 at 2047 50 / 41; 12 288 -> 4096 at 1000 153 / 108.
 // Gated outputs take an even number of tiles: of one group of rows each where that spreads few tiles over more units
 // (64 rows, 8192 -> 512: 17.4 us in tiles of two groups, 13.2; 2048 -> 2048 6.9, 5.7).  Tiles of 256 rows are counted in
-// whole workgroups per unit (1500 rows, 256 -> 8192: 17.8 us against 16.3 with tiles of 128).
+// whole workgroups per unit where all run at once (1500 rows, 256 -> 8192: 17.8 us against 16.3 with tiles of 128;
+// beyond two a unit, places are filled as they come free: 2047 rows, 2048 -> 14 400 161 us, 170 with tiles of 128).
 // Over 11 row counts from 17 to 2047, 8 input ranges and 4 widths (profiles/stack_product_forms.txt has every form's
 // time) the form picked is 2.3 % off the best one on average, 30 % (1 us of 4) at worst.
 static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
@@ -511,7 +512,8 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
     if (a.groups >= 4)
         for (const auto& f : lds) {
             const uint64_t wgs = (uint64_t)((a.ntiles + 7) / 8) * ((a.groups + f.groups - 1) / f.groups) * batch;
-            const float each = f.groups == 16 ? (float)((wgs + g.n_cus - 1) / g.n_cus) : (float)wgs / g.n_cus;
+            const bool at_once = f.groups == 16 && wgs <= 2 * g.n_cus;
+            const float each = at_once ? (float)((wgs + g.n_cus - 1) / g.n_cus) : (float)wgs / g.n_cus;
             offer(std::max(f.step, f.share * each), f.launch);
         }
     if (a.groups >= 4 && a.ktiles % 2 == 0 && a.ktiles >= 64)
