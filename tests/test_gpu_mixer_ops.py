@@ -226,7 +226,8 @@ def test_every_tile_of_many_rows(lib, N, K, rows):
 def test_two_workgroups_to_a_tile(lib, N, K):
     # narrow weights over long inputs, up to sixteen rows: one tile, as many as a launch holds, an odd number of k-steps;
     # one tile more and one k-step less, which a single workgroup takes.  A row's bits are its own whatever rows go with
-    # it and whichever workgroup is last, sixteen launches over; every destination.
+    # it and whichever workgroup is last, sixteen launches over; every destination (gated outputs take no such tile), with
+    # bias, activations and a factor.
     r = Run(lib, False, 1, N, K, 16)
     x = r.act(16, K)
     xd, y, y1 = r.up(x), hipattn.DeviceBuffer(16 * N * 4), hipattn.DeviceBuffer(N * 4)
@@ -243,9 +244,22 @@ def test_two_workgroups_to_a_tile(lib, N, K):
         h = hipattn.DeviceBuffer(16 * N * 2)
         r.go(xd, out=FRAG, h=h.p, h_kt=N // 32, relu2=1)
         r.close(r.frag_down(h, 16, N), np.maximum(want, 0) ** 2, eight_bits=True)
+        split = N // 2 // 32 * 32
+        r.go(xd, out=SPLIT, h=h.p, h_kt=split // 32, n_split=split, y_f32=y.p, ldy=N - split)
+        r.close(r.frag_down(h, 16, split), want[:, :split], eight_bits=True)
+        r.close(y.to_host((16, N - split)), want[:, split:])
         h.free()
+    bias = r.rng.standard_normal(N).astype(np.float32)
+    bd, ya, ld = hipattn.DeviceBuffer.from_host(bias), hipattn.DeviceBuffer(16 * (N + 8) * 2), N + 8
+    r.go(xd, out=ROWS, y_act=ya.p, ldy=ld, bias=bd.p, silu_end=N // 3, scale=0.5)
+    v = want + bias
+    got = O.bf16_to_f32(ya.to_host((16 * ld // 2,)).view(np.uint16)).reshape(16, ld)[:, :N]
+    r.close(got, 0.5 * np.concatenate([O.silu(v[:, :N // 3]), v[:, N // 3:]], axis=1), eight_bits=True)
+    r.go(xd, out=ROWS_F32, y_f32=y.p, ldy=N, bias=bd.p, silu_end=N // 4, tanh_end=N - 7)
+    v = np.concatenate([O.silu(v[:, :N // 4]), np.tanh(v[:, N // 4:N - 7]), v[:, N - 7:]], axis=1)
+    r.close(y.to_host((16, N)), v)
     r.end()
-    for b in (xd, y, y1):
+    for b in (xd, y, y1, bd, ya):
         b.free()
 
 
