@@ -221,30 +221,29 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(wv[t], xv[i], acc[t][i]);
     };
-    constexpr bool HALVES = F32 && GR > 1;
-    if constexpr (HALVES) {
-        // Half a turn is asked for, then the other half multiplied: 32 of these products to a k-step are as long as a
-        // load, and asked for behind them it is late (4096 -> 4096 at 24 rows 26.2 us, 21.2 now).  Past the end the last
-        // step is read again and not used.
-        static_assert(D == 4, "two halves of two");
+    if constexpr (F32) {
+        // Half a turn is asked for, then the other half multiplied: eight 32-bit products to a tile and k-step are as long
+        // as a load, and asked for behind them it is late (4096 -> 4096 at 24 rows 26.2 us, 21.2 now; gated, one row,
+        // 1536 -> 4096 9.8, 8.3).  Past the end the last step is read again and not used.
+        constexpr int H = D / 2;
         auto ask = [&](int d, uint32_t k) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) load(w[d + u], x[d + u], min(k + u, n - 1));
+            for (int u = 0; u < H; u++) load(w[d + u], x[d + u], min(k + u, n - 1));
         };
         auto take = [&](int d, uint32_t k) {
 #pragma unroll
-            for (int u = 0; u < 2; u++)
+            for (int u = 0; u < H; u++)
                 if (k + u < n) multiply(w[d + u], x[d + u]);
         };
         if (n) ask(0, 0);
-        for (uint32_t k = 0; k < n; k += 4) {
-            ask(2, k + 2);
+        for (uint32_t k = 0; k < n; k += D) {
+            ask(H, k + H);
             take(0, k);
-            ask(0, k + 4);
-            take(2, k + 2);
+            ask(0, k + D);
+            take(H, k + H);
         }
     }
-    const uint32_t turns = HALVES ? 0 : n / D, rest = HALVES ? 0 : n - turns * D;
+    const uint32_t turns = F32 ? 0 : n / D, rest = F32 ? 0 : n - turns * D;
     if (turns) {
 #pragma unroll
         for (int d = 0; d < D; d++) load(w[d], x[d], d);

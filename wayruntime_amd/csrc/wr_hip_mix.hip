@@ -599,11 +599,12 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
             if (pairs <= e * 64) return narrow ? launch_lds<4>(a, 1) : launch_split<false, 2, 4, 4, 4, true>(a, 1);
             return a.ntiles <= 64 && pairs < e * 256 ? launch_lds<2>(a, 1) : launch_lds<4>(a, 1);
         }
-        if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 4, true>(a, 1);
+        if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 8, true>(a, 1);
+        if (!gated && a.ntiles * a.groups < 384) return launch_split<false, 1, 1, 4, 8, true>(a, 1);   // (as one group of rows below)
         return launch_split<false, 2, 1, 4, 8, true>(a, 1);
     }
     if (f32) {
-        if (a.groups <= 1) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, batch) : launch_split<true, 1, 1, 4, 4, true>(a, batch);
+        if (a.groups <= 1) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, batch) : launch_split<true, 1, 1, 4, 8, true>(a, batch);
         return launch_split<true, 2, 2, 4, 4, false>(a, batch);
     }
     if (a.groups == 1) {
