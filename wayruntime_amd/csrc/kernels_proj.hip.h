@@ -530,9 +530,9 @@ __device__ __forceinline__ void proj_store_tile(const ProjArgs& a, f32x4 v, uint
 // the bytes and has no activation to work out (once per workgroup, in the kernels that
 // make their own operand terms).  The gate and the value are rounded as they would be
 // stored, so the result has the bits of the product followed by the activation.
-// 1024 -> 2 x 3072 -> 1024, launches of both products (us): one row 6.1 + 6.2 -> 5.8 +
-// 5.4; 16 rows 6.4 + 5.4 (fragments) + 5.9 -> 7.2 + 8.0; 2047 rows 70 + 14.2 + 44 ->
-// 62 + 11.5 + 44.
+// 1024 -> 2 x 3072 -> 1024, both products (us): one row 11.6 -> 10.9 (a whole token, 28
+// of them in 142 launches, shows no more than its spread); 16 rows 6.4 + 5.4 (fragments)
+// + 5.9 -> 7.2 + 8.0; 2047 rows 70 + 14.2 + 44 -> 62 + 11.5 + 44.
 __device__ __forceinline__ uint32_t proj_paired_tile(uint32_t pair, uint32_t t, uint32_t ntiles)
 {
     return min(pair, ntiles / 2 - 1) + t * (ntiles / 2);         // (a pair past the end re-reads the last; dropped)

@@ -993,8 +993,8 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     // one to two thousand waves.  A function of the weight's shape only: a row's
     // sums are then split the same way whether it travels alone or with up to
     // fifteen others, so a batched step's rows equal the serial steps' bit
-    // for bit (reference contract: src/core/batch.c:15-19).  Larger row counts
-    // (prefill chunks) use one wave per run.
+    // for bit (reference contract: src/core/batch.c:15-19).  From 17 rows on the
+    // kernels have splits of their own.
     const uint32_t tiles = w->n_out / 16;
     uint32_t ksplit = 1;
     if (groups <= 2) {
