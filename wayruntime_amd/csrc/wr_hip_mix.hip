@@ -442,8 +442,10 @@ constexpr uint32_t kPartsMinKtiles = 128;
 
 static int launch_parts(MixGemmArgs a)
 {
-    int rc = ensure_device(cx->d_part, (size_t)2 * a.ntiles * 64 * sizeof(f32x4));
-    if (rc) return rc;
+    if (ensure_device(cx->d_part, (size_t)2 * a.ntiles * 64 * sizeof(f32x4)) != WR_HIP_OK) {   // (256 KiB at most)
+        (void)hipGetLastError();
+        return launch_split<false, 1, 1, 4, 8, true>(a, 1);
+    }
     a.part = static_cast<float*>(cx->d_part.p);
     a.tickets = cx->d_counters;
     launch_main(mix_gemm_split_kernel<false, 1, 1, 4, 8, true, 2>, dim3(a.ntiles, 2), dim3(256), a);
