@@ -266,8 +266,7 @@ def test_two_workgroups_to_a_tile(lib, N, K):
 @pytest.mark.parametrize("N,K,runs_each,spare,experts", [
     (64, 352, 1, 1, 3), (2080, 96, 1, 1, 3),                   # few rows an expert: a stream of the weights
     (64, 352, 1, 0, 3), (2080, 96, 1, 0, 3),                   # as many runs as experts, tiles of 128 rows
-    (64, 352, 3, 0, 3), (2080, 96, 3, 0, 3), (1056, 32, 2, 0, 3),
-    (1040, 64, 2, 0, 3), (64, 352, 2, 0, 3),                   # ... of 64 rows, and of 128 on wider weights
+    (64, 352, 3, 0, 3), (2080, 96, 3, 0, 3), (1056, 32, 2, 0, 3), (64, 352, 2, 0, 3),    # ... and more than that
     (144, 2080, 1, 1, 60), (144, 2016, 1, 1, 60),              # narrow weights, a tile to a CU; one input tile fewer
 ])
 def test_runs_whose_last_groups_hold_no_pair(lib, N, K, runs_each, spare, experts):

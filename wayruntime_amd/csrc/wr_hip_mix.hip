@@ -587,19 +587,18 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     if (q->group_expert) {
         if (!f32 && q->tile_groups == 8) {
             // Rows an expert has on average, from how many groups route leaves room for: a run per expert more than the
-            // pairs fill.  Up to 64 the product is a stream of the experts' weights (64 experts of 2048 x 1024, 268 MB, 48
-            // rows each: 64 us against 82 to 89 with the tile of 128 rows, most of them empty) unless they are narrow:
-            // then a stream reads the rows as often as the weights, and tiles that find a CU each are faster from 2048
-            // inputs on (64 experts, 4096 -> 384: 68 us against 97, -> 512 87, 104; 48 experts, 4096 -> 640 77, 89; at 2048
-            // inputs a tenth; 1024 -> 512 the same; 32 experts, 2048 -> 512 30.7, 28.9).
-            // Above, up to 256 rows each, narrow weights take tiles of 64 rows, which skip the empty halves of runs (64 x
-            // (2048 -> 1024), 192 rows each: 115 us against 131; 384 rows, none empty: 182, 172; 4096 -> 2048: 226, 176).
+            // pairs fill.  Up to 48 the product is a stream of the experts' weights: 64 rows of an expert at a time, so most
+            // experts' weights pass once (64 experts of 2048 x 1024, 48 rows each, give or take a third: 67 us against 95
+            // with the tile of 128 rows, most of them empty; 32 of 4096 x 4096 235 against 244).  From 56 on a part of the
+            // experts passes twice (32 of 4096 x 4096 300 against 244, and 334 at 64 rows).
+            // Narrow weights are no stream either: it reads the rows as often as the weights, and tiles that find a CU each
+            // are faster from 2048 inputs on (64 experts, 4096 -> 384: 68 us against 97, -> 512 87, 104; 48 experts, 4096 ->
+            // 640 77, 89; at 2048 inputs a tenth; 1024 -> 512 the same; 32 experts, 2048 -> 512 30.7, 28.9).
             // As many runs as experts, or fewer, are not route's: the caller counted them, so they may be full.
             const uint64_t runs = a.groups / 8, e = q->w->batch, wgs = e * ((a.ntiles + 7) / 8);
-            const uint64_t pairs = runs > e ? (runs - e) * 128 : ~0ull;
+            const bool few = runs > e && (runs - e) * 128 <= e * 48;
             const bool narrow = a.ktiles >= 64 && a.ntiles < 64 && wgs * 10 >= g.n_cus * 4ull && (a.ntiles <= 32 || wgs <= g.n_cus);
-            if (pairs <= e * 64) return narrow ? launch_lds<4>(a, 1) : launch_split<false, 2, 4, 4, 4, true>(a, 1);
-            return a.ntiles <= 64 && pairs < e * 256 ? launch_lds<2>(a, 1) : launch_lds<4>(a, 1);
+            return few && !narrow ? launch_split<false, 2, 4, 4, 4, true>(a, 1) : launch_lds<4>(a, 1);
         }
         if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 8, true>(a, 1);
         if (!gated && a.ntiles * a.groups < 384) return launch_split<false, 1, 1, 4, 8, true>(a, 1);   // (as one group of rows below)
