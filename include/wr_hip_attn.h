@@ -472,6 +472,45 @@ int wr_hip_rows_qkv_append_q16_dev(const float *qkv_dev, uint32_t ld, uint32_t r
 int wr_hip_rows_swiglu_dev(const float *gate_up_dev, uint32_t ld, float *act_dev,
                            uint32_t ldo, uint32_t rows, uint32_t ffn);
 
+/* ---- a decode step's layers in one launch -----------------------------------
+ * The layers of one session's step (the block of src/core/session.c:440-534: norm,
+ * Q/K/V product, head norms, rotation, append, attention, output product, norm, gated
+ * feed-forward), for models whose steps are many short launches in a chain.  The weights of
+ * a layer: wqkv [nq + 2 nkv heads of hd], wo, wgu (gates, then the values they gate), wdown;
+ * norms on the device, q_norm / k_norm both or neither.
+ *
+ * create: WR_HIP_ERR_UNSUPPORTED for a model it is not built for (head_dim other than 128;
+ * products that do not fit one workgroup per compute unit and its registers: inputs that are no
+ * multiple of 512, more than 3072 of them, 1536 of wgu, or more tiles of 16 outputs than units).
+ *
+ * step_dev: row_dev [hidden], the embedded row, becomes the last layer's; K and V of every
+ * layer are appended at `pos`, and bits are those of wr_hip_proj_rows_norm_dev,
+ * wr_hip_attn_append_decode_batched_dev, wr_hip_proj_rows_dev and
+ * wr_hip_proj_rows_gated_dev layer by layer.  cos_sin_dev [n_rot][2].  WR_HIP_ERR_UNSUPPORTED, with
+ * nothing launched: the caller goes layer by layer (generic kernels forced, another alignment, a
+ * stream that records, a session cut into more than 16 key splits, or another thread's step on the
+ * device: the launch's workgroups wait for each other, so one of them runs at a time).
+ *
+ * step_done: every step_dev is followed by one on the same thread, after whatever was
+ * enqueued behind it.  Waits for the thread's stream; WR_HIP_ERR_STATE: a workgroup
+ * waited longer than 50 ms (its peers had no compute unit to run on), nothing of the step
+ * counts, and it is made again layer by layer (as the next 1000 then are).
+ * set_step_limit: that time in ticks of 10 ns, 0 for the default (for tests); steps that
+ * gave up before are forgotten. */
+typedef struct wr_hip_attn_step wr_hip_attn_step;
+typedef struct wr_hip_attn_step_layer {
+    const wr_hip_weight *wqkv, *wo, *wgu, *wdown;
+    const float *attn_norm, *ffn_norm, *q_norm, *k_norm;
+} wr_hip_attn_step_layer;
+int  wr_hip_attn_step_create(uint32_t n_layers, const wr_hip_attn_step_layer *layers,
+                             uint32_t nq, uint32_t nkv, uint32_t hd, float eps,
+                             wr_hip_attn_step **out);
+void wr_hip_attn_step_destroy(wr_hip_attn_step *step);
+int  wr_hip_attn_step_dev(wr_hip_attn_step *step, wr_hip_kv *kv, uint32_t pos, float *row_dev,
+                          const float *cos_sin_dev, uint32_t n_rot, float scale_override);
+int  wr_hip_attn_step_done(void);
+void wr_hip_attn_set_step_limit(uint32_t ticks);
+
 /* Tuning knobs for measurement (0 = automatic): keys handled per workgroup in
  * the split-K decode kernel, and a switch forcing the generic (non-MFMA)
  * kernels.  Not needed by a normal caller. */

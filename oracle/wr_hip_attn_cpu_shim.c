@@ -416,6 +416,20 @@ int wr_hip_proj_rows_gated_dev(const wr_hip_weight *w, uint32_t rows, const floa
     (void)w; (void)rows; (void)x; (void)ldx; (void)nw; (void)eps; (void)gelu; (void)act; (void)ldo;
     return WR_HIP_ERR_STATE;
 }
+int wr_hip_attn_step_create(uint32_t n_layers, const wr_hip_attn_step_layer *layers, uint32_t nq, uint32_t nkv, uint32_t hd,
+                            float eps, wr_hip_attn_step **out)
+{
+    (void)n_layers; (void)layers; (void)nq; (void)nkv; (void)hd; (void)eps; (void)out;
+    return WR_HIP_ERR_STATE;
+}
+void wr_hip_attn_step_destroy(wr_hip_attn_step *step) { (void)step; }
+int wr_hip_attn_step_dev(wr_hip_attn_step *step, wr_hip_kv *kv, uint32_t pos, float *row, const float *cs, uint32_t n_rot,
+                         float scale_override)
+{
+    (void)step; (void)kv; (void)pos; (void)row; (void)cs; (void)n_rot; (void)scale_override;
+    return WR_HIP_ERR_STATE;
+}
+int wr_hip_attn_step_done(void) { return WR_HIP_ERR_STATE; }
 int wr_hip_rows_swiglu_dev(const float *gu, uint32_t ld, float *act, uint32_t ldo, uint32_t rows,
                            uint32_t ffn)
 {

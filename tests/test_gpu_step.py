@@ -1,0 +1,156 @@
+"""A session's decode step as one launch for all layers (wr_hip_attn_step_dev) against the
+chain of launches it stands for: same logits, bit for bit, and the same cache behind them."""
+import ctypes as C
+import threading
+
+import numpy as np
+import pytest
+
+from wayruntime_amd import engine as E, gguf_writer as gw, hipattn
+
+pytestmark = pytest.mark.gpu
+
+VOCAB = 512
+
+
+def test_refusals():
+    """What the launch is not built for is refused before anything is launched."""
+    hipattn.init()
+    lib = hipattn.lib()
+    w = {n: hipattn.Weight([np.zeros(n, np.uint16)]) for n in [(1024, 512), (512, 512), (640, 512), (1024, 640)]}
+    vec = lib.wr_hip_attn_dev_alloc(4096)
+
+    def create(qkv, o, gu, down, nq=4, nkv=2, hd=128):
+        y = hipattn.StepLayer(w[qkv].h, w[o].h, w[gu].h, w[down].h, vec, vec, None, None)
+        h = C.c_void_p()
+        rc = lib.wr_hip_attn_step_create(1, C.byref(y), nq, nkv, hd, 1e-6, C.byref(h))
+        return rc, h
+
+    rc, h = create((1024, 512), (512, 512), (1024, 512), (512, 512))
+    assert rc == hipattn.OK
+    assert create((1024, 512), (512, 512), (1024, 512), (512, 512), hd=64)[0] == hipattn.ERR_UNSUPPORTED
+    assert create((640, 512), (512, 512), (1024, 512), (512, 512))[0] == hipattn.ERR_UNSUPPORTED
+    assert create((1024, 640), (512, 512), (1024, 512), (512, 512))[0] == hipattn.ERR_UNSUPPORTED
+    assert create((1024, 512), (512, 512), (1024, 512), (512, 512), nq=3)[0] == hipattn.ERR_INVAL
+    kv = hipattn.KVCache(1, 128, 2, 64)
+    other = hipattn.KVCache(1, 64, 2, 64)
+    assert lib.wr_hip_attn_step_dev(h, kv.h, 64, vec, None, 0, 0.0) == hipattn.ERR_CTX_FULL
+    assert lib.wr_hip_attn_step_dev(h, other.h, 0, vec, None, 0, 0.0) == hipattn.ERR_INVAL
+    assert lib.wr_hip_attn_step_dev(h, kv.h, 0, vec, None, 8, 0.0) == hipattn.ERR_INVAL
+    assert lib.wr_hip_attn_step_dev(h, kv.h, 0, vec + 4, None, 0, 0.0) == hipattn.ERR_UNSUPPORTED
+    lib.wr_hip_attn_set_tuning(0, 1)
+    try:
+        assert lib.wr_hip_attn_step_dev(h, kv.h, 0, vec, None, 0, 0.0) == hipattn.ERR_UNSUPPORTED
+    finally:
+        lib.wr_hip_attn_set_tuning(0, 0)
+    lib.wr_hip_attn_step_destroy(h)
+    for x in (kv, other):
+        x.close()
+    for x in w.values():
+        x.close()
+    lib.wr_hip_attn_dev_free(vec)
+
+
+@pytest.fixture(scope="module")
+def eng():
+    hipattn.shutdown()
+    e = E.Engine(E.HOST_SO)
+    yield e
+    e.close()
+
+
+def _models(eng, tmp_path, monkeypatch, **shape):
+    """The model with its steps in one launch, and as a chain."""
+    p = str(tmp_path / "m.gguf")
+    gw.write_model(p, gw.ModelShape(head_dim=128, vocab=VOCAB, context=8192, **shape), std=0.08)
+    out = []
+    for chain in ("0", "1"):
+        monkeypatch.setenv("WAYRT_STEP_LAUNCHES", chain)
+        out.append(eng.load(p, max_context=8192))
+    return out
+
+
+def _steps(model, prompt, tokens):
+    s = model.session()
+    if len(prompt):
+        assert s.prefill(prompt) == len(prompt)
+    rows = [np.array(s.step(int(t))) for t in tokens]
+    # the cache that the steps left: a prompt pass over it
+    assert s.prefill(tokens) == len(tokens)
+    rows.append(np.array(s.step(int(tokens[0]))))
+    s.close()
+    return rows
+
+
+def _launches(model):
+    lib, ms, n = hipattn.lib(), C.c_double(), C.c_uint32()
+    s = model.session()
+    assert lib.wr_hip_attn_profile_begin(1000) == hipattn.OK
+    s.step(1)
+    assert lib.wr_hip_attn_profile_end(C.byref(ms), C.byref(n)) == hipattn.OK
+    s.close()
+    return n.value
+
+
+# the fewest inputs and the most that a wave holds; KV groups of 1 to 8; with head norms and without
+@pytest.mark.parametrize("shape", [
+    dict(n_layers=2, hidden=512, ffn=512, n_q=4, n_kv=4),
+    dict(n_layers=1, hidden=512, ffn=2560, n_q=8, n_kv=1),
+    dict(n_layers=3, hidden=1536, ffn=3072, n_q=12, n_kv=3),
+    dict(n_layers=2, hidden=1024, ffn=1536, n_q=24, n_kv=3),
+    dict(n_layers=2, hidden=1024, ffn=3072, n_q=16, n_kv=8, arch="llama"),
+])
+def test_one_launch_equals_the_chain(eng, tmp_path, monkeypatch, shape):
+    one, chain = _models(eng, tmp_path, monkeypatch, **shape)
+    rng = np.random.default_rng(5)
+    # nothing cached; ends of a tile; the last split on its own; splits of a short, a medium and a long session
+    for n in (0, 1, 30, 31, 32, 33, 159, 160, 161, 300, 1000, 2047, 2100, 4096, 8100):
+        prompt, tokens = rng.integers(0, VOCAB, n).astype(np.uint32), rng.integers(0, VOCAB, 4).astype(np.uint32)
+        for a, b in zip(_steps(one, prompt, tokens), _steps(chain, prompt, tokens)):
+            assert np.isfinite(b).all() and np.array_equal(a, b), n
+    # (the layers and the LM head; five launches a layer and the head)
+    assert _launches(one) == 2 and _launches(chain) == 5 * shape["n_layers"] + 1
+    for m in (one, chain):
+        m.close()
+
+
+def test_a_step_that_gives_up_is_made_again(eng, tmp_path, monkeypatch):
+    one, chain = _models(eng, tmp_path, monkeypatch, n_layers=2, hidden=1024, ffn=3072, n_q=16, n_kv=8)
+    rng = np.random.default_rng(6)
+    prompt, tokens = rng.integers(0, VOCAB, 200).astype(np.uint32), rng.integers(0, VOCAB, 5).astype(np.uint32)
+    lib = hipattn.lib()
+    calls = eng.counters()[E.WR_CTR_ATTENTION_CALLS]
+    want = _steps(chain, prompt, tokens)
+    a_run = eng.counters()[E.WR_CTR_ATTENTION_CALLS] - calls
+    lib.wr_hip_attn_set_step_limit(1)            # every wait ends at once, the launch runs through without its rows
+    try:
+        got = _steps(one, prompt, tokens)
+    finally:
+        lib.wr_hip_attn_set_step_limit(0)
+    assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    assert all(np.array_equal(a, b) for a, b in zip(_steps(one, prompt, tokens), want))
+    assert eng.counters()[E.WR_CTR_ATTENTION_CALLS] - calls == 3 * a_run
+    for m in (one, chain):
+        m.close()
+
+
+def test_threads_step_beside_each_other(eng, tmp_path, monkeypatch):
+    """One launch at a time is on the device; whoever comes second takes the chain, and nobody sees a difference."""
+    one, chain = _models(eng, tmp_path, monkeypatch, n_layers=4, hidden=1024, ffn=3072, n_q=16, n_kv=8)
+    rng = np.random.default_rng(7)
+    work = [(rng.integers(0, VOCAB, 40 + 90 * i).astype(np.uint32), rng.integers(0, VOCAB, 24).astype(np.uint32)) for i in range(4)]
+    want = [_steps(chain, *w) for w in work]
+    got = [None] * 4
+
+    def run(i):
+        got[i] = _steps(one, *work[i])
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g, w in zip(got, want):
+        assert g is not None and all(np.array_equal(a, b) for a, b in zip(g, w))
+    for m in (one, chain):
+        m.close()

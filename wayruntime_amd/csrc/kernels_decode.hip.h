@@ -40,6 +40,8 @@
 // across the four 16-lane groups and one with the partner column.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hip.h"
 #include "row8.hip.h"
 
@@ -162,6 +164,27 @@ static_assert(sizeof(DecodeArgs::items) == kBatchMax * kMaxSplits * sizeof(uint1
 // device-wide release fence instead would write back the whole L2
 // (buffer_wbl2) from every workgroup: measured at 5-10x the kernel's run time. (part_store, part_load: common.hip.h.)
 
+// One element of a merged row from its partials' values and (m, l): log-sum-exp over the splits, one normalisation.
+template <int N>
+__device__ __forceinline__ float merge_partials(const float (&v)[N], float (&m)[N], const float (&l)[N], uint32_t n_splits)
+{
+    float M = -INFINITY;
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)N; i++)
+        if (i < n_splits) M = fmaxf(M, m[i]);
+    float L = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)N; i++) {
+        m[i] = (i < n_splits) ? fast_exp2(m[i] - M) : 0.f;
+        L += l[i] * m[i];
+    }
+    const float inv = (L > 0.f) ? 1.0f / L : 0.f;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)N; i++) acc[i & 3] += v[i] * (m[i] * inv);
+    return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+}
+
 // Merge of up to N partials per head, everything a thread needs asked for at
 // once: its output element's partial values and the head's (m, l) pairs; the
 // thread works the weights out for itself.  One trip to memory instead of two
@@ -184,21 +207,7 @@ __device__ __forceinline__ void merge_in_regs(const DecodeArgs& a, uint32_t sess
             m[i] = part_load(&a.part_ml[(p0 + ii) * 2]);
             l[i] = part_load(&a.part_ml[(p0 + ii) * 2 + 1]);
         }
-        float M = -INFINITY;
-#pragma unroll
-        for (uint32_t i = 0; i < (uint32_t)N; i++)
-            if (i < n_splits) M = fmaxf(M, m[i]);
-        float L = 0.f;
-#pragma unroll
-        for (uint32_t i = 0; i < (uint32_t)N; i++) {
-            m[i] = (i < n_splits) ? fast_exp2(m[i] - M) : 0.f;
-            L += l[i] * m[i];
-        }
-        const float inv = (L > 0.f) ? 1.0f / L : 0.f;
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (uint32_t i = 0; i < (uint32_t)N; i++) acc[i & 3] += v[i] * (m[i] * inv);
-        a.out[((size_t)sess * a.nq + head0 + h) * hd + d] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        a.out[((size_t)sess * a.nq + head0 + h) * hd + d] = merge_partials<N>(v, m, l, n_splits);
     }
 }
 
@@ -478,22 +487,27 @@ __device__ __forceinline__ void patch_new_row(DecodeFrag<HD>& f, const DecodeNew
     }
     if (g == (p >> 3)) {
         // element p % 8 of eight halves = one half of 32-bit word (p % 8) / 2: a
-        // bit-field insert per word and a select on the word index, not a chain
-        // of selects per half (this runs once per launch, in one wave, with the
-        // rest of the workgroup waiting for that wave's tile: its length in
-        // instructions is what it costs)
-        const uint32_t e = p & 7, w = e >> 1;
+        // bit-field insert in that word, and a branch on the word's index, which is the same for the launch
+        // (this runs once per launch, in one wave, with the rest of the
+        // workgroup waiting for that wave's tile: its length in instructions is
+        // what it costs; inserts and selects in every word took 0.4 us more)
+        const uint32_t e = p & 7;
         const uint32_t keep = (e & 1) ? 0x0000FFFFu : 0xFFFF0000u;
+        const auto put = [&](auto word) {
+            constexpr int w = decltype(word)::value;
 #pragma unroll
-        for (int dt = 0; dt < HD / 16; dt++) {
-            const uint32_t both = (uint32_t)nr.v[dt * 16 + m] * 0x10001u;
-            u32x4 words = __builtin_bit_cast(u32x4, f.v[dt]);
-#pragma unroll
-            for (int wi = 0; wi < 4; wi++) {
-                const uint32_t nw = (words[wi] & keep) | (both & ~keep);
-                words[wi] = ((uint32_t)wi == w) ? nw : words[wi];
+            for (int dt = 0; dt < HD / 16; dt++) {
+                const uint32_t both = (uint32_t)nr.v[dt * 16 + m] * 0x10001u;
+                u32x4 words = __builtin_bit_cast(u32x4, f.v[dt]);
+                words[w] = (words[w] & keep) | (both & ~keep);
+                f.v[dt] = __builtin_bit_cast(half8, words);
             }
-            f.v[dt] = __builtin_bit_cast(half8, words);
+        };
+        switch (__builtin_amdgcn_readfirstlane((int)(e >> 1))) {
+        case 0: put(std::integral_constant<int, 0>()); break;
+        case 1: put(std::integral_constant<int, 1>()); break;
+        case 2: put(std::integral_constant<int, 2>()); break;
+        default: put(std::integral_constant<int, 3>()); break;
         }
     }
 }

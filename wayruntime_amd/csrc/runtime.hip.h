@@ -40,11 +40,12 @@ struct Ctx {
     // Error word: page-locked host memory that kernels can write.  A kernel that
     // gives up a bounded wait (and so goes on with data it cannot vouch for) stores
     // (bit 31 | layer) there; the host reads it after every wait for the
-    // stream (no copy, no extra latency).  None of the present kernels waits on
-    // anything but the hardware barrier, so nothing writes it today; a kernel that
-    // spins on a flag must bound the spin and report here.
+    // stream (no copy, no extra latency).  Nothing writes it today.  The word behind it is
+    // step_layers_kernel's, whose waits are bounded: set when one met its deadline, and
+    // read by wr_hip_attn_step_done, after which the step is made another way.
     volatile uint32_t* err_host = nullptr;
     uint32_t* err_dev = nullptr;
+    uint32_t step_calls = 0;          // attention calls that the last step in one launch counted
     Buffer h_pin;                // pinned host staging
     std::vector<hipEvent_t> ev;  // kernel timing (profile_begin / profile_end of this thread)
     uint32_t ev_used = 0;
@@ -74,6 +75,9 @@ struct Lib {
     std::atomic<int> force_generic{0};
     std::atomic<uint32_t> prefill_part_mb{kMaxPrefillPartMb};    // WR_HIP_PREFILL_PART_MB: a thread's parts take no more; 0: no block is cut
     std::atomic<int> prefill_256_four_waves{0};   // WR_HIP_PREFILL_256_FOUR_WAVES=1: head dim 256 keeps the earlier four-wave prefill kernel
+    std::atomic<Ctx*> step_owner{nullptr};       // whose launch of a whole step's layers may be on the device (one at a time)
+    std::atomic<uint32_t> step_refused{0};       // steps that go layer by layer before one launch is tried again
+    std::atomic<uint32_t> step_limit{0};         // ticks until its waits end; 0: kStepLimitTicks
     std::atomic<int> prefill_two_waves{1};        // WR_HIP_PREFILL_TWO_WAVES=0: head dim 128 takes the one-wave-per-SIMD prefill kernel
 };
 extern Lib g;

@@ -27,6 +27,7 @@
 #include "kernels_prefill_ild.hip.h"
 #include "kernels_proj.hip.h"
 #include "kernels_rows.hip.h"
+#include "kernels_step.hip.h"
 
 using namespace wr;
 
@@ -62,6 +63,17 @@ struct wr_hip_kv {
     size_t vt_off[WR_HIP_MAX_LAYERS];
     uint8_t* slab;
     size_t bytes;
+};
+
+// What a model's steps in one launch keep: the layers' weights as the kernel reads them, and the rows that travel
+// between its workgroups.  Used by one launch at a time (Lib::step_owner).
+struct wr_hip_attn_step {
+    uint32_t n_layers, hidden, ffn, nq, nkv;
+    float eps;
+    StepLayer* layers;                   // device
+    u32x4* rows;                         // device: tagged rows, then partial rows
+    size_t row_bytes;
+    uint32_t next_tag;
 };
 
 namespace wr {
@@ -257,6 +269,95 @@ struct DecodeWorkspace {
     size_t bytes = 0;
 };
 
+struct SplitRule {
+    uint32_t tiles_per_wg, tail, n_splits;
+    bool pairs, shorts;      // long and short sessions, whose splits may share a workgroup
+};
+
+// The rule looks at ONE session only (its own visible
+// key range), never at the rest of the batch: a session's arithmetic is then
+// the same whether it is stepped alone or with others, which is what makes
+// the batched step bit-identical to serial steps (reference contract:
+// src/core/batch.c:15-19).  Half a MiB of K+V per workgroup (1024 keys at
+// head_dim 128, 512 at 256): 16 sessions of 4096 run as fast with it as
+// with twice that, and a single session's chain of tiles is half as long
+// (one session of 8192 keys: 27 -> 17 us); from
+// 8K keys up an eighth of the session per workgroup measured better
+// (fewer partials and workgroup turnovers: 82 % -> 86 % of HBM peak at
+// 16 x 32768).  A short session (up to 2048 keys at head_dim 128) takes a
+// quarter of that per workgroup: its launch is a chain of latencies, and a
+// workgroup that has all its tiles in flight at once ends sooner than one
+// that walks eight of them per wave (one session of 1024 keys: 12.0 -> 7.8 us,
+// of 2048: 13.8 -> 8.2 us; 16 sessions of ~520: the step of a 28-layer model
+// 2.03 -> 1.89 ms).  A medium session (more than 2048 and fewer than 4096 keys)
+// takes half: one session of 3000 keys 14 -> 10.6 us, the ragged batch of 16
+// 35.2 -> 34.6 us; at 4096 keys and beyond the full figure stands (16 x 4096
+// loses 4-8 % with halves).  The session's tiles are spread evenly over the workgroups,
+// and the floor keeps the in-kernel merge within kMaxSplits partials.
+// A long session (from 8K keys up at head_dim 128) is cut into twice as
+// many splits as it gets workgroups in a full launch, and a workgroup there
+// works through two consecutive splits, one after the other: the unit of
+// arithmetic (a split: one partial, the tiles dealt to the four waves in
+// turn) stays a function of the session alone, while a launch too small to
+// give every CU a workgroup sends each split to a workgroup of its own.
+// One session of 8192 keys: 64 -> 128 workgroups, 14.8 -> 11.2 us; of 16384:
+// 24.5 -> 16.2; of 32768: 43.9 -> 26.9.  The price in a full launch is one
+// extra merge of the four waves per workgroup: not measurable at 16 x 32768.
+// (The same from 4096 keys up costs 16 x 4096 4.5 %: those workgroups have
+// 32 tiles, and the waves meeting in the middle is 2 us of their 40.)
+// A caller that serves one session at a time can go further with
+// wr_hip_attn_set_tuning.
+SplitRule split_rule(uint32_t tiles, uint32_t hd, bool use_mfma, uint32_t tune)
+{
+    SplitRule r{};
+    uint32_t tpw, tail = 0;
+    if (tune) {
+        tpw = tune / kTileKeys;
+        if (tpw == 0) tpw = 1;
+    } else {
+        uint32_t cap = kDefaultTilesPerWg * 128u / (hd < 32 ? 32 : hd);
+        if (cap == 0) cap = 1;
+        if (tiles <= 2 * cap) {                                  // a short session: see above
+            cap = cap >= 4 ? cap / 4 : 1;
+            // ... whose LAST four tiles are a split of their own: one tile per
+            // wave.  In a decode step the last tile holds the new position: the
+            // workgroup that has it also makes the new row's K and V and patches
+            // them in, and with a full share of tiles on top it finishes last and
+            // the merge waits for it (timestamps: its ticket 2 us after the
+            // others').  With one tile per wave it finishes first, and a workgroup
+            // that is done anyway merges: the decode step of a 28-layer model at
+            // ~520 keys 1.02 -> 1.00 ms, sixteen sessions 1.90 -> 1.87 ms.  (A tail
+            // of ONE tile does the same for one session and costs sixteen 2-3 %:
+            // it adds a workgroup per session and KV head.)  A caller that has
+            // appended the row itself pays for the extra split instead: one
+            // session of 1024 keys 7.8 -> 8.2 us, of 2048 keys 8.1 -> 8.8 us.
+            if (tiles >= 6) tail = 4;
+            // In a launch that would not find a place for every split at once two
+            // consecutive splits of a short session share a workgroup as well (the
+            // splits keep their size): see below.
+            r.shorts = use_mfma && hd <= 128;
+        } else if (tiles < 4 * cap) {
+            cap = cap >= 2 ? cap / 2 : 1;                           // a medium one: see above
+        } else if (cap <= tiles / 8) {
+            cap = tiles / 8;
+            r.pairs = use_mfma && hd <= 128;                       // a long one: see above
+        }
+        const uint32_t body = tiles - tail;
+        const uint32_t want = (body + cap - 1) / cap;              // workgroups
+        tpw = (body + want - 1) / want;                            // even share
+        if (r.pairs) tpw = (tpw + 1) / 2;                         // two splits per workgroup
+        if (r.shorts) r.pairs = true;
+    }
+    const uint32_t body = tiles - tail;
+    const uint32_t room = kMaxSplits - (tail ? 1u : 0u);
+    const uint32_t floor_tiles = (body + room - 1) / room;
+    if (tpw < floor_tiles) tpw = floor_tiles;
+    r.tiles_per_wg = tpw;
+    r.tail = tail;
+    r.n_splits = (body + tpw - 1) / tpw + (tail ? 1u : 0u);
+    return r;
+}
+
 int decode_locked(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32_t* seq_k,
                   const float* q_dev, float* out_dev, uint32_t nq, float scale_override,
                   uint32_t window, const DecodeWorkspace& fixed = DecodeWorkspace(),
@@ -268,7 +369,6 @@ int decode_locked(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32
 
     DecodeArgs a;
     memset(&a, 0, sizeof a);
-    uint64_t tiles_total = 0;
     uint32_t tiles[kBatchMax];
     for (uint32_t i = 0; i < n; i++) {
         DecodeSession& s = a.s[i];
@@ -278,95 +378,20 @@ int decode_locked(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32
         s.key_lo = key_lo_for(window, seq_k[i]);
         s.ctx_pad = kv[i]->ctx_pad;
         tiles[i] = (s.seq_k + kTileKeys - 1) / kTileKeys - s.key_lo / kTileKeys;
-        tiles_total += tiles[i];
     }
 
-    // Keys per workgroup.  The rule looks at ONE session only (its own visible
-    // key range), never at the rest of the batch: a session's arithmetic is then
-    // the same whether it is stepped alone or with others, which is what makes
-    // the batched step bit-identical to serial steps (reference contract:
-    // src/core/batch.c:15-19).  Half a MiB of K+V per workgroup (1024 keys at
-    // head_dim 128, 512 at 256): 16 sessions of 4096 run as fast with it as
-    // with twice that, and a single session's chain of tiles is half as long
-    // (one session of 8192 keys: 27 -> 17 us); from
-    // 8K keys up an eighth of the session per workgroup measured better
-    // (fewer partials and workgroup turnovers: 82 % -> 86 % of HBM peak at
-    // 16 x 32768).  A short session (up to 2048 keys at head_dim 128) takes a
-    // quarter of that per workgroup: its launch is a chain of latencies, and a
-    // workgroup that has all its tiles in flight at once ends sooner than one
-    // that walks eight of them per wave (one session of 1024 keys: 12.0 -> 7.8 us,
-    // of 2048: 13.8 -> 8.2 us; 16 sessions of ~520: the step of a 28-layer model
-    // 2.03 -> 1.89 ms).  A medium session (more than 2048 and fewer than 4096 keys)
-    // takes half: one session of 3000 keys 14 -> 10.6 us, the ragged batch of 16
-    // 35.2 -> 34.6 us; at 4096 keys and beyond the full figure stands (16 x 4096
-    // loses 4-8 % with halves).  The session's tiles are spread evenly over the workgroups,
-    // and the floor keeps the in-kernel merge within kMaxSplits partials.
-    // A long session (from 8K keys up at head_dim 128) is cut into twice as
-    // many splits as it gets workgroups in a full launch, and a workgroup there
-    // works through two consecutive splits, one after the other: the unit of
-    // arithmetic (a split: one partial, the tiles dealt to the four waves in
-    // turn) stays a function of the session alone, while a launch too small to
-    // give every CU a workgroup sends each split to a workgroup of its own.
-    // One session of 8192 keys: 64 -> 128 workgroups, 14.8 -> 11.2 us; of 16384:
-    // 24.5 -> 16.2; of 32768: 43.9 -> 26.9.  The price in a full launch is one
-    // extra merge of the four waves per workgroup: not measurable at 16 x 32768.
-    // (The same from 4096 keys up costs 16 x 4096 4.5 %: those workgroups have
-    // 32 tiles, and the waves meeting in the middle is 2 us of their 40.)
-    // A caller that serves one session at a time can go further with
-    // wr_hip_attn_set_tuning.
-    (void)tiles_total;
     uint32_t max_splits = 1;
     const uint32_t tune = g.tune_keys_per_wg.load(std::memory_order_relaxed);
     bool pairs[kBatchMax], shorts[kBatchMax];
     uint32_t wgs_paired = 0, wgs_shorts_alone = 0;
     for (uint32_t i = 0; i < n; i++) {
-        uint32_t tpw, tail = 0;
-        pairs[i] = shorts[i] = false;
-        if (tune) {
-            tpw = tune / kTileKeys;
-            if (tpw == 0) tpw = 1;
-        } else {
-            uint32_t cap = kDefaultTilesPerWg * 128u / (hd < 32 ? 32 : hd);
-            if (cap == 0) cap = 1;
-            if (tiles[i] <= 2 * cap) {                                  // a short session: see above
-                cap = cap >= 4 ? cap / 4 : 1;
-                // ... whose LAST four tiles are a split of their own: one tile per
-                // wave.  In a decode step the last tile holds the new position: the
-                // workgroup that has it also makes the new row's K and V and patches
-                // them in, and with a full share of tiles on top it finishes last and
-                // the merge waits for it (timestamps: its ticket 2 us after the
-                // others').  With one tile per wave it finishes first, and a workgroup
-                // that is done anyway merges: the decode step of a 28-layer model at
-                // ~520 keys 1.02 -> 1.00 ms, sixteen sessions 1.90 -> 1.87 ms.  (A tail
-                // of ONE tile does the same for one session and costs sixteen 2-3 %:
-                // it adds a workgroup per session and KV head.)  A caller that has
-                // appended the row itself pays for the extra split instead: one
-                // session of 1024 keys 7.8 -> 8.2 us, of 2048 keys 8.1 -> 8.8 us.
-                if (tiles[i] >= 6) tail = 4;
-                // In a launch that would not find a place for every split at once two
-                // consecutive splits of a short session share a workgroup as well (the
-                // splits keep their size): see below.
-                shorts[i] = use_mfma && hd <= 128;
-            } else if (tiles[i] < 4 * cap) {
-                cap = cap >= 2 ? cap / 2 : 1;                           // a medium one: see above
-            } else if (cap <= tiles[i] / 8) {
-                cap = tiles[i] / 8;
-                pairs[i] = use_mfma && hd <= 128;                       // a long one: see above
-            }
-            const uint32_t body = tiles[i] - tail;
-            const uint32_t want = (body + cap - 1) / cap;              // workgroups
-            tpw = (body + want - 1) / want;                            // even share
-            if (pairs[i]) tpw = (tpw + 1) / 2;                         // two splits per workgroup
-            if (shorts[i]) pairs[i] = true;
-        }
-        const uint32_t body = tiles[i] - tail;
-        const uint32_t room = kMaxSplits - (tail ? 1u : 0u);
-        const uint32_t floor_tiles = (body + room - 1) / room;
-        if (tpw < floor_tiles) tpw = floor_tiles;
-        a.s[i].tiles_per_wg = tpw;
-        a.s[i].tail_tiles = (uint16_t)tail;
+        const SplitRule r = split_rule(tiles[i], hd, use_mfma, tune);
+        pairs[i] = r.pairs;
+        shorts[i] = r.shorts;
+        a.s[i].tiles_per_wg = r.tiles_per_wg;
+        a.s[i].tail_tiles = (uint16_t)r.tail;
         a.s[i].parts_per_wg = 1;
-        a.s[i].n_splits = (body + tpw - 1) / tpw + (tail ? 1u : 0u);
+        a.s[i].n_splits = r.n_splits;
         if (a.s[i].n_splits > max_splits) max_splits = a.s[i].n_splits;
         const uint32_t halves = (a.s[i].n_splits + 1) / 2;
         wgs_paired += pairs[i] ? halves : a.s[i].n_splits;
@@ -1273,6 +1298,9 @@ void wr_hip_attn_shutdown(void)
     g.device = -1;
     g.tune_keys_per_wg = 0;
     g.force_generic = 0;
+    g.step_owner = nullptr;
+    g.step_refused = 0;
+    g.step_limit = 0;
 }
 
 void wr_hip_attn_set_log(wr_hip_log_fn fn, void* user)
@@ -1651,6 +1679,203 @@ int wr_hip_attn_append_decode_batched_dev(uint32_t n, wr_hip_kv* const* kv, uint
     fz.eps = eps;
     ENTER();
     return decode_locked(n, kv, layer, seq_k, nullptr, out_dev, nq, scale_override, window, DecodeWorkspace(), &fz);
+}
+
+// ------------------------------------------- a decode step's layers in one launch --
+
+namespace {
+
+constexpr uint32_t kStepRefusedSteps = 1000;   // steps that take the chain of launches after a wait has met its deadline
+
+// Inputs and outputs of a product that a wave's registers hold a quarter of, four waves to the inputs (the rule
+// of proj_chunk_locked), a tile (pair) to a workgroup.
+bool step_product_ok(const wr_hip_weight* w, uint32_t n_in, uint32_t n_out, bool gated)
+{
+    if (!w || w->n_in != n_in || w->n_out != n_out) return false;
+    const uint32_t tiles = n_out / 16, per_wave = n_in / 128;      // k-steps; in fours
+    return n_in % 512 == 0 && per_wave <= kStepTiles / (gated ? 2 : 1) && tiles * 2 < 2048 &&
+           tiles / (gated ? 2 : 1) <= g.n_cus;
+}
+
+size_t step_part_bytes(uint32_t nq) { return (size_t)nq * kMergeInRegs * (128 + 2) * sizeof(uint64_t); }
+
+}  // namespace
+
+int wr_hip_attn_step_create(uint32_t n_layers, const wr_hip_attn_step_layer* layers, uint32_t nq, uint32_t nkv, uint32_t hd,
+                            float eps, wr_hip_attn_step** out)
+{
+    if (!out) return WR_HIP_ERR_INVAL;
+    *out = nullptr;
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    if (n_layers == 0 || !layers || nq == 0 || nkv == 0 || nq % nkv != 0) return WR_HIP_ERR_INVAL;
+    if (n_layers > WR_HIP_MAX_LAYERS) return WR_HIP_ERR_LIMIT;
+    for (uint32_t l = 0; l < n_layers; l++) {
+        const wr_hip_attn_step_layer& y = layers[l];
+        if (!y.wqkv || !y.wo || !y.wgu || !y.wdown || !y.attn_norm || !y.ffn_norm) return WR_HIP_ERR_INVAL;
+        if ((y.q_norm == nullptr) != (y.k_norm == nullptr)) return WR_HIP_ERR_INVAL;
+    }
+    const uint32_t hidden = layers[0].wqkv->n_in, ffn = layers[0].wdown->n_in;
+    if (hd != 128 || nq / nkv > (uint32_t)kMaxGroupMfma || nq > kMaxHeads) return WR_HIP_ERR_UNSUPPORTED;
+    StepLayer host[WR_HIP_MAX_LAYERS];
+    for (uint32_t l = 0; l < n_layers; l++) {
+        const wr_hip_attn_step_layer& y = layers[l];
+        const uintptr_t addrs = (uintptr_t)y.attn_norm | (uintptr_t)y.ffn_norm | (uintptr_t)y.q_norm | (uintptr_t)y.k_norm;
+        if (addrs % 16 != 0 || !step_product_ok(y.wqkv, hidden, (nq + 2 * nkv) * hd, false) ||
+            !step_product_ok(y.wo, nq * hd, hidden, false) || !step_product_ok(y.wgu, hidden, 2 * ffn, true) ||
+            !step_product_ok(y.wdown, ffn, hidden, false))
+            return WR_HIP_ERR_UNSUPPORTED;
+        host[l] = StepLayer{reinterpret_cast<const half8*>(y.wqkv->tiles), reinterpret_cast<const half8*>(y.wo->tiles),
+                            reinterpret_cast<const half8*>(y.wgu->tiles), reinterpret_cast<const half8*>(y.wdown->tiles),
+                            y.attn_norm, y.ffn_norm, y.q_norm, y.k_norm};
+    }
+    wr_hip_attn_step* p = new (std::nothrow) wr_hip_attn_step();
+    if (!p) return WR_HIP_ERR_NOMEM;
+    p->n_layers = n_layers;
+    p->hidden = hidden;
+    p->ffn = ffn;
+    p->nq = nq;
+    p->nkv = nkv;
+    p->eps = eps;
+    p->next_tag = 2;                     // (a cleared row bears tag 0, the row ahead of the first layer is not tagged)
+    p->row_bytes = (size_t)(kStepCopies * (2 * step_row_units(hidden) + step_row_units(nq * hd) + step_row_units(ffn)) +
+                            step_row_units((nq + 2 * nkv) * hd)) * 16 + step_part_bytes(nq);
+    Entered entered_;
+    int rc = entered_.ok() ? WR_HIP_OK : WR_HIP_ERR_NOMEM;
+    if (rc == WR_HIP_OK && (hipMalloc((void**)&p->layers, n_layers * sizeof(StepLayer)) != hipSuccess ||
+                            hipMalloc((void**)&p->rows, p->row_bytes) != hipSuccess))
+        rc = WR_HIP_ERR_NOMEM;
+    if (rc == WR_HIP_OK) {
+        hipError_t e = hipMemcpyAsync(p->layers, host, n_layers * sizeof(StepLayer), hipMemcpyHostToDevice, cx->stream);
+        if (e == hipSuccess) e = hipMemsetAsync(p->rows, 0, p->row_bytes, cx->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(cx->stream);
+        if (e != hipSuccess) rc = hip_fail(e, "step plan", 0);
+    }
+    if (rc != WR_HIP_OK) {
+        (void)hipGetLastError();
+        wr_hip_attn_step_destroy(p);
+        return rc;
+    }
+    *out = p;
+    return WR_HIP_OK;
+}
+
+void wr_hip_attn_step_destroy(wr_hip_attn_step* p)
+{
+    if (!p) return;
+    if (g.inited) {
+        Entered entered_;
+        if (entered_.ok()) (void)hipStreamSynchronize(cx->stream);
+        if (p->layers) (void)hipFree(p->layers);
+        if (p->rows) (void)hipFree(p->rows);
+    }
+    delete p;
+}
+
+void wr_hip_attn_set_step_limit(uint32_t ticks)
+{
+    g.step_limit = ticks;
+    g.step_refused = 0;
+}
+
+int wr_hip_attn_step_dev(wr_hip_attn_step* p, wr_hip_kv* kv, uint32_t pos, float* row_dev, const float* cos_sin_dev,
+                         uint32_t n_rot, float scale_override)
+{
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    if (!p || !kv || !row_dev || (n_rot > 0 && !cos_sin_dev) || n_rot > 64) return WR_HIP_ERR_INVAL;
+    if (kv->n_layers != p->n_layers || kv->nkv != p->nkv) return WR_HIP_ERR_INVAL;
+    for (uint32_t l = 0; l < kv->n_layers; l++)
+        if (kv->hd[l] != 128) return WR_HIP_ERR_INVAL;
+    if (pos >= kv->max_ctx) return WR_HIP_ERR_CTX_FULL;
+    if (n_rot % 8 != 0 || (((uintptr_t)row_dev | (uintptr_t)cos_sin_dev) & 15) || !mfma_shape(128, p->nq / p->nkv))
+        return WR_HIP_ERR_UNSUPPORTED;
+    const uint32_t tiles = (pos + kTileKeys) / kTileKeys;
+    const SplitRule r = split_rule(tiles, 128, true, g.tune_keys_per_wg.load(std::memory_order_relaxed));
+    if (r.n_splits > (uint32_t)kMergeInRegs || p->nkv * r.n_splits > g.n_cus) return WR_HIP_ERR_UNSUPPORTED;
+    ENTER();
+    // A launch that is recorded would run again with the same tags.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(cx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return WR_HIP_ERR_UNSUPPORTED;
+    }
+    if (g.step_refused.load(std::memory_order_relaxed) > 0) {
+        g.step_refused.fetch_sub(1, std::memory_order_relaxed);
+        return WR_HIP_ERR_UNSUPPORTED;
+    }
+    // Two launches whose workgroups wait for each other could each hold CUs the other needs: one at a time.
+    Ctx* nobody = nullptr;
+    if (!g.step_owner.compare_exchange_strong(nobody, cx, std::memory_order_acq_rel) && nobody != cx) return WR_HIP_ERR_UNSUPPORTED;
+
+    if (p->next_tag > 0xFFFFFFFFu - 2 * p->n_layers) {
+        // Tags begin again: what the rows still hold must not look like one to come.
+        const uint32_t words = (uint32_t)(p->row_bytes / 4);
+        hipLaunchKernelGGL(fill_u32_kernel, dim3((words + 255) / 256), dim3(256), 0, cx->stream, reinterpret_cast<uint32_t*>(p->rows), words, 0u);
+        p->next_tag = 2;
+    }
+    StepArgs a;
+    memset(&a, 0, sizeof a);
+    a.layers = p->layers;
+    a.x0 = row_dev;
+    a.y = row_dev;
+    a.cos_sin = n_rot ? cos_sin_dev : nullptr;
+    a.slab = kv->slab;
+    a.side = kv->vt_off[0];
+    u32x4* at = p->rows;
+    const auto take = [&](uint32_t n, uint32_t copies) { u32x4* row = at; at += copies * step_row_units(n); return row; };
+    a.x = take(p->hidden, kStepCopies);
+    a.x2 = take(p->hidden, kStepCopies);
+    a.qkv = take((p->nq + 2 * p->nkv) * 128, 1);
+    a.attn = take(p->nq * 128, kStepCopies);
+    a.act = take(p->ffn, kStepCopies);
+    a.part = reinterpret_cast<uint64_t*>(at);
+    a.part_ml = a.part + (size_t)p->nq * kMergeInRegs * 128;
+    a.expired = cx->err_dev + 1;
+    a.s.seq_k = pos + 1;
+    a.s.ctx_pad = kv->ctx_pad;
+    a.s.n_splits = r.n_splits;
+    a.s.tiles_per_wg = r.tiles_per_wg;
+    a.s.tail_tiles = (uint16_t)r.tail;
+    a.s.parts_per_wg = 1;
+    a.n_layers = p->n_layers;
+    a.hidden = p->hidden;
+    a.ffn = p->ffn;
+    a.nq = p->nq;
+    a.nkv = p->nkv;
+    a.n_rot = n_rot;
+    a.tag0 = p->next_tag;
+    const uint32_t limit = g.step_limit.load(std::memory_order_relaxed);
+    a.limit = limit ? limit : kStepLimitTicks;
+    a.eps = p->eps;
+    a.qscale = (scale_override > 0.0f ? scale_override : 1.0f / sqrtf(128.0f)) * kLog2e;
+    p->next_tag += p->n_layers;
+    g.calls.fetch_add(p->n_layers, std::memory_order_relaxed);
+    cx->step_calls = p->n_layers;
+    const size_t lds = (size_t)kStepTiles * 128 * 4;       // terms of the most inputs
+    launch_main(step_layers_kernel, dim3(g.n_cus), dim3(kStepThreads), a, lds);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        g.step_owner.store(nullptr, std::memory_order_release);
+        return hip_fail(e, "step launch", 0);
+    }
+    return WR_HIP_OK;
+}
+
+int wr_hip_attn_step_done(void)
+{
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    ENTER();
+    const int rc = sync_checked("step", 0);
+    const bool late = cx->err_host[1] != 0;
+    cx->err_host[1] = 0;
+    Ctx* mine = cx;
+    g.step_owner.compare_exchange_strong(mine, nullptr, std::memory_order_acq_rel);
+    if (rc) return rc;
+    if (late) {
+        g.step_refused = kStepRefusedSteps;
+        g.calls.fetch_sub(cx->step_calls, std::memory_order_relaxed);      // the step that is made instead counts its own
+        return WR_HIP_ERR_STATE;
+    }
+    return WR_HIP_OK;
 }
 
 int wr_hip_attn_decode_batched(uint32_t n, wr_hip_kv* const* kv, uint32_t layer,

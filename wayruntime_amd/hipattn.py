@@ -25,6 +25,11 @@ _u32 = C.c_uint32
 _f32p = C.POINTER(C.c_float)
 
 
+class StepLayer(C.Structure):
+    """wr_hip_attn_step_layer."""
+    _fields_ = [(n, _vp) for n in ("wqkv", "wo", "wgu", "wdown", "attn_norm", "ffn_norm", "q_norm", "k_norm")]
+
+
 class HipAttnError(RuntimeError):
     def __init__(self, rc: int, what: str):
         super().__init__(f"{what} failed with wr_status {rc}")
@@ -91,6 +96,11 @@ def load() -> C.CDLL:
         "wr_hip_proj_rows_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, _vp, _u32]),
         "wr_hip_proj_rows_norm_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, C.c_float, _vp, _vp, _u32]),
         "wr_hip_proj_rows_swiglu_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, _vp, _u32]),
+        "wr_hip_attn_step_create": (C.c_int, [_u32, C.POINTER(StepLayer), _u32, _u32, _u32, C.c_float, C.POINTER(_vp)]),
+        "wr_hip_attn_step_destroy": (None, [_vp]),
+        "wr_hip_attn_step_dev": (C.c_int, [_vp, _vp, _u32, _vp, _vp, _u32, C.c_float]),
+        "wr_hip_attn_step_done": (C.c_int, []),
+        "wr_hip_attn_set_step_limit": (None, [_u32]),
         "wr_hip_proj_rows_gated_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, C.c_float, C.c_int, _vp, _u32]),
         "wr_hip_rows_rmsnorm_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, _u32, _u32, _u32, C.c_float]),
         "wr_hip_rows_qkv_prep_dev": (C.c_int, [_vp, _u32, _u32, _u32, _u32, _u32, _vp, _vp, C.c_float,

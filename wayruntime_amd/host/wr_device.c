@@ -4,8 +4,9 @@
  * walks on the host).  Used when the device library offers projections
  * (WR_HIP_CAP_PROJ) and every matrix of the model is F16 with dimensions the
  * projection kernel takes; WAYRT_HOST_LAYERS=1 in the environment keeps the
- * host walk, WAYRT_STEP_TWO_LAUNCHES=1 keeps a decode step's row step and its
- * attention as two launches.  Per call the host embeds the rows and sends them up once; the
+ * host walk, WAYRT_STEP_LAUNCHES=1 keeps a session's decode step a chain of
+ * launches where one could take its layers, WAYRT_STEP_TWO_LAUNCHES=1 keeps a
+ * decode step's row step and its attention as two of them.  Per call the host embeds the rows and sends them up once; the
  * rotary angles of their positions are made on the device (the reference's
  * polynomial sin / cos and range reduction restated there bit for bit:
  * wr_hip_attn_rope_table_dev); the layers run without coming back, and the
@@ -41,6 +42,7 @@ struct wrh_dev_model {
      * 1 = yes, -1 = no (the two calls are made).  Read and written atomically:
      * sessions step from several threads. */
     int            step_in_one_launch;
+    wr_hip_attn_step *step;                                    /* a session's step in one launch for all layers, or NULL */
     /* prompt passes: does the library take Q as binary16 rows for this model's
      * attention (same meaning of 0 / 1 / -1)? */
     int            prefill_q16;
@@ -62,6 +64,7 @@ void wrh_device_model_free(wr_model *m)
         wr_hip_proj_weight_destroy(d->L[l].wdown);
     }
     wr_hip_proj_weight_destroy(d->lm_head);
+    wr_hip_attn_step_destroy(d->step);
     wr_hip_attn_dev_free(d->vecs);
     free(d);
     m->dev = NULL;
@@ -72,6 +75,22 @@ static int stack(wr_hip_weight **out, const wrh_weight *a, const wrh_weight *b, 
     const uint16_t *parts[3] = {a->data, b ? b->data : NULL, c ? c->data : NULL};
     uint32_t rows[3] = {a->rows, b ? b->rows : 0, c ? c->rows : 0};
     return wr_hip_proj_weight_create(c ? 3 : (b ? 2 : 1), parts, rows, a->cols, out);
+}
+
+/* The plan of a session's step in one launch, for models that have one. */
+static int step_plan(const wr_model *m, struct wrh_dev_model *d)
+{
+    const char *env = getenv("WAYRT_STEP_LAUNCHES");
+    int ok = !(env && env[0] == '1') && !m->is_gemma && d->step_in_one_launch >= 0;
+    wr_hip_attn_step_layer y[WRH_MAX_LAYERS];
+    for (uint32_t l = 0; l < m->n_layers && ok; l++) {
+        const dev_layer *s = &d->L[l];
+        ok = m->kv_src[l] == l && m->hd_layer[l] == m->head_dim;
+        y[l] = (wr_hip_attn_step_layer){s->wqkv, s->wo, s->wgu, s->wdown, s->attn_norm, s->ffn_norm, s->q_norm, s->k_norm};
+    }
+    if (!ok) return WR_HIP_OK;
+    const int rc = wr_hip_attn_step_create(m->n_layers, y, m->n_q, m->n_kv, m->head_dim, m->rms_eps, &d->step);
+    return rc == WR_HIP_ERR_UNSUPPORTED ? WR_HIP_OK : rc;
 }
 
 /* WR_OK with m->dev set, WR_OK with m->dev NULL when the model stays on the
@@ -150,6 +169,7 @@ wr_status wrh_device_model_init(wr_model *m)
         if (rc == WR_HIP_OK) rc = stack(&d->L[l].wdown, &m->w_down[l], NULL, NULL);
     }
     if (rc == WR_HIP_OK) rc = stack(&d->lm_head, &m->lm_head, NULL, NULL);
+    if (rc == WR_HIP_OK) rc = step_plan(m, d);
     /* the uploads ran on this thread's stream; sessions may step on others */
     if (rc == WR_HIP_OK) rc = wr_hip_attn_sync();
     if (rc != WR_HIP_OK) {
@@ -326,15 +346,12 @@ void wrh_stage_next_rows(wr_model *m, wrh_workspace *hs, uint32_t R, const uint3
     hs->staged_pos0 = pos0;
 }
 
-/* Same contract as the host walk's forward_rows (wr_session.c), plus: when
- * logits_host is not NULL, the LM head runs for the first `logit_rows` rows
- * and their logits [logit_rows][vocab] are brought down; when next_rows is not
- * zero (prefill), the host stages that many further tokens (tokens + R, at
- * pos0 + R) while the device works. */
-wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, uint32_t R,
-                                  wr_session *const *ss, const uint32_t *tokens, uint32_t pos0,
-                                  int batch, int prefill, int fail_layer, float *logits_host,
-                                  uint32_t logit_rows, uint32_t next_rows)
+/* wrh_forward_rows_device, below.  step: the plan that takes all layers of one row in one
+ * launch, or NULL; *again is set when that launch gave up and the pass has to be made without it. */
+static wr_status forward_pass(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, uint32_t R,
+                              wr_session *const *ss, const uint32_t *tokens, uint32_t pos0,
+                              int batch, int prefill, int fail_layer, float *logits_host,
+                              uint32_t logit_rows, uint32_t next_rows, wr_hip_attn_step *step, int *again)
 {
     wr_engine *e = m->engine;
     const struct wrh_dev_model *d = m->dev;
@@ -367,7 +384,15 @@ wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *
                                        m->rope_base_swa, 0), "angles");
     const float scale = gemma ? m->attn_scale : 0.0f;
 
-    for (L = 0; L < m->n_layers; L++) {
+    int stepped = 0;
+    if (step) {
+        const uint32_t at = batch ? ss[0]->pos : pos0;
+        rc = wr_hip_attn_step_dev(step, ss[0]->kv, at, ds->resid, ds->rope, n_rot, scale);
+        if (rc != WR_HIP_OK && rc != WR_HIP_ERR_UNSUPPORTED) return dev_fail(e, "step", L, rc);
+        stepped = rc == WR_HIP_OK;
+        for (uint32_t l = 0; l < m->n_layers && stepped; l++) ss[0]->kv_rows[l] = at + 1;
+    }
+    for (L = stepped ? m->n_layers : 0; L < m->n_layers; L++) {
         const dev_layer *dl = &d->L[L];
         /* per layer (Gemma; constant elsewhere): head_dim, rotary table, window, whose cache */
         const uint32_t hdl = m->hd_layer[L], qd = nq * hdl, kd = nkv * hdl;
@@ -483,15 +508,52 @@ wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *
         }
     }
     L = m->n_layers;
+    rc = WR_HIP_OK;
+    const char *what = "sync";
     if (logits_host && logit_rows) {
-        TRY(wr_hip_proj_rows_norm_dev(d->lm_head, logit_rows, ds->resid, hidden, d->final_norm,
-                                      m->rms_eps, NULL, ds->logits, m->vocab), "final norm + lm head");
-        TRY(wr_hip_attn_d2h(logits_host, ds->logits, (size_t)logit_rows * m->vocab * sizeof(float)),
-            "logits down");
+        what = "final norm + lm head";
+        rc = wr_hip_proj_rows_norm_dev(d->lm_head, logit_rows, ds->resid, hidden, d->final_norm,
+                                       m->rms_eps, NULL, ds->logits, m->vocab);
+        if (rc == WR_HIP_OK) {
+            what = "logits down";
+            rc = wr_hip_attn_d2h(logits_host, ds->logits, (size_t)logit_rows * m->vocab * sizeof(float));
+        }
     } else {
         /* both uploads above were synchronous: the host buffers are free again */
         if (next_rows) wrh_stage_next_rows(m, hs, next_rows, tokens + R, pos0 + R);
-        TRY(wr_hip_attn_sync(), "sync");
+        rc = wr_hip_attn_sync();
     }
-    return WR_OK;
+    if (stepped) {
+        const int done = wr_hip_attn_step_done();
+        *again = done == WR_HIP_ERR_STATE;
+        if (*again) {
+            wrh_logf(e, 1, "session: the step's one launch gave up waiting for its own workgroups; made again layer by layer");
+            return WR_ERR_INTERNAL;
+        }
+        if (rc == WR_HIP_OK && done != WR_HIP_OK) {
+            rc = done;
+            what = "step";
+        }
+    }
+    return rc == WR_HIP_OK ? WR_OK : dev_fail(e, what, L, rc);
+}
+
+/* Same contract as the host walk's forward_rows (wr_session.c), plus: when
+ * logits_host is not NULL, the LM head runs for the first `logit_rows` rows
+ * and their logits [logit_rows][vocab] are brought down; when next_rows is not
+ * zero (prefill), the host stages that many further tokens (tokens + R, at
+ * pos0 + R) while the device works. */
+wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, uint32_t R,
+                                  wr_session *const *ss, const uint32_t *tokens, uint32_t pos0,
+                                  int batch, int prefill, int fail_layer, float *logits_host,
+                                  uint32_t logit_rows, uint32_t next_rows)
+{
+    /* (an injected failure has a layer of its own to fail at) */
+    wr_hip_attn_step *step = R == 1 && !prefill && fail_layer < 0 ? m->dev->step : NULL;
+    int again = 0;
+    const wr_status st = forward_pass(m, hs, ds, R, ss, tokens, pos0, batch, prefill, fail_layer, logits_host,
+                                      logit_rows, next_rows, step, &again);
+    if (!again) return st;
+    return forward_pass(m, hs, ds, R, ss, tokens, pos0, batch, prefill, fail_layer, logits_host, logit_rows,
+                        next_rows, NULL, &again);
 }
