@@ -398,6 +398,12 @@ int wr_hip_proj_rows_gated_dev(const wr_hip_weight *w, uint32_t rows,
                                const float *norm_w_dev, float eps, int gelu,
                                float *act_dev, uint32_t ldo);
 
+/* Rows tokens[0 .. rows - 1] (host) of a weight as F32 rows times `scale`: the embedding,
+ * where the table is a weight of the device (a tied head's is; src/core/session.c:434-440).
+ * A token past n_out refuses the call.  ldx a multiple of 4, x_dev 16-byte aligned. */
+int wr_hip_proj_embed_dev(const wr_hip_weight *w, uint32_t rows, const uint32_t *tokens,
+                          float scale, float *x_dev, uint32_t ldx);
+
 /* ---- row steps between the projections and the attention path --------------
  * For callers that keep a layer's activations on the device.  All arguments
  * are device pointers (wr_hip_attn_dev_alloc), all calls are asynchronous on

@@ -416,6 +416,11 @@ int wr_hip_proj_rows_gated_dev(const wr_hip_weight *w, uint32_t rows, const floa
     (void)w; (void)rows; (void)x; (void)ldx; (void)nw; (void)eps; (void)gelu; (void)act; (void)ldo;
     return WR_HIP_ERR_STATE;
 }
+int wr_hip_proj_embed_dev(const wr_hip_weight *w, uint32_t rows, const uint32_t *tokens, float scale, float *x, uint32_t ldx)
+{
+    (void)w; (void)rows; (void)tokens; (void)scale; (void)x; (void)ldx;
+    return WR_HIP_ERR_STATE;
+}
 int wr_hip_attn_step_create(uint32_t n_layers, const wr_hip_attn_step_layer *layers, uint32_t nq, uint32_t nkv, uint32_t hd,
                             float eps, wr_hip_attn_step **out)
 {

@@ -563,3 +563,24 @@ def test_gated_product_refuses_an_odd_number_of_tiles():
     assert hipattn.lib().wr_hip_proj_rows_gated_dev(w.h, 1, b.p, 64, None, 1e-6, 0, b.p, 24) == hipattn.ERR_INVAL
     b.free()
     w.close()
+
+
+@pytest.mark.parametrize("n_out,n_in", [(16, 32), (208, 1024), (48, 1056), (32, 4096)])
+def test_embedding_rows(n_out, n_in):
+    """Rows of a weight by token, beyond one launch's arguments: the table's values, times the scale."""
+    rng = np.random.default_rng(n_in)
+    table = (rng.standard_normal((n_out, n_in)) * 2.0 ** rng.integers(-24, 4, (n_out, 1))).astype(np.float16)
+    w = hipattn.Weight([table.view(np.uint16)])
+    lib = hipattn.lib()
+    for rows, scale in ((1, 1.0), (17, 45.25), (960, 1.0), (961, 0.5), (2047, 1.0)):
+        ld = n_in + 4
+        tokens = rng.integers(0, n_out, rows).astype(np.uint32)
+        out = hipattn.DeviceBuffer.from_host(np.full((rows, ld), 7.0, dtype=np.float32))
+        assert lib.wr_hip_proj_embed_dev(w.h, rows, tokens.ctypes.data_as(C.POINTER(C.c_uint32)), scale, out.p, ld) == hipattn.OK
+        got = out.to_host((rows, ld))
+        assert np.array_equal(got[:, :n_in], table[tokens].astype(np.float32) * np.float32(scale)), rows
+        assert np.all(got[:, n_in:] == 7.0)
+        tokens[rows // 2] = n_out
+        assert lib.wr_hip_proj_embed_dev(w.h, rows, tokens.ctypes.data_as(C.POINTER(C.c_uint32)), scale, out.p, ld) == hipattn.ERR_INVAL
+        out.free()
+    w.close()

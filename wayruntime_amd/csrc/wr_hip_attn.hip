@@ -2258,6 +2258,29 @@ int wr_hip_proj_rows_gated_dev(const wr_hip_weight* w, uint32_t rows, const floa
     return proj_locked(w, rows, x_dev, ldx, src, nullptr, act_dev, ldo);
 }
 
+int wr_hip_proj_embed_dev(const wr_hip_weight* w, uint32_t rows, const uint32_t* tokens, float scale, float* x_dev, uint32_t ldx)
+{
+    int rc = check_proj(w, rows, tokens, 0, 0, x_dev, ldx, w ? w->n_in : 0);
+    if (rc || rows == 0) return rc;
+    if ((uintptr_t)x_dev & 15) return WR_HIP_ERR_INVAL;
+    for (uint32_t r = 0; r < rows; r++)
+        if (tokens[r] >= w->n_out) return WR_HIP_ERR_INVAL;               // never clamped
+    ENTER();
+    ProjEmbedArgs a;
+    a.w = reinterpret_cast<const half8*>(w->tiles);
+    a.ldx = ldx;
+    a.K = w->n_in;
+    a.scale = scale;
+    for (uint32_t done = 0; done < rows; done += kEmbedTokens) {
+        const uint32_t n = std::min(rows - done, kEmbedTokens);
+        a.x = x_dev + (size_t)done * ldx;
+        memcpy(a.tokens, tokens + done, n * sizeof(uint32_t));
+        hipLaunchKernelGGL(proj_embed_kernel, dim3(n), dim3(128), 0, cx->stream, a);
+    }
+    HIP_TRY(hipGetLastError(), "embedding launch", 0);
+    return WR_HIP_OK;
+}
+
 int wr_hip_proj_rows(const wr_hip_weight* w, uint32_t rows, const float* x, float* y)
 {
     if (w && (w->n_out % 4 != 0)) return WR_HIP_ERR_INVAL;

@@ -6,7 +6,8 @@
  * projection kernel takes; WAYRT_HOST_LAYERS=1 in the environment keeps the
  * host walk, WAYRT_STEP_LAUNCHES=1 keeps a session's decode step a chain of
  * launches where one could take its layers, WAYRT_STEP_TWO_LAUNCHES=1 keeps a
- * decode step's row step and its attention as two of them.  Per call the host embeds the rows and sends them up once; the
+ * decode step's row step and its attention as two of them.  Per call the rows are
+ * embedded on the device (by the host, and sent up, where the table is not F16); the
  * rotary angles of their positions are made on the device (the reference's
  * polynomial sin / cos and range reduction restated there bit for bit:
  * wr_hip_attn_rope_table_dev); the layers run without coming back, and the
@@ -35,6 +36,7 @@ typedef struct dev_layer {
 struct wrh_dev_model {
     dev_layer     L[WRH_MAX_LAYERS];
     wr_hip_weight *lm_head;
+    wr_hip_weight *embed;                                      /* lm_head where it is tied, NULL: rows are embedded on the host */
     float         *vecs;                                       /* one device block for all norm vectors */
     const float   *final_norm;
     /* decode steps: does the library take the row step (split, norms, rotation,
@@ -63,6 +65,7 @@ void wrh_device_model_free(wr_model *m)
         wr_hip_proj_weight_destroy(d->L[l].wgu);
         wr_hip_proj_weight_destroy(d->L[l].wdown);
     }
+    if (d->embed != d->lm_head) wr_hip_proj_weight_destroy(d->embed);
     wr_hip_proj_weight_destroy(d->lm_head);
     wr_hip_attn_step_destroy(d->step);
     wr_hip_attn_dev_free(d->vecs);
@@ -169,6 +172,8 @@ wr_status wrh_device_model_init(wr_model *m)
         if (rc == WR_HIP_OK) rc = stack(&d->L[l].wdown, &m->w_down[l], NULL, NULL);
     }
     if (rc == WR_HIP_OK) rc = stack(&d->lm_head, &m->lm_head, NULL, NULL);
+    if (rc == WR_HIP_OK && m->embed.data == m->lm_head.data) d->embed = d->lm_head;
+    else if (rc == WR_HIP_OK && proj_dims_ok(&m->embed)) rc = stack(&d->embed, &m->embed, NULL, NULL);
     if (rc == WR_HIP_OK) rc = step_plan(m, d);
     /* the uploads ran on this thread's stream; sessions may step on others */
     if (rc == WR_HIP_OK) rc = wr_hip_attn_sync();
@@ -363,11 +368,17 @@ static wr_status forward_pass(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, 
 
     const int staged = !batch && hs->staged_rows == R && hs->staged_tokens == tokens && hs->staged_pos0 == pos0;
     hs->staged_rows = 0;
-    if (!staged) {
-        rc = stage_rows(m, hs, R, tokens);
-        if (rc != WR_OK) return dev_fail(e, "embed", 0, rc);
+    if (d->embed) {
+        /* Gemma: scaled embeddings (session.c:262-283) */
+        const float times = m->is_gemma && m->embed_scale != 0.0f ? m->embed_scale : 1.0f;
+        TRY(wr_hip_proj_embed_dev(d->embed, R, tokens, times, ds->resid, hidden), "embed");
+    } else {
+        if (!staged) {
+            rc = stage_rows(m, hs, R, tokens);
+            if (rc != WR_OK) return dev_fail(e, "embed", 0, rc);
+        }
+        TRY(wr_hip_attn_h2d(ds->resid, hs->residual, (size_t)R * hidden * sizeof(float)), "rows up");
     }
-    TRY(wr_hip_attn_h2d(ds->resid, hs->residual, (size_t)R * hidden * sizeof(float)), "rows up");
     /* rotary tables of the rows' positions; Gemma's sliding-window layers have
      * their own head_dim and base and rotate fully (session.c:262-283) */
     uint32_t plist[WR_HIP_BATCH_MAX];
@@ -519,8 +530,8 @@ static wr_status forward_pass(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, 
             rc = wr_hip_attn_d2h(logits_host, ds->logits, (size_t)logit_rows * m->vocab * sizeof(float));
         }
     } else {
-        /* both uploads above were synchronous: the host buffers are free again */
-        if (next_rows) wrh_stage_next_rows(m, hs, next_rows, tokens + R, pos0 + R);
+        /* the upload above was synchronous: the host buffers are free again */
+        if (next_rows && !d->embed) wrh_stage_next_rows(m, hs, next_rows, tokens + R, pos0 + R);
         rc = wr_hip_attn_sync();
     }
     if (stepped) {
