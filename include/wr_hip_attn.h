@@ -209,6 +209,9 @@ void *wr_hip_attn_host_alloc(size_t bytes);
 void  wr_hip_attn_host_free(void *p);
 int   wr_hip_attn_h2d(void *dst_dev, const void *src_host, size_t bytes);
 int   wr_hip_attn_d2h(void *dst_host, const void *src_dev, size_t bytes);
+/* n (<= WR_HIP_BATCH_MAX) rows of row_floats (a multiple of 4) each into memory of
+ * wr_hip_attn_host_alloc, which kernels can also be handed as an output; waits. */
+int wr_hip_attn_rows_d2h(uint32_t n, float *const *dst_locked, const float *src_dev, size_t row_floats);
 int   wr_hip_attn_sync(void);
 void *wr_hip_attn_stream(void);          /* hipStream_t of the calling thread */
 

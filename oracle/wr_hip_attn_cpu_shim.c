@@ -416,6 +416,11 @@ int wr_hip_proj_rows_gated_dev(const wr_hip_weight *w, uint32_t rows, const floa
     (void)w; (void)rows; (void)x; (void)ldx; (void)nw; (void)eps; (void)gelu; (void)act; (void)ldo;
     return WR_HIP_ERR_STATE;
 }
+int wr_hip_attn_rows_d2h(uint32_t n, float *const *dst, const float *src, size_t row_floats)
+{
+    (void)n; (void)dst; (void)src; (void)row_floats;
+    return WR_HIP_ERR_STATE;
+}
 int wr_hip_proj_embed_dev(const wr_hip_weight *w, uint32_t rows, const uint32_t *tokens, float scale, float *x, uint32_t ldx)
 {
     (void)w; (void)rows; (void)tokens; (void)scale; (void)x; (void)ldx;

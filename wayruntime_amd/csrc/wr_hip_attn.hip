@@ -2104,6 +2104,25 @@ int wr_hip_attn_d2h(void* dst_host, const void* src_dev, size_t bytes)
     return sync_checked("d2h sync", 0);
 }
 
+int wr_hip_attn_rows_d2h(uint32_t n, float* const* dst_locked, const float* src_dev, size_t row_floats)
+{
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    if (!dst_locked || !src_dev) return WR_HIP_ERR_INVAL;
+    if (n == 0 || n > WR_HIP_BATCH_MAX) return WR_HIP_ERR_LIMIT;
+    if (row_floats == 0 || row_floats % 4 != 0 || row_floats / 4 > 0x7FFFFFFFu || ((uintptr_t)src_dev & 15)) return WR_HIP_ERR_INVAL;
+    RowsDownArgs a{};
+    for (uint32_t i = 0; i < n; i++) {
+        if (!dst_locked[i] || ((uintptr_t)dst_locked[i] & 15)) return WR_HIP_ERR_INVAL;
+        a.dst[i] = reinterpret_cast<f32x4*>(dst_locked[i]);
+    }
+    a.src = reinterpret_cast<const f32x4*>(src_dev);
+    a.units = a.ld_units = (uint32_t)(row_floats / 4);
+    ENTER();
+    hipLaunchKernelGGL(rows_down_kernel, dim3(std::min((a.units + 255) / 256, 64u), n), dim3(256), 0, cx->stream, a);
+    HIP_TRY(hipGetLastError(), "rows down launch", 0);
+    return sync_checked("rows down", 0);
+}
+
 int wr_hip_attn_sync(void)
 {
     if (!g.inited) return WR_HIP_ERR_STATE;

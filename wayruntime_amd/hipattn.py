@@ -68,6 +68,7 @@ def load() -> C.CDLL:
         "wr_hip_attn_dev_free": (None, [_vp]),
         "wr_hip_attn_h2d": (C.c_int, [_vp, _vp, C.c_size_t]),
         "wr_hip_attn_d2h": (C.c_int, [_vp, _vp, C.c_size_t]),
+        "wr_hip_attn_rows_d2h": (C.c_int, [_u32, C.POINTER(_vp), _vp, C.c_size_t]),
         "wr_hip_attn_sync": (C.c_int, []),
         "wr_hip_attn_stream": (_vp, []),
         "wr_hip_attn_append_dev": (C.c_int, [_vp, _u32, _u32, _u32, _vp, _vp]),

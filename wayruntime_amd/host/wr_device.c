@@ -232,7 +232,6 @@ static void scratch_destroy(struct wrh_scratch *sc)
     if (!sc) return;
     wrh_devspace_free(&sc->ds);
     wrh_workspace_free(&sc->ws);
-    if (sc->logits_host) wr_hip_attn_host_free(sc->logits_host);
     free(sc);
 }
 
@@ -244,10 +243,6 @@ static struct wrh_scratch *scratch_create(const wr_model *m, uint32_t rows, uint
     sc->logit_rows = logit_rows;
     int ok = wrh_workspace_init(&sc->ws, m, rows) == WR_OK;
     ok = ok && wrh_devspace_init(&sc->ds, m, rows, logit_rows) == WR_OK;
-    if (ok && logit_rows) {
-        sc->logits_host = wr_hip_attn_host_alloc((size_t)logit_rows * m->vocab * sizeof(float));
-        ok = sc->logits_host != NULL;
-    }
     if (!ok) {
         scratch_destroy(sc);
         return NULL;
@@ -301,6 +296,28 @@ void wrh_scratch_free_all(wr_model *m)
     scratch_destroy(m->batch_scratch);
     scratch_destroy(m->prefill_scratch);
     m->batch_scratch = m->prefill_scratch = NULL;
+    while (m->n_logit_rows) wr_hip_attn_host_free(m->logit_rows[--m->n_logit_rows]);
+}
+
+float *wrh_logits_acquire(wr_model *m)
+{
+    float *row = NULL;
+    pthread_mutex_lock(&m->lock);
+    if (m->n_logit_rows) row = m->logit_rows[--m->n_logit_rows];
+    pthread_mutex_unlock(&m->lock);
+    return row ? row : wr_hip_attn_host_alloc((size_t)m->vocab * sizeof(float));
+}
+
+void wrh_logits_release(wr_model *m, float *row)
+{
+    if (!row) return;
+    pthread_mutex_lock(&m->lock);
+    if (m->n_logit_rows < WR_BATCH_MAX) {
+        m->logit_rows[m->n_logit_rows++] = row;
+        row = NULL;
+    }
+    pthread_mutex_unlock(&m->lock);
+    if (row) wr_hip_attn_host_free(row);
 }
 
 /* --------------------------------------------------------------- forward -- */
@@ -355,8 +372,8 @@ void wrh_stage_next_rows(wr_model *m, wrh_workspace *hs, uint32_t R, const uint3
  * launch, or NULL; *again is set when that launch gave up and the pass has to be made without it. */
 static wr_status forward_pass(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, uint32_t R,
                               wr_session *const *ss, const uint32_t *tokens, uint32_t pos0,
-                              int batch, int prefill, int fail_layer, float *logits_host,
-                              uint32_t logit_rows, uint32_t next_rows, wr_hip_attn_step *step, int *again)
+                              int batch, int prefill, int fail_layer, int logits, uint32_t next_rows,
+                              wr_hip_attn_step *step, int *again)
 {
     wr_engine *e = m->engine;
     const struct wrh_dev_model *d = m->dev;
@@ -521,13 +538,17 @@ static wr_status forward_pass(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, 
     L = m->n_layers;
     rc = WR_HIP_OK;
     const char *what = "sync";
-    if (logits_host && logit_rows) {
+    if (logits) {
+        /* One row: the product writes it where the session keeps it, across the link while it reads the weight.
+         * More: 600 KB each at a vocabulary of 150 000, and the link would take longer than the product. */
+        float *rows[WR_BATCH_MAX];
+        for (uint32_t r = 0; r < R; r++) rows[r] = ss[r]->logits;
         what = "final norm + lm head";
-        rc = wr_hip_proj_rows_norm_dev(d->lm_head, logit_rows, ds->resid, hidden, d->final_norm,
-                                       m->rms_eps, NULL, ds->logits, m->vocab);
+        rc = wr_hip_proj_rows_norm_dev(d->lm_head, R, ds->resid, hidden, d->final_norm, m->rms_eps, NULL,
+                                       R == 1 ? rows[0] : ds->logits, m->vocab);
         if (rc == WR_HIP_OK) {
             what = "logits down";
-            rc = wr_hip_attn_d2h(logits_host, ds->logits, (size_t)logit_rows * m->vocab * sizeof(float));
+            rc = R == 1 ? wr_hip_attn_sync() : wr_hip_attn_rows_d2h(R, rows, ds->logits, m->vocab);
         }
     } else {
         /* the upload above was synchronous: the host buffers are free again */
@@ -549,22 +570,20 @@ static wr_status forward_pass(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, 
     return rc == WR_HIP_OK ? WR_OK : dev_fail(e, what, L, rc);
 }
 
-/* Same contract as the host walk's forward_rows (wr_session.c), plus: when
- * logits_host is not NULL, the LM head runs for the first `logit_rows` rows
- * and their logits [logit_rows][vocab] are brought down; when next_rows is not
- * zero (prefill), the host stages that many further tokens (tokens + R, at
- * pos0 + R) while the device works. */
+/* Same contract as the host walk's forward_rows (wr_session.c), plus: with
+ * `logits`, the LM head runs for all rows (a step's) and their logits come down to where
+ * their sessions keep them; when next_rows is not zero (prefill), the host
+ * stages that many further tokens (tokens + R, at pos0 + R) while the device
+ * works. */
 wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, uint32_t R,
                                   wr_session *const *ss, const uint32_t *tokens, uint32_t pos0,
-                                  int batch, int prefill, int fail_layer, float *logits_host,
-                                  uint32_t logit_rows, uint32_t next_rows)
+                                  int batch, int prefill, int fail_layer, int logits, uint32_t next_rows)
 {
     /* (an injected failure has a layer of its own to fail at) */
     wr_hip_attn_step *step = R == 1 && !prefill && fail_layer < 0 ? m->dev->step : NULL;
     int again = 0;
-    const wr_status st = forward_pass(m, hs, ds, R, ss, tokens, pos0, batch, prefill, fail_layer, logits_host,
-                                      logit_rows, next_rows, step, &again);
+    const wr_status st = forward_pass(m, hs, ds, R, ss, tokens, pos0, batch, prefill, fail_layer, logits, next_rows,
+                                      step, &again);
     if (!again) return st;
-    return forward_pass(m, hs, ds, R, ss, tokens, pos0, batch, prefill, fail_layer, logits_host, logit_rows,
-                        next_rows, NULL, &again);
+    return forward_pass(m, hs, ds, R, ss, tokens, pos0, batch, prefill, fail_layer, logits, next_rows, NULL, &again);
 }

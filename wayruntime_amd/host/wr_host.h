@@ -85,10 +85,14 @@ struct wr_model {
      * wr_batch_step, one for wr_prefill.  A call that finds its set taken by a
      * concurrent call allocates its own as before. */
     struct wrh_scratch *batch_scratch, *prefill_scratch;
+    /* Page-locked rows of logits that ended sessions of the device walk have left for
+     * the next ones (locking one takes longer than a step), at most a batch's. */
+    float          *logit_rows[WR_BATCH_MAX];
+    uint32_t        n_logit_rows;
 
     void           *map;         /* mmap of the GGUF file */
     size_t          map_bytes;
-    pthread_mutex_t lock;        /* guards session_refs */
+    pthread_mutex_t lock;        /* guards session_refs, the scratch sets and the rows of logits */
     uint32_t        session_refs;
 };
 
@@ -116,6 +120,9 @@ struct wrh_scratch;
 struct wrh_scratch *wrh_scratch_acquire(wr_model *m, int kind, uint32_t rows, uint32_t logit_rows);
 void wrh_scratch_release(wr_model *m, struct wrh_scratch *sc);
 void wrh_scratch_free_all(wr_model *m);
+/* A session's row of logits on the device walk: page-locked, kept by the model between sessions. */
+float *wrh_logits_acquire(wr_model *m);
+void   wrh_logits_release(wr_model *m, float *row);
 
 /* Device scratch for R rows of the device walk (wr_device.c). */
 typedef struct wrh_devspace {
@@ -136,7 +143,6 @@ typedef struct wrh_devspace {
 struct wrh_scratch {
     wrh_workspace ws;                    /* host rows (embedding) */
     wrh_devspace  ds;
-    float        *logits_host;           /* page-locked, [logit_rows][vocab]; NULL when logit_rows == 0 */
     uint32_t      rows, logit_rows;
     int           cached;                /* belongs to the model (else freed on release) */
     int           busy;
@@ -151,7 +157,7 @@ struct wr_session {
     struct wrh_mix_session *mix;             /* mixer-stack model: pages and state slot in the model's pool (no kv, ws1, ds1) */
     wr_hip_kv      *kv;                      /* device cache */
     uint32_t        kv_rows[WRH_MAX_LAYERS]; /* per-layer cursor (the reference's valid_rows) */
-    float          *logits;                  /* [vocab] */
+    float          *logits;                  /* [vocab]; device walk: page-locked, from the model (wrh_logits_acquire) */
     wrh_workspace   ws1;                     /* one-row scratch for wr_step */
     wrh_devspace    ds1;                     /* its device counterpart (device walk only) */
 };
@@ -192,8 +198,7 @@ int       wrh_devspace_init(wrh_devspace *ws, const wr_model *m, uint32_t rows, 
 void      wrh_devspace_free(wrh_devspace *ws);
 wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, uint32_t R,
                                   wr_session *const *ss, const uint32_t *tokens, uint32_t pos0,
-                                  int batch, int prefill, int fail_layer, float *logits_host,
-                                  uint32_t logit_rows, uint32_t next_rows);
+                                  int batch, int prefill, int fail_layer, int logits, uint32_t next_rows);
 
 /* ---- mixer-stack models (wr_mix.c) ------------------------------------------ */
 wr_status wrh_mix_session_create(wr_model *m, wr_session *s);

@@ -338,6 +338,12 @@ static void kv_rollback(wr_session *s)
 
 /* ------------------------------------------------------------- lifecycle -- */
 
+static void free_logits(wr_session *s)
+{
+    if (s->model->dev) wrh_logits_release(s->model, s->logits);
+    else free(s->logits);
+}
+
 static wr_status session_register(wr_model *m, wr_session *s, wr_session **out)
 {
     pthread_mutex_init(&s->lock, NULL);
@@ -390,10 +396,10 @@ wr_status wr_session_create(wr_model *m, const wr_session_params *params, wr_ses
         free(s);
         return (wr_status)rc;
     }
-    s->logits = malloc((size_t)m->vocab * sizeof(float));
+    s->logits = m->dev ? wrh_logits_acquire(m) : malloc((size_t)m->vocab * sizeof(float));
     if (!s->logits || wrh_workspace_init(&s->ws1, m, 1) != WR_OK ||
-        (m->dev && wrh_devspace_init(&s->ds1, m, 1, 1) != WR_OK)) {
-        free(s->logits);
+        (m->dev && wrh_devspace_init(&s->ds1, m, 1, 0) != WR_OK)) {
+        free_logits(s);
         wrh_workspace_free(&s->ws1);
         wr_hip_attn_kv_destroy(s->kv);
         free(s);
@@ -413,7 +419,7 @@ void wr_session_destroy(wr_session *s)
     wr_hip_attn_kv_destroy(s->kv);
     wrh_workspace_free(&s->ws1);
     wrh_devspace_free(&s->ds1);
-    free(s->logits);
+    free_logits(s);
     pthread_mutex_destroy(&s->lock);
     free(s);
 }
@@ -449,7 +455,7 @@ const float *wr_step(wr_session *s, uint32_t token)
         wr_session *one[1] = {s};
         if (m->dev) {
             st = wrh_forward_rows_device(m, &s->ws1, &s->ds1, 1, one, &token, s->pos, 0, 0,
-                                         take_fail_layer(m), s->logits, 1, 0);
+                                         take_fail_layer(m), 1, 0);
             if (st == WR_OK && m->is_gemma) wrh_softcap(s->logits, m->vocab, m->logit_softcap);
         } else {
             st = forward_rows(m, &s->ws1, 1, one, &token, s->pos, FWD_STEP);
@@ -503,7 +509,7 @@ int wr_prefill(wr_session *s, const uint32_t *ids, uint32_t n)
                 const uint32_t rows = (n - done < chunk) ? n - done : chunk;
                 const uint32_t left = n - done - rows;                 /* staged while the device works */
                 st = wrh_forward_rows_device(m, &sc->ws, &sc->ds, rows, one, ids + done, s->pos, 0, 1,
-                                             take_fail_layer(m), NULL, 0, left < chunk ? left : chunk);
+                                             take_fail_layer(m), 0, left < chunk ? left : chunk);
                 if (st == WR_OK) __atomic_store_n(&s->pos, s->pos + rows, __ATOMIC_RELEASE);
             }
             wrh_scratch_release(m, sc);
@@ -682,13 +688,12 @@ int wr_batch_step(wr_session *const *sessions, const uint32_t *tokens, uint32_t 
     int have_ws = 0;
     struct wrh_scratch *sc = NULL;
     if (st == WR_OK && m->dev) {
-        /* device walk: rows, device scratch and page-locked logits kept by the model */
+        /* device walk: rows and device scratch kept by the model, logits where the sessions keep them */
         sc = wrh_scratch_acquire(m, 0, n, n);
         if (!sc) st = WR_ERR_NOMEM;
         if (st == WR_OK)
             st = wrh_forward_rows_device(m, &sc->ws, &sc->ds, n, sessions, tokens, 0, 1, 0,
-                                         take_fail_layer(m), sc->logits_host, n, 0);
-        big = sc ? sc->logits_host : NULL;
+                                         take_fail_layer(m), 1, 0);
     } else if (st == WR_OK) {
         if (wrh_workspace_init(&ws, m, n) == WR_OK) have_ws = 1;
         else st = WR_ERR_NOMEM;
@@ -701,13 +706,13 @@ int wr_batch_step(wr_session *const *sessions, const uint32_t *tokens, uint32_t 
     if (st == WR_OK) {
         /* one LM-head product for all n rows (reference: batch.c:45-104), then demux */
         if (!m->dev) wrh_matmul(m->engine, ws.normed, n, m->hidden, &m->lm_head, big, m->vocab);
-        if (m->is_gemma) wrh_softcap(big, (uint64_t)n * m->vocab, m->logit_softcap);
-        {
-            /* 600 KB a session at a vocabulary of 150 000: one thread per session */
-            const int threads = (m->engine && m->engine->n_threads > 0) ? m->engine->n_threads : 1;
-#pragma omp parallel for num_threads(threads) schedule(static) if (n >= 4)
-            for (uint32_t i = 0; i < n; i++)
-                memcpy(sessions[i]->logits, big + (size_t)i * m->vocab, (size_t)m->vocab * sizeof(float));
+        /* 600 KB a session at a vocabulary of 150 000: one thread per session */
+        const int threads = (m->engine && m->engine->n_threads > 0) ? m->engine->n_threads : 1;
+#pragma omp parallel for num_threads(threads) schedule(static) if (n >= 4 && (big || m->is_gemma))
+        for (uint32_t i = 0; i < n; i++) {
+            float *row = sessions[i]->logits;
+            if (big) memcpy(row, big + (size_t)i * m->vocab, (size_t)m->vocab * sizeof(float));
+            if (m->is_gemma) wrh_softcap(row, m->vocab, m->logit_softcap);
         }
         for (uint32_t i = 0; i < n; i++)
             __atomic_store_n(&sessions[i]->pos, sessions[i]->pos + 1, __ATOMIC_RELEASE);
