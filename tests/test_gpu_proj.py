@@ -584,3 +584,35 @@ def test_embedding_rows(n_out, n_in):
         assert lib.wr_hip_proj_embed_dev(w.h, rows, tokens.ctypes.data_as(C.POINTER(C.c_uint32)), scale, out.p, ld) == hipattn.ERR_INVAL
         out.free()
     w.close()
+
+
+@pytest.mark.parametrize("n_in", [512, 1024, 1536, 2048, 2560, 3072])
+def test_rows_of_a_few_equal_the_row_alone(n_in):
+    # The kernel that makes its own operand terms takes four rows to a workgroup of a narrow
+    # weight and eight of a wider one: on either side of a workgroup's rows, and where the two
+    # meet (256 compute units, 64 tiles: 16 rows; 68 tiles: 12), the bits are those of a row alone.
+    lib = hipattn.lib()
+    D = hipattn.DeviceBuffer
+    for n_out in (1024, 1088):
+        x = synth.normal(81 + n_in, (17, n_in), std=2.0)
+        nw = synth.normal(82, (n_in,)) * np.float32(0.2) + np.float32(1.0)
+        add = synth.normal(83, (17, n_out))
+        w = hipattn.Weight([_w16(84, n_out, n_in, 0.1)])
+        xd, nwd, addd, y = D.from_host(x), D.from_host(nw), D.from_host(add), D(17 * n_out * 4)
+        for norm in (False, True):
+            def call(at, rows):
+                xp, ap = xd.p + at * n_in * 4, addd.p + at * n_out * 4
+                if norm:
+                    rc = lib.wr_hip_proj_rows_norm_dev(w.h, rows, xp, n_in, nwd.p, 1e-6, ap, y.p, n_out)
+                else:
+                    rc = lib.wr_hip_proj_rows_dev(w.h, rows, xp, n_in, ap, y.p, n_out)
+                assert rc == hipattn.OK
+                hipattn.sync()
+                return y.to_host((17, n_out))[:rows].copy()
+            alone = np.concatenate([call(i, 1) for i in range(16)])
+            for at, rows in ((0, 2), (3, 3), (1, 4), (2, 5), (4, 7), (0, 8), (5, 9), (1, 12), (0, 13), (0, 15), (0, 16)):
+                print("rows", n_in, n_out, norm, at, rows, flush=True)
+                assert call(at, rows).tobytes() == alone[at:at + rows].tobytes()
+        for d in (xd, nwd, addd, y):
+            d.free()
+        w.close()

@@ -532,14 +532,15 @@ __device__ __forceinline__ f32x4 proj_join_terms(f32x4 v)
     return v;
 }
 
+template <int ROWS = 8>
 __device__ __forceinline__ void proj_store_tile(const ProjArgs& a, f32x4 v, uint32_t nt, uint32_t group,
                                                 int lane, const float* scale = nullptr,
                                                 const f32x4* residual = nullptr)
 {
     const int c = lane & 15, g = lane >> 4;
     v = proj_join_terms(v);
-    const uint32_t row = group * 8 + (c & 7);
-    if (c < 8 && row < a.R && nt < a.N / 16) {
+    const uint32_t row = group * ROWS + (c & 7);
+    if (c < ROWS && row < a.R && nt < a.N / 16) {
         const float sc = scale ? *scale : a.scales[row];
         const size_t o = (size_t)row * a.ldy + nt * 16 + g * 4;
         f32x4 r;
@@ -569,14 +570,15 @@ __device__ __forceinline__ uint32_t proj_paired_tile(uint32_t pair, uint32_t t, 
     return min(pair, ntiles / 2 - 1) + t * (ntiles / 2);         // (a pair past the end re-reads the last; dropped)
 }
 
+template <int ROWS = 8>
 __device__ __forceinline__ void proj_store_pair(const ProjArgs& a, f32x4 gate, f32x4 value, uint32_t pair, uint32_t group,
                                                 int lane, const float* scale = nullptr)
 {
     const int c = lane & 15, g = lane >> 4;
     gate = proj_join_terms(gate);
     value = proj_join_terms(value);
-    const uint32_t row = group * 8 + (c & 7);
-    if (c < 8 && row < a.R && pair < a.N / 32) {
+    const uint32_t row = group * ROWS + (c & 7);
+    if (c < ROWS && row < a.R && pair < a.N / 32) {
         const float sc = scale ? *scale : a.scales[row];
         f32x4 r;
 #pragma unroll
@@ -1064,23 +1066,32 @@ __global__ __launch_bounds__(kProjThreads) void proj_row1_kernel(const ProjArgs 
 // order of the product's are those of proj_prep_kernel and of the kernels that share a
 // tile's inputs between four waves, so the result has the same bits.
 //
+// A workgroup of ROWS = 8 rows fills the operand's columns; one of four leaves half of them unused and has half the
+// terms to make, for narrow weights whose tiles of eight rows leave compute units without work.  Eight rows / four
+// (us, weights from HBM, plain rows): 16 rows, 3072 -> 1024 7.8 / 5.7, 2048 -> 1024 5.5 / 4.2, 1536 -> 512 4.6 / 3.7,
+// norm + 1024 -> 1024 4.5 / 3.6; 8 rows, 2048 -> 2048 5.6 / 4.7; 4 rows, norm + 1024 -> 4096 4.2 / 3.8; 1024 -> 1024
+// at any number of rows 3.7 / 3.7.
+//
 // 16 rows, weights from HBM, against proj_prep_kernel + proj_gemm_split_kernel<1, 1, 8>
 // (us): norm + 1024 -> 4096 8.1 -> 5.2, norm + 1024 -> 6144 9.3 -> 6.2, 2048 -> 1024
-// 7.7 -> 5.5, 3072 -> 1024 9.5 -> 7.8; 32 rows of the third 7.8 -> 5.5.  (A lane making
+// 7.7 -> 5.5 -> 4.2, 3072 -> 1024 9.5 -> 7.8 -> 5.7; 32 rows of the third 7.8 -> 5.5.  (A lane making
 // the terms of four inputs of its own operand column and trading them with the lane
 // eight on, no LDS: 5.7, 6.7, 5.8, 8.1.)
-template <int SRC, int D, int NT, bool GATED = false>
+template <int SRC, int D, int NT, bool GATED = false, int ROWS = 8>
 __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const ProjArgs a, const ProjPrepArgs p)
 {
     static_assert(D % 2 == 0 && (SRC == kProjSrcPlain || (SRC == kProjSrcRmsNorm && D <= 16)), "sources held in registers");
+    static_assert(ROWS == 8 || ROWS == 4, "operand columns: hi terms 0 .. ROWS - 1, lo terms eight on");
     static_assert(!GATED || NT % 2 == 0, "gates' tiles and values'");
     constexpr bool NORM = SRC == kProjSrcRmsNorm;
     constexpr int KT = 4 * D;                                    // k-steps of a row
-    constexpr int CH = D / 2;                                    // chunks of eight inputs per lane
+    constexpr int QS = 16 / ROWS;                                // k-steps that the lanes of a wave span
+    constexpr int CH = D / QS;                                   // chunks of eight inputs per lane
+    static_assert(D % QS == 0, "whole spans");
     extern __shared__ __attribute__((aligned(16))) unsigned char fused_smem[];
     // sums of squares of the chunks, by row, chunk of a k-step and k-step
-    __shared__ __attribute__((aligned(16))) float s_ss[NORM ? 8 : 1][NORM ? 4 : 1][NORM ? KT + 4 : 1];
-    __shared__ float s_mx[4][8];
+    __shared__ __attribute__((aligned(16))) float s_ss[NORM ? ROWS : 1][NORM ? 4 : 1][NORM ? KT + 4 : 1];
+    __shared__ float s_mx[4][ROWS];
     __shared__ f32x4 s_red[3 * NT * 64];
     const int lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1088,18 +1099,18 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
     const uint32_t k0 = wave * D;                                // this wave's quarter of the k-steps
     half8* frag = reinterpret_cast<half8*>(fused_smem) + k0 * 64;
 
-    // 1. the rows, what goes with them, then the weights, all at once.  A lane takes chunk lane / 8 of every two k-steps
-    // of row lane % 8: eight lanes read 256 bytes of a row.  (A row past the end re-reads the last; its columns are dropped.)
-    const uint32_t r = lane & 7, q = lane >> 3;
+    // 1. the rows, what goes with them, then the weights, all at once.  A lane takes chunk lane / ROWS of every QS k-steps
+    // of row lane % ROWS: eight lanes read 256 bytes of a row, sixteen 512.  (A row past the end re-reads the last; its columns are dropped.)
+    const uint32_t r = lane % ROWS, q = lane / ROWS;
     const uint32_t at = k0 * 32 + q * 8;
-    const float* xr = p.x + (size_t)min(group * 8 + r, a.R - 1) * p.ldx + at;
+    const float* xr = p.x + (size_t)min(group * ROWS + r, a.R - 1) * p.ldx + at;
     f32x4 x[CH][2], nw[NORM ? CH : 1][2];
 #pragma unroll
     for (int i = 0; i < CH; i++)
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            x[i][h] = *reinterpret_cast<const f32x4*>(xr + i * 64 + h * 4);
-            if constexpr (NORM) nw[i][h] = *reinterpret_cast<const f32x4*>(p.norm_w + at + i * 64 + h * 4);
+            x[i][h] = *reinterpret_cast<const f32x4*>(xr + i * QS * 32 + h * 4);
+            if constexpr (NORM) nw[i][h] = *reinterpret_cast<const f32x4*>(p.norm_w + at + i * QS * 32 + h * 4);
         }
     f32x4 resid[NT];
     half8 w[D][NT];
@@ -1107,7 +1118,7 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         const uint32_t tile = GATED ? proj_paired_tile((nt0 + t) / 2, t % 2, ntiles) : min(nt0 + t, ntiles - 1);   // (one past the end: dropped)
-        const uint32_t row = min(group * 8 + (lane & 7), a.R - 1);
+        const uint32_t row = min(group * ROWS + lane % ROWS, a.R - 1);
         resid[t] = *reinterpret_cast<const f32x4*>(
             !GATED && a.bias_rows ? a.bias_rows + (size_t)row * a.ldy + tile * 16 + (lane >> 4) * 4 : xr);
         wp[t] = a.w + ((size_t)tile * KT + k0) * 64;
@@ -1124,11 +1135,11 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
             float ss = 0.f;
 #pragma unroll
             for (int j = 0; j < 8; j++) ss = fmaf(x[i][j / 4][j % 4], x[i][j / 4][j % 4], ss);
-            s_ss[r][q & 3][k0 + 2 * i + (q >> 2)] = ss;
+            s_ss[r][q & 3][k0 + QS * i + (q >> 2)] = ss;
         }
         lds_barrier();
         // of 64 chunks = 16 k-steps: bits 5 .. 2 of a chunk's number are the k-step's, added in registers; bits 1 and 0
-        // the chunk of the k-step, which lanes 8 r' + r hold (q & 3 here, so that the lanes 16 and 8 on have the others)
+        // the chunk of the k-step, which lanes ROWS r' + r hold (q & 3 here, so that the lanes 2 ROWS and ROWS on have the others)
         float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < (KT + 15) / 16; j++) {
@@ -1144,8 +1155,8 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
             for (int half = 8; half >= 1; half /= 2)
 #pragma unroll
                 for (int i = 0; i < half; i++) v[i] += v[i + half];
-            v[0] += wave_xor_f32(v[0], 16);
-            part[j] = v[0] + wave_xor_f32(v[0], 8);
+            v[0] += wave_xor_f32(v[0], 2 * ROWS);
+            part[j] = v[0] + wave_xor_f32(v[0], ROWS);
         }
         const float inv_rms = 1.0f / sqrtf(((part[0] + part[1]) + (part[2] + part[3])) / (float)a.K + p.eps);
 #pragma unroll
@@ -1160,10 +1171,9 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
     for (int i = 0; i < CH; i++)
 #pragma unroll
         for (int j = 0; j < 8; j++) mx = fmaxf(mx, fabsf(x[i][j / 4][j % 4]));
-    mx = fmaxf(mx, wave_xor_f32(mx, 8));
-    mx = fmaxf(mx, wave_xor_f32(mx, 16));
-    mx = fmaxf(mx, wave_xor_f32(mx, 32));
-    if (lane < 8) s_mx[wave][lane] = mx;
+#pragma unroll
+    for (int off = ROWS; off < 64; off *= 2) mx = fmaxf(mx, wave_xor_f32(mx, off));
+    if (lane < ROWS) s_mx[wave][lane] = mx;
     lds_barrier();
     mx = fmaxf(fmaxf(s_mx[0][r], s_mx[1][r]), fmaxf(s_mx[2][r], s_mx[3][r]));
     uint32_t ex = (__float_as_uint(mx) >> 23) & 0xFFu;
@@ -1187,13 +1197,13 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
             hi[j] = h;
             lo[j] = (_Float16)fmaf((float)h, -kProjLoScale, sv * kProjLoScale);
         }
-        half8* to = frag + (2 * i + (q >> 2)) * 64 + 16 * (q & 3) + r;
+        half8* to = frag + (QS * i + (q >> 2)) * 64 + 16 * (q & 3) + r;
         to[0] = hi;
         to[8] = lo;
     }
 #pragma unroll
     for (int u = 0; u < D; u++) {
-        const half8 xb = frag[u * 64 + lane];
+        const half8 xb = frag[u * 64 + (lane & ~(8 - ROWS))];   // (ROWS = 4: columns 4 on are copies, dropped)
 #pragma unroll
         for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[u][t], xb, acc[t], 0, 0, 0);
     }
@@ -1214,9 +1224,9 @@ __global__ __launch_bounds__(kProjThreads, 1) void proj_rows_fused_kernel(const 
             for (int i = 0; i < 4; i++) acc[t][i] += other[i];
         }
         if constexpr (!GATED)
-            proj_store_tile(a, acc[t], nt0 + t, group, lane, &scale, &resid[t]);
+            proj_store_tile<ROWS>(a, acc[t], nt0 + t, group, lane, &scale, &resid[t]);
         else if (t % 2 == 1)
-            proj_store_pair(a, acc[t - 1], acc[t], (nt0 + t) / 2, group, lane, &scale);
+            proj_store_pair<ROWS>(a, acc[t - 1], acc[t], (nt0 + t) / 2, group, lane, &scale);
     }
 }
 

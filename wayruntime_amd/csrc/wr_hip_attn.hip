@@ -942,37 +942,38 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
 // proj_rows_fused_kernel<SRC, n_in / 128, nt>, or nullptr where none is built.
 using FusedKernel = void (*)(const ProjArgs, const ProjPrepArgs);
 
-template <int SRC, int D>
+template <int SRC, int D, int ROWS>
 FusedKernel fused_of(uint32_t nt, bool gated)
 {
     if (gated) {
         if constexpr (D <= 16)
-            if (nt == 2) return proj_rows_fused_kernel<SRC, D, 2, true>;
+            if (nt == 2) return proj_rows_fused_kernel<SRC, D, 2, true, ROWS>;
         if constexpr (D <= 8)
-            if (nt == 4) return proj_rows_fused_kernel<SRC, D, 4, true>;
+            if (nt == 4) return proj_rows_fused_kernel<SRC, D, 4, true, ROWS>;
         return nullptr;
     }
-    if (nt == 1) return proj_rows_fused_kernel<SRC, D, 1>;
+    if (nt == 1) return proj_rows_fused_kernel<SRC, D, 1, false, ROWS>;
     if constexpr (D <= 16)
-        if (nt == 2) return proj_rows_fused_kernel<SRC, D, 2>;
+        if (nt == 2) return proj_rows_fused_kernel<SRC, D, 2, false, ROWS>;
     if constexpr (D <= 8) {
-        if (nt == 3) return proj_rows_fused_kernel<SRC, D, 3>;
-        if (nt == 4) return proj_rows_fused_kernel<SRC, D, 4>;
+        if (nt == 3) return proj_rows_fused_kernel<SRC, D, 3, false, ROWS>;
+        if (nt == 4) return proj_rows_fused_kernel<SRC, D, 4, false, ROWS>;
     }
     return nullptr;
 }
 
+template <int ROWS>
 FusedKernel fused_kernel(int src, uint32_t n_in, uint32_t nt, bool gated)
 {
     const bool norm = src == kProjSrcRmsNorm;
     if (!norm && src != kProjSrcPlain) return nullptr;
     switch (n_in) {
-    case 512: return norm ? fused_of<kProjSrcRmsNorm, 4>(nt, gated) : fused_of<kProjSrcPlain, 4>(nt, gated);
-    case 1024: return norm ? fused_of<kProjSrcRmsNorm, 8>(nt, gated) : fused_of<kProjSrcPlain, 8>(nt, gated);
-    case 1536: return norm ? fused_of<kProjSrcRmsNorm, 12>(nt, gated) : fused_of<kProjSrcPlain, 12>(nt, gated);
-    case 2048: return norm ? fused_of<kProjSrcRmsNorm, 16>(nt, gated) : fused_of<kProjSrcPlain, 16>(nt, gated);
-    case 2560: return norm ? nullptr : fused_of<kProjSrcPlain, 20>(nt, gated);
-    case 3072: return norm ? nullptr : fused_of<kProjSrcPlain, 24>(nt, gated);
+    case 512: return norm ? fused_of<kProjSrcRmsNorm, 4, ROWS>(nt, gated) : fused_of<kProjSrcPlain, 4, ROWS>(nt, gated);
+    case 1024: return norm ? fused_of<kProjSrcRmsNorm, 8, ROWS>(nt, gated) : fused_of<kProjSrcPlain, 8, ROWS>(nt, gated);
+    case 1536: return norm ? fused_of<kProjSrcRmsNorm, 12, ROWS>(nt, gated) : fused_of<kProjSrcPlain, 12, ROWS>(nt, gated);
+    case 2048: return norm ? fused_of<kProjSrcRmsNorm, 16, ROWS>(nt, gated) : fused_of<kProjSrcPlain, 16, ROWS>(nt, gated);
+    case 2560: return norm ? nullptr : fused_of<kProjSrcPlain, 20, ROWS>(nt, gated);
+    case 3072: return norm ? nullptr : fused_of<kProjSrcPlain, 24, ROWS>(nt, gated);
     default: return nullptr;
     }
 }
@@ -982,10 +983,15 @@ FusedKernel fused_kernel(int src, uint32_t n_in, uint32_t nt, bool gated)
 // a CU would make the same rows' terms again, and that is vector-ALU time nothing
 // hides: 16 rows, norm + 1024 -> 4096, one / two / three / four tiles (512 / 256 / 172 /
 // 128 workgroups) 6.7 / 5.2 / 5.9 / 6.5 us; -> 6144 8.6 / 7.8 / 6.2 / 6.8.
-FusedKernel pick_fused(int src, uint32_t n_in, uint32_t tiles, uint32_t groups, bool gated, uint32_t* nt)
+//
+// Rows: four to a workgroup where there are CUs for it, eight otherwise, at the same number of tiles.  Halving the rows
+// for twice the tiles would double the weights that a CU has to take in (46 bytes a nanosecond at best): not done.
+FusedKernel pick_fused(int src, uint32_t n_in, uint32_t tiles, uint32_t rows, bool gated, uint32_t* nt, uint32_t* wg_rows)
 {
     for (*nt = gated ? 2 : 1; *nt <= 4; *nt += gated ? 2 : 1)
-        if ((tiles + *nt - 1) / *nt * groups <= (uint32_t)g.n_cus) return fused_kernel(src, n_in, *nt, gated);
+        for (*wg_rows = 4; *wg_rows <= 8; *wg_rows *= 2)
+            if ((tiles + *nt - 1) / *nt * ((rows + *wg_rows - 1) / *wg_rows) <= (uint32_t)g.n_cus)
+                return *wg_rows == 4 ? fused_kernel<4>(src, n_in, *nt, gated) : fused_kernel<8>(src, n_in, *nt, gated);
     return nullptr;
 }
 
@@ -1030,10 +1036,10 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     // up to a few dozen rows, where one workgroup per CU can take them all: so does each workgroup of the product.  It
     // reads the rows with 16-byte loads.
     // (Four waves to the inputs, as the kernel of one row then has: a row's bits are its own in a step of up to sixteen.)
-    uint32_t fused_nt = 0;
+    uint32_t fused_nt = 0, fused_rows = 0;
     const FusedKernel fused =
         rows > 1 && rows < kProjGroupRows && (gemm || ksplit == 4) && ldx % 4 == 0 && ((x0 | (uintptr_t)src.norm_w) & 15) == 0 && apart
-            ? pick_fused(src.kind, w->n_in, tiles, groups, src.gate != 0, &fused_nt)
+            ? pick_fused(src.kind, w->n_in, tiles, rows, src.gate != 0, &fused_nt, &fused_rows)
             : nullptr;
     const size_t frag_bytes = (size_t)groups * ktiles * 1024;
     int rc = ensure_device(cx->d_proj, frag_bytes + kProjMaxRows * sizeof(float));
@@ -1119,7 +1125,7 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
         else
             launch_main(proj_row1_kernel<kProjSrcPlain>, grid, block, a, pa, lds);
     } else if (fused)
-        launch_main(fused, dim3((tiles + fused_nt - 1) / fused_nt, groups), dim3(kProjThreads), a, pa, (size_t)w->n_in * 32);
+        launch_main(fused, dim3((tiles + fused_nt - 1) / fused_nt, (rows + fused_rows - 1) / fused_rows), dim3(kProjThreads), a, pa, (size_t)w->n_in * 32);
     else if (gemm)
         launch_proj_gemm(a, groups);
     else if (src.gate && groups == 1)
@@ -1272,7 +1278,10 @@ int wr_hip_attn_init(int device)
         for (uint32_t n_in = 512; n_in <= 3072; n_in += 512)
             for (uint32_t nt = 1; nt <= 4; nt++)
                 for (const int src : {kProjSrcPlain, kProjSrcRmsNorm})
-                    for (const bool gated : {false, true}) allow_lds(fused_kernel(src, n_in, nt, gated), (size_t)n_in * 32);
+                    for (const bool gated : {false, true}) {
+                        allow_lds(fused_kernel<4>(src, n_in, nt, gated), (size_t)n_in * 32);
+                        allow_lds(fused_kernel<8>(src, n_in, nt, gated), (size_t)n_in * 32);
+                    }
         if (e != hipSuccess) rc = hip_fail(e, "kernel LDS size", 0);
     }
     if (rc != WR_HIP_OK) {
