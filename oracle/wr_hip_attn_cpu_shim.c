@@ -351,6 +351,12 @@ int wr_hip_proj_rows_norm_dev(const wr_hip_weight *w, uint32_t rows, const float
     (void)w; (void)rows; (void)x; (void)ldx; (void)nw; (void)eps; (void)add; (void)y; (void)ldy;
     return WR_HIP_ERR_STATE;
 }
+int wr_hip_proj_rows_norm_down(const wr_hip_weight *w, uint32_t rows, const float *x, uint32_t ldx, const float *nw,
+                               float eps, float *const *dst, float *tmp)
+{
+    (void)w; (void)rows; (void)x; (void)ldx; (void)nw; (void)eps; (void)dst; (void)tmp;
+    return WR_HIP_ERR_STATE;
+}
 int wr_hip_proj_rows_swiglu_dev(const wr_hip_weight *w, uint32_t rows, const float *gu, uint32_t ld,
                                 const float *add, float *y, uint32_t ldy)
 {

@@ -616,3 +616,39 @@ def test_rows_of_a_few_equal_the_row_alone(n_in):
         for d in (xd, nwd, addd, y):
             d.free()
         w.close()
+
+
+@pytest.mark.parametrize("n_in,n_out", [(96, 32768), (1024, 32912), (64, 32800), (256, 144)])
+def test_rows_of_a_product_into_host_memory(n_in, n_out):
+    # One row, weights that a wave takes alone (ragged ends of a workgroup's 128 outputs among
+    # them) and a narrow one: the bits of the product in device memory, and nothing beside the rows.
+    lib = hipattn.lib()
+    D = hipattn.DeviceBuffer
+    x = synth.normal(91 + n_in, (17, n_in), std=2.0)
+    nw = synth.normal(92, (n_in,)) * np.float32(0.2) + np.float32(1.0)
+    w = hipattn.Weight([_w16(93, n_out, n_in, 0.1)])
+    xd, nwd, y = D.from_host(x), D.from_host(nw), D(17 * n_out * 4)
+    places = [lib.wr_hip_attn_host_alloc((n_out + 4) * 4) for _ in range(16)]
+    rows = [np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_float)), shape=(n_out + 4,)) for p in places]
+    dst = (C.c_void_p * 16)(*places)
+    for n in (1, 2, 3, 7, 8, 9, 13, 16):
+        for r in rows:
+            r[:] = 7.0
+        assert lib.wr_hip_proj_rows_norm_dev(w.h, n, xd.p, n_in, nwd.p, 1e-6, None, y.p, n_out) == hipattn.OK
+        hipattn.sync()
+        want = y.to_host((17, n_out))[:n]
+        print("rows down", n_in, n_out, n, flush=True)
+        assert lib.wr_hip_proj_rows_norm_down(w.h, n, xd.p, n_in, nwd.p, 1e-6, dst, y.p) == hipattn.OK
+        for i, r in enumerate(rows):
+            assert np.array_equal(r[:n_out], want[i]) if i < n else np.all(r == 7.0)
+            assert np.all(r[n_out:] == 7.0)
+    down = lib.wr_hip_proj_rows_norm_down
+    assert down(w.h, 17, xd.p, n_in, nwd.p, 1e-6, dst, y.p) == hipattn.ERR_LIMIT
+    assert down(w.h, 2, xd.p, n_in, None, 1e-6, dst, y.p) == hipattn.ERR_INVAL
+    assert down(w.h, 2, xd.p, n_in, nwd.p, 1e-6, (C.c_void_p * 2)(places[0], places[1] + 4), y.p) == hipattn.ERR_INVAL
+    assert down(w.h, 0, xd.p, n_in, nwd.p, 1e-6, dst, y.p) == hipattn.OK
+    for p in places:
+        lib.wr_hip_attn_host_free(p)
+    for d in (xd, nwd, y):
+        d.free()
+    w.close()

@@ -621,6 +621,83 @@ __device__ __forceinline__ void proj_step(f32x4 (&acc)[NT][GROUPS], const half8 
     }
 }
 
+// A wave's part of a product: NT tiles from nt0 on against all row groups, k-steps k_begin .. k_end - 1 in order.
+template <int GROUPS, int NT, bool GATED>
+__device__ __forceinline__ void proj_rows_sums(const ProjArgs& a, f32x4 (&acc)[NT][GROUPS], uint32_t nt0, uint32_t k_begin,
+                                               uint32_t k_end, int lane)
+{
+    constexpr int KB = kProjKBatch / NT;                               // k-steps per register batch
+    const uint32_t ktiles = a.K / 32, ntiles = a.N / 16;
+    const half8* xp = a.xfrag + lane;
+            // tile t of this wave; a run that sticks out past N re-reads the last tile and drops the result
+            const half8* wp[NT];
+    #pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const uint32_t nt = GATED ? proj_paired_tile(nt0, t, ntiles) : (nt0 + t < ntiles) ? nt0 + t : ntiles - 1;
+                wp[t] = a.w + (size_t)nt * ktiles * 64 + lane;
+            }
+            // W is read exactly once per launch (non-temporal); X fragments are
+            // shared by every wave of the grid and stay cached.  Loads inside the
+            // loop are unconditional and the last batch is peeled, so the
+            // compiler's load counting keeps the prefetched batch in flight.
+            half8 wa[KB][NT], wb[KB][NT];
+            // The operand fragments travel a batch ahead with the weights: read when
+            // needed they are cache hits, but a round trip to L2 per batch on a
+            // chain of four to thirty batches that is the launch's critical path.
+            half8 xa[KB][GROUPS], xb[KB][GROUPS];
+            auto load_x = [&](half8 (&xv)[KB][GROUPS], uint32_t k0) {
+    #pragma unroll
+                for (int u = 0; u < KB; u++)
+    #pragma unroll
+                    for (int gi = 0; gi < GROUPS; gi++) xv[u][gi] = xp[((size_t)gi * ktiles + k0 + u) * 64];
+            };
+            auto step = [&](const half8 (&wv)[NT], const half8 (&xv)[GROUPS]) {
+    #pragma unroll
+                for (int gi = 0; gi < GROUPS; gi++)
+    #pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        acc[t][gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[t], xv[gi], acc[t][gi], 0, 0, 0);
+            };
+            uint32_t kt = k_begin;
+    const uint32_t kper = k_end - k_begin;
+            const uint32_t full_end = k_begin + kper / KB * KB;
+            if (kt < full_end) {
+    #pragma unroll
+                for (int u = 0; u < KB; u++)
+    #pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        wa[u][t] = __builtin_nontemporal_load(&wp[t][(size_t)(kt + u) * 64]);
+                load_x(xa, kt);
+                while (kt + 2 * KB <= full_end) {
+    #pragma unroll
+                    for (int u = 0; u < KB; u++)
+    #pragma unroll
+                        for (int t = 0; t < NT; t++)
+                            wb[u][t] = __builtin_nontemporal_load(&wp[t][(size_t)(kt + KB + u) * 64]);
+                    load_x(xb, kt + KB);
+    #pragma unroll
+                    for (int u = 0; u < KB; u++) step(wa[u], xa[u]);
+    #pragma unroll
+                    for (int u = 0; u < KB; u++) {
+    #pragma unroll
+                        for (int t = 0; t < NT; t++) wa[u][t] = wb[u][t];
+    #pragma unroll
+                        for (int gi = 0; gi < GROUPS; gi++) xa[u][gi] = xb[u][gi];
+                    }
+                    kt += KB;
+                }
+    #pragma unroll
+                for (int u = 0; u < KB; u++) step(wa[u], xa[u]);
+                kt += KB;
+            }
+            for (; kt < k_end; kt++) {                               // part not a multiple of the batch
+                half8 wv[NT];
+    #pragma unroll
+                for (int t = 0; t < NT; t++) wv[t] = __builtin_nontemporal_load(&wp[t][(size_t)kt * 64]);
+                proj_step<GROUPS, NT>(acc, wv, xp, ktiles, kt);
+            }
+}
+
 // GROUPS = row groups of eight (one or two), NT = 16-output tiles per wave
 // (templates, so the accumulators stay in registers).  A workgroup is four
 // waves.  With ksplit = 1 they own four consecutive runs of 16*NT outputs; with
@@ -634,7 +711,6 @@ template <int GROUPS, int NT, bool GATED = false>
 __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs a)
 {
     static_assert(!GATED || NT == 2, "a gate's tile and a value's");
-    constexpr int KB = kProjKBatch / NT;                               // k-steps per register batch
     // partial sums of the waves with part > 0: (4 / S) runs x (S - 1) parts <= 3 entries
     __shared__ f32x4 s_part[3 * NT * GROUPS * 64];
 
@@ -648,7 +724,6 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
     const uint32_t ktiles = a.K / 32;
     const uint32_t kper = ktiles / S;                            // host guarantees divisibility
     const uint32_t k_begin = part * kper, k_end = k_begin + kper;
-    const half8* xp = a.xfrag + lane;
 
     f32x4 acc[NT][GROUPS];
 #pragma unroll
@@ -657,72 +732,7 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
         for (int gi = 0; gi < GROUPS; gi++) acc[t][gi] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     if (live) {
-        // tile t of this wave; a run that sticks out past N re-reads the last tile and drops the result
-        const half8* wp[NT];
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const uint32_t nt = GATED ? proj_paired_tile(nt0, t, ntiles) : (nt0 + t < ntiles) ? nt0 + t : ntiles - 1;
-            wp[t] = a.w + (size_t)nt * ktiles * 64 + lane;
-        }
-        // W is read exactly once per launch (non-temporal); X fragments are
-        // shared by every wave of the grid and stay cached.  Loads inside the
-        // loop are unconditional and the last batch is peeled, so the
-        // compiler's load counting keeps the prefetched batch in flight.
-        half8 wa[KB][NT], wb[KB][NT];
-        // The operand fragments travel a batch ahead with the weights: read when
-        // needed they are cache hits, but a round trip to L2 per batch on a
-        // chain of four to thirty batches that is the launch's critical path.
-        half8 xa[KB][GROUPS], xb[KB][GROUPS];
-        auto load_x = [&](half8 (&xv)[KB][GROUPS], uint32_t k0) {
-#pragma unroll
-            for (int u = 0; u < KB; u++)
-#pragma unroll
-                for (int gi = 0; gi < GROUPS; gi++) xv[u][gi] = xp[((size_t)gi * ktiles + k0 + u) * 64];
-        };
-        auto step = [&](const half8 (&wv)[NT], const half8 (&xv)[GROUPS]) {
-#pragma unroll
-            for (int gi = 0; gi < GROUPS; gi++)
-#pragma unroll
-                for (int t = 0; t < NT; t++)
-                    acc[t][gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[t], xv[gi], acc[t][gi], 0, 0, 0);
-        };
-        uint32_t kt = k_begin;
-        const uint32_t full_end = k_begin + kper / KB * KB;
-        if (kt < full_end) {
-#pragma unroll
-            for (int u = 0; u < KB; u++)
-#pragma unroll
-                for (int t = 0; t < NT; t++)
-                    wa[u][t] = __builtin_nontemporal_load(&wp[t][(size_t)(kt + u) * 64]);
-            load_x(xa, kt);
-            while (kt + 2 * KB <= full_end) {
-#pragma unroll
-                for (int u = 0; u < KB; u++)
-#pragma unroll
-                    for (int t = 0; t < NT; t++)
-                        wb[u][t] = __builtin_nontemporal_load(&wp[t][(size_t)(kt + KB + u) * 64]);
-                load_x(xb, kt + KB);
-#pragma unroll
-                for (int u = 0; u < KB; u++) step(wa[u], xa[u]);
-#pragma unroll
-                for (int u = 0; u < KB; u++) {
-#pragma unroll
-                    for (int t = 0; t < NT; t++) wa[u][t] = wb[u][t];
-#pragma unroll
-                    for (int gi = 0; gi < GROUPS; gi++) xa[u][gi] = xb[u][gi];
-                }
-                kt += KB;
-            }
-#pragma unroll
-            for (int u = 0; u < KB; u++) step(wa[u], xa[u]);
-            kt += KB;
-        }
-        for (; kt < k_end; kt++) {                               // part not a multiple of the batch
-            half8 wv[NT];
-#pragma unroll
-            for (int t = 0; t < NT; t++) wv[t] = __builtin_nontemporal_load(&wp[t][(size_t)kt * 64]);
-            proj_step<GROUPS, NT>(acc, wv, xp, ktiles, kt);
-        }
+        proj_rows_sums<GROUPS, NT, GATED>(a, acc, nt0, k_begin, k_end, lane);
     }
 
     if (S > 1) {                                                 // uniform over the workgroup
@@ -757,6 +767,62 @@ __global__ __launch_bounds__(kProjThreads) void proj_rows_kernel(const ProjArgs 
     for (int t = 0; t < NT; t++)
 #pragma unroll
         for (int gi = 0; gi < GROUPS; gi++) proj_store_tile(a, acc[t][gi], nt0 + t, gi, lane);
+}
+
+// The product of 2 to 16 rows and a wide weight (ksplit = 1: the sums of proj_rows_kernel) into rows of page-locked host
+// memory: the logits of a batched step, straight to where its sessions keep them.
+//
+// Bound by the link to the host: 16 rows of 151 936 are 9.7 MB, 175 us of it, against 66 for the weight from HBM (1024
+// inputs).  A workgroup's 128 outputs pass through LDS and go out 512 bytes of a row at a time, and its place on the
+// compute unit is free for the next one's weights while they travel.  The host gives a unit one workgroup (by its
+// LDS), so that the first results are on the link after a fifth of the weight has been read, and not after all of it: 16
+// rows, call to return, 216 us with all of 1187 workgroups at once, 205 so; 8 rows 133, 117; 2 rows 84, 78.  Against the
+// product to device memory and rows_down_kernel behind it (us): 1024 -> 151 936, 2 / 4 / 8 / 16 rows 87 / 109 / 154 / 257
+// -> 78 / 88 / 117 / 205; 2048 -> 65 536 70 / 79 / 98 / 141 -> 66 / 71 / 83 / 122; 4096 -> 32 768 70 / 73 / 83 / 101 ->
+// 63 / 64 / 74 / 95.  A step of sixteen sessions 1.45 -> 1.39 ms.
+struct ProjDownArgs {
+    f32x4* y[16];
+};
+
+constexpr int kDownCols = 128, kDownStride = kDownCols + 4;
+
+template <int GROUPS>
+__global__ __launch_bounds__(kProjThreads) void proj_rows_down_kernel(const ProjArgs a, const ProjDownArgs d)
+{
+    constexpr int NT = 2;
+    extern __shared__ __attribute__((aligned(16))) unsigned char down_smem[];
+    float* stage = reinterpret_cast<float*>(down_smem);          // [8 GROUPS][kDownStride]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t ntiles = a.N / 16, nt0 = (blockIdx.x * 4 + wave) * NT;
+    f32x4* to[GROUPS];                                           // thread t: unit t % 32 of rows t / 32 + 8 gi
+#pragma unroll
+    for (int gi = 0; gi < GROUPS; gi++) to[gi] = d.y[min(gi * 8 + threadIdx.x / 32, a.R - 1)];
+    f32x4 acc[NT][GROUPS];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int gi = 0; gi < GROUPS; gi++) acc[t][gi] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (nt0 < ntiles) proj_rows_sums<GROUPS, NT, false>(a, acc, nt0, 0, a.K / 32, lane);
+    const int c = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int gi = 0; gi < GROUPS; gi++) {
+        const float sc = a.scales[min((uint32_t)(gi * 8 + (c & 7)), a.R - 1)];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            f32x4 v = proj_join_terms(acc[t][gi]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] *= sc;
+            if (c < 8) *reinterpret_cast<f32x4*>(stage + (gi * 8 + c) * kDownStride + (wave * NT + t) * 16 + g * 4) = v;
+        }
+    }
+    lds_barrier();
+    const uint32_t unit = threadIdx.x % 32, at = blockIdx.x * (kDownCols / 4) + unit;
+    if (at >= a.N / 4) return;
+#pragma unroll
+    for (int gi = 0; gi < GROUPS; gi++) {
+        const uint32_t row = gi * 8 + threadIdx.x / 32;
+        if (row < a.R) to[gi][at] = *reinterpret_cast<const f32x4*>(stage + row * kDownStride + unit * 4);
+    }
 }
 
 // One row (a decode step): proj_rows_kernel<1, 1> with the fragment kernel

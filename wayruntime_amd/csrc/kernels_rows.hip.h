@@ -338,7 +338,8 @@ __global__ __launch_bounds__(256) void swiglu_rows_kernel(const float* __restric
 }
 
 // Rows of a block into page-locked host memory of their own, 16 bytes to a thread and store: a batched step's logits,
-// straight to where its sessions keep them.  Bound by the link to the host: sixteen rows of 151 936, 9.7 MB.  Against a
+// straight to where its sessions keep them, where the product cannot write them there itself (proj_rows_down_kernel:
+// it takes weights whose outputs are enough for a wave each).  Bound by the link to the host: sixteen rows of 151 936, 9.7 MB.  Against a
 // copy to one block (141 us) that the host's threads then shared out: a step of sixteen sessions 1.73 -> 1.55 ms.
 struct RowsDownArgs {
     f32x4* dst[16];

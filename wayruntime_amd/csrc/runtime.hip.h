@@ -89,6 +89,7 @@ constexpr uint32_t kDevErrLayerMask = 0x0000FFFFu;     // error word: bit 31 set
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr uint32_t kDefaultTilesPerWg = 32;  // split-K decode: 1024 keys per workgroup
 constexpr uint32_t kMaxHeads = 4096;        // query heads per session the ticket array is sized for
+constexpr size_t kOnePerCuLds = 82 * 1024;  // more than half of a compute unit's LDS
 constexpr size_t kPinSmall = 1u << 20;      // host copies up to this size go through pinned staging
 
 void logmsg(int level, const char* fmt, ...);

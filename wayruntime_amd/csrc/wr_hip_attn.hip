@@ -1004,10 +1004,28 @@ struct ProjSource {
     int gate = 0;            // kProjSrcSwiglu, kProjSrcGeglu: the weight's halves are gates and values (GATED kernels)
 };
 
-// y_dev[rows][ldy] = source(x_dev)[rows][n_in] . W^T (+ add_dev), rows <= kProjMaxRows.
-// The caller has entered.
+// Waves that share a run of outputs (contiguous parts of the inputs, summed
+// through LDS in a fixed order): enough that a narrow weight still gives
+// one to two thousand waves.  A function of the weight's shape only: a row's
+// sums are then split the same way whether it travels alone or with up to
+// fifteen others, so a batched step's rows equal the serial steps' bit
+// for bit (reference contract: src/core/batch.c:15-19).  From 17 rows on the
+// kernels have splits of their own.
+uint32_t proj_ksplit(const wr_hip_weight* w)
+{
+    const uint32_t tiles = w->n_out / 16, ktiles = w->n_in / 32;
+    uint32_t ksplit = 1;
+    while (ksplit < 4 && tiles * ksplit < 2048 && ktiles % (ksplit * 2) == 0 &&
+           ktiles / (ksplit * 2) >= 4)
+        ksplit *= 2;
+    return ksplit;
+}
+
+// y_dev[rows][ldy] = source(x_dev)[rows][n_in] . W^T (+ add_dev), rows <= kProjMaxRows;
+// or, with `down`, into those rows of host memory (2 to 16, a weight of ksplit 1).  The caller has entered.
 int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev, uint32_t ldx,
-                      const ProjSource& src, const float* add_dev, float* y_dev, uint32_t ldy)
+                      const ProjSource& src, const float* add_dev, float* y_dev, uint32_t ldy,
+                      const ProjDownArgs* down = nullptr)
 {
     const uint32_t groups = (rows + 7) / 8;                // row groups of eight
     const bool gemm = rows >= (uint32_t)kProjGemmMinRows;
@@ -1018,27 +1036,14 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     const uintptr_t x0 = (uintptr_t)x_dev, y0 = (uintptr_t)y_dev;
     const bool apart = x0 + ((size_t)(rows - 1) * ldx + x_cols) * 4 <= y0 || y0 + ((size_t)(rows - 1) * ldy + y_cols) * 4 <= x0;
     // one row: the fragment step runs inside the product's kernel (4 bytes of LDS per input)
-    const bool row1 = rows == 1 && apart && (size_t)w->n_in * 4 <= kProjRow1MaxLds;
-    // Waves that share a run of outputs (contiguous parts of the inputs, summed
-    // through LDS in a fixed order): enough that a narrow weight still gives
-    // one to two thousand waves.  A function of the weight's shape only: a row's
-    // sums are then split the same way whether it travels alone or with up to
-    // fifteen others, so a batched step's rows equal the serial steps' bit
-    // for bit (reference contract: src/core/batch.c:15-19).  From 17 rows on the
-    // kernels have splits of their own.
-    const uint32_t tiles = w->n_out / 16;
-    uint32_t ksplit = 1;
-    if (groups <= 2) {
-        while (ksplit < 4 && tiles * ksplit < 2048 && ktiles % (ksplit * 2) == 0 &&
-               ktiles / (ksplit * 2) >= 4)
-            ksplit *= 2;
-    }
+    const bool row1 = !down && rows == 1 && apart && (size_t)w->n_in * 4 <= kProjRow1MaxLds;
+    const uint32_t tiles = w->n_out / 16, ksplit = groups <= 2 ? proj_ksplit(w) : 1;
     // up to a few dozen rows, where one workgroup per CU can take them all: so does each workgroup of the product.  It
     // reads the rows with 16-byte loads.
     // (Four waves to the inputs, as the kernel of one row then has: a row's bits are its own in a step of up to sixteen.)
     uint32_t fused_nt = 0, fused_rows = 0;
     const FusedKernel fused =
-        rows > 1 && rows < kProjGroupRows && (gemm || ksplit == 4) && ldx % 4 == 0 && ((x0 | (uintptr_t)src.norm_w) & 15) == 0 && apart
+        !down && rows > 1 && rows < kProjGroupRows && (gemm || ksplit == 4) && ldx % 4 == 0 && ((x0 | (uintptr_t)src.norm_w) & 15) == 0 && apart
             ? pick_fused(src.kind, w->n_in, tiles, rows, src.gate != 0, &fused_nt, &fused_rows)
             : nullptr;
     const size_t frag_bytes = (size_t)groups * ktiles * 1024;
@@ -1103,7 +1108,10 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
     a.ldy = ldy;
     a.gate = (uint8_t)src.gate;
     a.ksplit = (uint8_t)ksplit;
-    if (row1) {
+    if (down) {
+        const dim3 grid((tiles + 7) / 8);
+        launch_main(groups == 1 ? proj_rows_down_kernel<1> : proj_rows_down_kernel<2>, grid, dim3(kProjThreads), a, *down, kOnePerCuLds);
+    } else if (row1) {
         const uint32_t per_block = 4 / ksplit, pair_blocks = (tiles / 2 + per_block - 1) / per_block;
         const bool pairs = src.gate && pair_blocks * 2 > g.n_cus;
         const dim3 grid(pairs ? pair_blocks : (tiles + per_block - 1) / per_block), block(kProjThreads);
@@ -1265,6 +1273,8 @@ int wr_hip_attn_init(int device)
                 e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         };
         // (a gated row: 6 KiB of partial tiles beside its terms, more than 64 KiB together from 14 848 inputs on)
+        allow_lds(proj_rows_down_kernel<1>, kOnePerCuLds);
+        allow_lds(proj_rows_down_kernel<2>, kOnePerCuLds);
         allow_lds(proj_row1_kernel<kProjSrcRmsNorm, kRow1Gated>, kProjRow1MaxLds);
         allow_lds(proj_row1_kernel<kProjSrcPlain, kRow1Gated>, kProjRow1MaxLds);
         allow_lds(proj_gemm_lds_kernel<8, 2, 3>, gemm_lds_bytes<8, 2, 3>());
@@ -2252,6 +2262,32 @@ int wr_hip_proj_rows_norm_dev(const wr_hip_weight* w, uint32_t rows, const float
     src.norm_w = norm_w_dev;
     src.eps = eps;
     return proj_dev_common(w, rows, x_dev, ldx, w ? w->n_in : 0, src, add_dev, y_dev, ldy);
+}
+
+int wr_hip_proj_rows_norm_down(const wr_hip_weight* w, uint32_t rows, const float* x_dev, uint32_t ldx,
+                               const float* norm_w_dev, float eps, float* const* dst_locked, float* tmp_dev)
+{
+    int rc = check_proj(w, rows, x_dev, ldx, w ? w->n_in : 0, tmp_dev, w ? w->n_out : 0, w ? w->n_out : 0);
+    if (rc || rows == 0) return rc;
+    if (rows > WR_HIP_BATCH_MAX) return WR_HIP_ERR_LIMIT;
+    if (!norm_w_dev || !dst_locked || ((uintptr_t)tmp_dev & 15)) return WR_HIP_ERR_INVAL;
+    ProjDownArgs d{};
+    for (uint32_t i = 0; i < rows; i++) {
+        if (!dst_locked[i] || ((uintptr_t)dst_locked[i] & 15)) return WR_HIP_ERR_INVAL;
+        d.y[i] = reinterpret_cast<f32x4*>(dst_locked[i]);
+    }
+    ProjSource src;
+    src.kind = kProjSrcRmsNorm;
+    src.norm_w = norm_w_dev;
+    src.eps = eps;
+    ENTER();
+    if (rows > 1 && proj_ksplit(w) == 1) {
+        rc = proj_chunk_locked(w, rows, x_dev, ldx, src, nullptr, tmp_dev, w->n_out, &d);
+        return rc ? rc : sync_checked("product down", 0);
+    }
+    rc = proj_locked(w, rows, x_dev, ldx, src, nullptr, rows == 1 ? dst_locked[0] : tmp_dev, w->n_out);
+    if (rc) return rc;
+    return rows == 1 ? sync_checked("product down", 0) : wr_hip_attn_rows_d2h(rows, dst_locked, tmp_dev, w->n_out);
 }
 
 int wr_hip_proj_rows_swiglu_dev(const wr_hip_weight* w, uint32_t rows, const float* gate_up_dev,

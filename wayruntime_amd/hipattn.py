@@ -95,6 +95,7 @@ def load() -> C.CDLL:
         "wr_hip_proj_weight_cols": (_u32, [_vp]),
         "wr_hip_proj_rows": (C.c_int, [_vp, _u32, _vp, _vp]),
         "wr_hip_proj_rows_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, _vp, _u32]),
+        "wr_hip_proj_rows_norm_down": (C.c_int, [_vp, _u32, _vp, _u32, _vp, C.c_float, C.POINTER(_vp), _vp]),
         "wr_hip_proj_rows_norm_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, C.c_float, _vp, _vp, _u32]),
         "wr_hip_proj_rows_swiglu_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, _vp, _u32]),
         "wr_hip_attn_step_create": (C.c_int, [_u32, C.POINTER(StepLayer), _u32, _u32, _u32, C.c_float, C.POINTER(_vp)]),

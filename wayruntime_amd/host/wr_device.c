@@ -539,17 +539,11 @@ static wr_status forward_pass(wr_model *m, wrh_workspace *hs, wrh_devspace *ds, 
     rc = WR_HIP_OK;
     const char *what = "sync";
     if (logits) {
-        /* One row: the product writes it where the session keeps it, across the link while it reads the weight.
-         * More: 600 KB each at a vocabulary of 150 000, and the link would take longer than the product. */
+        /* the product writes the rows where the sessions keep them, across the link while it reads the weight */
         float *rows[WR_BATCH_MAX];
         for (uint32_t r = 0; r < R; r++) rows[r] = ss[r]->logits;
         what = "final norm + lm head";
-        rc = wr_hip_proj_rows_norm_dev(d->lm_head, R, ds->resid, hidden, d->final_norm, m->rms_eps, NULL,
-                                       R == 1 ? rows[0] : ds->logits, m->vocab);
-        if (rc == WR_HIP_OK) {
-            what = "logits down";
-            rc = R == 1 ? wr_hip_attn_sync() : wr_hip_attn_rows_d2h(R, rows, ds->logits, m->vocab);
-        }
+        rc = wr_hip_proj_rows_norm_down(d->lm_head, R, ds->resid, hidden, d->final_norm, m->rms_eps, rows, ds->logits);
     } else {
         /* the upload above was synchronous: the host buffers are free again */
         if (next_rows && !d->embed) wrh_stage_next_rows(m, hs, next_rows, tokens + R, pos0 + R);
