@@ -160,7 +160,8 @@ typedef struct wr_hip_mix_gemm {
     uint32_t x_kt, x_kt_z;
     uint32_t rows;
     const int32_t *group_expert;
-    uint32_t tile_groups;          /* with group_expert: groups that share an expert come in runs of this many (1 or 8) */
+    uint32_t tile_groups;          /* with group_expert: groups that share an expert come in runs of this many (1 or 8); a
+                                    * negative expert: no rows, and nothing that can be relied on is stored for them */
     uint32_t out;
     float *y_f32;
     void *y_act;

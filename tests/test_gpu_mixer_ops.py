@@ -288,6 +288,33 @@ def test_runs_whose_last_groups_hold_no_pair(lib, N, K, runs_each, spare, expert
         b.free()
 
 
+@pytest.mark.parametrize("experts,spare", [(8, 3), (8, 4), (15, 5), (20, 7), (20, 10)])    # up to 48, 64 rows an expert; runs by XCD or not
+@pytest.mark.parametrize("N,K", [(64, 1024), (64, 1056), (1536, 544), (1568, 544), (96, 64), (32, 2080)])
+def test_runs_of_every_length(lib, experts, spare, N, K):
+    # a run of one to eight groups with rows: workgroups of four and of eight groups, an XCD to a run and runs dealt out
+    r = Run(lib, False, experts, N, K, 0)
+    runs = experts + spare
+    which = np.full(8 * runs, -1, dtype=np.int32)
+    for e in range(experts):
+        which[8 * e:8 * e + 1 + (5 * e) % 8] = e
+    rows, live = 16 * len(which), np.repeat(which, 16) >= 0
+    x = r.act(rows, K)
+    xd, gd = r.up(x), hipattn.DeviceBuffer.from_host(which.view(np.float32))
+    y, h = hipattn.DeviceBuffer(rows * N * 4), hipattn.DeviceBuffer(rows * (N // 32 * 16 + 32) * 2)
+    r.go(xd, rows=rows, group_expert=gd.p, tile_groups=8, out=ROWS_F32, y_f32=y.p, ldy=N)
+    want = np.concatenate([x[16 * g:16 * g + 16].astype(np.float64) @ r.w[e].T.astype(np.float64) for g, e in enumerate(which) if e >= 0])
+    r.close(y.to_host((rows, N))[live], want)
+    factor = r.rng.uniform(0, 2, rows).astype(np.float32)
+    fd = hipattn.DeviceBuffer.from_host(factor)
+    if N % 64 == 0:
+        r.go(xd, rows=rows, group_expert=gd.p, tile_groups=8, out=GATED, h=h.p, h_kt=N // 64, x_scale=fd.p)
+        t = (want * factor[live][:, None]).reshape(len(want), N // 32, 2, 16)
+        r.close(r.frag_down(h, rows, N // 2)[live], (O.silu(t[:, :, 0]) * t[:, :, 1]).reshape(len(want), -1), eight_bits=True)
+    r.end()
+    for b in (xd, gd, y, h, fd):
+        b.free()
+
+
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("N,K,tile", [(64, 96, 1), (48, 64, 8), (4096, 64, 8), (1024, 32, 1)])
 def test_matrix_per_row_group(lib, f32, N, K, tile):

@@ -27,7 +27,8 @@ struct MixGemmArgs {
     uint32_t out, ldy, h_kt, col_z, n_split, silu_end, sigmoid_end, tanh_end, relu2, gelu;
     float scale, limit, slope, up_bias;
     const float* bias;
-    uint32_t cols;                   // mix_gemm_lds_kernel without experts: XCDs that share out the outputs (xcd_tile)
+    uint32_t cols;                   // mix_gemm_lds_kernel without experts: XCDs that share out the outputs (xcd_tile);
+                                     // a stream of experts: runs that the XCDs share out, or 0
     const uint32_t* x_perm;
     const float* x_scale;            // a factor per row of the input (applied to its products), or nullptr
     float* y;
@@ -156,7 +157,11 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // Few rows: bound by the weights' bytes.  More rows: by the bytes that pass a
 // compute unit's vector cache, NT + GR KiB a k-step for NT x GR products.
 // STREAM: every weight tile is read by one workgroup only (no use in keeping it).
-// With group_expert the GR groups share an expert (GR divides tile_groups).
+// With group_expert the GR groups share an expert (GR divides tile_groups), and of a run's only those are read,
+// multiplied and stored that rows are in: a compute unit takes in 47 KiB a microsecond, 2 of weights and one for each
+// group of rows with every k-step.  64 experts, 48 rows each give or take a third, 2048 -> 1024: groups of four with the
+// empty ones 68 us, without them 64, all eight that a run may have in one workgroup 62, its workgroups on one XCD
+// 58; 64 rows each 88 (LDS tiles) -> 64.
 //
 // PARTS = 2 (one group of rows, one matrix, no gate): two workgroups take half of the
 // input range each, and the one that draws the tile's second ticket adds the other's
@@ -173,12 +178,27 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
     const int lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     static_assert(PARTS == 1 || (PARTS == 2 && NT == 1 && GR == 1), "one tile, two halves");
-    const uint32_t nt0 = blockIdx.x * NT, group0 = PARTS > 1 ? 0 : blockIdx.y * GR, part = PARTS > 1 ? blockIdx.y : 0, z = blockIdx.z;
-    uint32_t mat = z;
+    uint32_t bx = blockIdx.x, by = blockIdx.y;
+    if constexpr (STREAM && GR > 1) {
+        if (a.cols) {                                      // runs, up to a multiple of 8: a run's workgroups on one XCD
+            const uint32_t id = by * gridDim.x + bx, in_xcd = id / 8, y = in_xcd / gridDim.x * 8 + id % 8;
+            bx = in_xcd % gridDim.x;
+            by = y < a.cols ? y * (8 / GR) : (y - a.cols) * (8 / GR) + 1;       // GR = 4: first halves of all runs, then the second
+            if (by * GR >= a.groups) return;
+        }
+    }
+    const uint32_t nt0 = bx * NT, group0 = PARTS > 1 ? 0 : by * GR, part = PARTS > 1 ? by : 0, z = blockIdx.z;
+    uint32_t mat = z, live = GR;                           // live: groups that rows are in (those of a run come first)
     if (a.group_expert) {
         const int e = a.group_expert[group0];
         if (e < 0) return;                                 // uniform over the workgroup
         mat = (uint32_t)e;
+        if constexpr (STREAM && GR > 1) {
+            live = 1;
+#pragma unroll
+            for (uint32_t i = 1; i < GR; i++)
+                if (a.group_expert[group0 + i] >= 0) live = i + 1;
+        }
     }
     const uint32_t k_begin = a.ktiles * (part * WAVES + wave) / (PARTS * WAVES),
                    n = a.ktiles * (part * WAVES + wave + 1) / (PARTS * WAVES) - k_begin;
@@ -200,79 +220,102 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
         }
     }
 
-    f32x4 acc[NT][GR];
-#pragma unroll
-    for (int t = 0; t < NT; t++)
-#pragma unroll
-        for (int i = 0; i < GR; i++) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    bf16x8 w[D][NT];
-    V8 x[D][GR];
-    auto load = [&](bf16x8 (&wv)[NT], V8 (&xv)[GR], uint32_t k) {
+    const auto product = [&](auto groups) {
+        constexpr int L = decltype(groups)::value;
+        f32x4 acc[NT][L];
 #pragma unroll
         for (int t = 0; t < NT; t++)
-            wv[t] = STREAM ? __builtin_nontemporal_load(&wp[t][k * 64 + lane]) : wp[t][k * 64 + lane];
 #pragma unroll
-        for (int i = 0; i < GR; i++) xv[i] = xp[i][k * 64 + x_lane];
-    };
-    auto multiply = [&](const bf16x8 (&wv)[NT], const V8 (&xv)[GR]) {
+            for (int i = 0; i < L; i++) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+        bf16x8 w[D][NT];
+        V8 x[D][L];
+        auto load = [&](bf16x8 (&wv)[NT], V8 (&xv)[L], uint32_t k) {
 #pragma unroll
-        for (int i = 0; i < GR; i++)
+            for (int t = 0; t < NT; t++)
+                wv[t] = STREAM ? __builtin_nontemporal_load(&wp[t][k * 64 + lane]) : wp[t][k * 64 + lane];
 #pragma unroll
-            for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(wv[t], xv[i], acc[t][i]);
-    };
-    if constexpr (F32) {
-        // Half a turn is asked for, then the other half multiplied: eight 32-bit products to a tile and k-step are as long
-        // as a load, and asked for behind them it is late (4096 -> 4096 at 24 rows 26.2 us, 21.2 now; gated, one row,
-        // 1536 -> 4096 9.8, 8.3).  Past the end the last step is read again and not used.
-        constexpr int H = D / 2;
-        auto ask = [&](int d, uint32_t k) {
-#pragma unroll
-            for (int u = 0; u < H; u++) load(w[d + u], x[d + u], min(k + u, n - 1));
+            for (int i = 0; i < L; i++) xv[i] = xp[i][k * 64 + x_lane];
         };
-        auto take = [&](int d, uint32_t k) {
+        auto multiply = [&](const bf16x8 (&wv)[NT], const V8 (&xv)[L]) {
 #pragma unroll
-            for (int u = 0; u < H; u++)
-                if (k + u < n) multiply(w[d + u], x[d + u]);
+            for (int i = 0; i < L; i++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(wv[t], xv[i], acc[t][i]);
         };
-        if (n) ask(0, 0);
-        for (uint32_t k = 0; k < n; k += D) {
-            ask(H, k + H);
-            take(0, k);
-            ask(0, k + D);
-            take(H, k + H);
-        }
-    }
-    const uint32_t turns = F32 ? 0 : n / D, rest = F32 ? 0 : n - turns * D;
-    if (turns) {
+        if constexpr (F32) {
+            // Half a turn is asked for, then the other half multiplied: eight 32-bit products to a tile and k-step are as long
+            // as a load, and asked for behind them it is late (4096 -> 4096 at 24 rows 26.2 us, 21.2 now; gated, one row,
+            // 1536 -> 4096 9.8, 8.3).  Past the end the last step is read again and not used.
+            constexpr int H = D / 2;
+            auto ask = [&](int d, uint32_t k) {
 #pragma unroll
-        for (int d = 0; d < D; d++) load(w[d], x[d], d);
-        for (uint32_t turn = 1; turn < turns; turn++) {
+                for (int u = 0; u < H; u++) load(w[d + u], x[d + u], min(k + u, n - 1));
+            };
+            auto take = [&](int d, uint32_t k) {
 #pragma unroll
-            for (int d = 0; d < D; d++) {
-                multiply(w[d], x[d]);
-                load(w[d], x[d], turn * D + d);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int u = 0; u < H; u++)
+                    if (k + u < n) multiply(w[d + u], x[d + u]);
+            };
+            if (n) ask(0, 0);
+            for (uint32_t k = 0; k < n; k += D) {
+                ask(H, k + H);
+                take(0, k);
+                ask(0, k + D);
+                take(H, k + H);
             }
         }
+        const uint32_t turns = F32 ? 0 : n / D, rest = F32 ? 0 : n - turns * D;
+        if (turns) {
 #pragma unroll
-        for (int d = 0; d < D; d++) multiply(w[d], x[d]);
-    }
-    if (__builtin_expect(rest != 0, 0)) {
-        bf16x8 wr[D - 1][NT];
-        V8 xr[D - 1][GR];
+            for (int d = 0; d < D; d++) load(w[d], x[d], d);
+            for (uint32_t turn = 1; turn < turns; turn++) {
 #pragma unroll
-        for (int d = 0; d < D - 1; d++)
-            if ((uint32_t)d < rest) load(wr[d], xr[d], turns * D + d);
+                for (int d = 0; d < D; d++) {
+                    multiply(w[d], x[d]);
+                    load(w[d], x[d], turn * D + d);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
 #pragma unroll
-        for (int d = 0; d < D - 1; d++)
-            if ((uint32_t)d < rest) multiply(wr[d], xr[d]);
-    }
+            for (int d = 0; d < D; d++) multiply(w[d], x[d]);
+        }
+        if (__builtin_expect(rest != 0, 0)) {
+            bf16x8 wr[D - 1][NT];
+            V8 xr[D - 1][L];
+#pragma unroll
+            for (int d = 0; d < D - 1; d++)
+                if ((uint32_t)d < rest) load(wr[d], xr[d], turns * D + d);
+#pragma unroll
+            for (int d = 0; d < D - 1; d++)
+                if ((uint32_t)d < rest) multiply(wr[d], xr[d]);
+        }
 
 #pragma unroll
-    for (int t = 0; t < NT; t++)
+        for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int i = 0; i < GR; i++) s_part[((wave * NT + t) * GR + i) * 64 + lane] = acc[t][i];
+            for (int i = 0; i < L; i++) s_part[((wave * NT + t) * GR + i) * 64 + lane] = acc[t][i];
+    };
+    if constexpr (STREAM && GR > 1) {
+        static_assert(GR == 4 || GR == 8);
+        switch (live) {
+        case 1: product(std::integral_constant<int, 1>()); break;
+        case 2: product(std::integral_constant<int, 2>()); break;
+        case 3: product(std::integral_constant<int, 3>()); break;
+        case 4: product(std::integral_constant<int, 4>()); break;
+        default:
+            if constexpr (GR == 8) {
+                switch (live) {
+                case 5: product(std::integral_constant<int, 5>()); break;
+                case 6: product(std::integral_constant<int, 6>()); break;
+                case 7: product(std::integral_constant<int, 7>()); break;
+                default: product(std::integral_constant<int, 8>()); break;
+                }
+            }
+        }
+    } else {
+        product(std::integral_constant<int, GR>());
+    }
     lds_barrier();
     auto sum = [&](uint32_t i) {
         f32x4 v = s_part[i * 64 + lane];
@@ -308,6 +351,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
 #pragma unroll 1
             for (uint32_t u = wave; u < NT / 2 * GR; u += WAVES) {
                 const uint32_t t = u / GR * 2, i = u % GR;
+                if (i >= live) continue;
                 mix_store_tile<F32>(a, sum(t * GR + i), sum((t + 1) * GR + i), nt0 + t, group0 + i, z, lane);
             }
         }
@@ -315,6 +359,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
     }
 #pragma unroll 1
     for (uint32_t u = wave; u < NT * GR; u += WAVES) {
+        if (u % GR >= live) continue;
         const f32x4 v = sum(u);
         mix_store_tile<F32>(a, v, v, nt0 + u / GR, group0 + u % GR, z, lane);
     }

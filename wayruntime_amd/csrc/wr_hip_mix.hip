@@ -436,6 +436,29 @@ static int launch_split(const MixGemmArgs& a, uint32_t batch)
     return WR_HIP_OK;
 }
 
+// Runs of eight groups as a stream of their experts' weights.  A run's workgroups go to one XCD each run where that
+// leaves none more than a seventh without work (its rows then come into one L2 and not into eight, which is 8 rows / outputs
+// of the weights' bytes): up to 1536 outputs.  34 rows an expert, dealt out / by XCD (us): 64 experts, 4096 -> 384 64 / 43, -> 512 75
+// / 56, 2048 -> 1024 57 / 53; 128 experts, 2048 -> 768 86 / 79; 16 experts, 4096 -> 1536 46.5 / 40.6.  With more
+// outputs it is no gain (64 experts, 1024 -> 2048 58 / 59) or a loss (32 experts, 4096 -> 4096 199 / 209, 64, 384 ->
+// 4096 65 / 72: eight experts' weights and results at the same offsets).
+static bool runs_by_xcd(const MixGemmArgs& a, uint32_t experts)
+{
+    return a.ntiles <= 96 && (uint64_t)((experts + 7) / 8 * 8) * 7 <= (uint64_t)experts * 8;
+}
+
+template <int GR>
+static int launch_runs(const MixGemmArgs& args, uint32_t experts)
+{
+    MixGemmArgs a = args;
+    const uint32_t runs = a.groups / 8;
+    if (runs_by_xcd(a, experts)) a.cols = (runs + 7) / 8 * 8;
+    launch_main(mix_gemm_split_kernel<false, 2, GR, 4, 4, true>, dim3((a.ntiles + 1) / 2, (a.cols ? a.cols : runs) * (8 / GR)),
+                dim3(256), a);
+    HIP_TRY(hipGetLastError(), "product launch", 0);
+    return WR_HIP_OK;
+}
+
 // Two workgroups to a tile (PARTS), where both halves of all tiles run at once; from 4096 inputs on (figures at the
 // kernel).
 constexpr uint32_t kPartsMinKtiles = 128;
@@ -587,18 +610,25 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     if (q->group_expert) {
         if (!f32 && q->tile_groups == 8) {
             // Rows an expert has on average, from how many groups route leaves room for: a run per expert more than the
-            // pairs fill.  Up to 48 the product is a stream of the experts' weights: 64 rows of an expert at a time, so most
-            // experts' weights pass once (64 experts of 2048 x 1024, 48 rows each, give or take a third: 67 us against 95
-            // with the tile of 128 rows, most of them empty; 32 of 4096 x 4096 235 against 244).  From 56 on a part of the
-            // experts passes twice (32 of 4096 x 4096 300 against 244, and 334 at 64 rows).
-            // Narrow weights are no stream either: it reads the rows as often as the weights, and tiles that find a CU each
-            // are faster from 2048 inputs on (64 experts, 4096 -> 384: 68 us against 97, -> 512 87, 104; 48 experts, 4096 ->
-            // 640 77, 89; at 2048 inputs a tenth; 1024 -> 512 the same; 32 experts, 2048 -> 512 30.7, 28.9).
+            // pairs fill.  Up to 48 the product is a stream of the experts' weights that reads the rows that there are, and
+            // an expert's weights pass once, against a tile of 128 rows, most of them empty (us, stream / tile: 64
+            // experts, 2048 -> 1024 at 48 rows 58 / 88, 1024 -> 2048 62 / 83; 4096 -> 384 48 / 63; 128 experts, 2048 ->
+            // 768 85 / 128; 32 experts, 2048 -> 512 17.5 / 28.8, 4096 -> 4096 226 / 229; 8 experts, 4096 -> 14 336 202 /
+            // 210; the one that is slower, 16 experts, 1536 -> 4096 50 / 42).  Up to 64 rows where the weights are not so
+            // large that the tile is bound by them too, and the input range not so short that its ends are all of
+            // it (64 experts, 2048 -> 1024 64 / 88, 1024 -> 2048 73 / 83, 3072 -> 1536 149 / 173, 2048 -> 3072 156 / 183; 32
+            // experts, 1024 -> 2048 40 / 41; against 4096 -> 4096 250 / 229, 512 -> 2048 25 / 22.5), and to 80 where the runs
+            // are an XCD's each (64 experts, 2048 -> 1024 68 / 88, 3072 -> 1536 162 / 173, 4096 -> 384 59 / 64; 16
+            // experts, 4096 -> 1536 54 / 60).
+            // Over a short range workgroups of 64 rows, more to a compute unit, up to 48 rows (128 / 64 rows a workgroup:
+            // 64 experts, 384 -> 4096 70 / 58, 512 -> 4096 78 / 70, 1024 -> 2048 64 / 62; 2048 -> 1024 62 / 64; beyond, part of
+            // the experts' weights would pass twice: 1024 -> 2048 at 64 rows 73 / 80).
             // As many runs as experts, or fewer, are not route's: the caller counted them, so they may be full.
-            const uint64_t runs = a.groups / 8, e = q->w->batch, wgs = e * ((a.ntiles + 7) / 8);
-            const bool few = runs > e && (runs - e) * 128 <= e * 48;
-            const bool narrow = a.ktiles >= 64 && a.ntiles < 64 && wgs * 10 >= g.n_cus * 4ull && (a.ntiles <= 32 || wgs <= g.n_cus);
-            return few && !narrow ? launch_split<false, 2, 4, 4, 4, true>(a, 1) : launch_lds<4>(a, 1);
+            const uint64_t runs = a.groups / 8, e = q->w->batch, spare = runs > e ? (runs - e) * 128 : 0;
+            if (spare && spare <= e * 48 && a.ktiles <= 32) return launch_runs<4>(a, q->w->batch);
+            const uint32_t most = a.ktiles <= 16 || a.ntiles >= 256 ? 48 : runs_by_xcd(a, q->w->batch) ? 80 : 64;
+            if (spare && spare <= e * most) return launch_runs<8>(a, q->w->batch);
+            return launch_lds<4>(a, 1);
         }
         if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 8, true>(a, 1);
         if (!gated && a.ntiles * a.groups < 384) return launch_split<false, 1, 1, 4, 8, true>(a, 1);   // (as one group of rows below)
