@@ -315,6 +315,49 @@ def test_runs_of_every_length(lib, experts, spare, N, K):
         b.free()
 
 
+@pytest.mark.parametrize("N,K", [(1024, 544), (1040, 96), (512, 32), (1024, 512), (528, 2080)])
+def test_groups_of_an_expert_that_stand_together(lib, N, K):
+    # single groups in any order, a negative one among them; rows in order and picked one by one, of inputs that are the
+    # whole of their rows (brought together first) and of a part: each group's bits are those of the group by itself
+    experts = 5
+    r = Run(lib, False, experts, N, K, 0)
+    which = np.array([0] * 9 + [1, -1, 1, 1, 3, 2, 2, 2] + [4] * 5 + [-1, -1, 0, 0, 3, 3, 3, 3, 4, 0, 1], dtype=np.int32)
+    rows, live = 16 * len(which), np.repeat(which, 16) >= 0
+    x = r.act(rows, K)
+    xd, gd = r.up(x), hipattn.DeviceBuffer.from_host(which.view(np.float32))
+    y, y1 = hipattn.DeviceBuffer.from_host(np.full((rows, N), 7.0, dtype=np.float32)), hipattn.DeviceBuffer(16 * N * 4)
+    r.go(xd, rows=rows, group_expert=gd.p, tile_groups=1, out=ROWS_F32, y_f32=y.p, ldy=N)
+    got = y.to_host((rows, N))
+    want = np.concatenate([x[16 * g:16 * g + 16].astype(np.float64) @ r.w[e].T.astype(np.float64) for g, e in enumerate(which) if e >= 0])
+    r.close(got[live], want)
+    assert np.all(got[~live] == 7.0)
+    for g, e in enumerate(which):
+        if e < 0:
+            continue
+        one, ed = r.up(x[16 * g:16 * g + 16]), hipattn.DeviceBuffer.from_host(np.array([e], dtype=np.int32).view(np.float32))
+        r.go(one, rows=16, group_expert=ed.p, tile_groups=1, out=ROWS_F32, y_f32=y1.p, ldy=N)
+        assert y1.to_host((16, N)).tobytes() == got[16 * g:16 * g + 16].tobytes(), f"group {g}"
+        one.free()
+        ed.free()
+    pick = r.rng.integers(0, 37, rows).astype(np.uint32)
+    used = r.rng.random(rows) < 0.8
+    pd = hipattn.DeviceBuffer.from_host(np.where(used, pick, np.uint32(0xFFFFFFFF)).astype(np.uint32).view(np.float32))
+    few = r.act(37, K + 64)
+    fd, whole = r.up(few), r.up(np.ascontiguousarray(few[:, 32:32 + K]))
+    seen = live & used
+    want = np.concatenate([few[pick[16 * g:16 * g + 16], 32:32 + K].astype(np.float64) @ r.w[max(e, 0)].T.astype(np.float64)
+                           for g, e in enumerate(which)])[seen]
+    r.go(whole, rows=rows, group_expert=gd.p, tile_groups=1, out=ROWS_F32, y_f32=y.p, ldy=N, x_perm=pd.p)
+    got = y.to_host((rows, N))
+    r.close(got[seen], want)
+    assert np.all(got[~live] == 7.0)
+    r.go(fd, rows=rows, group_expert=gd.p, tile_groups=1, out=ROWS_F32, y_f32=y.p, ldy=N, x_perm=pd.p, x_kt=K // 32 + 2, x_kt0=1)
+    assert y.to_host((rows, N))[seen].tobytes() == got[seen].tobytes()
+    r.end()
+    for b in (xd, gd, y, y1, pd, fd, whole):
+        b.free()
+
+
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("N,K,tile", [(64, 96, 1), (48, 64, 8), (4096, 64, 8), (1024, 32, 1)])
 def test_matrix_per_row_group(lib, f32, N, K, tile):

@@ -161,7 +161,8 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // multiplied and stored that rows are in: a compute unit takes in 47 KiB a microsecond, 2 of weights and one for each
 // group of rows with every k-step.  64 experts, 48 rows each give or take a third, 2048 -> 1024: groups of four with the
 // empty ones 68 us, without them 64, all eight that a run may have in one workgroup 62, its workgroups on one XCD
-// 58; 64 rows each 88 (LDS tiles) -> 64.
+// 58; 64 rows each 88 (LDS tiles) -> 64.  PICKED: the same of single groups (tile_groups 1) in any order, cut at every
+// GR-th; alone a group has twice the k-steps on their way.
 //
 // PARTS = 2 (one group of rows, one matrix, no gate): two workgroups take half of the
 // input range each, and the one that draws the tile's second ticket adds the other's
@@ -170,7 +171,7 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // half of them idle is half the rate.  16 rows, weights from HBM: 8192 -> 2048 11.5 -> 9.4
 // us, -> 512 10.6 -> 7.8; 6144 -> 2048 9.4 -> 7.8; 4096 -> 2048 7.0 -> 6.6, -> 1024 6.7 ->
 // 6.0; at 2048 inputs the exchange costs more (4.8 -> 5.2).
-template <bool F32, int NT, int GR, int WAVES, int D, bool STREAM, int PARTS = 1>
+template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS = 1, bool PICKED = false>
 __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_kernel(const MixGemmArgs a)
 {
     using V8 = typename MixAct<F32>::V8;
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     static_assert(PARTS == 1 || (PARTS == 2 && NT == 1 && GR == 1), "one tile, two halves");
     uint32_t bx = blockIdx.x, by = blockIdx.y;
-    if constexpr (STREAM && GR > 1) {
+    if constexpr (STREAM && GR > 1 && !PICKED) {
         if (a.cols) {                                      // runs, up to a multiple of 8: a run's workgroups on one XCD
             const uint32_t id = by * gridDim.x + bx, in_xcd = id / 8, y = in_xcd / gridDim.x * 8 + id % 8;
             bx = in_xcd % gridDim.x;
@@ -187,13 +188,17 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
             if (by * GR >= a.groups) return;
         }
     }
-    const uint32_t nt0 = bx * NT, group0 = PARTS > 1 ? 0 : by * GR, part = PARTS > 1 ? by : 0, z = blockIdx.z;
+    const uint32_t nt0 = bx * NT, group0 = PARTS > 1 ? 0 : PICKED ? by : by * GR, part = PARTS > 1 ? by : 0, z = blockIdx.z;
     uint32_t mat = z, live = GR;                           // live: groups that rows are in (those of a run come first)
     if (a.group_expert) {
         const int e = a.group_expert[group0];
         if (e < 0) return;                                 // uniform over the workgroup
         mat = (uint32_t)e;
-        if constexpr (STREAM && GR > 1) {
+        if constexpr (PICKED) {                            // single groups: those of an expert that stand together, GR at most
+            if (group0 % GR && a.group_expert[group0 - 1] == e) return;
+            live = 1;
+            for (uint32_t i = group0 + 1; i % GR && i < a.groups && a.group_expert[i] == e; i++) live++;
+        } else if constexpr (STREAM && GR > 1) {
             live = 1;
 #pragma unroll
             for (uint32_t i = 1; i < GR; i++)
@@ -211,17 +216,22 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
 #pragma unroll
     for (int i = 0; i < GR; i++)
         xp[i] = reinterpret_cast<const V8*>(a.x) + ((size_t)min(group0 + i, a.groups - 1) * a.x_kt + (size_t)z * a.x_kt_z + k_begin) * 64;
-    uint32_t x_lane = lane;
-    if constexpr (GR == 1) {
+    uint32_t x_lane[GR];
+#pragma unroll
+    for (int i = 0; i < GR; i++) x_lane[i] = lane;
+    if constexpr (GR == 1 || PICKED) {
         if (a.x_perm) {                                    // rows picked one by one: the operand's lanes fetch their own
-            const uint32_t pick = a.x_perm[group0 * 16 + (lane & 15)], row = pick == 0xFFFFFFFFu ? 0 : pick;
-            xp[0] = reinterpret_cast<const V8*>(a.x) + (size_t)k_begin * 64;
-            x_lane = (row >> 4) * a.x_kt * 64 + (lane & 48) + (row & 15);
+#pragma unroll
+            for (int i = 0; i < GR; i++) {
+                const uint32_t pick = a.x_perm[min(group0 + i, a.groups - 1) * 16 + (lane & 15)], row = pick == 0xFFFFFFFFu ? 0 : pick;
+                xp[i] = reinterpret_cast<const V8*>(a.x) + (size_t)k_begin * 64;
+                x_lane[i] = (row >> 4) * a.x_kt * 64 + (lane & 48) + (row & 15);
+            }
         }
     }
 
     const auto product = [&](auto groups) {
-        constexpr int L = decltype(groups)::value;
+        constexpr int L = decltype(groups)::value, D = PICKED && L == 1 ? 2 * DEPTH : DEPTH;
         f32x4 acc[NT][L];
 #pragma unroll
         for (int t = 0; t < NT; t++)
@@ -235,7 +245,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
             for (int t = 0; t < NT; t++)
                 wv[t] = STREAM ? __builtin_nontemporal_load(&wp[t][k * 64 + lane]) : wp[t][k * 64 + lane];
 #pragma unroll
-            for (int i = 0; i < L; i++) xv[i] = xp[i][k * 64 + x_lane];
+            for (int i = 0; i < L; i++) xv[i] = xp[i][k * 64 + x_lane[i]];
         };
         auto multiply = [&](const bf16x8 (&wv)[NT], const V8 (&xv)[L]) {
 #pragma unroll

@@ -33,6 +33,7 @@ struct Ctx {
     hipStream_t stream = nullptr;
     Buffer d_stage;              // device staging for host-pointer entry points
     Buffer d_part;               // split-K partials
+    Buffer d_picked;             // experts' rows in slot order
     Buffer d_prefill;            // rows of prefill blocks cut into parts: at most kMaxPrefillPartMb, none where it is refused
     uint32_t prefill_refused = 0;     // launches that go uncut before memory for them is asked for again
     Buffer d_proj;               // projection operand fragments and row scales

@@ -718,6 +718,7 @@ void ctx_destroy(Ctx* c)
     for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
     if (c->d_stage.p) (void)hipFree(c->d_stage.p);
     if (c->d_part.p) (void)hipFree(c->d_part.p);
+    if (c->d_picked.p) (void)hipFree(c->d_picked.p);
     if (c->d_prefill.p) (void)hipFree(c->d_prefill.p);
     if (c->d_proj.p) (void)hipFree(c->d_proj.p);
     if (c->d_counters) (void)hipFree(c->d_counters);

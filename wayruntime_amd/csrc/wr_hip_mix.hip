@@ -436,12 +436,33 @@ static int launch_split(const MixGemmArgs& a, uint32_t batch)
     return WR_HIP_OK;
 }
 
+constexpr size_t kMaxPickedBytes = 64u << 20;
+
 // Runs of eight groups as a stream of their experts' weights.  A run's workgroups go to one XCD each run where that
 // leaves none more than a seventh without work (its rows then come into one L2 and not into eight, which is 8 rows / outputs
 // of the weights' bytes): up to 1536 outputs.  34 rows an expert, dealt out / by XCD (us): 64 experts, 4096 -> 384 64 / 43, -> 512 75
 // / 56, 2048 -> 1024 57 / 53; 128 experts, 2048 -> 768 86 / 79; 16 experts, 4096 -> 1536 46.5 / 40.6.  With more
 // outputs it is no gain (64 experts, 1024 -> 2048 58 / 59) or a loss (32 experts, 4096 -> 4096 199 / 209, 64, 384 ->
 // 4096 65 / 72: eight experts' weights and results at the same offsets).
+// Rows picked one by one, brought into the order of their slots first, when there is a place for them.
+static void pick_rows(MixGemmArgs& a)
+{
+    const size_t bytes = (size_t)a.groups * a.ktiles * 1024;
+    if (a.x_kt != a.ktiles || bytes > kMaxPickedBytes) return;
+    if (bytes > cx->d_picked.cap) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;     // (no allocation while a graph is recorded)
+        if (hipStreamIsCapturing(cx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
+            ensure_device(cx->d_picked, bytes) != WR_HIP_OK) {
+            (void)hipGetLastError();
+            return;
+        }
+    }
+    hipLaunchKernelGGL(mix_gather_kernel<false>, dim3((a.ktiles * 64 + 255) / 256, a.groups), dim3(256), 0, cx->stream, a.x, a.ktiles,
+                       a.groups, a.x_perm, a.group_expert, cx->d_picked.p);
+    a.x = cx->d_picked.p;
+    a.x_perm = nullptr;
+}
+
 static bool runs_by_xcd(const MixGemmArgs& a, uint32_t experts)
 {
     return a.ntiles <= 96 && (uint64_t)((experts + 7) / 8 * 8) * 7 <= (uint64_t)experts * 8;
@@ -632,6 +653,21 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
         }
         if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 8, true>(a, 1);
         if (!gated && a.ntiles * a.groups < 384) return launch_split<false, 1, 1, 4, 8, true>(a, 1);   // (as one group of rows below)
+        // Sixteen rows an expert and more, from how many groups route leaves room for, fill a second group here and
+        // there, which came with the weights once more: the groups of an expert that stand together, four at most, are one
+        // workgroup's.  Rows that are picked one by one are brought together first: a lane's sixteen bytes are a line
+        // each, and every workgroup of the launch asks for all of them again (us, as before / groups together / rows
+        // brought together too: 64 experts, 2048 -> 1024, 16 rows each 84 / 74 / 59, 30 rows 132 / 112 / 73; 32 experts, 4096
+        // -> 4096 308 / 268 / 200, 524 / 411 / 259; 128 experts, 1024 -> 384 35 / 36 / 35, 55 / 56 / 44; at 12 rows
+        // each 64 / 65 / 55, 226 / 223 / 188, 27.5 / 30.6 / 31.6).  Rows that are in order already gain less, and
+        // nothing over short ranges or few outputs (1024 -> 2048 57 / 51, 78 / 62; 4096 -> 4096 240 / 201; 384 -> 1024 23.4 /
+        // 25.1; 2048 -> 512 16.5 / 18.4).
+        if (a.groups >= 2 * q->w->batch && (a.x_perm || (a.ktiles > 16 && a.ntiles >= 64))) {
+            if (a.x_perm) pick_rows(a);
+            launch_main(mix_gemm_split_kernel<false, 2, 4, 4, 4, true, 1, true>, dim3((a.ntiles + 1) / 2, a.groups), dim3(256), a);
+            HIP_TRY(hipGetLastError(), "product launch", 0);
+            return WR_HIP_OK;
+        }
         return launch_split<false, 2, 1, 4, 8, true>(a, 1);
     }
     if (f32) {
