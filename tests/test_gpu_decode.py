@@ -1,6 +1,9 @@
 """Device decode attention and cache append against the CPU oracle, through
 the C ABI.  Tolerance: max-abs 2e-3 and rel-L2 1e-3 on the attention outputs
 (float32 accumulate), bit-exact on the cache contents."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
@@ -816,3 +819,47 @@ def test_append_decode_from_host_rows_refuses_what_it_must():
     gk, _gv = kv.read_f16(0, 3, 1)
     assert np.array_equal(gk[0], synth.f32_to_f16_trunc(k))
     kv.close(); other.close()
+
+
+def test_memory_of_ended_caches_is_bounded_and_comes_back_cleared():
+    def free_bytes():                                        # of the runtime that the library is linked with
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hipattn.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    nkv, hd, ctx = 4, 128, 70
+    x = synth.normal(7, (ctx, nkv, hd))
+    for _ in range(3):                                       # the same size again: what the one before held is gone
+        kv = hipattn.KVCache(2, hd, nkv, ctx)
+        for layer in (0, 1):
+            k, v = kv.read_f16(layer, 0, ctx)
+            assert not k.any() and not v.any()
+            assert kv.append(layer, 0, x, x) == hipattn.OK
+        kv.close()
+    free = free_bytes()
+    rows = 1 << 17                                           # 1 GiB a cache: two of them may be kept, and no more
+    caches = [hipattn.KVCache(4, hd, nkv, rows - 32 * i) for i in range(4)]
+    for kv in caches:
+        kv.close()
+    assert free - free_bytes() <= (2 << 30) + (64 << 20)
+    big = hipattn.KVCache(9, hd, nkv, rows)                  # more than is kept at all
+    big.close()
+    assert free - free_bytes() <= (2 << 30) + (64 << 20)
+
+    def walk(seed, out):                                     # sizes shared between threads, each with its own rows
+        r = np.random.default_rng(seed)
+        for _ in range(20):
+            kv = hipattn.KVCache(1, hd, nkv, ctx + 32 * int(r.integers(0, 2)))
+            rows = r.standard_normal((ctx, nkv, hd)).astype(np.float32)
+            ok = kv.append(0, 0, rows, rows) == hipattn.OK
+            k, _ = kv.read_f16(0, 0, ctx)
+            out.append(ok and np.array_equal(k, synth.f32_to_f16_trunc(rows)))
+            kv.close()
+
+    out = []
+    threads = [threading.Thread(target=walk, args=(i, out)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(out) == 80 and all(out)

@@ -60,6 +60,12 @@ struct Lib {
     uint32_t n_cus = 256;        // compute units of the device in use
     std::atomic<uint64_t> generation{0};   // bumped by every init: contexts of an earlier one are gone
     std::vector<Ctx*> ctxs;      // every context of this generation
+    struct Slab {
+        uint8_t* p;
+        size_t bytes;
+    };
+    std::mutex slab_mu;          // guards slabs; nothing else is locked while it is held
+    std::vector<Slab> slabs;     // memory of ended caches, cleared when it is taken again
     std::vector<Ctx*> idle;      // contexts whose thread has ended, for the next new thread
     char name[320] = "uninitialised";
     unsigned char* noalloc_ws[kMaxDevices] = {};   // device address of `scratch`, per device
@@ -102,6 +108,7 @@ int hip_fail(hipError_t e, const char* what, uint32_t layer);
         if (e_ != hipSuccess) return hip_fail(e_, what, layer);      \
     } while (0)
 
+hipError_t device_malloc(void** p, size_t bytes);
 int ensure_device(Buffer& b, size_t need);
 int ensure_pinned(Buffer& b, size_t need);
 int sync_checked(const char* what, uint32_t layer);

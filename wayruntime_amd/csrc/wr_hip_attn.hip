@@ -63,6 +63,7 @@ struct wr_hip_kv {
     size_t vt_off[WR_HIP_MAX_LAYERS];
     uint8_t* slab;
     size_t bytes;
+    int device;
 };
 
 // What a model's steps in one launch keep: the layers' weights as the kernel reads them, and the rows that travel
@@ -100,6 +101,78 @@ int hip_fail(hipError_t e, const char* what, uint32_t layer)
     return (e == hipErrorOutOfMemory) ? WR_HIP_ERR_NOMEM : WR_HIP_ERR_INTERNAL;
 }
 
+// Device memory of ended caches, for the next ones of their size: taking and giving back half a GiB is a third of a
+// millisecond a session, and thousands of sessions one after the other come to minutes in which the driver, which
+// clears what it is given back, takes 12 ms to each (a session of 10 tokens and one answer 2.1 -> 14.1 ms from some 250
+// sessions on, with calls 2.1 ms apart; 400 at 2.6).  Bounded, the longest kept goes first; given back with
+// the library, and when an allocation fails.
+constexpr size_t kKeptSlabs = 16, kKeptSlabBytes = (size_t)2 << 30;
+
+void slabs_free(std::vector<Lib::Slab>& slabs)
+{
+    for (const Lib::Slab& s : slabs) (void)hipFree(s.p);
+    slabs.clear();
+}
+
+// Everything kept: true if there was something.
+bool slabs_trim()
+{
+    std::vector<Lib::Slab> out;
+    {
+        std::lock_guard<std::mutex> lk(g.slab_mu);
+        out.swap(g.slabs);
+    }
+    const bool any = !out.empty();
+    slabs_free(out);
+    return any;
+}
+
+uint8_t* slab_take(size_t bytes)
+{
+    std::lock_guard<std::mutex> lk(g.slab_mu);
+    for (size_t i = 0; i < g.slabs.size(); i++)
+        if (g.slabs[i].bytes == bytes) {
+            uint8_t* p = g.slabs[i].p;
+            g.slabs.erase(g.slabs.begin() + (ptrdiff_t)i);
+            return p;
+        }
+    return nullptr;
+}
+
+// The slab of a cache that has ended, on the library's device.  As hipFree would, it waits for all of the device's streams.
+void slab_leave(uint8_t* p, size_t bytes)
+{
+    if (bytes > kKeptSlabBytes || hipDeviceSynchronize() != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(p);
+        return;
+    }
+    std::vector<Lib::Slab> out;
+    {
+        std::lock_guard<std::mutex> lk(g.slab_mu);
+        size_t kept = bytes;
+        for (const Lib::Slab& s : g.slabs) kept += s.bytes;
+        while (!g.slabs.empty() && (kept > kKeptSlabBytes || g.slabs.size() >= kKeptSlabs)) {
+            kept -= g.slabs.front().bytes;
+            out.push_back(g.slabs.front());
+            g.slabs.erase(g.slabs.begin());
+        }
+        g.slabs.push_back({p, bytes});
+    }
+    slabs_free(out);
+}
+
+// hipMalloc that what is kept makes room for.
+hipError_t device_malloc(void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && slabs_trim()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 int ensure_device(Buffer& b, size_t need)
 {
     if (need <= b.cap) return WR_HIP_OK;
@@ -108,7 +181,7 @@ int ensure_device(Buffer& b, size_t need)
     b.p = nullptr;
     b.cap = 0;
     const size_t want = need + need / 2 + 4096;
-    HIP_TRY(hipMalloc(&b.p, want), "workspace alloc", 0);
+    HIP_TRY(device_malloc(&b.p, want), "workspace alloc", 0);
     b.cap = want;
     return WR_HIP_OK;
 }
@@ -743,7 +816,7 @@ Ctx* ctx_create()
     if (rc == WR_HIP_OK) rc = ensure_device(c->d_stage, 2 * kPinSmall);
     if (rc == WR_HIP_OK) {
         const size_t cb = (size_t)WR_HIP_BATCH_MAX * kMaxHeads * sizeof(uint32_t);
-        e = hipMalloc((void**)&c->d_counters, cb);
+        e = device_malloc((void**)&c->d_counters, cb);
         if (e == hipSuccess) e = hipMemsetAsync(c->d_counters, 0, cb, c->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) rc = hip_fail(e, "ticket array", 0);
@@ -1312,6 +1385,11 @@ void wr_hip_attn_shutdown(void)
     g.ctxs.clear();
     g.idle.clear();
     cx = nullptr;
+    {
+        std::lock_guard<std::mutex> kept(g.slab_mu);
+        for (const Lib::Slab& s : g.slabs) (void)hipFree(s.p);
+        g.slabs.clear();
+    }
     if (g.noalloc_done) (void)hipEventDestroy(g.noalloc_done);
     g.noalloc_done = nullptr;
     g.inited = false;
@@ -1390,7 +1468,9 @@ int wr_hip_attn_kv_create(uint32_t n_layers, const uint32_t* hd_per_layer, uint3
     kv->bytes = cur;
 
     ENTER();
-    hipError_t e = hipMalloc((void**)&kv->slab, cur);
+    kv->device = g.device;
+    kv->slab = slab_take(cur);
+    hipError_t e = kv->slab ? hipSuccess : device_malloc((void**)&kv->slab, cur);
     if (e != hipSuccess) {
         logmsg(0, "session: device slab alloc failed (%zu bytes): %s", cur, hipGetErrorString(e));
         delete kv;
@@ -1413,7 +1493,8 @@ void wr_hip_attn_kv_destroy(wr_hip_kv* kv)
     if (g.inited) {
         Entered entered_;
         if (entered_.ok()) (void)hipStreamSynchronize(cx->stream);
-        if (kv->slab) (void)hipFree(kv->slab);     // (waits for the device's other streams by itself)
+        if (kv->slab && entered_.ok() && kv->device == g.device) slab_leave(kv->slab, kv->bytes);
+        else if (kv->slab) (void)hipFree(kv->slab);          // (waits for the device's other streams by itself)
     }
     delete kv;
 }
@@ -1761,8 +1842,8 @@ int wr_hip_attn_step_create(uint32_t n_layers, const wr_hip_attn_step_layer* lay
                             step_row_units((nq + 2 * nkv) * hd)) * 16 + step_part_bytes(nq);
     Entered entered_;
     int rc = entered_.ok() ? WR_HIP_OK : WR_HIP_ERR_NOMEM;
-    if (rc == WR_HIP_OK && (hipMalloc((void**)&p->layers, n_layers * sizeof(StepLayer)) != hipSuccess ||
-                            hipMalloc((void**)&p->rows, p->row_bytes) != hipSuccess))
+    if (rc == WR_HIP_OK && (device_malloc((void**)&p->layers, n_layers * sizeof(StepLayer)) != hipSuccess ||
+                            device_malloc((void**)&p->rows, p->row_bytes) != hipSuccess))
         rc = WR_HIP_ERR_NOMEM;
     if (rc == WR_HIP_OK) {
         hipError_t e = hipMemcpyAsync(p->layers, host, n_layers * sizeof(StepLayer), hipMemcpyHostToDevice, cx->stream);
@@ -2073,7 +2154,7 @@ void* wr_hip_attn_dev_alloc(size_t bytes)
     Entered entered_;
     if (!entered_.ok()) return nullptr;
     void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
+    if (device_malloc(&p, bytes) != hipSuccess) return nullptr;
     return p;
 }
 
@@ -2181,8 +2262,8 @@ int wr_hip_proj_weight_create(uint32_t n_parts, const uint16_t* const* parts_f16
 
     ENTER();
     void* rowmajor = nullptr;
-    hipError_t e = hipMalloc(&w->tiles, w->bytes);
-    if (e == hipSuccess) e = hipMalloc(&rowmajor, w->bytes);
+    hipError_t e = device_malloc((void**)&w->tiles, w->bytes);
+    if (e == hipSuccess) e = device_malloc((void**)&rowmajor, w->bytes);
     if (e != hipSuccess) {
         logmsg(0, "projection: device weight alloc failed (%zu bytes): %s", w->bytes,
                hipGetErrorString(e));

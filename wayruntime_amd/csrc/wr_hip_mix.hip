@@ -106,8 +106,8 @@ int wr_hip_mix_mat_create(uint32_t batch, uint32_t n_out, uint32_t n_in, const u
     }
     const size_t bytes = (size_t)batch * n_out * n_in * 2;
     void* rows = nullptr;
-    hipError_t e = hipMalloc(&w->tiles, bytes);
-    if (e == hipSuccess) e = hipMalloc(&rows, bytes);
+    hipError_t e = device_malloc((void**)&w->tiles, bytes);
+    if (e == hipSuccess) e = device_malloc((void**)&rows, bytes);
     if (e == hipSuccess) e = hipMemcpyAsync(rows, bf16, bytes, hipMemcpyHostToDevice, cx->stream);
     if (e == hipSuccess) {
         const uint64_t units = bytes / 16;
@@ -164,7 +164,7 @@ int wr_hip_mix_pool_create(int f32, uint32_t n_latent, const uint32_t* latent_di
     }
     p->bytes = at ? at : 256;
     Entered entered_;
-    hipError_t e = entered_.ok() ? hipMalloc((void**)&p->block, p->bytes) : hipErrorOutOfMemory;
+    hipError_t e = entered_.ok() ? device_malloc((void**)&p->block, p->bytes) : hipErrorOutOfMemory;
     if (e == hipSuccess) e = hipMemsetAsync(p->block, 0, p->bytes, cx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(cx->stream);
     if (e != hipSuccess) {
