@@ -91,7 +91,8 @@ const char *wr_hip_attn_device_name(void);
  * storage (KV-shared layers alias another layer, session.c:652-658; pass the
  * source layer's index to the other calls).  Allocation failure is
  * WR_HIP_ERR_NOMEM; max_ctx above the cap is WR_HIP_ERR_LIMIT
- * (session.c:755). */
+ * (session.c:755).  The device memory of destroyed caches is kept for later ones of
+ * its size, 2 GiB at most (of sixteen), until shutdown or until an allocation fails. */
 int  wr_hip_attn_kv_create(uint32_t n_layers, const uint32_t *hd_per_layer,
                            uint32_t nkv, uint32_t max_ctx, wr_hip_kv **out);
 void wr_hip_attn_kv_destroy(wr_hip_kv *kv);
