@@ -667,7 +667,7 @@ bool prefill_parts_ready(PrefillArgs& a, uint32_t parts)
         size_t want = (size_t)1 << 20;
         while (want < need) want *= 2;
         void* bigger = nullptr;
-        if (hipMalloc(&bigger, want) != hipSuccess) {
+        if (device_malloc(&bigger, want) != hipSuccess) {
             (void)hipGetLastError();
             logmsg(1, "prefill: no %zu MiB for parts of long blocks; they go uncut", want >> 20);
             cx->prefill_refused = kPrefillRefusedLaunches;
