@@ -37,6 +37,17 @@ static int late_error(void)
     return WR_HIP_OK;
 }
 
+/* Test hook: called at the start of every wr_hip_attn_kv_destroy (which waits for the whole device there). */
+static void (*g_on_kv_destroy)(void);
+void wr_hip_attn_debug_on_kv_destroy(void (*fn)(void));
+void wr_hip_attn_debug_on_kv_destroy(void (*fn)(void)) { g_on_kv_destroy = fn; }
+
+/* Test hook: the capabilities the library reports.  With projections among them weights can be made
+ * (empty ones) and a model is set up for the device walk; nothing can be run on it. */
+static uint32_t g_caps;
+void wr_hip_attn_debug_caps(uint32_t caps);
+void wr_hip_attn_debug_caps(uint32_t caps) { g_caps = caps; }
+
 int wr_hip_attn_init(int device)
 {
     (void)device;
@@ -83,6 +94,7 @@ int wr_hip_attn_kv_create(uint32_t n_layers, const uint32_t *hd, uint32_t nkv, u
 
 void wr_hip_attn_kv_destroy(wr_hip_kv *kv)
 {
+    if (g_on_kv_destroy) g_on_kv_destroy();
     if (!kv) return;
     for (uint32_t L = 0; L < kv->n_layers; L++) {
         free(kv->k[L]);
@@ -268,8 +280,9 @@ int wr_hip_attn_prefill(wr_hip_kv *kv, uint32_t layer, uint32_t p0, uint32_t T, 
 
 /* ---- not offered by the test double -----------------------------------------
  * The host engine asks wr_hip_attn_caps() before it uses any of these and keeps
- * its own CPU walk when the answer is 0; they exist so the engine links. */
-uint32_t wr_hip_attn_caps(void) { return 0; }
+ * its own CPU walk when the answer is 0 (as it is unless a test says otherwise);
+ * they exist so the engine links. */
+uint32_t wr_hip_attn_caps(void) { return g_caps; }
 void wr_hip_attn_set_tuning(uint32_t keys_per_wg, int force_generic) { (void)keys_per_wg; (void)force_generic; }
 void wr_hip_attn_set_prefill_one_wave(int on) { (void)on; }
 void wr_hip_attn_set_prefill_part_mb(uint32_t mb) { (void)mb; }
@@ -336,9 +349,11 @@ int wr_hip_proj_weight_create(uint32_t n_parts, const uint16_t *const *parts, co
 {
     (void)n_parts; (void)parts; (void)rows; (void)n_in;
     if (out) *out = NULL;
-    return WR_HIP_ERR_STATE;
+    if (!(g_caps & WR_HIP_CAP_PROJ)) return WR_HIP_ERR_STATE;
+    *out = malloc(1);
+    return *out ? WR_HIP_OK : WR_HIP_ERR_NOMEM;
 }
-void wr_hip_proj_weight_destroy(wr_hip_weight *w) { (void)w; }
+void wr_hip_proj_weight_destroy(wr_hip_weight *w) { free(w); }
 int wr_hip_proj_rows_dev(const wr_hip_weight *w, uint32_t rows, const float *x, uint32_t ldx,
                          const float *add, float *y, uint32_t ldy)
 {
@@ -435,8 +450,9 @@ int wr_hip_proj_embed_dev(const wr_hip_weight *w, uint32_t rows, const uint32_t 
 int wr_hip_attn_step_create(uint32_t n_layers, const wr_hip_attn_step_layer *layers, uint32_t nq, uint32_t nkv, uint32_t hd,
                             float eps, wr_hip_attn_step **out)
 {
-    (void)n_layers; (void)layers; (void)nq; (void)nkv; (void)hd; (void)eps; (void)out;
-    return WR_HIP_ERR_STATE;
+    (void)n_layers; (void)layers; (void)nq; (void)nkv; (void)hd; (void)eps;
+    *out = NULL;
+    return WR_HIP_ERR_UNSUPPORTED;
 }
 void wr_hip_attn_step_destroy(wr_hip_attn_step *step) { (void)step; }
 int wr_hip_attn_step_dev(wr_hip_attn_step *step, wr_hip_kv *kv, uint32_t pos, float *row, const float *cs, uint32_t n_rot,

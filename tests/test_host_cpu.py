@@ -11,9 +11,10 @@ import numpy as np
 import pytest
 
 import oracle
-from tests.golden.make_e2e_golden import TINY, workload
+from tests.golden.make_e2e_golden import SMALL16, TINY, workload
 from wayruntime_amd import engine as E, gguf_writer as gw
 
+CAP_PROJ = 1
 GOLD = os.path.join(os.path.dirname(__file__), "golden")
 
 
@@ -316,4 +317,33 @@ def test_gemma_batched_equals_serial_and_rolls_back(eng, gemma_path):
     assert rc == n and all(lb[i].tobytes() == ls[i].tobytes() for i in range(n))
     for s in batch + serial:
         s.close()
+    m.close()
+
+
+@pytest.mark.parametrize("walk", ["host", "device"])
+def test_a_model_outlives_the_end_of_its_last_session(eng, tmp_path, capfd, walk):
+    # The end of a session waits for the device and then hands things back to its model: until that is done
+    # the model is not another thread's to free.  The call comes from within the session's end here.
+    p = str(tmp_path / "m.gguf")
+    gw.write_model(p, SMALL16)
+    lib, hook_t = eng.lib, C.CFUNCTYPE(None)
+    lib.wr_hip_attn_debug_caps(CAP_PROJ if walk == "device" else 0)
+    try:
+        m = eng.load(p)
+    finally:
+        lib.wr_hip_attn_debug_caps(0)
+    s, seen = m.session(), []
+
+    def on_destroy():
+        lib.wr_model_free(m.h)
+        seen.append(capfd.readouterr().err)
+
+    hook = hook_t(on_destroy)
+    lib.wr_hip_attn_debug_on_kv_destroy(hook)
+    try:
+        s.close()
+    finally:
+        lib.wr_hip_attn_debug_on_kv_destroy(hook_t())
+    assert len(seen) == 1 and "1 session(s) still alive; refused" in seen[0]
+    m.session().close()                                        # the model is whole
     m.close()

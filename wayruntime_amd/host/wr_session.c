@@ -412,9 +412,6 @@ void wr_session_destroy(wr_session *s)
 {
     if (!s) return;
     wr_model *m = s->model;
-    pthread_mutex_lock(&m->lock);
-    if (m->session_refs) m->session_refs--;
-    pthread_mutex_unlock(&m->lock);
     if (s->mix) wrh_mix_session_destroy(s);
     wr_hip_attn_kv_destroy(s->kv);
     wrh_workspace_free(&s->ws1);
@@ -422,6 +419,10 @@ void wr_session_destroy(wr_session *s)
     free_logits(s);
     pthread_mutex_destroy(&s->lock);
     free(s);
+    /* last: from here on another thread may free the model */
+    pthread_mutex_lock(&m->lock);
+    if (m->session_refs) m->session_refs--;
+    pthread_mutex_unlock(&m->lock);
 }
 
 uint32_t wr_session_pos(const wr_session *s)
