@@ -438,12 +438,6 @@ static int launch_split(const MixGemmArgs& a, uint32_t batch)
 
 constexpr size_t kMaxPickedBytes = 64u << 20;
 
-// Runs of eight groups as a stream of their experts' weights.  A run's workgroups go to one XCD each run where that
-// leaves none more than a seventh without work (its rows then come into one L2 and not into eight, which is 8 rows / outputs
-// of the weights' bytes): up to 1536 outputs.  34 rows an expert, dealt out / by XCD (us): 64 experts, 4096 -> 384 64 / 43, -> 512 75
-// / 56, 2048 -> 1024 57 / 53; 128 experts, 2048 -> 768 86 / 79; 16 experts, 4096 -> 1536 46.5 / 40.6.  With more
-// outputs it is no gain (64 experts, 1024 -> 2048 58 / 59) or a loss (32 experts, 4096 -> 4096 199 / 209, 64, 384 ->
-// 4096 65 / 72: eight experts' weights and results at the same offsets).
 // Rows picked one by one, brought into the order of their slots first, when there is a place for them.
 static void pick_rows(MixGemmArgs& a)
 {
@@ -463,6 +457,12 @@ static void pick_rows(MixGemmArgs& a)
     a.x_perm = nullptr;
 }
 
+// Runs of eight groups as a stream of their experts' weights.  A run's workgroups go to one XCD each run where that
+// leaves none more than a seventh without work (its rows then come into one L2 and not into eight, which is 8 rows / outputs
+// of the weights' bytes): up to 1536 outputs.  34 rows an expert, dealt out / by XCD (us): 64 experts, 4096 -> 384 64 / 43, -> 512 75
+// / 56, 2048 -> 1024 57 / 53; 128 experts, 2048 -> 768 86 / 79; 16 experts, 4096 -> 1536 46.5 / 40.6.  With more
+// outputs it is no gain (64 experts, 1024 -> 2048 58 / 59) or a loss (32 experts, 4096 -> 4096 199 / 209, 64, 384 ->
+// 4096 65 / 72: eight experts' weights and results at the same offsets).
 static bool runs_by_xcd(const MixGemmArgs& a, uint32_t experts)
 {
     return a.ntiles <= 96 && (uint64_t)((experts + 7) / 8 * 8) * 7 <= (uint64_t)experts * 8;
