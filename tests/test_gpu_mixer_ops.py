@@ -358,6 +358,49 @@ def test_groups_of_an_expert_that_stand_together(lib, N, K):
         b.free()
 
 
+def test_picked_rows_of_a_recorded_product(lib):
+    # A recorded product picks its rows by itself: it is one launch, none of the thread's own memory is in
+    # the graph, and replays hold after a larger call has made that memory anew.
+    experts, N, K = 2, 64, 64
+    r = Run(lib, False, experts, N, K, 0)
+
+    def inputs(groups):
+        which = np.repeat(np.arange(experts), groups // experts).astype(np.int32)
+        few = r.act(33, K)
+        pick = r.rng.integers(0, 33, 16 * groups).astype(np.uint32)
+        want = np.concatenate([few[pick[16 * g:16 * g + 16]].astype(np.float64) @ r.w[e].T.astype(np.float64) for g, e in enumerate(which)])
+        y = hipattn.DeviceBuffer(16 * groups * N * 4)
+        bufs = r.up(few), hipattn.DeviceBuffer.from_host(which.view(np.float32)), hipattn.DeviceBuffer.from_host(pick.view(np.float32)), y
+        return bufs, Gemm(w=r.h, x=bufs[0].p, x_kt=K // 32, rows=16 * groups, group_expert=bufs[1].p, tile_groups=1, out=ROWS_F32,
+                          y_f32=y.p, ldy=N, x_perm=bufs[2].p), want
+
+    small, g, want = inputs(128)
+    large, g2, want2 = inputs(4096)
+    for _ in range(2):                                       # there is room for its rows from here on
+        assert lib.wr_hip_mix_gemm_run(0, C.byref(g)) == 0
+    hipattn.sync()
+    eager = small[3].to_host((2048, N)).copy()
+    r.close(eager, want)
+    stream, graph, run, n = vp(lib.wr_hip_attn_stream()), vp(), vp(), C.c_size_t()
+    assert lib.hipStreamBeginCapture(stream, 2) == 0         # relaxed
+    rc = lib.wr_hip_mix_gemm_run(0, C.byref(g))
+    assert lib.hipStreamEndCapture(stream, C.byref(graph)) == 0 and rc == 0
+    assert lib.hipGraphGetNodes(graph, None, C.byref(n)) == 0 and n.value == 1
+    assert lib.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for _ in range(3):
+        assert lib.wr_hip_mix_gemm_run(0, C.byref(g2)) == 0
+        hipattn.sync()
+        r.close(large[3].to_host((65536, N)), want2)
+        lib.wr_hip_attn_h2d(small[3].p, np.zeros((2048, N), np.float32).ctypes.data, eager.nbytes)
+        assert lib.hipGraphLaunch(run, stream) == 0
+        hipattn.sync()
+        assert small[3].to_host((2048, N)).tobytes() == eager.tobytes()
+    assert lib.hipGraphExecDestroy(run) == 0 and lib.hipGraphDestroy(graph) == 0
+    r.end()
+    for b in small + large:
+        b.free()
+
+
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("N,K,tile", [(64, 96, 1), (48, 64, 8), (4096, 64, 8), (1024, 32, 1)])
 def test_matrix_per_row_group(lib, f32, N, K, tile):

@@ -438,18 +438,17 @@ static int launch_split(const MixGemmArgs& a, uint32_t batch)
 
 constexpr size_t kMaxPickedBytes = 64u << 20;
 
-// Rows picked one by one, brought into the order of their slots first, when there is a place for them.
+// Rows picked one by one, brought into the order of their slots first, when there is a place for them.  Not while a
+// launch is recorded: the place is this thread's and gives way to a larger one, and a graph would keep its address.
 static void pick_rows(MixGemmArgs& a)
 {
     const size_t bytes = (size_t)a.groups * a.ktiles * 1024;
     if (a.x_kt != a.ktiles || bytes > kMaxPickedBytes) return;
-    if (bytes > cx->d_picked.cap) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;     // (no allocation while a graph is recorded)
-        if (hipStreamIsCapturing(cx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
-            ensure_device(cx->d_picked, bytes) != WR_HIP_OK) {
-            (void)hipGetLastError();
-            return;
-        }
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(cx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
+        ensure_device(cx->d_picked, bytes) != WR_HIP_OK) {
+        (void)hipGetLastError();
+        return;
     }
     hipLaunchKernelGGL(mix_gather_kernel<false>, dim3((a.ktiles * 64 + 255) / 256, a.groups), dim3(256), 0, cx->stream, a.x, a.ktiles,
                        a.groups, a.x_perm, a.group_expert, cx->d_picked.p);
