@@ -28,6 +28,7 @@
 #include "kernels_proj.hip.h"
 #include "kernels_rows.hip.h"
 #include "kernels_step.hip.h"
+#include "step_gate.h"
 
 using namespace wr;
 
@@ -1899,10 +1900,7 @@ int wr_hip_attn_step_dev(wr_hip_attn_step* p, wr_hip_kv* kv, uint32_t pos, float
         (void)hipGetLastError();
         return WR_HIP_ERR_UNSUPPORTED;
     }
-    if (g.step_refused.load(std::memory_order_relaxed) > 0) {
-        g.step_refused.fetch_sub(1, std::memory_order_relaxed);
-        return WR_HIP_ERR_UNSUPPORTED;
-    }
+    if (count_down(g.step_refused)) return WR_HIP_ERR_UNSUPPORTED;
     // Two launches whose workgroups wait for each other could each hold CUs the other needs: one at a time.
     Ctx* nobody = nullptr;
     if (!g.step_owner.compare_exchange_strong(nobody, cx, std::memory_order_acq_rel) && nobody != cx) return WR_HIP_ERR_UNSUPPORTED;
