@@ -502,8 +502,9 @@ int wr_hip_rows_swiglu_dev(const float *gate_up_dev, uint32_t ld, float *act_dev
  * wr_hip_attn_append_decode_batched_dev, wr_hip_proj_rows_dev and
  * wr_hip_proj_rows_gated_dev layer by layer.  cos_sin_dev [n_rot][2].  WR_HIP_ERR_UNSUPPORTED, with
  * nothing launched: the caller goes layer by layer (generic kernels forced, another alignment, a
- * stream that records, a session cut into more than 16 key splits, or another thread's step on the
- * device: the launch's workgroups wait for each other, so one of them runs at a time).
+ * stream that records, a session cut into more than 16 key splits, another thread's step on the
+ * device: the launch's workgroups wait for each other, so one of them runs at a time; or another thread
+ * in a call, unless its last product had 2 to WR_HIP_BATCH_MAX rows: the launch takes the whole device).
  *
  * step_done: every step_dev is followed by one on the same thread, after whatever was
  * enqueued behind it.  Waits for the thread's stream; WR_HIP_ERR_STATE: a workgroup

@@ -2,6 +2,7 @@
 chain of launches it stands for: same logits, bit for bit, and the same cache behind them."""
 import ctypes as C
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -82,13 +83,14 @@ def _steps(model, prompt, tokens):
     return rows
 
 
-def _launches(model):
+def _launches(model, session=None):
     lib, ms, n = hipattn.lib(), C.c_double(), C.c_uint32()
-    s = model.session()
+    s = session or model.session()
     assert lib.wr_hip_attn_profile_begin(1000) == hipattn.OK
     s.step(1)
     assert lib.wr_hip_attn_profile_end(C.byref(ms), C.byref(n)) == hipattn.OK
-    s.close()
+    if not session:
+        s.close()
     return n.value
 
 
@@ -152,5 +154,45 @@ def test_threads_step_beside_each_other(eng, tmp_path, monkeypatch):
         t.join()
     for g, w in zip(got, want):
         assert g is not None and all(np.array_equal(a, b) for a, b in zip(g, w))
+    for m in (one, chain):
+        m.close()
+
+
+@pytest.mark.parametrize("rows", [1, 8, 64])
+def test_a_step_beside_another_threads_work(eng, tmp_path, monkeypatch, rows):
+    """One launch would keep another thread's chain of launches or its prompt waiting for as long as it runs: the step
+    goes layer by layer then.  Beside a batched step's products, which fill the device too, it does not."""
+    one, chain = _models(eng, tmp_path, monkeypatch, n_layers=2, hidden=1024, ffn=3072, n_q=16, n_kv=8)
+    lib = hipattn.lib()
+    monkeypatch.setattr(hipattn, "_inited", True)            # by the engine
+    T, nq, hd = 8192, 32, 128
+    kv, w = hipattn.KVCache(1, hd, 8, T), hipattn.Weight([np.zeros((64, 64), np.uint16)])
+    q, out, x, y = (hipattn.DeviceBuffer(n * 4) for n in (T * nq * hd, T * nq * hd, 64 * 64, 64 * 64))
+    waiting, done = threading.Event(), threading.Event()
+
+    def other():
+        for _ in range(150):                                 # some 150 ms of it
+            assert lib.wr_hip_attn_prefill_dev(kv.h, 0, 0, T, q.p, out.p, nq, 0.0, 0) == hipattn.OK
+        assert lib.wr_hip_proj_rows_dev(w.h, rows, x.p, 64, None, y.p, 64) == hipattn.OK
+        waiting.set()
+        hipattn.sync()
+        done.set()
+
+    s = one.session()                                        # (making one and ending it waits for the whole device)
+    _launches(one, s)                                        # (a first call on every path)
+    t = threading.Thread(target=other)
+    t.start()
+    assert waiting.wait(60)
+    time.sleep(0.002)
+    beside = _launches(one, s)
+    assert not done.is_set()                                 # it was under way all the time
+    t.join()
+    assert beside == (2 if rows == 8 else 11)
+    assert _launches(one, s) == 2
+    s.close()
+    for o in (kv, w):
+        o.close()
+    for b in (q, out, x, y):
+        b.free()
     for m in (one, chain):
         m.close()

@@ -46,6 +46,9 @@ struct Ctx {
     // read by wr_hip_attn_step_done, after which the step is made another way.
     volatile uint32_t* err_host = nullptr;
     uint32_t* err_dev = nullptr;
+    // Read by other threads, to see whose work runs beside theirs: how deep the thread is in calls that touch the device
+    // (one may make another), and how many rows its last product had.
+    std::atomic<uint32_t> depth{0}, rows{0};
     uint32_t step_calls = 0;          // attention calls that the last step in one launch counted
     Buffer h_pin;                // pinned host staging
     std::vector<hipEvent_t> ev;  // kernel timing (profile_begin / profile_end of this thread)
@@ -147,6 +150,12 @@ void launch_main(Kern kernel, dim3 grid, dim3 block, const Args& args, size_t ld
 struct Entered {
     bool good = false;
     Entered();
+    ~Entered()
+    {
+        if (good) cx->depth.store(cx->depth.load(std::memory_order_relaxed) - 1, std::memory_order_relaxed);
+    }
+    Entered(const Entered&) = delete;
+    Entered& operator=(const Entered&) = delete;
     bool ok() const { return good; }
 };
 

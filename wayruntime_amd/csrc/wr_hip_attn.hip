@@ -875,6 +875,7 @@ Entered::Entered()
             g.idle.pop_back();
             c->profiling = false;            // the thread that had it before may have ended mid-measurement
             c->ev_used = 0;
+            c->rows = 0;
         } else {
             c = ctx_create();
             if (c) g.ctxs.push_back(c);
@@ -884,6 +885,7 @@ Entered::Entered()
     }
     cx = t_slot.c;
     good = cx != nullptr;
+    if (good) cx->depth.store(cx->depth.load(std::memory_order_relaxed) + 1, std::memory_order_relaxed);
 }
 
 }  // namespace wr
@@ -1102,6 +1104,7 @@ int proj_chunk_locked(const wr_hip_weight* w, uint32_t rows, const float* x_dev,
                       const ProjSource& src, const float* add_dev, float* y_dev, uint32_t ldy,
                       const ProjDownArgs* down = nullptr)
 {
+    cx->rows.store(rows, std::memory_order_relaxed);
     const uint32_t groups = (rows + 7) / 8;                // row groups of eight
     const bool gemm = rows >= (uint32_t)kProjGemmMinRows;
     const uint32_t ktiles = w->n_in / 32;
@@ -1799,6 +1802,23 @@ bool step_product_ok(const wr_hip_weight* w, uint32_t n_in, uint32_t n_out, bool
            tiles / (gated ? 2 : 1) <= g.n_cus;
 }
 
+// Whether another thread's work is under way that a step in one launch would keep waiting.  The launch holds
+// every compute unit for its half millisecond, where a chain of small launches shares the device with other chains and
+// with a prompt's launches.  28 layers, hidden 1024, threads that step a session of their own, us of all of them
+// together per step, one launch at a time among them / chains: 2 threads 564 / 504, 3 560 / 380, 4 420 to 540 / 481, 5 474 /
+// 415, 6 446 / 376 (8 375 / 397, 12 352 / 374).  A step beside prompts of 1024 tokens 1200 / 3100, the prompt 9000 /
+// 6270; chains were all there was before, at 2700 and 6900.  Products of 2 to 16 rows fill the device as well and
+// chains gain nothing beside them (steps beside steps of eight sessions, either 1560 / 1835): those do not count.
+bool step_beside_others()
+{
+    std::lock_guard<std::mutex> lk(g.mu);
+    for (const Ctx* c : g.ctxs) {
+        const uint32_t rows = c->rows.load(std::memory_order_relaxed);
+        if (c != cx && c->depth.load(std::memory_order_relaxed) && (rows < 2 || rows > WR_HIP_BATCH_MAX)) return true;
+    }
+    return false;
+}
+
 size_t step_part_bytes(uint32_t nq) { return (size_t)nq * kMergeInRegs * (128 + 2) * sizeof(uint64_t); }
 
 }  // namespace
@@ -1900,7 +1920,7 @@ int wr_hip_attn_step_dev(wr_hip_attn_step* p, wr_hip_kv* kv, uint32_t pos, float
         (void)hipGetLastError();
         return WR_HIP_ERR_UNSUPPORTED;
     }
-    if (count_down(g.step_refused)) return WR_HIP_ERR_UNSUPPORTED;
+    if (count_down(g.step_refused) || step_beside_others()) return WR_HIP_ERR_UNSUPPORTED;
     // Two launches whose workgroups wait for each other could each hold CUs the other needs: one at a time.
     Ctx* nobody = nullptr;
     if (!g.step_owner.compare_exchange_strong(nobody, cx, std::memory_order_acq_rel) && nobody != cx) return WR_HIP_ERR_UNSUPPORTED;

@@ -597,6 +597,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     if (q->x_scale && !q->group_expert) return WR_HIP_ERR_INVAL;
     if (q->x_perm && (!q->group_expert || q->tile_groups != 1)) return WR_HIP_ERR_INVAL;
     ENTER();
+    cx->rows.store(q->rows, std::memory_order_relaxed);
     MixGemmArgs a = {};
     a.w = reinterpret_cast<const bf16x8*>(q->w->tiles);
     a.x = static_cast<const uint8_t*>(q->x) + (size_t)q->x_kt0 * 512 * (f32 ? 4 : 2);
