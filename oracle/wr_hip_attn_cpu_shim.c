@@ -47,6 +47,10 @@ void wr_hip_attn_debug_on_kv_destroy(void (*fn)(void)) { g_on_kv_destroy = fn; }
 static uint32_t g_caps;
 void wr_hip_attn_debug_caps(uint32_t caps);
 void wr_hip_attn_debug_caps(uint32_t caps) { g_caps = caps; }
+/* Test hook: the k-th weight from now finds no memory. */
+static int g_refuse_weight_in;
+void wr_hip_attn_debug_refuse_weight_in(int k);
+void wr_hip_attn_debug_refuse_weight_in(int k) { g_refuse_weight_in = k; }
 
 int wr_hip_attn_init(int device)
 {
@@ -350,6 +354,7 @@ int wr_hip_proj_weight_create(uint32_t n_parts, const uint16_t *const *parts, co
     (void)n_parts; (void)parts; (void)rows; (void)n_in;
     if (out) *out = NULL;
     if (!(g_caps & WR_HIP_CAP_PROJ)) return WR_HIP_ERR_STATE;
+    if (g_refuse_weight_in > 0 && --g_refuse_weight_in == 0) return WR_HIP_ERR_NOMEM;
     *out = malloc(1);
     return *out ? WR_HIP_OK : WR_HIP_ERR_NOMEM;
 }

@@ -4,6 +4,7 @@ library).  Covers what needs no GPU: the GGUF loader, the greedy token stream of
 a toy model against the compiled reference's golden stream, context limits,
 all-or-nothing rollback, batched == serial, and the error contract."""
 import ctypes as C
+import dataclasses
 import os
 import struct
 
@@ -347,3 +348,24 @@ def test_a_model_outlives_the_end_of_its_last_session(eng, tmp_path, capfd, walk
     assert len(seen) == 1 and "1 session(s) still alive; refused" in seen[0]
     m.session().close()                                        # the model is whole
     m.close()
+
+
+def test_a_model_loads_without_device_memory_for_an_embedding_of_its_own(eng, tmp_path, capfd):
+    # The host has the table: only the head's weight and the layers' have to be on the device.
+    p = str(tmp_path / "m.gguf")
+    gw.write_model(p, dataclasses.replace(SMALL16, tied_head=False))
+    lib = eng.lib
+    lib.wr_hip_attn_debug_caps(CAP_PROJ)
+    try:
+        for k, says in ((0, "layers and the LM head are on the device"), (4 * SMALL16.n_layers + 2, "no device memory for the embedding")):
+            lib.wr_hip_attn_debug_refuse_weight_in(k)
+            m = eng.load(p)
+            assert says in capfd.readouterr().err
+            m.close()
+        lib.wr_hip_attn_debug_refuse_weight_in(4 * SMALL16.n_layers + 1)         # the head: it cannot do without
+        with pytest.raises(E.EngineError) as err:
+            eng.load(p)
+        assert err.value.rc == E.WR_ERR_NOMEM
+    finally:
+        lib.wr_hip_attn_debug_refuse_weight_in(0)
+        lib.wr_hip_attn_debug_caps(0)

@@ -171,6 +171,7 @@ hipError_t device_malloc(void** p, size_t bytes)
         (void)hipGetLastError();
         e = hipMalloc(p, bytes);
     }
+    if (e != hipSuccess) (void)hipGetLastError();          // (the caller may do without: not for the next launch's check to find)
     return e;
 }
 

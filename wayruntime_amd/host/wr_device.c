@@ -7,7 +7,8 @@
  * host walk, WAYRT_STEP_LAUNCHES=1 keeps a session's decode step a chain of
  * launches where one could take its layers, WAYRT_STEP_TWO_LAUNCHES=1 keeps a
  * decode step's row step and its attention as two of them.  Per call the rows are
- * embedded on the device (by the host, and sent up, where the table is not F16); the
+ * embedded on the device (by the host, and sent up, where the table is not F16 or there was no
+ * memory for one that the head does not share); the
  * rotary angles of their positions are made on the device (the reference's
  * polynomial sin / cos and range reduction restated there bit for bit:
  * wr_hip_attn_rope_table_dev); the layers run without coming back, and the
@@ -36,7 +37,8 @@ typedef struct dev_layer {
 struct wrh_dev_model {
     dev_layer     L[WRH_MAX_LAYERS];
     wr_hip_weight *lm_head;
-    wr_hip_weight *embed;                                      /* lm_head where it is tied, NULL: rows are embedded on the host */
+    wr_hip_weight *embed;                                      /* lm_head where it is tied; NULL (no F16 table, no memory for one of
+                                                                * its own): rows are embedded on the host */
     float         *vecs;                                       /* one device block for all norm vectors */
     const float   *final_norm;
     /* decode steps: does the library take the row step (split, norms, rotation,
@@ -173,7 +175,14 @@ wr_status wrh_device_model_init(wr_model *m)
     }
     if (rc == WR_HIP_OK) rc = stack(&d->lm_head, &m->lm_head, NULL, NULL);
     if (rc == WR_HIP_OK && m->embed.data == m->lm_head.data) d->embed = d->lm_head;
-    else if (rc == WR_HIP_OK && proj_dims_ok(&m->embed)) rc = stack(&d->embed, &m->embed, NULL, NULL);
+    else if (rc == WR_HIP_OK && proj_dims_ok(&m->embed)) {
+        rc = stack(&d->embed, &m->embed, NULL, NULL);
+        if (rc == WR_HIP_ERR_NOMEM) {                          /* the host has the table as well */
+            wrh_logf(m->engine, 1, "device layers: no device memory for the embedding; its rows are made on the host");
+            d->embed = NULL;
+            rc = WR_HIP_OK;
+        }
+    }
     if (rc == WR_HIP_OK) rc = step_plan(m, d);
     /* the uploads ran on this thread's stream; sessions may step on others */
     if (rc == WR_HIP_OK) rc = wr_hip_attn_sync();
