@@ -52,6 +52,11 @@ static int g_refuse_weight_in;
 void wr_hip_attn_debug_refuse_weight_in(int k);
 void wr_hip_attn_debug_refuse_weight_in(int k) { g_refuse_weight_in = k; }
 
+/* Test hook: what making the plan of a step in one launch comes to. */
+static int g_step_plan = WR_HIP_ERR_UNSUPPORTED;
+void wr_hip_attn_debug_step_plan(int rc);
+void wr_hip_attn_debug_step_plan(int rc) { g_step_plan = rc; }
+
 int wr_hip_attn_init(int device)
 {
     (void)device;
@@ -457,7 +462,7 @@ int wr_hip_attn_step_create(uint32_t n_layers, const wr_hip_attn_step_layer *lay
 {
     (void)n_layers; (void)layers; (void)nq; (void)nkv; (void)hd; (void)eps;
     *out = NULL;
-    return WR_HIP_ERR_UNSUPPORTED;
+    return g_step_plan;
 }
 void wr_hip_attn_step_destroy(wr_hip_attn_step *step) { (void)step; }
 int wr_hip_attn_step_dev(wr_hip_attn_step *step, wr_hip_kv *kv, uint32_t pos, float *row, const float *cs, uint32_t n_rot,

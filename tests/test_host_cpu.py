@@ -369,3 +369,21 @@ def test_a_model_loads_without_device_memory_for_an_embedding_of_its_own(eng, tm
     finally:
         lib.wr_hip_attn_debug_refuse_weight_in(0)
         lib.wr_hip_attn_debug_caps(0)
+
+
+@pytest.mark.parametrize("rc,loads", [(E.WR_ERR_UNSUPPORTED, True), (E.WR_ERR_NOMEM, True), (E.WR_ERR_INTERNAL, False)])
+def test_a_model_loads_without_a_plan_for_steps_in_one_launch(eng, tmp_path, rc, loads):
+    p = str(tmp_path / "m.gguf")
+    gw.write_model(p, SMALL16)
+    lib = eng.lib
+    lib.wr_hip_attn_debug_caps(CAP_PROJ)
+    lib.wr_hip_attn_debug_step_plan(rc)
+    try:
+        if loads:
+            eng.load(p).close()
+        else:
+            with pytest.raises(E.EngineError):
+                eng.load(p)
+    finally:
+        lib.wr_hip_attn_debug_step_plan(E.WR_ERR_UNSUPPORTED)
+        lib.wr_hip_attn_debug_caps(0)

@@ -95,7 +95,8 @@ static int step_plan(const wr_model *m, struct wrh_dev_model *d)
     }
     if (!ok) return WR_HIP_OK;
     const int rc = wr_hip_attn_step_create(m->n_layers, y, m->n_q, m->n_kv, m->head_dim, m->rms_eps, &d->step);
-    return rc == WR_HIP_ERR_UNSUPPORTED ? WR_HIP_OK : rc;
+    if (rc == WR_HIP_ERR_NOMEM) wrh_logf(m->engine, 1, "device layers: no device memory for a step's rows; it goes layer by layer");
+    return rc == WR_HIP_ERR_UNSUPPORTED || rc == WR_HIP_ERR_NOMEM ? WR_HIP_OK : rc;
 }
 
 /* WR_OK with m->dev set, WR_OK with m->dev NULL when the model stays on the
