@@ -526,6 +526,9 @@ int  wr_hip_attn_step_dev(wr_hip_attn_step *step, wr_hip_kv *kv, uint32_t pos, f
 int  wr_hip_attn_step_done(void);
 void wr_hip_attn_set_step_limit(uint32_t ticks);
 
+/* For tests: of the allocations of device memory from now on `after` are made and then `n` fail (0: none does). */
+void wr_hip_attn_set_alloc_failures(uint32_t n, uint32_t after);
+
 /* Tuning knobs for measurement (0 = automatic): keys handled per workgroup in
  * the split-K decode kernel, and a switch forcing the generic (non-MFMA)
  * kernels.  Not needed by a normal caller. */

@@ -401,6 +401,34 @@ def test_picked_rows_of_a_recorded_product(lib):
         b.free()
 
 
+def test_products_without_memory_for_picked_rows(lib):
+    # The memory is optional: one refusal is one warning, the products after it do not ask again, and all are whole.
+    experts, N, K, groups = 2, 64, 1024, 2048                 # 64 MiB of picked rows: more than any call before had
+    r = Run(lib, False, experts, N, K, 0)
+    which = np.repeat(np.arange(experts), groups // experts).astype(np.int32)
+    few = r.act(33, K)
+    pick = r.rng.integers(0, 33, 16 * groups).astype(np.uint32)
+    want = np.concatenate([(few.astype(np.float64) @ r.w[e].T.astype(np.float64))[pick[which.repeat(16) == e]] for e in range(experts)])
+    xd, gd, pd = r.up(few), hipattn.DeviceBuffer.from_host(which.view(np.float32)), hipattn.DeviceBuffer.from_host(pick.view(np.float32))
+    y, said = hipattn.DeviceBuffer(16 * groups * N * 4), []
+    log = C.CFUNCTYPE(None, C.c_int, C.c_char_p, vp)(lambda level, line, user: said.append((level, line)))
+    lib.wr_hip_attn_set_log(log, None)
+    lib.wr_hip_attn_set_alloc_failures(1000, 0)
+    try:
+        for call in range(6):
+            if call == 3:
+                lib.wr_hip_attn_set_alloc_failures(0, 0)
+            r.go(xd, rows=16 * groups, group_expert=gd.p, tile_groups=1, out=ROWS_F32, y_f32=y.p, ldy=N, x_perm=pd.p)
+            r.close(y.to_host((16 * groups, N)), want)
+    finally:
+        lib.wr_hip_attn_set_alloc_failures(0, 0)
+        lib.wr_hip_attn_set_log(C.cast(None, type(log)), None)
+    assert [level for level, _ in said] == [1] and b"picked rows" in said[0][1], said
+    r.end()
+    for b in (xd, gd, pd, y):
+        b.free()
+
+
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("N,K,tile", [(64, 96, 1), (48, 64, 8), (4096, 64, 8), (1024, 32, 1)])
 def test_matrix_per_row_group(lib, f32, N, K, tile):

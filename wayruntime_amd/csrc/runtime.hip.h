@@ -18,7 +18,7 @@ namespace wr {
 constexpr int kMaxDevices = 16;
 constexpr uint32_t kMaxPrefillParts = 32;    // prefill: parts a block's keys are cut into at most,
 constexpr uint32_t kMaxPrefillPartMb = 128;  // and the MiB that the parts' rows take
-constexpr uint32_t kPrefillRefusedLaunches = 1000;
+constexpr uint32_t kRefusedLaunches = 1000;  // that do without optional memory before it is asked for again
 
 struct Buffer {
     void* p = nullptr;
@@ -33,7 +33,8 @@ struct Ctx {
     hipStream_t stream = nullptr;
     Buffer d_stage;              // device staging for host-pointer entry points
     Buffer d_part;               // split-K partials
-    Buffer d_picked;             // experts' rows in slot order
+    Buffer d_picked;             // experts' rows in slot order: at most kMaxPickedBytes, none where it is refused
+    uint32_t picked_refused = 0;      // launches that do without before memory for them is asked for again
     Buffer d_prefill;            // rows of prefill blocks cut into parts: at most kMaxPrefillPartMb, none where it is refused
     uint32_t prefill_refused = 0;     // launches that go uncut before memory for them is asked for again
     Buffer d_proj;               // projection operand fragments and row scales
@@ -88,6 +89,7 @@ struct Lib {
     std::atomic<Ctx*> step_owner{nullptr};       // whose launch of a whole step's layers may be on the device (one at a time)
     std::atomic<uint32_t> step_refused{0};       // steps that go layer by layer before one launch is tried again
     std::atomic<uint32_t> step_limit{0};         // ticks until its waits end; 0: kStepLimitTicks
+    std::atomic<uint32_t> fail_allocs{0}, fail_after{0};   // for tests: this many allocations fail, behind so many that do not
     std::atomic<int> prefill_two_waves{1};        // WR_HIP_PREFILL_TWO_WAVES=0: head dim 128 takes the one-wave-per-SIMD prefill kernel
 };
 extern Lib g;
@@ -114,6 +116,7 @@ int hip_fail(hipError_t e, const char* what, uint32_t layer);
 hipError_t device_malloc(void** p, size_t bytes);
 int ensure_device(Buffer& b, size_t need);
 int ensure_pinned(Buffer& b, size_t need);
+bool optional_device(Buffer& b, uint32_t& refused, size_t need, const char* without);
 int sync_checked(const char* what, uint32_t layer);
 int copy_up(void* dst_dev, const void* src_host, size_t bytes, size_t pin_off);
 int copy_down_sync(void* dst_host, const void* src_dev, size_t bytes);

@@ -166,10 +166,14 @@ void slab_leave(uint8_t* p, size_t bytes)
 // hipMalloc that what is kept makes room for.
 hipError_t device_malloc(void** p, size_t bytes)
 {
-    hipError_t e = hipMalloc(p, bytes);
+    const auto take = [&] {
+        if (g.fail_allocs.load(std::memory_order_relaxed) && !count_down(g.fail_after) && count_down(g.fail_allocs)) return hipErrorOutOfMemory;
+        return hipMalloc(p, bytes);
+    };
+    hipError_t e = take();
     if (e != hipSuccess && slabs_trim()) {
         (void)hipGetLastError();
-        e = hipMalloc(p, bytes);
+        e = take();
     }
     if (e != hipSuccess) (void)hipGetLastError();          // (the caller may do without: not for the next launch's check to find)
     return e;
@@ -186,6 +190,36 @@ int ensure_device(Buffer& b, size_t need)
     HIP_TRY(device_malloc(&b.p, want), "workspace alloc", 0);
     b.cap = want;
     return WR_HIP_OK;
+}
+
+// The same for memory that a launch can do without, in a buffer of its own: nothing another launch must have
+// is given up to make it, and a refusal is no error.  A power of two of MiB; the old one goes only when the new one is
+// there.  False: there is none, and the launch does without (as do the next ones: asking costs a failed call each time).
+bool optional_device(Buffer& b, uint32_t& refused, size_t need, const char* without)
+{
+    if (need <= b.cap) return true;
+    if (refused) {
+        refused--;
+        return false;
+    }
+    size_t want = (size_t)1 << 20;
+    while (want < need) want *= 2;
+    void* bigger = nullptr;
+    if (device_malloc(&bigger, want) != hipSuccess) {
+        logmsg(1, "no %zu MiB for %s", want >> 20, without);
+        refused = kRefusedLaunches;
+        return false;
+    }
+    if (b.p) {                                     // launches that use it may still be on their way
+        if (hipStreamSynchronize(cx->stream) != hipSuccess) {
+            (void)hipFree(bigger);
+            return false;
+        }
+        (void)hipFree(b.p);
+    }
+    b.p = bigger;
+    b.cap = want;
+    return true;
 }
 
 int ensure_pinned(Buffer& b, size_t need)
@@ -655,36 +689,11 @@ uint32_t prefill_parts(const PrefillArgs& a, uint32_t BP, uint32_t nblk, uint32_
     return best;
 }
 
-// Room for the parts' rows, in a buffer of their own: a launch can do without them, so nothing another launch must have
-// is given up to make it, and a refusal is no error.  A power of two of MiB; the old one goes only when the new one is
-// there.  False: there is none, and the launch goes uncut (as do the next ones: asking costs a failed call each time).
+// Room for the parts' rows, in a buffer of their own.  False: there is none, and the launch goes uncut.
 bool prefill_parts_ready(PrefillArgs& a, uint32_t parts)
 {
     const size_t rows = (size_t)parts * a.T * a.nq, o = rows * a.hd * sizeof(float), need = o + rows * 2 * sizeof(float);
-    if (need > cx->d_prefill.cap) {
-        if (cx->prefill_refused) {
-            cx->prefill_refused--;
-            return false;
-        }
-        size_t want = (size_t)1 << 20;
-        while (want < need) want *= 2;
-        void* bigger = nullptr;
-        if (device_malloc(&bigger, want) != hipSuccess) {
-            (void)hipGetLastError();
-            logmsg(1, "prefill: no %zu MiB for parts of long blocks; they go uncut", want >> 20);
-            cx->prefill_refused = kPrefillRefusedLaunches;
-            return false;
-        }
-        if (cx->d_prefill.p) {                     // launches that use it may still be on their way
-            if (hipStreamSynchronize(cx->stream) != hipSuccess) {
-                (void)hipFree(bigger);
-                return false;
-            }
-            (void)hipFree(cx->d_prefill.p);
-        }
-        cx->d_prefill.p = bigger;
-        cx->d_prefill.cap = want;
-    }
+    if (!optional_device(cx->d_prefill, cx->prefill_refused, need, "parts of long blocks; they go uncut")) return false;
     a.n_parts = parts;
     a.part_o = reinterpret_cast<float*>(cx->d_prefill.p);
     a.part_ml = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(cx->d_prefill.p) + o);
@@ -1404,6 +1413,7 @@ void wr_hip_attn_shutdown(void)
     g.step_owner = nullptr;
     g.step_refused = 0;
     g.step_limit = 0;
+    g.fail_allocs = 0;
 }
 
 void wr_hip_attn_set_log(wr_hip_log_fn fn, void* user)
@@ -1892,6 +1902,12 @@ void wr_hip_attn_step_destroy(wr_hip_attn_step* p)
         if (p->rows) (void)hipFree(p->rows);
     }
     delete p;
+}
+
+void wr_hip_attn_set_alloc_failures(uint32_t n, uint32_t after)
+{
+    g.fail_after = after;
+    g.fail_allocs = n;
 }
 
 void wr_hip_attn_set_step_limit(uint32_t ticks)

@@ -446,7 +446,7 @@ static void pick_rows(MixGemmArgs& a)
     if (a.x_kt != a.ktiles || bytes > kMaxPickedBytes) return;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(cx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
-        ensure_device(cx->d_picked, bytes) != WR_HIP_OK) {
+        !optional_device(cx->d_picked, cx->picked_refused, bytes, "picked rows; products pick them again in every workgroup")) {
         (void)hipGetLastError();
         return;
     }
