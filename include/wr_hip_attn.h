@@ -92,10 +92,12 @@ const char *wr_hip_attn_device_name(void);
  * source layer's index to the other calls).  Allocation failure is
  * WR_HIP_ERR_NOMEM; max_ctx above the cap is WR_HIP_ERR_LIMIT
  * (session.c:755).  The device memory of destroyed caches is kept for later ones of
- * its size, 2 GiB at most (of sixteen), until shutdown or until an allocation fails. */
+ * its size, 2 GiB at most (of sixteen), while a sixteenth of the device's memory is free, until trim or
+ * shutdown or until an allocation here fails.  trim gives it back, for whoever else allocates. */
 int  wr_hip_attn_kv_create(uint32_t n_layers, const uint32_t *hd_per_layer,
                            uint32_t nkv, uint32_t max_ctx, wr_hip_kv **out);
 void wr_hip_attn_kv_destroy(wr_hip_kv *kv);
+void wr_hip_attn_trim(void);
 uint64_t wr_hip_attn_kv_bytes(const wr_hip_kv *kv);
 
 /* ---- append -------------------------------------------------------------

@@ -112,6 +112,11 @@ void wr_hip_attn_kv_destroy(wr_hip_kv *kv)
     free(kv);
 }
 
+static int g_trims;
+int wr_hip_attn_debug_trims(void);
+int wr_hip_attn_debug_trims(void) { return g_trims; }
+void wr_hip_attn_trim(void) { g_trims++; }
+
 uint64_t wr_hip_attn_kv_bytes(const wr_hip_kv *kv) { return kv ? kv->bytes : 0; }
 
 static int layer_ok(const wr_hip_kv *kv, uint32_t layer)

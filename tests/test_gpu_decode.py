@@ -845,6 +845,15 @@ def test_memory_of_ended_caches_is_bounded_and_comes_back_cleared():
     big = hipattn.KVCache(9, hd, nkv, rows)                  # more than is kept at all
     big.close()
     assert free - free_bytes() <= (2 << 30) + (64 << 20)
+    hipattn.lib().wr_hip_attn_trim()                         # for others to allocate
+    assert free - free_bytes() <= 64 << 20
+    free = free_bytes()
+    hipattn.KVCache(4, hd, nkv, rows).close()
+    assert free - free_bytes() >= (1 << 30) - (64 << 20)
+    hipattn.lib().wr_hip_attn_set_alloc_failures(1, 0)       # an allocation that fails takes what is kept and is made again
+    buf = hipattn.DeviceBuffer(4096)
+    assert free - free_bytes() <= 64 << 20
+    buf.free()
 
     def walk(seed, out):                                     # sizes shared between threads, each with its own rows
         r = np.random.default_rng(seed)

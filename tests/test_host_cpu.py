@@ -347,7 +347,9 @@ def test_a_model_outlives_the_end_of_its_last_session(eng, tmp_path, capfd, walk
         lib.wr_hip_attn_debug_on_kv_destroy(hook_t())
     assert len(seen) == 1 and "1 session(s) still alive; refused" in seen[0]
     m.session().close()                                        # the model is whole
+    trims = lib.wr_hip_attn_debug_trims()
     m.close()
+    assert lib.wr_hip_attn_debug_trims() == trims + 1          # ... and what its caches left is given back with it
 
 
 def test_a_model_loads_without_device_memory_for_an_embedding_of_its_own(eng, tmp_path, capfd):

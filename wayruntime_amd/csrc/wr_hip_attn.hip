@@ -106,8 +106,10 @@ int hip_fail(hipError_t e, const char* what, uint32_t layer)
 // millisecond a session, and thousands of sessions one after the other come to minutes in which the driver, which
 // clears what it is given back, takes 12 ms to each (a session of 10 tokens and one answer 2.1 -> 14.1 ms from some 250
 // sessions on, with calls 2.1 ms apart; 400 at 2.6).  Bounded, the longest kept goes first; given back with
-// the library, and when an allocation fails.
+// the library, with a model (wr_hip_attn_trim), and when an allocation fails.  Nobody else's allocation can ask for it:
+// where less than a sixteenth of the device is free nothing is kept.
 constexpr size_t kKeptSlabs = 16, kKeptSlabBytes = (size_t)2 << 30;
+constexpr size_t kKeptOfFree = 16;
 
 void slabs_free(std::vector<Lib::Slab>& slabs)
 {
@@ -143,7 +145,10 @@ uint8_t* slab_take(size_t bytes)
 // The slab of a cache that has ended, on the library's device.  As hipFree would, it waits for all of the device's streams.
 void slab_leave(uint8_t* p, size_t bytes)
 {
-    if (bytes > kKeptSlabBytes || hipDeviceSynchronize() != hipSuccess) {
+    size_t free_bytes = 0, total = 0;
+    const bool room = hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes >= total / kKeptOfFree;
+    if (!room) (void)slabs_trim();
+    if (!room || bytes > kKeptSlabBytes || hipDeviceSynchronize() != hipSuccess) {
         (void)hipGetLastError();
         (void)hipFree(p);
         return;
@@ -1512,6 +1517,13 @@ void wr_hip_attn_kv_destroy(wr_hip_kv* kv)
         else if (kv->slab) (void)hipFree(kv->slab);          // (waits for the device's other streams by itself)
     }
     delete kv;
+}
+
+void wr_hip_attn_trim(void)
+{
+    if (!g.inited) return;
+    Entered entered_;
+    if (entered_.ok()) (void)slabs_trim();
 }
 
 uint64_t wr_hip_attn_kv_bytes(const wr_hip_kv* kv) { return kv ? kv->bytes : 0; }

@@ -815,6 +815,7 @@ void wr_model_free(wr_model *m)
     wrh_scratch_free_all(m);
     wrh_device_model_free(m);
     wrh_mix_free(m->mix);
+    wr_hip_attn_trim();                                    /* its sessions' caches are of no use to another model */
     if (m->map) munmap(m->map, m->map_bytes);
     pthread_mutex_destroy(&m->lock);
     free(m);
