@@ -385,7 +385,8 @@ int wr_hip_proj_rows_norm_dev(const wr_hip_weight *w, uint32_t rows,
                               const float *norm_w_dev, float eps,
                               const float *add_dev, float *y_dev, uint32_t ldy);
 /* _norm_dev without `add` for up to WR_HIP_BATCH_MAX rows, row r into n_out floats at dst_locked[r] (16-byte aligned, in
- * memory of wr_hip_attn_host_alloc, apart from each other); waits.  tmp_dev: rows x n_out floats that it may use. */
+ * memory of wr_hip_attn_host_alloc, apart from each other); waits.  tmp_dev: rows x n_out floats that it may use, for more
+ * than one row (one row: not used, may be NULL). */
 int wr_hip_proj_rows_norm_down(const wr_hip_weight *w, uint32_t rows, const float *x_dev, uint32_t ldx,
                                const float *norm_w_dev, float eps, float *const *dst_locked, float *tmp_dev);
 int wr_hip_proj_rows_swiglu_dev(const wr_hip_weight *w, uint32_t rows,

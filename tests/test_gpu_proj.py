@@ -645,6 +645,11 @@ def test_rows_of_a_product_into_host_memory(n_in, n_out):
     down = lib.wr_hip_proj_rows_norm_down
     assert down(w.h, 17, xd.p, n_in, nwd.p, 1e-6, dst, y.p) == hipattn.ERR_LIMIT
     assert down(w.h, 2, xd.p, n_in, None, 1e-6, dst, y.p) == hipattn.ERR_INVAL
+    assert down(w.h, 2, xd.p, n_in, nwd.p, 1e-6, dst, None) == hipattn.ERR_INVAL
+    assert down(w.h, 1, xd.p, n_in, nwd.p, 1e-6, dst, None) == hipattn.OK           # one row needs no memory of the caller's
+    assert lib.wr_hip_proj_rows_norm_dev(w.h, 1, xd.p, n_in, nwd.p, 1e-6, None, y.p, n_out) == hipattn.OK
+    hipattn.sync()
+    assert np.array_equal(rows[0][:n_out], y.to_host((17, n_out))[0])
     assert down(w.h, 2, xd.p, n_in, nwd.p, 1e-6, (C.c_void_p * 2)(places[0], places[1] + 4), y.p) == hipattn.ERR_INVAL
     assert down(w.h, 0, xd.p, n_in, nwd.p, 1e-6, dst, y.p) == hipattn.OK
     for p in places:

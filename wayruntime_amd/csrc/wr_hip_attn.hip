@@ -2396,10 +2396,10 @@ int wr_hip_proj_rows_norm_dev(const wr_hip_weight* w, uint32_t rows, const float
 int wr_hip_proj_rows_norm_down(const wr_hip_weight* w, uint32_t rows, const float* x_dev, uint32_t ldx,
                                const float* norm_w_dev, float eps, float* const* dst_locked, float* tmp_dev)
 {
-    int rc = check_proj(w, rows, x_dev, ldx, w ? w->n_in : 0, tmp_dev, w ? w->n_out : 0, w ? w->n_out : 0);
+    int rc = check_proj(w, rows, x_dev, ldx, w ? w->n_in : 0, dst_locked, w ? w->n_out : 0, w ? w->n_out : 0);
     if (rc || rows == 0) return rc;
     if (rows > WR_HIP_BATCH_MAX) return WR_HIP_ERR_LIMIT;
-    if (!norm_w_dev || !dst_locked || ((uintptr_t)tmp_dev & 15)) return WR_HIP_ERR_INVAL;
+    if (!norm_w_dev || (rows > 1 && !tmp_dev) || ((uintptr_t)tmp_dev & 15)) return WR_HIP_ERR_INVAL;
     ProjDownArgs d{};
     for (uint32_t i = 0; i < rows; i++) {
         if (!dst_locked[i] || ((uintptr_t)dst_locked[i] & 15)) return WR_HIP_ERR_INVAL;

@@ -225,7 +225,7 @@ int wrh_devspace_init(wrh_devspace *ws, const wr_model *m, uint32_t rows, uint32
     ws->act = b;     b += r64(R * ffn);
     ws->rope = b;    b += r64(R * hd);
     ws->rope_swa = b; b += r64(R * hd);
-    ws->logits = b;
+    ws->logits = logit_rows ? b : NULL;
     return WR_OK;
 }
 
