@@ -644,10 +644,22 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
             // Over a short range workgroups of 64 rows, more to a compute unit, up to 48 rows (128 / 64 rows a workgroup:
             // 64 experts, 384 -> 4096 70 / 58, 512 -> 4096 78 / 70, 1024 -> 2048 64 / 62; 2048 -> 1024 62 / 64; beyond, part of
             // the experts' weights would pass twice: 1024 -> 2048 at 64 rows 73 / 80).
+            // Beyond 48 rows the tiles are the faster ones again where they come out even: sixteen columns of them, two to
+            // an XCD, that fill the device's last round by seven eighths, up to three rounds (stream / tile at 62 rows: 15
+            // experts, 1280 -> 2048 30.1 / 25.3, 3072 -> 2048 61.4 / 51.2; 32 experts, 768 -> 2048 36.3 / 31.0, 1536 -> 2048
+            // 59.3 / 54.4; 48 experts, 1280 -> 2048 74.3 / 68.2; against 18 experts 32.8 / 37.5 of the first, 34 55.3 / 60.6, and
+            // 16 experts, 1536 -> 3072 45.5 / 46.0), a single round by three quarters (12 experts, 3072 -> 2048 51.8 / 45.4), two
+            // beyond 56 (24 experts, 1408 -> 2048 at 54 rows 42.7 / 43.4, at 62 47.1 / 42.6), but for 1024 and 2048 inputs, whose tiles are slower by a tenth (16 experts 24.2 / 30.5 and
+            // 42.1 / 52.2, 32 42.4 / 46.2 and 71.4 / 75.9).  By XCD the narrowest end at 68 (64 experts, 4096 -> 384
+            // at 66 rows 62.5 / 63.7, at 72 70.3 / 64.8; -> 256 at 80 66 / 57; -> 512 96 / 113).
             // As many runs as experts, or fewer, are not route's: the caller counted them, so they may be full.
             const uint64_t runs = a.groups / 8, e = q->w->batch, spare = runs > e ? (runs - e) * 128 : 0;
             if (spare && spare <= e * 48 && a.ktiles <= 32) return launch_runs<4>(a, q->w->batch);
-            const uint32_t most = a.ktiles <= 16 || a.ntiles >= 256 ? 48 : runs_by_xcd(a, q->w->batch) ? 80 : 64;
+            const uint64_t columns = (a.ntiles + 7) / 8, rounds = (e * columns + g.n_cus - 1) / g.n_cus;
+            const uint64_t eighths = columns == 16 && rounds <= 3 && a.ktiles != 32 && a.ktiles != 64 ? e * columns * 8 / (rounds * g.n_cus) : 0;
+            const uint32_t most = a.ktiles <= 16 || a.ntiles >= 256 || eighths >= (rounds == 1 ? 6 : 7) ? 48
+                                  : eighths == 6 && rounds == 2 ? 56
+                                  : !runs_by_xcd(a, q->w->batch) ? 64 : a.ntiles < 32 ? 68 : 80;
             if (spare && spare <= e * most) return launch_runs<8>(a, q->w->batch);
             return launch_lds<4>(a, 1);
         }
