@@ -629,73 +629,73 @@ __device__ __forceinline__ void proj_rows_sums(const ProjArgs& a, f32x4 (&acc)[N
     constexpr int KB = kProjKBatch / NT;                               // k-steps per register batch
     const uint32_t ktiles = a.K / 32, ntiles = a.N / 16;
     const half8* xp = a.xfrag + lane;
-            // tile t of this wave; a run that sticks out past N re-reads the last tile and drops the result
-            const half8* wp[NT];
-    #pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const uint32_t nt = GATED ? proj_paired_tile(nt0, t, ntiles) : (nt0 + t < ntiles) ? nt0 + t : ntiles - 1;
-                wp[t] = a.w + (size_t)nt * ktiles * 64 + lane;
-            }
-            // W is read exactly once per launch (non-temporal); X fragments are
-            // shared by every wave of the grid and stay cached.  Loads inside the
-            // loop are unconditional and the last batch is peeled, so the
-            // compiler's load counting keeps the prefetched batch in flight.
-            half8 wa[KB][NT], wb[KB][NT];
-            // The operand fragments travel a batch ahead with the weights: read when
-            // needed they are cache hits, but a round trip to L2 per batch on a
-            // chain of four to thirty batches that is the launch's critical path.
-            half8 xa[KB][GROUPS], xb[KB][GROUPS];
-            auto load_x = [&](half8 (&xv)[KB][GROUPS], uint32_t k0) {
-    #pragma unroll
-                for (int u = 0; u < KB; u++)
-    #pragma unroll
-                    for (int gi = 0; gi < GROUPS; gi++) xv[u][gi] = xp[((size_t)gi * ktiles + k0 + u) * 64];
-            };
-            auto step = [&](const half8 (&wv)[NT], const half8 (&xv)[GROUPS]) {
-    #pragma unroll
-                for (int gi = 0; gi < GROUPS; gi++)
-    #pragma unroll
-                    for (int t = 0; t < NT; t++)
-                        acc[t][gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[t], xv[gi], acc[t][gi], 0, 0, 0);
-            };
-            uint32_t kt = k_begin;
+    // tile t of this wave; a run that sticks out past N re-reads the last tile and drops the result
+    const half8* wp[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const uint32_t nt = GATED ? proj_paired_tile(nt0, t, ntiles) : (nt0 + t < ntiles) ? nt0 + t : ntiles - 1;
+        wp[t] = a.w + (size_t)nt * ktiles * 64 + lane;
+    }
+    // W is read exactly once per launch (non-temporal); X fragments are
+    // shared by every wave of the grid and stay cached.  Loads inside the
+    // loop are unconditional and the last batch is peeled, so the
+    // compiler's load counting keeps the prefetched batch in flight.
+    half8 wa[KB][NT], wb[KB][NT];
+    // The operand fragments travel a batch ahead with the weights: read when
+    // needed they are cache hits, but a round trip to L2 per batch on a
+    // chain of four to thirty batches that is the launch's critical path.
+    half8 xa[KB][GROUPS], xb[KB][GROUPS];
+    auto load_x = [&](half8 (&xv)[KB][GROUPS], uint32_t k0) {
+#pragma unroll
+        for (int u = 0; u < KB; u++)
+#pragma unroll
+            for (int gi = 0; gi < GROUPS; gi++) xv[u][gi] = xp[((size_t)gi * ktiles + k0 + u) * 64];
+    };
+    auto step = [&](const half8 (&wv)[NT], const half8 (&xv)[GROUPS]) {
+#pragma unroll
+        for (int gi = 0; gi < GROUPS; gi++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                acc[t][gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[t], xv[gi], acc[t][gi], 0, 0, 0);
+    };
+    uint32_t kt = k_begin;
     const uint32_t kper = k_end - k_begin;
-            const uint32_t full_end = k_begin + kper / KB * KB;
-            if (kt < full_end) {
-    #pragma unroll
-                for (int u = 0; u < KB; u++)
-    #pragma unroll
-                    for (int t = 0; t < NT; t++)
-                        wa[u][t] = __builtin_nontemporal_load(&wp[t][(size_t)(kt + u) * 64]);
-                load_x(xa, kt);
-                while (kt + 2 * KB <= full_end) {
-    #pragma unroll
-                    for (int u = 0; u < KB; u++)
-    #pragma unroll
-                        for (int t = 0; t < NT; t++)
-                            wb[u][t] = __builtin_nontemporal_load(&wp[t][(size_t)(kt + KB + u) * 64]);
-                    load_x(xb, kt + KB);
-    #pragma unroll
-                    for (int u = 0; u < KB; u++) step(wa[u], xa[u]);
-    #pragma unroll
-                    for (int u = 0; u < KB; u++) {
-    #pragma unroll
-                        for (int t = 0; t < NT; t++) wa[u][t] = wb[u][t];
-    #pragma unroll
-                        for (int gi = 0; gi < GROUPS; gi++) xa[u][gi] = xb[u][gi];
-                    }
-                    kt += KB;
-                }
-    #pragma unroll
-                for (int u = 0; u < KB; u++) step(wa[u], xa[u]);
-                kt += KB;
+    const uint32_t full_end = k_begin + kper / KB * KB;
+    if (kt < full_end) {
+#pragma unroll
+        for (int u = 0; u < KB; u++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                wa[u][t] = __builtin_nontemporal_load(&wp[t][(size_t)(kt + u) * 64]);
+        load_x(xa, kt);
+        while (kt + 2 * KB <= full_end) {
+#pragma unroll
+            for (int u = 0; u < KB; u++)
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+                    wb[u][t] = __builtin_nontemporal_load(&wp[t][(size_t)(kt + KB + u) * 64]);
+            load_x(xb, kt + KB);
+#pragma unroll
+            for (int u = 0; u < KB; u++) step(wa[u], xa[u]);
+#pragma unroll
+            for (int u = 0; u < KB; u++) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) wa[u][t] = wb[u][t];
+#pragma unroll
+                for (int gi = 0; gi < GROUPS; gi++) xa[u][gi] = xb[u][gi];
             }
-            for (; kt < k_end; kt++) {                               // part not a multiple of the batch
-                half8 wv[NT];
-    #pragma unroll
-                for (int t = 0; t < NT; t++) wv[t] = __builtin_nontemporal_load(&wp[t][(size_t)kt * 64]);
-                proj_step<GROUPS, NT>(acc, wv, xp, ktiles, kt);
-            }
+            kt += KB;
+        }
+#pragma unroll
+        for (int u = 0; u < KB; u++) step(wa[u], xa[u]);
+        kt += KB;
+    }
+    for (; kt < k_end; kt++) {                               // part not a multiple of the batch
+        half8 wv[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) wv[t] = __builtin_nontemporal_load(&wp[t][(size_t)kt * 64]);
+        proj_step<GROUPS, NT>(acc, wv, xp, ktiles, kt);
+    }
 }
 
 // GROUPS = row groups of eight (one or two), NT = 16-output tiles per wave
