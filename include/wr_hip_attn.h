@@ -514,7 +514,8 @@ int wr_hip_rows_swiglu_dev(const float *gate_up_dev, uint32_t ld, float *act_dev
  * waited longer than 50 ms (its peers had no compute unit to run on), nothing of the step
  * counts, and it is made again layer by layer (as the next 1000 then are).
  * set_step_limit: that time in ticks of 10 ns, 0 for the default (for tests); steps that
- * gave up before are forgotten. */
+ * gave up before are forgotten.  step_set_tag: the number (2 and up) that the plan's next step counts
+ * its layers from, to see them begin again (for tests). */
 typedef struct wr_hip_attn_step wr_hip_attn_step;
 typedef struct wr_hip_attn_step_layer {
     const wr_hip_weight *wqkv, *wo, *wgu, *wdown;
@@ -528,6 +529,7 @@ int  wr_hip_attn_step_dev(wr_hip_attn_step *step, wr_hip_kv *kv, uint32_t pos, f
                           const float *cos_sin_dev, uint32_t n_rot, float scale_override);
 int  wr_hip_attn_step_done(void);
 void wr_hip_attn_set_step_limit(uint32_t ticks);
+void wr_hip_attn_step_set_tag(wr_hip_attn_step *step, uint32_t tag);
 
 /* For tests: of the allocations of device memory from now on `after` are made and then `n` fail (0: none does). */
 void wr_hip_attn_set_alloc_failures(uint32_t n, uint32_t after);

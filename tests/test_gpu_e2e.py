@@ -5,6 +5,7 @@ tests/golden/make_e2e_golden.py).  Every test runs twice: with the whole layer
 walk on the device (weights uploaded at load, the default for F16 models) and
 with the host walk that sends only the cache append and attention to the GPU
 (WAYRT_HOST_LAYERS=1 while the model loads)."""
+import dataclasses
 import os
 
 import numpy as np
@@ -292,3 +293,37 @@ def test_eight_threads_then_a_batch_beside_a_single_session(eng, tmp_path, walk)
         s.close()
     assert mism == 0 and side[0] == 0, (mism, side[0])
     m.close()
+
+
+def test_an_embedding_of_its_own(eng, tmp_path, monkeypatch, capfd):
+    # A head that is not the embedding: the table goes to the device as well, its rows are those the host makes (which
+    # does where the device has no memory for the table), and the walk is the host walk's to rounding.
+    shape = dataclasses.replace(SMALL16, tied_head=False)
+    p = str(tmp_path / "untied.gguf")
+    gw.write_model(p, shape)
+    lib = hipattn.lib()
+    prompt = workload(gw.ModelShape(vocab=shape.vocab), 40)
+
+    def run(m):
+        s = m.session(64)
+        assert s.prefill(prompt) == 40
+        rows = [np.array(s.step(t)) for t in (3, 5, 7)]
+        rc, batch = E.batch_step([s], [9])
+        assert rc == 1
+        s.close()
+        m.close()
+        return np.concatenate(rows + [np.array(batch[0])])
+
+    on_device = run(eng.load(p))
+    lib.wr_hip_attn_trim()
+    capfd.readouterr()
+    lib.wr_hip_attn_set_alloc_failures(1, 1 + 2 * (4 * shape.n_layers + 1))     # the norms, then two for each weight before it
+    try:
+        without = eng.load(p)
+    finally:
+        lib.wr_hip_attn_set_alloc_failures(0, 0)
+    assert "no device memory for the embedding" in capfd.readouterr().err
+    assert run(without).tobytes() == on_device.tobytes()
+    monkeypatch.setenv("WAYRT_HOST_LAYERS", "1")
+    on_host = run(eng.load(p))
+    assert np.linalg.norm(on_device - on_host) <= 1e-3 * np.linalg.norm(on_host)

@@ -52,6 +52,43 @@ def test_refusals():
     lib.wr_hip_attn_dev_free(vec)
 
 
+def test_tags_begin_again():
+    """Rows travel with a 32-bit number of their layer: a plan whose numbers run out clears its rows and begins again,
+    and the steps on either side are those of any other numbers.  One split of the keys, and several."""
+    hipattn.init()
+    lib, rng = hipattn.lib(), np.random.default_rng(8)
+    n, hidden = 2, 512
+    w = [[hipattn.Weight([(rng.standard_normal((o, 512)) / 16).astype(np.float16).view(np.uint16)]) for o in (1024, 512, 1024, 512)]
+         for _ in range(n)]
+    vec = hipattn.DeviceBuffer.from_host(rng.standard_normal(hidden).astype(np.float32))
+    layers = (hipattn.StepLayer * n)(*[hipattn.StepLayer(*[x.h for x in ws], vec.p, vec.p, None, None) for ws in w])
+    plan, kv = C.c_void_p(), hipattn.KVCache(n, 128, 2, 400)
+    assert lib.wr_hip_attn_step_create(n, layers, 4, 2, 128, 1e-6, C.byref(plan)) == hipattn.OK
+    x = rng.standard_normal(hidden).astype(np.float32)
+    row = hipattn.DeviceBuffer(hidden * 4)
+
+    def step(pos):
+        assert lib.wr_hip_attn_h2d(row.p, x.ctypes.data, x.nbytes) == hipattn.OK
+        assert lib.wr_hip_attn_step_dev(plan, kv.h, pos, row.p, None, 0, 0.0) == hipattn.OK
+        assert lib.wr_hip_attn_step_done() == hipattn.OK
+        return row.to_host((hidden,)).tobytes()
+
+    last = 2 ** 32 - 1 - 2 * n                               # the last number that a step's may begin at
+    for pos in (10, 390):
+        want = step(pos)
+        assert np.isfinite(np.frombuffer(want, np.float32)).all()
+        for tag in (last + 1, last, last - 1, last - 3, 2):
+            lib.wr_hip_attn_step_set_tag(plan, tag)
+            assert all(step(pos) == want for _ in range(4)), (pos, tag)
+    lib.wr_hip_attn_step_destroy(plan)
+    kv.close()
+    for ws in w:
+        for x in ws:
+            x.close()
+    for b in (vec, row):
+        b.free()
+
+
 @pytest.fixture(scope="module")
 def eng():
     hipattn.shutdown()
@@ -80,6 +117,20 @@ def _steps(model, prompt, tokens):
     assert s.prefill(tokens) == len(tokens)
     rows.append(np.array(s.step(int(tokens[0]))))
     s.close()
+    return rows
+
+
+def _batches(model, prompts, tokens):
+    ss = [model.session() for _ in prompts]
+    for s, p in zip(ss, prompts):
+        assert s.prefill(p) == len(p)
+    rows = []
+    for t in tokens:
+        rc, got = E.batch_step(ss, [int(t)] * len(ss))
+        assert rc == len(ss)
+        rows += [np.array(r) for r in got]
+    for s in ss:
+        s.close()
     return rows
 
 
@@ -194,5 +245,52 @@ def test_a_step_beside_another_threads_work(eng, tmp_path, monkeypatch, rows):
         o.close()
     for b in (q, out, x, y):
         b.free()
+    for m in (one, chain):
+        m.close()
+
+
+@pytest.mark.parametrize("limit", [0, 1])                    # 1: whichever step takes the launch gives up
+def test_steps_beside_prompts_and_batches(eng, tmp_path, monkeypatch, limit):
+    one, chain = _models(eng, tmp_path, monkeypatch, n_layers=3, hidden=1024, ffn=3072, n_q=16, n_kv=8)
+    rng = np.random.default_rng(9)
+    ids = lambda n: rng.integers(0, VOCAB, n).astype(np.uint32)
+    jobs = [(_steps, ids(50), ids(40)), (_steps, ids(700), ids(40)), (_steps, ids(1500), ids(2)),
+            (_batches, [ids(20 + 30 * i) for i in range(5)], ids(25))]
+    want = [f(chain, *args) for f, *args in jobs]
+    got = [None] * len(jobs)
+
+    def run(i):
+        f, *args = jobs[i]
+        got[i] = [f(one, *args) for _ in range(3)]
+
+    hipattn.lib().wr_hip_attn_set_step_limit(limit)
+    try:
+        threads = [threading.Thread(target=run, args=(i,)) for i in range(len(jobs))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        hipattn.lib().wr_hip_attn_set_step_limit(0)
+    for g, w in zip(got, want):
+        assert g is not None and all(np.array_equal(a, b) for again in g for a, b in zip(again, w))
+    assert _launches(one) == 2                               # and alone again
+    for m in (one, chain):
+        m.close()
+
+
+def test_more_sessions_than_rows_of_logits_are_kept(eng, tmp_path, monkeypatch):
+    one, chain = _models(eng, tmp_path, monkeypatch, n_layers=2, hidden=512, ffn=512, n_q=4, n_kv=4)
+    want = []
+    for i in range(20):
+        s = chain.session(64)
+        want.append(np.array(s.step(i)))
+        s.close()
+    for _ in range(3):                                       # sixteen of a round's rows are the next round's
+        ss = [one.session(64) for _ in range(20)]
+        rows = [s.step(i) for i, s in enumerate(ss)]
+        assert all(np.array_equal(a, b) for a, b in zip(rows, want))
+        for s in ss:
+            s.close()
     for m in (one, chain):
         m.close()

@@ -1922,6 +1922,11 @@ void wr_hip_attn_set_alloc_failures(uint32_t n, uint32_t after)
     g.fail_allocs = n;
 }
 
+void wr_hip_attn_step_set_tag(wr_hip_attn_step* p, uint32_t tag)
+{
+    if (p && tag >= 2) p->next_tag = tag;
+}
+
 void wr_hip_attn_set_step_limit(uint32_t ticks)
 {
     g.step_limit = ticks;

@@ -103,6 +103,7 @@ def load() -> C.CDLL:
         "wr_hip_attn_step_dev": (C.c_int, [_vp, _vp, _u32, _vp, _vp, _u32, C.c_float]),
         "wr_hip_attn_step_done": (C.c_int, []),
         "wr_hip_attn_set_step_limit": (None, [_u32]),
+        "wr_hip_attn_step_set_tag": (None, [_vp, _u32]),
         "wr_hip_attn_trim": (None, []),
         "wr_hip_attn_set_alloc_failures": (None, [_u32, _u32]),
         "wr_hip_proj_rows_gated_dev": (C.c_int, [_vp, _u32, _vp, _u32, _vp, C.c_float, C.c_int, _vp, _u32]),
