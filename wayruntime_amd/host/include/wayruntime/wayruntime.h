@@ -131,7 +131,8 @@ const float *wr_step(wr_session *s, uint32_t token);
 #define WR_BATCH_MAX 16
 /* Up to WR_BATCH_MAX distinct sessions of one model in one step, layer-major:
  * per layer one batched attention launch.  Returns n, or a negative status
- * with no session advanced. */
+ * with no session advanced.  (Logits that an earlier call lent out are the session's one
+ * row: the next call on it writes them anew, also where a device error then fails it.) */
 int wr_batch_step(wr_session *const *sessions, const uint32_t *tokens, uint32_t n,
                   const float **logits_out);
 
