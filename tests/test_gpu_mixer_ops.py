@@ -359,6 +359,75 @@ def test_groups_of_an_expert_that_stand_together(lib, N, K):
         b.free()
 
 
+# weights of 64 MiB and more, a workgroup to eight (sixteen) tiles of an expert's outputs: k-steps and tiles that do and do
+# not fill the last workgroup's turns, experts without rows, more runs or groups than a wave has lanes
+LARGE = [(64, 1024, 512), (64, 1040, 544), (40, 1168, 800)]
+
+
+@pytest.mark.parametrize("spare", [32, 64])
+@pytest.mark.parametrize("experts,N,K", LARGE)
+def test_large_experts_in_runs(lib, experts, N, K, spare):
+    r = Run(lib, False, experts, N, K, 0)
+    which = np.full((experts + spare, 8), -1, dtype=np.int32)
+    for i in range(experts + 3):
+        e = i if i < experts else i - experts                  # (three experts have a second run)
+        if e % 9 != 4:
+            which[i, :1 + (5 * i) % 8] = e
+    which = which.reshape(-1)
+    rows, live = 16 * len(which), np.repeat(which, 16) >= 0
+    x = r.act(rows, K)
+    xd, gd = r.up(x), hipattn.DeviceBuffer.from_host(which.view(np.float32))
+    y, h = hipattn.DeviceBuffer.from_host(np.full((rows, N), 7.0, dtype=np.float32)), hipattn.DeviceBuffer(rows * (N // 32 * 16 + 32) * 2)
+    r.go(xd, rows=rows, group_expert=gd.p, tile_groups=8, out=ROWS_F32, y_f32=y.p, ldy=N)
+    want = np.concatenate([x[16 * g:16 * g + 16].astype(np.float64) @ r.w[e].T.astype(np.float64) for g, e in enumerate(which) if e >= 0])
+    got = y.to_host((rows, N))
+    r.close(got[live], want)
+    assert np.all(got[np.repeat(which[::8], 128) < 0] == 7.0)      # (tiles write a run's empty groups too)
+    if N % 64 == 0:
+        factor = r.rng.uniform(0, 2, rows).astype(np.float32)
+        fd = hipattn.DeviceBuffer.from_host(factor)
+        r.go(xd, rows=rows, group_expert=gd.p, tile_groups=8, out=GATED, h=h.p, h_kt=N // 64, x_scale=fd.p)
+        t = (want * factor[live][:, None]).reshape(len(want), N // 32, 2, 16)
+        r.close(r.frag_down(h, rows, N // 2)[live], (O.silu(t[:, :, 0]) * t[:, :, 1]).reshape(len(want), -1), eight_bits=True)
+        fd.free()
+    r.end()
+    for b in (xd, gd, y, h):
+        b.free()
+
+
+@pytest.mark.parametrize("order", ["together", "scattered"])
+@pytest.mark.parametrize("experts,N,K", LARGE)
+def test_large_experts_in_single_groups(lib, experts, N, K, order):
+    # an expert's groups one after the other, up to nineteen, with gaps; and in an order that gives a piece to every group
+    r = Run(lib, False, experts, N, K, 0)
+    if order == "together":
+        which = np.concatenate([np.repeat(e, (3, 1, 8, 0, 19, 2, 9)[e % 7]) for e in range(experts)] + [[-1, -1, 0, 0, 5, -1]])
+        which[10] = -1
+    else:
+        which = np.arange(3 * experts) * 7 % experts
+    which = which.astype(np.int32)
+    rows, live = 16 * len(which), np.repeat(which, 16) >= 0
+    x = r.act(rows, K)
+    xd, gd = r.up(x), hipattn.DeviceBuffer.from_host(which.view(np.float32))
+    y = hipattn.DeviceBuffer.from_host(np.full((rows, N), 7.0, dtype=np.float32))
+    r.go(xd, rows=rows, group_expert=gd.p, tile_groups=1, out=ROWS_F32, y_f32=y.p, ldy=N)
+    got = y.to_host((rows, N))
+    r.close(got[live], np.concatenate([x[16 * g:16 * g + 16].astype(np.float64) @ r.w[e].T.astype(np.float64) for g, e in enumerate(which) if e >= 0]))
+    assert np.all(got[~live] == 7.0)
+    pick, used = r.rng.integers(0, 37, rows).astype(np.uint32), r.rng.random(rows) < 0.8
+    pd = hipattn.DeviceBuffer.from_host(np.where(used, pick, np.uint32(0xFFFFFFFF)).astype(np.uint32).view(np.float32))
+    few = r.act(37, K + 64)
+    fd, seen = r.up(few), live & used
+    r.go(fd, rows=rows, group_expert=gd.p, tile_groups=1, out=ROWS_F32, y_f32=y.p, ldy=N, x_perm=pd.p, x_kt=K // 32 + 2, x_kt0=1)
+    got = y.to_host((rows, N))
+    want = np.concatenate([few[pick[16 * g:16 * g + 16], 32:32 + K].astype(np.float64) @ r.w[max(e, 0)].T.astype(np.float64) for g, e in enumerate(which)])
+    r.close(got[seen], want[seen])
+    assert np.all(got[~live] == 7.0)
+    r.end()
+    for b in (xd, gd, y, pd, fd):
+        b.free()
+
+
 def test_picked_rows_of_a_recorded_product(lib):
     # A recorded product picks its rows by itself: it is one launch, none of the thread's own memory is in
     # the graph, and replays hold after a larger call has made that memory anew.

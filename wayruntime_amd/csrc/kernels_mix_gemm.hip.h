@@ -6,6 +6,7 @@
 //   mix_gemm_split_kernel  any row count, both activation types: a workgroup's waves
 //                          share a tile and split the input range (decode: HBM-bound
 //                          on the weight bytes)
+//   mix_gemm_runs_kernel   experts whose weights are large: HBM-bound on them up to some hundred rows each
 //   mix_gemm_lds_kernel    prompt-sized row counts, bfloat16: 128-output tiles
 //                          staged through LDS (MFMA-bound)
 #pragma once
@@ -372,6 +373,246 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
         if (u % GR >= live) continue;
         const f32x4 v = sum(u);
         mix_store_tile<F32>(a, v, v, nt0 + u / GR, group0 + u % GR, z, lane);
+    }
+}
+
+// Products of experts whose weights are large, as a stream of them.  A piece of work is up to eight groups of rows that
+// share an expert (a run's; SINGLE: an expert's that stand together) against WAVES x NT tiles of its outputs: a wave has
+// NT tiles over the whole input range, weights straight to registers (each byte is one wave's), two chunks of KC
+// k-steps on their way; the rows pass through LDS, a chunk in two buffers, for all waves.
+// Bound by HBM.  mix_gemm_split_kernel, which splits the input range over its waves, reads the rows once for every two tiles
+// (1.5 times the weights' bytes at 48 rows an expert), this one once for eight, and a piece's workgroups are on one XCD,
+// whichever runs there are (dealt out to all of them: 51 us -> 70).  Us, split kernel / this one: 64 experts, 2048 ->
+// 1024 in runs of 48 rows each 62.5 / 52 (5.2 TB/s; 20: 49 / 47, 128: 108, tiles, / 92), 4096 -> 4096 of 32 at 48
+// 235 / 186 (5.8 TB/s), 4096 -> 14 336 of 8 at 60 223 / 174; single groups, 64 experts of 2048 -> 1024 with 29 rows each 68 /
+// 48, picked one by one 76 / 53, 4096 -> 384 85 / 39.
+// Tried: two chunks of rows on their way (51.7 -> 54.5), four tiles to a wave (60 -> 65), one (60 -> 58.6 but 1024 -> 2048
+// 62 -> 65), two waves (62); a loop over pieces around this (spills, 52 -> 60).
+constexpr uint32_t kMixMaxPieces = 512;                    // groups (SINGLE) or runs that pieces are cut from
+
+// The launch's arguments, read again: what a kernel's end needs of them is not kept through its loops.
+__device__ __forceinline__ const MixGemmArgs& mix_fresh_args()
+{
+    typedef const __attribute__((address_space(4))) MixGemmArgs* Args;
+    Args p = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const MixGemmArgs*)p;
+}
+
+// One wave: tiles nt0 .. nt0 + tiles - 1 of the groups first, first + step, ..., one after the other: for orders of groups that
+// nobody makes in earnest (routing puts an expert's together), so that they are right all the same.
+__device__ __forceinline__ void mix_gemm_scattered(const MixGemmArgs& a, uint32_t nt0, uint32_t tiles, uint32_t first, uint32_t step, int lane)
+{
+    if (nt0 >= a.ntiles) return;
+    for (uint32_t group = first; group < a.groups; group += step) {
+        const int e = a.group_expert[group];
+        if (e < 0) continue;
+        const bf16x8* x = reinterpret_cast<const bf16x8*>(a.x) + (size_t)group * a.x_kt * 64 + lane;
+        if (a.x_perm) {
+            const uint32_t pick = a.x_perm[group * 16 + (lane & 15)], row = pick == 0xFFFFFFFFu ? 0 : pick;
+            x = reinterpret_cast<const bf16x8*>(a.x) + (size_t)(row >> 4) * a.x_kt * 64 + (lane & 48) + (row & 15);
+        }
+#pragma unroll 1
+        for (uint32_t t = 0; t < tiles; t += 2) {
+            const uint32_t nt = nt0 + t;
+            const bf16x8* w0 = a.w + ((size_t)(uint32_t)e * a.ntiles + min(nt, a.ntiles - 1)) * a.ktiles * 64 + lane;
+            const bf16x8* w1 = a.w + ((size_t)(uint32_t)e * a.ntiles + min(nt + 1, a.ntiles - 1)) * a.ktiles * 64 + lane;
+            f32x4 v0 = f32x4{0.f, 0.f, 0.f, 0.f}, v1 = v0;
+            for (uint32_t k = 0; k < a.ktiles; k++) {
+                const bf16x8 xv = x[k * 64];
+                v0 = mix_mfma(w0[k * 64], xv, v0);
+                v1 = mix_mfma(w1[k * 64], xv, v1);
+            }
+            mix_store_tile<false>(a, v0, v1, nt, group, 0, lane);
+            if (a.out < kMixOutGated) mix_store_tile<false>(a, v1, v1, nt + 1, group, 0, lane);
+        }
+    }
+}
+
+template <int NT, int WAVES, int KC, bool SINGLE>
+__global__ __launch_bounds__(WAVES * 64, 2) void mix_gemm_runs_kernel(const MixGemmArgs a)
+{
+    constexpr int GR = 8, D = 2 * KC, WORDS = (SINGLE ? kMixMaxPieces : 256) / 64, RUN = SINGLE ? 1 : GR;
+    __shared__ bf16x8 s_x[2][KC * GR * 64];
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t n = a.ktiles, last = n - 1;
+    // Where pieces begin, a bit to a run or group.
+    const uint32_t entries = a.groups / RUN, units = (a.ntiles + NT * WAVES - 1) / (NT * WAVES);
+    uint64_t begins[WORDS], edges[WORDS];                  // edges (SINGLE): where an expert's groups end or begin
+    int expert_of[WORDS];
+#pragma unroll
+    for (int i = 0; i < WORDS; i++) {
+        const uint32_t at = i * 64 + lane;
+        expert_of[i] = -1;
+        if (at < entries) expert_of[i] = a.group_expert[at * RUN];
+    }
+    uint32_t pieces = 0, start = 0;
+    int before = -1;
+#pragma unroll
+    for (int i = 0; i < WORDS; i++) {
+        const int e = expert_of[i];
+        bool begin = e >= 0;
+        if constexpr (SINGLE) {                            // the first of an expert's groups, and every eighth behind it
+            int prev = __shfl_up(e, 1, 64);
+            if (lane == 0) prev = before;
+            edges[i] = __ballot(e < 0 || e != prev);
+            const uint64_t firsts = __ballot(e >= 0 && e != prev), upto = firsts & (~0ull >> (63 - lane));
+            const uint32_t first = upto ? i * 64 + 63 - __builtin_clzll(upto) : start;
+            begin = begin && (i * 64 + lane - first) % GR == 0;
+            if (firsts) start = i * 64 + 63 - __builtin_clzll(firsts);
+            before = __builtin_amdgcn_readlane(e, 63);
+        }
+        begins[i] = __ballot(begin);
+        pieces += (uint32_t)__popcll(begins[i]);
+    }
+    const uint32_t xcd = blockIdx.x % 8, work = pieces * units;
+    if constexpr (SINGLE) {
+        if (work > gridDim.x) {                            // an expert's groups all over the place: more pieces than there are workgroups
+            const uint32_t step = gridDim.x / units, first = blockIdx.x / units;
+            if (first < step) mix_gemm_scattered(a, (blockIdx.x % units * WAVES + wave) * NT, NT, first, step, lane);
+            return;
+        }
+    }
+    // XCD x takes an eighth of the pieces, one after the other: a run's rows come into one L2
+    const uint32_t j = (uint32_t)((uint64_t)work * xcd / 8) + blockIdx.x / 8;
+    if (j >= (uint32_t)((uint64_t)work * (xcd + 1) / 8)) return;
+    uint32_t skip = j / units, group0 = 0, expert = 0, live = GR;        // live: groups that rows are in (they come first)
+    bool found = false;
+#pragma unroll
+    for (int i = 0; i < WORDS; i++) {
+        const uint32_t here = (uint32_t)__popcll(begins[i]);
+        if (!found && skip < here) {
+            uint64_t m = begins[i];
+            for (uint32_t s = 0; s < skip; s++) m &= m - 1;
+            const uint32_t bit = (uint32_t)__builtin_ctzll(m);
+            const int e = __builtin_amdgcn_readlane(expert_of[i], (int)bit);
+            group0 = (i * 64 + bit) * RUN;
+            if constexpr (SINGLE) {
+                const uint64_t behind = (edges[i] >> bit) >> 1 | (i + 1 < WORDS && bit ? edges[i + 1 < WORDS ? i + 1 : i] << (63 - bit) : 0);
+                expert = (uint32_t)e;
+                live = behind ? min((uint32_t)__builtin_ctzll(behind) + 1, (uint32_t)GR) : GR;
+                live = min(live, a.groups - group0);
+            } else {
+                expert = (uint32_t)e;
+                live = 1;
+#pragma unroll
+                for (uint32_t g = 1; g < GR; g++)
+                    if (a.group_expert[group0 + g] >= 0) live = g + 1;
+            }
+            found = true;
+        }
+        if (!found) skip -= here;
+    }
+    const uint32_t nt0 = (j % units * WAVES + wave) * NT;
+
+    const bf16x8* wp[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+        wp[t] = a.w + ((size_t)expert * a.ntiles + min(nt0 + t, a.ntiles - 1)) * n * 64;
+
+    const auto product = [&](auto groups) {
+        constexpr int L = decltype(groups)::value, S = (KC * L + WAVES - 1) / WAVES;
+        f32x4 acc[NT][L];
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int i = 0; i < L; i++) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        bf16x8 w[D][NT], xr[S];
+        // a wave's share of a chunk: blocks of one group and k-step
+        const bf16x8* xp[S];
+        uint32_t x_lane[S];
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            const uint32_t b = min(wave + s * WAVES, (uint32_t)(KC * L - 1)), group = group0 + b / KC;
+            xp[s] = reinterpret_cast<const bf16x8*>(a.x) + (size_t)group * a.x_kt * 64;
+            x_lane[s] = lane;
+            if constexpr (SINGLE) {
+                if (a.x_perm) {                        // rows picked one by one: the lanes fetch their own
+                    const uint32_t pick = a.x_perm[group * 16 + (lane & 15)], row = pick == 0xFFFFFFFFu ? 0 : pick;
+                    xp[s] = reinterpret_cast<const bf16x8*>(a.x);
+                    x_lane[s] = (row >> 4) * a.x_kt * 64 + (lane & 48) + (row & 15);
+                }
+            }
+        }
+        auto ask_rows = [&](uint32_t k0) {
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                const uint32_t b = min(wave + s * WAVES, (uint32_t)(KC * L - 1));
+                xr[s] = xp[s][min(k0 + b % KC, last) * 64 + x_lane[s]];
+            }
+        };
+        auto put_rows = [&](int buf) {
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                const uint32_t b = min(wave + s * WAVES, (uint32_t)(KC * L - 1));
+                s_x[buf][(b % KC * L + b / KC) * 64 + lane] = xr[s];
+            }
+        };
+        auto ask_weights = [&](int d, uint32_t k) {
+#pragma unroll
+            for (int t = 0; t < NT; t++) w[d][t] = __builtin_nontemporal_load(&wp[t][min(k, last) * 64 + lane]);
+        };
+        auto multiply = [&](int d) {
+            bf16x8 xv[L];
+#pragma unroll
+            for (int i = 0; i < L; i++) xv[i] = s_x[d / KC][(d % KC * L + i) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < L; i++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(w[d][t], xv[i], acc[t][i]);
+        };
+        ask_rows(0);
+#pragma unroll
+        for (int d = 0; d < D; d++) ask_weights(d, d);
+        put_rows(0);
+        lds_barrier();
+        uint32_t k = 0;
+        for (; k + D < n; k += D) {
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                if (d % KC == 0) ask_rows(k + d + KC);
+                multiply(d);
+                ask_weights(d, k + D + d);
+                __builtin_amdgcn_sched_barrier(0);
+                if (d % KC == KC - 1) {
+                    put_rows(1 - d / KC);
+                    lds_barrier();
+                }
+            }
+        }
+        ask_rows(k + KC);
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            if (k + d < n) multiply(d);
+            if (d == KC - 1) {
+                put_rows(1);
+                lds_barrier();
+            }
+        }
+        const MixGemmArgs& o = mix_fresh_args();
+        if (o.out >= kMixOutGated) {
+            if constexpr (NT % 2 == 0)
+#pragma unroll
+                for (int t = 0; t < NT; t += 2)
+#pragma unroll
+                    for (int i = 0; i < L; i++) mix_store_tile<false>(o, acc[t][i], acc[t + 1][i], nt0 + t, group0 + i, 0, lane);
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int i = 0; i < L; i++) mix_store_tile<false>(o, acc[t][i], acc[t][i], nt0 + t, group0 + i, 0, lane);
+    };
+    switch (live) {
+    case 1: product(std::integral_constant<int, 1>()); break;
+    case 2: product(std::integral_constant<int, 2>()); break;
+    case 3: product(std::integral_constant<int, 3>()); break;
+    case 4: product(std::integral_constant<int, 4>()); break;
+    case 5: product(std::integral_constant<int, 5>()); break;
+    case 6: product(std::integral_constant<int, 6>()); break;
+    case 7: product(std::integral_constant<int, 7>()); break;
+    default: product(std::integral_constant<int, 8>()); break;
     }
 }
 

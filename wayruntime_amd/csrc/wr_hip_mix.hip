@@ -467,6 +467,27 @@ static bool runs_by_xcd(const MixGemmArgs& a, uint32_t experts)
     return a.ntiles <= 96 && (uint64_t)((experts + 7) / 8 * 8) * 7 <= (uint64_t)experts * 8;
 }
 
+// Whether mix_gemm_runs_kernel is for these experts' weights: 64 MiB of them and more (less are read faster by the
+// split kernel's shorter chains: 12 experts, 768 -> 2048 11 us / 12; 32 experts, 2048 -> 512 16 / 20), workgroups of eight tiles
+// for two thirds of the compute units, but not a few more than units, which gives some of them two (18 experts, 1280 -> 2048,
+// 288 of them: 22.6 / 25), and 512 inputs (64 experts, 384 -> 4096 49 / 51).
+static bool streams(const MixGemmArgs& a, uint64_t experts)
+{
+    const uint64_t workgroups = experts * ((a.ntiles + 7) / 8), mib = experts * a.ntiles * a.ktiles >> 10;
+    const bool even = workgroups <= g.n_cus || workgroups * 2 >= g.n_cus * 3;
+    return mib >= 64 && a.ktiles >= 16 && workgroups * 3 >= g.n_cus * 2 && even;
+}
+
+template <int NT, int WAVES, int KC, bool SINGLE>
+static int launch_stream(const MixGemmArgs& a, uint32_t experts)
+{
+    const uint32_t units = (a.ntiles + NT * WAVES - 1) / (NT * WAVES), entries = SINGLE ? a.groups : a.groups / 8;
+    const uint32_t pieces = SINGLE ? std::min(a.groups, experts + a.groups / 8) : entries;
+    launch_main(mix_gemm_runs_kernel<NT, WAVES, KC, SINGLE>, dim3((pieces * units + 7) / 8 * 8), dim3(WAVES * 64), a);
+    HIP_TRY(hipGetLastError(), "product launch", 0);
+    return WR_HIP_OK;
+}
+
 template <int GR>
 static int launch_runs(const MixGemmArgs& args, uint32_t experts)
 {
@@ -631,7 +652,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     if (q->group_expert) {
         if (!f32 && q->tile_groups == 8) {
             // Rows an expert has on average, from how many groups route leaves room for: a run per expert more than the
-            // pairs fill.  Up to 48 the product is a stream of the experts' weights that reads the rows that there are, and
+            // pairs fill.  Weights that mix_gemm_runs_kernel is not for: up to 48 the product is a stream of them that reads the rows that there are, and
             // an expert's weights pass once, against a tile of 128 rows, most of them empty (us, stream / tile: 64
             // experts, 2048 -> 1024 at 48 rows 58 / 88, 1024 -> 2048 62 / 83; 4096 -> 384 48 / 63; 128 experts, 2048 ->
             // 768 85 / 128; 32 experts, 2048 -> 512 17.5 / 28.8, 4096 -> 4096 226 / 229; 8 experts, 4096 -> 14 336 202 /
@@ -653,7 +674,21 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
             // 42.1 / 52.2, 32 42.4 / 46.2 and 71.4 / 75.9).  By XCD the narrowest end at 68 (64 experts, 4096 -> 384
             // at 66 rows 62.5 / 63.7, at 72 70.3 / 64.8; -> 256 at 80 66 / 57; -> 512 96 / 113).
             // As many runs as experts, or fewer, are not route's: the caller counted them, so they may be full.
-            const uint64_t runs = a.groups / 8, e = q->w->batch, spare = runs > e ? (runs - e) * 128 : 0;
+            const uint64_t runs = a.groups / 8, e = q->w->batch, spare = runs > e ? (runs - e) * 128 : 0, mib = e * a.ntiles * a.ktiles >> 10;
+            // Large weights have a kernel of their own, from 44 rows an expert where they are less than 160 MiB (24 experts, 1408 ->
+            // 2048 at 20 rows 30.7 / 31.6, 128, 1024 -> 384 at 41 26.2 / 27.2, us, below / this).  Tiles of 128 rows take over where their
+            // columns share out evenly over the XCDs: at 104 rows (4096 -> 4096 of 32 experts at 96 rows, this / tiles: 241 / 263, at
+            // 128 327 / 312; 1536 -> 4096 of 16 at 112 70 / 64), many experts of few weights at 144 (64, 1024 -> 2048 at 128 89 / 97; 60, 1408 ->
+            // 2048 at 128 120 / 127, at 150 136 / 134), short input ranges at 72 (512 -> 2048 at 96 56 / 52); others are slower
+            // in tiles at any number (768 outputs of 128 experts at 128 rows 132 / 184, 1536 of 64 at 384 375 / 400).
+            // Beyond 96 rows sixteen tiles to a workgroup, unless they come out badly (64 experts, 2048 -> 1024 at 256 rows, eight /
+            // sixteen: 138 / 132; 128 experts, 768 outputs 194 / 180; 384 outputs 109 / 145).
+            if (runs <= kMixMaxPieces && spare >= e * (mib < 160 ? 44 : 1) && streams(a, e)) {
+                const uint64_t most = a.ktiles <= 16 ? 72 : a.ntiles % 128 ? 1u << 20 : e >= 48 && a.ntiles * a.ktiles <= 6144 ? 144 : 104;
+                const bool wide = (a.ntiles + 15) / 16 * 16 * 10 <= a.ntiles * 11;
+                if (spare <= e * most) return spare > e * 96 && wide ? launch_stream<2, 8, 2, false>(a, e) : launch_stream<2, 4, 4, false>(a, e);
+                return launch_lds<4>(a, 1);
+            }
             if (spare && spare <= e * 48 && a.ktiles <= 32) return launch_runs<4>(a, q->w->batch);
             const uint64_t columns = (a.ntiles + 7) / 8, rounds = (e * columns + g.n_cus - 1) / g.n_cus;
             const uint64_t eighths = columns == 16 && rounds <= 3 && a.ktiles != 32 && a.ktiles != 64 ? e * columns * 8 / (rounds * g.n_cus) : 0;
@@ -664,6 +699,16 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
             return launch_lds<4>(a, 1);
         }
         if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 8, true>(a, 1);
+        const uint64_t e = q->w->batch, spare = a.groups > e ? (a.groups - e) * 16 : 0;
+        if (a.groups <= kMixMaxPieces && streams(a, e)) {
+            // From so many rows an expert (us, without / with, as below): in order 12, 20 where the weights are less than 160 MiB (16
+            // experts, 1408 -> 2048 at 13 rows 18.8 / 20.9) and 24 over short ranges (64, 512 -> 2048 at 17 30.6 / 33.5); picked
+            // one by one, which all workgroups of the others do again, 4 (64, 2048 -> 1024 47 / 43; 32, 4096 -> 4096 182 / 167), 10 with
+            // few experts (16, 2048 -> 4096 at 4 rows 42 / 46, at 11 49 / 46), 8 over short ranges (64, 512 -> 2048 31 / 32 at 6, 35 / 33 at 9).
+            const uint64_t from = a.x_perm ? (a.ktiles < 32 ? 8 : e >= 32 || a.ktiles >= 128 ? 4 : 10)
+                                           : a.ktiles < 32 ? 24 : e * a.ntiles * a.ktiles >> 10 >= 160 ? 12 : 20;
+            if (spare >= e * from) return launch_stream<2, 4, 4, true>(a, e);
+        }
         if (!gated && a.ntiles * a.groups < 384) return launch_split<false, 1, 1, 4, 8, true>(a, 1);   // (as one group of rows below)
         // Sixteen rows an expert and more, from how many groups route leaves room for, fill a second group here and
         // there, which came with the weights once more: the groups of an expert that stand together, four at most, are one
