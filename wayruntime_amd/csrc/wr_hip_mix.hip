@@ -319,7 +319,11 @@ int wr_hip_mix_step_set(wr_hip_mix_step* s, const wr_hip_mix_pool* pool, uint32_
 
 static int launch_residual(int f32, bool embed, const MixRowArgs& a)
 {
-    const bool many = a.rows >= 64, held = a.wpad <= 4096, pair = a.pair_y[0] != nullptr;
+    // Four rows to a workgroup only where their shares of a fragment's 64-byte pieces are worth more than workgroups are: not without
+    // one, and not for so few rows that compute units stay without (width 2048, us, four / one: 512 rows 5.7 / 5.2, 700 5.9 / 6.2,
+    // 2047 10.8 / 15.3; with six experts' rows to add 100 rows 10.8 / 5.1, 512 12.1 / 7.9, 1500 22.6 / 18.7, 2047 24.0 / 26.1; without
+    // a fragment 512 11.0 / 5.1, 2047 22.4 / 20.7).
+    const bool many = a.next && a.rows >= (a.top ? 1792u : 600u), held = a.wpad <= 4096, pair = a.pair_y[0] != nullptr;
     const dim3 g1(a.rows), b1(MixRowShape<1>::kThreads), g4((a.rows + 3) / 4), b4(MixRowShape<4>::kThreads);
 #define WR_RESID(F, EMB, PAIR)                                                                   \
     do {                                                                                         \
