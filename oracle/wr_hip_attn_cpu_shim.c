@@ -454,8 +454,10 @@ int wr_hip_proj_rows_gated_dev(const wr_hip_weight *w, uint32_t rows, const floa
 }
 int wr_hip_attn_rows_d2h(uint32_t n, float *const *dst, const float *src, size_t row_floats)
 {
-    (void)n; (void)dst; (void)src; (void)row_floats;
-    return WR_HIP_ERR_STATE;
+    /* the launch waits for what is ahead of it, and does not run behind a failure */
+    if (wr_hip_attn_sync() != WR_HIP_OK) return WR_HIP_ERR_INTERNAL;
+    for (uint32_t i = 0; i < n; i++) memcpy(dst[i], src + i * row_floats, row_floats * sizeof(float));
+    return WR_HIP_OK;
 }
 int wr_hip_proj_embed_dev(const wr_hip_weight *w, uint32_t rows, const uint32_t *tokens, float scale, float *x, uint32_t ldx)
 {

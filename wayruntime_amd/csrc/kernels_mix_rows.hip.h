@@ -75,6 +75,24 @@ __device__ __forceinline__ void mix_store_unit(void* h, size_t unit, const float
     reinterpret_cast<typename MixAct<F32>::V8*>(h)[unit] = o;
 }
 
+// A step's descriptors, from page-locked memory: the parts of it that the step uses.  A copy would go through another engine,
+// and the step's first launch wait for that one's signal (sixteen rows, logits by launch too: 458 us a step, 408
+// so).  Bound by the link's latency.
+constexpr uint32_t kStepParts = 11;
+struct MixStepUpArgs {
+    const uint64_t* host;
+    uint64_t* dev;
+    uint32_t at[kStepParts], n[kStepParts];                // in units of eight bytes
+};
+
+__global__ __launch_bounds__(256) void mix_step_up_kernel(const MixStepUpArgs a)
+{
+    const uint64_t* s = a.host + a.at[blockIdx.y];
+    uint64_t* d = a.dev + a.at[blockIdx.y];
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < a.n[blockIdx.y]; i += gridDim.x * 256)
+        d[i] = __hip_atomic_load(s + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // (past what a cache holds of an earlier step)
+}
+
 struct MixRowArgs {
     uint32_t rows, width, wpad;      // wpad: width padded to 32, the row stride of x, y, add and the norms
     float eps;

@@ -303,8 +303,29 @@ int wr_hip_mix_step_set(wr_hip_mix_step* s, const wr_hip_mix_pool* pool, uint32_
     }
     memcpy(s->h<uint32_t>(s->o_tokens), tokens, rows * 4);
     if (n_want) memcpy(s->h<uint32_t>(s->o_want), want_rows, (size_t)n_want * 4);
-    HIP_TRY(hipMemcpyAsync(s->dev, s->host, s->o_pages + (size_t)page * 4, hipMemcpyHostToDevice, cx->stream),
-            "step descriptors", 0);
+    MixStepUpArgs up = {};
+    up.host = reinterpret_cast<const uint64_t*>(s->host);
+    up.dev = reinterpret_cast<uint64_t*>(s->dev);
+    uint32_t parts = 0, most = 0;
+    auto part = [&](size_t at, size_t bytes) {
+        if (!bytes) return;
+        up.at[parts] = (uint32_t)(at / 8);
+        up.n[parts] = (uint32_t)((bytes + 7) / 8);         // (parts begin at multiples of 256 bytes)
+        most = std::max(most, up.n[parts++]);
+    };
+    part(s->o_tokens, rows * 4);
+    part(s->o_seq, rows * 4);
+    part(s->o_pos, rows * 4);
+    part(s->o_want, (size_t)n_want * 4);
+    part(s->o_seqs, n_seq * sizeof(MixSeq));
+    part(s->o_chunks, chunk * sizeof(MixChunk));
+    part(s->o_all, (size_t)n_seq * 4);
+    part(s->o_short, (size_t)n_short * 4);
+    part(s->o_long, (size_t)n_long * 4);
+    part(s->o_short_rows, short_rows * sizeof(LatentRow));
+    part(s->o_pages, (size_t)page * 4);
+    hipLaunchKernelGGL(mix_step_up_kernel, dim3(std::min((most + 255) / 256, 64u), parts), dim3(256), 0, cx->stream, up);
+    HIP_TRY(hipGetLastError(), "step descriptors", 0);
     s->rows = (uint32_t)rows;
     s->n_seq = n_seq;
     s->n_want = n_want;

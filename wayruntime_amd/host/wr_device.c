@@ -315,7 +315,7 @@ float *wrh_logits_acquire(wr_model *m)
     pthread_mutex_lock(&m->lock);
     if (m->n_logit_rows) row = m->logit_rows[--m->n_logit_rows];
     pthread_mutex_unlock(&m->lock);
-    return row ? row : wr_hip_attn_host_alloc((size_t)m->vocab * sizeof(float));
+    return row ? row : wr_hip_attn_host_alloc((((size_t)m->vocab + 15) & ~(size_t)15) * sizeof(float));
 }
 
 void wrh_logits_release(wr_model *m, float *row)

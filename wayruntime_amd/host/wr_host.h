@@ -157,7 +157,8 @@ struct wr_session {
     struct wrh_mix_session *mix;             /* mixer-stack model: pages and state slot in the model's pool (no kv, ws1, ds1) */
     wr_hip_kv      *kv;                      /* device cache */
     uint32_t        kv_rows[WRH_MAX_LAYERS]; /* per-layer cursor (the reference's valid_rows) */
-    float          *logits;                  /* [vocab]; device walk: page-locked, from the model (wrh_logits_acquire) */
+    float          *logits;                  /* [vocab]; device walk, mixer stacks: page-locked, from the model (wrh_logits_acquire) */
+    int             logits_locked;           /* mixer stacks: 0 where there was no page-locked memory for them */
     wrh_workspace   ws1;                     /* one-row scratch for wr_step */
     wrh_devspace    ds1;                     /* its device counterpart (device walk only) */
 };
@@ -204,10 +205,12 @@ wr_status wrh_forward_rows_device(wr_model *m, wrh_workspace *hs, wrh_devspace *
 wr_status wrh_mix_session_create(wr_model *m, wr_session *s);
 void      wrh_mix_session_destroy(wr_session *s);
 /* Where a step's logits go, host, in the order of the entries and of `want`: rows of a block
- * [sum of n_want][vocab], or with `rows` a pointer for each. */
+ * [sum of n_want][vocab], or with `rows` a pointer for each; `locked`: all of them, up to
+ * WR_BATCH_MAX, are wrh_logits_acquire's, and a launch writes them.  (It runs only where everything ahead of it did.) */
 typedef struct wrh_logit_rows {
     float        *block;
     float *const *rows;
+    int           locked;
 } wrh_logit_rows;
 /* The sessions are locked and checked; positions advance on success and nothing
  * changes otherwise, logits included where the step wants one row per entry

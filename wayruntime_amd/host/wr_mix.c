@@ -778,7 +778,8 @@ static void hand_out(const wr_model *m, uint32_t n, const uint32_t *dest, const 
 
 /* Logits of the step's wanted rows, packed in h's rows after the final norm; row i belongs where `dest[i]` is in
  * `out`.  The rows come down in one copy per product.  The last product's, all there are in a step of single tokens,
- * stay in the block for the caller to hand out once the step is known to have worked; *rest is how many. */
+ * stay in the block for the caller to hand out once the step is known to have worked; *rest is how many.  Page-locked rows,
+ * one for each wanted place, are written by a launch instead. */
 static wr_status walk_logits(wr_model *m, const walk *w, uint32_t n_want, const uint32_t *dest, const wrh_logit_rows *out,
                              uint32_t *rest)
 {
@@ -794,6 +795,13 @@ static wr_status walk_logits(wr_model *m, const walk *w, uint32_t n_want, const 
         const wr_hip_mix_gemm head = {.w = mm->head, .x = x, .x_kt = wkt, .rows = *rest, .out = WR_HIP_MIX_OUT_ROWS_F32,
                                       .y_f32 = mm->logits_dev, .ldy = mm->vocab_p, .scale = mm->logit_scale};
         TRY(wr_hip_mix_gemm_run(mm->f32, &head), "head");
+        if (out->locked && *rest == n_want) {              /* straight to the sessions' rows */
+            float *rows[WR_BATCH_MAX];
+            for (uint32_t i = 0; i < n_want; i++) rows[i] = out->rows[dest[i]];
+            TRY(wr_hip_attn_rows_d2h(n_want, rows, mm->logits_dev, mm->vocab_p), "logits down");
+            *rest = 0;
+            break;
+        }
         TRY(wr_hip_attn_d2h(mm->logits_host, mm->logits_dev, (size_t)*rest * mm->vocab_p * sizeof(float)), "logits down");
     }
     return WR_OK;

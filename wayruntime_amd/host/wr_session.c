@@ -340,8 +340,16 @@ static void kv_rollback(wr_session *s)
 
 static void free_logits(wr_session *s)
 {
-    if (s->model->dev) wrh_logits_release(s->model, s->logits);
+    if (s->model->dev || s->logits_locked) wrh_logits_release(s->model, s->logits);
     else free(s->logits);
+}
+
+static int mix_logits(wr_session *s)
+{
+    s->logits = wrh_logits_acquire(s->model);
+    s->logits_locked = s->logits != NULL;
+    if (!s->logits) s->logits = malloc((size_t)s->model->vocab * sizeof(float));
+    return s->logits != NULL;
 }
 
 static wr_status session_register(wr_model *m, wr_session *s, wr_session **out)
@@ -380,8 +388,7 @@ wr_status wr_session_create(wr_model *m, const wr_session_params *params, wr_ses
             free(s);
             return st;
         }
-        s->logits = malloc((size_t)m->vocab * sizeof(float));
-        if (!s->logits) {
+        if (!mix_logits(s)) {
             wrh_mix_session_destroy(s);
             free(s);
             return WR_ERR_NOMEM;
@@ -450,7 +457,7 @@ const float *wr_step(wr_session *s, uint32_t token)
     } else if (m->mix) {
         const uint32_t first = 0;
         const wr_step_entry q = {s, &token, 1, 1, &first};
-        const wrh_logit_rows to = {s->logits, NULL};
+        const wrh_logit_rows to = {NULL, &s->logits, s->logits_locked};
         st = wrh_mix_step(m, &q, 1, &to, take_fail_layer(m));
     } else {
         wr_session *one[1] = {s};
@@ -549,13 +556,22 @@ static void sort_by_address(wr_session **a, uint32_t n)
 }
 
 /* Locks the entries' sessions, runs them as one step and publishes the status. */
-static wr_status locked_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, const wrh_logit_rows *logits)
+static wr_status locked_mix_step(wr_model *m, const wr_step_entry *entries, uint32_t n, float *block, int own_rows)
 {
     wr_session *locked[WR_BATCH_MAX];
     for (uint32_t i = 0; i < n; i++) locked[i] = entries[i].session;
     sort_by_address(locked, n);
     for (uint32_t i = 0; i < n; i++) pthread_mutex_lock(&locked[i]->lock);
-    const wr_status st = wrh_mix_step(m, entries, n, logits, take_fail_layer(m));
+    float *rows[WR_BATCH_MAX];
+    wrh_logit_rows to = {block, NULL, 0};
+    if (own_rows) {                                        /* one row a session, where the sessions keep them */
+        to = (wrh_logit_rows){NULL, rows, 1};
+        for (uint32_t i = 0; i < n; i++) {
+            rows[i] = entries[i].session->logits;
+            if (!entries[i].session->logits_locked) to.locked = 0;
+        }
+    }
+    const wr_status st = wrh_mix_step(m, entries, n, &to, take_fail_layer(m));
     for (uint32_t i = 0; i < n; i++) __atomic_store_n(&entries[i].session->last_status, st, __ATOMIC_RELEASE);
     for (uint32_t i = n; i > 0; i--) pthread_mutex_unlock(&locked[i - 1]->lock);
     return st;
@@ -567,12 +583,9 @@ static int batch_step_mix(wr_model *m, wr_session *const *sessions, const uint32
     static const uint32_t first = 0;
     wr_step_entry q[WR_BATCH_MAX];
     for (uint32_t i = 0; i < n; i++) q[i] = (wr_step_entry){sessions[i], tokens + i, 1, 1, &first};
-    float *rows[WR_BATCH_MAX];
-    for (uint32_t i = 0; i < n; i++) rows[i] = sessions[i]->logits;
-    const wrh_logit_rows to = {NULL, rows};
-    const wr_status st = locked_mix_step(m, q, n, &to);
+    const wr_status st = locked_mix_step(m, q, n, NULL, 1);
     for (uint32_t i = 0; i < n && st == WR_OK; i++)
-        if (logits_out) logits_out[i] = rows[i];
+        if (logits_out) logits_out[i] = sessions[i]->logits;
     return (st == WR_OK) ? (int)n : (int)st;
 }
 
@@ -657,8 +670,7 @@ int wr_mixed_step(const wr_step_entry *entries, uint32_t n, float *logits)
     }
     if (wanted && !logits) return WR_ERR_INVAL;
     if (wanted > 0x7FFFFFFFu) return WR_ERR_LIMIT;
-    const wrh_logit_rows to = {logits, NULL};
-    const wr_status st = m->mix ? locked_mix_step(m, entries, n, &to) : mixed_step_owned(entries, n, logits);
+    const wr_status st = m->mix ? locked_mix_step(m, entries, n, logits, 0) : mixed_step_owned(entries, n, logits);
     return (st == WR_OK) ? (int)wanted : (int)st;
 }
 
