@@ -222,6 +222,26 @@ def test_every_tile_of_many_rows(lib, N, K, rows):
         b.free()
 
 
+# tiles of 256 outputs by 256 and 128 rows: odd and even numbers of k-steps, a last tile of outputs that is not full, gated and not
+@pytest.mark.parametrize("N,rows,K", [(32768 + 64, 400, 1056), (16384 + 64, 1000, 2048), (4144, 1800, 2080), (4096 + 64, 2047, 4160)])
+def test_pipelined_tiles_of_many_rows(lib, N, rows, K):
+    r = Run(lib, False, 1, N, K, rows)
+    x = r.act(rows, K)
+    xd, y = r.up(x), hipattn.DeviceBuffer(rows * N * 4)
+    r.go(xd, out=ROWS_F32, y_f32=y.p, ldy=N)
+    want = x.astype(np.float64) @ r.w[0].T.astype(np.float64)
+    r.close(y.to_host((rows, N)), want)
+    if N % 64 == 0:
+        h = hipattn.DeviceBuffer(-(-rows // 16) * 16 * N)
+        r.go(xd, out=GATED, h=h.p, h_kt=N // 64)
+        t = want.reshape(rows, N // 32, 2, 16)
+        r.close(r.frag_down(h, rows, N // 2), (O.silu(t[:, :, 0]) * t[:, :, 1]).reshape(rows, -1), eight_bits=True)
+        h.free()
+    r.end()
+    for b in (xd, y):
+        b.free()
+
+
 @pytest.mark.parametrize("N,K", [(16, 4096), (2048, 4128), (80, 8192), (2064, 4096), (48, 4064)])
 def test_two_workgroups_to_a_tile(lib, N, K):
     # narrow weights over long inputs, up to sixteen rows: one tile, as many as a launch holds, an odd number of k-steps;

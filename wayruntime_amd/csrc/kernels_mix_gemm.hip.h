@@ -628,22 +628,31 @@ __global__ __launch_bounds__(WAVES * 64, 2) void mix_gemm_runs_kernel(const MixG
 // the lower half's.  For launches of one workgroup per compute unit and a long input
 // range: twice the waves per SIMD, half the chain.
 // 2047 rows, 8192 -> 2048, GROUPS 4: 93 -> 73 us; 1000 rows, GROUPS 2: 80 -> 55.
-template <int GROUPS, int KS = 1>
-constexpr size_t mix_gemm_lds_bytes() { return (size_t)(KS == 2 ? 8 : 3) * (8 + 2 * GROUPS) * 1024; }
+//
+// WN = 4: eight waves, 256 outputs, a ring of five stages (160 KiB) and a barrier for two k-steps; a step goes by quarters, a copy,
+// then reads of the next step's operands among the products.  Bound by the matrix pipes at the clock the device grants them:
+// a full device's step of 256 x 256 x 32 is 0.78 us, 0.51 of it products at 2.05 GHz, on 64 units alone 0.56 (2.4 GHz).  4095 rows,
+// 8192 -> 4096 216 -> 194 us (1.42 PFLOP/s).  On the way there: operands read behind the barrier and a barrier a step 0.83, read a step ahead
+// 0.80, the copies among the products 0.78.
+template <int GROUPS, int KS = 1, int WN = 2>
+constexpr int mix_gemm_ring() { return WN == 4 ? 5 : KS == 2 ? 4 : 3; }
+template <int GROUPS, int KS = 1, int WN = 2>
+constexpr size_t mix_gemm_lds_bytes() { return (size_t)KS * mix_gemm_ring<GROUPS, KS, WN>() * (4 * WN + 2 * GROUPS) * 1024; }
 
-template <int GROUPS, int KS = 1>
-__global__ __launch_bounds__(256 * KS, KS == 2 ? 1 : 2) void mix_gemm_lds_kernel(const MixGemmArgs a)
+template <int GROUPS, int KS = 1, int WN = 2>
+__global__ __launch_bounds__(128 * WN * KS, KS == 2 || WN == 4 ? 1 : 2) void mix_gemm_lds_kernel(const MixGemmArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char mix_smem[];
-    constexpr int NT = 4, CHUNKS = 8 + 2 * GROUPS, CPW = CHUNKS / 4, RING = KS == 2 ? 4 : 3;
-    static_assert(CHUNKS % 4 == 0, "every wave copies the same number of chunks");
+    constexpr int NT = 4, WAVES = 2 * WN, TILES = WN * NT, CHUNKS = TILES + 2 * GROUPS, CPW = CHUNKS / WAVES, RING = mix_gemm_ring<GROUPS, KS, WN>();
+    static_assert(CHUNKS % WAVES == 0, "every wave copies the same number of chunks");
+    static_assert(WN == 2 || KS == 1);
     constexpr uint32_t STAGE = CHUNKS * 1024;
     const int lane = threadIdx.x & 63;
     const uint32_t wave_wg = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t kh = wave_wg / 4, wave = wave_wg % 4;   // half of the input range, wave of the set
-    const uint32_t wn = wave & 1, wr = wave >> 1;
+    const uint32_t kh = wave_wg / WAVES, wave = wave_wg % WAVES;   // half of the input range, wave of the set
+    const uint32_t wn = wave % WN, wr = wave / WN;
     const uint32_t ktiles = a.ktiles / KS;                 // this set's k-steps
-    const uint32_t nx = (a.ntiles + 7) / 8, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS), z = blockIdx.y;
+    const uint32_t nx = (a.ntiles + TILES - 1) / TILES, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS), z = blockIdx.y;
     uint32_t px, py;
     if (!a.group_expert) {
         if (!xcd_tile(blockIdx.x, a.cols, nx, ny, px, py)) return;
@@ -658,7 +667,7 @@ __global__ __launch_bounds__(256 * KS, KS == 2 ? 1 : 2) void mix_gemm_lds_kernel
         py = few ? blockIdx.x / nx : slot / side % ny;
         if (px >= nx) return;
     }
-    const uint32_t nt_wg = px * 8, g_wg = py * 2 * GROUPS;
+    const uint32_t nt_wg = px * TILES, g_wg = py * 2 * GROUPS;
     uint32_t mat = z;
     if (a.group_expert) {
         const int e = a.group_expert[g_wg];
@@ -672,10 +681,10 @@ __global__ __launch_bounds__(256 * KS, KS == 2 ? 1 : 2) void mix_gemm_lds_kernel
     for (int i = 0; i < CPW; i++) {
         const uint32_t c = wave * CPW + i;
         const unsigned char* p =
-            c < 8 ? reinterpret_cast<const unsigned char*>(a.w) +
+            c < TILES ? reinterpret_cast<const unsigned char*>(a.w) +
                         ((size_t)mat * a.ntiles + min(nt_wg + c, a.ntiles - 1)) * a.ktiles * 1024
                   : reinterpret_cast<const unsigned char*>(a.x) +
-                        ((size_t)min(g_wg + c - 8, a.groups - 1) * a.x_kt + (size_t)z * a.x_kt_z) * 1024;
+                        ((size_t)min(g_wg + c - TILES, a.groups - 1) * a.x_kt + (size_t)z * a.x_kt_z) * 1024;
         src[i] = uniform_ptr(p + (size_t)kh * ktiles * 1024);
     }
     const uint32_t lane_off = lane * 16;
@@ -694,7 +703,7 @@ __global__ __launch_bounds__(256 * KS, KS == 2 ? 1 : 2) void mix_gemm_lds_kernel
 
 #pragma unroll
     for (int st0 = 0; st0 < RING - 1; st0++) issue(st0);
-    const uint32_t w_off = wn * NT * 1024 + lane * 16, x_off = (8 + wr * GROUPS) * 1024 + lane * 16;
+    const uint32_t w_off = wn * NT * 1024 + lane * 16, x_off = (TILES + wr * GROUPS) * 1024 + lane * 16;
     auto read_ops = [&](bf16x8 (&wv)[NT], bf16x8 (&xv)[GROUPS], uint32_t kt) {
         const unsigned char* st = mix_smem + ((kt % RING) * KS + kh) * STAGE;
 #pragma unroll
@@ -708,7 +717,48 @@ __global__ __launch_bounds__(256 * KS, KS == 2 ? 1 : 2) void mix_gemm_lds_kernel
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(wv[t], xv[i], acc[t][i]);
     };
-    if constexpr (KS == 2) {
+    if constexpr (WN == 4) {
+        bf16x8 w0[NT], x0[GROUPS], w1[NT], x1[GROUPS];
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(CPW * (RING - 2)) : "memory");
+        read_ops(w0, x0, 0);
+        // Two steps to a barrier: stages kt + 1 and kt + 2 have landed, kt + 3 may be in flight, kt + 4 and kt + 5 go where kt - 1 and
+        // kt were, whose reads are over.  (Left alone, the compiler puts most reads behind the products and waits for each
+        // few, and copies issued together keep a SIMD's two waves from the matrix pipe at the same time.)
+        static_assert(GROUPS % NT == 0 && CPW <= NT, "a quarter's share");
+        auto step = [&](const bf16x8 (&wv)[NT], const bf16x8 (&xv)[GROUPS], bf16x8 (&wn_)[NT], bf16x8 (&xn)[GROUPS], uint32_t k) {
+            constexpr int Q = NT, PER = GROUPS / Q;        // quarters of a step
+            const size_t from = (size_t)min(k + RING - 1, klast) * 1024;
+            const uint32_t to = lds0 + (k + RING - 1) % RING * STAGE + wave * CPW * 1024;
+            const unsigned char* st = mix_smem + (k + 1) % RING * STAGE;
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (q < CPW) lds_direct_load(to + q * 1024, src[q] + from, lane_off);
+                __builtin_amdgcn_sched_barrier(0);
+                wn_[q] = *reinterpret_cast<const bf16x8*>(st + w_off + q * 1024);
+#pragma unroll
+                for (int i = 0; i < PER; i++) xn[q * PER + i] = *reinterpret_cast<const bf16x8*>(st + x_off + (q * PER + i) * 1024);
+#pragma unroll
+                for (int i = 0; i < PER; i++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++) acc[t][q * PER + i] = mix_mfma(wv[t], xv[q * PER + i], acc[t][q * PER + i]);
+#pragma unroll
+                for (int i = 0; i < 1 + PER; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, NT * PER / (1 + PER), 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        uint32_t kt = 0;
+        for (; kt + 2 <= ktiles; kt += 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(CPW * (RING - 4)) : "memory");
+            step(w0, x0, w1, x1, kt);
+            step(w1, x1, w0, x0, kt + 1);
+        }
+        if (kt < ktiles) multiply(w0, x0);
+    } else if constexpr (KS == 2) {
         bf16x8 w0[NT], x0[GROUPS], w1[NT], x1[GROUPS];
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(CPW * (RING - 2)) : "memory");
         read_ops(w0, x0, 0);

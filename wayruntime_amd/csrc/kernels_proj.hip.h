@@ -1441,8 +1441,8 @@ __global__ __launch_bounds__(kProjThreads, GROUPS * NT == 8 ? 3 : 2) void proj_g
 // the chip with the large one.
 // WN = waves side by side along the outputs (2 or 4; two wave rows always),
 // RING = stages.  <8, 2, 3>: the tile above.  <4, 2, 3>: 128 x 64 for products
-// with too few rows to fill the chip with the large one.  <8, 4, 4>: eight
-// waves, 256 outputs x 128 rows, 32 KiB per stage copied three k-steps ahead,
+// with too few rows to fill the chip with the large one.  <8, 4, 5>: eight
+// waves, 256 outputs x 128 rows, 32 KiB per stage copied four k-steps ahead,
 // one workgroup per CU: a third fewer bytes per MFMA than the four-wave tile.
 template <int GROUPS, int WN, int RING, int KS = 1>
 constexpr size_t gemm_lds_bytes()
@@ -1453,7 +1453,11 @@ constexpr size_t gemm_lds_bytes()
 // PIPE: the operand reads of the next k-step are issued before this one's MFMAs
 // (two register sets), for launches that leave a SIMD with a single wave and
 // nobody else to cover its LDS latency; needs one more ring stage, because a
-// stage is now read one k-step before it is used.
+// stage is now read one k-step before it is used.  With five stages one barrier does for two
+// k-steps.  A step goes by quarters (copies and reads among the MFMAs).  us, before / now, operand
+// fragments included: 2047 rows, 1024 -> 4096 in <8, 4, 5> 54.1 / 51.7 (read behind a barrier a step in <8, 4, 4>
+// before), 4095 rows gated 1024 -> 2 x 3072 120.7 / 115.3; in <4, 2, 4> with two sets of waves 2047 rows 2048 -> 1024 33.0 / 31.9, 3072 ->
+// 1024 43.3 / 41.3.
 //
 // KS = 2: two such sets of waves in one workgroup, each with its own ring, take
 // one half of the input range each (the host asks for it only when the number of
@@ -1543,15 +1547,46 @@ __global__ __launch_bounds__(128 * WN * KS, (WN == 2 && KS == 1) ? 2 : 1) void p
         // per iteration so that no register set is copied; a step past the end
         // reads a stage that holds a repeat of the last one and is not used.
         uint32_t kt = 0;
+        // A step in quarters, a copy, then reads among the products: left alone, the compiler puts most reads behind the
+        // products and waits for each few, and copies issued together keep a SIMD's two waves from the matrix pipe at
+        // the same time.
+        auto step = [&](const half8 (&wv)[NT], const half8 (&xv)[GROUPS], half8 (&wn_)[NT], half8 (&xn)[GROUPS], uint32_t k) {
+            constexpr int PER = GROUPS / NT;
+            static_assert(GROUPS % NT == 0 && CPW <= NT, "a quarter's share");
+            const size_t from = (size_t)min(k + RING - 1, klast) * 1024;
+            const uint32_t to = lds0 + ((k + RING - 1) % RING * KS + kh) * STAGE + wave * CPW * 1024;
+            const unsigned char* st = gemm_smem + ((k + 1) % RING * KS + kh) * STAGE;
+#pragma unroll
+            for (int q = 0; q < NT; q++) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (q < CPW) lds_direct_load(to + q * 1024, src[q] + from, lane_off);
+                __builtin_amdgcn_sched_barrier(0);
+                wn_[q] = *reinterpret_cast<const half8*>(st + w_off + q * 1024);
+#pragma unroll
+                for (int i = 0; i < PER; i++) xn[q * PER + i] = *reinterpret_cast<const half8*>(st + x_off + (q * PER + i) * 1024);
+#pragma unroll
+                for (int i = 0; i < PER; i++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        acc[t][q * PER + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[t], xv[q * PER + i], acc[t][q * PER + i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 1 + PER; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, NT * PER / (1 + PER), 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        constexpr bool PAIR = RING >= 5;                   // one barrier for two steps
         for (; kt + 2 <= ktiles; kt += 2) {
-            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(CPW * (RING - 3)) : "memory");
-            issue(kt + RING - 1);
-            read_ops(w1, x1, kt + 1);
-            mfmas(w0, x0);
-            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(CPW * (RING - 3)) : "memory");
-            issue(kt + RING);
-            read_ops(w0, x0, kt + 2);
-            mfmas(w1, x1);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (PAIR)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(CPW * (RING - 4)) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(CPW * (RING - 3)) : "memory");
+            step(w0, x0, w1, x1, kt);
+            if constexpr (!PAIR) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(CPW * (RING - 3)) : "memory");
+            step(w1, x1, w0, x0, kt + 1);
         }
         if (kt < ktiles) mfmas(w0, x0);                   // odd number of k-steps
     } else

@@ -1015,7 +1015,7 @@ void launch_proj_gemm(const ProjArgs& a, uint32_t groups)
     const bool small_fills_better = n_small >= 512 && n_big * 100 < rounds_b * 512 * 70 &&
                                     (uint64_t)n_small * rounds_b * 100 >= (uint64_t)n_big * rounds_s * 100 + (uint64_t)rounds_b * rounds_s * 512 * 10;
     if (wide_fills)
-        launch_proj_lds<8, 4, 4, false, 1>(a, groups, 32);
+        launch_proj_lds<8, 4, 5, true, 1>(a, groups, 32);
     else if (n_big >= 512 && !small_fills_better)
         launch_proj_lds<8, 2, 3, false, 1>(a, groups, 64);
     else if (panels * ((groups + 7) / 8) >= 512)          // two and more per CU cover each other's latency
@@ -1370,14 +1370,14 @@ int wr_hip_attn_init(int device)
         allow_lds(proj_rows_down_kernel<2>, kOnePerCuLds);
         allow_lds(proj_row1_kernel<kProjSrcRmsNorm, kRow1Gated>, kProjRow1MaxLds);
         allow_lds(proj_row1_kernel<kProjSrcPlain, kRow1Gated>, kProjRow1MaxLds);
+        allow_lds(proj_gemm_lds_kernel<8, 4, 5, true>, gemm_lds_bytes<8, 4, 5>());
+        allow_lds(proj_gemm_lds_kernel<8, 4, 5, true, 1, true>, gemm_lds_bytes<8, 4, 5>());
         allow_lds(proj_gemm_lds_kernel<8, 2, 3>, gemm_lds_bytes<8, 2, 3>());
         allow_lds(proj_gemm_lds_kernel<8, 2, 3, false, 1, true>, gemm_lds_bytes<8, 2, 3>());
         allow_lds(proj_gemm_lds_kernel<4, 2, 4, true>, gemm_lds_bytes<4, 2, 4>());
         allow_lds(proj_gemm_lds_kernel<4, 2, 4, true, 1, true>, gemm_lds_bytes<4, 2, 4>());
         allow_lds(proj_gemm_lds_kernel<4, 2, 4, true, 2>, gemm_lds_bytes<4, 2, 4, 2>());
         allow_lds(proj_gemm_lds_kernel<4, 2, 4, true, 2, true>, gemm_lds_bytes<4, 2, 4, 2>());
-        allow_lds(proj_gemm_lds_kernel<8, 4, 4>, gemm_lds_bytes<8, 4, 4>());
-        allow_lds(proj_gemm_lds_kernel<8, 4, 4, false, 1, true>, gemm_lds_bytes<8, 4, 4>());
         for (uint32_t n_in = 512; n_in <= 3072; n_in += 512)
             for (uint32_t nt = 1; nt <= 4; nt++)
                 for (const int src : {kProjSrcPlain, kProjSrcRmsNorm})

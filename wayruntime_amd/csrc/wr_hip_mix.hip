@@ -542,17 +542,18 @@ static int launch_parts(MixGemmArgs a)
     return WR_HIP_OK;
 }
 
-template <int GROUPS, int KS = 1>
+template <int GROUPS, int KS = 1, int WN = 2>
 static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 {
-    int rc = allow_lds<mix_gemm_lds_kernel<GROUPS, KS>>(mix_gemm_lds_bytes<GROUPS, KS>());
+    constexpr uint32_t TILES = 4 * WN;
+    int rc = allow_lds<mix_gemm_lds_kernel<GROUPS, KS, WN>>(mix_gemm_lds_bytes<GROUPS, KS, WN>());
     if (rc) return rc;
     MixGemmArgs a = args;
-    const uint32_t nx = (a.ntiles + 7) / 8, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
+    const uint32_t nx = (a.ntiles + TILES - 1) / TILES, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
     uint32_t blocks = (nx < 8 ? nx : (nx + 7) / 8 * 8) * ny;
     if (!a.group_expert)
-        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, KS == 2 ? 32 : 64, &blocks);
-    launch_main(mix_gemm_lds_kernel<GROUPS, KS>, dim3(blocks, batch), dim3(256 * KS), a, mix_gemm_lds_bytes<GROUPS, KS>());
+        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, KS == 2 || WN == 4 ? 32 : 64, &blocks);
+    launch_main(mix_gemm_lds_kernel<GROUPS, KS, WN>, dim3(blocks, batch), dim3(128 * WN * KS), a, mix_gemm_lds_bytes<GROUPS, KS, WN>());
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
 }
@@ -566,6 +567,11 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 // before / with them: 2048 -> 2048 at 130 rows 9.2 / 7.2, at 300 13.9 / 9.3; 8192 -> 2048 37.6 / 26.7 at 300; 12 288
 // -> 4096 at 300 111 / 68; 2048 -> 14 400 at 45 27 / 15.3.  The halves: 8192 -> 2048 at 1000 rows 80 / 55, at 2047 93
 // / 73; 4096 -> 2048 at 2047 50 / 41; 12 288 -> 4096 at 1000 153 / 108.
+// The pipelined tiles of 256 outputs x 256 and 128 rows (mix_gemm_lds_kernel, WN = 4; from 1024 inputs on): a full round of one workgroup
+// per unit 0.78 and 0.44, with what its ends cost besides (8 and 5 us, 4 and 3 more where 32-bit rows go out), one that
+// leaves units without a workgroup less, as the others then have the clock and the caches. Against the tile of 128 x 256,
+// whose ends those figures split off too: 2047 rows, 2048 -> 32 768 into 32-bit rows 315 / 266 us, -> 14 400 137 / 114, 4096 -> 24 576 gated
+// 320 / 299; 2500 rows, 2048 -> 16 384, two and a half rounds, 142 / 156: the other tile's.
 // Gated outputs take an even number of tiles: of one group of rows each where that spreads few tiles over more units
 // (64 rows, 8192 -> 512: 17.4 us in tiles of two groups, 13.2; 2048 -> 2048 6.9, 5.7).  Tiles of 256 rows are counted in
 // whole workgroups per unit where all run at once (1500 rows, 256 -> 8192: 17.8 us against 16.3 with tiles of 128;
@@ -574,6 +580,7 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 // time) the form picked is 2.3 % off the best one on average, 30 % (1 us of 4) at worst.
 static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
 {
+    const bool rows32 = a.out == kMixOutRowsF32;
     struct Form {
         uint32_t nt, gr;
         int (*launch)(const MixGemmArgs&, uint32_t);
@@ -588,6 +595,11 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
         int (*launch)(const MixGemmArgs&, uint32_t);
     } lds[] = {{4, 0.34f, 0.177f, launch_lds<2>}, {8, 0.39f, 0.27f, launch_lds<4>}, {16, 0.58f, 0.5f, launch_lds<8>}},
       halves[] = {{4, 0.26f, 0.f, launch_lds<2, 2>}, {8, 0.28f, 0.f, launch_lds<4, 2>}};
+    static const struct {
+        uint32_t groups;
+        float full, part, more, ends, rows32;
+        int (*launch)(const MixGemmArgs&, uint32_t);
+    } piped[] = {{16, 0.78f, 0.50f, 0.26f, 8.f, 4.f, launch_lds<8, 1, 4>}, {8, 0.44f, 0.34f, 0.09f, 5.f, 3.f, launch_lds<4, 1, 4>}};
     int (*best)(const MixGemmArgs&, uint32_t) = nullptr;
     float least = 0.f;
     auto offer = [&](float cost, int (*launch)(const MixGemmArgs&, uint32_t)) {
@@ -605,7 +617,14 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
             const uint64_t wgs = (uint64_t)((a.ntiles + 7) / 8) * ((a.groups + f.groups - 1) / f.groups) * batch;
             const bool at_once = f.groups == 16 && wgs <= 2 * g.n_cus;
             const float each = at_once ? (float)((wgs + g.n_cus - 1) / g.n_cus) : (float)wgs / g.n_cus;
-            offer(std::max(f.step, f.share * each), f.launch);
+            const float share = f.groups == 16 && a.ktiles >= 32 ? 0.435f + (rows32 ? 11.f : 4.f) / (float)a.ktiles : f.share;
+            offer(std::max(f.step, share * each), f.launch);
+        }
+    if (a.groups >= 4 && a.ktiles >= 32)
+        for (const auto& f : piped) {
+            const uint64_t wgs = (uint64_t)((a.ntiles + 15) / 16) * ((a.groups + f.groups - 1) / f.groups) * batch;
+            const float ends = (f.ends + (rows32 ? f.rows32 : 0.f)) / (float)a.ktiles, left = (float)(wgs % g.n_cus) / (float)g.n_cus;
+            offer((float)(wgs / g.n_cus) * (f.full + ends) + (left > 0.f ? f.part + f.more * left + ends + (wgs > g.n_cus ? 0.08f : 0.f) : 0.f), f.launch);
         }
     if (a.groups >= 4 && a.ktiles % 2 == 0 && a.ktiles >= 64)
         for (const auto& f : halves) {
