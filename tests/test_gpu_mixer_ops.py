@@ -174,7 +174,8 @@ def test_frag_split_and_gated_out(lib, f32, N, K, rows):
 
 
 @pytest.mark.parametrize("f32", [False, True])
-@pytest.mark.parametrize("batch,N,K,rows", [(3, 64, 32, 1), (5, 32, 96, 40), (40, 512, 64, 300), (2, 128, 64, 130)])
+@pytest.mark.parametrize("batch,N,K,rows", [(3, 64, 32, 1), (5, 32, 96, 40), (40, 512, 64, 300), (2, 128, 64, 130), (4, 1040, 352, 300), (8, 528, 64, 500), (2, 2080, 352, 700),
+                                            (6, 1040, 96, 300)])
 def test_batch_of_matrices(lib, f32, batch, N, K, rows):
     # matrix z takes its own input columns and writes its own output columns
     r = Run(lib, f32, batch, N, K, rows)

@@ -627,15 +627,24 @@ __global__ __launch_bounds__(WAVES * 64, 2) void mix_gemm_runs_kernel(const MixG
 // one before it is multiplied; the upper half's sums pass through LDS and are added to
 // the lower half's.  For launches of one workgroup per compute unit and a long input
 // range: twice the waves per SIMD, half the chain.
-// 2047 rows, 8192 -> 2048, GROUPS 4: 93 -> 73 us; 1000 rows, GROUPS 2: 80 -> 55.
+// 2047 rows, 8192 -> 2048, GROUPS 4: 93 -> 73 us, by quarters 68; 1000 rows, GROUPS 2: 80 -> 55.  (One barrier for two steps is
+// up to 3 % faster there, and 10 to 17 % slower where weights come from HBM: 700 rows, 12 288 -> 4096 94 / 110.)
 //
-// WN = 4: eight waves, 256 outputs, a ring of five stages (160 KiB) and a barrier for two k-steps; a step goes by quarters, a copy,
-// then reads of the next step's operands among the products.  Bound by the matrix pipes at the clock the device grants them:
+// WN = 4: eight waves, 256 outputs, a ring of five stages (160 KiB) and a barrier for two k-steps; a step goes by quarters (as
+// with KS = 2 and GROUPS 4), a copy, then reads of the next step's operands among the products.  Bound by the matrix pipes at the clock the device grants them:
 // a full device's step of 256 x 256 x 32 is 0.78 us, 0.51 of it products at 2.05 GHz, on 64 units alone 0.56 (2.4 GHz).  4095 rows,
 // 8192 -> 4096 216 -> 194 us (1.42 PFLOP/s).  On the way there: operands read behind the barrier and a barrier a step 0.83, read a step ahead
 // 0.80, the copies among the products 0.78.
+// XCDs that a matrix of a batch is shared out to: as many as there are for each, so that its weights and rows come into
+// those L2s and no others.  us, every XCD for every matrix / so: 2047 rows, four of 2048 -> 2048 68 / 61, 4096 -> 4096 into
+// 32-bit rows 260 / 230; 32 of 512 -> 128 23 / 19.5, at 1000 rows 16.5 / 12.8.  (Other numbers than 2, 4 and multiples of eight would leave XCDs without one.)
+__host__ __device__ __forceinline__ uint32_t mix_batch_xcds(uint32_t batch)
+{
+    return batch % 8 == 0 ? 1u : batch == 2 || batch == 4 ? 8 / batch : 8u;
+}
+
 template <int GROUPS, int KS = 1, int WN = 2>
-constexpr int mix_gemm_ring() { return WN == 4 ? 5 : KS == 2 ? 4 : 3; }
+constexpr int mix_gemm_ring() { return WN == 4 || (KS == 2 && GROUPS == 4) ? 5 : KS == 2 ? 4 : 3; }
 template <int GROUPS, int KS = 1, int WN = 2>
 constexpr size_t mix_gemm_lds_bytes() { return (size_t)KS * mix_gemm_ring<GROUPS, KS, WN>() * (4 * WN + 2 * GROUPS) * 1024; }
 
@@ -652,9 +661,14 @@ __global__ __launch_bounds__(128 * WN * KS, KS == 2 || WN == 4 ? 1 : 2) void mix
     const uint32_t kh = wave_wg / WAVES, wave = wave_wg % WAVES;   // half of the input range, wave of the set
     const uint32_t wn = wave % WN, wr = wave / WN;
     const uint32_t ktiles = a.ktiles / KS;                 // this set's k-steps
-    const uint32_t nx = (a.ntiles + TILES - 1) / TILES, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS), z = blockIdx.y;
-    uint32_t px, py;
-    if (!a.group_expert) {
+    const uint32_t nx = (a.ntiles + TILES - 1) / TILES, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS), batch = gridDim.y;
+    uint32_t px, py, z = 0;
+    if (!a.group_expert && batch > 1) {                    // a batch: XCDs share out its matrices (mix_batch_xcds), or each of them the tiles
+        const uint32_t id = blockIdx.y * gridDim.x + blockIdx.x, n = mix_batch_xcds(batch), xcd = id % 8, slot = id / 8;
+        const uint32_t at = n == 8 ? blockIdx.x / 8 : slot % (gridDim.x / n);
+        z = n == 8 ? blockIdx.y : slot / (gridDim.x / n) * (8 / n) + xcd / n;
+        if (!xcd_tile_of(xcd % n, at, n, a.cols, nx, ny, px, py)) return;
+    } else if (!a.group_expert) {
         if (!xcd_tile(blockIdx.x, a.cols, nx, ny, px, py)) return;
     } else {
         // XCD x takes the output panels x, x + 8, ...: up to four side by side through all row panels, so that the rows
@@ -717,19 +731,19 @@ __global__ __launch_bounds__(128 * WN * KS, KS == 2 || WN == 4 ? 1 : 2) void mix
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[t][i] = mix_mfma(wv[t], xv[i], acc[t][i]);
     };
-    if constexpr (WN == 4) {
+    if constexpr (RING == 5) {
         bf16x8 w0[NT], x0[GROUPS], w1[NT], x1[GROUPS];
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(CPW * (RING - 2)) : "memory");
         read_ops(w0, x0, 0);
-        // Two steps to a barrier: stages kt + 1 and kt + 2 have landed, kt + 3 may be in flight, kt + 4 and kt + 5 go where kt - 1 and
-        // kt were, whose reads are over.  (Left alone, the compiler puts most reads behind the products and waits for each
+        // PAIR, two steps to a barrier: stages kt + 1 and kt + 2 have landed, kt + 3 may be in flight, kt + 4 and kt + 5 go where
+        // kt - 1 and kt were, whose reads are over.  One: kt + 1 has landed, kt + 2 and kt + 3 may be in flight.  (Left alone, the compiler puts most reads behind the products and waits for each
         // few, and copies issued together keep a SIMD's two waves from the matrix pipe at the same time.)
         static_assert(GROUPS % NT == 0 && CPW <= NT, "a quarter's share");
         auto step = [&](const bf16x8 (&wv)[NT], const bf16x8 (&xv)[GROUPS], bf16x8 (&wn_)[NT], bf16x8 (&xn)[GROUPS], uint32_t k) {
             constexpr int Q = NT, PER = GROUPS / Q;        // quarters of a step
             const size_t from = (size_t)min(k + RING - 1, klast) * 1024;
-            const uint32_t to = lds0 + (k + RING - 1) % RING * STAGE + wave * CPW * 1024;
-            const unsigned char* st = mix_smem + (k + 1) % RING * STAGE;
+            const uint32_t to = lds0 + ((k + RING - 1) % RING * KS + kh) * STAGE + wave * CPW * 1024;
+            const unsigned char* st = mix_smem + ((k + 1) % RING * KS + kh) * STAGE;
 #pragma unroll
             for (int q = 0; q < Q; q++) {
                 __builtin_amdgcn_sched_barrier(0);
@@ -750,11 +764,13 @@ __global__ __launch_bounds__(128 * WN * KS, KS == 2 || WN == 4 ? 1 : 2) void mix
             }
             __builtin_amdgcn_sched_barrier(0);
         };
+        constexpr bool PAIR = WN == 4;
         uint32_t kt = 0;
         for (; kt + 2 <= ktiles; kt += 2) {
             __builtin_amdgcn_sched_barrier(0);
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(CPW * (RING - 4)) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(CPW * (PAIR ? RING - 4 : RING - 3)) : "memory");
             step(w0, x0, w1, x1, kt);
+            if constexpr (!PAIR) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(CPW * (RING - 3)) : "memory");
             step(w1, x1, w0, x0, kt + 1);
         }
         if (kt < ktiles) multiply(w0, x0);

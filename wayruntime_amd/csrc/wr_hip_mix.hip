@@ -552,7 +552,8 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
     const uint32_t nx = (a.ntiles + TILES - 1) / TILES, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
     uint32_t blocks = (nx < 8 ? nx : (nx + 7) / 8 * 8) * ny;
     if (!a.group_expert)
-        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, KS == 2 || WN == 4 ? 32 : 64, &blocks);
+        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, KS == 2 || WN == 4 ? 32 : 64, &blocks,
+                          batch > 1 ? mix_batch_xcds(batch) : 8);
     launch_main(mix_gemm_lds_kernel<GROUPS, KS, WN>, dim3(blocks, batch), dim3(128 * WN * KS), a, mix_gemm_lds_bytes<GROUPS, KS, WN>());
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
