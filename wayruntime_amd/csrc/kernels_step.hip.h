@@ -27,10 +27,11 @@
 //   gate/up    a pair of tiles each              x2, norm -> act [ffn]
 //   down       a tile each                       act (+ x2) -> x
 //
-// What bounds it: the chain of exchanges.  28 layers, hidden 1024, 16/8 heads, ffn 3072, at 60 keys: 488 us in the
-// launch, 17.4 a layer (140 launches: 770), for 4.7 us of weights from HBM: six exchanges of 1.1 to 1.5 us (store, load,
-// and half a load's trip until the next look), four times 0.9 from row to terms and 0.6 from terms to the next row,
-// and 3 us in the attention.  A step (C call; row up, rotary table, logits' product and copy besides): 890 -> 593 us.
+// What bounds it: the chain of exchanges.  28 layers, hidden 1024, 16/8 heads, ffn 3072, at 60 keys: 464 us in the
+// launch, 16.6 a layer (140 launches: 770), for 4.7 us of weights from HBM: five exchanges of 0.8 to 1.4 us (store, load,
+// and half a load's trip until the next look; a sixth where keys are split), four times 0.8 from row to terms and 0.6 from
+// terms to the next row, and 3.5 us in the attention.  (488 and 17.4 before a layer's norm weights were asked for behind
+// attention and its first keys ahead of the Q/K/V weights: the Q/K/V row's exchange took 1.8 to 3.0 us.)
 //
 // A row's buffer is written once a layer.  Whoever writes it again has, through the rows in
 // between, waited for every reader of the last layer's values: each piece reads its row before it
@@ -163,6 +164,8 @@ __device__ __forceinline__ void step_poll(const StepArgs& a, float (&v)[N][4], _
         }
 }
 
+constexpr int kStepHeads = (kMaxGroupMfma + 2 + 3) / 4;     // heads of an attention piece (Q's, K, V) to a staging wave
+
 struct StepShared {
     f32x4 part[6 * 64];                                     // sums of compute waves 1 .. 3
     float sum[8];
@@ -174,6 +177,7 @@ struct StepShared {
     float o[kDecodeWaves][2 * kMaxGroupMfma][128 + 4];       // a head's hi column, G on its lo column
     float m[kDecodeWaves][kMaxGroupMfma];
     float l[kDecodeWaves][kMaxGroupMfma];
+    alignas(16) float head[4][kStepHeads][128];              // a staging wave's heads of the Q/K/V row
 };
 
 // What a staging lane holds of a row: quad i, of a chunk that others may not have.
@@ -424,8 +428,17 @@ __device__ __forceinline__ void step_put_copies(const StepArgs& a, uint32_t at, 
 __device__ __forceinline__ uint32_t step_head_dim(uint32_t i) { return (i & ~15u) + ((i >> 1) & 3) * 4 + ((i >> 3) & 1) * 2 + (i & 1); }
 
 // Attention of one (KV head, key split), compute waves; as decode_mfma_kernel<128, true>.
-__device__ __forceinline__ void step_attend(const StepArgs& a, StepShared& sh, uint32_t kvh, uint32_t split, const uint16_t* kc,
-                                            const uint16_t* vc, uint32_t tag, int lane, uint32_t wave)
+// `fa`: the wave's first tile, asked for (step_first_tile) ahead of the layer.
+__device__ __forceinline__ void step_first_tile(const StepArgs& a, DecodeFrag<128>& fa, uint32_t kvh, uint32_t split, const uint16_t* kc,
+                                                const uint16_t* vc, int lane, uint32_t wave)
+{
+    const TileRange tr = split_tiles(a.s, split);
+    load_frag<128>(fa, kc + (size_t)kvh * a.s.ctx_pad * 128, vc + (size_t)kvh * (a.s.ctx_pad / kVBlock) * 128 * kVBlock,
+                   min(tr.t_begin + wave, tr.t_end - 1), lane);
+}
+
+__device__ __forceinline__ void step_attend(const StepArgs& a, StepShared& sh, DecodeFrag<128>& fa, uint32_t kvh, uint32_t split,
+                                            const uint16_t* kc, const uint16_t* vc, uint32_t tag, int lane, uint32_t wave)
 {
     constexpr int HD = 128;
     const DecodeSession& S = a.s;
@@ -437,9 +450,7 @@ __device__ __forceinline__ void step_attend(const StepArgs& a, StepShared& sh, u
     const uint32_t new_tile = (S.seq_k - 1) / kTileKeys;
     const bool owner = new_tile >= tr.t_begin && new_tile < tr.t_end;
     const uint32_t patch_tile = (owner && (new_tile - tr.t_begin) % kDecodeWaves == wave) ? new_tile : 0xFFFFFFFFu;
-    DecodeFrag<HD> fa;
     uint32_t t = tr.t_begin + wave;
-    load_frag<HD>(fa, kbase, vtbase, min(t, tr.t_end - 1), lane);
     lds_barrier();                                           // Q^T and the new row are in LDS
 
     const int col_kind = (n < G) ? 0 : ((n < 2 * G) ? 1 : 2);
@@ -502,11 +513,21 @@ __device__ __forceinline__ void step_attend(const StepArgs& a, StepShared& sh, u
     }
 }
 
+// The head of an attention piece that a staging lane has its part of: Q's 0 .. G - 1, then K, then V, dealt to the waves
+// in turn, eight lanes each.
+constexpr uint32_t kStepNoHead = 0xFFFFFFFFu;
+__device__ __forceinline__ uint32_t step_head_slot(uint32_t t, uint32_t G)
+{
+    const uint32_t octet = (t & 63) >> 3, slot = octet * 4 + (t >> 6);
+    return octet < (uint32_t)kStepHeads && slot < G + 2 ? slot : kStepNoHead;
+}
+
 // The norm's weights (a layer ahead, as above) and the rotation of a staging lane's part of its head.  Asked for whether
 // they are used or not, from an address that is valid.
 __device__ __forceinline__ void step_head_weights(const StepArgs& a, Row8Loads<2>& rl, const StepLayer& ly, uint32_t t)
 {
-    const float* nw = (t >> 3) == 8 ? ly.k_norm : ly.q_norm;
+    const uint32_t G = a.nq / a.nkv;
+    const float* nw = step_head_slot(t, G) == G ? ly.k_norm : ly.q_norm;
     const StepNorm w = (StepNorm)(nw ? nw : a.x0);
 #pragma unroll
     for (int c = 0; c < 2; c++) {
@@ -533,21 +554,37 @@ __device__ __forceinline__ void step_attend_stage(const StepArgs& a, StepShared&
     const TileRange tr = split_tiles(S, split);
     const uint32_t new_pos = S.seq_k - 1, new_tile = new_pos / kTileKeys;
     const bool owner = new_tile >= tr.t_begin && new_tile < tr.t_end;
-    const uint32_t hslot = t >> 3, part = t & 7;
-    constexpr uint32_t kSlotK = 8, kSlotV = 16;
-    const bool slot_q = hslot < (uint32_t)G, slot_k = owner && hslot == kSlotK, slot_v = owner && hslot == kSlotV;
-    const uint32_t head = slot_k ? a.nq + kvh : slot_v ? a.nq + a.nkv + kvh : kvh * G + (slot_q ? hslot : 0u);
-    float v[2 * NJ][4];
-    const uint32_t q0 = head * 32 + part * 2;
-    const uint32_t q[2 * NJ] = {q0, q0 + 1, q0 + 16, q0 + 17};
-    step_poll<2 * NJ>(a, v, step_row(a.qkv, (a.nq + 2 * a.nkv) * HD), q, tag, deadline);
+    const uint32_t lane = t & 63, wave = t >> 6, part = t & 7, slot = step_head_slot(t, G);
+    const bool slot_q = slot < (uint32_t)G, slot_k = owner && slot == (uint32_t)G, slot_v = owner && slot == (uint32_t)G + 1;
+    // A wave asks for each of its heads with one load, 1024 bytes side by side, and takes them apart through LDS.
+    const __amdgpu_buffer_rsrc_t row = step_row(a.qkv, (a.nq + 2 * a.nkv) * HD);
+    u32x4 u[kStepHeads];
+    const auto used = [&](int i) { return i * 4 + wave < (uint32_t)(owner ? G + 2 : G); };      // (the same in all lanes)
+    for (uint32_t tries = 0;;) {
+        bool ok = true;
+        asm volatile("" ::: "memory");                       // (asked for again every time)
+#pragma unroll
+        for (int i = 0; i < kStepHeads; i++) {
+            const uint32_t sl = i * 4 + wave;
+            const uint32_t head = sl < (uint32_t)G ? kvh * G + sl : sl == (uint32_t)G ? a.nq + kvh : a.nq + a.nkv + kvh;
+            u[i] = u32x4{0, tag, 0, tag};
+            if (used(i)) u[i] = step_get_unit(row, head * 64 + lane);
+        }
+#pragma unroll
+        for (int i = 0; i < kStepHeads; i++) ok = ok && u[i][1] == tag && u[i][3] == tag;
+        if (__all(ok) || step_late(a, deadline, tries)) break;
+    }
+#pragma unroll
+    for (int i = 0; i < kStepHeads; i++) {
+        float2 two{__uint_as_float(u[i][0]), __uint_as_float(u[i][2])};
+        *reinterpret_cast<float2*>(&sh.head[wave][i][(lane >> 3) * 16 + (lane & 3) * 4 + (lane >> 2 & 1) * 2]) = two;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (its own wave's)
+    const float* mine = sh.head[wave][min(lane >> 3, (uint32_t)kStepHeads - 1)] + part * 8;
 #pragma unroll
     for (int c = 0; c < NJ; c++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            rl.x[c][0][e] = v[2 * c][e];
-            rl.x[c][1][e] = v[2 * c + 1][e];
-        }
+        for (int e = 0; e < 2; e++) rl.x[c][e] = *reinterpret_cast<const f32x4*>(mine + c * 64 + e * 4);
     float x[NJ][8];
     row8_head_finish<NJ>(x, rl, norm && !slot_v, false, a.eps, part, a.cos_sin != nullptr && !slot_v, a.n_rot);
     if (slot_q) {
@@ -558,8 +595,8 @@ __device__ __forceinline__ void step_attend_stage(const StepArgs& a, StepShared&
                 const int d = c * 64 + (int)part * 8 + e;
                 _Float16 hi, lo;
                 q_hi_lo(x[c][e], a.qscale, hi, lo);
-                sh.q[hslot][d] = hi;
-                sh.q[hslot + G][d] = lo;
+                sh.q[slot][d] = hi;
+                sh.q[slot + G][d] = lo;
             }
     }
     u32x4 packed[NJ];                                        // K or V as the cache holds them
@@ -667,7 +704,7 @@ __global__ __launch_bounds__(kStepThreads, 2) void step_layers_kernel(const Step
     lds_barrier();
     if (wave >= 4) {
         StepLayer next = step_layer(a, 0);
-        f32x4 attn_w[2], ffn_w[2];
+        f32x4 attn_w[2], ffn_w[2] = {};
         Row8Loads<2> rl;
         step_norm_weights(attn_w, next.attn_norm, threadIdx.x - 256, a.hidden);
         step_head_turn(a, rl, threadIdx.x - 256);
@@ -675,15 +712,18 @@ __global__ __launch_bounds__(kStepThreads, 2) void step_layers_kernel(const Step
         for (uint32_t L = 0; L < a.n_layers; L++) {
             const StepLayer ly = next;
             next = step_layer(a, min(L + 1, a.n_layers - 1));
-            step_norm_weights(ffn_w, ly.ffn_norm, threadIdx.x - 256, a.hidden);
             const uint32_t tag = a.tag0 + L;
             const float* x0 = L == 0 ? a.x0 : nullptr;       // the row ahead of the first layer; later ones bear the tag before
             uint16_t* kc = reinterpret_cast<uint16_t*>(a.slab + 2 * L * a.side);
             uint16_t* vc = reinterpret_cast<uint16_t*>(a.slab + (2 * L + 1) * a.side);
             for (uint32_t piece = kStepQkv; piece <= kStepDown; piece++) {
-                if (!(pieces >> piece & 1)) continue;
                 uint32_t t = threadIdx.x - 256;
                 asm volatile("" : "+v"(t));                  // what a piece derives from the lane is not kept through the others
+                if (piece == kStepOut) {                     // (attention's row, or a layer's first, would come in behind them)
+                    if (has_gu) step_norm_weights(ffn_w, ly.ffn_norm, t, a.hidden);
+                    if (has_qkv) step_norm_weights(attn_w, next.attn_norm, t, a.hidden);
+                }
+                if (!(pieces >> piece & 1)) continue;
                 if (piece == kStepAttend) {
                     if (has_attn) step_attend_stage(a, sh, rl, ly.q_norm != nullptr, kvh, split, kc, vc, tag, t, deadline);
                     step_head_weights(a, rl, next, t);
@@ -704,11 +744,14 @@ __global__ __launch_bounds__(kStepThreads, 2) void step_layers_kernel(const Step
                     stage(std::integral_constant<int, 2>());
                 else
                     stage(std::integral_constant<int, 3>());
-                if (qkv) step_norm_weights(attn_w, next.attn_norm, t, a.hidden);
             }
         }
         return;
     }
+    // What the staging waves poll for comes back behind all loads that the compute waves have made before: weights or
+    // keys that are asked for while a row is on its way hold it up by their own trip (the Q/K/V row reached attention 1.8 to
+    // 2.6 us after its last value was out; 1.1 to 1.6 now).  So a layer's first keys are asked for ahead of
+    // its Q/K/V weights.
     StepLayer next = step_layer(a, 0);
     for (uint32_t L = 0; L < a.n_layers; L++) {
         const StepLayer ly = next;
@@ -716,46 +759,65 @@ __global__ __launch_bounds__(kStepThreads, 2) void step_layers_kernel(const Step
         const uint32_t tag = a.tag0 + L;
         const uint16_t* kc = reinterpret_cast<const uint16_t*>(a.slab + 2 * L * a.side);
         const uint16_t* vc = reinterpret_cast<const uint16_t*>(a.slab + (2 * L + 1) * a.side);
-        for (uint32_t piece = kStepQkv; piece <= kStepDown; piece++) {
-            if (!(pieces >> piece & 1)) continue;
-            int ln = lane;
-            asm volatile("" : "+v"(ln));                     // what a piece derives from the lane is not kept through the others
-            if (piece == kStepAttend) {
-                if (has_attn) step_attend(a, sh, kvh, split, kc, vc, tag, ln, wave);
-            } else if (piece == kStepGateUp) {
-                f32x4 acc[2], r, none;
-                float sc;
-                step_product<2>(sh, sfrag, acc, sc, none, (StepWeights)ly.wgu, behind, behind + a.ffn / 16, a.hidden, true, ln, wave);
-                if (wave == 0) {
+        int ln = lane;
+        const auto apart = [&] { asm volatile("" : "+v"(ln)); };     // what a piece derives from the lane is not kept through the others
+        DecodeFrag<128> fa;
+        if (has_attn) step_first_tile(a, fa, kvh, split, kc, vc, lane, wave);
+        f32x4 acc[1], r, resid;
+        float sc;
+        if (has_qkv) {
+            step_product<1>(sh, sfrag, acc, sc, resid, (StepWeights)ly.wqkv, b, b, a.hidden, true, ln, wave);
+            if (wave == 0) {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        float x = acc[0][i] * sc, y = acc[1][i] * sc;
-                        asm volatile("" : "+v"(x), "+v"(y)); // the products end here: no contraction into the activation
-                        r[i] = silu_mul(x, y);
-                    }
-                    step_publish(a.act, a.ffn, kStepCopies, behind, ln, r, tag);
+                for (int i = 0; i < 4; i++) r[i] = acc[0][i] * sc;
+                step_publish(a.qkv, width, 1, b, ln, r, tag);    // (a head's share is read by its own workgroups only)
+            }
+        }
+        apart();
+        if (has_attn) step_attend(a, sh, fa, kvh, split, kc, vc, tag, ln, wave);
+        apart();
+        if (has_o) {
+            step_product<1>(sh, sfrag, acc, sc, resid, (StepWeights)ly.wo, b, b, qd, false, ln, wave);
+            if (wave == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float x = acc[0][i] * sc;
+                    r[i] = x + resid[i];
                 }
-            } else {
-                const bool qkv = piece == kStepQkv, o = piece == kStepOut;
-                f32x4 acc[1], r, resid;
-                float sc;
-                step_product<1>(sh, sfrag, acc, sc, resid, (StepWeights)(qkv ? ly.wqkv : o ? ly.wo : ly.wdown), b, b,
-                                qkv ? a.hidden : o ? qd : a.ffn, qkv, ln, wave);
-                if (wave == 0) {
+                step_publish(a.x2, a.hidden, kStepCopies, b, ln, r, tag);
+            }
+        }
+        apart();
+        if (has_gu) {
+            f32x4 two[2], none;
+            step_product<2>(sh, sfrag, two, sc, none, (StepWeights)ly.wgu, behind, behind + a.ffn / 16, a.hidden, true, ln, wave);
+            if (wave == 0) {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float x = acc[0][i] * sc, y = x + resid[i];
-                        r[i] = qkv ? x : y;
-                    }
-                    if (piece == kStepDown && L + 1 == a.n_layers) {
-                        if ((ln & 15) == 0) *reinterpret_cast<f32x4*>(a.y + b * 16 + 4 * (ln >> 4)) = r;
-                    } else {
-                        // (a head's share of the Q/K/V row is read by its own workgroups only)
-                        step_publish(qkv ? a.qkv : o ? a.x2 : a.x, qkv ? width : a.hidden, qkv ? 1u : kStepCopies, b, ln, r, tag);
-                    }
+                for (int i = 0; i < 4; i++) {
+                    float x = two[0][i] * sc, y = two[1][i] * sc;
+                    asm volatile("" : "+v"(x), "+v"(y));     // the products end here: no contraction into the activation
+                    r[i] = silu_mul(x, y);
+                }
+                step_publish(a.act, a.ffn, kStepCopies, behind, ln, r, tag);
+            }
+        }
+        apart();
+        if (has_o) {
+            step_product<1>(sh, sfrag, acc, sc, resid, (StepWeights)ly.wdown, b, b, a.ffn, false, ln, wave);
+            if (wave == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float x = acc[0][i] * sc;
+                    r[i] = x + resid[i];
+                }
+                if (L + 1 == a.n_layers) {
+                    if ((ln & 15) == 0) *reinterpret_cast<f32x4*>(a.y + b * 16 + 4 * (ln >> 4)) = r;
+                } else {
+                    step_publish(a.x, a.hidden, kStepCopies, b, ln, r, tag);
                 }
             }
         }
+        apart();
     }
 }
 
