@@ -748,9 +748,10 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
         if (a.groups <= kMixMaxPieces && streams(a, e)) {
             // From so many rows an expert (us, without / with, as below): in order 12, 20 where the weights are less than 160 MiB (16
             // experts, 1408 -> 2048 at 13 rows 18.8 / 20.9) and 24 over short ranges (64, 512 -> 2048 at 17 30.6 / 33.5); picked
-            // one by one, which all workgroups of the others do again, 4 (64, 2048 -> 1024 47 / 43; 32, 4096 -> 4096 182 / 167), 10 with
+            // one by one, which all workgroups of the others do again, 4 over long ranges (32, 4096 -> 4096 182 / 167), 5 else (six of 64,
+            // 2048 -> 2 x 1024 -> 2048, a whole pass at 4.3 rows 106.6 / 107.7, at 5.3 110.2 / 110.1, at 6 120.6 / 112.7), 10 with
             // few experts (16, 2048 -> 4096 at 4 rows 42 / 46, at 11 49 / 46), 8 over short ranges (64, 512 -> 2048 31 / 32 at 6, 35 / 33 at 9).
-            const uint64_t from = a.x_perm ? (a.ktiles < 32 ? 8 : e >= 32 || a.ktiles >= 128 ? 4 : 10)
+            const uint64_t from = a.x_perm ? (a.ktiles < 32 ? 8 : a.ktiles >= 128 ? 4 : e >= 32 ? 5 : 10)
                                            : a.ktiles < 32 ? 24 : e * a.ntiles * a.ktiles >> 10 >= 160 ? 12 : 20;
             if (spare >= e * from) return launch_stream<2, 4, 4, true>(a, e);
         }
