@@ -188,7 +188,7 @@ __device__ __forceinline__ uint32_t step_chunk(uint32_t t, int i)
 }
 __device__ __forceinline__ uint32_t step_quad(uint32_t t, int i, uint32_t nchunks) { return min(step_chunk(t, i), nchunks - 1) * 2 + (t & 1); }
 
-// Norm weights are asked for a layer ahead: a wave's loads come back in the order they were made, and the first look at
+// Norm weights are asked for behind the attention ahead of their rows: a wave's loads come back in the order they were made, and the first look at
 // a row would wait for the trip to memory that weights nobody has read yet take (1.7 us).
 __device__ __forceinline__ void step_norm_weights(f32x4 (&w)[2], const float* norm, uint32_t t, uint32_t hidden)
 {
