@@ -483,6 +483,25 @@ def test_sixteen_requests(eng, tmp_path, prec):
     case.close()
 
 
+def test_batched_row_depends_on_the_longest_request_only(eng, tmp_path):
+    # sixteen requests, the second one the longest: how far the others are decides nothing about the first one's sums
+    case = Case(eng, tmp_path, mw.shared_kv_config(64, 90, [(mw.keys_as_values(8, 8, 32, 1800), None)]), "bf16", pool=32768, slots=16)
+    got = []
+    for others in (40, 1400, 700):
+        todo = [case.tokens(n, seed=i) for i, n in enumerate([700, 1500] + [others] * 14)]
+        ss = [case.m.session() for _ in todo]
+        for s, t in zip(ss, todo):
+            assert s.prefill(t[:-1]) == len(t) - 1
+        rc, lg = E.batch_step(ss, [int(t[-1]) for t in todo])
+        assert rc == 16
+        got.append(np.array(lg[0]))
+        for s in ss:
+            s.close()
+    case.check(got[0][None], case.oracle(case.tokens(700, seed=0))[-1:], "the first of sixteen")
+    assert got[1].tobytes() == got[0].tobytes() and got[2].tobytes() == got[0].tobytes()
+    case.close()
+
+
 def test_greedy_generation(eng, tmp_path):
     # wr_prefill, wr_step and wr_batch_step against the oracle's own greedy streams (32-bit: no ties to lose)
     case = Case(eng, tmp_path, stack(), "f32")

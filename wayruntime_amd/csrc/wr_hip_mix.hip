@@ -1444,19 +1444,14 @@ static int window_mfma(wr_hip_mix_step* s, WindowArgs& a)
     }
     const uint32_t groups = a.kvh * ((a.group * MAPS + 15) / 16);
     // Shares: two workgroups per compute unit at a time; a round costs about three iterations before its first and one
-    // for each it makes, and the shares' sums about two more to put together.  Rounds are those of the workgroups that
-    // have keys: requests of different ages leave many of the longest one's shares without any (sixteen at 100 .. 1500 keys in
-    // shares of 256: 464 of 768; when all were counted they took shares of 384: 18.3 us, now 17.2).
+    // for each it makes, and the shares' sums about two more to put together.  Of the other requests only their number and
+    // the longest one's keys decide: counting the shares that have keys is faster where ages differ (sixteen at 100 .. 1500
+    // keys: 18.3 -> 17.2 us), but then the order of a row's sums changes with every other request's position.
     uint64_t best = ~(uint64_t)0;
-    for (uint32_t iters = 1; iters <= 256; iters += std::max(1u, iters / 8)) {
+    for (uint32_t iters = 1; iters <= 256; iters++) {
         const uint64_t share = (uint64_t)iters * 128, splits = (keys + share - 1) / share;
         if (splits > kWindowSplits) continue;
-        uint64_t live = 0;
-        for (uint32_t i = 0; i < n; i++) {
-            const uint32_t lo = window_lo(rows[i].pos, a.window, a.chunk);
-            live += (rows[i].pos + share - lo / 32 * 32) / share;
-        }
-        const uint64_t rounds = (live * groups + 2 * g.n_cus - 1) / (2 * g.n_cus);
+        const uint64_t rounds = ((uint64_t)n * groups * splits + 2 * g.n_cus - 1) / (2 * g.n_cus);
         const uint64_t cost = rounds * (iters + 3) + (splits > 1 ? 2 : 0);
         if (cost < best) {
             best = cost;
