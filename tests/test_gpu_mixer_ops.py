@@ -565,6 +565,111 @@ def test_matrix_per_row_group(lib, f32, N, K, tile):
         b.free()
 
 
+class Resid(C.Structure):
+    _fields_ = [("width", u32), ("eps", C.c_float), ("x", vp), ("y", vp), ("post", vp), ("add", vp), ("next", vp), ("gate", vp),
+                ("slot", vp), ("top", u32), ("wanted", u32), ("h", vp), ("side", vp), ("ident", vp), ("shared", vp),
+                ("pair_y", vp * 2), ("pair_post", vp * 2)]
+
+
+class Seq(C.Structure):
+    _fields_ = [("rows", u32), ("pos0", u32), ("slot", u32), ("buf_in", u32), ("buf_out", u32), ("n_pages", u32), ("pages", C.POINTER(u32))]
+
+
+class StepOf:
+    """A step of one request with these tokens."""
+
+    def __init__(self, lib, tokens, vocab):
+        pages = -(-len(tokens) // 64)
+        lib.wr_hip_mix_pool_destroy.argtypes = lib.wr_hip_mix_step_destroy.argtypes = [vp]
+        lib.wr_hip_mix_residual.argtypes = [vp, C.c_int, C.POINTER(Resid)]
+        lib.wr_hip_mix_embed.argtypes = [vp, C.c_int, vp, u32, vp, C.c_float, C.c_float, vp, vp, vp, vp]
+        self.lib, self.pool, self.h = lib, vp(), vp()
+        assert lib.wr_hip_mix_pool_create(0, 1, (u32 * 1)(32), pages, 0, None, 1, C.byref(self.pool)) == 0
+        assert lib.wr_hip_mix_step_create(pages, C.byref(self.h)) == 0
+        seq = Seq(len(tokens), 0, 0, 0, 1, pages, (u32 * pages)(*range(pages)))
+        assert lib.wr_hip_mix_step_set(self.h, self.pool, 1, C.byref(seq), (u32 * len(tokens))(*tokens), vocab, 0, None) == 0
+
+    def end(self):
+        hipattn.sync()
+        self.lib.wr_hip_mix_step_destroy(self.h)
+        self.lib.wr_hip_mix_pool_destroy(self.pool)
+
+
+# One row to a workgroup up to 599 rows (1791 with experts' rows) and wherever no fragment is written, four beyond; features
+# that a workgroup holds in registers (4096) and more.
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("width", [2048, 4200])
+@pytest.mark.parametrize("kind", ["plain", "no_fragment", "pair", "embed", "experts"])
+def test_row_steps_of_many_rows(lib, f32, width, kind):
+    rng = np.random.default_rng(width)
+    counts = (64, 1791, 1792, 1793) if kind == "experts" else (64, 599, 600, 601, 1501)
+    most, wpad, top, vocab, eps = max(counts), -(-width // 32) * 32, 3, 50, 1e-6
+
+    def rows(n):
+        v = np.zeros((n, wpad), dtype=np.float32)
+        v[:, :width] = rng.standard_normal((n, width), dtype=np.float32)
+        return v
+
+    def norm(v):
+        v = v.astype(np.float64)
+        return v / np.sqrt((v ** 2).sum(axis=-1, keepdims=True) / width + eps)
+
+    up = hipattn.DeviceBuffer.from_host
+    x0, y, add, post, nxt, post2 = rows(most), rows(most), rows(most), rows(1), rows(1), rows(2)
+    pairs, table = [rows(most), rows(most)], O.f32_to_bf16(rng.standard_normal((vocab, width), dtype=np.float32))
+    tokens, slot = rng.integers(0, vocab, most), rng.integers(0, most, (most, top)).astype(np.uint32)
+    gate = rng.uniform(0, 1, (most, top)).astype(np.float32)
+    slot[5, 1] = 0xFFFFFFFF                                    # left out
+    want = x0.astype(np.float64)
+    if kind == "embed":
+        want = norm(O.bf16_to_f32(table)[tokens]) * post[:, :width]
+        want = np.pad(want, ((0, 0), (0, wpad - width)))
+    elif kind == "experts":
+        g = np.where(slot == 0xFFFFFFFF, 0.0, gate).astype(np.float64)
+        want = want + norm((g[:, :, None] * y[np.minimum(slot, most - 1)]).sum(axis=1)) * post
+    else:
+        want = want + norm(y) * post + add
+        if kind == "pair":
+            want = want + norm(pairs[0]) * post2[0] + norm(pairs[1]) * post2[1]
+    yd, ad, pd, nd, td = up(y), up(add), up(post), up(nxt), up(table)
+    qd, ppd, sd, gd = [up(p) for p in pairs], [up(post2[i:i + 1]) for i in range(2)], up(slot.view(np.float32)), up(gate)
+    few = None
+    for n in counts:
+        s, xd = StepOf(lib, tokens[:n].tolist(), vocab), up(x0[:n])
+        hd = hipattn.DeviceBuffer(-(-n // 16) * 16 * wpad * (4 if f32 else 2))
+        if kind == "embed":
+            assert lib.wr_hip_mix_embed(s.h, int(f32), td.p, width, pd.p, 1.0, eps, xd.p, None, nd.p, hd.p) == 0
+        else:
+            a = Resid(width=width, eps=eps, x=xd.p, y=yd.p, post=pd.p)
+            if kind != "no_fragment":
+                a.next, a.h = nd.p, hd.p
+            if kind == "experts":
+                a.gate, a.slot, a.top = gd.p, sd.p, top
+            else:
+                a.add = ad.p
+            if kind == "pair":
+                for i in range(2):
+                    a.pair_y[i], a.pair_post[i] = qd[i].p, ppd[i].p
+            assert lib.wr_hip_mix_residual(s.h, int(f32), C.byref(a)) == 0
+        s.end()
+        got = [xd.to_host((n, wpad))]
+        scale = np.abs(want).max()
+        assert np.abs(got[0] - want[:n]).max() < 2e-6 * scale, (kind, n)      # (32-bit sums of some thousand terms)
+        if kind != "no_fragment":
+            m = -(-n // 16) * 16 * wpad
+            h = unfrag(hd.to_host((m,)) if f32 else O.bf16_to_f32(hd.to_host((m // 2,)).view(np.uint16)), n, wpad)
+            ref = norm(want[:n]) * nxt
+            assert np.abs(h - ref).max() < (2e-6 if f32 else 2.0 ** -8) * np.abs(ref).max(), (kind, n)
+            got.append(h)
+        few = few or got
+        for a, b in zip(got, few):                             # a row's bits are its own from 64 rows on
+            assert np.array_equal(a[:64], b), (kind, n)
+        for b in (xd, hd):
+            b.free()
+    for b in (yd, ad, pd, nd, td, sd, gd, *qd, *ppd):
+        b.free()
+
+
 def test_refusals(lib):
     r = Run(lib, False, 1, 32, 32, 16)
     y = hipattn.DeviceBuffer(16 * 32 * 4)

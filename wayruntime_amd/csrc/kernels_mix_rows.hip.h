@@ -17,13 +17,48 @@ struct MixRowShape {
     static constexpr int kHeld = RPW == 1 ? 2 : 4;       // chunks a thread can hold: 4096 features
 };
 
+// PAIRED: one row to a workgroup with the sums of four, bit by bit.  There a thread adds up every 128th chunk; here lanes L
+// and L + 32 take its chunks in turn and pass the sum on to each other.
+template <int RPW, bool PAIRED>
+__device__ __forceinline__ uint32_t mix_row_chunk()
+{
+    static_assert(!PAIRED || RPW == 1);
+    const uint32_t t = threadIdx.x;
+    return PAIRED ? t / 64 * 32 + t % 32 + t / 32 % 2 * 128 : t / RPW;
+}
+
+// (PAIRED: in the lower lane; all lanes take part)
+template <bool PAIRED>
+__device__ __forceinline__ float mix_add_squares(float ss, const float (&v)[8], bool there)
+{
+    const auto add = [&](float s) {
+        if (there) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) s = fmaf(v[j], v[j], s);
+        }
+        return s;
+    };
+    if constexpr (!PAIRED) return add(ss);
+    return wave_xor_f32(add(wave_xor_f32(add(ss), 32)), 32);
+}
+
 // Sum over the threads of a row; every thread gets its row's sum.
-template <int RPW>
+template <int RPW, bool PAIRED = false>
 __device__ __forceinline__ float mix_row_sum(float v, float* red)
 {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     constexpr int WAVES = MixRowShape<RPW>::kThreads / 64;
-    if constexpr (RPW == 1) {
+    if constexpr (PAIRED) {                                // sixteen lower lanes are a wave of four rows
+#pragma unroll
+        for (int off = 1; off <= 8; off <<= 1) v += wave_xor_f32(v, off);
+        if (lane < 32 && lane % 16 == 0) red[wave * 2 + lane / 16] = v;
+        __syncthreads();
+        float s = 0.f;
+#pragma unroll
+        for (int w = 0; w < 2 * WAVES; w++) s += red[w];
+        __syncthreads();
+        return s;
+    } else if constexpr (RPW == 1) {
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) v += wave_xor_f32(v, off);
         if (lane == 0) red[wave] = v;
@@ -162,14 +197,14 @@ __device__ __forceinline__ void mix_sub_chunk(const MixRowArgs& a, uint32_t r, u
 // x <- x + rmsnorm(y) * post (or + y) + add; h <- rmsnorm(x) * next
 // (EMBED: x <- rmsnorm(table[token]) * norm, or table[token] * scale, first;
 // PAIR: + rmsnorm(pair_y[i]) * pair_post[i] for both).
-template <bool F32, int RPW, bool EMBED, bool HELD, bool PAIR>
+template <bool F32, int RPW, bool PAIRED, bool EMBED, bool HELD, bool PAIR>
 __global__ __launch_bounds__(MixRowShape<RPW>::kThreads) void mix_residual_kernel(const MixRowArgs a)
 {
     using Sh = MixRowShape<RPW>;
     constexpr int CH = HELD ? Sh::kHeld : 1;
     __shared__ float red[64];
     const uint32_t t = threadIdx.x;
-    const uint32_t row = blockIdx.x * RPW + t % RPW, lr = t / RPW;
+    const uint32_t row = blockIdx.x * RPW + t % RPW, lr = mix_row_chunk<RPW, PAIRED>();
     const bool live = row < a.rows;
     const uint32_t rr = live ? row : a.rows - 1;
     const uint32_t r = a.gather ? a.gather[rr] : rr;
@@ -209,21 +244,18 @@ __global__ __launch_bounds__(MixRowShape<RPW>::kThreads) void mix_residual_kerne
 #pragma unroll
             for (int i = 0; i < CH; i++) {
                 const uint32_t q = lr + i * Sh::kPerRow;
-                if (q < nq) {
-                    first(q, held[i]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) ss = fmaf(held[i][j], held[i][j], ss);
-                }
+                if (q < nq) first(q, held[i]);
+                ss = mix_add_squares<PAIRED>(ss, held[i], q < nq);
             }
         } else {
-            for (uint32_t q = lr; q < nq; q += Sh::kPerRow) {
+            for (uint32_t q0 = 0; q0 < nq; q0 += Sh::kPerRow) {
+                const uint32_t q = lr + q0;
                 float v[8];
-                first(q, v);
-#pragma unroll
-                for (int j = 0; j < 8; j++) ss = fmaf(v[j], v[j], ss);
+                if (q < nq) first(q, v);
+                ss = mix_add_squares<PAIRED>(ss, v, q < nq);
             }
         }
-        if (normed) inv = 1.0f / sqrtf(mix_row_sum<RPW>(ss, red) * invw + a.eps);
+        if (normed) inv = 1.0f / sqrtf(mix_row_sum<RPW, PAIRED>(ss, red) * invw + a.eps);
     }
     float pair[PAIR ? 2 : 1][HELD && PAIR ? CH : 1][8], pinv[2];
     if constexpr (PAIR) {
@@ -235,19 +267,17 @@ __global__ __launch_bounds__(MixRowShape<RPW>::kThreads) void mix_residual_kerne
 #pragma unroll
                 for (int i = 0; i < CH; i++) {
                     const uint32_t q = lr + i * Sh::kPerRow;
-                    if (q >= nq) continue;
-                    mix_load8(p + q * 8, pair[k][i]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) ps = fmaf(pair[k][i][j], pair[k][i][j], ps);
+                    if (q < nq) mix_load8(p + q * 8, pair[k][i]);
+                    ps = mix_add_squares<PAIRED>(ps, pair[k][i], q < nq);
                 }
             } else {
-                for (uint32_t q = lr; q < nq; q += Sh::kPerRow) {
-                    mix_load8(p + q * 8, pair[k][0]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) ps = fmaf(pair[k][0][j], pair[k][0][j], ps);
+                for (uint32_t q0 = 0; q0 < nq; q0 += Sh::kPerRow) {
+                    const uint32_t q = lr + q0;
+                    if (q < nq) mix_load8(p + q * 8, pair[k][0]);
+                    ps = mix_add_squares<PAIRED>(ps, pair[k][0], q < nq);
                 }
             }
-            pinv[k] = 1.0f / sqrtf(mix_row_sum<RPW>(ps, red) * invw + a.eps);
+            pinv[k] = 1.0f / sqrtf(mix_row_sum<RPW, PAIRED>(ps, red) * invw + a.eps);
         }
     }
 
@@ -304,23 +334,22 @@ __global__ __launch_bounds__(MixRowShape<RPW>::kThreads) void mix_residual_kerne
 #pragma unroll
         for (int i = 0; i < CH; i++) {
             const uint32_t q = lr + i * Sh::kPerRow;
-            if (q < nq) {
-                second(q, held[i], i);
-#pragma unroll
-                for (int j = 0; j < 8; j++) ss = fmaf(held[i][j], held[i][j], ss);
-            }
+            if (q < nq) second(q, held[i], i);
+            ss = mix_add_squares<PAIRED>(ss, held[i], q < nq);
         }
     } else {
-        for (uint32_t q = lr; q < nq; q += Sh::kPerRow) {
+        for (uint32_t q0 = 0; q0 < nq; q0 += Sh::kPerRow) {
+            const uint32_t q = lr + q0;
             float v[8];
-            if (some) first(q, v);
-            second(q, v, 0);
-#pragma unroll
-            for (int j = 0; j < 8; j++) ss = fmaf(v[j], v[j], ss);
+            if (q < nq) {
+                if (some) first(q, v);
+                second(q, v, 0);
+            }
+            ss = mix_add_squares<PAIRED>(ss, v, q < nq);
         }
     }
     if (!a.next) return;                                   // uniform
-    inv = 1.0f / sqrtf(mix_row_sum<RPW>(ss, red) * invw + a.eps);
+    inv = 1.0f / sqrtf(mix_row_sum<RPW, PAIRED>(ss, red) * invw + a.eps);
     auto third = [&](uint32_t q, float (&v)[8]) {
         float w[8];
         mix_load8(a.next + q * 8, w);

@@ -341,21 +341,27 @@ int wr_hip_mix_step_set(wr_hip_mix_step* s, const wr_hip_mix_pool* pool, uint32_
 static int launch_residual(int f32, bool embed, const MixRowArgs& a)
 {
     // Four rows to a workgroup only where their shares of a fragment's 64-byte pieces are worth more than workgroups are: not without
-    // one, and not for so few rows that compute units stay without (width 2048, us, four / one: 512 rows 5.7 / 5.2, 700 5.9 / 6.2,
-    // 2047 10.8 / 15.3; with six experts' rows to add 100 rows 10.8 / 5.1, 512 12.1 / 7.9, 1500 22.6 / 18.7, 2047 24.0 / 26.1; without
-    // a fragment 512 11.0 / 5.1, 2047 22.4 / 20.7).
-    const bool many = a.next && a.rows >= (a.top ? 1792u : 600u), held = a.wpad <= 4096, pair = a.pair_y[0] != nullptr;
-    const dim3 g1(a.rows), b1(MixRowShape<1>::kThreads), g4((a.rows + 3) / 4), b4(MixRowShape<4>::kThreads);
-#define WR_RESID(F, EMB, PAIR)                                                                   \
-    do {                                                                                         \
-        if (many && held)                                                                        \
-            MIX_LAUNCH((mix_residual_kernel<F, 4, EMB, true, PAIR>), g4, b4, 0, a);              \
-        else if (many)                                                                           \
-            MIX_LAUNCH((mix_residual_kernel<F, 4, EMB, false, PAIR>), g4, b4, 0, a);             \
-        else if (held)                                                                           \
-            MIX_LAUNCH((mix_residual_kernel<F, 1, EMB, true, PAIR>), g1, b1, 0, a);              \
-        else                                                                                     \
-            MIX_LAUNCH((mix_residual_kernel<F, 1, EMB, false, PAIR>), g1, b1, 0, a);             \
+    // one, and not for so few rows that compute units stay without (width 2048, us, four / one: 512 rows 5.7 / 5.5, 700 5.9 / 6.2,
+    // 2047 10.8 / 15.3; with six experts' rows to add 100 rows 10.9 / 4.8, 512 12.1 / 8.3, 1500 22.6 / 19.0, 2047 24.0 / 26.1; these
+    // without a fragment 512 11.0 / 5.5, 2047 22.5 / 20.8).  From 64 rows on one row's sums are made in the order of four's
+    // (PAIRED: 0 to 0.5 us), so that a row's bits do not hang on how many others there are.
+    const bool many = a.next && a.rows >= (a.top ? 1792u : 600u), few = a.rows < 64, held = a.wpad <= 4096, pair = a.pair_y[0] != nullptr;
+#define WR_RESID_ROWS(F, EMB, PAIR, RPW, PAIRED)                                                    \
+    do {                                                                                            \
+        const dim3 grid((a.rows + RPW - 1) / RPW), block(MixRowShape<RPW>::kThreads);               \
+        if (held)                                                                                   \
+            MIX_LAUNCH((mix_residual_kernel<F, RPW, PAIRED, EMB, true, PAIR>), grid, block, 0, a);  \
+        else                                                                                        \
+            MIX_LAUNCH((mix_residual_kernel<F, RPW, PAIRED, EMB, false, PAIR>), grid, block, 0, a); \
+    } while (0)
+#define WR_RESID(F, EMB, PAIR)                                                                      \
+    do {                                                                                            \
+        if (many)                                                                                   \
+            WR_RESID_ROWS(F, EMB, PAIR, 4, false);                                                  \
+        else if (few)                                                                               \
+            WR_RESID_ROWS(F, EMB, PAIR, 1, false);                                                  \
+        else                                                                                        \
+            WR_RESID_ROWS(F, EMB, PAIR, 1, true);                                                   \
     } while (0)
     if (f32 && embed) WR_RESID(true, true, false);
     else if (f32 && pair) WR_RESID(true, false, true);
@@ -364,6 +370,7 @@ static int launch_residual(int f32, bool embed, const MixRowArgs& a)
     else if (pair) WR_RESID(false, false, true);
     else WR_RESID(false, false, false);
 #undef WR_RESID
+#undef WR_RESID_ROWS
     return WR_HIP_OK;
 }
 
