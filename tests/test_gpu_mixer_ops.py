@@ -416,6 +416,29 @@ def test_large_experts_in_runs(lib, experts, N, K, spare):
         b.free()
 
 
+# the most runs that the stream takes, one more and twice as many: the rows are in the first runs and the last
+@pytest.mark.parametrize("experts,N,K,runs", [(150, 512, 544, 256), (150, 512, 544, 257), (64, 1024, 544, 256), (64, 1024, 544, 257),
+                                              (64, 1024, 544, 512), (64, 1024, 544, 513)])
+def test_large_experts_in_many_runs(lib, experts, N, K, runs):
+    r = Run(lib, False, experts, N, K, 0)
+    which = np.full((runs, 8), -1, dtype=np.int32)
+    for i in range(runs):
+        if i < 3 or i >= runs - 60:
+            which[i, :1 + (5 * i) % 8] = 7 * i % experts
+    which = which.reshape(-1)
+    rows, live = 16 * len(which), np.repeat(which, 16) >= 0
+    x = r.act(rows, K)
+    xd, gd = r.up(x), hipattn.DeviceBuffer.from_host(which.view(np.float32))
+    y = hipattn.DeviceBuffer.from_host(np.full((rows, N), 7.0, dtype=np.float32))
+    r.go(xd, rows=rows, group_expert=gd.p, tile_groups=8, out=ROWS_F32, y_f32=y.p, ldy=N)
+    got = y.to_host((rows, N))
+    r.close(got[live], np.concatenate([x[16 * g:16 * g + 16].astype(np.float64) @ r.w[e].T.astype(np.float64) for g, e in enumerate(which) if e >= 0]))
+    assert np.all(got[np.repeat(which[::8], 128) < 0] == 7.0)
+    r.end()
+    for b in (xd, gd, y):
+        b.free()
+
+
 @pytest.mark.parametrize("order", ["together", "scattered"])
 @pytest.mark.parametrize("experts,N,K", LARGE)
 def test_large_experts_in_single_groups(lib, experts, N, K, order):

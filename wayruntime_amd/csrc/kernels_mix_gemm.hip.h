@@ -388,7 +388,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
 // 48, picked one by one 76 / 53, 4096 -> 384 85 / 39.
 // Tried: two chunks of rows on their way (51.7 -> 54.5), four tiles to a wave (60 -> 65), one (60 -> 58.6 but 1024 -> 2048
 // 62 -> 65), two waves (62); a loop over pieces around this (spills, 52 -> 60).
-constexpr uint32_t kMixMaxPieces = 512;                    // groups (SINGLE) or runs that pieces are cut from
+// What pieces are cut from, at most: a wave finds them with a ballot for every 64.
+constexpr uint32_t kMixStreamRuns = 256, kMixStreamGroups = 512;       // (groups: SINGLE)
 
 // The launch's arguments, read again: what a kernel's end needs of them is not kept through its loops.
 __device__ __forceinline__ const MixGemmArgs& mix_fresh_args()
@@ -432,7 +433,9 @@ __device__ __forceinline__ void mix_gemm_scattered(const MixGemmArgs& a, uint32_
 template <int NT, int WAVES, int KC, bool SINGLE>
 __global__ __launch_bounds__(WAVES * 64, 2) void mix_gemm_runs_kernel(const MixGemmArgs a)
 {
-    constexpr int GR = 8, D = 2 * KC, WORDS = (SINGLE ? kMixMaxPieces : 256) / 64, RUN = SINGLE ? 1 : GR;
+    constexpr uint32_t MOST = SINGLE ? kMixStreamGroups : kMixStreamRuns;
+    static_assert(MOST % 64 == 0);
+    constexpr int GR = 8, D = 2 * KC, WORDS = MOST / 64, RUN = SINGLE ? 1 : GR;
     __shared__ bf16x8 s_x[2][KC * GR * 64];
     const int lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -735,7 +735,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
             // in tiles at any number (768 outputs of 128 experts at 128 rows 132 / 184, 1536 of 64 at 384 375 / 400).
             // Beyond 96 rows sixteen tiles to a workgroup, unless they come out badly (64 experts, 2048 -> 1024 at 256 rows, eight /
             // sixteen: 138 / 132; 128 experts, 768 outputs 194 / 180; 384 outputs 109 / 145).
-            if (runs <= kMixMaxPieces && spare >= e * (mib < 160 ? 44 : 1) && streams(a, e)) {
+            if (runs <= kMixStreamRuns && spare >= e * (mib < 160 ? 44 : 1) && streams(a, e)) {
                 const uint64_t most = a.ktiles <= 16 ? 72 : a.ntiles % 128 ? 1u << 20 : e >= 48 && a.ntiles * a.ktiles <= 6144 ? 144 : 104;
                 const bool wide = (a.ntiles + 15) / 16 * 16 * 10 <= a.ntiles * 11;
                 if (spare <= e * most) return spare > e * 96 && wide ? launch_stream<2, 8, 2, false>(a, e) : launch_stream<2, 4, 4, false>(a, e);
@@ -752,7 +752,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
         }
         if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 8, true>(a, 1);
         const uint64_t e = q->w->batch, spare = a.groups > e ? (a.groups - e) * 16 : 0;
-        if (a.groups <= kMixMaxPieces && streams(a, e)) {
+        if (a.groups <= kMixStreamGroups && streams(a, e)) {
             // From so many rows an expert (us, without / with, as below): in order 12, 20 where the weights are less than 160 MiB (16
             // experts, 1408 -> 2048 at 13 rows 18.8 / 20.9) and 24 over short ranges (64, 512 -> 2048 at 17 30.6 / 33.5); picked
             // one by one, which all workgroups of the others do again, 4 over long ranges (32, 4096 -> 4096 182 / 167), 5 else (six of 64,
