@@ -531,7 +531,8 @@ int  wr_hip_attn_step_done(void);
 void wr_hip_attn_set_step_limit(uint32_t ticks);
 void wr_hip_attn_step_set_tag(wr_hip_attn_step *step, uint32_t tag);
 
-/* For tests: of the allocations of device memory from now on `after` are made and then `n` fail (0: none does). */
+/* For tests: of the allocations of device memory and of page-locked host memory from now on `after` are made and then `n` fail
+ * (0: none does). */
 void wr_hip_attn_set_alloc_failures(uint32_t n, uint32_t after);
 
 /* Tuning knobs for measurement (0 = automatic): keys handled per workgroup in

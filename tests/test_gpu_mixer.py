@@ -298,6 +298,31 @@ def test_greedy_generation(eng, tmp_path):
     case.close()
 
 
+def test_session_without_page_locked_logits(eng, tmp_path, prec):
+    # no page-locked memory for a session's logits: it keeps them in ordinary memory, and nothing else about it differs
+    case = Case(eng, tmp_path, stack(prec), prec)
+    t = case.tokens(12)
+    ss, lib = [case.m.session()], hipattn.lib()
+    lib.wr_hip_attn_set_alloc_failures(1, 0)
+    try:
+        ss.append(case.m.session())
+        spare = lib.wr_hip_attn_dev_alloc(64)                  # (the refusal was the session's)
+    finally:
+        lib.wr_hip_attn_set_alloc_failures(0, 0)
+    assert spare
+    first = [s.step(int(t[0])) for s in reversed(ss)]          # the one without ahead of all others
+    assert first[0] is not None and np.array_equal(*first)
+    for k in (1, 2):
+        rc, lg = E.batch_step(ss, [int(t[k])] * 2)
+        assert rc == 2 and np.array_equal(*lg)
+        case.check(np.stack(lg), case.oracle(t[:k + 1])[[k, k]], "two sessions", deep=True)
+    assert np.array_equal(*[s.step(int(t[3])) for s in ss])
+    lib.wr_hip_attn_dev_free(spare)
+    for s in ss:
+        s.close()
+    case.close()
+
+
 def test_failed_step_changes_nothing(eng, tmp_path, prec):
     case = Case(eng, tmp_path, stack(prec), prec)
     t = case.tokens(100)

@@ -168,19 +168,33 @@ void slab_leave(uint8_t* p, size_t bytes)
     slabs_free(out);
 }
 
+// For tests (wr_hip_attn_set_alloc_failures): true where an allocation is to fail, with a call's error left behind as a refused
+// allocation leaves its own.
+static bool alloc_refused()
+{
+    if (!g.fail_allocs.load(std::memory_order_relaxed) || count_down(g.fail_after) || !count_down(g.fail_allocs)) return false;
+    (void)hipSetDevice(-1);
+    return true;
+}
+
 // hipMalloc that what is kept makes room for.
 hipError_t device_malloc(void** p, size_t bytes)
 {
-    const auto take = [&] {
-        if (g.fail_allocs.load(std::memory_order_relaxed) && !count_down(g.fail_after) && count_down(g.fail_allocs)) return hipErrorOutOfMemory;
-        return hipMalloc(p, bytes);
-    };
+    const auto take = [&] { return alloc_refused() ? hipErrorOutOfMemory : hipMalloc(p, bytes); };
     hipError_t e = take();
     if (e != hipSuccess && slabs_trim()) {
         (void)hipGetLastError();
         e = take();
     }
     if (e != hipSuccess) (void)hipGetLastError();          // (the caller may do without: not for the next launch's check to find)
+    return e;
+}
+
+// hipHostMalloc: no error of it is left behind either.
+static hipError_t host_malloc(void** p, size_t bytes, unsigned flags = hipHostMallocDefault)
+{
+    const hipError_t e = alloc_refused() ? hipErrorOutOfMemory : hipHostMalloc(p, bytes, flags);
+    if (e != hipSuccess) (void)hipGetLastError();
     return e;
 }
 
@@ -235,7 +249,7 @@ int ensure_pinned(Buffer& b, size_t need)
     b.p = nullptr;
     b.cap = 0;
     const size_t want = need + need / 2 + 4096;
-    HIP_TRY(hipHostMalloc(&b.p, want, hipHostMallocDefault), "pinned alloc", 0);
+    HIP_TRY(host_malloc(&b.p, want), "pinned alloc", 0);
     b.cap = want;
     return WR_HIP_OK;
 }
@@ -840,7 +854,7 @@ Ctx* ctx_create()
     if (rc == WR_HIP_OK) {
         void* hp = nullptr;
         void* dp = nullptr;
-        e = hipHostMalloc(&hp, 64, hipHostMallocMapped);
+        e = host_malloc(&hp, 64, hipHostMallocMapped);
         if (e == hipSuccess) e = hipHostGetDevicePointer(&dp, hp, 0);
         if (e != hipSuccess) {
             rc = hip_fail(e, "error word", 0);
@@ -2229,7 +2243,7 @@ void* wr_hip_attn_host_alloc(size_t bytes)
     Entered entered_;
     if (!entered_.ok()) return nullptr;
     void* p = nullptr;
-    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) return nullptr;
+    if (host_malloc(&p, bytes) != hipSuccess) return nullptr;
     return p;
 }
 
