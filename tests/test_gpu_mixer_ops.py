@@ -622,7 +622,7 @@ class StepOf:
 # that a workgroup holds in registers (4096) and more.
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("width", [2048, 4200])
-@pytest.mark.parametrize("kind", ["plain", "no_fragment", "pair", "embed", "experts"])
+@pytest.mark.parametrize("kind", ["plain", "no_fragment", "no_norm", "pair", "embed", "experts"])
 def test_row_steps_of_many_rows(lib, f32, width, kind):
     rng = np.random.default_rng(width)
     counts = (64, 1791, 1792, 1793) if kind == "experts" else (64, 599, 600, 601, 1501)
@@ -651,7 +651,7 @@ def test_row_steps_of_many_rows(lib, f32, width, kind):
         g = np.where(slot == 0xFFFFFFFF, 0.0, gate).astype(np.float64)
         want = want + norm((g[:, :, None] * y[np.minimum(slot, most - 1)]).sum(axis=1)) * post
     else:
-        want = want + norm(y) * post + add
+        want = want + (y if kind == "no_norm" else norm(y) * post) + add
         if kind == "pair":
             want = want + norm(pairs[0]) * post2[0] + norm(pairs[1]) * post2[1]
     yd, ad, pd, nd, td = up(y), up(add), up(post), up(nxt), up(table)
@@ -663,8 +663,8 @@ def test_row_steps_of_many_rows(lib, f32, width, kind):
         if kind == "embed":
             assert lib.wr_hip_mix_embed(s.h, int(f32), td.p, width, pd.p, 1.0, eps, xd.p, None, nd.p, hd.p) == 0
         else:
-            a = Resid(width=width, eps=eps, x=xd.p, y=yd.p, post=pd.p)
-            if kind != "no_fragment":
+            a = Resid(width=width, eps=eps, x=xd.p, y=yd.p, post=None if kind == "no_norm" else pd.p)
+            if not kind.startswith("no_"):
                 a.next, a.h = nd.p, hd.p
             if kind == "experts":
                 a.gate, a.slot, a.top = gd.p, sd.p, top
@@ -678,7 +678,7 @@ def test_row_steps_of_many_rows(lib, f32, width, kind):
         got = [xd.to_host((n, wpad))]
         scale = np.abs(want).max()
         assert np.abs(got[0] - want[:n]).max() < 2e-6 * scale, (kind, n)      # (32-bit sums of some thousand terms)
-        if kind != "no_fragment":
+        if not kind.startswith("no_"):
             m = -(-n // 16) * 16 * wpad
             h = unfrag(hd.to_host((m,)) if f32 else O.bf16_to_f32(hd.to_host((m // 2,)).view(np.uint16)), n, wpad)
             ref = norm(want[:n]) * nxt

@@ -27,19 +27,18 @@ __device__ __forceinline__ uint32_t mix_row_chunk()
     return PAIRED ? t / 64 * 32 + t % 32 + t / 32 % 2 * 128 : t / RPW;
 }
 
-// (PAIRED: in the lower lane; all lanes take part)
-template <bool PAIRED>
-__device__ __forceinline__ float mix_add_squares(float ss, const float (&v)[8], bool there)
+__device__ __forceinline__ float mix_add_squares(float ss, const float (&v)[8])
 {
-    const auto add = [&](float s) {
-        if (there) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) s = fmaf(v[j], v[j], s);
-        }
-        return s;
-    };
-    if constexpr (!PAIRED) return add(ss);
-    return wave_xor_f32(add(wave_xor_f32(add(ss), 32)), 32);
+    for (int j = 0; j < 8; j++) ss = fmaf(v[j], v[j], ss);
+    return ss;
+}
+
+// (the sum is the lower lane's; all lanes take part)
+__device__ __forceinline__ float mix_add_paired(float ss, const float (&v)[8], bool there)
+{
+    ss = wave_xor_f32(there ? mix_add_squares(ss, v) : ss, 32);
+    return wave_xor_f32(there ? mix_add_squares(ss, v) : ss, 32);
 }
 
 // Sum over the threads of a row; every thread gets its row's sum.
@@ -244,15 +243,21 @@ __global__ __launch_bounds__(MixRowShape<RPW>::kThreads) void mix_residual_kerne
 #pragma unroll
             for (int i = 0; i < CH; i++) {
                 const uint32_t q = lr + i * Sh::kPerRow;
-                if (q < nq) first(q, held[i]);
-                ss = mix_add_squares<PAIRED>(ss, held[i], q < nq);
+                if (q < nq) {
+                    first(q, held[i]);
+                    if constexpr (!PAIRED) ss = mix_add_squares(ss, held[i]);
+                }
+                if constexpr (PAIRED) ss = mix_add_paired(ss, held[i], q < nq);
             }
         } else {
             for (uint32_t q0 = 0; q0 < nq; q0 += Sh::kPerRow) {
                 const uint32_t q = lr + q0;
                 float v[8];
-                if (q < nq) first(q, v);
-                ss = mix_add_squares<PAIRED>(ss, v, q < nq);
+                if (q < nq) {
+                    first(q, v);
+                    if constexpr (!PAIRED) ss = mix_add_squares(ss, v);
+                }
+                if constexpr (PAIRED) ss = mix_add_paired(ss, v, q < nq);
             }
         }
         if (normed) inv = 1.0f / sqrtf(mix_row_sum<RPW, PAIRED>(ss, red) * invw + a.eps);
@@ -267,14 +272,20 @@ __global__ __launch_bounds__(MixRowShape<RPW>::kThreads) void mix_residual_kerne
 #pragma unroll
                 for (int i = 0; i < CH; i++) {
                     const uint32_t q = lr + i * Sh::kPerRow;
-                    if (q < nq) mix_load8(p + q * 8, pair[k][i]);
-                    ps = mix_add_squares<PAIRED>(ps, pair[k][i], q < nq);
+                    if (q < nq) {
+                        mix_load8(p + q * 8, pair[k][i]);
+                        if constexpr (!PAIRED) ps = mix_add_squares(ps, pair[k][i]);
+                    }
+                    if constexpr (PAIRED) ps = mix_add_paired(ps, pair[k][i], q < nq);
                 }
             } else {
                 for (uint32_t q0 = 0; q0 < nq; q0 += Sh::kPerRow) {
                     const uint32_t q = lr + q0;
-                    if (q < nq) mix_load8(p + q * 8, pair[k][0]);
-                    ps = mix_add_squares<PAIRED>(ps, pair[k][0], q < nq);
+                    if (q < nq) {
+                        mix_load8(p + q * 8, pair[k][0]);
+                        if constexpr (!PAIRED) ps = mix_add_squares(ps, pair[k][0]);
+                    }
+                    if constexpr (PAIRED) ps = mix_add_paired(ps, pair[k][0], q < nq);
                 }
             }
             pinv[k] = 1.0f / sqrtf(mix_row_sum<RPW, PAIRED>(ps, red) * invw + a.eps);
@@ -334,8 +345,11 @@ __global__ __launch_bounds__(MixRowShape<RPW>::kThreads) void mix_residual_kerne
 #pragma unroll
         for (int i = 0; i < CH; i++) {
             const uint32_t q = lr + i * Sh::kPerRow;
-            if (q < nq) second(q, held[i], i);
-            ss = mix_add_squares<PAIRED>(ss, held[i], q < nq);
+            if (q < nq) {
+                second(q, held[i], i);
+                if constexpr (!PAIRED) ss = mix_add_squares(ss, held[i]);
+            }
+            if constexpr (PAIRED) ss = mix_add_paired(ss, held[i], q < nq);
         }
     } else {
         for (uint32_t q0 = 0; q0 < nq; q0 += Sh::kPerRow) {
@@ -344,8 +358,9 @@ __global__ __launch_bounds__(MixRowShape<RPW>::kThreads) void mix_residual_kerne
             if (q < nq) {
                 if (some) first(q, v);
                 second(q, v, 0);
+                if constexpr (!PAIRED) ss = mix_add_squares(ss, v);
             }
-            ss = mix_add_squares<PAIRED>(ss, v, q < nq);
+            if constexpr (PAIRED) ss = mix_add_paired(ss, v, q < nq);
         }
     }
     if (!a.next) return;                                   // uniform

@@ -344,8 +344,10 @@ static int launch_residual(int f32, bool embed, const MixRowArgs& a)
     // one, and not for so few rows that compute units stay without (width 2048, us, four / one: 512 rows 5.7 / 5.5, 700 5.9 / 6.2,
     // 2047 10.8 / 15.3; with six experts' rows to add 100 rows 10.9 / 4.8, 512 12.1 / 8.3, 1500 22.6 / 19.0, 2047 24.0 / 26.1; these
     // without a fragment 512 11.0 / 5.5, 2047 22.5 / 20.8).  From 64 rows on one row's sums are made in the order of four's
-    // (PAIRED: 0 to 0.5 us), so that a row's bits do not hang on how many others there are.
-    const bool many = a.next && a.rows >= (a.top ? 1792u : 600u), few = a.rows < 64, held = a.wpad <= 4096, pair = a.pair_y[0] != nullptr;
+    // (PAIRED: 0 to 0.5 us), so that a row's bits do not hang on how many others there are; not where nothing is normed, which
+    // takes no sums.
+    const bool many = a.next && a.rows >= (a.top ? 1792u : 600u), held = a.wpad <= 4096, pair = a.pair_y[0] != nullptr;
+    const bool few = a.rows < 64 || (!a.next && !pair && !(embed ? a.norm : a.post));
 #define WR_RESID_ROWS(F, EMB, PAIR, RPW, PAIRED)                                                    \
     do {                                                                                            \
         const dim3 grid((a.rows + RPW - 1) / RPW), block(MixRowShape<RPW>::kThreads);               \
