@@ -475,6 +475,7 @@ def test_rows_whose_workgroups_make_their_own_terms(rows, n_in, n_out):
     (1, 15360, 2064), (1, 15360, 32), (1, 15392, 32),             # ... more than 64 KiB of LDS, the most inputs, fragments apart
     (2, 512, 16), (16, 1024, 3072), (8, 1536, 2064), (9, 512, 4080),   # workgroups that make their own terms: a pair, two
     (24, 1024, 1024), (20, 1024, 2048), (17, 2048, 528), (100, 512, 272),    # ... more than two row groups, the last ones short
+    (17, 1024, 2736), (17, 1024, 2752), (40, 1024, 3264), (40, 512, 3280), (33, 1536, 2064),    # ... up to one a CU, two, more, no such form
     (5, 1056, 528), (16, 160, 48), (16, 1024, 16400),             # a wave per pair of tiles, inputs split and not
     (17, 1056, 528), (17, 800, 1376), (100, 288, 2064), (17, 800, 2736), (17, 1056, 4128),    # register tiles of 32 x 8, 32 x 16 (two), 32 x 32, 64 x 32
     (130, 1088, 4944), (200, 1056, 8208),                         # LDS tiles of 128 x 64 (few, two sets of waves; two a CU)

@@ -1093,15 +1093,21 @@ FusedKernel fused_kernel(int src, uint32_t n_in, uint32_t nt, bool gated)
 // Rows: four to a workgroup where there are CUs for it, eight otherwise, at the same number of tiles.  Halving the rows
 // for twice the tiles would double the weights that a CU has to take in (46 bytes a nanosecond at best): not done.
 //
-// Gated weights have a second workgroup on a CU up to 40 rows: the launch that makes the fragments costs more than terms made
-// twice (1024 -> 2 x 3072, apart / so: 17 rows 8.9 / 7.9 us, 32 9.2 / 8.7, 40 10.9 / 8.9, 45 11.0 / 11.1; plain 1024 -> 4096
-// 32 rows 6.6 / 7.7, 3072 -> 1024 40 rows 9.6 / 13.5).
+// Gated weights of 17 to 40 rows that are too wide for that have a second workgroup on a CU, of four tiles and eight rows each, which is built
+// for 512 and 1024 inputs: the launch that makes the fragments costs more than terms made twice (norm, us, apart / so: 1024 -> 2 x
+// 2048, 33 rows 8.9 / 7.7; -> 2 x 3072, 17 rows 9.6 / 8.3, 32 9.8 / 8.8, 40 11.3 / 8.9; -> 2 x 5120, 24 rows 12.6 / 10.0; 512 -> 2 x
+// 3072, 40 rows 8.8 / 5.6; without a norm 1024 -> 2 x 4096, 24 rows 8.5 / 8.8, 32 8.7 / 8.8, the others gain 2 to 33 %).
+// Where one workgroup of four tiles fits, two of two tiles lose (1024 -> 2 x 1536, 24 rows 6.1 / 6.9; 2048 -> 2 x 2048 11.3 /
+// 14.9), and so do weights that are not gated (1024 -> 4096, 32 rows 6.6 / 7.7, 3072 -> 1024, 40 rows 9.6 / 13.5).
 FusedKernel pick_fused(int src, uint32_t n_in, uint32_t tiles, uint32_t rows, bool gated, uint32_t* nt, uint32_t* wg_rows)
 {
     for (*nt = gated ? 2 : 1; *nt <= 4; *nt += gated ? 2 : 1)
         for (*wg_rows = 4; *wg_rows <= 8; *wg_rows *= 2)
-            if ((tiles + *nt - 1) / *nt * ((rows + *wg_rows - 1) / *wg_rows) <= (uint32_t)g.n_cus * (gated && rows > 16 && rows <= 40 && *wg_rows == 8 ? 2 : 1))
+            if ((tiles + *nt - 1) / *nt * ((rows + *wg_rows - 1) / *wg_rows) <= (uint32_t)g.n_cus)
                 return *wg_rows == 4 ? fused_kernel<4>(src, n_in, *nt, gated) : fused_kernel<8>(src, n_in, *nt, gated);
+    *nt = 4;
+    *wg_rows = 8;
+    if (gated && rows > 16 && rows <= 40 && (tiles + 3) / 4 * ((rows + 7) / 8) <= 2 * (uint32_t)g.n_cus) return fused_kernel<8>(src, n_in, 4, true);
     return nullptr;
 }
 
