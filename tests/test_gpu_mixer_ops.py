@@ -196,6 +196,25 @@ def test_batch_of_matrices(lib, f32, batch, N, K, rows):
         b.free()
 
 
+# ... in tiles of 256 outputs by 128 and 256 rows, the matrices on XCDs of their own (batches of 2, 4 and 8) and on all of them
+@pytest.mark.parametrize("batch,N,K,rows", [(2, 7584, 2080, 400), (4, 7712, 2080, 130), (8, 4000, 2080, 130), (3, 6688, 2080, 280),
+                                            (2, 7328, 1056, 910), (4, 7328, 1056, 400), (8, 7584, 1056, 130), (3, 6560, 1056, 670)])
+def test_batch_of_matrices_in_wide_tiles(lib, batch, N, K, rows):
+    r = Run(lib, False, batch, N, K, rows)
+    x = r.act(rows, (batch + 1) * K)
+    xd, h = r.up(x), hipattn.DeviceBuffer(-(-rows // 16) * 16 * N * batch * 2)
+    y = hipattn.DeviceBuffer(rows * batch * N * 4)
+    place = dict(x_kt=(batch + 1) * K // 32, x_kt_z=K // 32, x_kt0=K // 32, col_z=N)
+    want = np.concatenate([x[:, (z + 1) * K:(z + 2) * K].astype(np.float64) @ r.w[z].T.astype(np.float64) for z in range(batch)], axis=1)
+    r.go(xd, out=FRAG, h=h.p, h_kt=batch * N // 32, **place)
+    r.close(r.frag_down(h, rows, batch * N), want, eight_bits=True)
+    r.go(xd, out=ROWS_F32, y_f32=y.p, ldy=batch * N, **place)
+    r.close(y.to_host((rows, batch * N)), want)
+    r.end()
+    for b in (xd, h, y):
+        b.free()
+
+
 # every tile the rule picks among: register tiles of 1 x 1, 1 x 2, 2 x 1 (gated outputs), 2 x 2, 2 x 3, 2 x 4, 4 x 3, 4 x 4 (outputs x rows,
 # sixteens; gated outputs take even ones), LDS tiles of 64, 128 and 256 rows.  Input ranges that leave waves without
 # k-steps (96), that are less than a turn of eight and a turn and a rest of four (800), and that split unevenly with

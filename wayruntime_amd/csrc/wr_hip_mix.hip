@@ -555,7 +555,8 @@ template <int GROUPS, int KS = 1, int WN = 2>
 static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 {
     constexpr uint32_t TILES = 4 * WN;
-    int rc = allow_lds<mix_gemm_lds_kernel<GROUPS, KS, WN>>(mix_gemm_lds_bytes<GROUPS, KS, WN>());
+    constexpr size_t lds = mix_gemm_lds_bytes<GROUPS, KS, WN>();
+    int rc = batch > 1 ? allow_lds<mix_gemm_lds_kernel<GROUPS, KS, WN, true>>(lds) : allow_lds<mix_gemm_lds_kernel<GROUPS, KS, WN>>(lds);
     if (rc) return rc;
     MixGemmArgs a = args;
     const uint32_t nx = (a.ntiles + TILES - 1) / TILES, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
@@ -563,7 +564,8 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
     if (!a.group_expert)
         a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, KS == 2 || WN == 4 ? 32 : 64, &blocks,
                           batch > 1 ? mix_batch_xcds(batch) : 8);
-    launch_main(mix_gemm_lds_kernel<GROUPS, KS, WN>, dim3(blocks, batch), dim3(128 * WN * KS), a, mix_gemm_lds_bytes<GROUPS, KS, WN>());
+    launch_main(batch > 1 ? mix_gemm_lds_kernel<GROUPS, KS, WN, true> : mix_gemm_lds_kernel<GROUPS, KS, WN>, dim3(blocks, batch),
+                dim3(128 * WN * KS), a, lds);
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
 }
