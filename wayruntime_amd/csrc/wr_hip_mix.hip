@@ -570,6 +570,18 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
     return WR_HIP_OK;
 }
 
+constexpr uint32_t kXcdUnits = 32;
+
+// Workgroups of tiles x groups tiles, one to a compute unit at a time, that the XCD with the most of them has.
+static uint32_t busiest_xcd(const MixGemmArgs& a, uint32_t tiles, uint32_t groups, uint32_t batch)
+{
+    const uint32_t n = batch > 1 ? mix_batch_xcds(batch) : 8;
+    uint32_t blocks = 0;
+    xcd_cols((a.ntiles + tiles - 1) / tiles, (a.groups + groups - 1) / groups, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024,
+             kXcdUnits, &blocks, n);
+    return (uint32_t)((uint64_t)blocks * batch / 8);       // (a matrix has `n` of the eight, and 8 / n have theirs at the same time)
+}
+
 // Products of 17 rows and more, bfloat16: the form whose estimate is the least.  A register tile of NT x GR waits for
 // NT + GR KiB a k-step through a compute unit's vector cache, workgroup after workgroup; an LDS tile for its barrier
 // and its operands' latency per k-step, or, with several workgroups on a unit, for its share of the matrix pipes.
@@ -584,15 +596,21 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
 // leaves units without a workgroup less, as the others then have the clock and the caches. Against the tile of 128 x 256,
 // whose ends those figures split off too: 2047 rows, 2048 -> 32 768 into 32-bit rows 315 / 266 us, -> 14 400 137 / 114, 4096 -> 24 576 gated
 // 320 / 299; 2500 rows, 2048 -> 16 384, two and a half rounds, 142 / 156: the other tile's.
+// Where 32-bit rows go out all LDS tiles have ends that count from 1024 inputs on: 2, 4 and 11 us for a tile's share of the three, 4
+// and 10 for each round of two sets of waves behind the first.  (With those of the largest alone the tile of 128 x 128 seemed better than it is: 2048 ->
+// 14 400, 128 x 128 / 256 x 256: 2047 rows 148 / 116, 3000 223 / 174; four of 1024 -> 4096, 2047 rows 125 / 73.)
+// Rounds of one workgroup a unit are counted where they run, on the XCD with the most (1800 rows, 2048 -> 4160 into 32-bit rows: 17
+// x 15 tiles of 256 x 128 are a round of 255 and on one XCD 34 for 32 units: 62 us, 48 in tiles of 128 x 128).
 // Gated outputs take an even number of tiles: of one group of rows each where that spreads few tiles over more units
 // (64 rows, 8192 -> 512: 17.4 us in tiles of two groups, 13.2; 2048 -> 2048 6.9, 5.7).  Tiles of 256 rows are counted in
 // whole workgroups per unit where all run at once (1500 rows, 256 -> 8192: 17.8 us against 16.3 with tiles of 128;
 // beyond two a unit, places are filled as they come free: 2047 rows, 2048 -> 14 400 161 us, 170 with tiles of 128).
-// Over 11 row counts from 17 to 2047, 8 input ranges and 4 widths (profiles/stack_product_forms.txt has every form's
-// time) the form picked is 2.3 % off the best one on average, 30 % (1 us of 4) at worst.
+// profiles/stack_product_forms.txt has every form's time for 772 sizes, into fragments, into 32-bit rows, gated and in
+// batches: the form picked is 2.0 % off the best one on average, more than 10 % for 43 of them (59 % at worst: 300 rows, 4096 -> 4160).
 static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
 {
-    const bool rows32 = a.out == kMixOutRowsF32;
+    // 32-bit rows, or most of them (an input product of the parallel halves: 64 of 14 400 outputs are a fragment's)
+    const bool rows32 = a.out == kMixOutRowsF32 || (a.out == kMixOutSplit && a.n_split < a.ntiles * 8);
     struct Form {
         uint32_t nt, gr;
         int (*launch)(const MixGemmArgs&, uint32_t);
@@ -603,10 +621,14 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
                                  {4, 3, launch_split<false, 4, 3, 4, 4, false>}, {4, 4, launch_split<false, 4, 4, 4, 2, false>}};
     static const struct {
         uint32_t groups;
-        float step, share;
+        float step, share, share32, ends32;
         int (*launch)(const MixGemmArgs&, uint32_t);
-    } lds[] = {{4, 0.34f, 0.177f, launch_lds<2>}, {8, 0.39f, 0.27f, launch_lds<4>}, {16, 0.58f, 0.5f, launch_lds<8>}},
-      halves[] = {{4, 0.26f, 0.f, launch_lds<2, 2>}, {8, 0.28f, 0.f, launch_lds<4, 2>}};
+    } lds[] = {{4, 0.34f, 0.177f, 0.177f, 2.f, launch_lds<2>}, {8, 0.39f, 0.27f, 0.26f, 4.f, launch_lds<4>}, {16, 0.58f, 0.5f, 0.435f, 11.f, launch_lds<8>}};
+    static const struct {
+        uint32_t groups;
+        float step, ends32;
+        int (*launch)(const MixGemmArgs&, uint32_t);
+    } halves[] = {{4, 0.26f, 4.f, launch_lds<2, 2>}, {8, 0.28f, 10.f, launch_lds<4, 2>}};
     static const struct {
         uint32_t groups;
         float full, part, more, ends, rows32;
@@ -629,19 +651,25 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
             const uint64_t wgs = (uint64_t)((a.ntiles + 7) / 8) * ((a.groups + f.groups - 1) / f.groups) * batch;
             const bool at_once = f.groups == 16 && wgs <= 2 * g.n_cus;
             const float each = at_once ? (float)((wgs + g.n_cus - 1) / g.n_cus) : (float)wgs / g.n_cus;
-            const float share = f.groups == 16 && a.ktiles >= 32 ? 0.435f + (rows32 ? 11.f : 4.f) / (float)a.ktiles : f.share;
-            offer(std::max(f.step, share * each), f.launch);
+            float step = f.step, share = f.share;
+            if (a.ktiles >= 32 && rows32) {
+                share = f.share32 + f.ends32 / (float)a.ktiles;
+                if (f.groups == 8) step += f.ends32 / (float)a.ktiles;
+            } else if (a.ktiles >= 32 && f.groups == 16) {
+                share = 0.435f + 4.f / (float)a.ktiles;
+            }
+            offer(std::max(step, share * each), f.launch);
         }
     if (a.groups >= 4 && a.ktiles >= 32)
         for (const auto& f : piped) {
-            const uint64_t wgs = (uint64_t)((a.ntiles + 15) / 16) * ((a.groups + f.groups - 1) / f.groups) * batch;
-            const float ends = (f.ends + (rows32 ? f.rows32 : 0.f)) / (float)a.ktiles, left = (float)(wgs % g.n_cus) / (float)g.n_cus;
-            offer((float)(wgs / g.n_cus) * (f.full + ends) + (left > 0.f ? f.part + f.more * left + ends + (wgs > g.n_cus ? 0.08f : 0.f) : 0.f), f.launch);
+            const uint32_t wgs = busiest_xcd(a, 16, f.groups, batch);
+            const float ends = (f.ends + (rows32 ? f.rows32 : 0.f)) / (float)a.ktiles, left = (float)(wgs % kXcdUnits) / (float)kXcdUnits;
+            offer((float)(wgs / kXcdUnits) * (f.full + ends) + (left > 0.f ? f.part + f.more * left + ends + (wgs > kXcdUnits ? 0.08f : 0.f) : 0.f), f.launch);
         }
     if (a.groups >= 4 && a.ktiles % 2 == 0 && a.ktiles >= 64)
         for (const auto& f : halves) {
-            const uint64_t wgs = (uint64_t)((a.ntiles + 7) / 8) * ((a.groups + f.groups - 1) / f.groups) * batch;
-            offer(f.step * (float)((wgs + g.n_cus - 1) / g.n_cus), f.launch);
+            const float rounds = (float)((busiest_xcd(a, 8, f.groups, batch) + kXcdUnits - 1) / kXcdUnits);
+            offer(f.step * rounds + (rows32 ? f.ends32 * (rounds - 1) / (float)a.ktiles : 0.f), f.launch);
         }
     return best(a, batch);
 }
