@@ -84,6 +84,16 @@ def test_wide_rows(eng, tmp_path, prec):
     case.close()
 
 
+def test_prompt_of_many_expert_runs(eng, tmp_path):
+    # 520 rows that go to all of 64 experts: 320 runs of 128 rows, both products' weights 64 MiB; in portions of 100 rows 64 runs
+    case = Case(eng, tmp_path, mw.config(512, 50, [(mw.lightning(1, 16, 16, decay=[0.9]), mw.moe(64, 64, 1024))]), "bf16")
+    t = case.tokens(520)
+    parts = run_cut(case, t, [100])
+    case.check(parts[:10], case.oracle(t[:10]), "portions")
+    case.check(run_cut(case, t, [520]), parts.astype(np.float64), "whole")
+    case.close()
+
+
 def stack(prec):
     """Several layers, part of them looped.  In bfloat16 every expert is used: a choice among random experts
     now and then hangs on less than bfloat16 resolves."""
