@@ -766,11 +766,13 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
             // 2048 at 128 120 / 127, at 150 136 / 134), short input ranges at 72 (512 -> 2048 at 96 56 / 52); others are slower
             // in tiles at any number (768 outputs of 128 experts at 128 rows 132 / 184, 1536 of 64 at 384 375 / 400).
             // Beyond 96 rows sixteen tiles to a workgroup, unless they come out badly (64 experts, 2048 -> 1024 at 256 rows, eight /
-            // sixteen: 138 / 132; 128 experts, 768 outputs 194 / 180; 384 outputs 109 / 145).
+            // sixteen: 138 / 132; 128 experts, 768 outputs 194 / 180; 384 outputs 109 / 145), and up to 112 unless units would be left with none
+            // (13 experts, 1280 -> 2048 at 104 rows, 208 workgroups of eight or 104 of sixteen: 23.6 / 31.3, tiles 23.6; 16, 4096 -> 1536 52 / 74).
             if (runs <= kMixStreamRuns && spare >= e * (mib < 160 ? 44 : 1) && streams(a, e)) {
                 const uint64_t most = a.ktiles <= 16 ? 72 : a.ntiles % 128 ? 1u << 20 : e >= 48 && a.ntiles * a.ktiles <= 6144 ? 144 : 104;
-                const bool wide = (a.ntiles + 15) / 16 * 16 * 10 <= a.ntiles * 11;
-                if (spare <= e * most) return spare > e * 96 && wide ? launch_stream<2, 8, 2, false>(a, e) : launch_stream<2, 4, 4, false>(a, e);
+                const bool wide = spare > e * 96 && (a.ntiles + 15) / 16 * 16 * 10 <= a.ntiles * 11 &&
+                                  (spare > e * 112 || e * ((a.ntiles + 7) / 8) * 16 > g.n_cus * 15);
+                if (spare <= e * most) return wide ? launch_stream<2, 8, 2, false>(a, e) : launch_stream<2, 4, 4, false>(a, e);
                 return launch_lds<4>(a, 1);
             }
             if (spare && spare <= e * 48 && a.ktiles <= 32) return launch_runs<4>(a, q->w->batch);
