@@ -490,12 +490,11 @@ static void pick_rows(MixGemmArgs& a)
     a.x_perm = nullptr;
 }
 
-// Runs of eight groups as a stream of their experts' weights.  A run's workgroups go to one XCD each run where that
+// Runs of eight groups as a stream of their experts' weights through registers.  A run's workgroups go to one XCD each run where that
 // leaves none more than a seventh without work (its rows then come into one L2 and not into eight, which is 8 rows / outputs
-// of the weights' bytes): up to 1536 outputs.  34 rows an expert, dealt out / by XCD (us): 64 experts, 4096 -> 384 64 / 43, -> 512 75
-// / 56, 2048 -> 1024 57 / 53; 128 experts, 2048 -> 768 86 / 79; 16 experts, 4096 -> 1536 46.5 / 40.6.  With more
-// outputs it is no gain (64 experts, 1024 -> 2048 58 / 59) or a loss (32 experts, 4096 -> 4096 199 / 209, 64, 384 ->
-// 4096 65 / 72: eight experts' weights and results at the same offsets).
+// of the weights' bytes): up to 1536 outputs.  Dealt out / by XCD (us) at 20 and 64 rows an expert: 32 experts, 2048 -> 512 17.9 / 14.8, 29.4 /
+// 21.8; 256 111 / 94, 169 / 131; 300, 1024 -> 512 at 64 101 / 85.  With more outputs it is no gain or a loss (12, 768 -> 2048 at 64
+// 15.9 / 19.0; 256, 512 -> 2048 182.5 / 183.7: eight experts' weights and results at the same offsets).
 static bool runs_by_xcd(const MixGemmArgs& a, uint32_t experts)
 {
     return a.ntiles <= 96 && (uint64_t)((experts + 7) / 8 * 8) * 7 <= (uint64_t)experts * 8;
@@ -736,64 +735,48 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     if (q->group_expert) {
         if (!f32 && q->tile_groups == 8) {
             // Rows an expert has on average, from how many groups route leaves room for: a run per expert more than the
-            // pairs fill.  Weights that mix_gemm_runs_kernel is not for: up to 48 the product is a stream of them that reads the rows that there are, and
-            // an expert's weights pass once, against a tile of 128 rows, most of them empty (us, stream / tile: 64
-            // experts, 2048 -> 1024 at 48 rows 58 / 88, 1024 -> 2048 62 / 83; 4096 -> 384 48 / 63; 128 experts, 2048 ->
-            // 768 85 / 128; 32 experts, 2048 -> 512 17.5 / 28.8, 4096 -> 4096 226 / 229; 8 experts, 4096 -> 14 336 202 /
-            // 210; the one that is slower, 16 experts, 1536 -> 4096 50 / 42).  Up to 64 rows where the weights are not so
-            // large that the tile is bound by them too, and the input range not so short that its ends are all of
-            // it (64 experts, 2048 -> 1024 64 / 88, 1024 -> 2048 73 / 83, 3072 -> 1536 149 / 173, 2048 -> 3072 156 / 183; 32
-            // experts, 1024 -> 2048 40 / 41; against 4096 -> 4096 250 / 229, 512 -> 2048 25 / 22.5), and to 80 where the runs
-            // are an XCD's each (64 experts, 2048 -> 1024 68 / 88, 3072 -> 1536 162 / 173, 4096 -> 384 59 / 64; 16
-            // experts, 4096 -> 1536 54 / 60).
-            // Over a short range workgroups of 64 rows, more to a compute unit, up to 48 rows (128 / 64 rows a workgroup:
-            // 64 experts, 384 -> 4096 70 / 58, 512 -> 4096 78 / 70, 1024 -> 2048 64 / 62; 2048 -> 1024 62 / 64; beyond, part of
-            // the experts' weights would pass twice: 1024 -> 2048 at 64 rows 73 / 80).
-            // Beyond 48 rows the tiles are the faster ones again where they come out even: sixteen columns of them, two to
-            // an XCD, that fill the device's last round by seven eighths, up to three rounds (stream / tile at 62 rows: 15
-            // experts, 1280 -> 2048 30.1 / 25.3, 3072 -> 2048 61.4 / 51.2; 32 experts, 768 -> 2048 36.3 / 31.0, 1536 -> 2048
-            // 59.3 / 54.4; 48 experts, 1280 -> 2048 74.3 / 68.2; against 18 experts 32.8 / 37.5 of the first, 34 55.3 / 60.6, and
-            // 16 experts, 1536 -> 3072 45.5 / 46.0), a single round by three quarters (12 experts, 3072 -> 2048 51.8 / 45.4), two
-            // beyond 56 (24 experts, 1408 -> 2048 at 54 rows 42.7 / 43.4, at 62 47.1 / 42.6), but for 1024 and 2048 inputs, whose tiles are slower by a tenth (16 experts 24.2 / 30.5 and
-            // 42.1 / 52.2, 32 42.4 / 46.2 and 71.4 / 75.9).  By XCD the narrowest end at 68 (64 experts, 4096 -> 384
-            // at 66 rows 62.5 / 63.7, at 72 70.3 / 64.8; -> 256 at 80 66 / 57; -> 512 96 / 113).
-            // As many runs as experts, or fewer, are not route's: the caller counted them, so they may be full.
+            // pairs fill.  As many runs as experts, or fewer, are not route's: the caller counted them, so they may be full.
+            // (Figures: us a launch into 16-bit rows; profiles/experts_products.txt has every form's for 67 weights.)
             const uint64_t runs = a.groups / 8, e = q->w->batch, spare = runs > e ? (runs - e) * 128 : 0, mib = e * a.ntiles * a.ktiles >> 10;
-            // Large weights have a kernel of their own, from 44 rows an expert where they are less than 160 MiB (24 experts, 1408 ->
-            // 2048 at 20 rows 30.7 / 31.6, 128, 1024 -> 384 at 41 26.2 / 27.2, us, below / this).  Tiles of 128 rows take over where their
-            // columns share out evenly over the XCDs: at 104 rows (4096 -> 4096 of 32 experts at 96 rows, this / tiles: 241 / 263, at
-            // 128 327 / 312; 1536 -> 4096 of 16 at 112 70 / 64), many experts of few weights at 144 (64, 1024 -> 2048 at 128 89 / 97; 60, 1408 ->
-            // 2048 at 128 120 / 127, at 150 136 / 134), short input ranges at 72 (512 -> 2048 at 96 56 / 52); others are slower
-            // in tiles at any number (768 outputs of 128 experts at 128 rows 132 / 184, 1536 of 64 at 384 375 / 400).
-            // Beyond 96 rows sixteen tiles to a workgroup, unless they come out badly (64 experts, 2048 -> 1024 at 256 rows, eight /
-            // sixteen: 138 / 132; 128 experts, 768 outputs 194 / 180; 384 outputs 109 / 145), and up to 112 unless units would be left with none
+            // Large weights (streams) have a kernel of their own; where they are less than 160 MiB from 44 rows an expert on, below it is
+            // the register stream's turn (split kernel / this: 36 experts, 2048 -> 1024 at 20 rows 29.6 / 34.9; 128, 1024 -> 384 21.5 / 22.7).
+            // Tiles of 128 rows take over where their columns share out evenly over the XCDs: at 104 rows (this / tiles: 32 experts, 4096 ->
+            // 4096 at 96 rows 241 / 266, at 128 303 / 299, at 192 418 / 350; 16, 1536 -> 4096 at 104 56 / 63, at 128 64 / 61), many
+            // experts of few weights at 144 (128, 768 -> 2048 at 112 115 / 140; 64, 1024 -> 2048 at 128 85 / 100).  Others are slower in
+            // tiles at any number (128, 2048 -> 768 at 128 rows 129 / 187; 64, 3072 -> 1536 at 384 358 / 400).
+            // Beyond 96 rows sixteen tiles to a workgroup, unless they come out badly (eight / sixteen: 64, 4096 -> 512 at 160 rows
+            // 101 / 87; 128, 1024 -> 384 at 104 36 / 44), and up to 112 unless units would be left with none
             // (13 experts, 1280 -> 2048 at 104 rows, 208 workgroups of eight or 104 of sixteen: 23.6 / 31.3, tiles 23.6; 16, 4096 -> 1536 52 / 74).
             if (runs <= kMixStreamRuns && spare >= e * (mib < 160 ? 44 : 1) && streams(a, e)) {
-                const uint64_t most = a.ktiles <= 16 ? 72 : a.ntiles % 128 ? 1u << 20 : e >= 48 && a.ntiles * a.ktiles <= 6144 ? 144 : 104;
+                const uint64_t most = a.ntiles % 128 ? 1u << 20 : e >= 48 && a.ntiles * a.ktiles <= 6144 ? 144 : 104;
                 const bool wide = spare > e * 96 && (a.ntiles + 15) / 16 * 16 * 10 <= a.ntiles * 11 &&
                                   (spare > e * 112 || e * ((a.ntiles + 7) / 8) * 16 > g.n_cus * 15);
                 if (spare <= e * most) return wide ? launch_stream<2, 8, 2, false>(a, e) : launch_stream<2, 4, 4, false>(a, e);
                 return launch_lds<4>(a, 1);
             }
+            // Others, and more runs than that kernel takes: up to 48 rows a stream through registers that reads the rows that there are,
+            // where a tile of 128 rows is mostly empty; over a range of 512 inputs at most tiles from there (stream / tile: 64 experts,
+            // 256 -> 1024 at 48 rows 17.1 / 20.0, at 64 20.1 / 20.0; 256, 512 -> 2048 at 48 148 / 178, at 64 181 / 179), others up to 64, and
+            // to 80 where the runs are an XCD's each (32, 2048 -> 512 at 80 23.5 / 31.2; 256 at 80 142 / 176, at 96 172 / 183).
+            // Tiles would be better below 80 where sixteen columns of few experts fill the units evenly: 12, 768 -> 2048 at 72 rows 18.0 / 16.6.
+            // Up to 1024 inputs workgroups of 64 rows, more to a compute unit, up to 48 rows (128 / 64 rows a workgroup: 64 experts, 384 ->
+            // 4096 at 20 rows 62.6 / 48.5, 512 -> 2048 at 32 38.7 / 35.3); beyond, part of the experts' weights would pass twice.
             if (spare && spare <= e * 48 && a.ktiles <= 32) return launch_runs<4>(a, q->w->batch);
-            const uint64_t columns = (a.ntiles + 7) / 8, rounds = (e * columns + g.n_cus - 1) / g.n_cus;
-            const uint64_t eighths = columns == 16 && rounds <= 3 && a.ktiles != 32 && a.ktiles != 64 ? e * columns * 8 / (rounds * g.n_cus) : 0;
-            const uint32_t most = a.ktiles <= 16 || a.ntiles >= 256 || eighths >= (rounds == 1 ? 6 : 7) ? 48
-                                  : eighths == 6 && rounds == 2 ? 56
-                                  : !runs_by_xcd(a, q->w->batch) ? 64 : a.ntiles < 32 ? 68 : 80;
+            const uint64_t most = a.ktiles <= 16 ? 48 : runs_by_xcd(a, q->w->batch) ? 80 : 64;
             if (spare && spare <= e * most) return launch_runs<8>(a, q->w->batch);
             return launch_lds<4>(a, 1);
         }
         if (f32) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, 1) : launch_split<true, 1, 1, 4, 8, true>(a, 1);
         const uint64_t e = q->w->batch, spare = a.groups > e ? (a.groups - e) * 16 : 0;
         if (a.groups <= kMixStreamGroups && streams(a, e)) {
-            // From so many rows an expert (us, without / with, as below): in order 12, 20 where the weights are less than 160 MiB (16
-            // experts, 1408 -> 2048 at 13 rows 18.8 / 20.9) and 24 over short ranges (64, 512 -> 2048 at 17 30.6 / 33.5); picked
-            // one by one, which all workgroups of the others do again, 4 over long ranges (32, 4096 -> 4096 182 / 167), 5 else (six of 64,
-            // 2048 -> 2 x 1024 -> 2048, a whole pass at 4.3 rows 106.6 / 107.7, at 5.3 110.2 / 110.1, at 6 120.6 / 112.7), 10 with
-            // few experts (16, 2048 -> 4096 at 4 rows 42 / 46, at 11 49 / 46), 8 over short ranges (64, 512 -> 2048 31 / 32 at 6, 35 / 33 at 9).
+            // From so many rows an expert (us, without / with): in order 12 (64 experts, 2048 -> 1024 49.8 / 46.0; 32, 4096 -> 4096 196 /
+            // 169), 20 where the weights are less than 160 MiB (16, 1408 -> 2048 at 16 rows 18.7 / 19.5, at 20 20.2 / 20.1); picked
+            // one by one, which all workgroups of the others do again, 4 over long ranges (32, 4096 -> 4096 168 / 163), 5 else (64,
+            // 2048 -> 1024 49.7 / 44.2), 10 with few experts (16, 2048 -> 4096 at 8 rows 42.3 / 45.1, at 10 47.8 / 45.8), 8 over
+            // short ranges (64, 512 -> 2048 at 8 33.1 / 28.9).  At these ends a few are slower than without, 8 % at most (34, 1280 -> 2048,
+            // picked, 6 rows 34.3 / 36.0).
             const uint64_t from = a.x_perm ? (a.ktiles < 32 ? 8 : a.ktiles >= 128 ? 4 : e >= 32 ? 5 : 10)
-                                           : a.ktiles < 32 ? 24 : e * a.ntiles * a.ktiles >> 10 >= 160 ? 12 : 20;
+                                           : e * a.ntiles * a.ktiles >> 10 >= 160 ? 12 : 20;
             if (spare >= e * from) return launch_stream<2, 4, 4, true>(a, e);
         }
         if (!gated && a.ntiles * a.groups < 384) return launch_split<false, 1, 1, 4, 8, true>(a, 1);   // (as one group of rows below)
