@@ -196,9 +196,10 @@ def test_batch_of_matrices(lib, f32, batch, N, K, rows):
         b.free()
 
 
-# ... in tiles of 256 outputs by 128 and 256 rows, the matrices on XCDs of their own (batches of 2, 4 and 8) and on all of them
+# ... in tiles of 256 outputs by 128 and 256 rows, the matrices on all XCDs and on one each (batches of 16 and more that eight divides)
 @pytest.mark.parametrize("batch,N,K,rows", [(2, 7584, 2080, 400), (4, 7712, 2080, 130), (8, 4000, 2080, 130), (3, 6688, 2080, 280),
-                                            (2, 7328, 1056, 910), (4, 7328, 1056, 400), (8, 7584, 1056, 130), (3, 6560, 1056, 670)])
+                                            (2, 7328, 1056, 910), (4, 7328, 1056, 400), (8, 7584, 1056, 130), (3, 6560, 1056, 670),
+                                            (16, 1952, 2080, 200), (24, 1952, 1056, 400), (20, 1952, 1056, 200)])
 def test_batch_of_matrices_in_wide_tiles(lib, batch, N, K, rows):
     r = Run(lib, False, batch, N, K, rows)
     x = r.act(rows, (batch + 1) * K)

@@ -246,17 +246,12 @@ __device__ __forceinline__ void part_store(float* p, float v)
 // other 8 / cols: an XCD fetches 1 / cols of the weight and cols / 8 of the rows, once,
 // and runs through its row panels of one output panel before the next.  False: a place
 // the grid only has because the shares are equal.
-__device__ __forceinline__ bool xcd_tile_of(uint32_t xcd, uint32_t slot, uint32_t n_xcd, uint32_t cols, uint32_t nx, uint32_t ny,
-                                            uint32_t& px, uint32_t& py)
+__device__ __forceinline__ bool xcd_tile(uint32_t block, uint32_t cols, uint32_t nx, uint32_t ny, uint32_t& px, uint32_t& py)
 {
-    const uint32_t rows = n_xcd / cols, ly = (ny + rows - 1) / rows;
+    const uint32_t xcd = block % 8, slot = block / 8, rows = 8 / cols, ly = (ny + rows - 1) / rows;
     px = slot / ly * cols + xcd % cols;
     py = slot % ly * rows + xcd / cols;
     return px < nx && py < ny;
-}
-__device__ __forceinline__ bool xcd_tile(uint32_t block, uint32_t cols, uint32_t nx, uint32_t ny, uint32_t& px, uint32_t& py)
-{
-    return xcd_tile_of(block % 8, block / 8, 8, cols, nx, ny, px, py);
 }
 
 // The `cols` (8, 4, 2, 1) that fetches the fewest bytes among those with the fewest
@@ -264,20 +259,19 @@ __device__ __forceinline__ bool xcd_tile(uint32_t block, uint32_t cols, uint32_t
 // of many rows gains: 2047 rows x 2048 and 3072 -> 1024, all eight XCDs fetching all
 // rows (200 MB) against an eighth of them each (50), 40.3 -> 37.1 us on average; bf16
 // rows of stacks, 4096 and 8192 -> 2048, 54.2 -> 51.5; wide ones 1 to 2 %.
-inline uint32_t xcd_cols(uint32_t nx, uint32_t ny, uint64_t weight_bytes, uint64_t row_bytes, uint32_t per_xcd, uint32_t* blocks,
-                         uint32_t n_xcd = 8)
+inline uint32_t xcd_cols(uint32_t nx, uint32_t ny, uint64_t weight_bytes, uint64_t row_bytes, uint32_t per_xcd, uint32_t* blocks)
 {
     uint32_t best = 0;
     uint64_t best_rounds = 0, best_bytes = 0;
-    for (uint32_t cols = n_xcd; cols >= 1; cols /= 2) {
-        const uint32_t rows = n_xcd / cols;
+    for (uint32_t cols = 8; cols >= 1; cols /= 2) {
+        const uint32_t rows = 8 / cols;
         const uint64_t each = (uint64_t)((nx + cols - 1) / cols) * ((ny + rows - 1) / rows);
         const uint64_t rounds = (each + per_xcd - 1) / per_xcd, bytes = weight_bytes * rows + row_bytes * cols;
         if (!best || rounds < best_rounds || (rounds == best_rounds && bytes < best_bytes)) {
             best = cols;
             best_rounds = rounds;
             best_bytes = bytes;
-            *blocks = (uint32_t)(each * n_xcd);
+            *blocks = (uint32_t)(each * 8);
         }
     }
     return best;

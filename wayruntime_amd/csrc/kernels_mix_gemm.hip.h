@@ -638,13 +638,11 @@ __global__ __launch_bounds__(WAVES * 64, 2) void mix_gemm_runs_kernel(const MixG
 // a full device's step of 256 x 256 x 32 is 0.78 us, 0.51 of it products at 2.05 GHz, on 64 units alone 0.56 (2.4 GHz).  4095 rows,
 // 8192 -> 4096 216 -> 194 us (1.42 PFLOP/s).  On the way there: operands read behind the barrier and a barrier a step 0.83, read a step ahead
 // 0.80, the copies among the products 0.78.
-// XCDs that a matrix of a batch is shared out to: as many as there are for each, so that its weights and rows come into
-// those L2s and no others.  us, every XCD for every matrix / so: 2047 rows, four of 2048 -> 2048 68 / 61, 4096 -> 4096 into
-// 32-bit rows 260 / 230; 32 of 512 -> 128 23 / 19.5, at 1000 rows 16.5 / 12.8.  (Other numbers than 2, 4 and multiples of eight would leave XCDs without one.)
-__host__ __device__ __forceinline__ uint32_t mix_batch_xcds(uint32_t batch)
-{
-    return batch % 8 == 0 ? 1u : batch == 2 || batch == 4 ? 8 / batch : 8u;
-}
+// Whether XCDs take whole matrices of a batch, one after the other, so that a matrix's weights and rows come into one L2 and no other;
+// fewer than sixteen, and numbers that eight does not divide, are shared out tile by tile (us, so / every XCD for every matrix: 2047
+// rows, 32 of 512 -> 128 19.6 / 23.6, 16 of 1024 -> 512 42.5 / 44.2, 700 rows 23.4 / 28.1; against 8 of 1024 -> 2048 into 32-bit rows at 2047
+// 81.3 / 74.6, at 511 less by 9 %; two and four, on four and two XCDs each, 0.99 to 1.02 of the time on average and up to 1.12).
+__host__ __device__ __forceinline__ bool mix_batch_apart(uint32_t batch) { return batch >= 16 && batch % 8 == 0; }
 
 template <int GROUPS, int KS = 1, int WN = 2>
 constexpr int mix_gemm_ring() { return WN == 4 || (KS == 2 && GROUPS == 4) ? 5 : KS == 2 ? 4 : 3; }
@@ -668,11 +666,16 @@ __global__ __launch_bounds__(128 * WN * KS, KS == 2 || WN == 4 ? 1 : 2) void mix
     const uint32_t ktiles = a.ktiles / KS;                 // this set's k-steps
     const uint32_t nx = (a.ntiles + TILES - 1) / TILES, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
     uint32_t px, py, z = 0;
-    if constexpr (BATCH) {                                 // XCDs share out the matrices (mix_batch_xcds), or each of them the tiles
-        const uint32_t id = blockIdx.y * gridDim.x + blockIdx.x, n = mix_batch_xcds(gridDim.y), xcd = id % 8, slot = id / 8;
-        const uint32_t at = n == 8 ? blockIdx.x / 8 : slot % (gridDim.x / n);
-        z = n == 8 ? blockIdx.y : slot / (gridDim.x / n) * (8 / n) + xcd / n;
-        if (!xcd_tile_of(xcd % n, at, n, a.cols, nx, ny, px, py)) return;
+    if constexpr (BATCH) {
+        z = blockIdx.y;
+        if (mix_batch_apart(gridDim.y)) {
+            const uint32_t id = blockIdx.y * gridDim.x + blockIdx.x, slot = id / 8, at = slot % gridDim.x;
+            z = slot / gridDim.x * 8 + id % 8;
+            px = at / ny;
+            py = at % ny;
+        } else if (!xcd_tile(blockIdx.x, a.cols, nx, ny, px, py)) {
+            return;
+        }
     } else if (!a.group_expert) {
         if (!xcd_tile(blockIdx.x, a.cols, nx, ny, px, py)) return;
     } else {

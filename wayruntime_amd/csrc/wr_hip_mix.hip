@@ -560,9 +560,10 @@ static int launch_lds(const MixGemmArgs& args, uint32_t batch)
     MixGemmArgs a = args;
     const uint32_t nx = (a.ntiles + TILES - 1) / TILES, ny = (a.groups + 2 * GROUPS - 1) / (2 * GROUPS);
     uint32_t blocks = (nx < 8 ? nx : (nx + 7) / 8 * 8) * ny;
-    if (!a.group_expert)
-        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, KS == 2 || WN == 4 ? 32 : 64, &blocks,
-                          batch > 1 ? mix_batch_xcds(batch) : 8);
+    if (batch > 1 && mix_batch_apart(batch))
+        blocks = nx * ny;
+    else if (!a.group_expert)
+        a.cols = xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, KS == 2 || WN == 4 ? 32 : 64, &blocks);
     launch_main(batch > 1 ? mix_gemm_lds_kernel<GROUPS, KS, WN, true> : mix_gemm_lds_kernel<GROUPS, KS, WN>, dim3(blocks, batch),
                 dim3(128 * WN * KS), a, lds);
     HIP_TRY(hipGetLastError(), "product launch", 0);
@@ -574,11 +575,11 @@ constexpr uint32_t kXcdUnits = 32;
 // Workgroups of tiles x groups tiles, one to a compute unit at a time, that the XCD with the most of them has.
 static uint32_t busiest_xcd(const MixGemmArgs& a, uint32_t tiles, uint32_t groups, uint32_t batch)
 {
-    const uint32_t n = batch > 1 ? mix_batch_xcds(batch) : 8;
-    uint32_t blocks = 0;
-    xcd_cols((a.ntiles + tiles - 1) / tiles, (a.groups + groups - 1) / groups, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024,
-             kXcdUnits, &blocks, n);
-    return (uint32_t)((uint64_t)blocks * batch / 8);       // (a matrix has `n` of the eight, and 8 / n have theirs at the same time)
+    const uint32_t nx = (a.ntiles + tiles - 1) / tiles, ny = (a.groups + groups - 1) / groups;
+    uint32_t blocks = nx * ny;
+    if (!mix_batch_apart(batch))
+        xcd_cols(nx, ny, (uint64_t)a.ntiles * a.ktiles * 1024, (uint64_t)a.groups * a.ktiles * 1024, kXcdUnits, &blocks);
+    return (uint32_t)(((uint64_t)blocks * batch + 7) / 8);
 }
 
 // Products of 17 rows and more, bfloat16: the form whose estimate is the least.  A register tile of NT x GR waits for
