@@ -592,10 +592,13 @@ static uint32_t busiest_xcd(const MixGemmArgs& a, uint32_t tiles, uint32_t group
 // -> 4096 at 300 111 / 68; 2048 -> 14 400 at 45 27 / 15.3.  The halves: 8192 -> 2048 at 1000 rows 80 / 55, at 2047 93
 // / 73; 4096 -> 2048 at 2047 50 / 41; 12 288 -> 4096 at 1000 153 / 108.
 // The pipelined tiles of 256 outputs x 256 and 128 rows (mix_gemm_lds_kernel, WN = 4; from 1024 inputs on): a full round of one workgroup
-// per unit 0.78 and 0.44, with what its ends cost besides (8 and 5 us, 4 and 3 more where 32-bit rows go out), one that
+// per unit 0.78 and 0.46, with what its ends cost besides (8 and 5 us, 4 and 3 more where 32-bit rows go out), one that
 // leaves units without a workgroup less, as the others then have the clock and the caches. Against the tile of 128 x 256,
 // whose ends those figures split off too: 2047 rows, 2048 -> 32 768 into 32-bit rows 315 / 266 us, -> 14 400 137 / 114, 4096 -> 24 576 gated
 // 320 / 299; 2500 rows, 2048 -> 16 384, two and a half rounds, 142 / 156: the other tile's.
+// (0.44 for the second took rounds of it over long ranges that are the others': 4095 rows, 8192 -> 6144 into 32-bit rows 378, 256 x 256 359, 128 x
+// 256 347.  At 1024 inputs those split-off ends are more than the tile of 128 x 256 has: 1800 rows, 1024 -> 8192 39.3, as 128 x 128 42.8; never
+// more than the 0.5 of short ranges.)
 // Where 32-bit rows go out all LDS tiles have ends that count from 1024 inputs on: 2, 4 and 11 us for a tile's share of the three, 4
 // and 10 for each round of two sets of waves behind the first.  (With those of the largest alone the tile of 128 x 128 seemed better than it is: 2048 ->
 // 14 400, 128 x 128 / 256 x 256: 2047 rows 148 / 116, 3000 223 / 174; four of 1024 -> 4096, 2047 rows 125 / 73.)
@@ -605,8 +608,8 @@ static uint32_t busiest_xcd(const MixGemmArgs& a, uint32_t tiles, uint32_t group
 // (64 rows, 8192 -> 512: 17.4 us in tiles of two groups, 13.2; 2048 -> 2048 6.9, 5.7).  Tiles of 256 rows are counted in
 // whole workgroups per unit where all run at once (1500 rows, 256 -> 8192: 17.8 us against 16.3 with tiles of 128;
 // beyond two a unit, places are filled as they come free: 2047 rows, 2048 -> 14 400 161 us, 170 with tiles of 128).
-// profiles/stack_product_forms.txt has every form's time for 772 sizes, into fragments, into 32-bit rows, gated and in
-// batches: the form picked is 2.0 % off the best one on average, more than 10 % for 43 of them (59 % at worst: 300 rows, 4096 -> 4160).
+// profiles/stack_product_forms.txt has every form's time for 1006 sizes, into fragments, into 32-bit rows, gated and in
+// batches: the form picked is 2.5 % off the best one on average, more than 10 % for 84 of them (59 % at worst: 300 rows, 4096 -> 4160).
 static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
 {
     // 32-bit rows, or most of them (an input product of the parallel halves: 64 of 14 400 outputs are a fragment's)
@@ -633,7 +636,7 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
         uint32_t groups;
         float full, part, more, ends, rows32;
         int (*launch)(const MixGemmArgs&, uint32_t);
-    } piped[] = {{16, 0.78f, 0.50f, 0.26f, 8.f, 4.f, launch_lds<8, 1, 4>}, {8, 0.44f, 0.34f, 0.09f, 5.f, 3.f, launch_lds<4, 1, 4>}};
+    } piped[] = {{16, 0.78f, 0.50f, 0.26f, 8.f, 4.f, launch_lds<8, 1, 4>}, {8, 0.46f, 0.34f, 0.09f, 5.f, 3.f, launch_lds<4, 1, 4>}};
     int (*best)(const MixGemmArgs&, uint32_t) = nullptr;
     float least = 0.f;
     auto offer = [&](float cost, int (*launch)(const MixGemmArgs&, uint32_t)) {
@@ -656,7 +659,7 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
                 share = f.share32 + f.ends32 / (float)a.ktiles;
                 if (f.groups == 8) step += f.ends32 / (float)a.ktiles;
             } else if (a.ktiles >= 32 && f.groups == 16) {
-                share = 0.435f + 4.f / (float)a.ktiles;
+                share = std::min(share, 0.435f + 4.f / (float)a.ktiles);
             }
             offer(std::max(step, share * each), f.launch);
         }
