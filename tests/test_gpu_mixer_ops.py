@@ -329,7 +329,7 @@ def test_runs_whose_last_groups_hold_no_pair(lib, N, K, runs_each, spare, expert
         b.free()
 
 
-# up to 48, 64 and 80 rows an expert; runs by XCD or not; tiles of 2048 outputs that come out even (15 experts) or not
+# up to 48, 64 and 80 rows an expert; runs by XCD or not; tiles beyond
 @pytest.mark.parametrize("experts,spare", [(8, 3), (8, 4), (15, 5), (15, 6), (20, 7), (20, 10)])
 @pytest.mark.parametrize("N,K", [(64, 1024), (64, 1056), (1536, 544), (1568, 544), (96, 64), (32, 2080), (2048, 544)])
 def test_runs_of_every_length(lib, experts, spare, N, K):

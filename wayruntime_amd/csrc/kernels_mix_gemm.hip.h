@@ -619,6 +619,12 @@ __global__ __launch_bounds__(WAVES * 64, 2) void mix_gemm_runs_kernel(const MixG
     }
 }
 
+// Whether XCDs take whole matrices of a batch, one after the other, so that a matrix's weights and rows come into one L2 and no other;
+// fewer than sixteen, and numbers that eight does not divide, are shared out tile by tile (us, so / every XCD for every matrix: 2047
+// rows, 32 of 512 -> 128 19.6 / 23.6, 16 of 1024 -> 512 42.5 / 44.2, 700 rows 23.4 / 28.1; against 8 of 1024 -> 2048 into 32-bit rows at 2047
+// 81.3 / 74.6, at 511 less by 9 %; two and four, on four and two XCDs each, 0.99 to 1.02 of the time on average and up to 1.12).
+__host__ __device__ __forceinline__ bool mix_batch_apart(uint32_t batch) { return batch >= 16 && batch % 8 == 0; }
+
 // 2 x 2 waves of 64 outputs x 16 GROUPS rows each: 128 outputs x 32 GROUPS rows a
 // workgroup.  Per k-step 8 weight tiles and 2 GROUPS fragments, one KiB each and
 // already in operand order, go to LDS by direct loads two k-steps ahead in a ring
@@ -638,12 +644,6 @@ __global__ __launch_bounds__(WAVES * 64, 2) void mix_gemm_runs_kernel(const MixG
 // a full device's step of 256 x 256 x 32 is 0.78 us, 0.51 of it products at 2.05 GHz, on 64 units alone 0.56 (2.4 GHz).  4095 rows,
 // 8192 -> 4096 216 -> 194 us (1.42 PFLOP/s).  On the way there: operands read behind the barrier and a barrier a step 0.83, read a step ahead
 // 0.80, the copies among the products 0.78.
-// Whether XCDs take whole matrices of a batch, one after the other, so that a matrix's weights and rows come into one L2 and no other;
-// fewer than sixteen, and numbers that eight does not divide, are shared out tile by tile (us, so / every XCD for every matrix: 2047
-// rows, 32 of 512 -> 128 19.6 / 23.6, 16 of 1024 -> 512 42.5 / 44.2, 700 rows 23.4 / 28.1; against 8 of 1024 -> 2048 into 32-bit rows at 2047
-// 81.3 / 74.6, at 511 less by 9 %; two and four, on four and two XCDs each, 0.99 to 1.02 of the time on average and up to 1.12).
-__host__ __device__ __forceinline__ bool mix_batch_apart(uint32_t batch) { return batch >= 16 && batch % 8 == 0; }
-
 template <int GROUPS, int KS = 1, int WN = 2>
 constexpr int mix_gemm_ring() { return WN == 4 || (KS == 2 && GROUPS == 4) ? 5 : KS == 2 ? 4 : 3; }
 template <int GROUPS, int KS = 1, int WN = 2>
