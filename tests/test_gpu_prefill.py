@@ -240,6 +240,33 @@ def test_few_rows_over_many_keys_sampled_rows(nq, nkv, hd, p0, T, win):
     kv.close()
 
 
+@pytest.mark.parametrize("nq,nkv,hd,p0,T,win", [
+    (16, 8, 128, 0, 1024, 0), (16, 8, 128, 0, 1025, 0),      # two pairs to a workgroup while that gives every CU one, then four
+    (16, 8, 256, 31, 1024, 0), (16, 8, 256, 31, 1056, 0),
+    (8, 4, 256, 0, 2048, 500), (8, 4, 256, 0, 2081, 500),
+    (32, 8, 64, 0, 512, 0), (32, 8, 64, 0, 545, 0),
+    (8, 8, 128, 3, 95, 40),                                  # groups of one, four and eight in twos
+    (8, 2, 128, 64, 33, 0),
+    (16, 2, 64, 1, 63, 0),
+    (4, 4, 256, 33, 127, 64),
+])
+def test_two_and_four_pairs_to_a_workgroup_sampled_rows(nq, nkv, hd, p0, T, win):
+    """Either side of where a launch goes from workgroups of two (head, 32-row block) pairs to four, and groups that two
+    pairs take in several chunks of heads; without parts, so that the blocks' own kernels write the rows."""
+    print("forms", nq, nkv, hd, p0, T, win, flush=True)
+    kv, q, k16, v16 = _setup(nq, nkv, hd, p0, T, seed=4400 + T + hd)
+    hipattn.set_prefill_part_mb(0)
+    try:
+        whole = kv.prefill(0, p0, q, 0.0, win)
+    finally:
+        hipattn.set_prefill_part_mb()
+    cut = kv.prefill(0, p0, q, 0.0, win)
+    rows = sorted({0, 1, 31, 32, 33, 63, 64, T // 2, T - 33, T - 2, T - 1} & set(range(T)))
+    want = oracle.causal_prefill(q, k16, v16, p0=p0, window=win, rows=rows, threads=8)
+    print("  errors", util.assert_close(whole[rows], want[rows]), util.assert_close(cut[rows], want[rows]), flush=True)
+    kv.close()
+
+
 @pytest.mark.parametrize("where", ["first", "middle", "last", "down", "up"])
 @pytest.mark.parametrize("nq,nkv,hd", [(32, 8, 128), (4, 4, 64), (8, 4, 256)])
 def test_parts_whose_references_lie_far_apart(nq, nkv, hd, where):

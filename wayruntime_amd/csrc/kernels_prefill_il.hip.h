@@ -8,7 +8,14 @@
 // Workgroup = 8 waves = one KV head x 4 (head, 32-row block) pairs x 2 key sets:
 // waves 0-3 take the even 32-key tiles of the block's key range, waves 4-7 the
 // odd ones (split-K inside the workgroup, the two partial (m, l, O) triples merged
-// through LDS at the end), two waves per SIMD at <= 256 registers each.  Per wave
+// through LDS at the end), two waves per SIMD at <= 256 registers each.  NP = 2: two
+// pairs, 4 waves, one to a SIMD, for launches that leave CUs idle: twice as many
+// workgroups, each step 0.6 us where four pairs take 0.7 to 0.8, half the rows to
+// read, merge and store at a block's ends (16/8/128, 54 rows 9.0 -> 7.9 us, 1024 rows
+// 19.6 -> 17.7).  Full launches keep four: a tile copied into LDS then feeds twice the
+// rows, and a SIMD's second wave issues while the first waits (2048 rows, 32/8/128:
+// 50 us against 67).  A row's sums have the same order in both, but for the set that
+// the first tile of a window falls to.  Per wave
 // and tile, with the query row as the MFMA COLUMN (lane % 32):
 //   S^T[key][row]  = K[key][:] . Q^T[:][row]          HD/16 MFMAs, a dependent chain
 //   online softmax on the 16 scores a lane holds (+ one exchange with lane^32)
@@ -68,27 +75,30 @@
 
 namespace wr {
 
-constexpr int kSplitThreads = 512;
 constexpr int kRing = 3;
 
-template <int HD>
+// Threads of a workgroup of NP (head, 32-row block) pairs: a wave of each of the two sets to a pair.
+constexpr int split_threads(int np) { return 2 * np * 64; }
+
+template <int HD, int NP = 4>
 struct SplitLds {
     static constexpr int RB = 2 * HD;                     // bytes per K row
     static constexpr int CPR = HD / 8;                    // 16-byte chunks per K row
     static constexpr int RPB = 256 / RB > 0 ? 256 / RB : 1;   // K rows per 256-byte bank row
     static constexpr int KTILE = kTileKeys * RB;          // bytes of one tile's K
     static constexpr int VTILE = HD * kVBlock * 2;        // bytes of one tile's Vt block
-    static constexpr int NL = KTILE / 1024 / 4;           // loads per wave and tile, each of K and Vt
+    static constexpr int NL = KTILE / 1024 / NP;          // loads per wave and tile, each of K and Vt
+    static constexpr int KROWS = NP * (1024 / RB);        // K rows from one of them to the next
     static constexpr int SET_BYTES = kRing * (KTILE + VTILE);   // one wave set's ring
     static constexpr int V_IN_SET = kRing * KTILE;        // Vt slots follow the K slots
-    static constexpr int Q_OFF = 2 * SET_BYTES;           // Q staging, [4][32][HD + 8] halves
-    static constexpr int Q_BYTES = 4 * 32 * (HD + 8) * 2;
+    static constexpr int Q_OFF = 2 * SET_BYTES;           // Q staging, [NP][32][HD + 8] halves
+    static constexpr int Q_BYTES = NP * 32 * (HD + 8) * 2;
     // Merge scratch (end of a block): at the end of the kernel's LDS, over the Q
     // staging (Q is in registers by then) and, where 160 KiB are not enough for
     // everything, over the tail of the odd set's last Vt slot.  It stays clear of
     // every slot the first copies of a block go to, so the next block's first
     // tiles can be on their way while this block is merged and stored.
-    static constexpr int MERGE_BYTES = 4 * (HD / 2 + 2) * 64 * 4;
+    static constexpr int MERGE_BYTES = NP * (HD / 2 + 2) * 64 * 4;
     static constexpr int LDS_MAX = 160 * 1024;
     static constexpr int MERGE_OFF = (Q_OFF + Q_BYTES + MERGE_BYTES <= LDS_MAX) ? Q_OFF + Q_BYTES
                                                                                 : LDS_MAX - MERGE_BYTES;
@@ -96,15 +106,19 @@ struct SplitLds {
     static_assert(MERGE_OFF >= SET_BYTES + V_IN_SET + 2 * VTILE,
                   "merge scratch may overlap the odd set's third Vt slot only (no copy of a block's prologue lands there)");
     static_assert(KTILE == VTILE && NL >= 1, "one chunk schedule serves K and Vt");
+    static_assert(KROWS % 8 == 0, "eight K rows are 64 bytes of every 16-byte chunk's run in the cache");
     // slot permutation of K rows / Vt rows
     __device__ static constexpr int fk(int row) { return (row / RPB) & (CPR - 1); }
     __device__ static constexpr int fv(int row) { return (row >> 2) & 3; }
+    // What a K row's slot permutation does to a lane's place in the tile from a wave's first copy to its u-th: chunks
+    // lie 256 bytes apart.
+    __device__ static constexpr uint32_t copy_swap(int u) { return (uint32_t)fk(u * KROWS) * 256; }
 };
 
-template <int HD>
+template <int HD, int NP>
 constexpr size_t split_smem_bytes()
 {
-    return SplitLds<HD>::TOTAL;
+    return SplitLds<HD, NP>::TOTAL;
 }
 
 // max of three without the canonicalising self-maximum the compiler puts in
@@ -144,50 +158,50 @@ __device__ __forceinline__ uint32_t il_tile(const IlCtx<HD>& cx, uint32_t jt)
 }
 
 // One of this wave's NL copies of the set's K tile jt / Vt block jt into ring slot SLOT.
-template <int HD, int SLOT>
+template <int HD, int NP, int SLOT>
 __device__ __forceinline__ void il_issue_k1(const IlCtx<HD>& cx, uint32_t jt, int u)
 {
-    using L = SplitLds<HD>;
+    using L = SplitLds<HD, NP>;
     const unsigned char* src = cx.kbase + (size_t)il_tile(cx, jt) * L::KTILE;
-    lds_direct_load(cx.m0k + SLOT * L::KTILE + u * 4096, src + u * 128, cx.gk_off);
+    lds_direct_load(cx.m0k + SLOT * L::KTILE + u * NP * 1024, src + u * L::KROWS * 8, cx.gk_off ^ L::copy_swap(u));
 }
 
-template <int HD, int SLOT>
+template <int HD, int NP, int SLOT>
 __device__ __forceinline__ void il_issue_v1(const IlCtx<HD>& cx, uint32_t jt, int u)
 {
-    using L = SplitLds<HD>;
+    using L = SplitLds<HD, NP>;
     const unsigned char* src = cx.vtbase + (size_t)il_tile(cx, jt) * L::VTILE;
-    lds_direct_load(cx.m0v + SLOT * L::VTILE + u * 4096, src + u * 4096, cx.gv_off);
+    lds_direct_load(cx.m0v + SLOT * L::VTILE + u * NP * 1024, src + u * NP * 1024, cx.gv_off);
 }
 
-template <int HD, int SLOT>
+template <int HD, int NP, int SLOT>
 __device__ __forceinline__ void il_issue_k(const IlCtx<HD>& cx, uint32_t jt)
 {
 #pragma unroll
-    for (int u = 0; u < SplitLds<HD>::NL; u++) il_issue_k1<HD, SLOT>(cx, jt, u);
+    for (int u = 0; u < SplitLds<HD, NP>::NL; u++) il_issue_k1<HD, NP, SLOT>(cx, jt, u);
 }
 
-template <int HD, int SLOT>
+template <int HD, int NP, int SLOT>
 __device__ __forceinline__ void il_issue_v(const IlCtx<HD>& cx, uint32_t jt)
 {
 #pragma unroll
-    for (int u = 0; u < SplitLds<HD>::NL; u++) il_issue_v1<HD, SLOT>(cx, jt, u);
+    for (int u = 0; u < SplitLds<HD, NP>::NL; u++) il_issue_v1<HD, NP, SLOT>(cx, jt, u);
 }
 
 // Zeroes, in the staged Vt of the set's tile jt (ring slot SLOT), the positions
 // that were never appended: they may hold anything, and 0 * garbage must not
 // reach the accumulator.  Every lane patches the chunks its own copies
 // delivered, so only this wave's copies have to have landed.
-template <int HD, int SLOT>
+template <int HD, int NP, int SLOT>
 __device__ __forceinline__ void il_patch_tail(unsigned char* smem, const IlCtx<HD>& cx, uint32_t jt,
                                               int sub, int lane, uint32_t kv_valid)
 {
-    using L = SplitLds<HD>;
+    using L = SplitLds<HD, NP>;
     const uint32_t tile = il_tile(cx, jt);
     if (tile < cx.tail_tile) return;
 #pragma unroll
     for (int u = 0; u < L::NL; u++) {
-        const int q = sub + 4 * u;
+        const int q = sub + NP * u;
         const int row = q * 16 + lane / 4;                // Vt row (dimension)
         const int c = (lane & 3) ^ L::fv(row);            // key chunk this slot holds
         const uint32_t key0 = tile * kTileKeys + c * 8;
@@ -314,13 +328,13 @@ __device__ __forceinline__ void il_settle(PrefillRows<HD>& R, IlCtx<HD>& cx, f32
 // Step j of a wave (P == j % kRing).  On entry `cur` holds the scores of the set's
 // tile j (masked, reference settled), kf the K operands of tile j+1; on exit `nxt`
 // holds the scores of tile j+1 in the same state and kf the operands of tile j+2.
-template <int HD, int P>
+template <int HD, int NP, int P>
 __device__ __forceinline__ void il_step(PrefillRows<HD>& R, IlCtx<HD>& cx, f32x16& negm, const f32x16& cur,
                                         f32x16& nxt, u32x4 (&pop)[2], half8 (&kf)[HD / 16],
                                         half8 (&vf)[HD / 16], unsigned char* smem, uint32_t j, int sub,
                                         int lane, int g, uint32_t kv_valid)
 {
-    using L = SplitLds<HD>;
+    using L = SplitLds<HD, NP>;
     constexpr int NS = HD / 16, ND = HD / 32;
     constexpr int PAIRS = 8 / NS;         // pairs of probabilities formed behind each link of the chain
     static_assert(kRing == 3 && 8 % NS == 0 && NS >= 2 * L::NL, "slot and interleave arithmetic below");
@@ -360,8 +374,8 @@ __device__ __forceinline__ void il_step(PrefillRows<HD>& R, IlCtx<HD>& cx, f32x1
         R.o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i], __builtin_bit_cast(half8, pop[t]), R.o[dt], 0, 0,
                                                            0);
         kf[i] = *reinterpret_cast<const half8*>(cx.kop[i] + KS * L::KTILE);
-        if (i < L::NL) il_issue_k1<HD, KC>(cx, j + 4, i);
-        else if (i < 2 * L::NL) il_issue_v1<HD, VC>(cx, j + 2, i - L::NL);
+        if (i < L::NL) il_issue_k1<HD, NP, KC>(cx, j + 4, i);
+        else if (i < 2 * L::NL) il_issue_v1<HD, NP, VC>(cx, j + 2, i - L::NL);
     }
     // The row maximum runs in the products' shadow as if the tile were plain; a
     // tile with invisible (row, key) pairs is masked afterwards and its maximum
@@ -377,7 +391,7 @@ __device__ __forceinline__ void il_step(PrefillRows<HD>& R, IlCtx<HD>& cx, f32x1
     // all copies but this step's have landed: K of tile j+3 and Vt of tile j+1,
     // which the next step reads once the barrier has published them
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * L::NL) : "memory");
-    il_patch_tail<HD, TS>(smem, cx, j + 1, sub, lane, kv_valid);
+    il_patch_tail<HD, NP, TS>(smem, cx, j + 1, sub, lane, kv_valid);
     // (no wait for this step's K operand reads here: their slot is not overwritten
     // before the step after next, long after the next chain has consumed them)
     __builtin_amdgcn_sched_barrier(0);
@@ -442,16 +456,16 @@ __device__ __forceinline__ bool il_ctx_tiles(IlCtx<HD>& cx, const PrefillArgs& a
 
 // The copies and loads a block starts with: the first three K tiles and two Vt
 // blocks of the set into their ring slots, in order of need, and the wave's Q rows.
-template <int HD>
+template <int HD, int NP>
 __device__ __forceinline__ void il_first_loads(const IlCtx<HD>& cx, IlQRows<HD>& q, const PrefillArgs& a,
                                                uint32_t row0, uint32_t head, int kg, int lane)
 {
     il_load_q<HD>(q, a, row0, head, kg, lane);
-    il_issue_k<HD, 0>(cx, 0);
-    il_issue_k<HD, 1>(cx, 1);
-    il_issue_v<HD, 0>(cx, 0);
-    il_issue_k<HD, 2>(cx, 2);
-    il_issue_v<HD, 1>(cx, 1);
+    il_issue_k<HD, NP, 0>(cx, 0);
+    il_issue_k<HD, NP, 1>(cx, 1);
+    il_issue_v<HD, NP, 0>(cx, 0);
+    il_issue_k<HD, NP, 2>(cx, 2);
+    il_issue_v<HD, NP, 1>(cx, 1);
 }
 
 // One position block.  started: the block's first loads are already on their way
@@ -459,21 +473,20 @@ __device__ __forceinline__ void il_first_loads(const IlCtx<HD>& cx, IlQRows<HD>&
 // loads of block next_pb are issued, before the merge and the stores, and q
 // returns its Q rows.  PART: part `part` of the block's tiles only; the rows leave
 // unnormalised, beside their reference and sum.
-template <int HD, bool PART>
+template <int HD, int NP, bool PART>
 __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* smem, uint32_t pb,
                                          uint32_t kvh, uint32_t hc, const unsigned char* kbase, const unsigned char* vtbase,
                                          bool started, IlQRows<HD>& q, int next_pb, uint32_t part)
 {
-    using L = SplitLds<HD>;
-    static_assert(L::NL == 1 || L::NL == 2, "one or two copies per wave, tile and operand");
+    using L = SplitLds<HD, NP>;
     const int tid = threadIdx.x;
     const int lane = il_fresh_lane();                     // per call: nothing lane-derived is shared between the blocks of a workgroup
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // in a scalar register
     const int n = lane & 31, g = lane >> 5;
-    const int kg = wave >> 2, sub = wave & 3;             // key set (tile parity), rows served
+    const int kg = wave / NP, sub = wave % NP;            // key set (tile parity), rows served
     const uint32_t G = a.group;
-    const uint32_t Gw = G < 4 ? G : 4;
-    const uint32_t BP = 32 * (4 / Gw);                    // positions per block
+    const uint32_t Gw = G < NP ? G : NP;
+    const uint32_t BP = 32 * (NP / Gw);                   // positions per block
     // wave-uniform, and pinned to scalar registers: integer division runs on the
     // vector unit, and a quotient left there costs a vector register for the
     // whole block (or a spill)
@@ -537,8 +550,7 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
         // Vt: rows of 64 bytes, four slots each
         const int vrow = sub * 16 + lane / 4;
         cx.gv_off = vrow * 64 + ((lane & 3) ^ L::fv(vrow)) * 16;
-        static_assert(L::NL == 1 || (4 * (1024 / L::RB) == 16 && L::fk(16) == L::fk(0) && L::fv(64) == L::fv(0)),
-                      "the second copy is 16 K rows (128 bytes in the cache) / 64 Vt rows (4 KiB) further");
+        static_assert(L::fv(NP * 16) == L::fv(0), "a wave's copies of a Vt block have one permutation");
         const int krow = prefill_key_perm(n);             // tile row this lane feeds to MFMA row n
         const uint32_t kread = krow * L::RB + ((g ^ L::fk(krow)) * 16);
         const uint32_t vread = n * 64 + ((g ^ L::fv(n)) * 16);
@@ -553,7 +565,7 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
     const uint32_t nsteps = (t_last - t_first) / 2 + 1;
 
     // everything the first two vector blocks read, in order of need, and Q
-    if (!started) il_first_loads<HD>(cx, q, a, row0, head, kg, lane);
+    if (!started) il_first_loads<HD, NP>(cx, q, a, row0, head, kg, lane);
 
     // Q is converted to pre-scaled F16 and turned into the per-lane operand
     // layout through LDS (the two waves serving a sub-block take 16 rows each).
@@ -579,7 +591,7 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
 #pragma unroll
     for (int r = 0; r < 16; r++) sa[r] = sb[r] = negm[r] = 0.f;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    il_patch_tail<HD, 0>(smem, cx, 0, sub, lane, kv_valid);
+    il_patch_tail<HD, NP, 0>(smem, cx, 0, sub, lane, kv_valid);
     il_barrier();                                         // first tiles and Q visible to all
 #pragma unroll
     for (int i = 0; i < HD / 16; i++)
@@ -591,7 +603,7 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
     for (int i = 0; i < HD / 16; i++)
         sa = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i], R.qop[i], sa, 0, 0, 0);
     il_barrier();                                         // slot 0 of K has been read by all: it is refilled
-    il_issue_k<HD, 0>(cx, 3);
+    il_issue_k<HD, NP, 0>(cx, 3);
 #pragma unroll
     for (int i = 0; i < HD / 16; i++) kf[i] = *reinterpret_cast<const half8*>(cx.kop[i] + L::KTILE);
     {
@@ -608,7 +620,7 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
     // fewer and spends its last step on probabilities of zero); the same in every
     // wave, and every step ends with the workgroup's barrier
 #define WR_IL_STEP(PHASE, CUR, NXT)                                                          \
-    il_step<HD, PHASE>(R, cx, negm, CUR, NXT, pop, kf, vf, smem, j, sub, lane, g, kv_valid); \
+    il_step<HD, NP, PHASE>(R, cx, negm, CUR, NXT, pop, kf, vf, smem, j, sub, lane, g, kv_valid); \
     if (++j >= nsteps) break;
 #pragma unroll 1
     for (uint32_t j = 0;;) {
@@ -636,7 +648,7 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
         IlCtx<HD> cn = cx;
         uint32_t nf, nl;
         (void)il_ctx_tiles<HD, false>(cn, a, (uint32_t)next_pb, BP, kg, nf, nl, 0);
-        il_first_loads<HD>(cn, q, a, (uint32_t)next_pb * BP + sub_rows, head, kg, lane_e);
+        il_first_loads<HD, NP>(cn, q, a, (uint32_t)next_pb * BP + sub_rows, head, kg, lane_e);
     }
     if (kg == 1) {
 #pragma unroll
@@ -706,16 +718,15 @@ __device__ __forceinline__ void il_block(const PrefillArgs& a, unsigned char* sm
 // a.single: grid.y = blocks, one block per workgroup, long blocks first.
 // PART (with a.single): grid.z = parts of a block's tiles, for few rows over many
 // keys, whose blocks alone would leave most CUs idle (the host's rule says when).
-template <int HD, bool PART>
-__global__ __launch_bounds__(kSplitThreads, 1) void prefill_il_kernel(const PrefillArgs a)
+template <int HD, int NP, bool PART>
+__global__ __launch_bounds__(split_threads(NP), 2) void prefill_il_kernel(const PrefillArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char prefill_smem_raw[];
     const uint32_t G = a.group;
-    const uint32_t Gw = G < 4 ? G : 4;
-    const uint32_t chunks = G / Gw;
-    const uint32_t kvh = (uint32_t)__builtin_amdgcn_readfirstlane(blockIdx.x / chunks);
-    const uint32_t hc = (uint32_t)__builtin_amdgcn_readfirstlane(blockIdx.x % chunks);
-    const uint32_t BP = 32 * (4 / Gw);
+    const uint32_t Gw = G < NP ? G : NP;
+    const uint32_t kvh = (uint32_t)__builtin_amdgcn_readfirstlane(blockIdx.x % a.nkv);
+    const uint32_t hc = (uint32_t)__builtin_amdgcn_readfirstlane(blockIdx.x / a.nkv);
+    const uint32_t BP = 32 * (NP / Gw);
     const uint32_t nblk = (uint32_t)__builtin_amdgcn_readfirstlane((a.T + BP - 1) / BP);
     const uint32_t lo = blockIdx.y, hi = nblk - 1 - blockIdx.y;
     // this KV head's K / Vt, in scalar registers for both blocks
@@ -725,11 +736,11 @@ __global__ __launch_bounds__(kSplitThreads, 1) void prefill_il_kernel(const Pref
         a.vt + (size_t)kvh * (a.ctx_pad / kVBlock) * HD * kVBlock));
     IlQRows<HD> q;
     if (PART || a.single || hi == lo) {
-        il_block<HD, PART>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, false, q, -1, blockIdx.z);
+        il_block<HD, NP, PART>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, false, q, -1, blockIdx.z);
     } else if constexpr (!PART) {
-        il_block<HD, false>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, false, q, (int)lo, 0);
+        il_block<HD, NP, false>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, false, q, (int)lo, 0);
         lds_barrier();                                    // LDS changes hands
-        il_block<HD, false>(a, prefill_smem_raw, lo, kvh, hc, kbase, vtbase, true, q, -1, 0);
+        il_block<HD, NP, false>(a, prefill_smem_raw, lo, kvh, hc, kbase, vtbase, true, q, -1, 0);
     }
 }
 

@@ -12,6 +12,9 @@
 //
 //   workgroup = 8 waves = one KV head x 4 (head, 32-row block) pairs x 2 halves:
 //   waves 0-3 own dimensions 0-127, waves 4-7 dimensions 128-255, of every tile.
+//   NP = 2: two pairs, 4 waves, as in kernels_prefill_il.hip.h (16/8/256, 177 rows
+//   13.9 -> 11.3 us, 1501 rows 53 -> 41; 8/4/256, 1501 rows of a 512-key window 25.1 ->
+//   21.3; 4096 rows, 16/8/256: 165 us with four pairs, 205 with two).
 //
 // Per wave and tile:
 //   S'^T[key][row] = K[key][own dims] . Q^T[own dims][row]    8 MFMAs (half the contraction)
@@ -61,19 +64,24 @@ namespace wr {
 
 constexpr int kIldHalf = 128;                             // dimensions a wave owns
 
+template <int NP>
 struct IldLds {
-    using L = SplitLds<kIldHalf>;
-    static constexpr int X_OFF = 2 * L::SET_BYTES;        // exchange of partial scores: [2 parities][4 pairs][2 halves][16][64] floats
+    using L = SplitLds<kIldHalf, NP>;
+    static constexpr int X_OFF = 2 * L::SET_BYTES;        // exchange of partial scores: [2 parities][NP pairs][2 halves][16][64] floats
     static constexpr int X_WAVE = 16 * 64 * 4;
-    static constexpr int X_PARITY = 8 * X_WAVE;
+    static constexpr int X_PARITY = 2 * NP * X_WAVE;
     static constexpr int X_BYTES = 2 * X_PARITY;
-    // rows leave through LDS, row-major, once the rings are quiet: [8 waves][32][128 + 4] floats from 0
+    // rows leave through LDS, row-major, once the rings are quiet: [2 NP waves][32][128 + 4] floats from 0
     static constexpr int O_WAVE = 32 * (kIldHalf + 4) * 4;
-    static constexpr int TOTAL = (X_OFF + X_BYTES > 8 * O_WAVE) ? X_OFF + X_BYTES : 8 * O_WAVE;
+    static constexpr int TOTAL = (X_OFF + X_BYTES > 2 * NP * O_WAVE) ? X_OFF + X_BYTES : 2 * NP * O_WAVE;
     static_assert(TOTAL <= 160 * 1024, "fits a CU's LDS");
 };
 
-constexpr size_t ild_smem_bytes() { return IldLds::TOTAL; }
+template <int NP>
+constexpr size_t ild_smem_bytes()
+{
+    return IldLds<NP>::TOTAL;
+}
 
 // tile jt of the block (both halves walk every tile), clamped to its last one
 __device__ __forceinline__ uint32_t ild_tile(const IlCtx<kIldHalf>& cx, uint32_t jt)
@@ -81,51 +89,51 @@ __device__ __forceinline__ uint32_t ild_tile(const IlCtx<kIldHalf>& cx, uint32_t
     return min(cx.t0 + jt, cx.t_last);
 }
 
-// One of this wave's two copies of its half of K tile jt / Vt block jt into ring
+// One of this wave's NL copies of its half of K tile jt / Vt block jt into ring
 // slot SLOT.  A K tile of 256 dimensions is 16 KiB in the cache, a Vt block too;
 // the half's share of the latter is contiguous, of the former two runs (one per
 // half of the tile's keys) that gk_off addresses.
-template <int SLOT>
+template <int NP, int SLOT>
 __device__ __forceinline__ void ild_issue_k1(const IlCtx<kIldHalf>& cx, uint32_t jt, int u)
 {
-    using L = SplitLds<kIldHalf>;
+    using L = SplitLds<kIldHalf, NP>;
     const unsigned char* src = cx.kbase + (size_t)ild_tile(cx, jt) * (2 * L::KTILE);
-    lds_direct_load(cx.m0k + SLOT * L::KTILE + u * 4096, src + u * 128, cx.gk_off);
+    lds_direct_load(cx.m0k + SLOT * L::KTILE + u * NP * 1024, src + u * L::KROWS * 8, cx.gk_off ^ L::copy_swap(u));
 }
 
-template <int SLOT>
+template <int NP, int SLOT>
 __device__ __forceinline__ void ild_issue_v1(const IlCtx<kIldHalf>& cx, uint32_t jt, int u)
 {
-    using L = SplitLds<kIldHalf>;
+    using L = SplitLds<kIldHalf, NP>;
     const unsigned char* src = cx.vtbase + (size_t)ild_tile(cx, jt) * (2 * L::VTILE);
-    lds_direct_load(cx.m0v + SLOT * L::VTILE + u * 4096, src + u * 4096, cx.gv_off);
+    lds_direct_load(cx.m0v + SLOT * L::VTILE + u * NP * 1024, src + u * NP * 1024, cx.gv_off);
 }
 
-template <int SLOT>
+template <int NP, int SLOT>
 __device__ __forceinline__ void ild_issue_k(const IlCtx<kIldHalf>& cx, uint32_t jt)
 {
-    ild_issue_k1<SLOT>(cx, jt, 0);
-    ild_issue_k1<SLOT>(cx, jt, 1);
+#pragma unroll
+    for (int u = 0; u < SplitLds<kIldHalf, NP>::NL; u++) ild_issue_k1<NP, SLOT>(cx, jt, u);
 }
 
-template <int SLOT>
+template <int NP, int SLOT>
 __device__ __forceinline__ void ild_issue_v(const IlCtx<kIldHalf>& cx, uint32_t jt)
 {
-    ild_issue_v1<SLOT>(cx, jt, 0);
-    ild_issue_v1<SLOT>(cx, jt, 1);
+#pragma unroll
+    for (int u = 0; u < SplitLds<kIldHalf, NP>::NL; u++) ild_issue_v1<NP, SLOT>(cx, jt, u);
 }
 
 // il_patch_tail for this kernel's tile walk.
-template <int SLOT>
+template <int NP, int SLOT>
 __device__ __forceinline__ void ild_patch_tail(unsigned char* smem, const IlCtx<kIldHalf>& cx, uint32_t jt,
                                                int sub, int lane, uint32_t kv_valid)
 {
-    using L = SplitLds<kIldHalf>;
+    using L = SplitLds<kIldHalf, NP>;
     const uint32_t tile = ild_tile(cx, jt);
     if (tile < cx.tail_tile) return;
 #pragma unroll
     for (int u = 0; u < L::NL; u++) {
-        const int q = sub + 4 * u;
+        const int q = sub + NP * u;
         const int row = q * 16 + lane / 4;                // Vt row (dimension of the half)
         const int c = (lane & 3) ^ L::fv(row);            // key chunk this slot holds
         const uint32_t key0 = tile * kTileKeys + c * 8;
@@ -201,21 +209,21 @@ __device__ __forceinline__ void ild_send(float* xw, const f32x16& c, int lane)
 // wave's partial scores of tile j and kf the K operands of tile j+1; on exit
 // `nxt` holds the partial scores of tile j+1 (sent to the exchange buffer of the
 // other parity) and kf the operands of tile j+2.
-template <int P, int XB>
+template <int NP, int P, int XB>
 __device__ __forceinline__ void ild_step(PrefillRows<kIldHalf>& R, IlCtx<kIldHalf>& cx, f32x16& negm, f32x16& cur,
                                          f32x16& nxt, u32x4 (&pop)[2], half8 (&kf)[8], half8 (&vf)[8],
                                          unsigned char* smem, float* xw, const float* xr_at, uint32_t j, int sub,
                                          int lane, int g, uint32_t kv_valid, bool upper, float& pend,
                                          uint32_t& pend_on)
 {
-    using L = SplitLds<kIldHalf>;
+    using L = SplitLds<kIldHalf, NP>;
     constexpr int NS = 8, ND = 4;
     constexpr int VS = P;                 // slot of Vt of tile j
     constexpr int KS = (P + 2) % 3;       // slot of K of tile j+2
     constexpr int KC = (P + 1) % 3;       // K of tile j+4 replaces K of tile j+1 (read in the previous step)
     constexpr int VC = (P + 2) % 3;       // Vt of tile j+2 replaces Vt of tile j-1 (read in the previous step)
     constexpr int TS = (P + 1) % 3;       // slot of Vt of tile j+1, whose tail is patched once it has landed
-    constexpr int XF = IldLds::X_PARITY / 4;              // floats between the two exchange buffers
+    constexpr int XF = IldLds<NP>::X_PARITY / 4;              // floats between the two exchange buffers
 
     float psum = 0.f;
     const half2v ones = {(_Float16)1.0f, (_Float16)1.0f};
@@ -277,15 +285,15 @@ __device__ __forceinline__ void ild_step(PrefillRows<kIldHalf>& R, IlCtx<kIldHal
         kf[i] = *reinterpret_cast<const half8*>(cx.kop[i] + KS * L::KTILE);
         if (i < 3) pair(5 + i);                           // the second half of P is first used by product 4
         if (i >= 1 && i <= 4) ild_send1(xw + (XB ^ 1) * XF, nxt, lane, i - 1);
-        if (i < L::NL) ild_issue_k1<KC>(cx, j + 4, i);
-        else if (i < 2 * L::NL) ild_issue_v1<VC>(cx, j + 2, i - L::NL);
+        if (i < L::NL) ild_issue_k1<NP, KC>(cx, j + 4, i);
+        else if (i < 2 * L::NL) ild_issue_v1<NP, VC>(cx, j + 2, i - L::NL);
         __builtin_amdgcn_sched_barrier(0);
     }
     R.l_run += psum;
     // all copies but this step's have landed: K of tile j+3 and Vt of tile j+1,
     // which the next step reads once the barrier has published them
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * L::NL) : "memory");
-    ild_patch_tail<TS>(smem, cx, j + 1, sub, lane, kv_valid);
+    ild_patch_tail<NP, TS>(smem, cx, j + 1, sub, lane, kv_valid);
     __builtin_amdgcn_sched_barrier(0);
     // LDS operations complete in the order issued: with at most the three operand
     // reads issued after the last piece of the partial scores outstanding, those
@@ -299,23 +307,24 @@ __device__ __forceinline__ void ild_step(PrefillRows<kIldHalf>& R, IlCtx<kIldHal
 }
 
 // One position block (PART: part `part` of its tiles, as il_block).
-template <bool PART>
+template <int NP, bool PART>
 __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* smem, uint32_t pb, uint32_t kvh,
                                           uint32_t hc, const unsigned char* kbase, const unsigned char* vtbase,
                                           uint32_t part)
 {
-    using L = SplitLds<kIldHalf>;
+    using L = SplitLds<kIldHalf, NP>;
+    using X = IldLds<NP>;
     constexpr int HD = 2 * kIldHalf, H = kIldHalf;
     const int tid = threadIdx.x;
     const int lane = il_fresh_lane();
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kg = wave >> 2;                             // the half of the dimensions owned
+    const int kg = wave / NP;                             // the half of the dimensions owned
     const bool upper = kg != 0;
     const int n = lane & 31, g = lane >> 5;
-    const int sub = wave & 3;                             // the (head, 32-row block) pair served
+    const int sub = wave % NP;                            // the (head, 32-row block) pair served
     const uint32_t G = a.group;
-    const uint32_t Gw = G < 4 ? G : 4;
-    const uint32_t BP = 32 * (4 / Gw);                    // positions per block
+    const uint32_t Gw = G < NP ? G : NP;
+    const uint32_t BP = 32 * (NP / Gw);                   // positions per block
     const uint32_t head = (uint32_t)__builtin_amdgcn_readfirstlane(kvh * G + hc * Gw + (sub % Gw));
     const uint32_t sub_rows = (uint32_t)__builtin_amdgcn_readfirstlane((sub / Gw) * 32);
     const uint32_t row0 = pb * BP + sub_rows;             // first chunk row of this wave
@@ -393,11 +402,11 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
     const uint32_t nsteps = cx.nt;                        // the same in every wave
 
     // everything the first two vector blocks read, in order of need
-    ild_issue_k<0>(cx, 0);
-    ild_issue_k<1>(cx, 1);
-    ild_issue_v<0>(cx, 0);
-    ild_issue_k<2>(cx, 2);
-    ild_issue_v<1>(cx, 1);
+    ild_issue_k<NP, 0>(cx, 0);
+    ild_issue_k<NP, 1>(cx, 1);
+    ild_issue_v<NP, 0>(cx, 0);
+    ild_issue_k<NP, 2>(cx, 2);
+    ild_issue_v<NP, 1>(cx, 1);
     // The wave's Q: 32 rows x its 128 dimensions, read in whole half rows (512
     // contiguous bytes per 32 lanes)
     float4 qx[16];
@@ -406,8 +415,8 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
         const uint32_t row = min(row0 + 2 * jj + (lane >> 5), a.T - 1);   // idle rows re-read the last one
         qx[jj] = *reinterpret_cast<const float4*>(a.q + ((size_t)row * a.nq + head) * HD + kg * H + (lane & 31) * 4);
     }
-    float* xw = reinterpret_cast<float*>(smem + IldLds::X_OFF + (sub * 2 + kg) * IldLds::X_WAVE);
-    const float* xr_at = reinterpret_cast<const float*>(smem + IldLds::X_OFF + (sub * 2 + (kg ^ 1)) * IldLds::X_WAVE);
+    float* xw = reinterpret_cast<float*>(smem + X::X_OFF + (sub * 2 + kg) * X::X_WAVE);
+    const float* xr_at = reinterpret_cast<const float*>(smem + X::X_OFF + (sub * 2 + (kg ^ 1)) * X::X_WAVE);
 
     f32x16 sa, sb, negm;
     u32x4 pop[2];
@@ -421,8 +430,8 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
         // lane's own row) through the wave's share of the exchange buffers, which
         // nothing uses before the first step: rows of 256 bytes, the 16-byte chunk
         // c of row r at slot c ^ (r % 16).  Nobody else reads it: no barrier.
-        unsigned char* qs = smem + IldLds::X_OFF + wave * 8192;
-        static_assert(8 * 8192 <= IldLds::X_BYTES, "the staged Q operands fit the exchange buffers");
+        unsigned char* qs = smem + X::X_OFF + wave * 8192;
+        static_assert(2 * NP * 8192 <= X::X_BYTES, "the staged Q operands fit the exchange buffers");
 #pragma unroll
         for (int jj = 0; jj < 16; jj++) {
             const int r = 2 * jj + (lane >> 5), c = (lane & 31) >> 1;
@@ -435,7 +444,7 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
             R.qop[i] = *reinterpret_cast<const half8*>(qs + n * 256 + (((2 * i + g) ^ (n & 15)) * 16));
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read back before the first partial scores land there
     }
-    ild_patch_tail<0>(smem, cx, 0, sub, lane, kv_valid);
+    ild_patch_tail<NP, 0>(smem, cx, 0, sub, lane, kv_valid);
     il_barrier();                                         // first tiles visible to all
     // scores of the first tile
 #pragma unroll
@@ -444,7 +453,7 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
     for (int i = 0; i < 8; i++) sa = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i], R.qop[i], sa, 0, 0, 0);
     ild_send(xw, sa, lane);                               // tile 0: the exchange buffer of parity 0
     il_barrier();                                         // partial scores out; slot 0 of K has been read by all
-    ild_issue_k<0>(cx, 3);
+    ild_issue_k<NP, 0>(cx, 3);
 #pragma unroll
     for (int i = 0; i < 8; i++) kf[i] = *reinterpret_cast<const half8*>(cx.kop[i] + L::KTILE);
     il_barrier();                                         // slot 1 of K has been read by all: step 0 refills it
@@ -452,7 +461,7 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
     uint32_t pend_on = 0;
 
 #define WR_ILD_STEP(PHASE, XB, CUR, NXT)                                                                     \
-    ild_step<PHASE, XB>(R, cx, negm, CUR, NXT, pop, kf, vf, smem, xw, xr_at, j, sub, lane, g, kv_valid, upper, \
+    ild_step<NP, PHASE, XB>(R, cx, negm, CUR, NXT, pop, kf, vf, smem, xw, xr_at, j, sub, lane, g, kv_valid, upper, \
                         pend, pend_on);                                                                      \
     if (++j >= nsteps) break;
 #pragma unroll 1
@@ -482,7 +491,7 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
     }
     // rows leave through LDS: the wave's tile row-major in its own scratch, then
     // whole half rows (512 contiguous bytes) per 32 lanes
-    float (*os)[H + 4] = reinterpret_cast<float (*)[H + 4]>(smem + (size_t)wave * IldLds::O_WAVE);
+    float (*os)[H + 4] = reinterpret_cast<float (*)[H + 4]>(smem + (size_t)wave * X::O_WAVE);
 #pragma unroll
     for (int dt = 0; dt < H / 32; dt++)
 #pragma unroll
@@ -511,28 +520,27 @@ __device__ __forceinline__ void ild_block(const PrefillArgs& a, unsigned char* s
 }
 
 // grid = (KV heads x head chunks, ceil(blocks / 2)), as prefill_il_kernel; PART: grid.z = parts.
-template <bool PART>
-__global__ __launch_bounds__(kSplitThreads, 1) void prefill_ild_kernel(const PrefillArgs a)
+template <int NP, bool PART>
+__global__ __launch_bounds__(split_threads(NP), 2) void prefill_ild_kernel(const PrefillArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char prefill_smem_raw[];
     constexpr int HD = 2 * kIldHalf;
     const uint32_t G = a.group;
-    const uint32_t Gw = G < 4 ? G : 4;
-    const uint32_t chunks = G / Gw;
-    const uint32_t kvh = (uint32_t)__builtin_amdgcn_readfirstlane(blockIdx.x / chunks);
-    const uint32_t hc = (uint32_t)__builtin_amdgcn_readfirstlane(blockIdx.x % chunks);
-    const uint32_t BP = 32 * (4 / Gw);
+    const uint32_t Gw = G < NP ? G : NP;
+    const uint32_t kvh = (uint32_t)__builtin_amdgcn_readfirstlane(blockIdx.x % a.nkv);
+    const uint32_t hc = (uint32_t)__builtin_amdgcn_readfirstlane(blockIdx.x / a.nkv);
+    const uint32_t BP = 32 * (NP / Gw);
     const uint32_t nblk = (uint32_t)__builtin_amdgcn_readfirstlane((a.T + BP - 1) / BP);
     const uint32_t lo = blockIdx.y, hi = nblk - 1 - blockIdx.y;
     const unsigned char* kbase =
         uniform_ptr(reinterpret_cast<const unsigned char*>(a.k + (size_t)kvh * a.ctx_pad * HD));
     const unsigned char* vtbase = uniform_ptr(reinterpret_cast<const unsigned char*>(
         a.vt + (size_t)kvh * (a.ctx_pad / kVBlock) * HD * kVBlock));
-    ild_block<PART>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, blockIdx.z);
+    ild_block<NP, PART>(a, prefill_smem_raw, hi, kvh, hc, kbase, vtbase, blockIdx.z);
     if constexpr (!PART) {
         if (!a.single && hi != lo) {
             __syncthreads();                              // LDS changes hands
-            ild_block<false>(a, prefill_smem_raw, lo, kvh, hc, kbase, vtbase, 0);
+            ild_block<NP, false>(a, prefill_smem_raw, lo, kvh, hc, kbase, vtbase, 0);
         }
     }
 }

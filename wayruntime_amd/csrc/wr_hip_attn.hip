@@ -670,39 +670,71 @@ int check_decode(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32_
     return WR_HIP_OK;
 }
 
-// Into how many parts a launch's blocks are cut (one: not at all).  A launch of few rows lasts as long as its
-// longest block, whose keys one workgroup walks while most CUs stand idle; cut, every part pays a block's ends
-// (Q in, the sets' merge, rows out) and the rows go through memory once more.  In microseconds: the ends of a block,
-// a step (64 keys of a 32-row unit at head dims up to 128, 32 keys at 256; fewer workgroups than CUs), the combine
-// launch, what it takes a part, and the bytes it and the parts move.
-// Fitted to nine shapes by ten row counts by eight lengths before them, 1 to 32 parts each (profiles/prefill_parts.txt):
-// the parts picked are 0.6 to 1.1 % off the best on average, 19 % (2 us of 10) at worst, and never slower than none by
-// more than 4 %.  With one set of figures for all head dims, from 128, launches of 64 were cut too often and too fine
-// (500 rows behind 1024 keys, 32/8/64: 17.9 us whole, 20.6 cut).
-uint32_t prefill_parts(const PrefillArgs& a, uint32_t BP, uint32_t nblk, uint32_t ny)
+// How a prefill launch is cut: (head, 32-row block) pairs to a workgroup, one block or a long and a short one, and into how many
+// parts the blocks' keys go (one: not at all).
+struct PrefillPlan {
+    uint32_t np, nblk, ny, parts;
+    bool single;
+};
+
+// Four pairs to a workgroup feed eight waves, two to a SIMD, from each tile: the form for launches that fill the chip.  Launches
+// of fewer workgroups than CUs last as long as their longest block; with two pairs a workgroup has half the rows, a wave to
+// a SIMD whose steps take two thirds to nine tenths of the time, and there are twice as many.  A launch whose longest block is still a long chain
+// is cut into parts: every part pays a block's ends (Q in, the sets' merge, rows out) and the rows go through memory once more.
+// In microseconds: the ends of a block and a step (64 keys of a 32-row unit at head dims up to 128, 32 keys at 256) in
+// either form, the combine launch, what it takes a part, and the bytes it and the parts move.  Fitted to eleven shapes by thirteen
+// row counts by nine contexts and windows, both forms, 1 to 32 parts (profiles/prefill_parts.txt): what is picked is 0.7 to 1.4 % off the best
+// on average, 28 % at worst, and takes 0.91 (64), 0.93 (128) and 0.92 (256) of what the parts picked for four pairs alone take, 8 %
+// more at worst.  us a call, four pairs / two: 32/8/64, 500 rows 10.2 / 8.8; 16/8/128, 54 rows 9.0 / 7.9, 1024 rows 19.6 / 17.7; 16/8/256, 177
+// rows 13.9 / 11.3, 1501 rows 53 / 41; 8/4/256, 1501 rows of a 512-key window 25.1 / 21.3.
+PrefillPlan prefill_plan(const PrefillArgs& a, bool parts_form)
 {
     struct Cost {
-        float step, mb_us, part;
+        float ends[2], step[2], combine, part, mb_us;
     };
-    const Cost c = a.hd == 64 ? Cost{0.7f, 2.f, 0.2f} : a.hd == 128 ? Cost{0.8f, 2.5f, 0.2f} : Cost{1.f, 4.f, 0.25f};
-    const float ends = 8.f, combine = 3.f;
+    const Cost c = a.hd == 64    ? Cost{{6.5f, 10.2f}, {0.61f, 0.72f}, 4.9f, 0.33f, 3.2f}
+                   : a.hd == 128 ? Cost{{7.2f, 9.f}, {0.6f, 0.68f}, 2.5f, 0.22f, 3.5f}
+                                 : Cost{{7.f, 8.7f}, {0.89f, 0.96f}, 2.1f, 0.45f, 4.6f};
     const float row_mb = (float)a.T * a.nq * a.hd * 4e-6f;
     const uint64_t row_bytes = (uint64_t)a.T * a.nq * (a.hd + 2) * 4;
     const uint64_t room = (uint64_t)g.prefill_part_mb.load(std::memory_order_relaxed) << 20;
-    const uint32_t last_lo = a.p0 + (nblk - 1) * BP, hi = a.p0 + a.T;          // the last block's first position, keys
-    const uint32_t lo = (a.window > 0 && last_lo + 1 > a.window) ? last_lo + 1 - a.window : 0;
-    const uint32_t tiles = (hi + kTileKeys - 1) / kTileKeys - lo / kTileKeys, per_step = a.hd == 256 ? 1 : 2;
-    uint32_t best = 1;
+    const uint32_t per_step = a.hd == 256 ? 1 : 2;
+    PrefillPlan best{};
     float least = 0.f;
-    for (uint32_t p = 1; p <= kMaxPrefillParts; p++) {
-        if (p > 1 && p * row_bytes > room) break;
-        const uint32_t rounds = (nblk * ny * p + g.n_cus - 1) / g.n_cus;
-        const uint32_t steps = ((tiles + p - 1) / p + per_step - 1) / per_step;
-        float t = rounds * (ends + c.step * steps);
-        if (p > 1) t += combine + c.part * p + 2.f * p * row_mb / c.mb_us;
-        if (p == 1 || t < least) {
-            least = t;
-            best = p;
+    for (uint32_t np = 4; np >= (parts_form ? 2u : 4u); np -= 2) {
+        const uint32_t Gw = std::min(a.group, np), BP = 32 * (np / Gw);
+        const uint32_t nblk = (a.T + BP - 1) / BP, ny = a.nkv * (a.group / Gw);
+        const float ends = c.ends[np / 4], step = c.step[np / 4];
+        // tiles of the first and the last block, and of a block on average: as many as the last from where the window is full on
+        const auto tiles_of = [&](uint32_t b) {
+            const uint32_t lo = a.p0 + b * BP, hi = a.p0 + std::min(a.T, (b + 1) * BP);
+            const uint32_t from = (a.window > 0 && lo + 1 > a.window) ? lo + 1 - a.window : 0;
+            return (hi + kTileKeys - 1) / kTileKeys - from / kTileKeys;
+        };
+        const uint32_t first = tiles_of(0), longest = std::max(first, tiles_of(nblk - 1));
+        const float ramp = a.window == 0 ? 1.f : a.window > a.p0 ? std::min(1.f, (float)(a.window - a.p0) / a.T) : 0.f;
+        const float mean = longest - ramp * (longest - first) * 0.5f;
+        // Four pairs: a long and a short block to a workgroup balance the causal triangle, but each pays its own
+        // prologue and epilogue: when the pairs of blocks would not even give every CU a workgroup, one block per workgroup
+        // finishes with the longest block instead of with a pair's sum plus a second prologue and epilogue.
+        const uint32_t two = (nblk + 1) / 2 * ny;
+        const bool single = np == 2 || two < g.n_cus;
+        for (uint32_t p = 1; p <= (parts_form && single ? std::min(kMaxPrefillParts, longest) : 1u); p++) {
+            if (p > 1 && p * row_bytes > room) break;
+            float t;
+            if (!single) {
+                t = ((two + g.n_cus - 1) / g.n_cus) * (2.f * ends - 2.f + step * 2.f * mean / per_step);
+            } else {
+                const uint32_t rounds = (nblk * ny * p + g.n_cus - 1) / g.n_cus;
+                t = ends + step * (((longest + p - 1) / p + per_step - 1) / per_step);
+                if (rounds > 1)                              // long blocks first: the rounds even out
+                    t = std::max(t, rounds * (np == 2 ? 0.95f : 1.f) * (ends + step * mean / (p * per_step)));
+            }
+            if (p > 1) t += c.combine + c.part * p + 2.f * p * row_mb / c.mb_us;
+            if (best.np == 0 || t < least) {
+                least = t;
+                best = PrefillPlan{np, nblk, ny, p, single};
+            }
         }
     }
     return best;
@@ -746,47 +778,45 @@ int prefill_locked(wr_hip_kv* kv, uint32_t layer, uint32_t p0, uint32_t T, const
                       (G == 1 || G == 2 || G == 4 || G == 8);
     if (q16_dev && !(mfma && (hd == 64 || hd == 128))) return WR_HIP_ERR_UNSUPPORTED;
     if (mfma) {
-        const uint32_t Gw = G < 4 ? G : 4;
-        const uint32_t BP = 32 * (4 / Gw);
-        const uint32_t nblk = (T + BP - 1) / BP;
-        const uint32_t ny = kv->nkv * (G / Gw);
-        // A long and a short block per workgroup balance the causal triangle, but
-        // every block pays its own prologue and epilogue: when the pairs would
-        // not even give every CU a workgroup, one block per workgroup finishes
-        // with the longest block instead of with a pair's sum plus a second
-        // prologue and epilogue.
-        a.single = ((nblk + 1) / 2) * ny < g.n_cus ? 1 : 0;
-        const uint32_t nwg = a.single ? nblk : (nblk + 1) / 2;
-        const bool parts_form = hd == 64 || (hd == 128 && g.prefill_two_waves) || (hd == 256 && !g.prefill_256_four_waves);
-        const uint32_t parts = parts_form && a.single ? prefill_parts(a, BP, nblk, ny) : 1;
-        if (parts > 1 && prefill_parts_ready(a, parts)) {
-            const dim3 grid(ny, nblk, parts);
-            if (hd == 64)
-                launch_main(prefill_il_kernel<64, true>, grid, dim3(kSplitThreads), a, split_smem_bytes<64>());
-            else if (hd == 128)
-                launch_main(prefill_il_kernel<128, true>, grid, dim3(kSplitThreads), a, split_smem_bytes<128>());
-            else
-                launch_main(prefill_ild_kernel<true>, grid, dim3(kSplitThreads), a, ild_smem_bytes());
-            HIP_TRY(hipGetLastError(), "prefill launch", layer);
-            const uint32_t units = T * nq * (hd / 4);     // (bounded: few workgroups made these rows)
-            hipLaunchKernelGGL(prefill_combine_kernel, dim3((units + 255) / 256), dim3(256), 0, cx->stream, a);
-        } else if (hd == 64)
-            launch_main(prefill_il_kernel<64, false>, dim3(ny, nwg), dim3(kSplitThreads), a,
-                        split_smem_bytes<64>());
-        else if (hd == 128 && !g.prefill_two_waves) {
+        const bool one_wave = hd == 128 && !g.prefill_two_waves, four_waves = hd == 256 && g.prefill_256_four_waves;
+        PrefillPlan p = prefill_plan(a, !one_wave && !four_waves);
+        a.single = p.single;
+        if (p.parts > 1 && !prefill_parts_ready(a, p.parts)) p.parts = 1;
+        const dim3 grid(p.ny, p.single ? p.nblk : (p.nblk + 1) / 2, p.parts);
+        if (one_wave) {
             if (q16_dev)
-                launch_main(prefill_pair_kernel<128, true>, dim3(ny, nwg), dim3(kPairThreads), a,
-                            pair_smem_bytes<128>());
+                launch_main(prefill_pair_kernel<128, true>, grid, dim3(kPairThreads), a, pair_smem_bytes<128>());
             else
-                launch_main(prefill_pair_kernel<128, false>, dim3(ny, nwg), dim3(kPairThreads), a,
-                            pair_smem_bytes<128>());
-        } else if (hd == 128)
-            launch_main(prefill_il_kernel<128, false>, dim3(ny, nwg), dim3(kSplitThreads), a,
-                        split_smem_bytes<128>());
-        else if (!g.prefill_256_four_waves)   // 256: the wave sets divide the dimensions
-            launch_main(prefill_ild_kernel<false>, dim3(ny, nwg), dim3(kSplitThreads), a, ild_smem_bytes());
-        else   // the earlier form: one wave per SIMD owns all 256 dimensions of its rows
-            launch_main(prefill_mfma_kernel<256>, dim3(nwg, ny), dim3(kPrefillThreads), a);
+                launch_main(prefill_pair_kernel<128, false>, grid, dim3(kPairThreads), a, pair_smem_bytes<128>());
+        } else if (four_waves) {   // the earlier form: one wave per SIMD owns all 256 dimensions of its rows
+            launch_main(prefill_mfma_kernel<256>, dim3(grid.y, grid.x), dim3(kPrefillThreads), a);
+        } else {
+            const auto launch = [&](auto np, auto part) {
+                constexpr int NP = decltype(np)::value;
+                constexpr bool PART = decltype(part)::value;
+                if (hd == 64)
+                    launch_main(prefill_il_kernel<64, NP, PART>, grid, dim3(split_threads(NP)), a, split_smem_bytes<64, NP>());
+                else if (hd == 128)
+                    launch_main(prefill_il_kernel<128, NP, PART>, grid, dim3(split_threads(NP)), a, split_smem_bytes<128, NP>());
+                else   // 256: the wave sets divide the dimensions
+                    launch_main(prefill_ild_kernel<NP, PART>, grid, dim3(split_threads(NP)), a, ild_smem_bytes<NP>());
+            };
+            const auto whole_or_parts = [&](auto np) {
+                if (p.parts > 1)
+                    launch(np, std::true_type());
+                else
+                    launch(np, std::false_type());
+            };
+            if (p.np == 2)
+                whole_or_parts(std::integral_constant<int, 2>());
+            else
+                whole_or_parts(std::integral_constant<int, 4>());
+            if (p.parts > 1) {
+                HIP_TRY(hipGetLastError(), "prefill launch", layer);
+                const uint32_t units = T * nq * (hd / 4);     // (bounded: few workgroups made these rows)
+                hipLaunchKernelGGL(prefill_combine_kernel, dim3((units + 255) / 256), dim3(256), 0, cx->stream, a);
+            }
+        }
     } else {
         launch_main(prefill_generic_kernel, dim3(T, nq), dim3(kDecodeThreads), a);
     }
@@ -1356,39 +1386,26 @@ int wr_hip_attn_init(int device)
         }
     }
     if (rc == WR_HIP_OK) {
-        // the two-waves-per-SIMD prefill kernels stage more than the 64 KiB a
-        // kernel may use without asking
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<64, false>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)split_smem_bytes<64>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<128, false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)split_smem_bytes<128>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<64, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_smem_bytes<64>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_il_kernel<128, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)split_smem_bytes<128>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_ild_kernel<true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)ild_smem_bytes());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_pair_kernel<128, false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)pair_smem_bytes<128>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_pair_kernel<128, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)pair_smem_bytes<128>());
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_ild_kernel<false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)ild_smem_bytes());
+        hipError_t e = hipSuccess;
         const auto allow_lds = [&](auto kernel, size_t bytes) {
             if (kernel && e == hipSuccess)
                 e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         };
+        // the prefill kernels stage more than the 64 KiB a kernel may use without asking
+        allow_lds(prefill_il_kernel<64, 4, false>, split_smem_bytes<64, 4>());
+        allow_lds(prefill_il_kernel<64, 4, true>, split_smem_bytes<64, 4>());
+        allow_lds(prefill_il_kernel<64, 2, false>, split_smem_bytes<64, 2>());
+        allow_lds(prefill_il_kernel<64, 2, true>, split_smem_bytes<64, 2>());
+        allow_lds(prefill_il_kernel<128, 4, false>, split_smem_bytes<128, 4>());
+        allow_lds(prefill_il_kernel<128, 4, true>, split_smem_bytes<128, 4>());
+        allow_lds(prefill_il_kernel<128, 2, false>, split_smem_bytes<128, 2>());
+        allow_lds(prefill_il_kernel<128, 2, true>, split_smem_bytes<128, 2>());
+        allow_lds(prefill_ild_kernel<4, false>, ild_smem_bytes<4>());
+        allow_lds(prefill_ild_kernel<4, true>, ild_smem_bytes<4>());
+        allow_lds(prefill_ild_kernel<2, false>, ild_smem_bytes<2>());
+        allow_lds(prefill_ild_kernel<2, true>, ild_smem_bytes<2>());
+        allow_lds(prefill_pair_kernel<128, false>, pair_smem_bytes<128>());
+        allow_lds(prefill_pair_kernel<128, true>, pair_smem_bytes<128>());
         // (a gated row: 6 KiB of partial tiles beside its terms, more than 64 KiB together from 14 848 inputs on)
         allow_lds(proj_rows_down_kernel<1>, kOnePerCuLds);
         allow_lds(proj_rows_down_kernel<2>, kOnePerCuLds);
