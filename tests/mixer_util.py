@@ -13,13 +13,13 @@ TOL = {"f32": 2e-5, "bf16": 4e-2}
 class Case:
     """A model on the device and its oracle."""
 
-    def __init__(self, eng, tmp_path, cfg, prec, seed=1, edit=None, pool=1024, slots=4):
+    def __init__(self, eng, tmp_path, cfg, prec, seed=1, edit=None, pool=1024, slots=4, rank=24):
         self.cfg, self.prec = cfg, prec
-        bits = dict(mw.random_tensors(cfg, seed))
+        bits = dict(mw.random_tensors(cfg, seed, rank=rank))
         if edit:
             edit(bits)
         self.w = {k: O.bf16_to_f32(v) for k, v in bits.items()}
-        self.m = eng.load(mw.write_model(str(tmp_path / "model"), cfg, bits), max_context=pool,
+        self.m = eng.load(mw.write_model(str(tmp_path / "model"), cfg, bits, rank=rank), max_context=pool,
                           quant=E.WR_QUANT_F32 if prec == "f32" else E.WR_QUANT_AUTO)
         self.m.set_cache_pool(pool, slots)
 

@@ -357,6 +357,20 @@ def test_token_shift_over_every_border(eng, tmp_path, prec):
     case.close()
 
 
+@pytest.mark.parametrize("rank", [20, 40, 64, 97, 128, 130])
+@pytest.mark.parametrize("dim", [16, 40, 64, 128])
+def test_decays_of_short_portions(eng, tmp_path, prec, dim, rank):
+    # one to four tiles of the decays' ranks, a tile to a quarter of the threads, and a rank too large for that;
+    # portions of one row, of two and of several, whose rows are asked for one ahead
+    cfg = mw.prenorm_config(72, 90, [(mw.wkv(2, dim), None), (par(right=(2, dim), **RIGHT), None)])
+    case = Case(eng, tmp_path, cfg, prec, rank=rank)
+    t = case.tokens(31)
+    want = case.oracle(t)
+    for cuts in ([1], [2, 1, 3], [9, 15, 7]):
+        case.check(run_cut(case, t, cuts), want, f"rank {rank}, dim {dim}, cuts {cuts}")
+    case.close()
+
+
 def test_long_decoding(eng, tmp_path, prec):
     case = Case(eng, tmp_path, stack(), prec)
     t = case.tokens(420)

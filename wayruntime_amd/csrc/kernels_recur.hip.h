@@ -110,58 +110,87 @@ __device__ __forceinline__ float recur_wave_sum(float v)
     return v;
 }
 
-// Row r's product with output n of the decay's matrix.
+// Ranks (in tiles of 32) up to which a decoded token's decays are made in passing: a tile to each quarter of the threads.
+constexpr uint32_t kDecayTiles = 4;
+
+// What a thread reads of a row: asked for a row ahead.
 template <bool F32>
-__device__ __forceinline__ float recur_z(const RecurArgs& a, uint32_t r, uint32_t n)
-{
-    using V8 = typename MixAct<F32>::V8;
-    float z = 0.f;
-    for (uint32_t kt = 0; kt < a.low_kt; kt++) {
-        bf16x8 w[4];
-        V8 x[4];
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            w[g] = a.wd[((size_t)(n / 16) * a.low_kt + kt) * 64 + 16 * g + n % 16];
-            x[g] = reinterpret_cast<const V8*>(a.low)[frag_unit(r, kt * 4 + g, a.low_kt)];
-        }
-#pragma unroll
-        for (int g = 0; g < 4; g++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) z = fmaf((float)w[g][j], (float)x[g][j], z);
-    }
-    return z;
-}
+struct RecurRow {
+    float v, r, k, g, a, z;
+    typename MixAct<F32>::V8 x[4];   // its quarter's tile of the decay's input
+};
 
 // grid (requests, heads), 4 DP threads: thread t has value column t % DP, channels DPT (t / DP) .. +DPT
+//
+// Few rows: bound by a chain of trips to memory, of which there are three: arguments, the request's record, then its state,
+// its row, the decay's input and weights side by side (one after the other, and the list of requests where that is all of them, they
+// were six; 32 heads of 64: 16 requests 9.3 -> 8.2 us, 8 rows of one 15 -> 11.4).
 template <bool F32, int DP, bool DELTA>
 __global__ __launch_bounds__(4 * DP) void recur_step_kernel(const RecurArgs a)
 {
+    using V8 = typename MixAct<F32>::V8;
     constexpr int DPT = DP / 4, WV = DP >= 64 ? DP / 64 : 1;       // waves that hold the channels' own values
-    __shared__ float sr[DP], sk[DP], sw[DP], sn[DP], sb[DP], red[8 * DP], sums[3 * WV], sq[WV];
+    __shared__ float sr[DP], sk[DP], sw[DP], sn[DP], sb[DP], red[8 * DP], sums[3 * WV], sq[WV], sz[4 * DP];
     const uint32_t t = threadIdx.x, head = blockIdx.y, part = t / DP, c = t % DP, d0 = part * DPT, D = a.dim;
     const uint32_t lane = t & 63, wave = t >> 6;
     const bool has = c < D, own = t < DP && has;                  // (own: also the thread of channel c's values)
-    const MixSeq s = a.seqs[a.list[blockIdx.x]];
+    const uint32_t hd = head * D, npad = (a.heads * D + 31) / 32 * 32, cc = has ? c : 0;
+    const MixSeq s = a.seqs[a.list ? a.list[blockIdx.x] : blockIdx.x];
+    const float w0 = a.w0[hd + cc], nrm = a.norm[hd + cc], ub = DELTA ? a.ab[hd + cc] : a.u[hd + cc];
+    const bool low = a.wd != nullptr, tile = low && part < a.low_kt;
+    bf16x8 wd[4];
+    if (tile) {
+        const uint32_t n = hd + cc;
+#pragma unroll
+        for (int g = 0; g < 4; g++) wd[g] = a.wd[((size_t)(n / 16) * a.low_kt + part) * 64 + 16 * g + n % 16];
+    }
+    const auto ask = [&](RecurRow<F32>& q, uint32_t r) {
+        const float* row = a.in + (size_t)r * a.ld + hd + cc;
+        if (tile) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) q.x[g] = reinterpret_cast<const V8*>(a.low)[frag_unit(r, part * 4 + g, a.low_kt)];
+        }
+        if (t < DP) {
+            q.r = row[a.col_r];
+            q.k = row[a.col_k];
+            q.g = row[a.col_g];
+            q.a = DELTA ? row[a.col_a] : 0.f;
+            q.z = low ? 0.f : a.z[(size_t)r * a.ldz + hd + cc];
+        }
+        q.v = row[a.col_v];
+    };
+    RecurRow<F32> next;
+    ask(next, s.row0);
     const size_t head_elems = (size_t)D * D;
     const float* in = a.state + ((size_t)s.state_in * a.heads + head) * head_elems;
     float* out = a.state + ((size_t)s.state_out * a.heads + head) * head_elems;
-    const uint32_t hd = head * D, npad = (a.heads * D + 31) / 32 * 32;
     float S[DPT];
 #pragma unroll
     for (int j = 0; j < DPT; j++) S[j] = (s.pos0 > 0 && has && d0 + j < D) ? in[(size_t)(d0 + j) * D + c] : 0.f;
-    const float w0 = own ? a.w0[hd + c] : 0.f, nrm = own ? a.norm[hd + c] : 0.f;
-    const float ub = own ? (DELTA ? a.ab[hd + c] : a.u[hd + c]) : 0.f;
     for (uint32_t i = 0; i < s.rows; i++) {
         const uint32_t r = s.row0 + i;
-        const float* row = a.in + (size_t)r * a.ld + hd;
-        const float vv = has ? row[a.col_v + c] : 0.f;
-        float g = 0.f;
+        const float vv = has ? next.v : 0.f, rr = own ? next.r : 0.f, kk = own ? next.k : 0.f, g = own ? next.g : 0.f, za = next.a;
+        float z = next.z;
+        if (low) {                                                // the row's product with the decay's matrix, a tile of inputs to a quarter
+            if (tile) {
+                z = 0.f;
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) z = fmaf((float)wd[q][j], (float)next.x[q][j], z);
+                sz[t] = z;
+            }
+            __syncthreads();
+            if (own) {
+                z = sz[c];
+                for (uint32_t q = 1; q < a.low_kt; q++) z += sz[q * DP + c];
+            }
+        }
+        if (i + 1 < s.rows) ask(next, r + 1);
         if (wave < WV) {
-            const float rr = own ? row[a.col_r + c] : 0.f, kk = own ? row[a.col_k + c] : 0.f;
-            const float w = own ? recur_decay(a, (a.wd ? recur_z<F32>(a, r, hd + c) : a.z[(size_t)r * a.ldz + hd + c]) + w0) : 0.f;
-            g = own ? row[a.col_g + c] : 0.f;
+            const float w = own ? recur_decay(a, z + w0) : 0.f;
             if constexpr (DELTA) {
-                const float rate = own ? 1.0f / (1.0f + expf(-(row[a.col_a + c] + ub))) : 0.f;
+                const float rate = own ? 1.0f / (1.0f + expf(-(za + ub))) : 0.f;
                 const float k2 = recur_wave_sum(kk * kk), rk = recur_wave_sum(rr * kk), rak = recur_wave_sum(rr * rate * kk);
                 if (lane == 0) {
                     sums[wave] = k2;
@@ -176,7 +205,7 @@ __global__ __launch_bounds__(4 * DP) void recur_step_kernel(const RecurArgs a)
                     sb[t] = rate * kk;
                 }
             } else {
-                const float ruk = recur_wave_sum(rr * ub * kk);
+                const float ruk = recur_wave_sum(own ? rr * ub * kk : 0.f);
                 if (lane == 0) sums[wave] = ruk;
                 if (t < DP) {
                     sr[t] = rr;

@@ -992,9 +992,6 @@ static int recur_chunks(wr_hip_mix_step* s, RecurArgs& a)
     return WR_HIP_OK;
 }
 
-// Ranks (in tiles of 32) up to which a decoded token's decays are made in passing.
-constexpr uint32_t kDecayTiles = 4;
-
 template <bool F32, bool DELTA>
 static int recur_run(wr_hip_mix_step* s, RecurArgs& a, const wr_hip_mix_recurrence* q)
 {
@@ -1024,7 +1021,7 @@ static int recur_run(wr_hip_mix_step* s, RecurArgs& a, const wr_hip_mix_recurren
         else rc = recur_chunks<F32, 4, RULE, 8>(s, a);
         if (rc) return rc;
     }
-    a.list = s->d<uint32_t>(chunked ? s->o_short : s->o_all);
+    a.list = chunked ? s->d<uint32_t>(s->o_short) : nullptr;      // (all requests)
     return recur_steps<F32, DELTA>(a, chunked ? s->n_short : s->n_seq);
 }
 
