@@ -179,6 +179,8 @@ typedef struct wr_hip_mix_gemm {
     const float *x_scale;          /* with group_expert: row i's outputs are those of x_scale[i] times its input */
 } wr_hip_mix_gemm;
 int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm *a);
+/* The same for two products that neither read nor overwrite what the other writes; few rows take one launch where the second is small. */
+int wr_hip_mix_gemm_run_two(int f32, const wr_hip_mix_gemm *a, const wr_hip_mix_gemm *small);
 
 /* ---- decayed linear attention ------------------------------------------------
  * Per head S_t = decay S_(t-1) + k_t v_t^T, o_t = S_t^T q_t.  qkv: activation-type
@@ -281,6 +283,12 @@ uint32_t wr_hip_mix_window_pad(uint32_t dim);
 int wr_hip_mix_window_append(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t run, int f32,
                              const wr_hip_mix_window *g, const float *in_dev, uint32_t ld, uint32_t col_q,
                              uint32_t col_k, uint32_t col_v, const float *table_dev, void *q_dev);
+/* wr_hip_mix_window_append, then wr_hip_mix_recur with layer run recur_run, neither of which reads or overwrites what the other
+ * writes; a step of few rows takes one launch for both. */
+int wr_hip_mix_window_append_recur(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t run, int f32,
+                                   const wr_hip_mix_window *g, const float *in_dev, uint32_t ld, uint32_t col_q,
+                                   uint32_t col_k, uint32_t col_v, const float *table_dev, void *q_dev,
+                                   uint32_t recur_run, const wr_hip_mix_recurrence *recur);
 /* Softmax attention over the cached rows inside the window; with `sink`, a head's weights
  * are exp(score) / (exp(sink[head]) + sum of exp(score)).  With two maps a head's output is
  * first - diff * second, over its root mean square (eps).  Head h's output times out_scale,

@@ -288,6 +288,12 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm *a)
     return WR_HIP_OK;
 }
 
+int wr_hip_mix_gemm_run_two(int f32, const wr_hip_mix_gemm *a, const wr_hip_mix_gemm *small)
+{
+    const int rc = wr_hip_mix_gemm_run(f32, a);
+    return rc ? rc : wr_hip_mix_gemm_run(f32, small);
+}
+
 int wr_hip_mix_lightning(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t run, int f32, uint32_t heads, uint32_t dim,
                          uint32_t vdim, const float *decay, const void *qkv, uint32_t ld, uint32_t col_k, uint32_t col_v,
                          float *o, uint32_t ldo)
@@ -586,6 +592,14 @@ int wr_hip_mix_window_append(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t
         }
     }
     return WR_HIP_OK;
+}
+
+int wr_hip_mix_window_append_recur(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t run, int f32, const wr_hip_mix_window *g,
+                                   const float *in, uint32_t ld, uint32_t col_q, uint32_t col_k, uint32_t col_v, const float *table,
+                                   void *qv, uint32_t recur_run, const wr_hip_mix_recurrence *recur)
+{
+    const int rc = wr_hip_mix_window_append(s, pool, run, f32, g, in, ld, col_q, col_k, col_v, table, qv);
+    return rc ? rc : wr_hip_mix_recur(s, pool, recur_run, f32, recur);
 }
 
 int wr_hip_mix_window_attend(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t run, int f32, const wr_hip_mix_window *g,

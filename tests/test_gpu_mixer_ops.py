@@ -196,6 +196,30 @@ def test_batch_of_matrices(lib, f32, batch, N, K, rows):
         b.free()
 
 
+# (batch, outputs, small one's outputs and inputs, rows): one launch where both are of sixteen rows at most and the second is small; else two
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("batch,N,K,n,k,rows", [(4, 1536, 288, 64, 288, 16), (1, 6144, 512, 16, 96, 1), (3, 2064, 1056, 48, 2048, 7), (2, 3088, 2080, 32, 4128, 5),
+                                                (4, 1536, 288, 64, 2080, 9), (4, 1536, 256, 64, 288, 3), (4, 1520, 288, 64, 288, 16), (4, 1536, 288, 400, 288, 16),
+                                                (4, 1536, 288, 64, 288, 17)])
+def test_two_products(lib, f32, batch, N, K, n, k, rows):
+    lib.wr_hip_mix_gemm_run_two.argtypes = [C.c_int, C.POINTER(Gemm), C.POINTER(Gemm)]
+    r, q = Run(lib, f32, batch, N, K, rows), Run(lib, f32, 1, n, k, rows, seed=1)
+    x, u = r.act(rows, batch * K), q.act(rows, k)
+    xd, ud = r.up(x), q.up(u)
+    y, h = hipattn.DeviceBuffer(rows * batch * N * 4), hipattn.DeviceBuffer(-(-rows // 16) * 16 * (n + 31) // 32 * 32 * (4 if f32 else 2))
+    a = Gemm(w=r.h, x=xd.p, x_kt=batch * K // 32, x_kt_z=K // 32, rows=rows, out=ROWS_F32, y_f32=y.p, ldy=batch * N, col_z=N)
+    b = Gemm(w=q.h, x=ud.p, x_kt=k // 32, rows=rows, out=FRAG, h=h.p, h_kt=(n + 31) // 32, tanh_end=n)
+    assert lib.wr_hip_mix_gemm_run_two(int(f32), C.byref(a), C.byref(b)) == 0
+    hipattn.sync()
+    r.close(y.to_host((rows, batch * N)), np.einsum("rzk,znk->rzn", x.reshape(rows, batch, K).astype(np.float64), r.w.astype(np.float64)).reshape(rows, -1))
+    q.close(q.frag_down(h, rows, (n + 31) // 32 * 32)[:, :n], np.tanh(u.astype(np.float64) @ q.w[0].T.astype(np.float64)), eight_bits=True)
+    b.h = None                                             # refused whole, whichever of the two it is
+    assert lib.wr_hip_mix_gemm_run_two(int(f32), C.byref(a), C.byref(b)) == hipattn.ERR_INVAL
+    r.end(), q.end()
+    for d in (xd, ud, y, h):
+        d.free()
+
+
 # ... in tiles of 256 outputs by 128 and 256 rows, the matrices on all XCDs and on one each (batches of 16 and more that eight divides)
 @pytest.mark.parametrize("batch,N,K,rows", [(2, 7584, 2080, 400), (4, 7712, 2080, 130), (8, 4000, 2080, 130), (3, 6688, 2080, 280),
                                             (2, 7328, 1056, 910), (4, 7328, 1056, 400), (8, 7584, 1056, 130), (3, 6560, 1056, 670),

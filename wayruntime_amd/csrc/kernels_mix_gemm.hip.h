@@ -172,15 +172,14 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // half of them idle is half the rate.  16 rows, weights from HBM: 8192 -> 2048 11.5 -> 9.4
 // us, -> 512 10.6 -> 7.8; 6144 -> 2048 9.4 -> 7.8; 4096 -> 2048 7.0 -> 6.6, -> 1024 6.7 ->
 // 6.0; at 2048 inputs the exchange costs more (4.8 -> 5.2).
-template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS = 1, bool PICKED = false>
-__global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_kernel(const MixGemmArgs a)
+template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS, bool PICKED>
+__device__ __forceinline__ void mix_gemm_split(const MixGemmArgs& a, uint32_t bx, uint32_t by, uint32_t z)
 {
     using V8 = typename MixAct<F32>::V8;
     __shared__ f32x4 s_part[WAVES * NT * GR * 64];
     const int lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     static_assert(PARTS == 1 || (PARTS == 2 && NT == 1 && GR == 1), "one tile, two halves");
-    uint32_t bx = blockIdx.x, by = blockIdx.y;
     if constexpr (STREAM && GR > 1 && !PICKED) {
         if (a.cols) {                                      // runs, up to a multiple of 8: a run's workgroups on one XCD
             const uint32_t id = by * gridDim.x + bx, in_xcd = id / 8, y = in_xcd / gridDim.x * 8 + id % 8;
@@ -189,7 +188,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
             if (by * GR >= a.groups) return;
         }
     }
-    const uint32_t nt0 = bx * NT, group0 = PARTS > 1 ? 0 : PICKED ? by : by * GR, part = PARTS > 1 ? by : 0, z = blockIdx.z;
+    const uint32_t nt0 = bx * NT, group0 = PARTS > 1 ? 0 : PICKED ? by : by * GR, part = PARTS > 1 ? by : 0;
     uint32_t mat = z, live = GR;                           // live: groups that rows are in (those of a run come first)
     if (a.group_expert) {
         const int e = a.group_expert[group0];
@@ -373,6 +372,27 @@ __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_
         if (u % GR >= live) continue;
         const f32x4 v = sum(u);
         mix_store_tile<F32>(a, v, v, nt0 + u / GR, group0 + u % GR, z, lane);
+    }
+}
+
+template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS = 1, bool PICKED = false>
+__global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_kernel(const MixGemmArgs a)
+{
+    mix_gemm_split<F32, NT, GR, WAVES, DEPTH, STREAM, PARTS, PICKED>(a, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// Two products of up to sixteen rows that do not wait for each other: a's batch of matrices, and a small one whose few tiles took a launch
+// of their own (16 rows, four of 2048 -> 2048 and 2048 -> 64: 8.7 and 4.6 us, 10.6 together).
+// The small one's workgroups come first: they end as the others do.
+template <int WAVES, int DEPTH>
+__global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_two_kernel(const MixGemmArgs a, const MixGemmArgs b)
+{
+    const uint32_t of_b = (b.ntiles + 1) / 2, of_a = (a.ntiles + 1) / 2;
+    if (blockIdx.x < of_b) {
+        mix_gemm_split<false, 2, 1, WAVES, DEPTH, true, 1, false>(b, blockIdx.x, 0, 0);
+    } else {
+        const uint32_t i = blockIdx.x - of_b;
+        mix_gemm_split<false, 2, 1, WAVES, DEPTH, true, 1, false>(a, i % of_a, 0, i / of_a);
     }
 }
 

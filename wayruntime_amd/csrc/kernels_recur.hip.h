@@ -113,6 +113,28 @@ __device__ __forceinline__ float recur_wave_sum(float v)
 // Ranks (in tiles of 32) up to which a decoded token's decays are made in passing: a tile to each quarter of the threads.
 constexpr uint32_t kDecayTiles = 4;
 
+// Row r's product with output n of the decay's matrix.
+template <bool F32>
+__device__ __forceinline__ float recur_z(const RecurArgs& a, uint32_t r, uint32_t n)
+{
+    using V8 = typename MixAct<F32>::V8;
+    float z = 0.f;
+    for (uint32_t kt = 0; kt < a.low_kt; kt++) {
+        bf16x8 w[4];
+        V8 x[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            w[g] = a.wd[((size_t)(n / 16) * a.low_kt + kt) * 64 + 16 * g + n % 16];
+            x[g] = reinterpret_cast<const V8*>(a.low)[frag_unit(r, kt * 4 + g, a.low_kt)];
+        }
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) z = fmaf((float)w[g][j], (float)x[g][j], z);
+    }
+    return z;
+}
+
 // What a thread reads of a row: asked for a row ahead.
 template <bool F32>
 struct RecurRow {
@@ -120,24 +142,25 @@ struct RecurRow {
     typename MixAct<F32>::V8 x[4];   // its quarter's tile of the decay's input
 };
 
-// grid (requests, heads), 4 DP threads: thread t has value column t % DP, channels DPT (t / DP) .. +DPT
+// One request and head, 4 DP threads: thread t has value column t % DP, channels DPT (t / DP) .. +DPT
 //
 // Few rows: bound by a chain of trips to memory, of which there are three: arguments, the request's record, then its state,
 // its row, the decay's input and weights side by side (one after the other, and the list of requests where that is all of them, they
 // were six; 32 heads of 64: 16 requests 9.3 -> 8.2 us, 8 rows of one 15 -> 11.4).
 template <bool F32, int DP, bool DELTA>
-__global__ __launch_bounds__(4 * DP) void recur_step_kernel(const RecurArgs a)
+__device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request, uint32_t head)
 {
     using V8 = typename MixAct<F32>::V8;
     constexpr int DPT = DP / 4, WV = DP >= 64 ? DP / 64 : 1;       // waves that hold the channels' own values
-    __shared__ float sr[DP], sk[DP], sw[DP], sn[DP], sb[DP], red[8 * DP], sums[3 * WV], sq[WV], sz[4 * DP];
-    const uint32_t t = threadIdx.x, head = blockIdx.y, part = t / DP, c = t % DP, d0 = part * DPT, D = a.dim;
+    constexpr bool QUARTERS = DP < 256;                           // (1024 threads have 128 registers each, and spill as it is)
+    __shared__ float sr[DP], sk[DP], sw[DP], sb[DP], red[8 * DP], sums[3 * WV], sq[WV], sz[QUARTERS ? 4 * DP : 1];
+    const uint32_t t = threadIdx.x, part = t / DP, c = t % DP, d0 = part * DPT, D = a.dim;
     const uint32_t lane = t & 63, wave = t >> 6;
     const bool has = c < D, own = t < DP && has;                  // (own: also the thread of channel c's values)
     const uint32_t hd = head * D, npad = (a.heads * D + 31) / 32 * 32, cc = has ? c : 0;
-    const MixSeq s = a.seqs[a.list ? a.list[blockIdx.x] : blockIdx.x];
+    const MixSeq s = a.seqs[a.list ? a.list[request] : request];
     const float w0 = a.w0[hd + cc], nrm = a.norm[hd + cc], ub = DELTA ? a.ab[hd + cc] : a.u[hd + cc];
-    const bool low = a.wd != nullptr, tile = low && part < a.low_kt;
+    const bool low = a.wd != nullptr, tile = QUARTERS && low && part < a.low_kt;
     bf16x8 wd[4];
     if (tile) {
         const uint32_t n = hd + cc;
@@ -171,13 +194,17 @@ __global__ __launch_bounds__(4 * DP) void recur_step_kernel(const RecurArgs a)
         const uint32_t r = s.row0 + i;
         const float vv = has ? next.v : 0.f, rr = own ? next.r : 0.f, kk = own ? next.k : 0.f, g = own ? next.g : 0.f, za = next.a;
         float z = next.z;
-        if (low) {                                                // the row's product with the decay's matrix, a tile of inputs to a quarter
+        if (!QUARTERS) {
+            if (low && own) z = recur_z<F32>(a, r, hd + c);
+        } else if (low) {                                         // the row's product with the decay's matrix, a tile of inputs to a quarter
             if (tile) {
                 z = 0.f;
 #pragma unroll
-                for (int q = 0; q < 4; q++)
+                for (int q = 0; q < 4; q++) {
+                    asm volatile("" : "+v"(wd[q]));               // (widened here, not ahead of the loop into twice the registers)
 #pragma unroll
                     for (int j = 0; j < 8; j++) z = fmaf((float)wd[q][j], (float)next.x[q][j], z);
+                }
                 sz[t] = z;
             }
             __syncthreads();
@@ -201,7 +228,6 @@ __global__ __launch_bounds__(4 * DP) void recur_step_kernel(const RecurArgs a)
                     sr[t] = rr * w;
                     sk[t] = kk;
                     sw[t] = w;
-                    sn[t] = kk;
                     sb[t] = rate * kk;
                 }
             } else {
@@ -224,7 +250,7 @@ __global__ __launch_bounds__(4 * DP) void recur_step_kernel(const RecurArgs a)
 #pragma unroll
         for (int j = 0; j < DPT; j++) {
             o = fmaf(sr[d0 + j], S[j], o);
-            if constexpr (DELTA) p = fmaf(sn[d0 + j], S[j], p);
+            if constexpr (DELTA) p = fmaf(sk[d0 + j], S[j], p);
         }
         red[t] = o;
         if constexpr (DELTA) red[4 * DP + t] = p;
@@ -275,6 +301,16 @@ __global__ __launch_bounds__(4 * DP) void recur_step_kernel(const RecurArgs a)
 #pragma unroll
     for (int j = 0; j < DPT; j++)
         if (has && d0 + j < D) out[(size_t)(d0 + j) * D + c] = S[j];
+}
+
+// Waves to a SIMD: three, so that the workgroups of sixteen requests of 32 heads are there at once, with an append's.
+constexpr int recur_step_waves(int dp) { return dp <= 64 ? 3 : 1; }
+
+// grid (requests, heads)
+template <bool F32, int DP, bool DELTA>
+__global__ __launch_bounds__(4 * DP, recur_step_waves(DP)) void recur_step_kernel(const RecurArgs a)
+{
+    recur_step<F32, DP, DELTA>(a, blockIdx.x, blockIdx.y);
 }
 
 // FORGET.  grid (requests, heads), 4 CP threads: thread t has value column t % CP, channels DPT (t / CP) .. +DPT

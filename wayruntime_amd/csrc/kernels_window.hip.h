@@ -30,6 +30,7 @@
 #pragma once
 
 #include "kernels_latent_mfma.hip.h"
+#include "kernels_recur.hip.h"
 
 namespace wr {
 
@@ -177,17 +178,17 @@ __device__ __forceinline__ float window_value(const WindowArgs& a, uint32_t r, u
     return v[d] * cs[0] + (d & 1 ? v[d - 1] : -v[d + 1]) * cs[1];
 }
 
-// grid (rows / 4, key_heads + slices of 4 rows' query units)
+// Four rows' keys and values of one head, or a slice of their query units (slice >= key_heads).
 template <bool F32>
-__global__ __launch_bounds__(256) void window_append_kernel(const WindowArgs a)
+__device__ __forceinline__ void window_append(const WindowArgs& a, uint32_t rows4, uint32_t slice)
 {
     using E = typename MixAct<F32>::E;
     using V4 = typename MixAct<F32>::V4;
     __shared__ float s_inv[4];
-    const uint32_t t = threadIdx.x, r0 = blockIdx.x * 4, n = min(4u, a.rows - r0), per_map = a.dimp / 8;
-    const bool whole = window_whole(a, blockIdx.y >= a.key_heads ? a.col_q : a.col_k);       // uniform
-    if (blockIdx.y >= a.key_heads) {
-        const uint32_t per = a.heads * a.maps * per_map, u0 = (blockIdx.y - a.key_heads) * kWindowQUnits;
+    const uint32_t t = threadIdx.x, r0 = rows4 * 4, n = min(4u, a.rows - r0), per_map = a.dimp / 8;
+    const bool whole = window_whole(a, slice >= a.key_heads ? a.col_q : a.col_k);       // uniform
+    if (slice >= a.key_heads) {
+        const uint32_t per = a.heads * a.maps * per_map, u0 = (slice - a.key_heads) * kWindowQUnits;
         for (uint32_t u = u0 + t; u < min(u0 + kWindowQUnits, 4 * per); u += 256) {
             const uint32_t i = u % 4, q = u / 4, r = r0 + min(i, n - 1);
             const float* x = a.in + (size_t)r * a.ld + a.col_q + q / per_map * a.dim;
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(256) void window_append_kernel(const WindowArgs a)
         }
         return;
     }
-    const uint32_t kvh = blockIdx.y, block = kMixPage * (a.dimk + a.vdimp);
+    const uint32_t kvh = slice, block = kMixPage * (a.dimk + a.vdimp);
     auto head_block = [&](uint32_t r) {
         const MixSeq s = a.seqs[a.row_seq[r]];
         return reinterpret_cast<E*>(a.cache) + ((size_t)a.pages[s.page0 + a.row_pos[r] / kMixPage] * a.kvh + kvh) * block;
@@ -248,6 +249,26 @@ __global__ __launch_bounds__(256) void window_append_kernel(const WindowArgs a)
             for (uint32_t i = 0; i < n; i++)
                 head_block(r0 + i)[kMixPage * a.dimk + window_v_elem(a.row_pos[r0 + i] % kMixPage, d, a.vdimp)] = x[i];
         }
+    }
+}
+
+// grid (rows / 4, key_heads + slices of 4 rows' query units)
+template <bool F32>
+__global__ __launch_bounds__(256) void window_append_kernel(const WindowArgs a)
+{
+    window_append<F32>(a, blockIdx.x, blockIdx.y);
+}
+
+// A step's recurrence and the append beside it, which read one product's rows and write apart: workgroups below
+// `steps` are a request and head each, the others the append's, append_x of them to a slice.  In launches of their own the append's
+// few workgroups took as long as a launch takes (16 rows, 16/8 heads of 128 beside 32 of 64: 6.2 and 8.3 us, 9.6 together).
+__global__ __launch_bounds__(256, recur_step_waves(64)) void window_append_recur_kernel(const WindowArgs a, const RecurArgs r, uint32_t steps, uint32_t append_x)
+{
+    if (blockIdx.x < steps) {
+        recur_step<false, 64, true>(r, blockIdx.x / r.heads, blockIdx.x % r.heads);
+    } else {
+        const uint32_t i = blockIdx.x - steps;
+        window_append<false>(a, i % append_x, i / append_x);
     }
 }
 

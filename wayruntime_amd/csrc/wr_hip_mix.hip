@@ -677,13 +677,15 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
     return best(a, batch);
 }
 
-int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
+// A product's arguments, checked; `rows32`, `gated`: what goes out.
+static int gemm_args(int f32, const wr_hip_mix_gemm* q, MixGemmArgs& a, uint32_t& batch, bool& gated)
 {
-    if (!g.inited) return WR_HIP_ERR_STATE;
     if (!q || !q->w || !q->x || !q->rows) return WR_HIP_ERR_INVAL;
-    const uint32_t ktiles = q->w->n_in / 32, batch = q->group_expert ? 1 : q->w->batch;
+    const uint32_t ktiles = q->w->n_in / 32;
+    batch = q->group_expert ? 1 : q->w->batch;
     if ((uint64_t)q->x_kt0 + (uint64_t)q->x_kt_z * (batch - 1) + ktiles > q->x_kt) return WR_HIP_ERR_INVAL;
-    const bool split_gated = q->out == WR_HIP_MIX_OUT_SPLIT_GATED, gated = q->out == WR_HIP_MIX_OUT_GATED || split_gated;
+    const bool split_gated = q->out == WR_HIP_MIX_OUT_SPLIT_GATED;
+    gated = q->out == WR_HIP_MIX_OUT_GATED || split_gated;
     const bool frag = q->out == WR_HIP_MIX_OUT_FRAG || q->out == WR_HIP_MIX_OUT_SPLIT || gated;
     if (q->out > WR_HIP_MIX_OUT_SPLIT_GATED || (frag && !q->h)) return WR_HIP_ERR_INVAL;
     if (split_gated && (q->n_split % 32 || q->n_split > q->w->n_out || batch != 1 || q->group_expert)) return WR_HIP_ERR_INVAL;
@@ -704,9 +706,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     if (q->bias && (batch != 1 || q->out == WR_HIP_MIX_OUT_GATED || q->group_expert)) return WR_HIP_ERR_INVAL;
     if (q->x_scale && !q->group_expert) return WR_HIP_ERR_INVAL;
     if (q->x_perm && (!q->group_expert || q->tile_groups != 1)) return WR_HIP_ERR_INVAL;
-    ENTER();
-    cx->rows.store(q->rows, std::memory_order_relaxed);
-    MixGemmArgs a = {};
+    a = MixGemmArgs{};
     a.w = reinterpret_cast<const bf16x8*>(q->w->tiles);
     a.x = static_cast<const uint8_t*>(q->x) + (size_t)q->x_kt0 * 512 * (f32 ? 4 : 2);
     a.ntiles = q->w->n_out / 16;
@@ -736,6 +736,28 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     a.y = q->y_f32;
     a.ya = q->y_act;
     a.h = frag ? static_cast<uint8_t*>(q->h) + (size_t)q->h_kt0 * 512 * (f32 ? 4 : 2) : q->h;
+    return WR_HIP_OK;
+}
+
+// Up to sixteen rows, bfloat16: whether two tiles to a workgroup are the form, of eight waves over a short range or four with twice the k-steps each
+// over a long one, which share the rows' operand (16 rows; us, one tile / this: 2048 -> 14 400 16.8 / 11.4, -> 32 768
+// 32.7 / 21.6, 4096 -> 24 576 40.4 / 36.0, -> 6144 13.7 / 11.1; narrow ones 4096 -> 4096 8.4 / 7.8).
+static bool gemm_two_tiles(const MixGemmArgs& a, uint32_t batch, bool gated)
+{
+    return gated || a.ntiles * batch >= 384;
+}
+constexpr uint32_t kEightWaveKtiles = 64;
+
+int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
+{
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    MixGemmArgs a;
+    uint32_t batch;
+    bool gated;
+    const int rc = gemm_args(f32, q, a, batch, gated);
+    if (rc) return rc;
+    ENTER();
+    cx->rows.store(q->rows, std::memory_order_relaxed);
     if (q->group_expert) {
         if (!f32 && q->tile_groups == 8) {
             // Rows an expert has on average, from how many groups route leaves room for: a run per expert more than the
@@ -808,14 +830,39 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     if (a.groups == 1) {
         // a short input range: more outputs per workgroup, or the launch is all workgroups and no work
         if (!gated && a.ktiles <= 8 && a.ntiles % 4 == 0 && a.ntiles * batch >= 1024) return launch_split<false, 4, 1, 4, 2, true>(a, batch);
-        // wide weights share the rows' operand between two tiles; over a short range eight waves, over a long one
-        // four with twice the k-steps each (16 rows; us, before / now: 2048 -> 14 400 16.8 / 11.4, -> 32 768
-        // 32.7 / 21.6, 4096 -> 24 576 40.4 / 36.0, -> 6144 13.7 / 11.1; narrow ones 4096 -> 4096 8.4 / 7.8)
         if (!gated && batch == 1 && a.ktiles >= kPartsMinKtiles && a.ntiles * 2 <= g.n_cus) return launch_parts(a);
-        if (!gated && a.ntiles * batch < 384) return launch_split<false, 1, 1, 4, 8, true>(a, batch);
-        return a.ktiles <= 64 ? launch_split<false, 2, 1, 8, 4, true>(a, batch) : launch_split<false, 2, 1, 4, 8, true>(a, batch);
+        if (!gemm_two_tiles(a, batch, gated)) return launch_split<false, 1, 1, 4, 8, true>(a, batch);
+        return a.ktiles <= kEightWaveKtiles ? launch_split<false, 2, 1, 8, 4, true>(a, batch) : launch_split<false, 2, 1, 4, 8, true>(a, batch);
     }
     return launch_rows(a, batch, gated);
+}
+
+int wr_hip_mix_gemm_run_two(int f32, const wr_hip_mix_gemm* q, const wr_hip_mix_gemm* small)
+{
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    MixGemmArgs a, b;
+    uint32_t batch, batch_b;
+    bool gated, gated_b;
+    int rc = gemm_args(f32, q, a, batch, gated);
+    if (rc == WR_HIP_OK) rc = gemm_args(f32, small, b, batch_b, gated_b);
+    if (rc) return rc;
+    // One launch where the first is in tiles of two and not by the short range's rule (wr_hip_mix_gemm_run), and the second adds a sixteenth at most
+    const bool together = !f32 && !q->group_expert && !small->group_expert && a.groups == 1 && b.groups == 1 && batch_b == 1 &&
+                          gemm_two_tiles(a, batch, gated) && a.ktiles > 8 && (a.ktiles <= kEightWaveKtiles) == (b.ktiles <= kEightWaveKtiles) &&
+                          b.ntiles <= a.ntiles && (uint64_t)b.ntiles * 16 <= (uint64_t)a.ntiles * batch;
+    if (!together) {
+        rc = wr_hip_mix_gemm_run(f32, q);
+        return rc ? rc : wr_hip_mix_gemm_run(f32, small);
+    }
+    ENTER();
+    cx->rows.store(q->rows, std::memory_order_relaxed);
+    const dim3 grid((a.ntiles + 1) / 2 * batch + (b.ntiles + 1) / 2);
+    if (a.ktiles <= kEightWaveKtiles)
+        launch_main(mix_gemm_two_kernel<8, 4>, grid, dim3(512), a, b, 0);
+    else
+        launch_main(mix_gemm_two_kernel<4, 8>, grid, dim3(256), a, b, 0);
+    HIP_TRY(hipGetLastError(), "product launch", 0);
+    return WR_HIP_OK;
 }
 
 // -------------------------------------------------------------- lightning --
@@ -1060,9 +1107,8 @@ static int forget_run(wr_hip_mix_step* s, RecurArgs& a)
     return forget_steps_v<F32, 64>(a, n);
 }
 
-int wr_hip_mix_recur(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, int f32, const wr_hip_mix_recurrence* q)
+static int recur_args(const wr_hip_mix_step* s, const wr_hip_mix_pool* pool, uint32_t run, const wr_hip_mix_recurrence* q, RecurArgs& a)
 {
-    if (!g.inited) return WR_HIP_ERR_STATE;
     if (!s || !s->rows || !pool || run >= pool->state.size() || !q || !q->heads || !q->dim || !q->w0 || !q->norm || !q->in ||
         !q->h || q->rule > WR_HIP_MIX_RULE_FORGET)
         return WR_HIP_ERR_INVAL;
@@ -1077,8 +1123,7 @@ int wr_hip_mix_recur(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, in
         (delta && q->col_a + hd > q->ld) || q->col_h + (hv + 31) / 32 * 32 > (uint64_t)q->h_kt * 32)
         return WR_HIP_ERR_INVAL;
     if (!forget && (q->w_decay->batch != 1 || q->w_decay->n_out < hd)) return WR_HIP_ERR_INVAL;
-    ENTER();
-    RecurArgs a = {};
+    a = RecurArgs{};
     a.seqs = s->d<MixSeq>(s->o_seqs);
     a.chunks = s->d<MixChunk>(s->o_chunks);
     a.heads = q->heads;
@@ -1108,6 +1153,17 @@ int wr_hip_mix_recur(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, in
     a.h = q->h;
     a.h_kt = q->h_kt;
     a.col_h = q->col_h;
+    return WR_HIP_OK;
+}
+
+int wr_hip_mix_recur(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, int f32, const wr_hip_mix_recurrence* q)
+{
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    RecurArgs a;
+    const int rc = recur_args(s, pool, run, q, a);
+    if (rc) return rc;
+    const bool delta = q->rule == WR_HIP_MIX_RULE_DELTA, forget = q->rule == WR_HIP_MIX_RULE_FORGET;
+    ENTER();
     if (forget) return f32 ? forget_run<true>(s, a) : forget_run<false>(s, a);
     if (f32) return delta ? recur_run<true, true>(s, a, q) : recur_run<true, false>(s, a, q);
     return delta ? recur_run<false, true>(s, a, q) : recur_run<false, false>(s, a, q);
@@ -1397,20 +1453,18 @@ static WindowArgs window_args(const wr_hip_mix_step* s, const wr_hip_mix_pool* p
     return a;
 }
 
-int wr_hip_mix_window_append(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, int f32, const wr_hip_mix_window* q,
-                             const float* in_dev, uint32_t ld, uint32_t col_q, uint32_t col_k, uint32_t col_v,
-                             const float* table_dev, void* q_dev)
+// The append's arguments, checked.
+static int append_args(const wr_hip_mix_step* s, const wr_hip_mix_pool* pool, uint32_t run, int f32, const wr_hip_mix_window* q, const float* in_dev,
+                       uint32_t ld, uint32_t col_q, uint32_t col_k, uint32_t col_v, const float* table_dev, void* q_dev, WindowArgs& a, dim3& grid)
 {
-    if (!g.inited) return WR_HIP_ERR_STATE;
-    int rc = check_window(s, pool, run, f32, q);
+    const int rc = check_window(s, pool, run, f32, q);
     if (rc) return rc;
     const bool keys = col_k != WR_HIP_MIX_NO_KEYS;
     if (!in_dev || !q_dev || (q->rot_half && !table_dev) || (uint64_t)col_q + (uint64_t)q->heads * q->maps * q->dim > ld ||
         (keys && ((uint64_t)col_k + (uint64_t)q->kv_heads * q->maps * q->dim > ld ||
                   (uint64_t)col_v + (uint64_t)q->kv_heads * q->vdim > ld)))
         return WR_HIP_ERR_INVAL;
-    ENTER();
-    WindowArgs a = window_args(s, pool, run, q);
+    a = window_args(s, pool, run, q);
     a.in = in_dev;
     a.ld = ld;
     a.col_q = col_q;
@@ -1419,9 +1473,47 @@ int wr_hip_mix_window_append(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t
     a.table = table_dev;
     a.q = q_dev;
     a.key_heads = keys ? a.kvh : 0;
-    const dim3 grid((s->rows + 3) / 4, a.key_heads + (4 * a.heads * (a.dimk / 8) + kWindowQUnits - 1) / kWindowQUnits);
+    grid = dim3((s->rows + 3) / 4, a.key_heads + (4 * a.heads * (a.dimk / 8) + kWindowQUnits - 1) / kWindowQUnits);
+    return WR_HIP_OK;
+}
+
+int wr_hip_mix_window_append(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, int f32, const wr_hip_mix_window* q,
+                             const float* in_dev, uint32_t ld, uint32_t col_q, uint32_t col_k, uint32_t col_v,
+                             const float* table_dev, void* q_dev)
+{
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    WindowArgs a;
+    dim3 grid;
+    const int rc = append_args(s, pool, run, f32, q, in_dev, ld, col_q, col_k, col_v, table_dev, q_dev, a, grid);
+    if (rc) return rc;
+    ENTER();
     if (f32) MIX_LAUNCH(window_append_kernel<true>, grid, dim3(256), 0, a);
     else MIX_LAUNCH(window_append_kernel<false>, grid, dim3(256), 0, a);
+    return WR_HIP_OK;
+}
+
+int wr_hip_mix_window_append_recur(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, int f32, const wr_hip_mix_window* q,
+                                   const float* in_dev, uint32_t ld, uint32_t col_q, uint32_t col_k, uint32_t col_v,
+                                   const float* table_dev, void* q_dev, uint32_t recur_run, const wr_hip_mix_recurrence* recur)
+{
+    if (!g.inited) return WR_HIP_ERR_STATE;
+    WindowArgs a;
+    RecurArgs r;
+    dim3 grid;
+    int rc = append_args(s, pool, run, f32, q, in_dev, ld, col_q, col_k, col_v, table_dev, q_dev, a, grid);
+    if (rc == WR_HIP_OK) rc = recur_args(s, pool, recur_run, recur, r);
+    if (rc) return rc;
+    // One launch where the step's requests all take the recurrence token by token in workgroups of the append's size
+    // (recur_steps), the decays' product in passing (recur_run), and the append is no more than a few rows'
+    const uint64_t steps = (uint64_t)s->n_seq * r.heads, appends = (uint64_t)grid.x * grid.y;
+    if (f32 || recur->rule != WR_HIP_MIX_RULE_DELTA || s->n_long || r.low_kt > kDecayTiles || r.dim <= 32 || r.dim > 64 || steps + appends > 1u << 20) {
+        rc = wr_hip_mix_window_append(s, pool, run, f32, q, in_dev, ld, col_q, col_k, col_v, table_dev, q_dev);
+        return rc ? rc : wr_hip_mix_recur(s, pool, recur_run, f32, recur);
+    }
+    ENTER();
+    r.wd = reinterpret_cast<const bf16x8*>(recur->w_decay->tiles);
+    r.low = recur->low;
+    MIX_LAUNCH(window_append_recur_kernel, dim3((uint32_t)(steps + appends)), dim3(256), 0, a, r, (uint32_t)steps, grid.x);
     return WR_HIP_OK;
 }
 

@@ -445,11 +445,9 @@ static wr_status walk_latent(wr_model *m, const wrh_mix_layer *L, uint32_t r, co
     return WR_OK;
 }
 
-/* The recurrence, the decay's second product included; `rec` has the rest filled in. */
-static wr_status walk_recur(wr_model *m, const wrh_mix_recur *q, uint32_t r, uint32_t store, const void *low, float *z,
-                            wr_hip_mix_recurrence *rec)
+/* What both recurrences with a decay's second product take besides their own. */
+static void fill_recur(const struct wrh_mix_model *mm, const wrh_mix_recur *q, const void *low, float *z, wr_hip_mix_recurrence *rec)
 {
-    struct wrh_mix_model *mm = m->mix;
     rec->heads = q->heads;
     rec->dim = q->dim;
     rec->eps = mm->eps;
@@ -458,8 +456,6 @@ static wr_status walk_recur(wr_model *m, const wrh_mix_recur *q, uint32_t r, uin
     rec->w_decay = q->w_decay;
     rec->low = low;
     rec->z = z;
-    TRY(wr_hip_mix_recur(mm->step, mm->pool, store, mm->f32, rec), "matrix-state recurrence");
-    return WR_OK;
 }
 
 /* Takes the residual from w->x and the sublayer output `y` waiting to join it (or NULL) to w->x_next. */
@@ -478,14 +474,13 @@ static wr_status walk_wkv(wr_model *m, const wrh_mix_layer *L, uint32_t r, walk 
     }
     const wr_hip_mix_gemm in = {.w = L->w_rkvg, .x = t.mix, .x_kt = 5 * wkt, .x_kt_z = wkt, .rows = R,
                                 .out = WR_HIP_MIX_OUT_ROWS_F32, .y_f32 = t.in, .ldy = 4 * hd, .col_z = hd};
-    TRY(wr_hip_mix_gemm_run(mm->f32, &in), "r/k/v/gate projection");
     const wr_hip_mix_gemm low = {.w = L->w_low, .x = t.mix, .x_kt = 5 * wkt, .x_kt0 = 4 * wkt, .rows = R, .out = WR_HIP_MIX_OUT_FRAG,
                                  .h = t.low, .h_kt = q->rank_p / 32, .tanh_end = q->rank_p};
-    TRY(wr_hip_mix_gemm_run(mm->f32, &low), "decay's low-rank product");
+    TRY(wr_hip_mix_gemm_run_two(mm->f32, &in, &low), "r/k/v/gate projection and decay's low-rank product");
     wr_hip_mix_recurrence rec = {.rule = WR_HIP_MIX_RULE_BONUS, .out_scale = 1.0f, .gate_silu = 1, .u = q->u, .in = t.in,
                                  .ld = 4 * hd, .col_k = hd, .col_v = 2 * hd, .col_g = 3 * hd, .h = t.oh, .h_kt = hd / 32};
-    const wr_status st = walk_recur(m, q, r, mm->runs[r].store, t.low, t.z, &rec);
-    if (st != WR_OK) return st;
+    fill_recur(mm, q, t.low, t.z, &rec);
+    TRY(wr_hip_mix_recur(mm->step, mm->pool, mm->runs[r].store, mm->f32, &rec), "matrix-state recurrence");
     const wr_hip_mix_gemm out = {.w = L->w_o, .x = t.oh, .x_kt = hd / 32, .rows = R, .out = WR_HIP_MIX_OUT_ROWS_F32,
                                  .y_f32 = w->y, .ldy = mm->width_p};
     TRY(wr_hip_mix_gemm_run(mm->f32, &out), "output projection");
@@ -502,16 +497,15 @@ static wr_status walk_parallel(wr_model *m, const wrh_mix_layer *L, uint32_t r, 
                                 .h = t.low, .h_kt = q->rank_p / 32, .n_split = q->rank_p, .tanh_end = q->rank_p,
                                 .y_f32 = t.in, .ldy = L->ld_in};
     TRY(wr_hip_mix_gemm_run(mm->f32, &in), "both halves' projections");
-    TRY(wr_hip_mix_window_append(mm->step, mm->pool, store, mm->f32, &L->win, t.in, L->ld_in, L->col_q, L->col_k, L->col_v,
-                                 w->rope[L->rope], t.q), "rotation + cache append");
-    TRY(wr_hip_mix_window_attend(mm->step, mm->pool, store, mm->f32, &L->win, t.q, L->sink, NULL, 0, t.oh, kt_o),
-        "windowed attention");
     wr_hip_mix_recurrence rec = {.rule = WR_HIP_MIX_RULE_DELTA, .gain = WRH_DELTA_GAIN, .unit_eps = WRH_DELTA_UNIT_EPS,
                                  .out_scale = L->right_scale, .a_bias = q->a_bias, .in = t.in, .ld = L->ld_in,
                                  .col_r = L->col_rr, .col_k = L->col_rk, .col_v = L->col_rv, .col_a = L->col_ra,
                                  .col_g = L->col_rg, .h = t.oh, .h_kt = kt_o, .col_h = L->heads * L->win.vdim_pad};
-    const wr_status st = walk_recur(m, q, r, mm->runs[r].store2, t.low, t.z, &rec);
-    if (st != WR_OK) return st;
+    fill_recur(mm, q, t.low, t.z, &rec);
+    TRY(wr_hip_mix_window_append_recur(mm->step, mm->pool, store, mm->f32, &L->win, t.in, L->ld_in, L->col_q, L->col_k, L->col_v,
+                                       w->rope[L->rope], t.q, mm->runs[r].store2, &rec), "rotation + cache append, matrix-state recurrence");
+    TRY(wr_hip_mix_window_attend(mm->step, mm->pool, store, mm->f32, &L->win, t.q, L->sink, NULL, 0, t.oh, kt_o),
+        "windowed attention");
     const wr_hip_mix_gemm out = {.w = L->w_o, .x = t.oh, .x_kt = kt_o, .rows = R, .out = WR_HIP_MIX_OUT_ROWS_F32,
                                  .y_f32 = w->y, .ldy = mm->width_p};
     TRY(wr_hip_mix_gemm_run(mm->f32, &out), "output projection");
