@@ -196,6 +196,22 @@ def test_batch_of_matrices(lib, f32, batch, N, K, rows):
         b.free()
 
 
+# whose tiles an XCD takes side by side: launches of fewer workgroups than XCDs, of a few more, of many and a rest; one tile to
+# a workgroup, two, two workgroups to a tile, batches
+@pytest.mark.parametrize("batch,N,K,rows", [(1, 16, 1024, 1), (1, 144, 1024, 16), (1, 6160, 1024, 9), (1, 14416, 2048, 16), (1, 48, 4096, 3), (1, 1104, 4096, 2),
+                                            (3, 2064, 1024, 5)])
+def test_tiles_by_region(lib, batch, N, K, rows):
+    r = Run(lib, False, batch, N, K, rows)
+    x = r.act(rows, batch * K)
+    xd, y = r.up(x), hipattn.DeviceBuffer(rows * batch * N * 4)
+    r.go(xd, x_kt=batch * K // 32, x_kt_z=K // 32, out=ROWS_F32, y_f32=y.p, ldy=batch * N, col_z=N)
+    want = np.stack([x.reshape(rows, batch, K)[:, z].astype(np.float64) @ r.w[z].T.astype(np.float64) for z in range(batch)], 1)
+    r.close(y.to_host((rows, batch * N)), want.reshape(rows, -1))
+    r.end()
+    for b in (xd, y):
+        b.free()
+
+
 # (batch, outputs, small one's outputs and inputs, rows): one launch where both are of sixteen rows at most and the second is small; else two
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("batch,N,K,n,k,rows", [(4, 1536, 288, 64, 288, 16), (1, 6144, 512, 16, 96, 1), (3, 2064, 1056, 48, 2048, 7), (2, 3088, 2080, 32, 4128, 5),

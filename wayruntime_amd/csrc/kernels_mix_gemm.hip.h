@@ -29,7 +29,8 @@ struct MixGemmArgs {
     float scale, limit, slope, up_bias;
     const float* bias;
     uint32_t cols;                   // mix_gemm_lds_kernel without experts: XCDs that share out the outputs (xcd_tile);
-                                     // a stream of experts: runs that the XCDs share out, or 0
+                                     // a stream of experts: runs that the XCDs share out, or 0; up to sixteen rows of others:
+                                     // whether an XCD's workgroups take neighbouring tiles (xcd_region)
     const uint32_t* x_perm;
     const float* x_scale;            // a factor per row of the input (applied to its products), or nullptr
     float* y;
@@ -378,7 +379,11 @@ __device__ __forceinline__ void mix_gemm_split(const MixGemmArgs& a, uint32_t bx
 template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS = 1, bool PICKED = false>
 __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_kernel(const MixGemmArgs a)
 {
-    mix_gemm_split<F32, NT, GR, WAVES, DEPTH, STREAM, PARTS, PICKED>(a, blockIdx.x, blockIdx.y, blockIdx.z);
+    uint32_t bx = blockIdx.x;
+    if constexpr (STREAM && GR == 1 && !PICKED) {
+        if (a.cols) bx = xcd_region(bx, gridDim.x);
+    }
+    mix_gemm_split<F32, NT, GR, WAVES, DEPTH, STREAM, PARTS, PICKED>(a, bx, blockIdx.y, blockIdx.z);
 }
 
 // Two products of up to sixteen rows that do not wait for each other: a's batch of matrices, and a small one whose few tiles took a launch
@@ -388,10 +393,11 @@ template <int WAVES, int DEPTH>
 __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_two_kernel(const MixGemmArgs a, const MixGemmArgs b)
 {
     const uint32_t of_b = (b.ntiles + 1) / 2, of_a = (a.ntiles + 1) / 2;
-    if (blockIdx.x < of_b) {
-        mix_gemm_split<false, 2, 1, WAVES, DEPTH, true, 1, false>(b, blockIdx.x, 0, 0);
+    const uint32_t item = a.cols ? xcd_region(blockIdx.x, gridDim.x) : blockIdx.x;
+    if (item < of_b) {
+        mix_gemm_split<false, 2, 1, WAVES, DEPTH, true, 1, false>(b, item, 0, 0);
     } else {
-        const uint32_t i = blockIdx.x - of_b;
+        const uint32_t i = item - of_b;
         mix_gemm_split<false, 2, 1, WAVES, DEPTH, true, 1, false>(a, i % of_a, 0, i / of_a);
     }
 }

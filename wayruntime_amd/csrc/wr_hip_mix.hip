@@ -748,6 +748,11 @@ static bool gemm_two_tiles(const MixGemmArgs& a, uint32_t batch, bool gated)
 }
 constexpr uint32_t kEightWaveKtiles = 64;
 
+// Up to sixteen rows: whether an XCD's workgroups take neighbouring tiles: where tiles are a multiple of 32 KiB (us, dealt out / so: 2048 -> 16 384
+// gated 13.3 / 12.7, 8192 -> 2048 10.3 / 9.5, 4096 -> 24 576 37.6 / 33.4, four of 2048 -> 2048 8.2 / 7.9; level for weights
+// of 8 MB; others lose a little, 1536 -> 12 288 9.7 / 9.9).
+static uint32_t gemm_regions(const MixGemmArgs& a) { return a.ktiles % 32 == 0; }
+
 int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
 {
     if (!g.inited) return WR_HIP_ERR_STATE;
@@ -828,6 +833,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
         return launch_split<true, 2, 2, 4, 4, false>(a, batch);
     }
     if (a.groups == 1) {
+        a.cols = gemm_regions(a);
         // a short input range: more outputs per workgroup, or the launch is all workgroups and no work
         if (!gated && a.ktiles <= 8 && a.ntiles % 4 == 0 && a.ntiles * batch >= 1024) return launch_split<false, 4, 1, 4, 2, true>(a, batch);
         if (!gated && batch == 1 && a.ktiles >= kPartsMinKtiles && a.ntiles * 2 <= g.n_cus) return launch_parts(a);
@@ -856,6 +862,7 @@ int wr_hip_mix_gemm_run_two(int f32, const wr_hip_mix_gemm* q, const wr_hip_mix_
     }
     ENTER();
     cx->rows.store(q->rows, std::memory_order_relaxed);
+    a.cols = gemm_regions(a);
     const dim3 grid((a.ntiles + 1) / 2 * batch + (b.ntiles + 1) / 2);
     if (a.ktiles <= kEightWaveKtiles)
         launch_main(mix_gemm_two_kernel<8, 4>, grid, dim3(512), a, b, 0);
