@@ -821,6 +821,60 @@ def test_append_decode_from_host_rows_refuses_what_it_must():
     kv.close(); other.close()
 
 
+def _write_through(call, kv, layer, pos, rows):
+    """Rows into the cache at pos ..., by one of the calls that append; the bits of both sides."""
+    lib, nkv, hd, n = hipattn.lib(), kv.nkv, kv.hd[layer], rows.shape[0]
+    if call == "append":
+        assert kv.append(layer, pos, rows, rows) == hipattn.OK
+    elif call == "write_f16":
+        kv.write_f16(layer, pos, synth.f32_to_f16_trunc(rows), synth.f32_to_f16_trunc(rows))
+    elif call == "append_decode":
+        for i in range(n):
+            kv.append_decode(layer, pos + i, rows[i], rows[i], rows[i])
+    else:
+        dev = hipattn.DeviceBuffer.from_host(rows)
+        wide = hipattn.DeviceBuffer.from_host(np.concatenate([rows] * 3, axis=1).copy())      # Q, K and V heads of each row
+        q, h = hipattn.DeviceBuffer(rows.nbytes), (C.c_void_p * 1)(kv.h)
+        if call == "append_batched_dev":
+            for i in range(n):
+                at = C.c_void_p(dev.p + i * nkv * hd * 4)
+                assert lib.wr_hip_attn_append_batched_dev(1, h, layer, (C.c_uint32 * 1)(pos + i), at, at) == hipattn.OK
+        else:
+            assert lib.wr_hip_rows_qkv_append_dev(wide.p, 3 * nkv * hd, n, nkv, None, None, 1e-6, None, 0, 1, h, layer,
+                                                  (C.c_uint32 * 1)(pos), q.p, 0) == hipattn.OK
+        hipattn.sync()
+        for b in (dev, wide, q):
+            b.free()
+
+
+@pytest.mark.parametrize("call", ["append", "write_f16", "append_decode", "append_batched_dev", "qkv_append"])
+@pytest.mark.parametrize("pos,n", [(0, 1), (31, 2), (63, 1), (64, 1), (400, 33)])
+def test_memory_of_a_short_cache_comes_back_cleared(call, pos, n):
+    # Caches of one size in bytes and different layers, heads and widths follow each other: each finds zeros wherever it looks,
+    # and only the first positions of the one before it were written.
+    for hds, nkv in [([128, 128], 4), ([128, 0, 128], 4), ([256], 4), ([128], 8), ([128] * 4, 2)]:
+        kv = hipattn.KVCache(len(hds), hds, nkv, 1024)
+        assert kv.bytes == 4 << 20
+        for layer in range(len(hds)):
+            if hds[layer]:
+                k, v = kv.read_f16(layer, 0, 1024)
+                assert not k.any() and not v.any(), (hds, nkv, layer)
+        if call != "append_decode" or hds[0] == 128:
+            rows = synth.normal(7, (n, nkv, hds[0]))
+            _write_through(call, kv, 0 if n > 1 else len(hds) - 1, pos, rows)
+            k, _ = kv.read_f16(0 if n > 1 else len(hds) - 1, pos, n)
+            assert k.any()
+        kv.close()
+    for hd in (20, 7):                                       # heads of no whole 16 bytes, which K pads and V does not
+        for again in range(2):
+            kv = hipattn.KVCache(1, hd, 3, 1024)
+            k, v = kv.read_f16(0, 0, 1024)
+            assert not k.any() and not v.any(), (hd, again)
+            rows = synth.normal(8, (n, 3, hd))
+            assert kv.append(0, pos, rows, rows) == hipattn.OK
+            kv.close()
+
+
 def test_memory_of_ended_caches_is_bounded_and_comes_back_cleared():
     def free_bytes():                                        # of the runtime that the library is linked with
         free, total = C.c_size_t(), C.c_size_t()

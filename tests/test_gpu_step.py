@@ -89,6 +89,35 @@ def test_tags_begin_again():
         b.free()
 
 
+def test_memory_that_steps_wrote_comes_back_cleared():
+    """A step writes its K and V by itself, in every layer: the next cache of that size finds zeros there too."""
+    hipattn.init()
+    lib, rng = hipattn.lib(), np.random.default_rng(9)
+    n, hidden, ctx = 2, 512, 1000
+    w = [[hipattn.Weight([(rng.standard_normal((o, 512)) / 16).astype(np.float16).view(np.uint16)]) for o in (1024, 512, 1024, 512)]
+         for _ in range(n)]
+    vec = hipattn.DeviceBuffer.from_host(rng.standard_normal(hidden).astype(np.float32))
+    layers = (hipattn.StepLayer * n)(*[hipattn.StepLayer(*[x.h for x in ws], vec.p, vec.p, None, None) for ws in w])
+    plan = C.c_void_p()
+    assert lib.wr_hip_attn_step_create(n, layers, 4, 2, 128, 1e-6, C.byref(plan)) == hipattn.OK
+    row = hipattn.DeviceBuffer.from_host(rng.standard_normal(hidden).astype(np.float32))
+    for pos in (0, 31, 32, 300, 7):
+        kv = hipattn.KVCache(n, 128, 2, ctx)
+        for layer in range(n):
+            assert not any(x.any() for x in kv.read_f16(layer, 0, ctx)), pos
+        assert lib.wr_hip_attn_step_dev(plan, kv.h, pos, row.p, None, 0, 0.0) == hipattn.OK
+        assert lib.wr_hip_attn_step_done() == hipattn.OK
+        for layer in range(n):
+            assert all(x.any() for x in kv.read_f16(layer, pos, 1))
+        kv.close()
+    lib.wr_hip_attn_step_destroy(plan)
+    for ws in w:
+        for x in ws:
+            x.close()
+    for b in (vec, row):
+        b.free()
+
+
 @pytest.fixture(scope="module")
 def eng():
     hipattn.shutdown()

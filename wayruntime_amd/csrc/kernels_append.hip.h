@@ -9,6 +9,7 @@
 #pragma once
 
 #include "common.hip.h"
+#include "runtime.hip.h"
 
 namespace wr {
 
@@ -308,6 +309,19 @@ __global__ __launch_bounds__(256) void export_kv_kernel(const uint16_t* __restri
     const uint32_t r = (uint32_t)(idx / ((size_t)hd * nkv));
     k_out[idx] = k[k_offset(kvh, ctx_pad, pos + r, d, hd)];
     v_out[idx] = vt[vt_offset(kvh, ctx_pad, pos + r, d, hd)];
+}
+
+// The first a.tiles runs of 32 positions of every layer's and head's K and Vt back to zeros.
+// grid (any number, 2 nkv, layers).  Bound by HBM's write rate where there is much to clear.
+__global__ __launch_bounds__(256) void clear_cache_kernel(const ClearArgs a, uint8_t* slab)
+{
+    const uint32_t layer = blockIdx.z, hd = a.hd[layer], head = blockIdx.y % a.nkv;
+    if (hd == 0) return;
+    const bool v = blockIdx.y >= a.nkv;
+    const uint32_t width = v ? hd : k_padded_hd(hd);       // (of 32 positions a multiple of 64 bytes)
+    u32x4* at = reinterpret_cast<u32x4*>(slab + (v ? a.vt_off[layer] : a.k_off[layer]) + (size_t)head * a.ctx_pad * width * 2);
+    const size_t units = (size_t)a.tiles * kKTile * width / 8;
+    for (size_t i = blockIdx.x * 256 + threadIdx.x; i < units; i += (size_t)gridDim.x * 256) at[i] = u32x4{0, 0, 0, 0};
 }
 
 }  // namespace wr

@@ -57,6 +57,13 @@ struct Ctx {
     bool profiling = false;
 };
 
+// Where a cache has been written (clear_cache_kernel).
+struct ClearArgs {
+    uint32_t nkv, ctx_pad, tiles;        // tiles: runs of 32 positions, from the first on
+    uint32_t hd[WR_HIP_MAX_LAYERS];      // 0: no cache
+    uint64_t k_off[WR_HIP_MAX_LAYERS], vt_off[WR_HIP_MAX_LAYERS];
+};
+
 struct Lib {
     std::mutex mu;               // init / shutdown, the set of thread contexts, the knobs
     std::atomic<bool> inited{false};   // read without the lock by every entry point
@@ -67,9 +74,11 @@ struct Lib {
     struct Slab {
         uint8_t* p;
         size_t bytes;
+        uint32_t n_layers;
+        ClearArgs cleared;       // where its last cache has written
     };
     std::mutex slab_mu;          // guards slabs; nothing else is locked while it is held
-    std::vector<Slab> slabs;     // memory of ended caches, cleared when it is taken again
+    std::vector<Slab> slabs;     // memory of ended caches; what they wrote is cleared when it is taken again
     std::vector<Ctx*> idle;      // contexts whose thread has ended, for the next new thread
     char name[320] = "uninitialised";
     unsigned char* noalloc_ws[kMaxDevices] = {};   // device address of `scratch`, per device
