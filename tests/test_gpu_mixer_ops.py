@@ -678,6 +678,50 @@ class StepOf:
         self.lib.wr_hip_mix_pool_destroy(self.pool)
 
 
+class Router(C.Structure):
+    _fields_ = [("experts", u32), ("identity", u32), ("top", u32), ("groups", u32), ("keep", u32), ("softmax_all", u32), ("shared_gate", u32),
+                ("scale", C.c_float), ("correction", vp), ("logistic", u32)]
+
+
+# The choice with the order up to 32 rows and before it beyond; pairs of whole turns of eight thousand, two less, one more, and of two turns and a rest; outputs a lane
+# holds one, four and sixteen of; identity outputs; runs of one group and of eight.
+@pytest.mark.parametrize("experts,identity,top,rows,run", [(64, 0, 6, 1, 1), (64, 0, 6, 32, 1), (64, 0, 6, 33, 1), (64, 0, 6, 64, 8), (60, 4, 2, 4095, 8),
+                                                           (60, 0, 2, 4096, 8), (64, 0, 3, 2731, 8), (64, 0, 6, 2800, 8), (120, 8, 5, 40, 1), (300, 12, 9, 32, 2),
+                                                           (300, 12, 9, 33, 2), (1000, 24, 64, 257, 1)])
+def test_routes(lib, experts, identity, top, rows, run):
+    lib.wr_hip_mix_route.argtypes = [vp, vp, u32, C.POINTER(Router), u32, vp, vp, vp, vp, vp, vp]
+    lib.wr_hip_mix_route_groups.restype = u32
+    outputs, rng = experts + identity, np.random.default_rng(rows)
+    z = rng.standard_normal((rows, outputs), dtype=np.float32)
+    groups = lib.wr_hip_mix_route_groups(rows, experts, top, run)
+    s, zd = StepOf(lib, [0] * rows, 1), hipattn.DeviceBuffer.from_host(z)
+    gate, side, weight, slot, perm, owner = [hipattn.DeviceBuffer.from_host(np.full(n, 7.0, np.float32))
+                                             for n in (rows * top, rows * 2, groups * 16, rows * top, groups * 16, groups)]
+    q = Router(experts=experts, identity=identity, top=top)
+    for weighed in (weight.p, None):
+        assert lib.wr_hip_mix_route(s.h, zd.p, outputs, C.byref(q), run, gate.p, side.p, weighed, slot.p, perm.p, owner.p) == 0
+        hipattn.sync()
+        g, at = gate.to_host((rows, top)), slot.to_host((rows, top)).view(np.uint32)
+        row, expert = perm.to_host((groups * 16,)).view(np.uint32), owner.to_host((groups,)).view(np.int32)
+        best = np.argsort(-z, axis=1, kind="stable")[:, :top]
+        chosen = np.take_along_axis(z, best, axis=1).astype(np.float64)
+        e = np.exp(chosen - chosen[:, :1])
+        # differences of logits below 10 round by 2^-21; exp, the sum in turn and the quotient by a few 2^-24 each
+        assert np.abs(g / (e / e.sum(axis=1, keepdims=True)) - 1).max() <= 2.0 ** -20 + (top + 8) * 2.0 ** -24
+        real = best < experts
+        assert (at[~real] == 0xFFFFFFFF).all() and len(set(at[real].tolist())) == real.sum()
+        assert np.array_equal(row[at[real]], np.nonzero(real)[0]) and np.array_equal(expert[at[real] // 16], best[real])
+        empty = np.ones(groups * 16, bool)
+        empty[at[real]] = False
+        assert (row[empty] == 0xFFFFFFFF).all() and (expert[empty.reshape(-1, 16).all(axis=1)] == -1).all()
+        if weighed:
+            w = weight.to_host((groups * 16,))
+            assert np.array_equal(w[at[real]], g[real]) and not w[empty].any()
+    s.end()
+    for b in (zd, gate, side, weight, slot, perm, owner):
+        b.free()
+
+
 # One row to a workgroup up to 599 rows (1791 with experts' rows) and wherever no fragment is written, four beyond; features
 # that a workgroup holds in registers (4096) and more.
 @pytest.mark.parametrize("f32", [False, True])

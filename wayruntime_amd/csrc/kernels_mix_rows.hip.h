@@ -698,7 +698,12 @@ __global__ __launch_bounds__(256) void mix_top_kernel(const MixRouteArgs a)
     if (row < a.rows) mix_top<PER>(a, row, threadIdx.x & 63, [&](uint32_t t, uint32_t e) { a.slot[(size_t)row * a.top + t] = e; });
 }
 
-constexpr uint32_t kOrderRows = 64, kOrderPairs = kOrderRows * 64;      // of a step whose choice is made with the order
+// Of a step whose choice is made with the order: a wave takes 2.4 us to a row and sixteen run side by side, and a launch of its own for the
+// choice 5 us and its gap (64 outputs, top 6: 16 rows 5.2 us in one launch and 10.6 in two, 32 7.6 and 10.6, 48 11.9 and 10.6, 64 14.7 and 10.6).
+constexpr uint32_t kOrderRows = 32, kOrderPairs = kOrderRows * 64;
+// Pairs a thread asks for at once: the launch is one workgroup, bound by what a pair waits for and by the scattered stores (1500 rows of
+// top 6 one by one 11.0 us, so 9.7; 4096 rows 27.0 and 21.6).
+constexpr uint32_t kOrderAhead = 8;
 
 // One workgroup: orders the chosen (row, expert) pairs by expert.  Each expert's
 // pairs take whole runs of tile_groups groups of 16 slots.  Which slot of its
@@ -727,8 +732,14 @@ __global__ __launch_bounds__(1024) void mix_order_kernel(const MixRouteArgs a)
                 if (e < a.experts) atomicAdd(&count[e], 1u);
             });
     } else {
-        for (uint32_t i = t; i < pairs; i += 1024)
-            if (a.slot[i] < a.experts) atomicAdd(&count[a.slot[i]], 1u);
+        for (uint32_t i0 = t; i0 < pairs; i0 += 1024 * kOrderAhead) {
+            uint32_t e[kOrderAhead];
+#pragma unroll
+            for (uint32_t k = 0; k < kOrderAhead; k++) e[k] = a.slot[min(i0 + 1024 * k, pairs - 1)];
+#pragma unroll
+            for (uint32_t k = 0; k < kOrderAhead; k++)
+                if (i0 + 1024 * k < pairs && e[k] < a.experts) atomicAdd(&count[e[k]], 1u);
+        }
     }
     __syncthreads();
     const uint32_t mine = (count[t] + run - 1) / run * run;
@@ -744,18 +755,29 @@ __global__ __launch_bounds__(1024) void mix_order_kernel(const MixRouteArgs a)
     for (uint32_t g = 0; g < (count[t] + 15) / 16; g++) a.group_expert[(upto - mine) / 16 + g] = (int32_t)t;   // (a run's empty groups stay -1)
     count[t] = upto - mine;                                // from here on: the expert's next slot
     __syncthreads();
-    for (uint32_t i = t; i < pairs; i += 1024) {
-        uint32_t e;
-        if constexpr (TOP) e = pick[i];
-        else e = a.slot[i];
-        if (e >= a.experts) {                              // the input itself: nothing to compute
-            a.slot[i] = 0xFFFFFFFFu;
-            continue;
+    for (uint32_t i0 = t; i0 < pairs; i0 += 1024 * kOrderAhead) {
+        uint32_t e[kOrderAhead];
+        float w[kOrderAhead];
+#pragma unroll
+        for (uint32_t k = 0; k < kOrderAhead; k++) {
+            const uint32_t i = min(i0 + 1024 * k, pairs - 1);
+            if constexpr (TOP) e[k] = pick[i];
+            else e[k] = a.slot[i];
+            w[k] = a.slot_weight ? a.gate[i] : 0.f;        // (made here: ahead of two barriers)
         }
-        const uint32_t s = atomicAdd(&count[e], 1u);
-        a.slot[i] = s;
-        a.perm[s] = i / a.top;
-        if (a.slot_weight) a.slot_weight[s] = a.gate[i];   // (made here: ahead of two barriers)
+#pragma unroll
+        for (uint32_t k = 0; k < kOrderAhead; k++) {
+            const uint32_t i = i0 + 1024 * k;
+            if (i >= pairs) break;
+            if (e[k] >= a.experts) {                       // the input itself: nothing to compute
+                a.slot[i] = 0xFFFFFFFFu;
+                continue;
+            }
+            const uint32_t s = atomicAdd(&count[e[k]], 1u);
+            a.slot[i] = s;
+            a.perm[s] = i / a.top;
+            if (a.slot_weight) a.slot_weight[s] = w[k];
+        }
     }
 }
 
