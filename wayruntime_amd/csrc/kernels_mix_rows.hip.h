@@ -755,18 +755,19 @@ __global__ __launch_bounds__(1024) void mix_order_kernel(const MixRouteArgs a)
     for (uint32_t g = 0; g < (count[t] + 15) / 16; g++) a.group_expert[(upto - mine) / 16 + g] = (int32_t)t;   // (a run's empty groups stay -1)
     count[t] = upto - mine;                                // from here on: the expert's next slot
     __syncthreads();
-    for (uint32_t i0 = t; i0 < pairs; i0 += 1024 * kOrderAhead) {
-        uint32_t e[kOrderAhead];
-        float w[kOrderAhead];
+    constexpr uint32_t AHEAD = TOP ? 1 : kOrderAhead;      // (few pairs: a thread's first is its only one)
+    for (uint32_t i0 = t; i0 < pairs; i0 += 1024 * AHEAD) {
+        uint32_t e[AHEAD];
+        float w[AHEAD];
 #pragma unroll
-        for (uint32_t k = 0; k < kOrderAhead; k++) {
+        for (uint32_t k = 0; k < AHEAD; k++) {
             const uint32_t i = min(i0 + 1024 * k, pairs - 1);
             if constexpr (TOP) e[k] = pick[i];
             else e[k] = a.slot[i];
             w[k] = a.slot_weight ? a.gate[i] : 0.f;        // (made here: ahead of two barriers)
         }
 #pragma unroll
-        for (uint32_t k = 0; k < kOrderAhead; k++) {
+        for (uint32_t k = 0; k < AHEAD; k++) {
             const uint32_t i = i0 + 1024 * k;
             if (i >= pairs) break;
             if (e[k] >= a.experts) {                       // the input itself: nothing to compute
