@@ -304,6 +304,16 @@ def test_rope_table_on_device_is_the_oracles_bytes(hd, theta, rot_pairs):
     assert np.array_equal(got.view(np.uint32), want[31000:31077].view(np.uint32))
 
 
+@pytest.mark.parametrize("hd,theta", [(64, 1e4), (128, 1e6), (128, 1.0)])
+def test_rope_table_around_powers_of_two(hd, theta):
+    # angles on either side of every edge that turns are counted between, up to the last position
+    positions = sorted({min(max(2 ** k + d, 0), 131071) for k in range(3, 18) for d in (-7, -6, -1, 0, 1, 6, 7)})
+    for i in range(0, len(positions), 16):
+        some = positions[i:i + 16]
+        want = np.concatenate([oracle.rope_table(1, hd, p, theta, 0) for p in some])
+        assert hipattn.rope_table_dev(len(some), hd, theta, pos=some).tobytes() == want.tobytes(), some
+
+
 def test_rope_table_on_device_listed_positions():
     positions = [0, 32767, 5, 4096, 4095, 1, 77, 20000, 31, 32, 33, 9999, 16384, 2, 3, 12345]
     for n in (1, 7, 16):

@@ -1674,10 +1674,10 @@ int wr_hip_attn_rope_table_dev(float* cos_sin_dev, uint32_t rows, uint32_t pos0,
     if (!cos_sin_dev || rows == 0) return WR_HIP_ERR_INVAL;
     if (hd < 2 || (hd & 1)) return WR_HIP_ERR_INVAL;
     if (pos && rows > WR_HIP_BATCH_MAX) return WR_HIP_ERR_INVAL;
-    // The kernel folds an angle into [-pi, pi] by subtracting 2 pi in a loop, as
+    // The kernel folds an angle into [-pi, pi] by subtracting 2 pi turn by turn, as
     // the reference does (src/core/mathx.c:112-147); from an angle of 2^27 on a
     // float's spacing exceeds 2 pi, the subtraction rounds back to itself and the
-    // loop never ends.  The reference's callers stay below WR_ATTN_MAX_SEQ: the
+    // turns never end.  The reference's callers stay below WR_ATTN_MAX_SEQ: the
     // same bound here, before anything is launched.
     if (!pos && (uint64_t)pos0 + rows > WR_HIP_ATTN_MAX_SEQ) return WR_HIP_ERR_LIMIT;
     for (uint32_t i = 0; pos && i < rows; i++)
