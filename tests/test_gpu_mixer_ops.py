@@ -722,6 +722,126 @@ def test_routes(lib, experts, identity, top, rows, run):
         b.free()
 
 
+class Recurrence(C.Structure):
+    _fields_ = [("heads", u32), ("dim", u32), ("rule", u32), ("gain", C.c_float), ("unit_eps", C.c_float), ("eps", C.c_float),
+                ("out_scale", C.c_float), ("gate_silu", u32), ("w0", vp), ("u", vp), ("a_bias", vp), ("norm", vp), ("in_", vp),
+                ("ld", u32), ("col_r", u32), ("col_k", u32), ("col_v", u32), ("col_a", u32), ("col_g", u32), ("w_decay", vp),
+                ("low", vp), ("z", vp), ("h", vp), ("h_kt", u32), ("col_h", u32), ("vdim", u32), ("lower", vp)]
+
+
+class Window(C.Structure):
+    _fields_ = [("heads", u32), ("kv_heads", u32), ("dim", u32), ("dim_pad", u32), ("vdim", u32), ("vdim_pad", u32), ("rot_half", u32),
+                ("window", u32), ("scale", C.c_float), ("out_scale", C.c_float), ("norm_values", u32), ("eps", C.c_float), ("maps", u32),
+                ("neighbours", u32), ("softcap", C.c_float), ("diff", C.c_float), ("q_norm", vp), ("k_norm", vp), ("chunk", u32),
+                ("gate_wide", u32), ("turn_values", vp)]
+
+
+BONUS, DELTA, FORGET = range(3)
+
+
+class Recur:
+    """A recurrence (and, with `win`, a windowed layer beside it) over steps of requests that bring `rows` rows each."""
+
+    def __init__(self, lib, f32, heads, dim, rank, rows, rule=DELTA, win=None, ld=None):
+        self.lib, self.f32, self.rows = lib, f32, rows
+        lib.wr_hip_mix_pool_destroy.argtypes = lib.wr_hip_mix_step_destroy.argtypes = [vp]
+        lib.wr_hip_mix_pool_create.argtypes = [C.c_int, u32, vp, u32, u32, vp, u32, C.POINTER(vp)]
+        lib.wr_hip_mix_recur.argtypes = [vp, vp, u32, C.c_int, C.POINTER(Recurrence)]
+        lib.wr_hip_mix_window_append.argtypes = [vp, vp, u32, C.c_int, C.POINTER(Window), vp, u32, u32, u32, u32, vp, vp]
+        lib.wr_hip_mix_window_append_recur.argtypes = lib.wr_hip_mix_window_append.argtypes + [u32, C.POINTER(Recurrence)]
+        lib.wr_hip_mix_window_attend.argtypes = [vp, vp, u32, C.c_int, C.POINTER(Window), vp, vp, vp, u32, vp, u32]
+        self.step, hd, self.total = vp(), heads * dim, sum(rows)
+        self.padded = -(-self.total // 16) * 16
+        self.e, self.kt, wide = 4 if f32 else 2, -(-hd // 32), -(-hd // 32) * 32
+        self.pages, self.bufs, self.pools = [-(-3 * n // 64) for n in rows], [], []       # (room for three such steps)
+        self.dims = (u32 * 1)(win.kv_heads * (win.maps * win.dim_pad + win.vdim_pad) if win else 32)
+        self.state = (C.c_uint64 * 1)(hd * dim)
+        assert lib.wr_hip_mix_step_create(sum(self.pages), C.byref(self.step)) == 0
+        self.win, self.ld = win, ld or 5 * wide
+        rng = self.rng = np.random.default_rng(dim + rank)
+        self.r = Run(lib, f32, 1, -(-hd // 16) * 16, rank, self.total)
+        self.h = self.fill(self.padded * self.kt * 32 * self.e)
+        self.rec = Recurrence(heads=heads, dim=dim, rule=rule, unit_eps=1e-6, eps=1e-12, out_scale=1.0, gate_silu=0, ld=self.ld,
+                              col_k=wide, col_v=2 * wide, col_a=3 * wide if rule == DELTA else 0, col_g=4 * wide, w_decay=self.r.h,
+                              low=self.up(self.r.act(self.total, rank)), z=self.fill(self.padded * wide * 4).p, h=self.h.p, h_kt=self.kt,
+                              w0=self.put(np.full(wide, -1.0)), u=self.put(np.ones(wide)), a_bias=self.put(np.full(wide, -100.0)),
+                              norm=self.put(np.ones(wide)), in_=self.put(rng.standard_normal((self.total, self.ld))))
+
+    def keep(self, b):
+        self.bufs.append(b)
+        return b
+
+    def put(self, x):
+        return self.keep(hipattn.DeviceBuffer.from_host(np.asarray(x, np.float32))).p
+
+    def up(self, x):
+        return self.keep(self.r.up(x)).p
+
+    def fill(self, n):
+        return self.keep(hipattn.DeviceBuffer.from_host(np.full(n, 0x3C, np.uint8)))
+
+    def pool(self):
+        p = vp()
+        assert self.lib.wr_hip_mix_pool_create(int(self.f32), 1, self.dims, sum(self.pages), 1, self.state, len(self.rows), C.byref(p)) == 0
+        self.pools.append(p)
+        return p
+
+    def set(self, pool, nth=0):
+        seqs, page, lists = (Seq * len(self.rows))(), 0, []
+        for i, n in enumerate(self.rows):
+            lists.append((u32 * self.pages[i])(*range(page, page + self.pages[i])))
+            seqs[i], page = Seq(n, nth * n, i, (nth + 1) % 2, nth % 2, self.pages[i], lists[-1]), page + self.pages[i]
+        assert self.lib.wr_hip_mix_step_set(self.step, pool, len(self.rows), seqs, (u32 * self.total)(), 1, 0, None) == 0
+
+    def out(self):
+        hipattn.sync()
+        return self.r.frag_down(self.h, self.total, self.kt * 32)
+
+    def end(self):
+        hipattn.sync()
+        self.r.end()
+        self.lib.wr_hip_mix_step_destroy(self.step)
+        for p in self.pools:
+            self.lib.wr_hip_mix_pool_destroy(p)
+        for b in self.bufs:
+            b.free()
+
+
+# A decoded token's decays: one sum in the order of the low-rank product's outputs, over one to four tiles of them and whatever head size, as
+# the rest of its tile and the next tiles lose a one beside 2^24 and what is added tile by tile does not.
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("rule", [BONUS, DELTA])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4])
+@pytest.mark.parametrize("dim", [16, 30, 64, 65, 128, 200])
+def test_decays_are_one_sum_in_order(lib, f32, rule, tiles, dim):
+    heads, rank = 5, 32 * tiles
+    t = Recur(lib, f32, heads, dim, rank, [3, 3], rule)
+    w, low = np.zeros((1, t.r.N, rank), np.float32), np.zeros((6, rank), np.float32)
+    w[:, :, [0, rank - 2, rank - 1]], low[[1, 4]] = [4096.0, 1.0, -4096.0], 1.0
+    low[[[1], [4]], [0, rank - 1]] = 4096.0
+    lib.wr_hip_mix_mat_destroy(t.r.h)
+    assert lib.wr_hip_mix_mat_create(1, t.r.N, rank, O.f32_to_bf16(w).ctypes.data, C.byref(t.r.h)) == 0
+    t.rec.w_decay, t.rec.low = t.r.h, t.up(low)
+    # row 0 makes the state k v^T, row 1 lets it decay, row 2 reads w v + v': one channel a head
+    x, at, wide = np.zeros((6, t.ld), np.float32), [0, 1, dim // 2, dim - 2, dim - 1], t.rec.col_k
+    v0, v2 = np.where(np.arange(dim) % 2, -1.0, 1.0), np.ones(dim)
+    for first in (0, 3):
+        for h in range(heads):
+            x[[first, first + 2], wide + h * dim + at[h]] = 1.0
+            x[first + 2, h * dim + at[h]] = 1.0
+            x[first, 2 * wide + h * dim:][:dim], x[first + 2, 2 * wide + h * dim:][:dim] = v0, v2
+    t.rec.in_ = t.put(x)
+    p = t.pool()
+    t.set(p)
+    assert lib.wr_hip_mix_recur(t.step, p, 0, int(f32), C.byref(t.rec)) == 0
+    o = np.exp(-np.exp(-1.0)) ** (2 if rule == DELTA else 1) * v0 + v2     # (DELTA reads the state behind row 2's decay, of a product of zeros)
+    want = 0.5 * np.tile(o / np.sqrt((o * o).mean()), heads)            # (the gate: logistic of 0)
+    got = t.out()[[2, 5], :heads * dim]
+    # bfloat16: half a unit in the last place of outputs below 1; 32 bits: sums of one product and a norm over 200, each rounded a few times
+    assert np.abs(got - want).max() < (0.0 if f32 else 2.0 ** -9) + 2e-6, np.abs(got - want).max()
+    t.end()
+
+
 # One row to a workgroup up to 599 rows (1791 with experts' rows) and wherever no fragment is written, four beyond; features
 # that a workgroup holds in registers (4096) and more.
 @pytest.mark.parametrize("f32", [False, True])

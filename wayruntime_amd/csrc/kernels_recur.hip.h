@@ -110,7 +110,7 @@ __device__ __forceinline__ float recur_wave_sum(float v)
     return v;
 }
 
-// Ranks (in tiles of 32) up to which a decoded token's decays are made in passing: a tile to each quarter of the threads.
+// Ranks (in tiles of 32) up to which a decoded token's decays are made in passing: a tile to each quarter of the threads, the last one to the first.
 constexpr uint32_t kDecayTiles = 4;
 
 // Row r's product with output n of the decay's matrix.
@@ -153,25 +153,26 @@ __device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request,
     using V8 = typename MixAct<F32>::V8;
     constexpr int DPT = DP / 4, WV = DP >= 64 ? DP / 64 : 1;       // waves that hold the channels' own values
     constexpr bool QUARTERS = DP < 256;                           // (1024 threads have 128 registers each, and spill as it is)
-    __shared__ float sr[DP], sk[DP], sw[DP], sb[DP], red[8 * DP], sums[3 * WV], sq[WV], sz[QUARTERS ? 4 * DP : 1];
+    __shared__ float sr[DP], sk[DP], sw[DP], sb[DP], red[8 * DP], sums[3 * WV], sq[WV], sz[QUARTERS ? DP : 1];
     const uint32_t t = threadIdx.x, part = t / DP, c = t % DP, d0 = part * DPT, D = a.dim;
     const uint32_t lane = t & 63, wave = t >> 6;
     const bool has = c < D, own = t < DP && has;                  // (own: also the thread of channel c's values)
     const uint32_t hd = head * D, npad = (a.heads * D + 31) / 32 * 32, cc = has ? c : 0;
     const MixSeq s = a.seqs[a.list ? a.list[request] : request];
-    const float w0 = a.w0[hd + cc], nrm = a.norm[hd + cc], ub = DELTA ? a.ab[hd + cc] : a.u[hd + cc];
+    const float w0 = a.w0[hd + cc], nrm = a.norm[hd + cc], ub_at = DELTA ? a.ab[hd + cc] : a.u[hd + cc], ub = own ? ub_at : 0.f;
     const bool low = a.wd != nullptr, tile = QUARTERS && low && part < a.low_kt;
+    const uint32_t kt = tile ? a.low_kt - 1 - part : 0;
     bf16x8 wd[4];
     if (tile) {
         const uint32_t n = hd + cc;
 #pragma unroll
-        for (int g = 0; g < 4; g++) wd[g] = a.wd[((size_t)(n / 16) * a.low_kt + part) * 64 + 16 * g + n % 16];
+        for (int g = 0; g < 4; g++) wd[g] = a.wd[((size_t)(n / 16) * a.low_kt + kt) * 64 + 16 * g + n % 16];
     }
     const auto ask = [&](RecurRow<F32>& q, uint32_t r) {
         const float* row = a.in + (size_t)r * a.ld + hd + cc;
         if (tile) {
 #pragma unroll
-            for (int g = 0; g < 4; g++) q.x[g] = reinterpret_cast<const V8*>(a.low)[frag_unit(r, part * 4 + g, a.low_kt)];
+            for (int g = 0; g < 4; g++) q.x[g] = reinterpret_cast<const V8*>(a.low)[frag_unit(r, kt * 4 + g, a.low_kt)];
         }
         if (t < DP) {
             q.r = row[a.col_r];
@@ -196,21 +197,21 @@ __device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request,
         float z = next.z;
         if (!QUARTERS) {
             if (low && own) z = recur_z<F32>(a, r, hd + c);
-        } else if (low) {                                         // the row's product with the decay's matrix, a tile of inputs to a quarter
-            if (tile) {
-                z = 0.f;
+        } else if (low) {
+            // the row's product with the decay's matrix, one sum in the order of the inputs (recur_z): a quarter goes on where the one
+            // before it stopped, the channels' own threads last
+            for (uint32_t q = a.low_kt; q-- > 0;) {
+                if (part == q) {
+                    z = kt ? sz[c] : 0.f;
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    asm volatile("" : "+v"(wd[q]));               // (widened here, not ahead of the loop into twice the registers)
+                    for (int u = 0; u < 4; u++) {
+                        asm volatile("" : "+v"(wd[u]));           // (widened here, not ahead of the loop into twice the registers)
 #pragma unroll
-                    for (int j = 0; j < 8; j++) z = fmaf((float)wd[q][j], (float)next.x[q][j], z);
+                        for (int j = 0; j < 8; j++) z = fmaf((float)wd[u][j], (float)next.x[u][j], z);
+                    }
+                    if (q) sz[c] = z;
                 }
-                sz[t] = z;
-            }
-            __syncthreads();
-            if (own) {
-                z = sz[c];
-                for (uint32_t q = 1; q < a.low_kt; q++) z += sz[q * DP + c];
+                if (q) __syncthreads();
             }
         }
         if (i + 1 < s.rows) ask(next, r + 1);
@@ -231,7 +232,7 @@ __device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request,
                     sb[t] = rate * kk;
                 }
             } else {
-                const float ruk = recur_wave_sum(own ? rr * ub * kk : 0.f);
+                const float ruk = recur_wave_sum(rr * ub * kk);
                 if (lane == 0) sums[wave] = ruk;
                 if (t < DP) {
                     sr[t] = rr;
