@@ -212,27 +212,54 @@ def test_tiles_by_region(lib, batch, N, K, rows):
         b.free()
 
 
-# (batch, outputs, small one's outputs and inputs, rows): one launch where both are of sixteen rows at most and the second is small; else two
+# (batch, outputs, small one's outputs and inputs, rows): one launch where both are of sixteen rows at most and the second is small; else two.
+# Inputs a multiple of 1024 wide: the launch's items by region, of a multiple of eight workgroups and not, of eight and of four waves; odd
+# numbers of the small one's tiles; small ones that alone are two workgroups' or would be in tiles of two; a gated first.
 @pytest.mark.parametrize("f32", [False, True])
-@pytest.mark.parametrize("batch,N,K,n,k,rows", [(4, 1536, 288, 64, 288, 16), (1, 6144, 512, 16, 96, 1), (3, 2064, 1056, 48, 2048, 7), (2, 3088, 2080, 32, 4128, 5),
-                                                (4, 1536, 288, 64, 2080, 9), (4, 1536, 256, 64, 288, 3), (4, 1520, 288, 64, 288, 16), (4, 1536, 288, 400, 288, 16),
-                                                (4, 1536, 288, 64, 288, 17)])
-def test_two_products(lib, f32, batch, N, K, n, k, rows):
+@pytest.mark.parametrize("batch,N,K,n,k,rows,gated", [(4, 1536, 288, 64, 288, 16, 0), (1, 6144, 512, 16, 96, 1, 0), (3, 2064, 1056, 48, 2048, 7, 0),
+                                                      (2, 3088, 2080, 32, 4128, 5, 0), (4, 1536, 288, 64, 2080, 9, 0), (4, 1536, 256, 64, 288, 3, 0),
+                                                      (4, 1520, 288, 64, 288, 16, 0), (4, 1536, 288, 400, 288, 16, 0), (4, 1536, 288, 64, 288, 17, 0),
+                                                      (4, 2048, 2048, 64, 2048, 16, 0), (4, 1552, 1024, 48, 1024, 13, 0), (3, 2064, 1024, 16, 2080, 16, 0),
+                                                      (2, 3088, 3072, 80, 3072, 6, 0), (1, 6160, 4096, 32, 2048, 16, 0), (1, 6160, 1024, 32, 4096, 16, 0),
+                                                      (1, 2048, 1024, 64, 1024, 9, 1), (1, 2048, 4096, 64, 2080, 16, 1), (1, 2048, 1056, 16, 1056, 1, 1)])
+def test_two_products(lib, f32, batch, N, K, n, k, rows, gated):
     lib.wr_hip_mix_gemm_run_two.argtypes = [C.c_int, C.POINTER(Gemm), C.POINTER(Gemm)]
     r, q = Run(lib, f32, batch, N, K, rows), Run(lib, f32, 1, n, k, rows, seed=1)
     x, u = r.act(rows, batch * K), q.act(rows, k)
     xd, ud = r.up(x), q.up(u)
-    y, h = hipattn.DeviceBuffer(rows * batch * N * 4), hipattn.DeviceBuffer(-(-rows // 16) * 16 * (n + 31) // 32 * 32 * (4 if f32 else 2))
-    a = Gemm(w=r.h, x=xd.p, x_kt=batch * K // 32, x_kt_z=K // 32, rows=rows, out=ROWS_F32, y_f32=y.p, ldy=batch * N, col_z=N)
-    b = Gemm(w=q.h, x=ud.p, x_kt=k // 32, rows=rows, out=FRAG, h=h.p, h_kt=(n + 31) // 32, tanh_end=n)
+    first = -(-rows // 16) * 16 * N // 2 * (4 if f32 else 2) if gated else rows * batch * N * 4
+    second = -(-rows // 16) * 16 * (n + 31) // 32 * 32 * (4 if f32 else 2)
+    y, h, y2, h2 = [hipattn.DeviceBuffer.from_host(np.full(size, 7, np.uint8)) for size in (first, second) * 2]
+
+    def pair(y, h):
+        a = Gemm(w=r.h, x=xd.p, x_kt=batch * K // 32, x_kt_z=K // 32, rows=rows, out=ROWS_F32, y_f32=y.p, ldy=batch * N, col_z=N)
+        if gated:
+            a = Gemm(w=r.h, x=xd.p, x_kt=K // 32, rows=rows, out=GATED, h=y.p, h_kt=N // 64)
+        return a, Gemm(w=q.h, x=ud.p, x_kt=k // 32, rows=rows, out=FRAG, h=h.p, h_kt=(n + 31) // 32, tanh_end=n)
+
+    for which in (0, 1):                                   # refused whole, whichever of the two it is
+        bad = pair(y, h)
+        bad[which].rows = 0
+        assert lib.wr_hip_mix_gemm_run_two(int(f32), C.byref(bad[0]), C.byref(bad[1])) == hipattn.ERR_INVAL
+        hipattn.sync()
+        assert (y.to_host((first,), np.uint8) == 7).all() and (h.to_host((second,), np.uint8) == 7).all()
+    a, b = pair(y, h)
     assert lib.wr_hip_mix_gemm_run_two(int(f32), C.byref(a), C.byref(b)) == 0
     hipattn.sync()
-    r.close(y.to_host((rows, batch * N)), np.einsum("rzk,znk->rzn", x.reshape(rows, batch, K).astype(np.float64), r.w.astype(np.float64)).reshape(rows, -1))
+    want = np.stack([x.reshape(rows, batch, K)[:, z].astype(np.float64) @ r.w[z].T.astype(np.float64) for z in range(batch)], 1).reshape(rows, -1)
+    if gated:
+        t = want.reshape(rows, N // 32, 2, 16)
+        r.close(r.frag_down(y, rows, N // 2), (O.silu(t[:, :, 0]) * t[:, :, 1]).reshape(rows, -1), eight_bits=True)
+    else:
+        r.close(y.to_host((rows, batch * N)), want)
     q.close(q.frag_down(h, rows, (n + 31) // 32 * 32)[:, :n], np.tanh(u.astype(np.float64) @ q.w[0].T.astype(np.float64)), eight_bits=True)
-    b.h = None                                             # refused whole, whichever of the two it is
-    assert lib.wr_hip_mix_gemm_run_two(int(f32), C.byref(a), C.byref(b)) == hipattn.ERR_INVAL
+    for g in pair(y2, h2):                                 # the bits of two calls
+        assert lib.wr_hip_mix_gemm_run(int(f32), C.byref(g)) == 0
+    hipattn.sync()
+    assert np.array_equal(y.to_host((first,), np.uint8), y2.to_host((first,), np.uint8))
+    assert np.array_equal(h.to_host((second,), np.uint8), h2.to_host((second,), np.uint8))
     r.end(), q.end()
-    for d in (xd, ud, y, h):
+    for d in (xd, ud, y, h, y2, h2):
         d.free()
 
 

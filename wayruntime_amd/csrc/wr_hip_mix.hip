@@ -677,7 +677,7 @@ static int launch_rows(const MixGemmArgs& a, uint32_t batch, bool gated)
     return best(a, batch);
 }
 
-// A product's arguments, checked; `rows32`, `gated`: what goes out.
+// A product's arguments, checked; `gated`: whether pairs of tiles are gate and up.
 static int gemm_args(int f32, const wr_hip_mix_gemm* q, MixGemmArgs& a, uint32_t& batch, bool& gated)
 {
     if (!q || !q->w || !q->x || !q->rows) return WR_HIP_ERR_INVAL;
@@ -739,12 +739,16 @@ static int gemm_args(int f32, const wr_hip_mix_gemm* q, MixGemmArgs& a, uint32_t
     return WR_HIP_OK;
 }
 
-// Up to sixteen rows, bfloat16: whether two tiles to a workgroup are the form, of eight waves over a short range or four with twice the k-steps each
-// over a long one, which share the rows' operand (16 rows; us, one tile / this: 2048 -> 14 400 16.8 / 11.4, -> 32 768
-// 32.7 / 21.6, 4096 -> 24 576 40.4 / 36.0, -> 6144 13.7 / 11.1; narrow ones 4096 -> 4096 8.4 / 7.8).
-static bool gemm_two_tiles(const MixGemmArgs& a, uint32_t batch, bool gated)
+// Up to sixteen rows, bfloat16, no experts: four tiles to a workgroup over a short input range (or the launch is all workgroups and no work);
+// two workgroups to a tile (launch_parts); two tiles to a workgroup, of eight waves over a short range or four with twice the k-steps each over a long
+// one, which share the rows' operand (16 rows; us, one tile / this: 2048 -> 14 400 16.8 / 11.4, -> 32 768 32.7 / 21.6, 4096 -> 24 576 40.4 / 36.0, ->
+// 6144 13.7 / 11.1; narrow ones 4096 -> 4096 8.4 / 7.8); else one.
+enum class FewRows { kFour, kHalves, kTwo, kOne };
+static FewRows few_rows_form(const MixGemmArgs& a, uint32_t batch, bool gated)
 {
-    return gated || a.ntiles * batch >= 384;
+    if (!gated && a.ktiles <= 8 && a.ntiles % 4 == 0 && a.ntiles * batch >= 1024) return FewRows::kFour;
+    if (!gated && batch == 1 && a.ktiles >= kPartsMinKtiles && a.ntiles * 2 <= g.n_cus) return FewRows::kHalves;
+    return gated || a.ntiles * batch >= 384 ? FewRows::kTwo : FewRows::kOne;
 }
 constexpr uint32_t kEightWaveKtiles = 64;
 
@@ -834,10 +838,12 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
     }
     if (a.groups == 1) {
         a.cols = gemm_regions(a);
-        // a short input range: more outputs per workgroup, or the launch is all workgroups and no work
-        if (!gated && a.ktiles <= 8 && a.ntiles % 4 == 0 && a.ntiles * batch >= 1024) return launch_split<false, 4, 1, 4, 2, true>(a, batch);
-        if (!gated && batch == 1 && a.ktiles >= kPartsMinKtiles && a.ntiles * 2 <= g.n_cus) return launch_parts(a);
-        if (!gemm_two_tiles(a, batch, gated)) return launch_split<false, 1, 1, 4, 8, true>(a, batch);
+        switch (few_rows_form(a, batch, gated)) {
+        case FewRows::kFour: return launch_split<false, 4, 1, 4, 2, true>(a, batch);
+        case FewRows::kHalves: return launch_parts(a);
+        case FewRows::kOne: return launch_split<false, 1, 1, 4, 8, true>(a, batch);
+        case FewRows::kTwo: break;
+        }
         return a.ktiles <= kEightWaveKtiles ? launch_split<false, 2, 1, 8, 4, true>(a, batch) : launch_split<false, 2, 1, 4, 8, true>(a, batch);
     }
     return launch_rows(a, batch, gated);
@@ -852,9 +858,9 @@ int wr_hip_mix_gemm_run_two(int f32, const wr_hip_mix_gemm* q, const wr_hip_mix_
     int rc = gemm_args(f32, q, a, batch, gated);
     if (rc == WR_HIP_OK) rc = gemm_args(f32, small, b, batch_b, gated_b);
     if (rc) return rc;
-    // One launch where the first is in tiles of two and not by the short range's rule (wr_hip_mix_gemm_run), and the second adds a sixteenth at most
+    // One launch where the first is in tiles of two and the second in single ones, and the second adds a sixteenth at most
     const bool together = !f32 && !q->group_expert && !small->group_expert && a.groups == 1 && b.groups == 1 && batch_b == 1 &&
-                          gemm_two_tiles(a, batch, gated) && a.ktiles > 8 && (a.ktiles <= kEightWaveKtiles) == (b.ktiles <= kEightWaveKtiles) &&
+                          few_rows_form(a, batch, gated) == FewRows::kTwo && few_rows_form(b, 1, gated_b) == FewRows::kOne &&
                           b.ntiles <= a.ntiles && (uint64_t)b.ntiles * 16 <= (uint64_t)a.ntiles * batch;
     if (!together) {
         rc = wr_hip_mix_gemm_run(f32, q);
@@ -863,11 +869,11 @@ int wr_hip_mix_gemm_run_two(int f32, const wr_hip_mix_gemm* q, const wr_hip_mix_
     ENTER();
     cx->rows.store(q->rows, std::memory_order_relaxed);
     a.cols = gemm_regions(a);
-    const dim3 grid((a.ntiles + 1) / 2 * batch + (b.ntiles + 1) / 2);
+    const uint32_t of_a = (a.ntiles + 1) / 2 * batch;
     if (a.ktiles <= kEightWaveKtiles)
-        launch_main(mix_gemm_two_kernel<8, 4>, grid, dim3(512), a, b, 0);
+        launch_main(mix_gemm_two_kernel<8, 4>, dim3(of_a + (b.ntiles + 1) / 2), dim3(512), a, b, 0);
     else
-        launch_main(mix_gemm_two_kernel<4, 8>, grid, dim3(256), a, b, 0);
+        launch_main(mix_gemm_two_kernel<4, 8>, dim3(of_a + b.ntiles), dim3(256), a, b, 0);
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
 }
