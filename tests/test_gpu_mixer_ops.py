@@ -869,6 +869,30 @@ def test_decays_are_one_sum_in_order(lib, f32, rule, tiles, dim):
     t.end()
 
 
+# Sixteen requests of 64 heads: more workgroups than find a place at once where rows are asked for ahead.  The bits of each request alone.
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("rule", [BONUS, DELTA])
+@pytest.mark.parametrize("dim,rank,rows", [(64, 64, 1), (40, 128, 3)])
+def test_recurrence_of_many_workgroups(lib, f32, rule, dim, rank, rows):
+    many, alone = Recur(lib, f32, 64, dim, rank, [rows] * 16, rule), Recur(lib, f32, 64, dim, rank, [rows], rule)
+    x, low = many.rng.standard_normal((16 * rows, many.ld), dtype=np.float32), many.r.act(16 * rows, rank)
+    many.rec.in_, many.rec.low = many.put(x), many.up(low)
+    p, got = many.pool(), []
+    for nth in (0, 1):
+        many.set(p, nth)
+        assert lib.wr_hip_mix_recur(many.step, p, 0, int(f32), C.byref(many.rec)) == 0
+        got.append(many.out())
+    for i in (0, 7, 15):
+        at = slice(i * rows, (i + 1) * rows)
+        alone.rec.in_, alone.rec.low = alone.put(x[at]), alone.up(low[at])
+        p = alone.pool()
+        for nth in (0, 1):
+            alone.set(p, nth)
+            assert lib.wr_hip_mix_recur(alone.step, p, 0, int(f32), C.byref(alone.rec)) == 0
+            assert np.isfinite(got[nth][at]).all() and np.array_equal(alone.out(), got[nth][at]), (i, nth)
+    many.end(), alone.end()
+
+
 # One row to a workgroup up to 599 rows (1791 with experts' rows) and wherever no fragment is written, four beyond; features
 # that a workgroup holds in registers (4096) and more.
 @pytest.mark.parametrize("f32", [False, True])

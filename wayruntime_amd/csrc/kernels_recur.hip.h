@@ -146,21 +146,29 @@ struct RecurRow {
 //
 // Few rows: bound by a chain of trips to memory, of which there are three: arguments, the request's record, then its state,
 // its row, the decay's input and weights side by side (one after the other, and the list of requests where that is all of them, they
-// were six; 32 heads of 64: 16 requests 9.3 -> 8.2 us, 8 rows of one 15 -> 11.4).
-template <bool F32, int DP, bool DELTA>
-__device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request, uint32_t head)
+// were six; 32 heads of 64: 16 requests 9.3 -> 8.2 us, 8 rows of one 15 -> 11.4).  AHEAD: a quarter of the threads holds a tile of the decay's
+// input, and a row is asked for while the one before it is worked on.  Not where its registers cost more than the trips: 1024 threads have
+// 128 each and spill as it is (BONUS, a request of 8 heads of 256: 31.5 us ahead, 20.8), and of many workgroups a compute unit would have fewer
+// at a time (recur_ahead).  (The arguments by value: by reference the spills of 1024 threads come out otherwise, a request of 16 rows, DELTA, 531 us for 443.)
+template <bool F32, int DP, bool DELTA, bool AHEAD>
+__device__ __forceinline__ void recur_step(const RecurArgs a, uint32_t request, uint32_t head)
 {
     using V8 = typename MixAct<F32>::V8;
     constexpr int DPT = DP / 4, WV = DP >= 64 ? DP / 64 : 1;       // waves that hold the channels' own values
-    constexpr bool QUARTERS = DP < 256;                           // (1024 threads have 128 registers each, and spill as it is)
-    __shared__ float sr[DP], sk[DP], sw[DP], sb[DP], red[8 * DP], sums[3 * WV], sq[WV], sz[QUARTERS ? DP : 1];
+    __shared__ float sr[DP], sk[DP], sw[DP], sn[AHEAD ? 1 : DP], sb[DP], red[8 * DP], sums[3 * WV], sq[WV], sz[AHEAD ? DP : 1];
     const uint32_t t = threadIdx.x, part = t / DP, c = t % DP, d0 = part * DPT, D = a.dim;
     const uint32_t lane = t & 63, wave = t >> 6;
     const bool has = c < D, own = t < DP && has;                  // (own: also the thread of channel c's values)
     const uint32_t hd = head * D, npad = (a.heads * D + 31) / 32 * 32, cc = has ? c : 0;
     const MixSeq s = a.seqs[a.list ? a.list[request] : request];
-    const float w0 = a.w0[hd + cc], nrm = a.norm[hd + cc], ub_at = DELTA ? a.ab[hd + cc] : a.u[hd + cc], ub = own ? ub_at : 0.f;
-    const bool low = a.wd != nullptr, tile = QUARTERS && low && part < a.low_kt;
+    float w0 = 0.f, nrm = 0.f, ub = 0.f;
+    if constexpr (AHEAD) {
+        w0 = a.w0[hd + cc];
+        nrm = a.norm[hd + cc];
+        ub = DELTA ? a.ab[hd + cc] : a.u[hd + cc];
+        ub = own ? ub : 0.f;
+    }
+    const bool low = a.wd != nullptr, tile = AHEAD && low && part < a.low_kt;
     const uint32_t kt = tile ? a.low_kt - 1 - part : 0;
     bf16x8 wd[4];
     if (tile) {
@@ -184,23 +192,34 @@ __device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request,
         q.v = row[a.col_v];
     };
     RecurRow<F32> next;
-    ask(next, s.row0);
+    if constexpr (AHEAD) ask(next, s.row0);
     const size_t head_elems = (size_t)D * D;
     const float* in = a.state + ((size_t)s.state_in * a.heads + head) * head_elems;
     float* out = a.state + ((size_t)s.state_out * a.heads + head) * head_elems;
     float S[DPT];
 #pragma unroll
     for (int j = 0; j < DPT; j++) S[j] = (s.pos0 > 0 && has && d0 + j < D) ? in[(size_t)(d0 + j) * D + c] : 0.f;
+    if constexpr (!AHEAD) {
+        w0 = own ? a.w0[hd + c] : 0.f;
+        nrm = own ? a.norm[hd + c] : 0.f;
+        ub = own ? (DELTA ? a.ab[hd + c] : a.u[hd + c]) : 0.f;
+    }
     for (uint32_t i = 0; i < s.rows; i++) {
         const uint32_t r = s.row0 + i;
-        const float vv = has ? next.v : 0.f, rr = own ? next.r : 0.f, kk = own ? next.k : 0.f, g = own ? next.g : 0.f, za = next.a;
-        float z = next.z;
-        if (!QUARTERS) {
-            if (low && own) z = recur_z<F32>(a, r, hd + c);
-        } else if (low) {
+        const float* row = a.in + (size_t)r * a.ld + hd;
+        float vv, rr = 0.f, kk = 0.f, g = 0.f, za = 0.f, z = 0.f;
+        if constexpr (AHEAD) {
+            vv = has ? next.v : 0.f;
+            if (own) {
+                rr = next.r;
+                kk = next.k;
+                g = next.g;
+                za = next.a;
+                z = next.z;
+            }
             // the row's product with the decay's matrix, one sum in the order of the inputs (recur_z): a quarter goes on where the one
             // before it stopped, the channels' own threads last
-            for (uint32_t q = a.low_kt; q-- > 0;) {
+            for (uint32_t q = low ? a.low_kt : 0; q-- > 0;) {
                 if (part == q) {
                     z = kt ? sz[c] : 0.f;
 #pragma unroll
@@ -213,12 +232,19 @@ __device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request,
                 }
                 if (q) __syncthreads();
             }
+            if (i + 1 < s.rows) ask(next, r + 1);
+        } else {
+            vv = has ? row[a.col_v + c] : 0.f;
         }
-        if (i + 1 < s.rows) ask(next, r + 1);
         if (wave < WV) {
-            const float w = own ? recur_decay(a, z + w0) : 0.f;
+            if constexpr (!AHEAD) {
+                rr = own ? row[a.col_r + c] : 0.f;
+                kk = own ? row[a.col_k + c] : 0.f;
+            }
+            const float w = own ? recur_decay(a, (AHEAD ? z : a.wd ? recur_z<F32>(a, r, hd + c) : a.z[(size_t)r * a.ldz + hd + c]) + w0) : 0.f;
+            if constexpr (!AHEAD) g = own ? row[a.col_g + c] : 0.f;
             if constexpr (DELTA) {
-                const float rate = own ? 1.0f / (1.0f + expf(-(za + ub))) : 0.f;
+                const float rate = own ? 1.0f / (1.0f + expf(-((AHEAD ? za : row[a.col_a + c]) + ub))) : 0.f;
                 const float k2 = recur_wave_sum(kk * kk), rk = recur_wave_sum(rr * kk), rak = recur_wave_sum(rr * rate * kk);
                 if (lane == 0) {
                     sums[wave] = k2;
@@ -229,6 +255,7 @@ __device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request,
                     sr[t] = rr * w;
                     sk[t] = kk;
                     sw[t] = w;
+                    if constexpr (!AHEAD) sn[t] = kk;              // (read beside sr: one array for both spills more)
                     sb[t] = rate * kk;
                 }
             } else {
@@ -251,7 +278,7 @@ __device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request,
 #pragma unroll
         for (int j = 0; j < DPT; j++) {
             o = fmaf(sr[d0 + j], S[j], o);
-            if constexpr (DELTA) p = fmaf(sk[d0 + j], S[j], p);
+            if constexpr (DELTA) p = fmaf((AHEAD ? sk : sn)[d0 + j], S[j], p);
         }
         red[t] = o;
         if constexpr (DELTA) red[4 * DP + t] = p;
@@ -304,14 +331,14 @@ __device__ __forceinline__ void recur_step(const RecurArgs& a, uint32_t request,
         if (has && d0 + j < D) out[(size_t)(d0 + j) * D + c] = S[j];
 }
 
-// Waves to a SIMD: three, so that the workgroups of sixteen requests of 32 heads are there at once, with an append's.
-constexpr int recur_step_waves(int dp) { return dp <= 64 ? 3 : 1; }
+// Waves to a SIMD for head sizes up to 64: four where the registers allow it.
+constexpr int recur_waves(bool f32, bool delta, bool ahead) { return ahead && (f32 || delta) ? 3 : 4; }
 
 // grid (requests, heads)
-template <bool F32, int DP, bool DELTA>
-__global__ __launch_bounds__(4 * DP, recur_step_waves(DP)) void recur_step_kernel(const RecurArgs a)
+template <bool F32, int DP, bool DELTA, bool AHEAD>
+__global__ __launch_bounds__(4 * DP, DP <= 64 ? recur_waves(F32, DELTA, AHEAD) : 1) void recur_step_kernel(const RecurArgs a)
 {
-    recur_step<F32, DP, DELTA>(a, blockIdx.x, blockIdx.y);
+    recur_step<F32, DP, DELTA, AHEAD>(a, blockIdx.x, blockIdx.y);
 }
 
 // FORGET.  grid (requests, heads), 4 CP threads: thread t has value column t % CP, channels DPT (t / CP) .. +DPT

@@ -180,7 +180,7 @@ __device__ __forceinline__ float window_value(const WindowArgs& a, uint32_t r, u
 
 // Four rows' keys and values of one head, or a slice of their query units (slice >= key_heads).
 template <bool F32>
-__device__ __forceinline__ void window_append(const WindowArgs& a, uint32_t rows4, uint32_t slice)
+__device__ __forceinline__ void window_append(const WindowArgs a, uint32_t rows4, uint32_t slice)
 {
     using E = typename MixAct<F32>::E;
     using V4 = typename MixAct<F32>::V4;
@@ -262,10 +262,11 @@ __global__ __launch_bounds__(256) void window_append_kernel(const WindowArgs a)
 // A step's recurrence and the append beside it, which read one product's rows and write apart: workgroups below
 // `steps` are a request and head each, the others the append's, append_x of them to a slice.  In launches of their own the append's
 // few workgroups took as long as a launch takes (16 rows, 16/8 heads of 128 beside 32 of 64: 6.2 and 8.3 us, 9.6 together).
-__global__ __launch_bounds__(256, recur_step_waves(64)) void window_append_recur_kernel(const WindowArgs a, const RecurArgs r, uint32_t steps, uint32_t append_x)
+template <bool AHEAD>
+__global__ __launch_bounds__(256, recur_waves(false, true, AHEAD)) void window_append_recur_kernel(const WindowArgs a, const RecurArgs r, uint32_t steps, uint32_t append_x)
 {
     if (blockIdx.x < steps) {
-        recur_step<false, 64, true>(r, blockIdx.x / r.heads, blockIdx.x % r.heads);
+        recur_step<false, 64, true, AHEAD>(r, blockIdx.x / r.heads, blockIdx.x % r.heads);
     } else {
         const uint32_t i = blockIdx.x - steps;
         window_append<false>(a, i % append_x, i / append_x);

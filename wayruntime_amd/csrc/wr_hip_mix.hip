@@ -994,16 +994,27 @@ int wr_hip_mix_gate_norm(wr_hip_mix_step* s, int f32, const float* o_dev, uint32
 
 // ------------------------------------------------------------- recurrence --
 
+// Head sizes 33 to 64: whether rows are asked for ahead.  In that form a compute unit has three of the workgroups at a time and not four (BONUS of
+// bfloat16 rows: four), so not where that takes more rounds of them: sixteen requests of 16 rows, DELTA, us ahead / not: 48 heads of 64 41.8 / 48.1, 64
+// 68.5 / 53.5, 96 74 / 93, 112 95 / 98; of one row, 64 heads 13.2 / 10.8.
+template <bool F32, bool DELTA>
+static bool recur_ahead(uint64_t workgroups)
+{
+    const uint64_t at_once = recur_waves(F32, DELTA, true) * g.n_cus, otherwise = recur_waves(F32, DELTA, false) * g.n_cus;
+    return (workgroups + at_once - 1) / at_once == (workgroups + otherwise - 1) / otherwise;
+}
+
 template <bool F32, bool DELTA>
 static int recur_steps(const RecurArgs& a, uint32_t n)
 {
     if (n == 0) return WR_HIP_OK;
     const dim3 grid(n, a.heads);
-    if (a.dim <= 16) MIX_LAUNCH((recur_step_kernel<F32, 16, DELTA>), grid, dim3(64), 0, a);
-    else if (a.dim <= 32) MIX_LAUNCH((recur_step_kernel<F32, 32, DELTA>), grid, dim3(128), 0, a);
-    else if (a.dim <= 64) MIX_LAUNCH((recur_step_kernel<F32, 64, DELTA>), grid, dim3(256), 0, a);
-    else if (a.dim <= 128) MIX_LAUNCH((recur_step_kernel<F32, 128, DELTA>), grid, dim3(512), 0, a);
-    else MIX_LAUNCH((recur_step_kernel<F32, 256, DELTA>), grid, dim3(1024), 0, a);
+    if (a.dim <= 16) MIX_LAUNCH((recur_step_kernel<F32, 16, DELTA, true>), grid, dim3(64), 0, a);
+    else if (a.dim <= 32) MIX_LAUNCH((recur_step_kernel<F32, 32, DELTA, true>), grid, dim3(128), 0, a);
+    else if (a.dim <= 64 && recur_ahead<F32, DELTA>((uint64_t)n * a.heads)) MIX_LAUNCH((recur_step_kernel<F32, 64, DELTA, true>), grid, dim3(256), 0, a);
+    else if (a.dim <= 64) MIX_LAUNCH((recur_step_kernel<F32, 64, DELTA, false>), grid, dim3(256), 0, a);
+    else if (a.dim <= 128) MIX_LAUNCH((recur_step_kernel<F32, 128, DELTA, true>), grid, dim3(512), 0, a);
+    else MIX_LAUNCH((recur_step_kernel<F32, 256, DELTA, false>), grid, dim3(1024), 0, a);
     return WR_HIP_OK;
 }
 
@@ -1516,17 +1527,23 @@ int wr_hip_mix_window_append_recur(wr_hip_mix_step* s, wr_hip_mix_pool* pool, ui
     int rc = append_args(s, pool, run, f32, q, in_dev, ld, col_q, col_k, col_v, table_dev, q_dev, a, grid);
     if (rc == WR_HIP_OK) rc = recur_args(s, pool, recur_run, recur, r);
     if (rc) return rc;
-    // One launch where the step's requests all take the recurrence token by token in workgroups of the append's size
-    // (recur_steps), the decays' product in passing (recur_run), and the append is no more than a few rows'
+    // One launch where the step's requests all take the recurrence token by token (sixteen rows each at most) in workgroups of the append's size
+    // (recur_steps), the decays' product in passing (recur_run).  Of sixteen requests of one and of 16 rows, 16/8 heads of 128 beside so many of 64, us, two
+    // launches / one: 32 12.4 / 8.3, 44.2 / 38.3; 64 16.6 / 13.8, 58.5 / 56.4.  Where rows are not asked for ahead only up to eight a request: 64 heads
+    // of 40, 16 rows 49.7 / 53.5 (the append's registers beside it).  (The last bound is the grid's alone.)
     const uint64_t steps = (uint64_t)s->n_seq * r.heads, appends = (uint64_t)grid.x * grid.y;
-    if (f32 || recur->rule != WR_HIP_MIX_RULE_DELTA || s->n_long || r.low_kt > kDecayTiles || r.dim <= 32 || r.dim > 64 || steps + appends > 1u << 20) {
+    const bool ahead = recur_ahead<false, true>(steps);
+    if (f32 || recur->rule != WR_HIP_MIX_RULE_DELTA || s->n_long || r.low_kt > kDecayTiles || r.dim <= 32 || r.dim > 64 ||
+        (!ahead && s->rows > 8 * s->n_seq) || steps + appends > 1u << 20) {
         rc = wr_hip_mix_window_append(s, pool, run, f32, q, in_dev, ld, col_q, col_k, col_v, table_dev, q_dev);
         return rc ? rc : wr_hip_mix_recur(s, pool, recur_run, f32, recur);
     }
     ENTER();
     r.wd = reinterpret_cast<const bf16x8*>(recur->w_decay->tiles);
     r.low = recur->low;
-    MIX_LAUNCH(window_append_recur_kernel, dim3((uint32_t)(steps + appends)), dim3(256), 0, a, r, (uint32_t)steps, grid.x);
+    const dim3 together((uint32_t)(steps + appends));
+    if (ahead) MIX_LAUNCH(window_append_recur_kernel<true>, together, dim3(256), 0, a, r, (uint32_t)steps, grid.x);
+    else MIX_LAUNCH(window_append_recur_kernel<false>, together, dim3(256), 0, a, r, (uint32_t)steps, grid.x);
     return WR_HIP_OK;
 }
 
