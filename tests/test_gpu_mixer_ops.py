@@ -710,9 +710,11 @@ class Router(C.Structure):
                 ("scale", C.c_float), ("correction", vp), ("logistic", u32)]
 
 
-# The choice with the order up to 32 rows and before it beyond; pairs of whole turns of eight thousand, two less, one more, and of two turns and a rest; outputs a lane
+# The choice with the order up to 32 rows, up to 64 where few are chosen of few, and before it beyond; pairs one by one and, past 2048, eight at a time: of whole turns of eight
+# thousand, two less, one more, and of two turns and a rest; outputs a lane
 # holds one, four and sixteen of; identity outputs; runs of one group and of eight.
-@pytest.mark.parametrize("experts,identity,top,rows,run", [(64, 0, 6, 1, 1), (64, 0, 6, 32, 1), (64, 0, 6, 33, 1), (64, 0, 6, 64, 8), (60, 4, 2, 4095, 8),
+@pytest.mark.parametrize("experts,identity,top,rows,run", [(64, 0, 6, 1, 1), (64, 0, 6, 32, 1), (64, 0, 6, 33, 1), (64, 0, 6, 64, 8), (64, 0, 1, 64, 1), (64, 0, 2, 40, 1), (64, 0, 2, 41, 1),
+                                                           (100, 28, 1, 48, 1), (100, 28, 1, 49, 8), (64, 0, 8, 256, 1), (64, 0, 8, 257, 1), (60, 4, 2, 4095, 8),
                                                            (60, 0, 2, 4096, 8), (64, 0, 3, 2731, 8), (64, 0, 6, 2800, 8), (120, 8, 5, 40, 1), (300, 12, 9, 32, 2),
                                                            (300, 12, 9, 33, 2), (1000, 24, 64, 257, 1)])
 def test_routes(lib, experts, identity, top, rows, run):

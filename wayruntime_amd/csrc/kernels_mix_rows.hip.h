@@ -698,23 +698,24 @@ __global__ __launch_bounds__(256) void mix_top_kernel(const MixRouteArgs a)
     if (row < a.rows) mix_top<PER>(a, row, threadIdx.x & 63, [&](uint32_t t, uint32_t e) { a.slot[(size_t)row * a.top + t] = e; });
 }
 
-// Of a step whose choice is made with the order: a wave takes 2.4 us to a row and sixteen run side by side, and a launch of its own for the
-// choice 5 us and its gap (64 outputs, top 6: 16 rows 5.2 us in one launch and 10.6 in two, 32 7.6 and 10.6, 48 11.9 and 10.6, 64 14.7 and 10.6).
+// Of a step whose choice is made with the order (mix_order_too).
 constexpr uint32_t kOrderRows = 32, kOrderPairs = kOrderRows * 64;
-// Pairs a thread asks for at once: the launch is one workgroup, bound by what a pair waits for and by the scattered stores (1500 rows of
-// top 6 one by one 11.0 us, so 9.7; 4096 rows 27.0 and 21.6).
-constexpr uint32_t kOrderAhead = 8;
+// Beyond kOrderFew pairs a thread asks for eight at once: the launch is one workgroup, bound by what a pair waits for and by the scattered stores
+// (1500 rows of top 6 one by one 11.0 us, so 9.7; 4096 rows 27.0 and 21.6).  Up to there it has one or two, and would ask for eight in vain (64 outputs,
+// 256 rows, choice and order, one by one / eight: top 4 7.5 / 8.5, top 8 10.3 / 10.3, top 16 16.2 / 14.4).
+constexpr uint32_t kOrderAhead = 8, kOrderFew = 2048;
 
 // One workgroup: orders the chosen (row, expert) pairs by expert.  Each expert's
 // pairs take whole runs of tile_groups groups of 16 slots.  Which slot of its
 // expert a pair gets may differ from run to run; nothing computed for it does
 // (a slot's column of a matrix product depends on that column alone).
-// PER: outputs a lane holds where the choice is made here too (few rows), else 0.
-template <int PER>
+// PER: outputs a lane holds where the choice is made here too (few rows), else 0.  AHEAD: pairs a thread asks for at once.
+template <int PER, uint32_t AHEAD>
 __global__ __launch_bounds__(1024) void mix_order_kernel(const MixRouteArgs a)
 {
     constexpr bool TOP = PER > 0;
     __shared__ uint32_t count[1024], wave_sum[16];
+    static_assert(!TOP || AHEAD == 1, "few pairs");
     __shared__ uint16_t pick[TOP ? kOrderPairs : 1];
     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const uint32_t n_slots = a.n_groups * 16, pairs = a.rows * a.top, run = a.tile_groups * 16;
@@ -731,13 +732,16 @@ __global__ __launch_bounds__(1024) void mix_order_kernel(const MixRouteArgs a)
                 pick[r * a.top + k] = (uint16_t)e;
                 if (e < a.experts) atomicAdd(&count[e], 1u);
             });
+    } else if constexpr (AHEAD == 1) {
+        for (uint32_t i = t; i < pairs; i += 1024)
+            if (a.slot[i] < a.experts) atomicAdd(&count[a.slot[i]], 1u);
     } else {
-        for (uint32_t i0 = t; i0 < pairs; i0 += 1024 * kOrderAhead) {
-            uint32_t e[kOrderAhead];
+        for (uint32_t i0 = t; i0 < pairs; i0 += 1024 * AHEAD) {
+            uint32_t e[AHEAD];
 #pragma unroll
-            for (uint32_t k = 0; k < kOrderAhead; k++) e[k] = a.slot[min(i0 + 1024 * k, pairs - 1)];
+            for (uint32_t k = 0; k < AHEAD; k++) e[k] = a.slot[min(i0 + 1024 * k, pairs - 1)];
 #pragma unroll
-            for (uint32_t k = 0; k < kOrderAhead; k++)
+            for (uint32_t k = 0; k < AHEAD; k++)
                 if (i0 + 1024 * k < pairs && e[k] < a.experts) atomicAdd(&count[e[k]], 1u);
         }
     }
@@ -755,29 +759,31 @@ __global__ __launch_bounds__(1024) void mix_order_kernel(const MixRouteArgs a)
     for (uint32_t g = 0; g < (count[t] + 15) / 16; g++) a.group_expert[(upto - mine) / 16 + g] = (int32_t)t;   // (a run's empty groups stay -1)
     count[t] = upto - mine;                                // from here on: the expert's next slot
     __syncthreads();
-    constexpr uint32_t AHEAD = TOP ? 1 : kOrderAhead;      // (few pairs: a thread's first is its only one)
-    for (uint32_t i0 = t; i0 < pairs; i0 += 1024 * AHEAD) {
-        uint32_t e[AHEAD];
-        float w[AHEAD];
-#pragma unroll
-        for (uint32_t k = 0; k < AHEAD; k++) {
-            const uint32_t i = min(i0 + 1024 * k, pairs - 1);
-            if constexpr (TOP) e[k] = pick[i];
-            else e[k] = a.slot[i];
-            w[k] = a.slot_weight ? a.gate[i] : 0.f;        // (made here: ahead of two barriers)
+    const auto place = [&](uint32_t i, uint32_t e, auto weight) {
+        if (e >= a.experts) {                              // the input itself: nothing to compute
+            a.slot[i] = 0xFFFFFFFFu;
+            return;
         }
+        const uint32_t s = atomicAdd(&count[e], 1u);
+        a.slot[i] = s;
+        a.perm[s] = i / a.top;
+        if (a.slot_weight) a.slot_weight[s] = weight();    // (the gate: made here, ahead of two barriers)
+    };
+    if constexpr (AHEAD == 1) {
+        for (uint32_t i = t; i < pairs; i += 1024) place(i, TOP ? pick[TOP ? i : 0] : a.slot[i], [&] { return a.gate[i]; });
+    } else {
+        for (uint32_t i0 = t; i0 < pairs; i0 += 1024 * AHEAD) {
+            uint32_t e[AHEAD];
+            float w[AHEAD];
 #pragma unroll
-        for (uint32_t k = 0; k < AHEAD; k++) {
-            const uint32_t i = i0 + 1024 * k;
-            if (i >= pairs) break;
-            if (e[k] >= a.experts) {                       // the input itself: nothing to compute
-                a.slot[i] = 0xFFFFFFFFu;
-                continue;
+            for (uint32_t k = 0; k < AHEAD; k++) {
+                const uint32_t i = min(i0 + 1024 * k, pairs - 1);
+                e[k] = a.slot[i];
+                w[k] = a.slot_weight ? a.gate[i] : 0.f;
             }
-            const uint32_t s = atomicAdd(&count[e[k]], 1u);
-            a.slot[i] = s;
-            a.perm[s] = i / a.top;
-            if (a.slot_weight) a.slot_weight[s] = w[k];
+#pragma unroll
+            for (uint32_t k = 0; k < AHEAD; k++)
+                if (i0 + 1024 * k < pairs) place(i0 + 1024 * k, e[k], [&] { return w[k]; });
         }
     }
 }

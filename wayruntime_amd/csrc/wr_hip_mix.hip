@@ -1678,6 +1678,14 @@ uint32_t wr_hip_mix_route_groups(uint32_t rows, uint32_t experts, uint32_t top, 
     return (uint32_t)(runs * tile_groups);
 }
 
+// Whether one launch chooses and orders: a wave takes its rows one after the other, sixteen rows side by side; a launch of its own for the choice is some 5
+// us and its gap.  us a call, one launch / two: 64 outputs, top 6, 33 rows 9.6 / 8.1, 64 15.3 / 8.3; top 1, 33 rows 5.5 / 6.9, 64 7.2 / 7.4; top 2,
+// 40 rows 6.8 / 7.8, 48 7.4 / 7.1; 256 outputs, top 1, 48 rows 6.7 / 7.0, 64 7.6 / 7.0; 512, top 1, 33 rows 9.3 / 7.2.
+static bool mix_order_too(uint32_t rows, uint32_t outputs, uint32_t top)
+{
+    return rows <= kOrderRows || (rows <= 64 && rows * top <= (outputs <= 64 ? 80u : outputs <= 256 ? 48u : 0u));
+}
+
 int wr_hip_mix_route(wr_hip_mix_step* s, const float* z_dev, uint32_t ldz, const wr_hip_mix_router* q, uint32_t tile_groups,
                      float* gate_dev, float* side_dev, float* slot_weight_dev, uint32_t* slot_dev, uint32_t* perm_dev,
                      int32_t* group_expert_dev)
@@ -1717,17 +1725,18 @@ int wr_hip_mix_route(wr_hip_mix_step* s, const float* z_dev, uint32_t ldz, const
     a.perm = perm_dev;
     a.group_expert = group_expert_dev;
     static_assert(WR_HIP_MIX_MAX_TOP * kOrderRows <= kOrderPairs, "choices of a short step");
-    if (s->rows <= kOrderRows) {
-        if (outputs <= 64) MIX_LAUNCH(mix_order_kernel<1>, dim3(1), dim3(1024), 0, a);
-        else if (outputs <= 256) MIX_LAUNCH(mix_order_kernel<4>, dim3(1), dim3(1024), 0, a);
-        else MIX_LAUNCH(mix_order_kernel<16>, dim3(1), dim3(1024), 0, a);
+    if (mix_order_too(s->rows, (uint32_t)outputs, q->top)) {
+        if (outputs <= 64) MIX_LAUNCH((mix_order_kernel<1, 1>), dim3(1), dim3(1024), 0, a);
+        else if (outputs <= 256) MIX_LAUNCH((mix_order_kernel<4, 1>), dim3(1), dim3(1024), 0, a);
+        else MIX_LAUNCH((mix_order_kernel<16, 1>), dim3(1), dim3(1024), 0, a);
         return WR_HIP_OK;
     }
     const dim3 grid((s->rows + 3) / 4), block(256);
     if (outputs <= 64) MIX_LAUNCH(mix_top_kernel<1>, grid, block, 0, a);
     else if (outputs <= 256) MIX_LAUNCH(mix_top_kernel<4>, grid, block, 0, a);
     else MIX_LAUNCH(mix_top_kernel<16>, grid, block, 0, a);
-    MIX_LAUNCH(mix_order_kernel<0>, dim3(1), dim3(1024), 0, a);
+    if (s->rows * q->top <= kOrderFew) MIX_LAUNCH((mix_order_kernel<0, 1>), dim3(1), dim3(1024), 0, a);
+    else MIX_LAUNCH((mix_order_kernel<0, kOrderAhead>), dim3(1), dim3(1024), 0, a);
     return WR_HIP_OK;
 }
 
