@@ -875,6 +875,23 @@ def test_memory_of_a_short_cache_comes_back_cleared(call, pos, n):
             kv.close()
 
 
+@pytest.mark.parametrize("nkv,hd,n", [(1, 64, 60000), (1, 256, 3000), (3, 64, 20000)])
+def test_memory_of_a_long_cache_of_few_heads_comes_back_cleared(nkv, hd, n):
+    # more workgroups to a head than the eight that many layers take
+    for _ in range(2):
+        kv = hipattn.KVCache(1, hd, nkv, 131072)
+        for at in (0, n - 40, n + 5, 131000):
+            k, v = kv.read_f16(0, at, 72)
+            assert not k.any() and not v.any(), at
+        for at in range(0, n, 4096):
+            rows = np.ones((min(4096, n - at), nkv, hd), np.float32)
+            assert kv.append(0, at, rows, rows) == hipattn.OK
+        kv.close()
+    kv = hipattn.KVCache(1, hd, nkv, 131072)
+    assert not any(x.any() for x in kv.read_f16(0, 0, n + 64))
+    kv.close()
+
+
 def test_memory_of_ended_caches_is_bounded_and_comes_back_cleared():
     def free_bytes():                                        # of the runtime that the library is linked with
         free, total = C.c_size_t(), C.c_size_t()

@@ -157,7 +157,12 @@ hipError_t slab_clear(const Lib::Slab& s)
     if (s.cleared.tiles == 0) return hipSuccess;
     if (s.cleared.tiles * 2 >= s.cleared.ctx_pad / kTileKeys || s.cleared.nkv > 0xFFFF / 2)   // (nearly all of it; no grid)
         return hipMemsetAsync(s.p, 0, s.bytes, cx->stream);
-    hipLaunchKernelGGL(clear_cache_kernel, dim3(8, 2 * s.cleared.nkv, s.n_layers), dim3(256), 0, cx->stream, s.cleared, s.p);
+    // eight workgroups to a layer's head, and more where there are few of these: 2048 in all, of four stores a thread and more
+    uint32_t hd = 0;
+    for (uint32_t L = 0; L < s.n_layers; L++) hd = std::max(hd, s.cleared.hd[L]);
+    const uint64_t stores = (uint64_t)s.cleared.tiles * kTileKeys * hd / 8, spread = 2048 / (2 * s.cleared.nkv * s.n_layers);
+    const uint32_t x = (uint32_t)std::max<uint64_t>(8, std::min(spread, stores / 1024));
+    hipLaunchKernelGGL(clear_cache_kernel, dim3(x, 2 * s.cleared.nkv, s.n_layers), dim3(256), 0, cx->stream, s.cleared, s.p);
     return hipGetLastError();
 }
 
