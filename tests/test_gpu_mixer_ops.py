@@ -196,10 +196,10 @@ def test_batch_of_matrices(lib, f32, batch, N, K, rows):
         b.free()
 
 
-# whose tiles an XCD takes side by side: launches of fewer workgroups than XCDs, of a few more, of many and a rest; one tile to
+# whose tiles an XCD takes side by side, and beside them inputs and batches for which it does not: launches of fewer workgroups than XCDs, of a few more, of many and a rest; one tile to
 # a workgroup, two, two workgroups to a tile, batches
 @pytest.mark.parametrize("batch,N,K,rows", [(1, 16, 1024, 1), (1, 144, 1024, 16), (1, 6160, 1024, 9), (1, 14416, 2048, 16), (1, 48, 4096, 3), (1, 1104, 4096, 2),
-                                            (3, 2064, 1024, 5)])
+                                            (3, 2064, 1024, 5), (3, 2064, 2048, 16), (8, 1040, 4096, 7), (16, 512, 2048, 16), (1, 4112, 3072, 16)])
 def test_tiles_by_region(lib, batch, N, K, rows):
     r = Run(lib, False, batch, N, K, rows)
     x = r.act(rows, batch * K)

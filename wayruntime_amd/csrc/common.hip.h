@@ -255,8 +255,8 @@ __device__ __forceinline__ bool xcd_tile(uint32_t block, uint32_t cols, uint32_t
 }
 
 // Work item of workgroup `block` of `n` such that an XCD's workgroups (block % 8) take neighbouring items: a weight that is
-// read once, as a stream, is then one region to an XCD.  Where the regions that items begin at lie on the same memory channels (a multiple of
-// 32 KiB), all of a launch's streams walk those together, and each XCD holds few of them open this way: 268 MB in streams of
+// read once, as a stream, is then one region to an XCD.  Where items begin on the same memory channels (32 KiB times a
+// power of two), all of a launch's streams walk those together, and each XCD holds few of them open this way: 268 MB in streams of
 // 64 KiB, two to a wave, 48.2 us dealt out, 41.1 in regions.
 __device__ __forceinline__ uint32_t xcd_region(uint32_t block, uint32_t n)
 {

@@ -29,8 +29,7 @@ struct MixGemmArgs {
     float scale, limit, slope, up_bias;
     const float* bias;
     uint32_t cols;                   // mix_gemm_lds_kernel without experts: XCDs that share out the outputs (xcd_tile);
-                                     // a stream of experts: runs that the XCDs share out, or 0; up to sixteen rows of others:
-                                     // whether an XCD's workgroups take neighbouring tiles (xcd_region)
+                                     // a stream of experts: runs that the XCDs share out, or 0
     const uint32_t* x_perm;
     const float* x_scale;            // a factor per row of the input (applied to its products), or nullptr
     float* y;
@@ -158,7 +157,7 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // trip to memory each: 16 rows, 768 -> 2048 5.5 us, 3.9 now; 1536 -> 512 5.5, 4.3.
 // Few rows: bound by the weights' bytes.  More rows: by the bytes that pass a
 // compute unit's vector cache, NT + GR KiB a k-step for NT x GR products.
-// STREAM: every weight tile is read by one workgroup only (no use in keeping it).  s_part: WAVES x NT x GR x 64 of LDS.
+// STREAM: every weight tile is read by one workgroup only (no use in keeping it).
 // With group_expert the GR groups share an expert (GR divides tile_groups), and of a run's only those are read,
 // multiplied and stored that rows are in: a compute unit takes in 47 KiB a microsecond, 2 of weights and one for each
 // group of rows with every k-step.  64 experts, 48 rows each give or take a third, 2048 -> 1024: groups of four with the
@@ -173,11 +172,21 @@ __device__ __forceinline__ void mix_store_tile(const MixGemmArgs& a, f32x4 v, f3
 // half of them idle is half the rate.  16 rows, weights from HBM: 8192 -> 2048 11.5 -> 9.4
 // us, -> 512 10.6 -> 7.8; 6144 -> 2048 9.4 -> 7.8; 4096 -> 2048 7.0 -> 6.6, -> 1024 6.7 ->
 // 6.0; at 2048 inputs the exchange costs more (4.8 -> 5.2).
-template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS, bool PICKED>
-__device__ __forceinline__ void mix_gemm_split(const MixGemmArgs& a, uint32_t bx, uint32_t by, uint32_t z, uint32_t wave, f32x4* s_part)
+// SETS: so many sets of WAVES waves, each with tiles of its own.  (The arguments by value: by reference the loads come out in another order, 1 to
+// 4 % slower for one tile over inputs that are no power of two.)
+template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS, bool PICKED, int SETS = 1>
+__device__ __forceinline__ void mix_gemm_split(const MixGemmArgs a, uint32_t bx, uint32_t by, uint32_t z)
 {
     using V8 = typename MixAct<F32>::V8;
+    constexpr uint32_t SET = WAVES * NT * GR * 64;
+    __shared__ f32x4 s_part[SETS * SET];
     const int lane = threadIdx.x & 63;
+    uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t mine = SETS > 1 ? wave / WAVES * SET : 0;
+    if constexpr (SETS > 1) {
+        bx = bx * SETS + wave / WAVES;
+        wave %= WAVES;
+    }
     static_assert(PARTS == 1 || (PARTS == 2 && NT == 1 && GR == 1), "one tile, two halves");
     if constexpr (STREAM && GR > 1 && !PICKED) {
         if (a.cols) {                                      // runs, up to a multiple of 8: a run's workgroups on one XCD
@@ -303,7 +312,7 @@ __device__ __forceinline__ void mix_gemm_split(const MixGemmArgs& a, uint32_t bx
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int i = 0; i < L; i++) s_part[((wave * NT + t) * GR + i) * 64 + lane] = acc[t][i];
+            for (int i = 0; i < L; i++) s_part[mine + ((wave * NT + t) * GR + i) * 64 + lane] = acc[t][i];
     };
     if constexpr (STREAM && GR > 1) {
         static_assert(GR == 4 || GR == 8);
@@ -327,10 +336,10 @@ __device__ __forceinline__ void mix_gemm_split(const MixGemmArgs& a, uint32_t bx
     }
     lds_barrier();
     auto sum = [&](uint32_t i) {
-        f32x4 v = s_part[i * 64 + lane];
+        f32x4 v = s_part[mine + i * 64 + lane];
 #pragma unroll
         for (int p = 1; p < WAVES; p++) {
-            const f32x4 o = s_part[(p * NT * GR + i) * 64 + lane];
+            const f32x4 o = s_part[mine + (p * NT * GR + i) * 64 + lane];
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] += o[j];
         }
@@ -374,35 +383,29 @@ __device__ __forceinline__ void mix_gemm_split(const MixGemmArgs& a, uint32_t bx
     }
 }
 
-template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS = 1, bool PICKED = false>
+// REGION: an XCD's workgroups take neighbouring tiles (xcd_region).  A form of its own: asked in the kernel, the question was 0.2 us of every launch.
+template <bool F32, int NT, int GR, int WAVES, int DEPTH, bool STREAM, int PARTS = 1, bool PICKED = false, bool REGION = false>
 __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_split_kernel(const MixGemmArgs a)
 {
-    __shared__ f32x4 s_part[WAVES * NT * GR * 64];
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint32_t bx = blockIdx.x;
-    if constexpr (STREAM && GR == 1 && !PICKED) {
-        if (a.cols) bx = xcd_region(bx, gridDim.x);
-    }
-    mix_gemm_split<F32, NT, GR, WAVES, DEPTH, STREAM, PARTS, PICKED>(a, bx, blockIdx.y, blockIdx.z, wave, s_part);
+    const uint32_t bx = REGION ? xcd_region(blockIdx.x, (a.ntiles + NT - 1) / NT) : blockIdx.x;
+    mix_gemm_split<F32, NT, GR, WAVES, DEPTH, STREAM, PARTS, PICKED>(a, bx, blockIdx.y, blockIdx.z);
 }
 
 // Two products of up to sixteen rows that do not wait for each other: a's batch of matrices, and a small one whose few tiles took a launch
 // of their own (16 rows, four of 2048 -> 2048 and 2048 -> 64: 8.7 and 4.6 us, 10.6 together).  Each in the form that it has alone, so the
 // same bits: four waves to a tile of the small one's, a workgroup's other four with the next.
 // The small one's workgroups come first: they end as the others do.
-template <int WAVES, int DEPTH>
+template <int WAVES, int DEPTH, bool REGION>
 __global__ __launch_bounds__(WAVES * 64, WAVES > 4 ? 1 : 2) void mix_gemm_two_kernel(const MixGemmArgs a, const MixGemmArgs b)
 {
-    constexpr uint32_t SETS = WAVES / 4;
-    __shared__ f32x4 s_part[WAVES * 2 * 64];
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int SETS = WAVES / 4;
     const uint32_t of_b = (b.ntiles + SETS - 1) / SETS, of_a = (a.ntiles + 1) / 2;
-    const uint32_t item = a.cols ? xcd_region(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t item = REGION ? xcd_region(blockIdx.x, gridDim.x) : blockIdx.x;
     if (item < of_b) {
-        mix_gemm_split<false, 1, 1, 4, 8, true, 1, false>(b, item * SETS + wave / 4, 0, 0, wave % 4, s_part + wave / 4 * 256);
+        mix_gemm_split<false, 1, 1, 4, 8, true, 1, false, SETS>(b, item, 0, 0);
     } else {
         const uint32_t i = item - of_b;
-        mix_gemm_split<false, 2, 1, WAVES, DEPTH, true, 1, false>(a, i % of_a, 0, i / of_a, wave, s_part);
+        mix_gemm_split<false, 2, 1, WAVES, DEPTH, true, 1, false>(a, i % of_a, 0, i / of_a);
     }
 }
 

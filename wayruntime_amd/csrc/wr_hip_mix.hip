@@ -461,10 +461,10 @@ int wr_hip_mix_shift(wr_hip_mix_step* s, wr_hip_mix_pool* pool, uint32_t run, in
 
 // --------------------------------------------------------------- products --
 
-template <bool F32, int NT, int GR, int WAVES, int D, bool STREAM>
+template <bool F32, int NT, int GR, int WAVES, int D, bool STREAM, bool REGION = false>
 static int launch_split(const MixGemmArgs& a, uint32_t batch)
 {
-    launch_main(mix_gemm_split_kernel<F32, NT, GR, WAVES, D, STREAM>,
+    launch_main(mix_gemm_split_kernel<F32, NT, GR, WAVES, D, STREAM, 1, false, REGION>,
                 dim3((a.ntiles + NT - 1) / NT, (a.groups + GR - 1) / GR, batch), dim3(WAVES * 64), a);
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
@@ -537,15 +537,16 @@ static int launch_runs(const MixGemmArgs& args, uint32_t experts)
 // kernel).
 constexpr uint32_t kPartsMinKtiles = 128;
 
+template <bool REGION>
 static int launch_parts(MixGemmArgs a)
 {
     if (ensure_device(cx->d_part, (size_t)2 * a.ntiles * 64 * sizeof(f32x4)) != WR_HIP_OK) {   // (256 KiB at most)
         (void)hipGetLastError();
-        return launch_split<false, 1, 1, 4, 8, true>(a, 1);
+        return launch_split<false, 1, 1, 4, 8, true, REGION>(a, 1);
     }
     a.part = static_cast<float*>(cx->d_part.p);
     a.tickets = cx->d_counters;
-    launch_main(mix_gemm_split_kernel<false, 1, 1, 4, 8, true, 2>, dim3(a.ntiles, 2), dim3(256), a);
+    launch_main(mix_gemm_split_kernel<false, 1, 1, 4, 8, true, 2, false, REGION>, dim3(a.ntiles, 2), dim3(256), a);
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
 }
@@ -752,10 +753,29 @@ static FewRows few_rows_form(const MixGemmArgs& a, uint32_t batch, bool gated)
 }
 constexpr uint32_t kEightWaveKtiles = 64;
 
-// Up to sixteen rows: whether an XCD's workgroups take neighbouring tiles: where tiles are a multiple of 32 KiB (us, dealt out / so: 2048 -> 16 384
-// gated 13.3 / 12.7, 8192 -> 2048 10.3 / 9.5, 4096 -> 24 576 37.6 / 33.4, four of 2048 -> 2048 8.2 / 7.9; level for weights
-// of 8 MB; others lose a little, 1536 -> 12 288 9.7 / 9.9).
-static uint32_t gemm_regions(const MixGemmArgs& a) { return a.ktiles % 32 == 0; }
+// Up to sixteen rows: whether an XCD's workgroups take neighbouring tiles: where tiles are 32 KiB times a power of two, whose beginnings lie on
+// the same memory channels (16 rows; us, dealt out / so: 2048 -> 8192 8.0 / 7.6, 8192 -> 2048 10.1 / 9.4, 4096 -> 8192 14.8 / 12.8, 8192 -> 8192 26.9 / 22.5, 16 384
+// -> 4096 26.9 / 23.6; others are level or lose up to 3 %, 3072 -> 4096 6.7 / 6.9, 5120 -> 2048 7.4 / 7.6).  A matrix of a batch is shared out by itself: not
+// small ones (16 of 2048 -> 512 8.0 / 9.8, 8 of 4096 -> 512 8.0 / 9.5, 16 of 8192 -> 256 17.1 / 18.1; four of 4096 -> 2048 14.9 / 12.8, 8 of 4096 -> 1024
+// 15.0 / 13.4).  profiles/stack_few_rows_regions.txt has 251 sizes.
+static bool gemm_regions(const MixGemmArgs& a, uint32_t batch)
+{
+    return a.ktiles >= 32 && (a.ktiles & (a.ktiles - 1)) == 0 &&
+           (batch == 1 || a.ktiles == 32 || (a.ntiles >= 32 && (uint64_t)a.ntiles * a.ktiles >= 8192));
+}
+
+template <bool REGION>
+static int launch_few(const MixGemmArgs& a, uint32_t batch, bool gated)
+{
+    switch (few_rows_form(a, batch, gated)) {
+    case FewRows::kFour: return launch_split<false, 4, 1, 4, 2, true>(a, batch);
+    case FewRows::kHalves: return launch_parts<REGION>(a);
+    case FewRows::kOne: return launch_split<false, 1, 1, 4, 8, true, REGION>(a, batch);
+    case FewRows::kTwo: break;
+    }
+    return a.ktiles <= kEightWaveKtiles ? launch_split<false, 2, 1, 8, 4, true, REGION>(a, batch)
+                                        : launch_split<false, 2, 1, 4, 8, true, REGION>(a, batch);
+}
 
 int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
 {
@@ -836,16 +856,7 @@ int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm* q)
         if (a.groups <= 1) return gated ? launch_split<true, 2, 1, 4, 4, true>(a, batch) : launch_split<true, 1, 1, 4, 8, true>(a, batch);
         return launch_split<true, 2, 2, 4, 4, false>(a, batch);
     }
-    if (a.groups == 1) {
-        a.cols = gemm_regions(a);
-        switch (few_rows_form(a, batch, gated)) {
-        case FewRows::kFour: return launch_split<false, 4, 1, 4, 2, true>(a, batch);
-        case FewRows::kHalves: return launch_parts(a);
-        case FewRows::kOne: return launch_split<false, 1, 1, 4, 8, true>(a, batch);
-        case FewRows::kTwo: break;
-        }
-        return a.ktiles <= kEightWaveKtiles ? launch_split<false, 2, 1, 8, 4, true>(a, batch) : launch_split<false, 2, 1, 4, 8, true>(a, batch);
-    }
+    if (a.groups == 1) return gemm_regions(a, batch) ? launch_few<true>(a, batch, gated) : launch_few<false>(a, batch, gated);
     return launch_rows(a, batch, gated);
 }
 
@@ -868,12 +879,16 @@ int wr_hip_mix_gemm_run_two(int f32, const wr_hip_mix_gemm* q, const wr_hip_mix_
     }
     ENTER();
     cx->rows.store(q->rows, std::memory_order_relaxed);
-    a.cols = gemm_regions(a);
     const uint32_t of_a = (a.ntiles + 1) / 2 * batch;
-    if (a.ktiles <= kEightWaveKtiles)
-        launch_main(mix_gemm_two_kernel<8, 4>, dim3(of_a + (b.ntiles + 1) / 2), dim3(512), a, b, 0);
-    else
-        launch_main(mix_gemm_two_kernel<4, 8>, dim3(of_a + b.ntiles), dim3(256), a, b, 0);
+    const auto launch = [&](auto region) {
+        constexpr bool REGION = decltype(region)::value;
+        if (a.ktiles <= kEightWaveKtiles)
+            launch_main(mix_gemm_two_kernel<8, 4, REGION>, dim3(of_a + (b.ntiles + 1) / 2), dim3(512), a, b, 0);
+        else
+            launch_main(mix_gemm_two_kernel<4, 8, REGION>, dim3(of_a + b.ntiles), dim3(256), a, b, 0);
+    };
+    if (gemm_regions(a, 1)) launch(std::true_type());      // (all matrices' tiles are one sequence here)
+    else launch(std::false_type());
     HIP_TRY(hipGetLastError(), "product launch", 0);
     return WR_HIP_OK;
 }
