@@ -25,6 +25,7 @@
 #include "kernels_prefill_il.hip.h"
 #include "kernels_prefill_pair.hip.h"
 #include "kernels_prefill_ild.hip.h"
+#include "prefill_plan.h"
 #include "kernels_proj.hip.h"
 #include "kernels_rows.hip.h"
 #include "kernels_step.hip.h"
@@ -711,76 +712,6 @@ int check_decode(uint32_t n, wr_hip_kv* const* kv, uint32_t layer, const uint32_
     return WR_HIP_OK;
 }
 
-// How a prefill launch is cut: (head, 32-row block) pairs to a workgroup, one block or a long and a short one, and into how many
-// parts the blocks' keys go (one: not at all).
-struct PrefillPlan {
-    uint32_t np, nblk, ny, parts;
-    bool single;
-};
-
-// Four pairs to a workgroup feed eight waves, two to a SIMD, from each tile: the form for launches that fill the chip.  Launches
-// of fewer workgroups than CUs last as long as their longest block; with two pairs a workgroup has half the rows, a wave to
-// a SIMD whose steps take two thirds to nine tenths of the time, and there are twice as many.  A launch whose longest block is still a long chain
-// is cut into parts: every part pays a block's ends (Q in, the sets' merge, rows out) and the rows go through memory once more.
-// In microseconds: the ends of a block and a step (64 keys of a 32-row unit at head dims up to 128, 32 keys at 256) in
-// either form, the combine launch, what it takes a part, and the bytes it and the parts move.  Fitted to eleven shapes by thirteen
-// row counts by nine contexts and windows, both forms, 1 to 32 parts (profiles/prefill_parts.txt): what is picked is 0.7 to 1.4 % off the best
-// on average, 28 % at worst, and takes 0.91 (64), 0.93 (128) and 0.92 (256) of what the parts picked for four pairs alone take, 8 %
-// more at worst.  us a call, four pairs / two: 32/8/64, 500 rows 10.2 / 8.8; 16/8/128, 54 rows 9.0 / 7.9, 1024 rows 19.6 / 17.7; 16/8/256, 177
-// rows 13.9 / 11.3, 1501 rows 53 / 41; 8/4/256, 1501 rows of a 512-key window 25.1 / 21.3.
-PrefillPlan prefill_plan(const PrefillArgs& a, bool parts_form)
-{
-    struct Cost {
-        float ends[2], step[2], combine, part, mb_us;
-    };
-    const Cost c = a.hd == 64    ? Cost{{6.5f, 10.2f}, {0.61f, 0.72f}, 4.9f, 0.33f, 3.2f}
-                   : a.hd == 128 ? Cost{{7.2f, 9.f}, {0.6f, 0.68f}, 2.5f, 0.22f, 3.5f}
-                                 : Cost{{7.f, 8.7f}, {0.89f, 0.96f}, 2.1f, 0.45f, 4.6f};
-    const float row_mb = (float)a.T * a.nq * a.hd * 4e-6f;
-    const uint64_t row_bytes = (uint64_t)a.T * a.nq * (a.hd + 2) * 4;
-    const uint64_t room = (uint64_t)g.prefill_part_mb.load(std::memory_order_relaxed) << 20;
-    const uint32_t per_step = a.hd == 256 ? 1 : 2;
-    PrefillPlan best{};
-    float least = 0.f;
-    for (uint32_t np = 4; np >= (parts_form ? 2u : 4u); np -= 2) {
-        const uint32_t Gw = std::min(a.group, np), BP = 32 * (np / Gw);
-        const uint32_t nblk = (a.T + BP - 1) / BP, ny = a.nkv * (a.group / Gw);
-        const float ends = c.ends[np / 4], step = c.step[np / 4];
-        // tiles of the first and the last block, and of a block on average: as many as the last from where the window is full on
-        const auto tiles_of = [&](uint32_t b) {
-            const uint32_t lo = a.p0 + b * BP, hi = a.p0 + std::min(a.T, (b + 1) * BP);
-            const uint32_t from = (a.window > 0 && lo + 1 > a.window) ? lo + 1 - a.window : 0;
-            return (hi + kTileKeys - 1) / kTileKeys - from / kTileKeys;
-        };
-        const uint32_t first = tiles_of(0), longest = std::max(first, tiles_of(nblk - 1));
-        const float ramp = a.window == 0 ? 1.f : a.window > a.p0 ? std::min(1.f, (float)(a.window - a.p0) / a.T) : 0.f;
-        const float mean = longest - ramp * (longest - first) * 0.5f;
-        // Four pairs: a long and a short block to a workgroup balance the causal triangle, but each pays its own
-        // prologue and epilogue: when the pairs of blocks would not even give every CU a workgroup, one block per workgroup
-        // finishes with the longest block instead of with a pair's sum plus a second prologue and epilogue.
-        const uint32_t two = (nblk + 1) / 2 * ny;
-        const bool single = np == 2 || two < g.n_cus;
-        for (uint32_t p = 1; p <= (parts_form && single ? std::min(kMaxPrefillParts, longest) : 1u); p++) {
-            if (p > 1 && p * row_bytes > room) break;
-            float t;
-            if (!single) {
-                t = ((two + g.n_cus - 1) / g.n_cus) * (2.f * ends - 2.f + step * 2.f * mean / per_step);
-            } else {
-                const uint32_t rounds = (nblk * ny * p + g.n_cus - 1) / g.n_cus;
-                t = ends + step * (((longest + p - 1) / p + per_step - 1) / per_step);
-                if (rounds > 1)                              // long blocks first: the rounds even out
-                    t = std::max(t, rounds * (np == 2 ? 0.95f : 1.f) * (ends + step * mean / (p * per_step)));
-            }
-            if (p > 1) t += c.combine + c.part * p + 2.f * p * row_mb / c.mb_us;
-            if (best.np == 0 || t < least) {
-                least = t;
-                best = PrefillPlan{np, nblk, ny, p, single};
-            }
-        }
-    }
-    return best;
-}
-
 // Room for the parts' rows, in a buffer of their own.  False: there is none, and the launch goes uncut.
 bool prefill_parts_ready(PrefillArgs& a, uint32_t parts)
 {
@@ -820,9 +751,13 @@ int prefill_locked(wr_hip_kv* kv, uint32_t layer, uint32_t p0, uint32_t T, const
     if (q16_dev && !(mfma && (hd == 64 || hd == 128))) return WR_HIP_ERR_UNSUPPORTED;
     if (mfma) {
         const bool one_wave = hd == 128 && !g.prefill_two_waves, four_waves = hd == 256 && g.prefill_256_four_waves;
-        PrefillPlan p = prefill_plan(a, !one_wave && !four_waves);
+        const PrefillSizes sizes = {p0, T, window, nq, kv->nkv, hd};
+        const auto plan = [&](uint32_t parts) {
+            return prefill_plan(sizes, g.n_cus, !one_wave && !four_waves, parts, (uint64_t)g.prefill_part_mb.load(std::memory_order_relaxed) << 20);
+        };
+        PrefillPlan p = plan(kMaxPrefillParts);
+        if (p.parts > 1 && !prefill_parts_ready(a, p.parts)) p = plan(1);
         a.single = p.single;
-        if (p.parts > 1 && !prefill_parts_ready(a, p.parts)) p.parts = 1;
         const dim3 grid(p.ny, p.single ? p.nblk : (p.nblk + 1) / 2, p.parts);
         if (one_wave) {
             if (q16_dev)
