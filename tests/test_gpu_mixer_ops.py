@@ -895,6 +895,49 @@ def test_recurrence_of_many_workgroups(lib, f32, rule, dim, rank, rows):
     many.end(), alone.end()
 
 
+# The append and the recurrence of a step in one launch (bfloat16, DELTA, head sizes 33 to 64, ranks up to 128, no request of more than 16 rows, 8 a request where rows
+# are not asked for ahead) and
+# either side of each of these: the bits of the two calls, in rows, keys, values and states; refused whole, whichever of the two it is.
+@pytest.mark.parametrize("f32,rule,dim,rank,rows,heads", [(False, DELTA, 64, 64, [1], 3), (False, DELTA, 33, 32, [1] * 16, 3), (False, DELTA, 64, 128, [16] * 16, 3),
+                                                          (False, DELTA, 40, 96, [3, 1, 16], 3), (False, DELTA, 64, 160, [2, 1], 3), (False, DELTA, 32, 64, [2, 1], 3),
+                                                          (False, DELTA, 65, 64, [2, 1], 3), (False, BONUS, 64, 64, [2, 1], 3), (False, DELTA, 64, 64, [2, 17], 3),
+                                                          (True, DELTA, 64, 64, [2, 1], 3), (False, DELTA, 40, 64, [1] * 16, 64), (False, DELTA, 40, 64, [8] * 15 + [9], 64)])
+def test_append_and_recurrence(lib, f32, rule, dim, rank, rows, heads):
+    win = Window(heads=6, kv_heads=3, dim=40, dim_pad=64, vdim=24, vdim_pad=32, rot_half=8, window=1 << 20, scale=0.2, out_scale=1.0, eps=1e-6, maps=1)
+    of_win = 6 * 40 + 3 * 40 + 3 * 24
+    wide = -(-heads * dim // 32) * 32
+    t = Recur(lib, f32, heads, dim, rank, rows, rule, win, 5 * wide + of_win + 4)
+    angles = t.put(t.rng.uniform(-1, 1, (t.total, 8, 2)))
+    cols, kt = (5 * wide, 5 * wide + 240, 5 * wide + 360), 6 * 64 // 32
+    q, o = t.fill(t.padded * kt * 32 * t.e), t.fill(t.padded * 6 * t.e * 32)
+
+    def step(pool, nth, together):
+        t.set(pool, nth)
+        head = (t.step, pool, 0, int(f32), C.byref(win), t.rec.in_, t.ld, *cols, angles, q.p)
+        if together:
+            assert lib.wr_hip_mix_window_append_recur(*head, 0, C.byref(t.rec)) == 0
+        else:
+            assert lib.wr_hip_mix_window_append(*head) == 0
+            assert lib.wr_hip_mix_recur(t.step, pool, 0, int(f32), C.byref(t.rec)) == 0
+        assert lib.wr_hip_mix_window_attend(t.step, pool, 0, int(f32), C.byref(win), q.p, None, None, 0, o.p, 6) == 0
+        out = t.out()
+        return [out] + [t.r.frag_down(b, t.total, n * 32) for b, n in ((q, kt), (o, 6))]
+
+    one, two = t.pool(), t.pool()
+    for nth in (0, 1):                                     # from nothing, then from what the first left
+        for a, b in zip(step(one, nth, True), step(two, nth, False)):
+            assert np.isfinite(a).all() and a.any() and np.array_equal(a, b), nth
+    t.set(one, 2)
+    clean = q.to_host((q.nbytes,), np.uint8), t.h.to_host((t.h.nbytes,), np.uint8)
+    lib.wr_hip_attn_h2d(t.rec.in_, np.zeros((t.total, t.ld), np.float32).ctypes.data, t.total * t.ld * 4)
+    for bad_win, bad_run in ((win, 1), (Window(), 0)):
+        assert lib.wr_hip_mix_window_append_recur(t.step, one, 0, int(f32), C.byref(bad_win), t.rec.in_, t.ld, *cols, angles, q.p, bad_run,
+                                                  C.byref(t.rec)) == hipattn.ERR_INVAL
+        hipattn.sync()
+        assert np.array_equal(q.to_host((q.nbytes,), np.uint8), clean[0]) and np.array_equal(t.h.to_host((t.h.nbytes,), np.uint8), clean[1])
+    t.end()
+
+
 # One row to a workgroup up to 599 rows (1791 with experts' rows) and wherever no fragment is written, four beyond; features
 # that a workgroup holds in registers (4096) and more.
 @pytest.mark.parametrize("f32", [False, True])
