@@ -179,7 +179,8 @@ typedef struct wr_hip_mix_gemm {
     const float *x_scale;          /* with group_expert: row i's outputs are those of x_scale[i] times its input */
 } wr_hip_mix_gemm;
 int wr_hip_mix_gemm_run(int f32, const wr_hip_mix_gemm *a);
-/* The same for two products that neither read nor overwrite what the other writes; few rows take one launch where the second is small. */
+/* The same for two products that neither read nor overwrite what the other writes; both are checked before either is launched, and up to sixteen
+ * rows take one launch where the second is small. */
 int wr_hip_mix_gemm_run_two(int f32, const wr_hip_mix_gemm *a, const wr_hip_mix_gemm *small);
 
 /* ---- decayed linear attention ------------------------------------------------
@@ -284,7 +285,8 @@ int wr_hip_mix_window_append(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t
                              const wr_hip_mix_window *g, const float *in_dev, uint32_t ld, uint32_t col_q,
                              uint32_t col_k, uint32_t col_v, const float *table_dev, void *q_dev);
 /* wr_hip_mix_window_append, then wr_hip_mix_recur with layer run recur_run, neither of which reads or overwrites what the other
- * writes; a step of few rows takes one launch for both. */
+ * writes; both are checked before either is launched, and a step whose requests bring sixteen rows each at most takes one launch for both
+ * where the recurrence has a form of the append's size (bfloat16, DELTA, dim 33 to 64). */
 int wr_hip_mix_window_append_recur(wr_hip_mix_step *s, wr_hip_mix_pool *pool, uint32_t run, int f32,
                                    const wr_hip_mix_window *g, const float *in_dev, uint32_t ld, uint32_t col_q,
                                    uint32_t col_k, uint32_t col_v, const float *table_dev, void *q_dev,

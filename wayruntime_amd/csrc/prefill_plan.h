@@ -20,7 +20,7 @@ struct PrefillPlan {
 
 // Four pairs to a workgroup feed eight waves, two to a SIMD, from each tile: the form for launches that fill the chip.  Launches
 // of fewer workgroups than CUs last as long as their longest block; with two pairs a workgroup has half the rows, a wave to
-// a SIMD whose steps take 0.74 to 0.89 of the time, and there are twice as many.  A launch whose longest block is still a long chain
+// a SIMD whose steps take 0.74 to 0.87 of the time, and there are twice as many.  A launch whose longest block is still a long chain
 // is cut into parts: every part pays a block's ends (Q in, the sets' merge, rows out) and the rows go through memory once more.
 // In microseconds: the ends of a block, a step (64 keys of a 32-row unit at head dims up to 128, 32 keys at 256) and the tiles' way into LDS in
 // either form, the combine launch, what it takes a part and eight of them beyond the first (it asks for eight at a time: 32/8/64, 3 rows behind 4000 keys, 8 parts
@@ -31,9 +31,9 @@ struct PrefillPlan {
 // rows 29.0 and 25.2.)  At head dim 64 two workgroups of two pairs fit a CU: one that shares it takes 1.49 of a step, and 512 are a
 // round (16/16/64, 1501 rows 21.9 us in fours, 18.2; 3000 39.0 and 33.7).
 // Fitted to eleven shapes by thirteen row counts by nine contexts and windows, both forms, 1 to 32 parts (profiles/prefill_parts.txt has all
-// of them, with what is picked and what was picked of four pairs alone): what is picked is 0.5 to 0.8 % off the best on average, 13 % at worst, and takes 0.90 (64), 0.93
-// (128) and 0.92 (256) of what the parts picked for four pairs alone take; more than 2 % more at two sizes (8/2/256, 2048 rows of a window of 128
-// behind 100 keys, 256 workgroups on 256 CUs: 18.8, 20.2; 8/4/256, 33 rows behind 16 000 keys: 32.2, 33.7).
+// of them, with what is picked and what was picked of four pairs alone): what is picked is 0.2 to 0.5 % off the best on average, 25 % at worst, and takes 0.90 (64), 0.92
+// (128) and 0.91 (256) of what the parts picked for four pairs alone take; more than 2.5 % more at two sizes (8/2/256, 2048 rows of a window of 128
+// behind 100 keys, 256 workgroups on 256 CUs: 18.6, 20.0; 8/4/256, 33 rows behind 16 000 keys: 31.0, 33.2).
 // `parts`: most parts; `twos`: whether workgroups of two pairs are there; `room`: bytes for the parts' rows.
 inline PrefillPlan prefill_plan(const PrefillSizes& a, uint32_t n_cus, bool twos, uint32_t parts, uint64_t room)
 {
